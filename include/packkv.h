@@ -315,6 +315,12 @@ int pkv_attn_decode(const pkv_attn_args *args, float *ms_out, pkv_stream_t s);
  * pkv_attn_decode itself uses the same array when its stream is capturing a graph and has no scratch of its own. */
 int pkv_attn_decode_noalloc(const pkv_attn_args *args, pkv_stream_t s);
 
+/* pkv_dense_view: the dense K and V [B, Hkv, T_c + T_w, 128] `dtype` behind the same arguments (q, out, Hq, sm_scale,
+ * variant and flags are not looked at): the compressed tokens as the reference stores them, dtype(dtype(code + zero) *
+ * scale) (utils/compute.py:173-179), then the T_w window rows -- the tensors the reference's cache returns from
+ * `update` (models/cache/packkv_quant.py:84-85).  k_bits and v_bits 2..8; outputs and windows 16-byte aligned. */
+int pkv_dense_view(const pkv_attn_args *args, void *k_out, void *v_out, pkv_stream_t s);
+
 /* pkv_stream_release: gives back the device memory the library keeps for stream `s` of the current device -- its
  * scratch buffers (attention partials, the encoders' look-back state), its tile counters and every buffer it has
  * outgrown (kept until now because a captured HIP graph might still hold its address).  It has no counterpart in the

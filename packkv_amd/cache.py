@@ -219,22 +219,10 @@ class PackKVCompressedCache:
         """(K, V) [B, H, T, 128]: the dequantised prefix followed by the window, i.e. the tensors the reference's
         ``update`` returns for decompress-then-attend."""
         L = self._layer(layer_idx)
-        out = []
-        for side, win in ((L.k, L.k_win), (L.v, L.v_win)):
-            parts = []
-            if side.tokens:
-                hidden = side.B * side.H * 128
-                codes = torch.empty(side.tokens, hidden, dtype=torch.uint8, device=win.device)
-                dec = ops.k_decode if side.is_k else ops.v_decode
-                nblk = side.tokens // 128 * side.blocks_per_tile
-                dec(side.stream, side.info[:nblk], codes, bits=side.bits)
-                sc = side.scale[:, :side.tokens].contiguous()
-                ze = side.zero[:, :side.tokens].contiguous()
-                parts.append(ops.dequantize(codes, sc, ze, side.B, side.H))
-            if L.win_len:
-                parts.append(win[:, :, :L.win_len])
-            out.append(torch.cat(parts, dim=2) if parts else None)
-        return out[0], out[1]
+        if not L.k.tokens and not L.win_len:
+            return None, None
+        return ops.dense_view(L.k.as_dict() if L.k.tokens else None, L.v.as_dict() if L.k.tokens else None,
+                              L.k_win if L.win_len else None, L.v_win if L.win_len else None, L.win_len)
 
     def cache_bytes(self, layer_idx=None):
         """Bytes the cache holds (streams in use, block_info and parameters of the encoded tokens, the 16-bit

@@ -85,49 +85,53 @@ __device__ __forceinline__ void unit_parse2(const uint8_t *blk_a, uint32_t off_a
     }
 }
 
-// ---- widths 5..8 (format extension): pack words of up to 128 bits, plain field-by-field code ----
-typedef unsigned __int128 word128;
+// ---- the codes of a unit -------------------------------------------------------------------------------------
+// unit_codes hands lane t's four packs to `sink(k, c4)` token by token: c4 holds the codes of slots 0..3 at token k of
+// the pack, one per byte, slot 0 lowest.
 
-template <bool IS_K>
-__device__ __forceinline__ void unit_decode_wide(const uint8_t *blk, uint32_t unit_off, int unit, int t,
-                                                 const UnitGeom g, uint8_t *tile, int hid_blk) {
+// Widths 5..8 (format extension): pack words of up to 128 bits, the four slots' words shifted down one field at a time
+// (token 15 sits in the lowest field).
+template <class Sink>
+__device__ __forceinline__ void unit_codes_wide(const uint8_t *blk, uint32_t unit_off, int t, const UnitGeom g, Sink sink) {
     const uint32_t minsw = lds_meta_word(blk + unit_off, t, g.W);
     const uint32_t lensw = lds_meta_word(blk + unit_off + g.mins_bytes, t, g.LB);
     const uint32_t pay0 = unit_off + g.mins_bytes + g.lens_bytes;
-    uint32_t len[4], mn[4], off[4], payload;
+    uint32_t len[4], mn[4], off[4], mask[4], d[4][4], payload;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         len[i] = (lensw >> (i * g.LB)) & ((1u << g.LB) - 1u);
         mn[i] = (minsw >> (i * g.W)) & ((1u << g.W) - 1u);
+        mask[i] = (1u << len[i]) - 1u;
     }
     pack_offsets(len, off, payload);
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        // the word as four dwords, shifted down one field at a time (token 15 sits in the lowest field)
         const uint64_t lo = lds_load64(blk, pay0 + off[i]), hi = lds_load64(blk, pay0 + off[i] + 8u);
-        uint32_t d0 = (uint32_t)lo, d1 = (uint32_t)(lo >> 32), d2 = (uint32_t)hi, d3 = (uint32_t)(hi >> 32);
-        const uint32_t mask = (1u << len[i]) - 1u, sh = len[i];
+        d[i][0] = (uint32_t)lo; d[i][1] = (uint32_t)(lo >> 32); d[i][2] = (uint32_t)hi; d[i][3] = (uint32_t)(hi >> 32);
+    }
 #pragma unroll
-        for (int k = kPackTok - 1; k >= 0; k--) {
-            tile[tile_index<IS_K>(unit, i, k, t, hid_blk)] = (uint8_t)((d0 & mask) + mn[i]);
-            d0 = __builtin_amdgcn_alignbit(d1, d0, sh);
-            d1 = __builtin_amdgcn_alignbit(d2, d1, sh);
-            d2 = __builtin_amdgcn_alignbit(d3, d2, sh);
-            d3 >>= sh;
+    for (int k = kPackTok - 1; k >= 0; k--) {
+        uint32_t c4 = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            c4 |= (((d[i][0] & mask[i]) + mn[i]) & 0xFFu) << (8 * i);
+            d[i][0] = __builtin_amdgcn_alignbit(d[i][1], d[i][0], len[i]);
+            d[i][1] = __builtin_amdgcn_alignbit(d[i][2], d[i][1], len[i]);
+            d[i][2] = __builtin_amdgcn_alignbit(d[i][3], d[i][2], len[i]);
+            d[i][3] >>= len[i];
         }
+        sink(k, c4);
     }
 }
 
-// Decode one unit whose bytes start at blk[unit_off] into the LDS tile.
 // The four pack words are cut into 16-bit windows of four tokens (packs 0|1 and 2|3 share a
 // register), so one packed 16-bit shift moves two packs at a time and a byte permute gathers the
 // four codes of a token: 5 instructions per four codes instead of a 64-bit shift per code.
-template <bool IS_K>
-__device__ __forceinline__ void unit_decode(const uint8_t *blk, uint32_t unit_off, int unit, int t,
-                                            const UnitGeom g, uint8_t *tile, int hid_blk) {
+template <class Sink>
+__device__ __forceinline__ void unit_codes(const uint8_t *blk, uint32_t unit_off, int t, const UnitGeom g, Sink sink) {
     typedef unsigned short u16pair __attribute__((ext_vector_type(2)));
     if (g.W > 4) {      // uniform
-        unit_decode_wide<IS_K>(blk, unit_off, unit, t, g, tile, hid_blk);
+        unit_codes_wide(blk, unit_off, t, g, sink);
         return;
     }
     UnitPacks u;
@@ -154,20 +158,27 @@ __device__ __forceinline__ void unit_decode(const uint8_t *blk, uint32_t unit_of
         const uint32_t w23 = __builtin_amdgcn_perm(qd[3], qd[2], 0x05040100u);
 #pragma unroll
         for (int pp = 0; pp < 4; pp++) {
-            const int k = 4 * q + pp;
             const u16pair s01 = __builtin_bit_cast(u16pair, len01 * (uint32_t)(3 - pp));
             const u16pair s23 = __builtin_bit_cast(u16pair, len23 * (uint32_t)(3 - pp));
             const uint32_t x01 = __builtin_bit_cast(uint32_t, (u16pair)(__builtin_bit_cast(u16pair, w01) >> s01));
             const uint32_t x23 = __builtin_bit_cast(uint32_t, (u16pair)(__builtin_bit_cast(u16pair, w23) >> s23));
-            const uint32_t c4 = (__builtin_amdgcn_perm(x23, x01, 0x06040200u) & mq) + minq;   // codes of slots 0..3
-            if (IS_K) {   // slots are the four adjacent channels 4t..4t+3 of token k
-                *reinterpret_cast<uint32_t *>(tile + tile_index<true>(unit, 0, k, t, hid_blk)) = c4;
-            } else {      // slots are four rounds of channel t
-#pragma unroll
-                for (int i = 0; i < 4; i++) tile[tile_index<false>(unit, i, k, t, hid_blk)] = (uint8_t)(c4 >> (8 * i));
-            }
+            sink(4 * q + pp, (__builtin_amdgcn_perm(x23, x01, 0x06040200u) & mq) + minq);
         }
     }
+}
+
+// Decode one unit whose bytes start at blk[unit_off] into the LDS tile.
+template <bool IS_K>
+__device__ __forceinline__ void unit_decode(const uint8_t *blk, uint32_t unit_off, int unit, int t,
+                                            const UnitGeom g, uint8_t *tile, int hid_blk) {
+    unit_codes(blk, unit_off, t, g, [&](int k, uint32_t c4) {
+        if (IS_K) {   // slots are the four adjacent channels 4t..4t+3 of token k
+            *reinterpret_cast<uint32_t *>(tile + tile_index<true>(unit, 0, k, t, hid_blk)) = c4;
+        } else {      // slots are four rounds of channel t
+#pragma unroll
+            for (int i = 0; i < 4; i++) tile[tile_index<false>(unit, i, k, t, hid_blk)] = (uint8_t)(c4 >> (8 * i));
+        }
+    });
 }
 
 // Gather lane t's four packs of `unit` from the LDS code tile and compute min / len / word
@@ -251,6 +262,8 @@ __device__ __forceinline__ void unit_emit(uint8_t *blk, uint32_t unit_off, int t
         if (len > 3u) dst[3] = (uint16_t)(hi >> 16);
     }
 }
+
+typedef unsigned __int128 word128;
 
 // Widths 5..8: analyse lane t's four packs of `unit` and write them at blk[unit_off] (the unit's size is
 // known from a first call with blk == nullptr, which only returns it).  The metadata fields do not fall on byte

@@ -761,6 +761,42 @@ def fused_wv(our_wv, w, v_quant_zero, v_quant_scale, term1):
 
 # ------------------------------------------------- fused decompress-attention --------
 
+def dense_view(k, v, k_win=None, v_win=None, win_len=None):
+    """(K, V) [B, H, T, 128] behind a compressed cache: k and v as attn_decode takes them (stream, info, scale, zero,
+    bits, ``tokens``, ``heads``) or None, dequantised as the reference stores them (utils/compute.py:173-179), followed
+    by the `win_len` rows in use of the 16-bit windows k_win / v_win [B, H, cap, 128].  One launch."""
+    a = AttnArgs()
+    like = k["scale"] if k is not None else k_win
+    if k is not None:
+        T_c, B = int(k.get("tokens", k["scale"].size(1))), k["scale"].size(0)
+        H = int(k["heads"]) if "heads" in k else k["info"].numel() // 2 // (T_c // 64) // B
+        a.k_stream, a.k_info, a.k_scale, a.k_zero = _ptr(k["stream"]), _ptr(k["info"]), _ptr(k["scale"]), _ptr(k["zero"])
+        a.v_stream, a.v_info, a.v_scale, a.v_zero = _ptr(v["stream"]), _ptr(v["info"]), _ptr(v["scale"]), _ptr(v["zero"])
+        a.k_bytes, a.v_bytes = k["stream"].numel(), v["stream"].numel()
+        a.k_bits, a.v_bits, a.par_stride = int(k["bits"]), int(v["bits"]), k["scale"].size(1)
+        for d in (k, v):
+            _require(d["scale"].shape == k["scale"].shape and d["zero"].shape == k["scale"].shape and d["scale"].size(1) >= T_c
+                     and d["info"].numel() // 2 >= T_c // 64 * B * H and all(d[f].is_cuda and d[f].is_contiguous()
+                                                                             for f in ("stream", "info", "scale", "zero")),
+                     "stream, info, scale and zero must be contiguous device tensors that hold the tokens in use")
+    else:
+        T_c, H, B = 0, k_win.size(1), k_win.size(0)
+    T_w = 0
+    if k_win is not None:
+        T_w = k_win.size(2) if win_len is None else int(win_len)
+        _require(k_win.is_cuda and v_win.is_cuda and k_win.is_contiguous() and v_win.is_contiguous() and k_win.shape == v_win.shape
+                 and k_win.shape[:2] == (B, H) and k_win.size(3) == 128 and 0 <= T_w <= k_win.size(2) and k_win.dtype == like.dtype
+                 and v_win.dtype == like.dtype, "window tensors must be contiguous [B, H, cap, 128] of the cache's dtype")
+        a.k_win, a.v_win, a.win_stride = _ptr(k_win), _ptr(v_win), k_win.size(2)
+    a.B, a.Hkv, a.T_c, a.T_w, a.dtype = B, H, T_c, T_w, _dtype_code(like)
+    k_out = torch.empty(B, H, T_c + T_w, 128, dtype=like.dtype, device=like.device)
+    v_out = torch.empty_like(k_out)
+    with torch.cuda.device(like.device):
+        rc = _lib.load().pkv_dense_view(ctypes.byref(a), _ptr(k_out), _ptr(v_out), _stream(like.device))
+    _lib.check(rc)
+    return k_out, v_out
+
+
 class AttnPlan:
     """The checked, filled-in arguments of one decode step, kept for callers that repeat it (a decode loop over the
     same layer): ``plan()`` launches again without re-validating; ``plan(q=..., out=...)`` swaps the query / output

@@ -246,3 +246,25 @@ def test_reference_cache_class_and_its_two_line_hook(cuda):
     finally:
         PackKVCacheConfigStatic.config = None
         PackKVCacheConfigStatic.max_tokens = 32768
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rel,T_c,T_w", [(0.5, 128, 1), (0.2, 384, 64), (0.1, 256, 65), (0.1, 0, 191), (0.05, 128, 0), (0.025, 256, 63),
+                                         (0.0125, 128, 130), (0.00625, 128, 5)])
+def test_dense_view_equals_the_restated_dequantisation(cuda, dtype, rel, T_c, T_w):
+    """Widths 2..8, with and without compressed tokens, window rows around the 64-row pieces: bit for bit (the window
+    is a copy, and every dequantised element is two single roundings of exact values)."""
+    B, H, cap = 2, 3, 200
+    k, v = synth.make_kv(B, H, max(T_c, 128), seed=77, dtype=dtype)
+    kw, vw = synth.make_kv(B, H, cap, seed=78, dtype=dtype)
+    sides, want = [], []
+    for x, w, enc in ((k, kw, ops.k_quant_encode), (v, vw, ops.v_quant_encode)):
+        parts = [w[:, :, :T_w]]
+        if T_c:
+            c, z, s = oq.quant_ints(x, 64, rel)
+            parts.insert(0, oq.dequant(c, z, s))
+        want.append(torch.cat(parts, dim=2))
+        sides.append(dict(enc(x.to(cuda), rel), heads=H) if T_c else None)
+    got = ops.dense_view(sides[0], sides[1], kw.to(cuda), vw.to(cuda), T_w)
+    for g, w in zip(got, want):
+        assert g.shape == w.shape and torch.equal(g.cpu().view(torch.int16), w.view(torch.int16))
