@@ -266,11 +266,6 @@ __global__ void __launch_bounds__(256) pack_group_kernel(const uint8_t *__restri
         reinterpret_cast<uint16_t *>(dst + done)[i] = reinterpret_cast<const uint16_t *>(gbuf + done)[i];
 }
 
-__global__ void zero_state_kernel(uint64_t *p, size_t n) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0;
-}
-
 struct CodecShape {
     int nunits, threads, nblocks;
     uint32_t blk_cap, lds_bytes;
@@ -327,40 +322,6 @@ static int run_unpack(bool is_k, const uint8_t *stream, uint64_t stream_bytes, c
     return tm.end(ms_out);
 }
 
-// Shared tail of every encoder: read back {error, total} when the caller wants the size.
-int finish_encode(ScanState *st, uint64_t *size_out, int bits, hipStream_t s) {
-    if (!size_out) return PKV_OK;
-    struct { uint32_t ticket, error; uint64_t total; uint32_t max_code, pad; } h;
-    PKV_HIP_CHECK(hipMemcpyAsync(&h, st, sizeof(h), hipMemcpyDeviceToHost, s));
-    PKV_HIP_CHECK(hipStreamSynchronize(s));
-    if (h.error == (uint32_t)PKV_ERR_CAPACITY) {
-        set_error("compressed stream does not fit the output buffer");
-        return PKV_ERR_CAPACITY;
-    }
-    if (h.error) {
-        set_error("device-side encode failure (code %u)", h.error);
-        return (int)h.error;
-    }
-    if (bits > 0 && h.max_code >= (1u << bits)) {
-        set_error("not supported: code %u does not fit bits_len %d", h.max_code, bits);
-        return PKV_ERR_UNSUPPORTED;
-    }
-    *size_out = h.total;
-    return PKV_OK;
-}
-
-int prepare_scan_state(uint32_t nblocks, ScanState **out, hipStream_t s) {
-    void *p = nullptr;
-    const size_t bytes = sizeof(ScanState) + (size_t)nblocks * sizeof(uint64_t);
-    int rc = scratch_get(bytes, s, &p, kScratchEncoder);
-    if (rc) return rc;
-    const size_t n64 = (bytes + 7) / 8;
-    zero_state_kernel<<<(unsigned)((n64 + 255) / 256), 256, 0, s>>>((uint64_t *)p, n64);
-    PKV_HIP_CHECK(hipGetLastError());
-    *out = (ScanState *)p;
-    return PKV_OK;
-}
-
 static int run_pack(bool is_k, const uint8_t *codes, uint8_t *stream, uint64_t capacity, uint32_t *info,
                     int ctx_len, int hidden_dim, int ctx_blk, int hid_blk, int bits, uint64_t *size_out,
                     float *ms_out, hipStream_t s) {
@@ -373,7 +334,7 @@ static int run_pack(bool is_k, const uint8_t *codes, uint8_t *stream, uint64_t c
     CodecShape cs;
     int rc = codec_shape(is_k, ctx_len, hidden_dim, ctx_blk, hid_blk, bits, &cs);
     if (rc) return rc;
-    ScanState *st = nullptr;
+    ScanHandle sh;
     // blocks of four units, 16-byte aligned rows: eight blocks per workgroup (not at 8 bits, where the group's 88 KB
     // of LDS leave one workgroup per CU and the per-block kernel is 10 % faster)
     const bool grouped = cs.nunits == 4 && bits <= 7 && hid_blk % 16 == 0 && hidden_dim % 16 == 0 &&
@@ -384,17 +345,19 @@ static int run_pack(bool is_k, const uint8_t *codes, uint8_t *stream, uint64_t c
                        (is_k ? (ctx_blk == 64 && hid_blk == 128) : (ctx_blk == 128 && hid_blk == 64));
     if (cells) {
         const uint32_t ngroups = (uint32_t)cs.nblocks / (is_k ? 8u : 16u);
-        if ((rc = prepare_scan_state(ngroups, &st, s))) return rc;
+        if ((rc = prepare_scan_state(ngroups, &sh, s))) return rc;
+        ScanState *st = sh.st;
         LaunchTimer tm(s, ms_out != nullptr);
         if ((rc = tm.begin())) return rc;
         if ((rc = launch_code_cells(is_k, codes, ctx_len, hidden_dim, bits, cs.blk_cap, stream, capacity, info, st, ngroups, s))) return rc;
         if ((rc = tm.end(ms_out))) return rc;
-        return finish_encode(st, size_out, 0, s);
+        return finish_encode(sh, size_out, 0, s);
     }
     if (grouped) {
         const uint32_t ngroups = ((uint32_t)cs.nblocks + kPackGroup - 1) / kPackGroup;
         const uint32_t lds = 2u * (uint32_t)(ctx_blk * hid_blk) + (uint32_t)kPackGroup * cs.blk_cap + 32u;
-        if ((rc = prepare_scan_state(ngroups, &st, s))) return rc;
+        if ((rc = prepare_scan_state(ngroups, &sh, s))) return rc;
+        ScanState *st = sh.st;
         auto kern = bits > 4 ? (is_k ? pack_group_kernel<true, true> : pack_group_kernel<false, true>)
                              : (is_k ? pack_group_kernel<true, false> : pack_group_kernel<false, false>);
         if (lds > 48u * 1024u)
@@ -407,9 +370,10 @@ static int run_pack(bool is_k, const uint8_t *codes, uint8_t *stream, uint64_t c
                                        (uint32_t)cs.nblocks, ngroups, sg);
         PKV_HIP_CHECK(hipGetLastError());
         if ((rc = tm.end(ms_out))) return rc;
-        return finish_encode(st, size_out, 0, s);
+        return finish_encode(sh, size_out, 0, s);
     }
-    if ((rc = prepare_scan_state((uint32_t)cs.nblocks, &st, s))) return rc;
+    if ((rc = prepare_scan_state((uint32_t)cs.nblocks, &sh, s))) return rc;
+    ScanState *st = sh.st;
     LaunchTimer tm(s, ms_out != nullptr);
     if ((rc = tm.begin())) return rc;
     if (is_k)
@@ -422,7 +386,7 @@ static int run_pack(bool is_k, const uint8_t *codes, uint8_t *stream, uint64_t c
             (uint32_t)cs.nblocks);
     PKV_HIP_CHECK(hipGetLastError());
     if ((rc = tm.end(ms_out))) return rc;
-    return finish_encode(st, size_out, 0, s);
+    return finish_encode(sh, size_out, 0, s);
 }
 
 }  // namespace pkv
@@ -453,16 +417,6 @@ int pkv_v_decode(const uint8_t *stream, uint64_t stream_bytes, const uint32_t *b
                  int hidden_dim, int ctx_blk, int hid_blk, int bits, float *ms_out, pkv_stream_t s) {
     return pkv::run_unpack(false, stream, stream_bytes, block_info, codes, ctx_len, hidden_dim, ctx_blk, hid_blk, bits,
                            ms_out, (hipStream_t)s);
-}
-
-int pkv_encode_status(pkv_stream_t s_, int bits, uint64_t *size_out) {
-    using namespace pkv;
-    hipStream_t s = (hipStream_t)s_;
-    PKV_REQUIRE(size_out != nullptr, PKV_ERR_INVALID, "null pointer argument");
-    void *st = nullptr;
-    int rc = encoder_state_peek(s, &st);
-    if (rc) return rc;
-    return finish_encode(static_cast<ScanState *>(st), size_out, bits, s);
 }
 
 uint64_t pkv_block_bound(int is_k, int ctx_blk, int hid_blk, int bits) {

@@ -893,8 +893,9 @@ static int run_pack_long(bool is_k, const uint8_t *codes, uint8_t *stream, uint6
     PKV_REQUIRE(capacity > 0, PKV_ERR_INVALID, "compressed_buffer must be a non-empty tensor");
     if (capacity > (1ull << 32)) capacity = 1ull << 32;          // block_info offsets are 32 bits: never wrapped
     const uint32_t nblocks = (uint32_t)(ctx_len / ((is_k ? 4 : 8) * P)) * (uint32_t)(hidden_dim / (is_k ? 128 : 64));
-    ScanState *st = nullptr;
-    if ((rc = prepare_scan_state(nblocks, &st, s))) return rc;
+    ScanHandle sh;
+    if ((rc = prepare_scan_state(nblocks, &sh, s))) return rc;
+    ScanState *st = sh.st;
     LaunchTimer tm(s, ms_out != nullptr);
     if ((rc = tm.begin())) return rc;
     const int threads = 128 * long_chunks(P);
@@ -948,7 +949,7 @@ static int run_pack_long(bool is_k, const uint8_t *codes, uint8_t *stream, uint6
     }
     PKV_HIP_CHECK(hipGetLastError());
     if ((rc = tm.end(ms_out))) return rc;
-    return finish_encode(st, size_out, 0, s);
+    return finish_encode(sh, size_out, 0, s);
 }
 
 static int run_unpack_long(bool is_k, const uint8_t *stream, uint64_t stream_bytes, const uint32_t *info, uint8_t *codes,

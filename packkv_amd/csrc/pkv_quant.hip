@@ -1972,7 +1972,7 @@ static int run_quant_encode(const void *x, int dtype, int B, int H, int T, float
     // that would grow past 4 GiB is reported as a full buffer instead of wrapping its offsets
     if (capacity > (1ull << 32)) capacity = 1ull << 32;
     PKV_REQUIRE(base <= capacity, PKV_ERR_CAPACITY, "stream offset beyond 4 GiB: block_info offsets are 32 bits");
-    ScanState *st = nullptr;
+    ScanHandle sh;
     // One workgroup per run of up to eight heads of a (context block, sequence) group -- K: its up to eight blocks;
     // V: its up to sixteen -- or, with fewer than five heads, per 8 / H groups.
     {
@@ -1985,7 +1985,8 @@ static int run_quant_encode(const void *x, int dtype, int B, int H, int T, float
         const uint32_t nruns_all = (uint32_t)(T / ctx_blk) * (uint32_t)B * (uint32_t)nruns;
         PKV_REQUIRE((uint64_t)nsub + (uint64_t)nruns_all * (uint64_t)ctx_blk < (1ull << 31), PKV_ERR_UNSUPPORTED, "batch x tokens too large");
         const uint32_t xwords = H <= kSubBlocks ? 0u : nruns_all * (uint32_t)ctx_blk;
-        if ((rc = prepare_scan_state(nsub + xwords, &st, s))) return rc;
+        if ((rc = prepare_scan_state(nsub + xwords, &sh, s))) return rc;
+        ScanState *st = sh.st;
         LaunchTimer tm(s, ms_out != nullptr);
         if ((rc = tm.begin())) return rc;
         if (!IS_K && H <= 8) {               // one workgroup per group of 2 H blocks
@@ -2084,7 +2085,7 @@ static int run_quant_encode(const void *x, int dtype, int B, int H, int T, float
         }
         PKV_HIP_CHECK(hipGetLastError());
         if ((rc = tm.end(ms_out))) return rc;
-        return finish_encode(st, size_out, bits, s);
+        return finish_encode(sh, size_out, bits, s);
     }
 }
 

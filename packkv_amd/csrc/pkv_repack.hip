@@ -867,8 +867,9 @@ int pkv_greedy_repack(const uint8_t *k_codes, const uint8_t *v_codes, uint8_t *k
     }
     int rc;
     if (groups > 0) {
-        ScanState *st = nullptr;
-        if ((rc = prepare_scan_state(groups * 2u * members * 128u, &st, s))) return rc;
+        ScanHandle sh;
+        if ((rc = prepare_scan_state(groups * 2u * members * 128u, &sh, s))) return rc;
+        ScanState *st = sh.st;
         LaunchTimer tm(s, ms_out != nullptr);
         if ((rc = tm.begin())) return rc;
         if (wide)
@@ -880,12 +881,10 @@ int pkv_greedy_repack(const uint8_t *k_codes, const uint8_t *v_codes, uint8_t *k
         if (rows) gather_rows_kernel<<<(unsigned)ctx_len, 256, 0, s>>>(k_codes, v_codes, k_out, v_out, perm, block_size, hidden_dim);
         PKV_HIP_CHECK(hipGetLastError());
         if ((rc = tm.end(ms_out))) return rc;
-        if (ms_out) {                                  // a timed call has waited for the kernels: look at the error word
-            uint32_t head[2] = {0u, 0u};
-            PKV_HIP_CHECK(hipMemcpyAsync(head, st, sizeof(head), hipMemcpyDeviceToHost, s));
-            PKV_HIP_CHECK(hipStreamSynchronize(s));
-            PKV_REQUIRE(head[1] == 0u, PKV_ERR_INTERNAL, "greedy order: a workgroup waited too long for the sums of its group");
-        }
+        uint64_t none = 0;                             // a timed call waits for the kernels: it looks at the error word too
+        rc = finish_encode(sh, ms_out ? &none : nullptr, 0, s);
+        PKV_REQUIRE(rc != PKV_ERR_INTERNAL, PKV_ERR_INTERNAL, "greedy order: a workgroup waited too long for the sums of its group");
+        if (rc) return rc;
         return PKV_OK;
     }
     // longer blocks: the cost word holds (bits << 8 | token): bits <= 8 * 2 * hidden_dim must stay below 2^24

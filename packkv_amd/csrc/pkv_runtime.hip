@@ -5,7 +5,9 @@
 #include <tuple>
 #include <map>
 
+#include <chrono>
 #include <cstdarg>
+#include <cstddef>
 #include <cstdio>
 #include <mutex>
 #include <vector>
@@ -29,11 +31,21 @@ namespace {
 struct Workspace {
     int dev;
     hipStream_t stream;
-    void *ptr[2];           // kScratchGeneral, kScratchEncoder
-    size_t bytes[2];
+    void *ptr;              // general scratch
+    size_t bytes;
     uint32_t *counters;     // kAttnCounters tile counters of the attention kernel, zero between launches
-    bool encoded;           // an encoder has run on this stream: ptr[kScratchEncoder] starts with its ScanState
+    void *enc;              // the encoders' look-back state, zero between encodes
+    size_t enc_bytes;
+    bool enc_dirty;         // between prepare_scan_state and the launch of the clearing kernel
+    uint64_t *last;         // pinned, host and device: outcome of the last encode on this stream (kOutcomeWords)
+    bool encoded;           // an encoder has run on this stream
+    std::shared_ptr<std::mutex> enc_mu;
 };
+constexpr int kOutcomeWords = 2, kSlotWords = 8;      // a slot: two outcomes (a cache line)
+constexpr int kSlotsPerChunk = 64;
+std::vector<uint64_t *> g_chunks;                     // pinned slots of the encodes that are waited for (any device)
+std::vector<uint64_t *> g_free_slots;                 // as many as host threads have waited at once, in chunks of 64
+uint32_t g_seq = 0;                                   // tag of an outcome, 30 bits, never 0
 std::vector<Workspace> g_ws;
 struct Retired { int dev; hipStream_t stream; void *ptr; };
 std::vector<Retired> g_retired;     // superseded buffers, kept until their stream is released (a captured graph may hold them)
@@ -44,7 +56,7 @@ int workspace_for(hipStream_t s, Workspace **out) {     // caller holds g_ws_mu
     PKV_HIP_CHECK(hipGetDevice(&dev));
     for (Workspace &w : g_ws)
         if (w.dev == dev && w.stream == s) { *out = &w; return PKV_OK; }
-    g_ws.push_back(Workspace{dev, s, {nullptr, nullptr}, {0, 0}, nullptr, false});
+    g_ws.push_back(Workspace{dev, s, nullptr, 0, nullptr, nullptr, 0, false, nullptr, false, std::make_shared<std::mutex>()});
     *out = &g_ws.back();
     return PKV_OK;
 }
@@ -63,37 +75,199 @@ static bool capturing(hipStream_t s) {
     return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
 }
 
-int scratch_get(size_t bytes, hipStream_t s, void **out, int kind) {
+int scratch_get(size_t bytes, hipStream_t s, void **out) {
     std::lock_guard<std::mutex> lock(g_ws_mu);
     Workspace *w = nullptr;
     int rc = workspace_for(s, &w);
     if (rc) return rc;
-    if (kind == kScratchEncoder) w->encoded = true;
-    if (w->bytes[kind] < bytes) {
+    if (w->bytes < bytes) {
         if (capturing(s)) {
             set_error("stream is capturing a graph and has no scratch buffer of %zu bytes yet: make one eager call "
                       "of the same shape on this stream first", bytes);
             return PKV_ERR_CAPTURING;
         }
-        const size_t want = scratch_grown_size(w->bytes[kind], bytes);
+        const size_t want = scratch_grown_size(w->bytes, bytes);
         void *fresh = nullptr;
         PKV_HIP_CHECK(hipMalloc(&fresh, want));
-        if (w->ptr[kind]) g_retired.push_back(Retired{w->dev, s, w->ptr[kind]});
-        w->ptr[kind] = fresh;
-        w->bytes[kind] = want;
+        if (w->ptr) g_retired.push_back(Retired{w->dev, s, w->ptr});
+        w->ptr = fresh;
+        w->bytes = want;
     }
-    *out = w->ptr[kind];
+    *out = w->ptr;
     return PKV_OK;
 }
 
-int encoder_state_peek(hipStream_t s, void **out) {
-    std::lock_guard<std::mutex> lock(g_ws_mu);
+// ---- the encoders' look-back state and outcome ------------------------------------------------------------------
+// An outcome is two words, each valid by itself through its tag: total (34 bits) | tag << 34 and error (8 bits) |
+// largest code (16 bits) << 8 | tag << 34.
+__device__ __forceinline__ void publish_outcome(uint64_t *dst, const ScanState *st, uint64_t tag) {
+    const uint64_t total = st->total & ((1ull << 34) - 1ull), code = min(st->max_code, 0xFFFFu);
+    __hip_atomic_store(dst, total | (tag << 34), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(dst + 1, (uint64_t)(st->error & 0xFFu) | (code << 8) | (tag << 34), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The outcome of the encode before it on the stream to `last` and, for a waiting caller, to `slot`; the state back to
+// zero.  Four words per thread: the state of 1 GiB of input (8192 tickets) is cleared by nine workgroups in 2 us.
+__global__ void __launch_bounds__(256) finish_encode_kernel(ScanState *st, ScanState *second, uint64_t *words, uint32_t n, uint64_t *last,
+                                                            uint64_t *slot, uint32_t tag) {
+    constexpr uint32_t kHead = offsetof(ScanState, status) / 8;
+    const uint32_t head2 = second ? (uint32_t)(reinterpret_cast<uint64_t *>(second) - words) : 0xFFFFFFFFu;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (slot) publish_outcome(slot, st, tag);
+        if (slot && second) publish_outcome(slot + kOutcomeWords, second, tag);
+        publish_outcome(last, second ? second : st, tag);
+        for (uint32_t i = 0; i < kHead; i++) {
+            words[i] = 0;
+            if (second) words[head2 + i] = 0;
+        }
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++) {
+        const uint32_t i = kHead + (blockIdx.x * 4u + k) * 256u + threadIdx.x;
+        if (i < n && (i < head2 || i >= head2 + kHead)) words[i] = 0;
+    }
+}
+__global__ void __launch_bounds__(256) clear_state_kernel(uint64_t *p, size_t n) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) p[i] = 0;
+}
+
+int prepare_scan_state(uint32_t nblocks, ScanHandle *out, hipStream_t s, uint32_t nblocks2) {
+    constexpr size_t head = offsetof(ScanState, status) / 8;
+    const size_t n1 = head + nblocks, n = n1 + (nblocks2 ? head + nblocks2 : 0);
     Workspace *w = nullptr;
-    int rc = workspace_for(s, &w);
-    if (rc) return rc;
-    PKV_REQUIRE(w->encoded && w->ptr[kScratchEncoder], PKV_ERR_INVALID, "no encode has been launched on this stream");
-    *out = w->ptr[kScratchEncoder];
+    int rc;
+    {
+        std::lock_guard<std::mutex> lock(g_ws_mu);
+        if ((rc = workspace_for(s, &w))) return rc;
+        out->mu = w->enc_mu;
+    }
+    out->held = std::unique_lock<std::mutex>(*out->mu);
+    std::lock_guard<std::mutex> lock(g_ws_mu);
+    if ((rc = workspace_for(s, &w))) return rc;            // (the list may have moved meanwhile)
+    bool clear = w->enc_dirty;                     // an earlier call failed between its two launches
+    if (w->enc_bytes < n * 8 || !w->last) {
+        if (capturing(s)) {
+            set_error("stream is capturing a graph and has no scratch buffer of %zu bytes yet: make one eager call "
+                      "of the same shape on this stream first", n * 8);
+            return PKV_ERR_CAPTURING;
+        }
+        if (!w->last) PKV_HIP_CHECK(hipHostMalloc((void **)&w->last, kOutcomeWords * 8, hipHostMallocMapped | hipHostMallocCoherent));
+        if (w->enc_bytes < n * 8) {
+            const size_t want = scratch_grown_size(w->enc_bytes, n * 8);
+            void *fresh = nullptr;
+            PKV_HIP_CHECK(hipMalloc(&fresh, want));
+            if (w->enc) g_retired.push_back(Retired{w->dev, s, w->enc});
+            w->enc = fresh;
+            w->enc_bytes = want;
+            clear = true;
+        }
+    }
+    if (clear) {
+        const size_t all = w->enc_bytes / 8;
+        clear_state_kernel<<<(unsigned)((all + 255) / 256), 256, 0, s>>>((uint64_t *)w->enc, all);
+        PKV_HIP_CHECK(hipGetLastError());
+    }
+    w->enc_dirty = true;
+    out->st = (ScanState *)w->enc;
+    out->second = nblocks2 ? (ScanState *)((uint64_t *)w->enc + n1) : nullptr;
+    out->words64 = n;
     return PKV_OK;
+}
+
+static int outcome(const volatile uint64_t *o, uint64_t *size_out, int bits) {
+    const uint32_t error = (uint32_t)(o[1] & 0xFFu), max_code = (uint32_t)(o[1] >> 8) & 0xFFFFu;
+    if (error == (uint32_t)PKV_ERR_CAPACITY) {
+        set_error("compressed stream does not fit the output buffer");
+        return PKV_ERR_CAPACITY;
+    }
+    if (error) {
+        set_error("device-side encode failure (code %u)", error);
+        return (int)error;
+    }
+    if (bits > 0 && max_code >= (1u << bits)) {
+        set_error("not supported: code %u does not fit bits_len %d", max_code, bits);
+        return PKV_ERR_UNSUPPORTED;
+    }
+    *size_out = o[0] & ((1ull << 34) - 1ull);
+    return PKV_OK;
+}
+
+// Polls pinned memory until `n` words carry the tag: the answer is there a microsecond or two after the kernel wrote
+// it, where a copy and a stream synchronisation take about 20.  After 20 ms -- a long queue ahead, or a fault -- the
+// stream is waited for in the ordinary way.
+static int wait_words(const volatile uint64_t *w, int n, uint32_t tag, hipStream_t s) {
+    const auto t0 = std::chrono::steady_clock::now();
+    for (bool synced = false;;) {
+        for (int i = 0; i < 256; i++) {
+            bool there = true;
+            for (int k = 0; k < n; k++) there = there && (uint32_t)(w[k] >> 34) == tag;
+            if (there) return PKV_OK;
+            __builtin_ia32_pause();
+        }
+        PKV_REQUIRE(!synced, PKV_ERR_INTERNAL, "the encoder's outcome did not arrive");
+        if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(20)) {
+            PKV_HIP_CHECK(hipStreamSynchronize(s));
+            synced = true;
+        }
+    }
+}
+
+int finish_encode(ScanHandle &h, uint64_t *size_out, int bits, hipStream_t s, uint64_t *size2_out, int bits2) {
+    uint64_t *slot = nullptr;
+    uint32_t tag = 0;
+    {
+        std::lock_guard<std::mutex> lock(g_ws_mu);
+        Workspace *w = nullptr;
+        int rc = workspace_for(s, &w);
+        if (rc) return rc;
+        g_seq = (g_seq + 1) & 0x3FFFFFFFu;
+        if (!g_seq) g_seq = 1;
+        tag = g_seq;
+        if (size_out) {
+            if (g_free_slots.empty()) {
+                void *chunk = nullptr;
+                PKV_HIP_CHECK(hipHostMalloc(&chunk, (size_t)kSlotsPerChunk * kSlotWords * 8,
+                                            hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable));
+                g_chunks.push_back((uint64_t *)chunk);
+                for (int i = 0; i < kSlotsPerChunk; i++) g_free_slots.push_back((uint64_t *)chunk + (size_t)i * kSlotWords);
+            }
+            slot = g_free_slots.back();
+            g_free_slots.pop_back();
+        }
+        const uint32_t n = (uint32_t)h.words64;
+        finish_encode_kernel<<<(n + 1023u) / 1024u, 256, 0, s>>>(h.st, h.second, (uint64_t *)h.st, n, w->last, slot, tag);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) {
+            if (slot) g_free_slots.push_back(slot);
+            set_error("launch of the encoder's last kernel failed: %s", hipGetErrorString(e));
+            return PKV_ERR_HIP;
+        }
+        w->enc_dirty = false;
+        w->encoded = true;
+    }
+    h.held.unlock();
+    if (!slot) return PKV_OK;
+    int rc = wait_words(slot, h.second ? 4 : 2, tag, s);
+    if (!rc) rc = outcome(slot, size_out, bits);
+    if (!rc && h.second && size2_out) rc = outcome(slot + kOutcomeWords, size2_out, bits2);
+    std::lock_guard<std::mutex> lock(g_ws_mu);
+    g_free_slots.push_back(slot);
+    return rc;
+}
+
+static int encode_status(hipStream_t s, int bits, uint64_t *size_out) {
+    const uint64_t *last = nullptr;
+    {
+        std::lock_guard<std::mutex> lock(g_ws_mu);
+        Workspace *w = nullptr;
+        int rc = workspace_for(s, &w);
+        if (rc) return rc;
+        PKV_REQUIRE(w->encoded && w->last, PKV_ERR_INVALID, "no encode has been launched on this stream");
+        last = w->last;
+    }
+    PKV_HIP_CHECK(hipStreamSynchronize(s));
+    return outcome(last, size_out, bits);
 }
 
 int attn_counters_get(hipStream_t s, uint32_t **out) {
@@ -132,8 +306,9 @@ int stream_release(hipStream_t s) {
     PKV_HIP_CHECK(hipStreamSynchronize(s));
     if (at < g_ws.size()) {
         Workspace &w = g_ws[at];
-        for (int k = 0; k < 2; k++)
-            if (w.ptr[k]) PKV_HIP_CHECK(hipFree(w.ptr[k]));
+        if (w.ptr) PKV_HIP_CHECK(hipFree(w.ptr));
+        if (w.enc) PKV_HIP_CHECK(hipFree(w.enc));
+        if (w.last) PKV_HIP_CHECK(hipHostFree(w.last));
         if (w.counters) PKV_HIP_CHECK(hipFree(w.counters));
         g_ws.erase(g_ws.begin() + (long)at);
     }
@@ -206,5 +381,10 @@ int pkv_abi_version(void) { return PKV_ABI_VERSION; }
 const char *pkv_last_error(void) { return pkv::g_error; }
 
 }  // extern "C"
+
+extern "C" int pkv_encode_status(pkv_stream_t s, int bits, uint64_t *size_out) {
+    PKV_REQUIRE(size_out != nullptr, PKV_ERR_INVALID, "null pointer argument");
+    return pkv::encode_status((hipStream_t)s, bits, size_out);
+}
 
 extern "C" int pkv_stream_release(pkv_stream_t s) { return pkv::stream_release((hipStream_t)s); }
