@@ -156,6 +156,23 @@ int pkv_v_quant_encode_append(const void *x, int dtype, int B, int H, int T_new,
                                void *scale_tail, void *zero_tail, int par_stride, uint64_t *size_out,
                                float *ms_out, pkv_stream_t s);
 
+/* pkv_kv_quant_encode_append: the two appends of a cut with one wait.  T_new (a multiple of 128) tokens of K and of V,
+ * each read where it lies: element strides from one sequence, head and token to the next (multiples of 8, the rows on
+ * 16-byte boundaries), so a cut needs no copy of the prompt it is taken from.  k_size / v_size receive the bytes in
+ * use after the append; both encodes are launched before the call waits for either. */
+typedef struct pkv_append_side {
+    const void *x;
+    int64_t stride_b, stride_h, stride_t;
+    uint8_t *stream;
+    uint64_t capacity, used;
+    uint32_t *info_tail;
+    void *scale_tail, *zero_tail;
+    float rel;
+    int bits;
+} pkv_append_side;
+int pkv_kv_quant_encode_append(const pkv_append_side *k, const pkv_append_side *v, int dtype, int B, int H, int T_new,
+                               int par_stride, uint64_t *k_size, uint64_t *v_size, pkv_stream_t s);
+
 /* ---- the decode step's write into a cache's 16-bit window ------------------------------
  * pkv_window_append: rows win_pos .. win_pos + n - 1 of the windows k_win / v_win [B, H, win_stride, 128] receive the
  * new tokens k_new / v_new [B, H, n, 128] (element strides stride_b / stride_h / stride_t, channels contiguous; the
@@ -167,6 +184,26 @@ int pkv_v_quant_encode_append(const void *x, int dtype, int B, int H, int T_new,
 int pkv_window_append(const void *k_new, const void *v_new, const void *cos, const void *sin, int dtype, int B, int H,
                       int n, int64_t stride_b, int64_t stride_h, int64_t stride_t, int64_t rot_stride_b, void *k_win,
                       void *v_win, int win_pos, int win_stride, pkv_stream_t s);
+
+/* pkv_window_cut: the rest of such a write when 64-token blocks leave the window for the streams (`cut_tensor`,
+ * utils/compute.py:54-67, and the reference's cat / slice around it, models/cache/packkv_quant.py:59-83).  The tokens at
+ * hand, in order: the originals of a pending cut (k_pend / v_pend [B, H, 64, 128], pend = 64 or 0), rows pend ..
+ * pend + buf - 1 of k_win / v_win, the n new tokens (strides and rotary embedding as in pkv_window_append, all strides
+ * multiples of 8).  The first `stage` of them are written to k_stage / v_stage [B, H, stage, 128] for the encoder; a NULL
+ * stage buffer leaves a side out, which is allowed where the encoder can read the new tokens as they are (nothing pending
+ * or buffered; K: no rotary embedding).  The next pend_out (64 or 0) tokens are the new pending cut: originals to
+ * k_pend_out / v_pend_out, and rows 0 .. 63 of the new window receive them quantised at k_rel / v_rel and dequantised.
+ * What remains fills the rows behind.  The new window k_win_out / v_win_out has the old one's shape and buffers of its
+ * own.  All buffers 16-byte aligned. */
+typedef struct pkv_cut_args {
+    const void *k_new, *v_new, *cos, *sin;
+    int64_t stride_b, stride_h, stride_t, rot_stride_b;
+    const void *k_pend, *v_pend, *k_win, *v_win;
+    void *k_stage, *v_stage, *k_pend_out, *v_pend_out, *k_win_out, *v_win_out;
+    int dtype, B, H, n, pend, buf, stage, pend_out, win_stride;
+    float k_rel, v_rel;
+} pkv_cut_args;
+int pkv_window_cut(const pkv_cut_args *args, pkv_stream_t s);
 
 /* ---- token repacking and the analytic pack-size model ---------------------------------
  * On the uint8 code matrix [ctx_len, hidden_dim] (channel = (b * H + h) * 128 + d).

@@ -18,6 +18,7 @@ ATTN_REF_ROUNDING, ATTN_OUT_F32 = 1, 2
 _vp = ctypes.c_void_p
 _i = ctypes.c_int
 _u64 = ctypes.c_uint64
+_i64 = ctypes.c_int64
 _f = ctypes.c_float
 _fp = ctypes.POINTER(ctypes.c_float)
 _u64p = ctypes.POINTER(ctypes.c_uint64)
@@ -33,6 +34,20 @@ class AttnArgs(ctypes.Structure):
         ("k_bits", _i), ("v_bits", _i), ("dtype", _i), ("sm_scale", _f), ("variant", _i),
         ("par_stride", _i), ("win_stride", _i), ("flags", _i),
     ]
+
+
+class AppendSide(ctypes.Structure):
+    _fields_ = [("x", _vp), ("stride_b", _i64), ("stride_h", _i64), ("stride_t", _i64), ("stream", _vp), ("capacity", _u64),
+                ("used", _u64), ("info_tail", _vp), ("scale_tail", _vp), ("zero_tail", _vp), ("rel", _f), ("bits", _i)]
+
+
+class CutArgs(ctypes.Structure):
+    _fields_ = ([(n, _vp) for n in ("k_new", "v_new", "cos", "sin")] +
+                [(n, _i64) for n in ("stride_b", "stride_h", "stride_t", "rot_stride_b")] +
+                [(n, _vp) for n in ("k_pend", "v_pend", "k_win", "v_win", "k_stage", "v_stage", "k_pend_out", "v_pend_out",
+                                    "k_win_out", "v_win_out")] +
+                [(n, _i) for n in ("dtype", "B", "H", "n", "pend", "buf", "stage", "pend_out", "win_stride")] +
+                [("k_rel", _f), ("v_rel", _f)])
 
 
 # name -> (restype, argtypes); every symbol include/packkv.h declares
@@ -60,6 +75,8 @@ SIGNATURES = {
     "pkv_v_quant_encode": (_i, [_vp, _i, _i, _i, _i, _f, _i, _vp, _u64, _vp, _vp, _vp, _u64p, _fp, _vp]),
     "pkv_k_quant_encode_append": (_i, [_vp, _i, _i, _i, _i, _f, _i, _vp, _u64, _u64, _vp, _vp, _vp, _i, _u64p, _fp, _vp]),
     "pkv_v_quant_encode_append": (_i, [_vp, _i, _i, _i, _i, _f, _i, _vp, _u64, _u64, _vp, _vp, _vp, _i, _u64p, _fp, _vp]),
+    "pkv_kv_quant_encode_append": (_i, [ctypes.POINTER(AppendSide), ctypes.POINTER(AppendSide), _i, _i, _i, _i, _i, _u64p, _u64p, _vp]),
+    "pkv_window_cut": (_i, [ctypes.POINTER(CutArgs), _vp]),
     "pkv_window_append": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64,
                                ctypes.c_int64, _vp, _vp, _i, _i, _vp]),
     "pkv_bit_pack_size": (_i, [_vp, _i, _i, _i, _u64p, ctypes.POINTER(ctypes.c_uint32), _fp, _vp]),

@@ -62,14 +62,16 @@ class _Side:
         self.bound = ops.block_bound(is_k, ctx_blk, hid_blk, bits)
         self.par_stride = (max_tokens + 127) // 128 * 128
         self.info = torch.empty(self.par_stride // 128 * self.blocks_per_tile, 2, dtype=torch.uint32, device=device)
-        self.scale = torch.zeros(B, self.par_stride, dtype=dtype, device=device)
-        self.zero = torch.zeros(B, self.par_stride, dtype=dtype, device=device)
+        self.scale = torch.empty(B, self.par_stride, dtype=dtype, device=device)
+        self.zero = torch.empty(B, self.par_stride, dtype=dtype, device=device)
         self.stream = torch.empty(0, dtype=torch.uint8, device=device)
         self.used = 0          # bytes of the stream in use
         self.tokens = 0        # tokens encoded
 
-    def _reserve(self, n_tiles):
+    def reserve(self, n_tiles):
         """Room for n_tiles more tiles at their worst-case size, plus the slack the readers ask for."""
+        if self.tokens + 128 * n_tiles > self.par_stride:
+            raise RuntimeError("compressed cache is full (%d tokens)" % self.par_stride)
         need = self.used + n_tiles * self.blocks_per_tile * self.bound + 16
         if need > self.stream.numel():
             # grow by what the cache has needed so far per token, at least half as much again
@@ -77,15 +79,8 @@ class _Side:
             grown[: self.used] = self.stream[: self.used]
             self.stream = grown
 
-    def append(self, x):
-        """x [B, H, n, 128], n a multiple of 128: encode and append."""
-        n = x.size(2)
-        if self.tokens + n > self.par_stride:
-            raise RuntimeError("compressed cache is full (%d tokens)" % self.par_stride)
-        self._reserve(n // 128)
-        self.used = ops.quant_encode_append(self.is_k, x, self.rel, self.bits, self.stream, self.used, self.info,
-                                            self.tokens, self.scale, self.zero)
-        self.tokens += n
+    def args(self):
+        return (self.rel, self.bits, self.stream, self.used, self.info, self.scale, self.zero)
 
     def as_dict(self):
         return {"stream": self.stream, "info": self.info, "scale": self.scale, "zero": self.zero, "bits": self.bits,
@@ -143,29 +138,22 @@ class PackKVCompressedCache:
                               cache_kwargs["sin"] if rotary else None, L.k_win, L.v_win, L.win_len)
             L.win_len += n
         else:
-            if rotary:
-                key_states = apply_rotary_pos_emb_single(key_states, cache_kwargs["cos"], cache_kwargs["sin"])
-            kbuf = torch.cat([L.k_win[:, :, L.pend:L.win_len], key_states], dim=2)
-            vbuf = torch.cat([L.v_win[:, :, L.pend:L.win_len], value_states], dim=2)
-            k_cut, v_cut = kbuf[:, :, :n_cut], vbuf[:, :, :n_cut]
-            if L.pend:
-                k_cut, v_cut = torch.cat([L.k_pend, k_cut], dim=2), torch.cat([L.v_pend, v_cut], dim=2)
-            whole = k_cut.size(2) // 128 * 128
-            if whole:
-                L.k.append(k_cut[:, :, :whole].contiguous())
-                L.v.append(v_cut[:, :, :whole].contiguous())
-            L.pend = k_cut.size(2) - whole
+            cut = L.pend + n_cut                    # tokens that are quantised now or were and wait for their partner
+            whole = cut // 128 * 128
             left = total - n_cut
-            if L.pend + left > L.cap:
-                raise RuntimeError("not supported: %d tokens left in the 16-bit window" % (L.pend + left))
-            if L.pend:
-                L.k_pend, L.v_pend = k_cut[:, :, whole:].contiguous(), v_cut[:, :, whole:].contiguous()
-                L.k_win[:, :, :L.pend] = self._quant_dequant(L.k_pend, cfg.k_quant_scale_rel)
-                L.v_win[:, :, :L.pend] = self._quant_dequant(L.v_pend, cfg.v_quant_scale_rel)
-            else:
-                L.k_pend = L.v_pend = None
-            L.k_win[:, :, L.pend:L.pend + left] = kbuf[:, :, n_cut:]
-            L.v_win[:, :, L.pend:L.pend + left] = vbuf[:, :, n_cut:]
+            if cut - whole + left > L.cap:
+                raise RuntimeError("not supported: %d tokens left in the 16-bit window" % (cut - whole + left))
+            if whole:
+                L.k.reserve(whole // 128)
+                L.v.reserve(whole // 128)
+            k_enc, v_enc, k_pend, v_pend, k_win, v_win = ops.window_cut(
+                key_states, value_states, cache_kwargs["cos"] if rotary else None, cache_kwargs["sin"] if rotary else None,
+                L.k_pend, L.v_pend, L.k_win, L.v_win, L.win_len, whole, cut - whole, cfg.k_quant_scale_rel, cfg.v_quant_scale_rel)
+            if whole:
+                L.k.used, L.v.used = ops.kv_quant_encode_append(k_enc, v_enc, whole, L.k.args(), L.v.args(), L.k.tokens)
+                L.k.tokens += whole
+                L.v.tokens += whole
+            L.pend, L.k_pend, L.v_pend, L.k_win, L.v_win = cut - whole, k_pend, v_pend, k_win, v_win
             L.win_len = L.pend + left
             L.plan = None                  # token counts (and possibly the stream buffers) changed
         if return_dense:
@@ -209,12 +197,6 @@ class PackKVCompressedCache:
         return res.unsqueeze(2) if squeeze else res
 
     # -- dense view and accounting ---------------------------------------------------------------------
-    @staticmethod
-    def _quant_dequant(x, rel):
-        scale, zero = ops.quant_params(x, rel)
-        codes, _ = ops.quantize(x, scale, zero)
-        return ops.dequantize(codes, scale, zero, x.size(0), x.size(1))
-
     def materialize(self, layer_idx):
         """(K, V) [B, H, T, 128]: the dequantised prefix followed by the window, i.e. the tensors the reference's
         ``update`` returns for decompress-then-attend."""

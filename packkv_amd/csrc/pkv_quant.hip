@@ -289,6 +289,63 @@ __global__ void __launch_bounds__(256) dequantize_kernel(const uint8_t *__restri
     }
 }
 
+// ---- quantise and dequantise at once ---------------------------------------------------
+// A 64-token cut that waits for its partner is attended in the form the streams will give it: parameters, codes and
+// dequantised values of n tokens in one launch, K and V in the grid's third dimension.  grid (ceil(n / 16), B, 2), the
+// thread roles of quantize_kernel over all heads; the second read of the rows comes from L1 / L2.  Latency-bound: a few
+// workgroups, once every 128 tokens (params, quantize and dequantize kernels with their read-back took 70 us a side).
+struct QdqSide { const uint16_t *x; uint16_t *out; float rel; };
+template <int DT>
+__global__ void __launch_bounds__(256) quant_dequant_kernel(const QdqSide k, const QdqSide v, int H, int n, int out_rows) {
+    const QdqSide sd = blockIdx.z ? v : k;
+    const int b = blockIdx.y, tok = blockIdx.x * 16 + (threadIdx.x >> 4), l16 = threadIdx.x & 15;
+    if (tok >= n) return;                                    // (whole rows of 16 lanes)
+    float mn = INFINITY, mx = -INFINITY;
+    const uint16_t *rows = sd.x + ((size_t)b * H * n + tok) * kHeadDim + l16 * 8;
+#pragma unroll 4
+    for (int h = 0; h < H; h++) {
+        float f[8];
+        unpack8<DT>(*reinterpret_cast<const uint4 *>(rows + (size_t)h * n * kHeadDim), f);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            mn = fminf(mn, f[i]);
+            mx = fmaxf(mx, f[i]);
+        }
+    }
+#pragma unroll
+    for (int d = 8; d >= 1; d >>= 1) {
+        mn = fminf(mn, __shfl_xor(mn, d, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, d, 16));
+    }
+    const float sc = round_t<DT>(round_t<DT>(mx - mn) * sd.rel);
+    const float z = round_t<DT>(rintf(round_t<DT>(__fdiv_rn(mn, sc))));
+    const TokPar tp = token_par<DT>(sc, T16<DT>::to_bits(z), false);
+    uint16_t *out = sd.out + ((size_t)b * H * out_rows + tok) * kHeadDim + l16 * 8;
+#pragma unroll 2
+    for (int h = 0; h < H; h++) {
+        const uint4 w = *reinterpret_cast<const uint4 *>(rows + (size_t)h * n * kHeadDim);
+        uint32_t c[4], r[4];                                 // codes of adjacent channels as 16-bit pairs
+        quant4<DT, false>(make_uint2(w.x, w.y), tp, c[0], c[1]);
+        quant4<DT, false>(make_uint2(w.z, w.w), tp, c[2], c[3]);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float a0 = (float)(c[i] & 0xFFu), a1 = (float)((c[i] >> 16) & 0xFFu);
+            r[i] = T16<DT>::to_bits(round_t<DT>(a0 + z) * sc) | (T16<DT>::to_bits(round_t<DT>(a1 + z) * sc) << 16);
+        }
+        *reinterpret_cast<uint4 *>(out + (size_t)h * out_rows * kHeadDim) = make_uint4(r[0], r[1], r[2], r[3]);
+    }
+}
+
+int launch_quant_dequant(const void *k, const void *v, void *k_out, void *v_out, int dtype, int B, int H, int n, int out_rows, float k_rel,
+                         float v_rel, hipStream_t s) {
+    const QdqSide ks{(const uint16_t *)k, (uint16_t *)k_out, k_rel}, vs{(const uint16_t *)v, (uint16_t *)v_out, v_rel};
+    const dim3 grid((unsigned)((n + 15) / 16), (unsigned)B, 2);
+    if (dtype == PKV_F16) quant_dequant_kernel<PKV_F16><<<grid, 256, 0, s>>>(ks, vs, H, n, out_rows);
+    else quant_dequant_kernel<PKV_BF16><<<grid, 256, 0, s>>>(ks, vs, H, n, out_rows);
+    PKV_HIP_CHECK(hipGetLastError());
+    return PKV_OK;
+}
+
 // bit_length of both 16-bit halves, clamped to 4 (values above 15 mean the codes overflow the
 // format; the launch reports that through max_code)
 __device__ __forceinline__ uint32_t pk_bitlen4(uint32_t d) {
@@ -388,20 +445,24 @@ __device__ __forceinline__ f16x2 pk_max_h(f16x2 a, f16x2 b) {
     return r;
 }
 
+// Where the rows of x lie: elements from one sequence, head and token to the next (channels contiguous, every row on a
+// 16-byte boundary).  A cut of a prompt is encoded where it is, also as a transposed projection output.
+struct XRows { int64_t sb, sh, st; };
+
 // Token parameters of one round of the round-major encoders for a group of up to four heads (several of which share
 // a workgroup).  256 threads per 16 tokens: thread (tt = token, l16) reads 8 channels of every head; lane l16 == 0
 // writes the token's scale and zero and its constants for quant4.  `rows` is x at (sequence, head 0, the round's first
 // token) and uniform, so the loads are one 32-bit lane offset on scalar bases; only the rows that exist are
 // fetched and compared.
 template <int DT>
-__device__ __forceinline__ void round_token_params_few(const uint16_t *rows, size_t head_stride, int H, int tt, int l16, float rel,
+__device__ __forceinline__ void round_token_params_few(const uint16_t *rows, const XRows xs, int H, int tt, int l16, float rel,
                                                        uint16_t *scale_out, uint16_t *zero_out, TokPar *par_out) {
-    const uint32_t lane_off = (uint32_t)(tt * kHeadDim + l16 * 8) * 2u;          // bytes
+    const uint32_t lane_off = ((uint32_t)tt * (uint32_t)xs.st + (uint32_t)l16 * 8u) * 2u;          // bytes (row strides are below 2^25 elements)
     uint4 v[4];
     v[0] = *reinterpret_cast<const uint4 *>(reinterpret_cast<const char *>(rows) + lane_off);
 #pragma unroll
     for (int i = 1; i < 4; i++)
-        if (i < H) v[i] = *reinterpret_cast<const uint4 *>(reinterpret_cast<const char *>(rows + (size_t)i * head_stride) + lane_off);
+        if (i < H) v[i] = *reinterpret_cast<const uint4 *>(reinterpret_cast<const char *>(rows + i * xs.sh) + lane_off);
     float mn, mx;
     if (DT == PKV_F16) {
         f16x2 lo, hi;
@@ -434,9 +495,19 @@ __device__ __forceinline__ void round_token_params_few(const uint16_t *rows, siz
     }
 }
 
-__device__ __forceinline__ void cell_load(const uint16_t *xc, uint2 xr[16]) {
+// `rows` (uniform) is the first of the cell's 16 token rows, `lane_off` the lane's byte offset from it, `row_bytes` (uniform)
+// the bytes from row to row: a load is one 32-bit lane offset on a scalar base.  (Rows as immediates of a per-lane 64-bit
+// address need the row stride as a constant, and a branch between the two forms took registers: 131 and 149 instead of
+// 128 at most in the K kernel, fused K + V encode of 2 x 1 GiB 630 -> 723 us.)
+__device__ __forceinline__ void cell_load(const char *rows, int64_t row_bytes, uint32_t lane_off, uint2 xr[16]) {
 #pragma unroll
-    for (int k = 0; k < 16; k++) xr[k] = *reinterpret_cast<const uint2 *>(xc + (size_t)k * kHeadDim);
+    for (int k = 0; k < 16; k++) xr[k] = *reinterpret_cast<const uint2 *>(rows + k * row_bytes + lane_off);
+}
+
+// The same where the lanes of a wavefront do not share a base (several groups to a workgroup).
+__device__ __forceinline__ void cell_load_lanes(const uint16_t *xc, int64_t st, uint2 xr[16]) {
+#pragma unroll
+    for (int k = 0; k < 16; k++) xr[k] = *reinterpret_cast<const uint2 *>(xc + k * st);
 }
 
 // The same cell from permuted rows: row k is token rows[k] (uniform: the indices come from scalar loads) of the
@@ -836,9 +907,9 @@ __device__ __forceinline__ void cell_token_minmax_halves(const uint2 xr[16], flo
 // has one barrier), and the next round's cells are requested as soon as this round's are quantized -- into the same
 // registers -- so that they travel while the packs are formed and emitted.  For 5..8 heads (one group per
 // workgroup); PERM as in the round-major kernel.  Same stream, parameters and block_info as that kernel.
-template <int DT, bool WIDE, bool PERM, bool XCH = false>
+template <int DT, bool WIDE, bool PERM, bool XCH = false, bool STRIDED = false>
 __global__ void __launch_bounds__(256) k_quant_encode_cells_kernel(
-    const uint16_t *__restrict__ x, int B, int H, int T, float rel, uint16_t *__restrict__ scale,
+    const uint16_t *__restrict__ x, int B, int H, int T, const XRows xs, float rel, uint16_t *__restrict__ scale,
     uint16_t *__restrict__ zero, uint8_t *__restrict__ stream, uint64_t capacity, uint32_t *__restrict__ info,
     ScanState *st, int W, uint32_t ngroups, uint32_t bound, uint64_t base, int par_stride,
     const uint32_t *__restrict__ perm, int perm_block, const Stagger stagger, int nsg = 1, uint64_t *xw = nullptr) {
@@ -871,7 +942,12 @@ __global__ void __launch_bounds__(256) k_quant_encode_cells_kernel(
     uint8_t *blk = gbuf + (size_t)j * bound;
     uint32_t my_off = 8u;
     uint32_t cmax_all = 0;
-    const uint16_t *cells = x + (((size_t)b * H_all + hbase + jc) * T + tok0) * kHeadDim + 4 * t;
+    // (a wavefront holds two heads: rows of the ordinary stride hang off a per-lane pointer, others off the scalar base of
+    // the first head)
+    const int j0 = STRIDED ? min(2 * __builtin_amdgcn_readfirstlane(wave), H - 1) : jc;
+    const char *cells = reinterpret_cast<const char *>(x + b * xs.sb + (hbase + j0) * xs.sh + (int64_t)tok0 * (STRIDED ? xs.st : kHeadDim) + (STRIDED ? 0 : 4 * t));
+    const uint32_t cell_off = STRIDED ? ((uint32_t)(jc - j0) * (uint32_t)xs.sh + 4u * (uint32_t)t) * 2u : 0u;
+    const int64_t row_bytes = STRIDED ? 2 * xs.st : 2 * kHeadDim;
     // PERM: the rows of a round are tokens perm[...] of the repacking block that holds this context block
     const uint16_t *pseq = x + (((size_t)b * H) * T + (tok0 / (size_t)(PERM ? perm_block : 1)) * (size_t)(PERM ? perm_block : 1)) * kHeadDim;
     const uint32_t plane = (uint32_t)(((size_t)jc * T * kHeadDim + 4 * t) * 2);
@@ -881,13 +957,13 @@ __global__ void __launch_bounds__(256) k_quant_encode_cells_kernel(
     uint2 xr[16];
     if (AHEAD) {
         if (PERM) cell_load_rows(pseq, perm + tok0, (uint32_t)perm_block - 1u, plane, xr);
-        else cell_load(cells, xr);
+        else cell_load(cells, row_bytes, cell_off, xr);
     }
 #pragma unroll 1
     for (int r = 0; r < 4; r++) {
         if (!AHEAD) {
             if (PERM) cell_load_rows(pseq, perm + tok0 + 16 * r, (uint32_t)perm_block - 1u, plane, xr);
-            else cell_load(cells + (size_t)r * 16 * kHeadDim, xr);
+            else cell_load(cells + r * 16 * row_bytes, row_bytes, cell_off, xr);
         }
         __builtin_amdgcn_s_setprio(PKV_EPRIO_STAT);
         {
@@ -959,7 +1035,7 @@ __global__ void __launch_bounds__(256) k_quant_encode_cells_kernel(
         cell_quant<DT>(xr, my_par, c01, c23);
         if (AHEAD && r < 3) {                              // travels while the packs are formed
             if (PERM) cell_load_rows(pseq, perm + tok0 + 16 * (r + 1), (uint32_t)perm_block - 1u, plane, xr);
-            else cell_load(cells + (size_t)(r + 1) * 16 * kHeadDim, xr);
+            else cell_load(cells + (r + 1) * 16 * row_bytes, row_bytes, cell_off, xr);
         }
         typename PacksOf<WIDE>::type u;
         uint32_t cmax;
@@ -1021,7 +1097,7 @@ __global__ void __launch_bounds__(256) k_quant_encode_cells_kernel(
 // kernel above, which reads a round once.)  `ngroups` counts workgroups, `ngroups_all` groups.
 template <int DT, bool WIDE>
 __global__ void __launch_bounds__(256) k_quant_encode_rounds_kernel(
-    const uint16_t *__restrict__ x, int B, int H, int T, float rel, uint16_t *__restrict__ scale,
+    const uint16_t *__restrict__ x, int B, int H, int T, const XRows xs, float rel, uint16_t *__restrict__ scale,
     uint16_t *__restrict__ zero, uint8_t *__restrict__ stream, uint64_t capacity, uint32_t *__restrict__ info,
     ScanState *st, int W, uint32_t ngroups, uint32_t bound, uint64_t base, int par_stride, const Stagger stagger,
     int gpw, uint32_t ngroups_all) {
@@ -1061,13 +1137,13 @@ __global__ void __launch_bounds__(256) k_quant_encode_rounds_kernel(
                 const uint32_t gq = grp_first + (uint32_t)q;
                 const uint32_t cq = gq / (uint32_t)B, bq = gq % (uint32_t)B;
                 const size_t tq = (size_t)bq * par_stride + (size_t)cq * 64 + 16 * r + tt;
-                round_token_params_few<DT>(x + (((size_t)bq * H) * T + (size_t)cq * 64 + 16 * r) * kHeadDim, (size_t)T * kHeadDim, H,
+                round_token_params_few<DT>(x + bq * xs.sb + (int64_t)(cq * 64u + 16u * r) * xs.st, xs, H,
                                            tt, l16, rel, scale + tq, zero + tq, s_par + 16 * q + tt);
             }
         }
         // the same rows again, as cells (issued before the barrier; they hit the lines just fetched)
         uint2 xr[16];
-        cell_load(x + (((size_t)b * H + jh) * T + tok0 + 16 * r) * kHeadDim + 4 * t, xr);
+        cell_load_lanes(x + b * xs.sb + jh * xs.sh + (int64_t)(tok0 + 16 * r) * xs.st + 4 * t, xs.st, xr);
         __syncthreads();
         __builtin_amdgcn_s_setprio(PKV_EPRIO_PACK);
         typename PacksOf<WIDE>::type u;
@@ -1186,7 +1262,7 @@ __device__ __forceinline__ uint32_t oct_incl_scan(uint32_t v, int m, uint32_t &t
 // `ngroups_total` groups.
 template <int DT, bool WIDE>
 __global__ void __launch_bounds__(512) v_quant_encode_rounds_kernel(
-    const uint16_t *__restrict__ x, int B, int H, int T, float rel, uint16_t *__restrict__ scale,
+    const uint16_t *__restrict__ x, int B, int H, int T, const XRows xs, float rel, uint16_t *__restrict__ scale,
     uint16_t *__restrict__ zero, uint8_t *__restrict__ stream, uint64_t capacity, uint32_t *__restrict__ info,
     ScanState *st, int W, uint32_t ngroups, uint32_t unit_slot, uint64_t base, int par_stride, const Stagger stagger,
     int gpw, uint32_t ngroups_total) {
@@ -1231,13 +1307,13 @@ __global__ void __launch_bounds__(512) v_quant_encode_rounds_kernel(
                 const uint32_t gq = grp_first + (uint32_t)q;
                 const uint32_t cq = gq / (uint32_t)B, bq = gq % (uint32_t)B;
                 const size_t tq = (size_t)bq * par_stride + (size_t)cq * 128 + 32 * it + tt;
-                round_token_params_few<DT>(x + (((size_t)bq * H) * T + (size_t)cq * 128 + 32 * it) * kHeadDim, (size_t)T * kHeadDim,
+                round_token_params_few<DT>(x + bq * xs.sb + (int64_t)(cq * 128u + 32u * it) * xs.st, xs,
                                            H, tt, l16, rel, scale + tq, zero + tq, s_par + 32 * q + tt);
             }
         }
         // the same rows again, as cells (issued before the barrier; they hit the lines just fetched)
         uint2 xr[16];
-        cell_load(x + (((size_t)b * H + jh) * T + tok0 + 32 * it + 16 * rp) * kHeadDim + 4 * t, xr);
+        cell_load_lanes(x + b * xs.sb + jh * xs.sh + (int64_t)(tok0 + 32 * it + 16 * rp) * xs.st + 4 * t, xs.st, xr);
         __syncthreads();
         __builtin_amdgcn_s_setprio(PKV_EPRIO_PACK);
         typename PacksOf<WIDE>::type u;
@@ -1336,9 +1412,9 @@ __global__ void __launch_bounds__(512) v_quant_encode_rounds_kernel(
 // PERM: the tokens in the order of a repacking, as in the round-major kernel; with scale_in / zero_in (the tokens'
 // parameters in the order of x, known from the pass that made the order) nothing is left to exchange and an
 // iteration has no barrier at all.
-template <int DT, bool WIDE, bool PERM, bool XCH = false>
+template <int DT, bool WIDE, bool PERM, bool XCH = false, bool STRIDED = false>
 __global__ void __launch_bounds__(512) v_quant_encode_cells_kernel(
-    const uint16_t *__restrict__ x, int B, int H, int T, float rel, uint16_t *__restrict__ scale,
+    const uint16_t *__restrict__ x, int B, int H, int T, const XRows xs, float rel, uint16_t *__restrict__ scale,
     uint16_t *__restrict__ zero, uint8_t *__restrict__ stream, uint64_t capacity, uint32_t *__restrict__ info,
     ScanState *st, int W, uint32_t ngroups, uint32_t unit_slot, uint64_t base, int par_stride,
     const uint32_t *__restrict__ perm, int perm_block, const uint16_t *__restrict__ scale_in,
@@ -1354,7 +1430,7 @@ __global__ void __launch_bounds__(512) v_quant_encode_cells_kernel(
     stagger_first_generation(stagger);
     if (tid == 0) s_idx = atomicAdd(&st->ticket, 1u);
     __syncthreads();
-    const uint32_t gidx = PERM ? (uint32_t)__builtin_amdgcn_readfirstlane((int)s_idx) : s_idx;
+    const uint32_t gidx = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_idx);
     if (gidx >= ngroups) return;
     // XCH (more than eight heads): runs of eight heads that exchange the minima and maxima of their heads per token,
     // as in the K kernel; a run's words are [iteration][token of the iteration]
@@ -1376,7 +1452,9 @@ __global__ void __launch_bounds__(512) v_quant_encode_cells_kernel(
         reinterpret_cast<uint32_t *>(gbuf + (size_t)(i / (meta / 4u)) * unit_slot)[i % (meta / 4u)] = 0u;
     uint32_t run_off = 0;
     uint32_t cmax_all = 0;
-    const uint16_t *cells = x + (((size_t)b * H_all + hbase + jc) * T + tok0 + 16 * rp) * kHeadDim + 4 * t;
+    const char *cells = reinterpret_cast<const char *>(x + b * xs.sb + (hbase + __builtin_amdgcn_readfirstlane(jc)) * xs.sh + (int64_t)tok0 * xs.st);
+    const uint32_t cell_off = (16u * (uint32_t)rp * (uint32_t)xs.st + 4u * (uint32_t)t) * 2u;
+    const int64_t row_bytes = STRIDED ? 2 * xs.st : 2 * kHeadDim;
     const uint32_t plane = (uint32_t)(((size_t)jc * T * kHeadDim + 4 * t) * 2);
     const bool known = PERM && scale_in != nullptr;              // uniform
     if (known) __syncthreads();                                  // the metadata zeros are in place before the first OR (no barrier below)
@@ -1387,7 +1465,7 @@ __global__ void __launch_bounds__(512) v_quant_encode_cells_kernel(
         // PERM: (the 32 tokens of an iteration lie in one repacking block: perm_block is a multiple of 64)
         const size_t rb = PERM ? ((tok0 + 32 * it) / (size_t)perm_block) * (size_t)perm_block : 0;
         if (PERM) cell_load_rows_lanes(x + (((size_t)b * H) * T + rb) * kHeadDim, perm + tok0 + 32 * it + 16 * rp, (uint32_t)perm_block - 1u, plane, xr);
-        else cell_load(cells + (size_t)it * 32 * kHeadDim, xr);
+        else cell_load(cells + it * 32 * row_bytes, row_bytes, cell_off, xr);
         __builtin_amdgcn_s_setprio(PKV_EPRIO_STAT);
         if (known) {
             if (lane < 32) {
@@ -1941,12 +2019,39 @@ static int check_xshape(const void *x, int dtype, int B, int H, int T) {
     return PKV_OK;
 }
 
+// One encode of the fused path: where its tokens are, where they go.
+struct EncodeJob {
+    const void *x;
+    XRows xs;
+    float rel;
+    int bits;
+    uint8_t *stream;
+    uint64_t capacity, base;
+    uint32_t *info;
+    void *scale, *zero;
+    int par_stride;
+    const uint32_t *perm = nullptr;
+    int perm_block = 0;
+    const void *scale_in = nullptr, *zero_in = nullptr;
+};
+
+// 64-bit words of look-back state the job takes: status words (one per ticket), then, with more than eight heads, the
+// words the runs of a group exchange: one per (run, token).
+static uint64_t state_words(bool is_k, int B, int H, int T) {
+    const uint64_t ctx_blk = is_k ? 64 : 128, groups = (uint64_t)T / ctx_blk * (uint64_t)B;
+    const uint64_t nsub = groups * (uint64_t)(((is_k ? H : 2 * H) + kSubBlocks - 1) / kSubBlocks);
+    return nsub + (H <= kSubBlocks ? 0 : groups * (uint64_t)((H + kSubBlocks - 1) / kSubBlocks) * ctx_blk);
+}
+
 template <bool IS_K>
-static int run_quant_encode(const void *x, int dtype, int B, int H, int T, float rel, int bits,
-                            uint8_t *stream, uint64_t capacity, uint64_t base, uint32_t *info, void *scale,
-                            void *zero, int par_stride, uint64_t *size_out, float *ms_out, hipStream_t s,
-                            const uint32_t *perm = nullptr, int perm_block = 0, const void *scale_in = nullptr,
-                            const void *zero_in = nullptr) {
+static int check_job(EncodeJob &job, int dtype, int B, int H, int T) {
+    const void *x = job.x, *scale = job.scale, *zero = job.zero;
+    const uint8_t *stream = job.stream;
+    const uint32_t *info = job.info, *perm = job.perm;
+    const int bits = job.bits, par_stride = job.par_stride, perm_block = job.perm_block;
+    const float rel = job.rel;
+    const uint64_t base = job.base;
+    uint64_t &capacity = job.capacity;
     int rc = check_xshape(x, dtype, B, H, T);
     if (rc) return rc;
     PKV_REQUIRE(stream && info && scale && zero, PKV_ERR_INVALID, "null pointer argument");
@@ -1972,23 +2077,53 @@ static int run_quant_encode(const void *x, int dtype, int B, int H, int T, float
     // that would grow past 4 GiB is reported as a full buffer instead of wrapping its offsets
     if (capacity > (1ull << 32)) capacity = 1ull << 32;
     PKV_REQUIRE(base <= capacity, PKV_ERR_CAPACITY, "stream offset beyond 4 GiB: block_info offsets are 32 bits");
-    ScanHandle sh;
+    // (the cells kernels reach the second head of a wavefront through a 32-bit byte offset)
+    PKV_REQUIRE((H <= 4 || job.xs.sh < (1ll << 31) - 128) && job.xs.st < (1 << 25), PKV_ERR_UNSUPPORTED,
+                "not supported: 4 GiB or more from one head to the next");
+    PKV_REQUIRE(state_words(IS_K, B, H, T) < (1ull << 31), PKV_ERR_UNSUPPORTED, "batch x tokens too large");
+    return PKV_OK;
+}
+
+// The cells kernel of a width, a type, a token order and a row stride.
+template <bool IS_K, bool WIDE, int DT>
+static auto cells_kernel_of(bool perm, bool xch, bool strided) {
+    if constexpr (IS_K)
+        return perm ? k_quant_encode_cells_kernel<DT, WIDE, true>
+                    : xch ? (strided ? k_quant_encode_cells_kernel<DT, WIDE, false, true, true> : k_quant_encode_cells_kernel<DT, WIDE, false, true>)
+                          : (strided ? k_quant_encode_cells_kernel<DT, WIDE, false, false, true> : k_quant_encode_cells_kernel<DT, WIDE, false>);
+    else
+        return perm ? v_quant_encode_cells_kernel<DT, WIDE, true>
+                    : xch ? (strided ? v_quant_encode_cells_kernel<DT, WIDE, false, true, true> : v_quant_encode_cells_kernel<DT, WIDE, false, true>)
+                          : (strided ? v_quant_encode_cells_kernel<DT, WIDE, false, false, true> : v_quant_encode_cells_kernel<DT, WIDE, false>);
+}
+template <bool IS_K>
+static auto cells_kernel(int bits, int dtype, bool perm, bool xch, bool strided) {
+    if (bits > 4) return dtype == PKV_F16 ? cells_kernel_of<IS_K, true, PKV_F16>(perm, xch, strided) : cells_kernel_of<IS_K, true, PKV_BF16>(perm, xch, strided);
+    return dtype == PKV_F16 ? cells_kernel_of<IS_K, false, PKV_F16>(perm, xch, strided) : cells_kernel_of<IS_K, false, PKV_BF16>(perm, xch, strided);
+}
+
+template <bool IS_K>
+static int launch_quant_encode(const EncodeJob &job, int dtype, int B, int H, int T, ScanState *st, hipStream_t s) {
+    const void *x = job.x;
+    const XRows xs = job.xs;
+    const float rel = job.rel;
+    const int bits = job.bits, par_stride = job.par_stride, perm_block = job.perm_block;
+    uint8_t *stream = job.stream;
+    const uint64_t capacity = job.capacity, base = job.base;
+    uint32_t *info = job.info;
+    void *scale = job.scale, *zero = job.zero;
+    const uint32_t *perm = job.perm;
+    const void *scale_in = job.scale_in, *zero_in = job.zero_in;
+    const int ctx_blk = IS_K ? 64 : 128, hid_blk = IS_K ? 128 : 64;
+    int rc;
     // One workgroup per run of up to eight heads of a (context block, sequence) group -- K: its up to eight blocks;
     // V: its up to sixteen -- or, with fewer than five heads, per 8 / H groups.
     {
         const int HB = IS_K ? H : 2 * H;
         const uint32_t bound = IS_K ? (uint32_t)k_block_bound(ctx_blk, bits) : (uint32_t)v_block_bound(hid_blk, bits);
         const uint32_t nsub = (uint32_t)(T / ctx_blk) * (uint32_t)B * (uint32_t)((HB + kSubBlocks - 1) / kSubBlocks);
-        // status words (one per ticket; nsub bounds the tickets of every kernel below), then, with more than eight
-        // heads, the words the runs of a group exchange: one per (run, token)
         const int nruns = (H + kSubBlocks - 1) / kSubBlocks;                // runs of eight heads per group
         const uint32_t nruns_all = (uint32_t)(T / ctx_blk) * (uint32_t)B * (uint32_t)nruns;
-        PKV_REQUIRE((uint64_t)nsub + (uint64_t)nruns_all * (uint64_t)ctx_blk < (1ull << 31), PKV_ERR_UNSUPPORTED, "batch x tokens too large");
-        const uint32_t xwords = H <= kSubBlocks ? 0u : nruns_all * (uint32_t)ctx_blk;
-        if ((rc = prepare_scan_state(nsub + xwords, &sh, s))) return rc;
-        ScanState *st = sh.st;
-        LaunchTimer tm(s, ms_out != nullptr);
-        if ((rc = tm.begin())) return rc;
         if (!IS_K && H <= 8) {               // one workgroup per group of 2 H blocks
             const uint32_t unit_slot = (uint32_t)(((bound - 8u) / 4u + 15u) & ~15u);
             const uint32_t lds = 64u * unit_slot + 64u;
@@ -2005,23 +2140,16 @@ static int run_quant_encode(const void *x, int dtype, int B, int H, int T, float
                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
             Stagger sg;
             if (gpw == 1) {                         // five to eight heads, or any token order: x read once, as cells
-                auto cells = perm ? (bits > 4 ? (dtype == PKV_F16 ? v_quant_encode_cells_kernel<PKV_F16, true, true>
-                                                                  : v_quant_encode_cells_kernel<PKV_BF16, true, true>)
-                                              : (dtype == PKV_F16 ? v_quant_encode_cells_kernel<PKV_F16, false, true>
-                                                                  : v_quant_encode_cells_kernel<PKV_BF16, false, true>))
-                                  : (bits > 4 ? (dtype == PKV_F16 ? v_quant_encode_cells_kernel<PKV_F16, true, false>
-                                                                  : v_quant_encode_cells_kernel<PKV_BF16, true, false>)
-                                              : (dtype == PKV_F16 ? v_quant_encode_cells_kernel<PKV_F16, false, false>
-                                                                  : v_quant_encode_cells_kernel<PKV_BF16, false, false>));
+                auto cells = cells_kernel<false>(bits, dtype, perm != nullptr, false, xs.st != kHeadDim);
                 PKV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(cells),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
                 if ((rc = stagger_for(reinterpret_cast<const void *>(cells), 512, lds, ngroups, &sg))) return rc;
-                cells<<<ngroups, 512, lds, s>>>((const uint16_t *)x, B, H, T, rel, (uint16_t *)scale, (uint16_t *)zero,
+                cells<<<ngroups, 512, lds, s>>>((const uint16_t *)x, B, H, T, xs, rel, (uint16_t *)scale, (uint16_t *)zero,
                                                 stream, capacity, info, st, bits, ngroups, unit_slot, base, par_stride, perm, perm_block,
                                                 (const uint16_t *)scale_in, (const uint16_t *)zero_in, sg, 1, nullptr);
             } else {
                 if ((rc = stagger_for(reinterpret_cast<const void *>(kern), 512, lds, ngroups, &sg))) return rc;
-                kern<<<ngroups, 512, lds, s>>>((const uint16_t *)x, B, H, T, rel, (uint16_t *)scale, (uint16_t *)zero,
+                kern<<<ngroups, 512, lds, s>>>((const uint16_t *)x, B, H, T, xs, rel, (uint16_t *)scale, (uint16_t *)zero,
                                                stream, capacity, info, st, bits, ngroups, unit_slot, base, par_stride, sg, gpw,
                                                ngroups_all);
             }
@@ -2039,54 +2167,60 @@ static int run_quant_encode(const void *x, int dtype, int B, int H, int T, float
                                                       : k_quant_encode_rounds_kernel<PKV_BF16, false>);
             Stagger sg;
             if (gpw == 1) {                         // five to eight heads: x read once, as cells
-                auto cells = perm ? (bits > 4 ? (dtype == PKV_F16 ? k_quant_encode_cells_kernel<PKV_F16, true, true>
-                                                                  : k_quant_encode_cells_kernel<PKV_BF16, true, true>)
-                                              : (dtype == PKV_F16 ? k_quant_encode_cells_kernel<PKV_F16, false, true>
-                                                                  : k_quant_encode_cells_kernel<PKV_BF16, false, true>))
-                                  : (bits > 4 ? (dtype == PKV_F16 ? k_quant_encode_cells_kernel<PKV_F16, true, false>
-                                                                  : k_quant_encode_cells_kernel<PKV_BF16, true, false>)
-                                              : (dtype == PKV_F16 ? k_quant_encode_cells_kernel<PKV_F16, false, false>
-                                                                  : k_quant_encode_cells_kernel<PKV_BF16, false, false>));
+                auto cells = cells_kernel<true>(bits, dtype, perm != nullptr, false, xs.st != kHeadDim);
                 if ((rc = stagger_for(reinterpret_cast<const void *>(cells), 256, lds, nwg, &sg))) return rc;
-                cells<<<nwg, 256, lds, s>>>((const uint16_t *)x, B, H, T, rel, (uint16_t *)scale, (uint16_t *)zero, stream,
+                cells<<<nwg, 256, lds, s>>>((const uint16_t *)x, B, H, T, xs, rel, (uint16_t *)scale, (uint16_t *)zero, stream,
                                             capacity, info, st, bits, nwg, slot, base, par_stride, perm, perm_block, sg, 1, nullptr);
             } else {
                 if ((rc = stagger_for(reinterpret_cast<const void *>(kern), 256, lds, nwg, &sg))) return rc;
-                kern<<<nwg, 256, lds, s>>>((const uint16_t *)x, B, H, T, rel, (uint16_t *)scale, (uint16_t *)zero, stream,
+                kern<<<nwg, 256, lds, s>>>((const uint16_t *)x, B, H, T, xs, rel, (uint16_t *)scale, (uint16_t *)zero, stream,
                                            capacity, info, st, bits, nwg, slot, base, par_stride, sg, gpw, nsub);
             }
         } else if (IS_K) {                           // more than eight heads: runs of eight, one workgroup each, that exchange their minima and maxima
             const uint32_t slot = (bound + 15u) & ~15u;
             const uint32_t lds = (uint32_t)kSubBlocks * slot + 32u;
             const int nsg = (H + kSubBlocks - 1) / kSubBlocks;
-            auto kern = bits > 4 ? (dtype == PKV_F16 ? k_quant_encode_cells_kernel<PKV_F16, true, false, true>
-                                                      : k_quant_encode_cells_kernel<PKV_BF16, true, false, true>)
-                                 : (dtype == PKV_F16 ? k_quant_encode_cells_kernel<PKV_F16, false, false, true>
-                                                      : k_quant_encode_cells_kernel<PKV_BF16, false, false, true>);
+            auto kern = cells_kernel<true>(bits, dtype, false, true, xs.st != kHeadDim);
             Stagger sg;
             if ((rc = stagger_for(reinterpret_cast<const void *>(kern), 256, lds, nsub, &sg))) return rc;
-            kern<<<nsub, 256, lds, s>>>((const uint16_t *)x, B, H, T, rel, (uint16_t *)scale, (uint16_t *)zero, stream,
+            kern<<<nsub, 256, lds, s>>>((const uint16_t *)x, B, H, T, xs, rel, (uint16_t *)scale, (uint16_t *)zero, stream,
                                         capacity, info, st, bits, nsub, slot, base, par_stride, nullptr, 0, sg, nsg,
                                         st->status + nsub);
         } else {                                     // V, more than eight heads: the same runs of eight
             const uint32_t unit_slot = (uint32_t)(((bound - 8u) / 4u + 15u) & ~15u);
             const uint32_t lds = 64u * unit_slot + 64u;
-            auto kern = bits > 4 ? (dtype == PKV_F16 ? v_quant_encode_cells_kernel<PKV_F16, true, false, true>
-                                                      : v_quant_encode_cells_kernel<PKV_BF16, true, false, true>)
-                                 : (dtype == PKV_F16 ? v_quant_encode_cells_kernel<PKV_F16, false, false, true>
-                                                      : v_quant_encode_cells_kernel<PKV_BF16, false, false, true>);
+            auto kern = cells_kernel<false>(bits, dtype, false, true, xs.st != kHeadDim);
             PKV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
             Stagger sg;
             if ((rc = stagger_for(reinterpret_cast<const void *>(kern), 512, lds, nruns_all, &sg))) return rc;
-            kern<<<nruns_all, 512, lds, s>>>((const uint16_t *)x, B, H, T, rel, (uint16_t *)scale, (uint16_t *)zero,
+            kern<<<nruns_all, 512, lds, s>>>((const uint16_t *)x, B, H, T, xs, rel, (uint16_t *)scale, (uint16_t *)zero,
                                              stream, capacity, info, st, bits, nruns_all, unit_slot, base, par_stride, nullptr, 0,
                                              nullptr, nullptr, sg, nruns, st->status + nruns_all);
         }
         PKV_HIP_CHECK(hipGetLastError());
-        if ((rc = tm.end(ms_out))) return rc;
-        return finish_encode(sh, size_out, bits, s);
     }
+    return PKV_OK;
+}
+
+static XRows dense_rows(int H, int T) { return XRows{(int64_t)H * T * kHeadDim, (int64_t)T * kHeadDim, kHeadDim}; }
+
+template <bool IS_K>
+static int run_quant_encode(const void *x, int dtype, int B, int H, int T, float rel, int bits,
+                            uint8_t *stream, uint64_t capacity, uint64_t base, uint32_t *info, void *scale,
+                            void *zero, int par_stride, uint64_t *size_out, float *ms_out, hipStream_t s,
+                            const uint32_t *perm = nullptr, int perm_block = 0, const void *scale_in = nullptr,
+                            const void *zero_in = nullptr) {
+    EncodeJob job{x, dense_rows(H, T), rel, bits, stream, capacity, base, info, scale, zero, par_stride, perm, perm_block, scale_in, zero_in};
+    int rc = check_job<IS_K>(job, dtype, B, H, T);
+    if (rc) return rc;
+    ScanHandle sh;
+    if ((rc = prepare_scan_state((uint32_t)state_words(IS_K, B, H, T), &sh, s))) return rc;
+    LaunchTimer tm(s, ms_out != nullptr);
+    if ((rc = tm.begin())) return rc;
+    if ((rc = launch_quant_encode<IS_K>(job, dtype, B, H, T, sh.st, s))) return rc;
+    if ((rc = tm.end(ms_out))) return rc;
+    return finish_encode(sh, size_out, bits, s);
 }
 
 }  // namespace pkv
@@ -2226,6 +2360,31 @@ int pkv_v_quant_encode_append(const void *x, int dtype, int B, int H, int T_new,
     return pkv::run_quant_encode<false>(x, dtype, B, H, T_new, rel, bits, stream, capacity, stream_used,
                                         block_info_tail, scale_tail, zero_tail, par_stride, size_out, ms_out,
                                         (hipStream_t)s);
+}
+
+int pkv_kv_quant_encode_append(const pkv_append_side *k, const pkv_append_side *v, int dtype, int B, int H, int T_new,
+                               int par_stride, uint64_t *k_size, uint64_t *v_size, pkv_stream_t s_) {
+    using namespace pkv;
+    hipStream_t s = (hipStream_t)s_;
+    PKV_REQUIRE(k && v && k_size && v_size, PKV_ERR_INVALID, "null pointer argument");
+    const pkv_append_side *sides[2] = {k, v};
+    EncodeJob job[2];
+    int rc;
+    for (int i = 0; i < 2; i++) {
+        const pkv_append_side &a = *sides[i];
+        PKV_REQUIRE(a.stride_b >= 0 && a.stride_h >= 0 && a.stride_t >= 0 && a.stride_t < (1 << 25) &&
+                        (a.stride_b | a.stride_h | a.stride_t) % 8 == 0 && (reinterpret_cast<uintptr_t>(a.x) & 15u) == 0,
+                    PKV_ERR_INVALID, "rows must start on 16-byte boundaries (row stride below 2^25 elements)");
+        job[i] = EncodeJob{a.x, XRows{a.stride_b, a.stride_h, a.stride_t}, a.rel, a.bits, a.stream, a.capacity, a.used, a.info_tail,
+                           a.scale_tail, a.zero_tail, par_stride};
+        rc = i == 0 ? check_job<true>(job[i], dtype, B, H, T_new) : check_job<false>(job[i], dtype, B, H, T_new);
+        if (rc) return rc;
+    }
+    ScanHandle sh;
+    if ((rc = prepare_scan_state((uint32_t)state_words(true, B, H, T_new), &sh, s, (uint32_t)state_words(false, B, H, T_new)))) return rc;
+    if ((rc = launch_quant_encode<true>(job[0], dtype, B, H, T_new, sh.st, s))) return rc;
+    if ((rc = launch_quant_encode<false>(job[1], dtype, B, H, T_new, sh.second, s))) return rc;
+    return finish_encode(sh, k_size, job[0].bits, s, v_size, job[1].bits);
 }
 
 }  // extern "C"

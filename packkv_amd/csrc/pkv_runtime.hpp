@@ -42,6 +42,11 @@ struct LaunchTimer {
 // medians in their original order (pkv_repack.hip).
 int launch_block_order(const uint8_t *median, int ctx_len, int block_size, uint32_t *perm, hipStream_t s);
 
+// Rows 0 .. n-1 of the windows k_out / v_out [B, H, out_rows, 128] = the dequantised codes of k / v [B, H, n, 128]
+// (pkv_quant.hip).
+int launch_quant_dequant(const void *k, const void *v, void *k_out, void *v_out, int dtype, int B, int H, int n, int out_rows, float k_rel,
+                         float v_rel, hipStream_t s);
+
 struct ScanState;
 struct Stagger;
 // The stagger of the first resident generation (stagger_first_generation, pkv_block.hpp) for `kernel` launched with

@@ -441,6 +441,90 @@ def window_append(k_new, v_new, cos, sin, k_win, v_win, win_pos):
     _lib.check(rc)
 
 
+def _rows16(t):
+    """Whether the rows of t [.., 128] can be read 16 bytes at a time where they are."""
+    return t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(st % 8 == 0 for st in t.stride()[:-1])
+
+
+def kv_quant_encode_append(k, v, n, k_side, v_side, tokens):
+    """quant_encode_append for the first n tokens (a multiple of 128) of k and of v [B, H, >= n, 128], with one wait for
+    both.  The rows are read where they are (any strides whose rows start on 16-byte boundaries).  k_side / v_side:
+    (rel, bits, stream, used, info, scale, zero) as quant_encode_append takes them.  Returns the bytes in use of K and V."""
+    B, H = k.size(0), k.size(1)
+    _require(n % 128 == 0 and tokens % 128 == 0, "token counts must be multiples of the block length")
+    sides, sizes = [], (ctypes.c_uint64(0), ctypes.c_uint64(0))
+    for x, (rel, bits, stream, used, info, scale, zero), per_tile, ctx_blk in ((k, k_side, B * H, 64), (v, v_side, 2 * B * H, 128)):
+        _require(x.is_cuda and x.dim() == 4 and x.size(0) == B and x.size(1) == H and x.size(2) >= n and x.size(3) == 128 and _rows16(x),
+                 "x must be a device tensor [B, H, n, 128] with rows on 16-byte boundaries")
+        _require(info.is_cuda and info.dtype == torch.uint32 and info.is_contiguous()
+                 and info.numel() >= 2 * ((tokens + n) // ctx_blk * per_tile), "block_info_buffer too small")
+        _require(scale.shape == zero.shape == k_side[5].shape and scale.dim() == 2 and scale.size(0) == B and scale.dtype == x.dtype
+                 and zero.dtype == x.dtype and scale.is_contiguous() and zero.is_contiguous() and scale.size(1) >= tokens + n,
+                 "scale / zero must be contiguous [B, row] with room for the new tokens")
+        _require(stream.is_cuda and stream.dtype == torch.uint8 and stream.is_contiguous() and 0 <= used <= stream.numel(),
+                 "compressed_buffer must be a contiguous device UInt8 tensor holding the bytes in use")
+        es = scale.element_size()
+        sides.append(_lib.AppendSide(x.data_ptr(), x.stride(0), x.stride(1), x.stride(2), stream.data_ptr(), stream.numel(), int(used),
+                                     info.data_ptr() + 8 * (tokens // ctx_blk * per_tile), scale.data_ptr() + es * tokens,
+                                     zero.data_ptr() + es * tokens, float(rel), int(bits)))
+    with torch.cuda.device(k.device):
+        rc = _lib.load().pkv_kv_quant_encode_append(ctypes.byref(sides[0]), ctypes.byref(sides[1]), _dtype_code(k), B, H, n,
+                                                    k_side[5].size(1), ctypes.byref(sizes[0]), ctypes.byref(sizes[1]), _stream(k.device))
+    _lib.check(rc)
+    return int(sizes[0].value), int(sizes[1].value)
+
+
+def window_cut(k_new, v_new, cos, sin, k_pend, v_pend, k_win, v_win, win_len, stage, pend_out, k_rel, v_rel):
+    """The write into the cache's window when its first tokens leave for the streams (utils/compute.py:54-67,
+    models/cache/packkv_quant.py:59-83).  Tokens in order: the pending cut's originals k_pend / v_pend [B, H, 64, 128] or
+    None, the window rows behind them up to win_len, the new tokens [B, H, n, 128] (keys with their rotary embedding when
+    cos / sin [B, n, 128] are given).  The first `stage` go to the encoder, `pend_out` (0 or 64) wait as the next pending
+    cut, the rest are the new window.  Returns (k_stage, v_stage, k_pend, v_pend, k_win, v_win): what the encoder reads
+    (the new tokens themselves where nothing has to be done to them), the new pending originals or None, the new windows."""
+    B, H, n, D = k_new.shape
+    _require(D == 128 and v_new.shape == k_new.shape and k_new.is_cuda and v_new.is_cuda and v_new.dtype == k_new.dtype,
+             "K and V must be device tensors [B, H, n, 128] of one dtype")
+    _require(k_win.is_contiguous() and v_win.is_contiguous() and k_win.shape == v_win.shape and k_win.dim() == 4
+             and k_win.size(0) == B and k_win.size(1) == H and k_win.size(3) == 128 and k_win.dtype == k_new.dtype,
+             "windows must be contiguous [B, H, cap, 128] of the tokens' dtype")
+    if k_new.stride() != v_new.stride() or not _rows16(k_new) or not _rows16(v_new):
+        k_new, v_new = k_new.contiguous(), v_new.contiguous()
+    pend = 64 if k_pend is not None else 0
+    buf = win_len - pend
+    a = _lib.CutArgs()
+    if cos is not None:
+        cos, sin = cos.expand(B, n, 128), sin.expand(B, n, 128)
+        _require(cos.dtype == k_new.dtype and sin.dtype == k_new.dtype, "cos / sin must be [B, n, 128] of the tokens' dtype")
+        if cos.stride(2) != 1 or (n > 1 and cos.stride(1) != 128) or cos.stride() != sin.stride() or not _rows16(cos) or not _rows16(sin):
+            cos, sin = cos.contiguous(), sin.contiguous()
+        a.cos, a.sin, a.rot_stride_b = cos.data_ptr(), sin.data_ptr(), cos.stride(0) if B > 1 else 0
+    empty = lambda rows: torch.empty(B, H, rows, 128, dtype=k_new.dtype, device=k_new.device)
+    k_stage, v_stage = k_new, v_new
+    if stage and (pend + buf or cos is not None):
+        k_stage = empty(stage)
+        a.k_stage = k_stage.data_ptr()
+    if stage and pend + buf:
+        v_stage = empty(stage)
+        a.v_stage = v_stage.data_ptr()
+    kp, vp = (empty(64), empty(64)) if pend_out else (None, None)
+    kw, vw = (torch.empty_like(k_win), torch.empty_like(v_win)) if win_len else (k_win, v_win)
+    a.k_new, a.v_new = k_new.data_ptr(), v_new.data_ptr()
+    a.stride_b, a.stride_h, a.stride_t = k_new.stride(0), k_new.stride(1), k_new.stride(2)
+    if pend:
+        a.k_pend, a.v_pend = k_pend.data_ptr(), v_pend.data_ptr()
+    if win_len:
+        a.k_win, a.v_win = k_win.data_ptr(), v_win.data_ptr()
+    if pend_out:
+        a.k_pend_out, a.v_pend_out = kp.data_ptr(), vp.data_ptr()
+    a.k_win_out, a.v_win_out, a.win_stride = kw.data_ptr(), vw.data_ptr(), k_win.size(2)
+    a.dtype, a.B, a.H, a.n, a.pend, a.buf, a.stage, a.pend_out = _dtype_code(k_new), B, H, n, pend, buf, stage, pend_out
+    a.k_rel, a.v_rel = float(k_rel), float(v_rel)
+    with torch.cuda.device(k_new.device):
+        rc = _lib.load().pkv_window_cut(ctypes.byref(a), _stream(k_new.device))
+    _lib.check(rc)
+    return k_stage, v_stage, kp, vp, kw, vw
+
+
 # ------------------------------------------------- repacking and analytic size ------
 
 def _check_code_matrix(c, name):

@@ -268,3 +268,57 @@ def test_dense_view_equals_the_restated_dequantisation(cuda, dtype, rel, T_c, T_
     got = ops.dense_view(sides[0], sides[1], kw.to(cuda), vw.to(cuda), T_w)
     for g, w in zip(got, want):
         assert g.shape == w.shape and torch.equal(g.cpu().view(torch.int16), w.view(torch.int16))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,H,T,rel", [(1, 1, 128, 0.1), (3, 3, 256, 0.1), (2, 4, 384, 0.05), (2, 8, 256, 0.1), (1, 8, 128, 0.05), (2, 12, 256, 0.1)])
+def test_append_reads_the_rows_where_they_are(cuda, dtype, B, H, T, rel):
+    """K and V as transposed projection outputs ([B, T, heads, 128] slices, heads beside them) appended in two pieces,
+    one wait for both sides: the streams, tables and parameters of one encode of the contiguous tensors."""
+    k, v = synth.make_kv(B, H, T, seed=31, dtype=dtype, device=cuda)
+    both = torch.stack((k, v), dim=2).permute(0, 3, 1, 2, 4).reshape(B, T, 2 * H, 128).contiguous()
+    kt, vt = both[:, :, 0::2].transpose(1, 2), both[:, :, 1::2].transpose(1, 2)
+    assert not kt.is_contiguous() and torch.equal(kt, k) and torch.equal(vt, v)
+    want = (ops.k_quant_encode(k, rel), ops.v_quant_encode(v, rel))
+    bits, row = want[0]["bits"], T + 128
+    sides = []
+    for w in want:
+        sides.append([rel, bits, torch.empty(w["stream"].numel() + 64, dtype=torch.uint8, device=cuda), 0,
+                      torch.empty(2 * w["info"].size(0), 2, dtype=torch.uint32, device=cuda),
+                      torch.empty(B, row, dtype=dtype, device=cuda), torch.empty(B, row, dtype=dtype, device=cuda)])
+    first = T // 2 // 128 * 128
+    for lo, n in ((0, first), (first, T - first)):
+        if n:
+            sides[0][3], sides[1][3] = ops.kv_quant_encode_append(kt[:, :, lo:], vt[:, :, lo:], n, sides[0], sides[1], lo)
+    for w, s in zip(want, sides):
+        assert s[3] == w["size"] and torch.equal(s[2][:s[3]], w["stream"][:w["size"]])
+        assert torch.equal(s[4][:w["info"].size(0)].view(torch.int32), w["info"].view(torch.int32))
+        assert torch.equal(s[5][:, :T], w["scale"]) and torch.equal(s[6][:, :T], w["zero"])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("pend,buf,n,rope", [(0, 0, 300, True), (0, 0, 1, False), (64, 150, 70, True), (64, 64, 257, False), (0, 191, 1, True)])
+def test_window_cut_moves_every_row(cuda, dtype, pend, buf, n, rope):
+    """The rows of a cut against the same chain of torch operations (rotary embedding, concatenation, slices): staged
+    tokens, the new pending originals and the window are copies or single 16-bit roundings, hence bit for bit; the
+    pending rows of the window are quant_params / quantize / dequantize of those originals."""
+    from packkv_amd.cache import apply_rotary_pos_emb_single
+    B, H, cap = 2, 3, 320
+    k, v = synth.make_kv(B, H, 64 + cap + n, seed=41, dtype=dtype, device=cuda)
+    kp, vp, kw, vw = k[:, :, :64].contiguous(), v[:, :, :64].contiguous(), k[:, :, 64:64 + cap].contiguous(), v[:, :, 64:64 + cap].contiguous()
+    kn, vn = k[:, :, 64 + cap:], v[:, :, 64 + cap:]
+    cos, sin = (t.to(cuda) for t in _rope_tables(B, 7, n, dtype)) if rope else (None, None)
+    kr = apply_rotary_pos_emb_single(kn, cos, sin) if rope else kn
+    ks = torch.cat(([kp] if pend else []) + [kw[:, :, pend:pend + buf], kr], dim=2)
+    vs = torch.cat(([vp] if pend else []) + [vw[:, :, pend:pend + buf], vn], dim=2)
+    stage, pend_out = max(0, ks.size(2) - 200) // 128 * 128, 64 if ks.size(2) >= 64 else 0
+    got = ops.window_cut(kn, vn, cos, sin, kp if pend else None, vp if pend else None, kw, vw, pend + buf, stage, pend_out, 0.1, 0.05)
+    for x, st, po, w, rel in ((ks, got[0], got[2], got[4], 0.1), (vs, got[1], got[3], got[5], 0.05)):
+        assert torch.equal(st[:, :, :stage], x[:, :, :stage])
+        if pend_out:
+            cut = x[:, :, stage:stage + 64].contiguous()
+            assert torch.equal(po, cut)
+            scale, zero = ops.quant_params(cut, rel)
+            want = ops.dequantize(ops.quantize(cut, scale, zero)[0], scale, zero, B, H)
+            assert torch.equal(w[:, :, :64], want)
+        assert torch.equal(w[:, :, pend_out:x.size(2) - stage], x[:, :, stage + pend_out:])
