@@ -58,8 +58,8 @@ struct AttnParams {
     int k_bits, v_bits, dtype;
     float sm_scale;
     int tiles_per_split, nsplit, nparts;
-    int win_piece;        // > 0: split i of the compressed part also takes window tokens [i * win_piece, ...) and
-                          // writes partial nsplit + i; 0: the window has a kernel of its own (partial nparts - 1)
+    int win_piece;        // window tokens per piece; piece i writes partial nsplit + i
+    int win_members;      // async-copy kernel: workgroups of their own per KV head for the pieces; 0: split i takes piece i
     uint32_t k_cap, v_cap, blk_stride;
     uint32_t k_bytes, v_bytes;   // valid bytes of the streams
     int out_f32;          // `out` holds fp32 instead of the 16-bit storage type
@@ -313,117 +313,179 @@ __device__ __forceinline__ float wave_sum(float x) {
     return s;
 }
 
-// ---- 16-bit tail window: dense attention over T_w tokens, one workgroup per (kv head, batch)
-// Attention of the G query heads of KV head (h, b) over tokens [t0, t1) of the uncompressed tail window, written
-// as partial `part_idx` (an empty range writes a partial of weight zero).  `lds` provides G * (128 + t1 - t0)
-// floats.  Called by all 256 threads of a workgroup.
-constexpr int kWinPieceLds = 36864;   // LDS every instance of the async-copy kernel has in its two slots
+// ---- 16-bit tail window ------------------------------------------------------------------------------------------
+// Attention of the query heads of KV head (h, b) over tokens [t0, t1) of the uncompressed tail window, written as
+// partial `part_idx` (an empty range writes a partial of weight zero).  `lds` provides min(G, 4) * 528 floats.  Called by
+// all 256 threads of a workgroup.
+// Latency is all there is to it (64 rows of K and V are 32 KB), so a workgroup makes one trip to memory per 64 tokens:
+// thread (tt = tid / 16, c = tid % 16) asks for 16 bytes of K and of V of tokens tt, tt + 16, tt + 32, tt + 48, and
+// everything until the end stays inside the wavefront -- scores by DPP sums over the 16 lanes of a row, a maximum, sums
+// and outputs of the wavefront's own -- so that one barrier, before the four wavefronts' results are combined, is the
+// only one.
+constexpr int kWinChunk = 64;         // tokens per trip
+constexpr int kWinLds = 528;          // floats of LDS per query head: four wavefronts' outputs, maxima and sums
+constexpr int kWinPieceLds = 4 * kWinLds * 4;   // LDS every instance of the async-copy kernel has in its two slots
 
-template <int G>
-__device__ __forceinline__ void window_body(const AttnParams &p, uint8_t *lds, int h, int b, int t0, int t1,
-                                            int part_idx) {
-    float *qf = reinterpret_cast<float *>(lds);   // [G][128]
-    float *S = qf + G * kHeadDim;                 // [G][Tw]
-    __shared__ float st_m[G], st_l[G];
-    const int tid = threadIdx.x;
-    const int Tw = t1 > t0 ? t1 - t0 : 0;
-    for (int i = tid; i < G * kHeadDim; i += 256)
-        qf[i] = i < p.Gq * kHeadDim ? a_ld16(p.q, ((size_t)b * p.Hq + (size_t)h * p.Gq) * kHeadDim + i, p.dtype) : 0.f;
-    __syncthreads();
-    const uint16_t *kbase = p.k_win + (((size_t)b * p.Hkv + h) * p.win_stride + t0) * kHeadDim;
-    const uint16_t *vbase = p.v_win + (((size_t)b * p.Hkv + h) * p.win_stride + t0) * kHeadDim;
-    {   // scores: 16 tokens per pass, 16 threads per token, each with 8 channels of the row
-        const int c = tid & 15;
-        float qr[G][8];
+template <bool BF>
+__device__ __forceinline__ void cvt_pair(uint32_t w, float &lo, float &hi) {
+    if (!BF) {
+        lo = __half2float(__ushort_as_half((unsigned short)(w & 0xFFFFu)));
+        hi = __half2float(__ushort_as_half((unsigned short)(w >> 16)));
+    } else {
+        lo = __uint_as_float(w << 16);
+        hi = __uint_as_float(w & 0xFFFF0000u);
+    }
+}
+template <bool BF>
+__device__ __forceinline__ void cvt8(const uint4 v, float f[8]) {
+    cvt_pair<BF>(v.x, f[0], f[1]); cvt_pair<BF>(v.y, f[2], f[3]); cvt_pair<BF>(v.z, f[4], f[5]); cvt_pair<BF>(v.w, f[6], f[7]);
+}
+// x of this lane and of the lane 32 (16) positions away: the halves (rows) of two registers change places
+__device__ __forceinline__ float add_swap32(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float((uint32_t)r[0]) + __uint_as_float((uint32_t)r[1]);
+}
+__device__ __forceinline__ float add_swap16(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float((uint32_t)r[0]) + __uint_as_float((uint32_t)r[1]);
+}
+
+// Heads gb .. gb + G - 1 of the group, G <= 4.
+template <int G, bool BF>
+__device__ __forceinline__ void window_heads(const AttnParams &p, uint8_t *lds, int h, int b, int gb, int t0, int t1,
+                                             int part_idx) {
+    float *red = reinterpret_cast<float *>(lds);             // [4 wavefronts][G][128], then maxima and sums [4][G] each
+    float *red_m = red + 4 * G * kHeadDim, *red_l = red_m + 4 * G;
+    const int tid = threadIdx.x, tt = tid >> 4, c = tid & 15, wave = tid >> 6, lane = tid & 63;
+    const size_t row0 = ((size_t)b * p.Hkv + h) * p.win_stride;
+    const uint4 *kbase = reinterpret_cast<const uint4 *>(p.k_win + row0 * kHeadDim) + c, *vbase = reinterpret_cast<const uint4 *>(p.v_win + row0 * kHeadDim) + c;
+    float q[G][8], acc[G][8], m[G], l[G];
 #pragma unroll
-        for (int g = 0; g < G; g++)
+    for (int g = 0; g < G; g++) {
+        uint4 w = make_uint4(0u, 0u, 0u, 0u);                // an idle head slot (group of 3 in the kernel of 4, ...)
+        if (gb + g < p.Gq) w = reinterpret_cast<const uint4 *>(p.q + ((size_t)b * p.Hq + (size_t)h * p.Gq + gb + g) * kHeadDim)[c];
+        cvt8<BF>(w, q[g]);
+        m[g] = -INFINITY; l[g] = 0.f;
 #pragma unroll
-            for (int j = 0; j < 8; j++) qr[g][j] = qf[g * kHeadDim + 8 * c + j];
-        for (int base = 0; base < Tw; base += 16) {
-            const int t = base + (tid >> 4);
-            float dot[G];
+        for (int j = 0; j < 8; j++) acc[g][j] = 0.f;
+    }
+    for (int base = t0; base < t1; base += kWinChunk) {
+        uint4 kr[4], vr[4];
 #pragma unroll
-            for (int g = 0; g < G; g++) dot[g] = 0.f;
-            if (t < Tw) {
-                const uint4 v = reinterpret_cast<const uint4 *>(kbase + (size_t)t * kHeadDim)[c];
-                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+        for (int i = 0; i < 4; i++) kr[i] = kbase[(size_t)min(base + 16 * i + tt, t1 - 1) * 16];      // (past the end: the last row again, weight zero)
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const float k0 = p.dtype == PKV_F16 ? __half2float(__ushort_as_half((unsigned short)(w[i] & 0xFFFFu)))
-                                                        : __uint_as_float(w[i] << 16);
-                    const float k1 = p.dtype == PKV_F16 ? __half2float(__ushort_as_half((unsigned short)(w[i] >> 16)))
-                                                        : __uint_as_float(w[i] & 0xFFFF0000u);
+        for (int i = 0; i < 4; i++) vr[i] = vbase[(size_t)min(base + 16 * i + tt, t1 - 1) * 16];
+        float s[G][4];
 #pragma unroll
-                    for (int g = 0; g < G; g++) dot[g] += qr[g][2 * i] * k0 + qr[g][2 * i + 1] * k1;
-                }
-            }
+        for (int i = 0; i < 4; i++) {
+            float k8[8];
+            cvt8<BF>(kr[i], k8);
+            const bool in = base + 16 * i + tt < t1;
 #pragma unroll
             for (int g = 0; g < G; g++) {
-                const float d = row16_sum(dot[g]);
-                if (c == 0 && t < Tw) S[g * Tw + t] = d * p.sm_scale;
+                float d = 0.f;
+#pragma unroll
+                for (int j = 0; j < 8; j++) d = fmaf(q[g][j], k8[j], d);
+                s[g][i] = in ? row16_sum(d) * p.sm_scale : -INFINITY;
             }
         }
-    }
-    __syncthreads();
-    for (int g = tid >> 6; g < G; g += 4) {
-        const int lane = tid & 63;
-        float mx = -INFINITY;
-        for (int t = lane; t < Tw; t += 64) mx = fmaxf(mx, S[g * Tw + t]);
 #pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 64));
-        float sum = 0.f;
-        for (int t = lane; t < Tw; t += 64) {
-            const float e = __expf(S[g * Tw + t] - mx);
-            S[g * Tw + t] = e;
-            sum += e;
-        }
+        for (int g = 0; g < G; g++) {
+            const float mx = fmaxf(m[g], wave_max(fmaxf(fmaxf(s[g][0], s[g][1]), fmaxf(s[g][2], s[g][3]))));
+            const float ref = mx == -INFINITY ? 0.f : mx;    // a wavefront without tokens: weights of zero, not NaN
+            const float alpha = __expf(m[g] - ref);
+            m[g] = mx;
+            l[g] *= alpha;
 #pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
-        if (lane == 0) { st_m[g] = mx; st_l[g] = sum; }
-    }
-    __syncthreads();
-    {   // weighted V sum: thread = (token parity, channel); the odd half hands its sums over through qf
-        const int half = tid >> 7, ch = tid & (kHeadDim - 1);
-        float acc[G];
+            for (int j = 0; j < 8; j++) acc[g][j] *= alpha;
 #pragma unroll
-        for (int g = 0; g < G; g++) acc[g] = 0.f;
-        int t = half;
-        for (; t + 6 < Tw; t += 8) {
-            float v[4];
-#pragma unroll
-            for (int u = 0; u < 4; u++) v[u] = a_ld16(vbase, (size_t)(t + 2 * u) * kHeadDim + ch, p.dtype);
-#pragma unroll
-            for (int u = 0; u < 4; u++)
-#pragma unroll
-                for (int g = 0; g < G; g++) acc[g] += S[g * Tw + t + 2 * u] * v[u];
-        }
-        for (; t < Tw; t += 2) {
-            const float v = a_ld16(vbase, (size_t)t * kHeadDim + ch, p.dtype);
-#pragma unroll
-            for (int g = 0; g < G; g++) acc[g] += S[g * Tw + t] * v;
-        }
-        if (half) {
-#pragma unroll
-            for (int g = 0; g < G; g++) qf[g * kHeadDim + ch] = acc[g];
-        }
-        __syncthreads();
-        if (!half) {
-#pragma unroll
-            for (int g = 0; g < G; g++) {
-                if (g >= p.Gq) break;
-                const size_t hq = (size_t)b * p.Hq + (size_t)h * p.Gq + g;
-                float *dst = p.part + (hq * p.nparts + part_idx) * kPartStride;
-                dst[2 + ch] = acc[g] + qf[g * kHeadDim + ch];
-                if (ch == 0) { dst[0] = st_m[g]; dst[1] = st_l[g]; }
+            for (int i = 0; i < 4; i++) {
+                s[g][i] = __expf(s[g][i] - ref);
+                l[g] += s[g][i];
             }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            float v8[8];
+            cvt8<BF>(vr[i], v8);
+#pragma unroll
+            for (int g = 0; g < G; g++)
+#pragma unroll
+                for (int j = 0; j < 8; j++) acc[g][j] = fmaf(s[g][i], v8[j], acc[g][j]);
+        }
+    }
+    // sums over the wavefront's four rows: while there are heads to share out, a step trades half of them with the lanes
+    // 32 (16) positions away, so that afterwards a row holds G / 4 heads (all of them when G is 1)
+    constexpr int G2 = G >= 2 ? G / 2 : 1, G4 = G >= 4 ? G / 4 : 1;
+#pragma unroll
+    for (int g = 0; g < G2; g++) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) acc[g][j] = add_swap32(acc[g][j], acc[G >= 2 ? g + G2 : g][j]);
+        l[g] = add_swap32(l[g], l[G >= 2 ? g + G2 : g]);
+    }
+#pragma unroll
+    for (int g = 0; g < G4; g++) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) acc[g][j] = add_swap16(acc[g][j], acc[G >= 4 ? g + G4 : g][j]);
+        l[g] = add_swap16(l[g], l[G >= 4 ? g + G4 : g]);
+    }
+    const int g0 = (G >= 2 ? (lane >> 5) * G2 : 0) + (G >= 4 ? ((lane >> 4) & 1) * G4 : 0);
+    if (G >= 4 || (lane & (G == 2 ? 16 : 48)) == 0) {
+#pragma unroll
+        for (int g = 0; g < G4; g++) {
+            float4v *dst = reinterpret_cast<float4v *>(red + (wave * G + g0 + g) * kHeadDim + 8 * c);
+            dst[0] = (float4v){acc[g][0], acc[g][1], acc[g][2], acc[g][3]};
+            dst[1] = (float4v){acc[g][4], acc[g][5], acc[g][6], acc[g][7]};
+            if (c == 0) red_l[wave * G + g0 + g] = l[g];
+        }
+    }
+    if (lane == 0) {
+#pragma unroll
+        for (int g = 0; g < G; g++) red_m[wave * G + g] = m[g];
+    }
+    __syncthreads();
+    for (int i = tid; i < min(G, p.Gq - gb) * kHeadDim; i += 256) {
+        const int g = i >> 7, ch = i & (kHeadDim - 1);
+        const float M = fmaxf(fmaxf(red_m[g], red_m[G + g]), fmaxf(red_m[2 * G + g], red_m[3 * G + g]));
+        const float ref = M == -INFINITY ? 0.f : M;
+        float num = 0.f, den = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            const float e = __expf(red_m[w * G + g] - ref);
+            num = fmaf(e, red[(w * G + g) * kHeadDim + ch], num);
+            den = fmaf(e, red_l[w * G + g], den);
+        }
+        const size_t hq = (size_t)b * p.Hq + (size_t)h * p.Gq + gb + g;
+        if (p.direct_out) {                                  // the only partial: the result itself
+            p.out[hq * kHeadDim + ch] = a_st16(num / den, p.dtype);
+            continue;
+        }
+        float *dst = p.part + (hq * p.nparts + part_idx) * kPartStride;
+        dst[2 + ch] = num;
+        if (ch == 0) { dst[0] = M; dst[1] = den; }
+    }
+}
+
+// (groups of eight heads in two halves: their queries and sums together need 170 registers)
+template <int G, bool BF>
+__device__ __forceinline__ void window_body(const AttnParams &p, uint8_t *lds, int h, int b, int t0, int t1, int part_idx) {
+    if constexpr (G <= 4) {
+        window_heads<G, BF>(p, lds, h, b, 0, t0, t1, part_idx);
+    } else {
+#pragma unroll 1
+        for (int gb = 0; gb < p.Gq; gb += 4) {
+            if (gb) __syncthreads();                         // the first half's results are read
+            window_heads<4, BF>(p, lds, h, b, gb, t0, t1, part_idx);
         }
     }
 }
 
-template <int G>
+// The window in pieces of its own: grid (Hkv, B, pieces), partial nsplit + piece.
+template <int G, bool BF>
 __global__ void __launch_bounds__(256) attn_window_kernel(const AttnParams p) {
-    extern __shared__ __align__(16) uint8_t lds[];
-    window_body<G>(p, lds, blockIdx.x, blockIdx.y, 0, p.T_w, p.nparts - 1);
+    __shared__ __attribute__((aligned(16))) uint8_t lds[kWinPieceLds];
+    const int t0 = (int)blockIdx.z * p.win_piece;
+    window_body<G, BF>(p, lds, blockIdx.x, blockIdx.y, t0, min(t0 + p.win_piece, p.T_w), p.nsplit + (int)blockIdx.z);
 }
 
 // ---- merge of the per-split partials: grid (Hq, B), 256 threads, nparts floats of dynamic LDS ----
@@ -516,7 +578,7 @@ namespace pkv {
 template <int G, int KW, int VW>
 static int launch_dma(const AttnParams &p, hipStream_t s) {
     static_assert(dma_lds_bytes<G, KW, VW>() >= kWinPieceLds, "window pieces borrow the slots");
-    const dim3 grid((unsigned)p.nsplit * (unsigned)p.Hkv * (unsigned)p.B);
+    const dim3 grid((unsigned)(p.nsplit + p.win_members) * (unsigned)p.Hkv * (unsigned)p.B);
     if (p.dtype == PKV_BF16)
         attn_dma_kernel<G, KW, VW, true><<<grid, 256, 0, s>>>(p);
     else
@@ -604,15 +666,14 @@ static int launch_attn(const AttnParams &p, int variant, bool aligned16, bool re
             attn_tiles_kernel<G, false><<<grid, 256, lds_bytes, s>>>(p);
         PKV_HIP_CHECK(hipGetLastError());
     }
-    if (p.T_w > 0 && p.win_piece == 0) {
-        const uint32_t lds_bytes = (uint32_t)sizeof(float) * (G * kHeadDim + G * p.T_w);
-        PKV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(attn_window_kernel<G>),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
-        attn_window_kernel<G><<<dim3((unsigned)p.Hkv, (unsigned)p.B), 256, lds_bytes, s>>>(p);
+    const bool dma_path = p.T_c > 0 && variant == 0 && aligned16;
+    if (p.T_w > 0 && !dma_path) {
+        const dim3 grid((unsigned)p.Hkv, (unsigned)p.B, (unsigned)((p.T_w + p.win_piece - 1) / p.win_piece));
+        if (p.dtype == PKV_BF16) attn_window_kernel<G, true><<<grid, 256, 0, s>>>(p);
+        else attn_window_kernel<G, false><<<grid, 256, 0, s>>>(p);
         PKV_HIP_CHECK(hipGetLastError());
     }
-    const bool dma_path = p.T_c > 0 && variant == 0 && aligned16;
-    if (!(dma_path && p.direct_out)) {       // a single partial is the result: the async-copy kernel wrote it out itself
+    if (!((dma_path || p.T_c == 0) && p.direct_out)) {       // a single partial is the result: its kernel wrote it out itself
         attn_merge_kernel<<<dim3((unsigned)p.Hq, (unsigned)p.B), 256, (size_t)p.nparts * sizeof(float), s>>>(
             p.part, out, p.Hq, p.nparts, p.dtype, p.out_f32);
         PKV_HIP_CHECK(hipGetLastError());
@@ -713,19 +774,32 @@ int pkv::attn_decode_impl(const pkv_attn_args *a, float *ms_out, hipStream_t s, 
     p.Gq = Gq;
     p.par_stride = par_stride; p.win_stride = win_stride;
     p.k_bits = a->k_bits; p.v_bits = a->v_bits; p.dtype = a->dtype; p.sm_scale = a->sm_scale;
-    const int n_tiles = a->T_c / kTile;
-    int nsplit = 0, tps = 0;
+    // the matrix-core kernels take the reference's widths and, in the asynchronous-copy kernel, the extension widths
+    // 5 and 6 (the other side then 4, 5 or 6); any other combination with an extension width runs the plain kernel
+    const bool narrow = a->T_c == 0 || (a->k_bits <= 4 && a->v_bits <= 4);
+    const bool wide_fast = !narrow && a->k_bits >= 4 && a->v_bits >= 4 && a->k_bits <= 6 && a->v_bits <= 6 && a->variant == 0;
+    const bool aligned16 = (narrow || wide_fast) &&
+                           ((reinterpret_cast<uintptr_t>(a->k_stream) | reinterpret_cast<uintptr_t>(a->v_stream)) & 15u) == 0;
+    const bool dma_path = a->T_c > 0 && a->variant == 0 && aligned16;
+    const int n_tiles = a->T_c / kTile, pairs = a->B * a->Hkv;
+    // The tail window goes in pieces of 64 tokens, one trip to memory each, to workgroups of their own -- in the
+    // async-copy kernel's launch while they are at most a quarter of the workgroups that are resident at once (the tiles
+    // keep the rest: 8 sequences x 4096 tokens), otherwise every split takes a share of the window behind its tiles (32
+    // sequences: 69 us, the share being 40 tokens of a 160-token window); other paths give it a kernel of its own, with longer
+    // pieces once there are more than four per CU (or more partials than the static array holds).
+    int nsplit = 0, tps = 0, win_members = (a->T_w + kWinChunk - 1) / kWinChunk;
     if (n_tiles > 0) {
         // Members per (sequence, KV head): about PKV_SPLIT_TARGET workgroups in all for the reference's widths -- four resident on each of 256
         // CUs.  When the heads do not divide that number, rounding the members up leaves a few workgroups over that
         // only start once others have finished, each with a full share of tiles (12 sequences x 8 heads: 11 members,
         // 1056 workgroups, 115 us per step against 99 us with 10 members); so both roundings are priced as
         // generations x tiles per member and the cheaper one is taken, the finer cut on a tie.
-        const int pairs = a->B * a->Hkv;
         // (as many members as are resident at once: widths 5 and 6 run two workgroups per CU -- 193 us per step with
         // 512 members against 199 us with 1024 in two generations, 6 bits 201 against 218 us -- and groups of eight
         // query heads three: 156 against 165 us)
-        const int target = PKV_SPLIT_TARGET / 4 * PKV_DMA_WAVES((a->k_bits > a->v_bits ? a->k_bits : a->v_bits), G);
+        const int resident = PKV_SPLIT_TARGET / 4 * PKV_DMA_WAVES((a->k_bits > a->v_bits ? a->k_bits : a->v_bits), G);
+        if (dma_path && 4 * (int64_t)pairs * win_members > resident) win_members = 0;
+        const int target = resident - (dma_path ? pairs * win_members : 0);
         long best_cost = -1;
         for (int up = 1; up >= 0; up--) {
             int want = up ? (target + pairs - 1) / pairs : target / pairs;
@@ -736,22 +810,17 @@ int pkv::attn_decode_impl(const pkv_attn_args *a, float *ms_out, hipStream_t s, 
             if (best_cost < 0 || cost < best_cost) { best_cost = cost; tps = t; nsplit = n; }
         }
     }
-    p.tiles_per_split = tps; p.nsplit = nsplit;
-    // The async-copy kernel spreads the tail window over its splits (each takes win_piece tokens after its
-    // tiles and writes one more partial), so the window costs no launch and no idle tail; other paths
-    // give the window a kernel of its own.
-    // the matrix-core kernels take the reference's widths and, in the asynchronous-copy kernel, the extension widths
-    // 5 and 6 (the other side then 4, 5 or 6); any other combination with an extension width runs the plain kernel
-    const bool narrow = a->T_c == 0 || (a->k_bits <= 4 && a->v_bits <= 4);
-    const bool wide_fast = !narrow && a->k_bits >= 4 && a->v_bits >= 4 && a->k_bits <= 6 && a->v_bits <= 6 && a->variant == 0;
-    const bool aligned16 = (narrow || wide_fast) &&
-                           ((reinterpret_cast<uintptr_t>(a->k_stream) | reinterpret_cast<uintptr_t>(a->v_stream)) & 15u) == 0;
-    p.win_piece = 0;
-    if (a->T_w > 0 && nsplit > 0 && a->variant == 0 && aligned16) {
-        const int piece = (a->T_w + nsplit - 1) / nsplit;
-        if ((size_t)G * (kHeadDim + piece) * sizeof(float) <= (size_t)kWinPieceLds) p.win_piece = piece;
+    const bool shared_window = dma_path && win_members == 0 && a->T_w > 0;      // every split writes a piece, empty or not
+    if (a->T_w > 0 && !dma_path) {
+        int64_t most = PKV_SPLIT_TARGET / pairs;
+        const int64_t room = (int64_t)(kStaticPartBytes / ((size_t)a->B * a->Hq * kPartStride * sizeof(float))) - nsplit;
+        if (room < most) most = room;
+        if (most < win_members) win_members = most < 1 ? 1 : (int)most;
     }
-    p.nparts = nsplit + (a->T_w > 0 ? (p.win_piece ? nsplit : 1) : 0);
+    p.tiles_per_split = tps; p.nsplit = nsplit;
+    p.win_piece = a->T_w > 0 ? (a->T_w + (shared_window ? nsplit : win_members) - 1) / (shared_window ? nsplit : win_members) : 0;
+    p.win_members = dma_path ? win_members : 0;
+    p.nparts = nsplit + (shared_window ? nsplit : a->T_w > 0 ? (a->T_w + p.win_piece - 1) / p.win_piece : 0);
     p.k_cap = a->T_c > 0 ? (uint32_t)k_block_bound(64, a->k_bits) : 0;
     p.v_cap = a->T_c > 0 ? (uint32_t)v_block_bound(64, a->v_bits) : 0;
     const uint32_t cap = p.k_cap > p.v_cap ? p.k_cap : p.v_cap;
@@ -762,7 +831,6 @@ int pkv::attn_decode_impl(const pkv_attn_args *a, float *ms_out, hipStream_t s, 
     p.direct_out = p.nparts == 1 && !p.out_f32;
     // The async-copy kernel balances the members of a head through two counters per head (with one member there is
     // nothing to balance).
-    const bool dma_path = a->T_c > 0 && a->variant == 0 && aligned16 && (narrow || wide_fast);
     // Tiles by counter pay when a member has many tiles (the first five are its own anyway): short launches -- a few
     // tiles per member, the small-batch decode steps -- only get the counters' atomic round trips on top (batch 1,
     // 32768 tokens: 46 us against 19 us with fixed shares).  And only up to eight members per head: every member asks

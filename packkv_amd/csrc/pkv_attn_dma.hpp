@@ -293,6 +293,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PKV_DM
     const int split = (int)blockIdx.x / n_heads, slot_ = (int)blockIdx.x % n_heads;
     const int bh_ = (n_heads & 7) == 0 ? (slot_ & 7) * (n_heads >> 3) + (slot_ >> 3) : slot_;
     const int h = bh_ % p.Hkv, b = bh_ / p.Hkv;
+    if (split >= p.nsplit) {                                                  // a piece of the window, nothing else
+        const int t0 = (split - p.nsplit) * p.win_piece;
+        window_body<G, BF>(p, smem, h, b, t0, min(t0 + p.win_piece, p.T_w), split);
+        return;
+    }
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     __builtin_assume(wave >= 0 && wave < 4);
@@ -924,9 +929,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PKV_DM
     }
     // this split's share of the 16-bit tail window, as a partial of its own (the slots are free: every
     // wave drained its copies before the barrier above)
-    if (p.win_piece > 0) {
+    if (p.win_piece > 0 && p.win_members == 0) {
         const int t0 = split * p.win_piece, t1 = min(t0 + p.win_piece, p.T_w);
-        window_body<G>(p, smem, h, b, t0, t1, p.nsplit + split);
+        window_body<G, BF>(p, smem, h, b, t0, t1, p.nsplit + split);
     }
 }
 

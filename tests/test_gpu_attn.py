@@ -494,3 +494,37 @@ def test_attn_decode_survives_damaged_block_info(cuda, variant):
     G = Hq // Hkv
     for h in (0, 3):
         assert torch.equal(got.float().cpu()[1, h * G:(h + 1) * G], good[1, h * G:(h + 1) * G])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,Hq,Hkv,T,Tw", [(1, 2, 2, 0, 1), (2, 8, 4, 0, 63), (2, 12, 4, 0, 64), (1, 8, 2, 0, 65), (1, 12, 2, 0, 130), (3, 8, 1, 0, 320),
+                                           (1, 6, 1, 128, 64), (2, 8, 2, 256, 129), (80, 8, 2, 128, 65), (40, 16, 4, 256, 191), (34, 32, 4, 128, 33)])
+def test_attn_decode_window_pieces(cuda, dtype, B, Hq, Hkv, T, Tw):
+    """The window at the edges of its 64-token pieces, for every group size (idle head slots included): alone, beside a
+    few tiles (workgroups of its own) and with so many heads that every split takes a share of it (80 x 2, 40 x 4 and
+    34 x 4 pairs).  Bound: 2e-5 for the fp32 arithmetic (attn_bounds) and, with tiles, what the matrix cores get: every
+    softmax weight and every per-pack sum of weights (it meets the pack minimum, at most the code) rounded to fp16,
+    2^-11 sum(w (|v| + v_scale code)), and a query split into digits of 2^-21 of its largest value, which
+    moves a score by at most E = 2^-21 max|q| k_scale sum(codes) / sqrt(128) (the zero point meets the exact sum of q) and
+    the result by 2 E sum(w |v|).  A 16-bit result adds half an ulp of its own."""
+    k, v = synth.make_kv(B, Hkv, T + Tw, seed=Tw, dtype=dtype)
+    q = synth.make_q(B, Hq, seed=3, dtype=dtype)
+    kc, kw, vc, vw = k[:, :, :T].contiguous(), k[:, :, T:].contiguous(), v[:, :, :T].contiguous(), v[:, :, T:].contiguous()
+    ke, ve = (ops.k_quant_encode(kc.to(cuda), 0.1), ops.v_quant_encode(vc.to(cuda), 0.1)) if T else (None, None)
+    kd, vd = kw.double(), vw.double()
+    if T:
+        (ck, zk, sk), (cv, zv, sv) = oq.quant_ints(kc, 64, 0.1), oq.quant_ints(vc, 64, 0.1)
+        kd = torch.cat([((ck.double() + zk.double()) * sk.double()).reshape(kc.shape), kd], dim=2)
+        vd = torch.cat([((cv.double() + zv.double()) * sv.double()).reshape(vc.shape), vd], dim=2)
+    exact = torch.as_tensor(oq.attention_f64_np(q.unsqueeze(2), kd, vd)).squeeze(2)
+    bound = torch.full_like(exact, 2e-5)
+    if T:
+        moved = 2.0 ** -21 * float(q.abs().max()) * float((ck.double() * sk.double()).reshape(kc.shape).sum(-1).max()) * 128 ** -0.5
+        codes = torch.cat([(cv.double() * sv.double()).reshape(vc.shape), torch.zeros_like(vw.double())], dim=2)
+        of = lambda x: torch.as_tensor(oq.attention_f64_np(q.unsqueeze(2), kd, x)).squeeze(2)
+        bound += 2.0 ** -11 * of(vd.abs() + codes) + 2 * moved * of(vd.abs())
+    half_ulp = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype] * exact.abs() * 1.05
+    got = ops.attn_decode(q.to(cuda), ke, ve, kw.to(cuda), vw.to(cuda), out_f32=True)
+    assert bool(((got.cpu().double() - exact).abs() <= bound).all())
+    got = ops.attn_decode(q.to(cuda), ke, ve, kw.to(cuda), vw.to(cuda))
+    assert bool(((got.cpu().double() - exact).abs() <= bound + half_ulp).all())
