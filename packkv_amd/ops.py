@@ -7,6 +7,7 @@ All tensors are caller-allocated and written in place, as in the reference.  PyT
 for device memory and the current stream only; every computation happens in
 libpackkv_hip.so.
 """
+import contextlib
 import ctypes
 import math
 
@@ -36,8 +37,20 @@ def _ptr(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
 
 
+_raw_stream = torch._C._cuda_getCurrentRawStream
+_current_device = torch._C._cuda_getDevice
+_here = contextlib.nullcontext()
+
+
+# Every op makes `dev` current and passes on its current stream.  A stream object and a device context that is entered
+# although the device is current take 3.5 us of host time a call -- a decode step is two calls and 13 us of GPU time --
+# these two take 0.5.
 def _stream(dev):
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    return _raw_stream(_current_device() if dev.index is None else dev.index)
+
+
+def _on(dev):
+    return _here if dev.type == "cuda" and dev.index in (None, _current_device()) else torch.cuda.device(dev)
 
 
 def _require(cond, msg):
@@ -109,7 +122,7 @@ def _encode(is_k, codes, stream, info, ctx_len, hidden_dim, ctx_blk, hid_blk, bi
     size = ctypes.c_uint64(0)
     ms = ctypes.c_float(0.0)
     fn = lib.pkv_k_encode if is_k else lib.pkv_v_encode
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = fn(_ptr(d_codes), _ptr(d_stream), d_stream.numel() * d_stream.element_size(), _ptr(d_info), ctx_len, hidden_dim,
                 ctx_blk, hid_blk, bits, ctypes.byref(size) if (want_size or on_host) else None,
                 ctypes.byref(ms) if timed else None, _stream(dev))
@@ -132,7 +145,7 @@ def _decode(is_k, stream, info, codes, ctx_len, hidden_dim, ctx_blk, hid_blk, bi
     d_codes = torch.empty_like(codes, device=dev) if on_host else codes
     ms = ctypes.c_float(0.0)
     fn = lib.pkv_k_decode if is_k else lib.pkv_v_decode
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = fn(_ptr(d_stream), d_stream.numel() * d_stream.element_size(), _ptr(d_info), _ptr(d_codes), ctx_len, hidden_dim, ctx_blk, hid_blk, bits,
                 ctypes.byref(ms) if timed else None, _stream(dev))
     _lib.check(rc)
@@ -146,7 +159,7 @@ def stream_release(stream=None):
     scratch buffers, tile counters and the buffers it has outgrown.  For callers that create and destroy streams:
     call it before the stream goes away, and only when no HIP graph captured on it will be replayed again."""
     st = torch.cuda.current_stream() if stream is None else stream
-    with torch.cuda.device(st.device):
+    with _on(st.device):
         rc = _lib.load().pkv_stream_release(ctypes.c_void_p(st.cuda_stream))
     _lib.check(rc)
 
@@ -156,7 +169,7 @@ def encode_status(device=None, bits=0):
     stream and raises what the encode would have raised (a stream that did not fit, a code wider than `bits`)."""
     dev = torch.device("cuda", torch.cuda.current_device()) if device is None else torch.device(device)
     size = ctypes.c_uint64(0)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _lib.load().pkv_encode_status(_stream(dev), int(bits), ctypes.byref(size))
     _lib.check(rc)
     return int(size.value)
@@ -251,7 +264,7 @@ def encode_p(is_k, codes, stream, info, pack_len, bits, want_size=True, timed=Fa
     dev = _device_of(codes, stream, info)
     size, ms = ctypes.c_uint64(0), ctypes.c_float(0.0)
     fn = _lib.load().pkv_k_encode_p if is_k else _lib.load().pkv_v_encode_p
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = fn(_ptr(codes), _ptr(stream), stream.numel(), _ptr(info), codes.size(0), codes.size(1), pack_len, bits,
                 ctypes.byref(size) if want_size else None, ctypes.byref(ms) if timed else None, _stream(dev))
     _lib.check(rc)
@@ -263,7 +276,7 @@ def decode_p(is_k, stream, info, codes, pack_len, bits, timed=False):
     dev = _device_of(codes, stream, info)
     ms = ctypes.c_float(0.0)
     fn = _lib.load().pkv_k_decode_p if is_k else _lib.load().pkv_v_decode_p
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = fn(_ptr(stream), stream.numel(), _ptr(info), _ptr(codes), codes.size(0), codes.size(1), pack_len, bits,
                 ctypes.byref(ms) if timed else None, _stream(dev))
     _lib.check(rc)
@@ -292,7 +305,7 @@ def quant_params(x, rel, timed=False):
     scale = torch.empty(B, T, dtype=x.dtype, device=x.device)
     zero = torch.empty(B, T, dtype=x.dtype, device=x.device)
     ms = ctypes.c_float(0.0)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = _lib.load().pkv_quant_params(_ptr(x), _dtype_code(x), B, H, T, float(rel), _ptr(scale),
                                           _ptr(zero), ctypes.byref(ms) if timed else None, _stream(x.device))
     _lib.check(rc)
@@ -305,7 +318,7 @@ def quantize(x, scale, zero):
     _check_params(scale, zero, B, T, x.dtype, x.device)
     codes = torch.empty(T, B * H * 128, dtype=torch.uint8, device=x.device)
     mx = torch.zeros(1, dtype=torch.int32, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = _lib.load().pkv_quantize(_ptr(x), _dtype_code(x), B, H, T, _ptr(scale), _ptr(zero), _ptr(codes),
                                       _ptr(mx), None, _stream(x.device))
     _lib.check(rc)
@@ -319,7 +332,7 @@ def dequantize(codes, scale, zero, B, H):
     T = codes.size(0)
     _check_params(scale, zero, B, T, scale.dtype, codes.device)
     x = torch.empty(B, H, T, 128, dtype=scale.dtype, device=codes.device)
-    with torch.cuda.device(codes.device):
+    with _on(codes.device):
         rc = _lib.load().pkv_dequantize(_ptr(codes), _dtype_code(scale), B, H, T, _ptr(scale), _ptr(zero),
                                         _ptr(x), None, _stream(codes.device))
     _lib.check(rc)
@@ -353,7 +366,7 @@ def _quant_encode(is_k, x, rel, bits, stream, info, want_size, timed, perm=None,
     zero = torch.empty(B, T, dtype=x.dtype, device=x.device)
     size = ctypes.c_uint64(0)
     ms = ctypes.c_float(0.0)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         tail = (_ptr(stream), stream.numel(), _ptr(info), _ptr(scale), _ptr(zero), ctypes.byref(size) if want_size else None,
                 ctypes.byref(ms) if timed else None, _stream(x.device))
         if perm is None:
@@ -404,7 +417,7 @@ def quant_encode_append(is_k, x, rel, bits, stream, used, info, tokens, scale, z
     es = scale.element_size()
     size = ctypes.c_uint64(0)
     fn = _lib.load().pkv_k_quant_encode_append if is_k else _lib.load().pkv_v_quant_encode_append
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = fn(_ptr(x), _dtype_code(x), B, H, n, float(rel), int(bits), _ptr(stream), stream.numel(), int(used),
                 ctypes.c_void_p(info.data_ptr() + 8 * nblk_done), ctypes.c_void_p(scale.data_ptr() + es * tokens),
                 ctypes.c_void_p(zero.data_ptr() + es * tokens), scale.size(1), ctypes.byref(size), None,
@@ -433,11 +446,12 @@ def window_append(k_new, v_new, cos, sin, k_win, v_win, win_pos):
         if cos.stride(2) != 1 or (n > 1 and cos.stride(1) != 128) or cos.stride() != sin.stride():
             cos, sin = cos.contiguous(), sin.contiguous()
         rot_sb = cos.stride(0) if B > 1 else 0
-    with torch.cuda.device(k_new.device):
-        rc = _lib.load().pkv_window_append(_ptr(k_new), _ptr(v_new), _ptr(cos) if cos is not None else None,
-                                           _ptr(sin) if cos is not None else None, _dtype_code(k_new), B, H, n,
-                                           k_new.stride(0), k_new.stride(1), k_new.stride(2), rot_sb, _ptr(k_win),
-                                           _ptr(v_win), int(win_pos), k_win.size(2), _stream(k_new.device))
+    sb, sh, st, _ = k_new.stride()
+    with _on(k_new.device):
+        rc = _lib.load().pkv_window_append(k_new.data_ptr(), v_new.data_ptr(), cos.data_ptr() if cos is not None else None,
+                                           sin.data_ptr() if cos is not None else None, _dtype_code(k_new), B, H, n, sb, sh, st,
+                                           rot_sb, k_win.data_ptr(), v_win.data_ptr(), int(win_pos), k_win.size(2),
+                                           _stream(k_new.device))
     _lib.check(rc)
 
 
@@ -467,7 +481,7 @@ def kv_quant_encode_append(k, v, n, k_side, v_side, tokens):
         sides.append(_lib.AppendSide(x.data_ptr(), x.stride(0), x.stride(1), x.stride(2), stream.data_ptr(), stream.numel(), int(used),
                                      info.data_ptr() + 8 * (tokens // ctx_blk * per_tile), scale.data_ptr() + es * tokens,
                                      zero.data_ptr() + es * tokens, float(rel), int(bits)))
-    with torch.cuda.device(k.device):
+    with _on(k.device):
         rc = _lib.load().pkv_kv_quant_encode_append(ctypes.byref(sides[0]), ctypes.byref(sides[1]), _dtype_code(k), B, H, n,
                                                     k_side[5].size(1), ctypes.byref(sizes[0]), ctypes.byref(sizes[1]), _stream(k.device))
     _lib.check(rc)
@@ -519,7 +533,7 @@ def window_cut(k_new, v_new, cos, sin, k_pend, v_pend, k_win, v_win, win_len, st
     a.k_win_out, a.v_win_out, a.win_stride = kw.data_ptr(), vw.data_ptr(), k_win.size(2)
     a.dtype, a.B, a.H, a.n, a.pend, a.buf, a.stage, a.pend_out = _dtype_code(k_new), B, H, n, pend, buf, stage, pend_out
     a.k_rel, a.v_rel = float(k_rel), float(v_rel)
-    with torch.cuda.device(k_new.device):
+    with _on(k_new.device):
         rc = _lib.load().pkv_window_cut(ctypes.byref(a), _stream(k_new.device))
     _lib.check(rc)
     return k_stage, v_stage, kp, vp, kw, vw
@@ -539,7 +553,7 @@ def code_stats(codes, pack_len, timed=False):
     _check_code_matrix(codes, "codes")
     ctx, hidden = codes.shape
     len_sum, n_unique, ms = ctypes.c_uint64(0), ctypes.c_uint32(0), ctypes.c_float(0.0)
-    with torch.cuda.device(codes.device):
+    with _on(codes.device):
         rc = _lib.load().pkv_bit_pack_size(_ptr(codes), ctx, hidden, int(pack_len), ctypes.byref(len_sum),
                                            ctypes.byref(n_unique), ctypes.byref(ms) if timed else None,
                                            _stream(codes.device))
@@ -578,7 +592,7 @@ def median_repacking(k_codes, v_codes, block_size=64, timed=False):
     k_out, v_out = torch.empty_like(k_codes), torch.empty_like(v_codes)
     perm = torch.empty(ctx, dtype=torch.int32, device=k_codes.device)
     ms = ctypes.c_float(0.0)
-    with torch.cuda.device(k_codes.device):
+    with _on(k_codes.device):
         rc = _lib.load().pkv_median_repack(_ptr(k_codes), _ptr(v_codes), _ptr(k_out), _ptr(v_out), _ptr(perm), ctx,
                                            hidden, int(block_size), ctypes.byref(ms) if timed else None,
                                            _stream(k_codes.device))
@@ -598,7 +612,7 @@ def greedy_repacking(k_codes, v_codes, pack_len=16, block_size=64, timed=False):
     k_out, v_out = torch.empty_like(k_codes), torch.empty_like(v_codes)
     perm = torch.empty(ctx, dtype=torch.int32, device=k_codes.device)
     ms = ctypes.c_float(0.0)
-    with torch.cuda.device(k_codes.device):
+    with _on(k_codes.device):
         rc = _lib.load().pkv_greedy_repack(_ptr(k_codes), _ptr(v_codes), _ptr(k_out), _ptr(v_out), _ptr(perm), ctx,
                                            hidden, int(block_size), int(pack_len), ctypes.byref(ms) if timed else None,
                                            _stream(k_codes.device))
@@ -614,7 +628,7 @@ def greedy_order(k_codes, v_codes, pack_len=16, block_size=64):
     _require(k_codes.shape == v_codes.shape, "K and V code matrices must have one shape")
     ctx, hidden = k_codes.shape
     perm = torch.empty(ctx, dtype=torch.int32, device=k_codes.device)
-    with torch.cuda.device(k_codes.device):
+    with _on(k_codes.device):
         rc = _lib.load().pkv_greedy_repack(_ptr(k_codes), _ptr(v_codes), None, None, _ptr(perm), ctx, hidden,
                                            int(block_size), int(pack_len), None, _stream(k_codes.device))
     _lib.check(rc)
@@ -644,7 +658,7 @@ def median_order(v, rel, bits=None, block_size=64, timed=False, want_params=Fals
     scale = torch.empty(B, T, dtype=v.dtype, device=v.device) if want_params else None
     zero = torch.empty(B, T, dtype=v.dtype, device=v.device) if want_params else None
     ms = ctypes.c_float(0.0)
-    with torch.cuda.device(v.device):
+    with _on(v.device):
         rc = _lib.load().pkv_median_order(_ptr(v), _dtype_code(v), B, H, T, float(rel), bits, int(block_size), _ptr(perm),
                                           _ptr(scale) if want_params else None, _ptr(zero) if want_params else None,
                                           ctypes.byref(ms) if timed else None, _stream(v.device))
@@ -742,7 +756,7 @@ def kq_mat_vec_mul(compressed_buffer, block_info_buffer, q, kq_out, ctx_len, hid
         print("Unsupported data type")
         return 0.0
     ms = ctypes.c_float(0.0)
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         rc = _lib.load().pkv_kq_mat_vec_mul(_ptr(compressed_buffer), compressed_buffer.numel() * compressed_buffer.element_size(), _ptr(block_info_buffer), _ptr(q),
                                             _ptr(kq_out), ctx_len, hidden_dim, ctx_len_block_size,
                                             hidden_dim_block_size, bits_len, _dtype_code(q),
@@ -765,7 +779,7 @@ def wv_mat_vec_mul(compressed_buffer, block_info_buffer, w, wv_out, ctx_len, hid
     if wv_out.dtype != torch.float32:
         raise RuntimeError("wv_out must be a float32 tensor")
     ms = ctypes.c_float(0.0)
-    with torch.cuda.device(w.device):
+    with _on(w.device):
         rc = _lib.load().pkv_wv_mat_vec_mul(_ptr(compressed_buffer), compressed_buffer.numel() * compressed_buffer.element_size(), _ptr(block_info_buffer), _ptr(w),
                                             _ptr(wv_out), ctx_len, hidden_dim, ctx_len_block_size,
                                             hidden_dim_block_size, bits_len, _dtype_code(w),
@@ -803,7 +817,7 @@ def fused_kq(our_kq, q, k_quant_zero, k_quant_scale, t):
     # contiguous copies of strided inputs must outlive the call: a temporary released between two .contiguous() calls
     # can be handed the same memory again
     q_c, z_c, s_c, t_c = q.contiguous(), k_quant_zero.contiguous(), k_quant_scale.contiguous(), t.contiguous()
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         rc = _lib.load().pkv_fused_kq(_ptr(our_kq), _ptr(q_c), _ptr(z_c), _ptr(s_c), _ptr(t_c), M, K, N,
                                       _dtype_code(q), ctypes.byref(ms), _stream(q.device))
     del q_c, z_c, s_c, t_c
@@ -835,7 +849,7 @@ def fused_wv(our_wv, w, v_quant_zero, v_quant_scale, term1):
     if not our_wv.is_contiguous(): raise RuntimeError("our_wv must be contiguous")
     ms = ctypes.c_float(0.0)
     w_c, z_c, s_c, t_c = w.contiguous(), v_quant_zero.contiguous(), v_quant_scale.contiguous(), term1.contiguous()
-    with torch.cuda.device(w.device):
+    with _on(w.device):
         rc = _lib.load().pkv_fused_wv(_ptr(our_wv), _ptr(w_c), _ptr(z_c), _ptr(s_c), _ptr(t_c), M, N, D,
                                       _dtype_code(w), ctypes.byref(ms), _stream(w.device))
     del w_c, z_c, s_c, t_c
@@ -875,7 +889,7 @@ def dense_view(k, v, k_win=None, v_win=None, win_len=None):
     a.B, a.Hkv, a.T_c, a.T_w, a.dtype = B, H, T_c, T_w, _dtype_code(like)
     k_out = torch.empty(B, H, T_c + T_w, 128, dtype=like.dtype, device=like.device)
     v_out = torch.empty_like(k_out)
-    with torch.cuda.device(like.device):
+    with _on(like.device):
         rc = _lib.load().pkv_dense_view(ctypes.byref(a), _ptr(k_out), _ptr(v_out), _stream(like.device))
     _lib.check(rc)
     return k_out, v_out
@@ -903,13 +917,14 @@ class AttnPlan:
             a.par_stride = k["scale"].size(1)
             for name, d in (("k", k), ("v", v)):
                 for f in ("stream", "info", "scale", "zero"):
-                    _require(d[f].is_cuda and d[f].is_contiguous(), "%s.%s must be a contiguous device tensor" % (name, f))
+                    if not (d[f].is_cuda and d[f].is_contiguous()):
+                        _require(False, "%s.%s must be a contiguous device tensor" % (name, f))
             nblk_k = k["info"].numel() // 2
             Hkv = int(k["heads"]) if "heads" in k else nblk_k // (T_c // 64) // B
             _require(nblk_k >= (T_c // 64) * B * Hkv and v["info"].numel() // 2 >= (T_c // 128) * B * Hkv * 2,
                      "block_info_buffer block num mismatch")
-            a.k_stream, a.k_info = _ptr(k["stream"]), _ptr(k["info"])
-            a.v_stream, a.v_info = _ptr(v["stream"]), _ptr(v["info"])
+            a.k_stream, a.k_info = k["stream"].data_ptr(), k["info"].data_ptr()
+            a.v_stream, a.v_info = v["stream"].data_ptr(), v["info"].data_ptr()
             # readable bytes of each buffer.  The default kernel copies whole dwords and needs no slack; the gather
             # kernel (variant 2, and variant 0 on streams that are not 16-byte aligned) fetches pack words as whole
             # 8-byte words and needs 7 readable bytes behind the encoded size: without them the plain kernel runs
@@ -917,8 +932,8 @@ class AttnPlan:
             if gathers and any(d.get("size") and d["stream"].numel() < int(d["size"]) + 7 for d in (k, v)):
                 variant = 1
             a.k_bytes, a.v_bytes = k["stream"].numel(), v["stream"].numel()
-            a.k_scale, a.k_zero = _ptr(k["scale"]), _ptr(k["zero"])
-            a.v_scale, a.v_zero = _ptr(v["scale"]), _ptr(v["zero"])
+            a.k_scale, a.k_zero = k["scale"].data_ptr(), k["zero"].data_ptr()
+            a.v_scale, a.v_zero = v["scale"].data_ptr(), v["zero"].data_ptr()
             a.k_bits, a.v_bits = int(k["bits"]), int(v["bits"])
         T_w = 0
         if k_win is not None:
@@ -931,7 +946,7 @@ class AttnPlan:
             a.win_stride = k_win.size(2)
             _require(Hkv is None or Hkv == k_win.size(1), "window head count mismatch")
             Hkv = k_win.size(1)
-            a.k_win, a.v_win = _ptr(k_win), _ptr(v_win)
+            a.k_win, a.v_win = k_win.data_ptr(), v_win.data_ptr()
         _require(Hkv is not None, "empty cache")
         out_dtype = torch.float32 if out_f32 else q.dtype
         if out is None:
@@ -939,7 +954,7 @@ class AttnPlan:
         _require(out.is_cuda and out.shape == q.shape and out.dtype == out_dtype and out.is_contiguous(),
                  "out must be a contiguous device tensor of q's shape (fp32 with out_f32, else q's dtype)")
         a.flags = (_lib.ATTN_REF_ROUNDING if ref_rounding else 0) | (_lib.ATTN_OUT_F32 if out_f32 else 0)
-        a.q, a.out = _ptr(q), _ptr(out)
+        a.q, a.out = q.data_ptr(), out.data_ptr()
         a.B, a.Hq, a.Hkv, a.T_c, a.T_w = B, Hq, Hkv, T_c, T_w
         a.dtype = _dtype_code(q)
         a.sm_scale = float(sm_scale if sm_scale is not None else 128 ** -0.5)
@@ -960,14 +975,14 @@ class AttnPlan:
         if q is not None:
             _require(q.is_cuda and q.shape == self._shape and q.dtype == self._dtype and q.is_contiguous(),
                      "q must match the plan's query tensor")
-            a.q = _ptr(q)
+            a.q = q.data_ptr()
         if out is not None:
             _require(out.is_cuda and out.shape == self._shape and out.dtype == self._out_dtype and out.is_contiguous(),
                      "out must match the plan's output tensor")
-            a.out = _ptr(out)
+            a.out = out.data_ptr()
             self.out = out
-        ms = ctypes.c_float(0.0)
-        with torch.cuda.device(self.device):
+        ms = ctypes.c_float(0.0) if timed else None
+        with _on(self.device):
             if self._fn_noalloc is not None:
                 _require(not timed, "the entry point that allocates nothing does not time its launch")
                 rc = self._fn_noalloc(self._ref, _stream(self.device))
