@@ -70,21 +70,21 @@ def crs_evaluation_with_data(config, key_caches, value_caches, device="cuda"):
     for k, v in zip(key_caches, value_caches):
         if k.shape != v.shape or k.dim() != 4 or k.size(2) % config.block_size:
             raise RuntimeError("K and V must be [B, H, T, D] of one shape with T a multiple of block_size")
-        codes, orig = {}, {}
+        codes, orig, before = {}, {}, {}
         for side, x, rel in (("k", k, config.k_quant_scale_rel), ("v", v, config.v_quant_scale_rel)):
             xd = x.to(device).contiguous()
-            scale, zero = ops.quant_params(xd, rel)
-            c, _ = ops.quantize(xd, scale, zero)
+            c, scale, zero = ops.quant_codes(xd, rel)
             codes[side] = c
             orig[side] = x.numel() * x.element_size()
             # every code at quant_bit_num bits plus one zero and one scale per (batch, token) in the storage dtype
-            n_unique = ops.code_stats(c, config.pack_size)[1]
+            len_sum, n_unique = ops.code_stats(c, config.pack_size)
+            before[side] = ops._packed_bytes(c, config.pack_size, len_sum, n_unique)
             quant_size = c.numel() * _bit_num(n_unique) // 8 + (zero.numel() + scale.numel()) * x.element_size()
             res[side + "_original_size"].append(orig[side])
             res[side + "_quant_size"].append(quant_size)
             res[side + "_quant_cr"].append(orig[side] / quant_size)
-        k_pre, v_pre, k_aft, v_aft = ops.repack_and_encode(codes["k"], codes["v"], config.pack_size,
-                                                           config.repack_method, config.block_size)
+        k_pre, v_pre, k_aft, v_aft = ops._repack_and_encode(codes["k"], codes["v"], config.pack_size, config.repack_method,
+                                                            config.block_size, (before["k"], before["v"]))
         for side, pre, aft in (("k", k_pre, k_aft), ("v", v_pre, v_aft)):
             res[side + "_encode_size_before_repack"].append(pre)
             res[side + "_encode_size_after_repack"].append(aft)
@@ -104,8 +104,7 @@ def crs_evaluation_detail(config, key_caches, value_caches, device="cuda"):
         codes, pars = {}, {}
         for side, x, rel in (("k", k, config.k_quant_scale_rel), ("v", v, config.v_quant_scale_rel)):
             xd = x.to(device).contiguous()
-            scale, zero = ops.quant_params(xd, rel)
-            codes[side], _ = ops.quantize(xd, scale, zero)
+            codes[side], scale, zero = ops.quant_codes(xd, rel)
             pars[side] = (zero.numel() * x.element_size(), scale.numel() * x.element_size())
             res[side + "_original_size"].append(x.numel() * x.element_size())
         kc, vc, _ = ops.median_repacking(codes["k"], codes["v"], config.block_size)

@@ -677,15 +677,12 @@ __global__ void __launch_bounds__(256) gather_rows_kernel(const uint8_t *__restr
 }
 
 // ---- analytic size: sum of bit_length(max - min) over packs, and which code values occur ----
-struct PackSizeOut {
-    unsigned long long len_sum;
-    uint32_t present[256];
+// State between the workgroups of a launch: words of the stream's look-back state, zero before and after it.
+struct PackSizeState {
+    unsigned long long sum;             // workgroups that are done << kPackSizeDone | sum of the pack widths so far
+    unsigned long long present[4];      // bit v: code v occurs
 };
-
-__global__ void pack_size_zero_kernel(PackSizeOut *out) {
-    if (threadIdx.x == 0) out->len_sum = 0ull;
-    out->present[threadIdx.x] = 0u;
-}
+constexpr int kPackSizeDone = 52;       // 2^11 workgroups at most; 2^52 bits are 2^49 bytes of codes at the very least
 
 // 256 threads per workgroup, a grid-stride walk over the items (pack, 16 adjacent channels), the channel chunk
 // running fastest so that a wavefront reads whole rows; four rows in flight per thread; minima and maxima as packed
@@ -693,10 +690,16 @@ __global__ void pack_size_zero_kernel(PackSizeOut *out) {
 // one after the other, so their number, not the bytes, would set the time of a grid with a workgroup per pack.
 // Bound by instruction issue: 7 vector instructions per dword for the ranges and 8 for the presence flags (a
 // register bit mask for values below 32 instead of the LDS flags costs the same).
+// The last workgroup to finish hands the result to the waiting host thread (a tagged slot in pinned memory) and leaves
+// the state clear: a launch to zero the result, a copy and a stream synchronisation around it, and a pair of events,
+// made a call 55 us around a kernel of 12 (16384 tokens x 8 heads of fp16 K and V, greedy record: 641 -> 388 us, with the sizes
+// before the repacking counted once).  Everything crosses workgroups by atomics that are complete before the workgroup's one
+// addition to `sum` (which also counts it done): no fence, no cached read of another workgroup's data.
 typedef unsigned short pk_u16x2 __attribute__((ext_vector_type(2)));
 
 __global__ void __launch_bounds__(256) pack_size_kernel(const uint8_t *__restrict__ codes, int hidden, int pack_len,
-                                                        size_t n_items, PackSizeOut *out) {
+                                                        size_t n_items, PackSizeState *st, unsigned long long *slot,
+                                                        uint32_t tag) {
     // a presence word per (code value, lane % 32): a lane marks its own column, so the marks of a wavefront never
     // share a bank however few values the matrix holds (one word per value made every mark a same-address conflict)
     __shared__ uint32_t seen[256 * 32];
@@ -752,12 +755,35 @@ __global__ void __launch_bounds__(256) pack_size_kernel(const uint8_t *__restric
     for (int d = 32; d >= 1; d >>= 1) lens += __shfl_xor(lens, d, 64);
     if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = lens;
     __syncthreads();
-    if (threadIdx.x == 0) atomicAdd(&out->len_sum, wsum[0] + wsum[1] + wsum[2] + wsum[3]);
     {   // value threadIdx.x: any of its 32 columns (read rotated, so that the threads of a wavefront spread over the banks)
         uint32_t any = 0u;
 #pragma unroll 8
         for (int c = 0; c < 32; c++) any |= seen[32 * threadIdx.x + ((c + threadIdx.x) & 31)];
-        if (any) out->present[threadIdx.x] = 1u;
+        const unsigned long long mine = __ballot(any != 0u);
+        if ((threadIdx.x & 63) == 0) {
+            // (most workgroups find what they saw already marked: a load in parallel instead of one more atomic in line)
+            unsigned long long *word = st->present + (threadIdx.x >> 6);
+            if (mine & ~__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                __hip_atomic_fetch_or(word, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");            // this wavefront's marks have reached memory
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const unsigned long long mine = (1ull << kPackSizeDone) + (wsum[0] + wsum[1] + wsum[2] + wsum[3]);
+        const unsigned long long all = __hip_atomic_fetch_add(&st->sum, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + mine;
+        if ((all >> kPackSizeDone) == gridDim.x) {
+            const unsigned long long total = all & ((1ull << kPackSizeDone) - 1ull), t = (unsigned long long)tag << 34;
+            uint32_t n = 0;
+            for (int i = 0; i < 4; i++) {
+                n += (uint32_t)__popcll(__hip_atomic_load(st->present + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                __hip_atomic_store(st->present + i, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            __hip_atomic_store(&st->sum, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(slot, (total & 0xFFFFFFFFull) | t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(slot + 1, (total >> 32) | t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(slot + 2, (unsigned long long)n | t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
     }
 }
 
@@ -774,25 +800,24 @@ int pkv_bit_pack_size(const uint8_t *codes, int ctx_len, int hidden_dim, int pac
     PKV_REQUIRE(hidden_dim % 16 == 0 && (reinterpret_cast<uintptr_t>(codes) & 15u) == 0, PKV_ERR_INVALID,
                 "hidden_dim must be a multiple of 16 and the code matrix 16-byte aligned");
     PKV_REQUIRE(ctx_len % pack_len == 0, PKV_ERR_INVALID, "ctx_len must be divisible by the pack length");
-    void *scratch = nullptr;
-    int rc = scratch_get(sizeof(PackSizeOut), s, &scratch);
-    if (rc) return rc;
-    PackSizeOut *out = static_cast<PackSizeOut *>(scratch);
+    int rc;
+    OutcomeSlot slot;
+    if ((rc = slot.take(s))) return rc;
+    ScanHandle sh;
+    if ((rc = prepare_scan_state((uint32_t)(sizeof(PackSizeState) / 8), &sh, s))) return rc;
     LaunchTimer tm(s, ms_out != nullptr);
     if ((rc = tm.begin())) return rc;
-    pack_size_zero_kernel<<<1, 256, 0, s>>>(out);
     const size_t n_items = (size_t)(ctx_len / pack_len) * (size_t)(hidden_dim / 16);
     const size_t wanted = (n_items + 255) / 256;
-    pack_size_kernel<<<(unsigned)(wanted < 2048 ? wanted : 2048), 256, 0, s>>>(codes, hidden_dim, pack_len, n_items, out);
+    pack_size_kernel<<<(unsigned)(wanted < 2048 ? wanted : 2048), 256, 0, s>>>(
+        codes, hidden_dim, pack_len, n_items, reinterpret_cast<PackSizeState *>(sh.st), (unsigned long long *)slot.words, slot.tag);
     PKV_HIP_CHECK(hipGetLastError());
+    if ((rc = scan_state_cleared(sh, s))) return rc;
     if ((rc = tm.end(ms_out))) return rc;
-    PackSizeOut h;
-    PKV_HIP_CHECK(hipMemcpyAsync(&h, out, sizeof(h), hipMemcpyDeviceToHost, s));
-    PKV_HIP_CHECK(hipStreamSynchronize(s));
-    uint32_t n = 0;
-    for (int i = 0; i < 256; i++) n += h.present[i];
-    *len_sum_out = h.len_sum;
-    *n_unique_out = n;
+    uint64_t v[3];
+    if ((rc = slot.wait(3, s, v))) return rc;
+    *len_sum_out = v[0] | v[1] << 32;
+    *n_unique_out = (uint32_t)v[2];
     return PKV_OK;
 }
 

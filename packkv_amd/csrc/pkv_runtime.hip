@@ -213,6 +213,54 @@ static int wait_words(const volatile uint64_t *w, int n, uint32_t tag, hipStream
     }
 }
 
+static int slot_take(uint64_t **slot, uint32_t *tag) {       // caller holds g_ws_mu; slot NULL: the tag alone
+    if (slot) {
+        if (g_free_slots.empty()) {
+            void *chunk = nullptr;
+            PKV_HIP_CHECK(hipHostMalloc(&chunk, (size_t)kSlotsPerChunk * kSlotWords * 8,
+                                        hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable));
+            g_chunks.push_back((uint64_t *)chunk);
+            for (int i = 0; i < kSlotsPerChunk; i++) g_free_slots.push_back((uint64_t *)chunk + (size_t)i * kSlotWords);
+        }
+        *slot = g_free_slots.back();
+        g_free_slots.pop_back();
+    }
+    g_seq = (g_seq + 1) & 0x3FFFFFFFu;
+    if (!g_seq) g_seq = 1;
+    *tag = g_seq;
+    return PKV_OK;
+}
+
+int OutcomeSlot::take(hipStream_t s) {
+    PKV_REQUIRE(!capturing(s), PKV_ERR_HIP, "the result is waited for: not possible while the stream is capturing a graph");
+    std::lock_guard<std::mutex> lock(g_ws_mu);
+    return slot_take(&words, &tag);
+}
+
+int OutcomeSlot::wait(int n, hipStream_t s, uint64_t *values) {
+    const int rc = wait_words(words, n, tag, s);
+    for (int i = 0; i < n && !rc; i++) values[i] = ((const volatile uint64_t *)words)[i] & ((1ull << 34) - 1ull);
+    return rc;
+}
+
+OutcomeSlot::~OutcomeSlot() {
+    if (!words) return;
+    std::lock_guard<std::mutex> lock(g_ws_mu);
+    g_free_slots.push_back(words);
+}
+
+int scan_state_cleared(ScanHandle &h, hipStream_t s) {
+    {
+        std::lock_guard<std::mutex> lock(g_ws_mu);
+        Workspace *w = nullptr;
+        int rc = workspace_for(s, &w);
+        if (rc) return rc;
+        w->enc_dirty = false;
+    }
+    h.held.unlock();
+    return PKV_OK;
+}
+
 int finish_encode(ScanHandle &h, uint64_t *size_out, int bits, hipStream_t s, uint64_t *size2_out, int bits2) {
     uint64_t *slot = nullptr;
     uint32_t tag = 0;
@@ -221,20 +269,7 @@ int finish_encode(ScanHandle &h, uint64_t *size_out, int bits, hipStream_t s, ui
         Workspace *w = nullptr;
         int rc = workspace_for(s, &w);
         if (rc) return rc;
-        g_seq = (g_seq + 1) & 0x3FFFFFFFu;
-        if (!g_seq) g_seq = 1;
-        tag = g_seq;
-        if (size_out) {
-            if (g_free_slots.empty()) {
-                void *chunk = nullptr;
-                PKV_HIP_CHECK(hipHostMalloc(&chunk, (size_t)kSlotsPerChunk * kSlotWords * 8,
-                                            hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable));
-                g_chunks.push_back((uint64_t *)chunk);
-                for (int i = 0; i < kSlotsPerChunk; i++) g_free_slots.push_back((uint64_t *)chunk + (size_t)i * kSlotWords);
-            }
-            slot = g_free_slots.back();
-            g_free_slots.pop_back();
-        }
+        if ((rc = slot_take(size_out ? &slot : nullptr, &tag))) return rc;
         const uint32_t n = (uint32_t)h.words64;
         finish_encode_kernel<<<(n + 1023u) / 1024u, 256, 0, s>>>(h.st, h.second, (uint64_t *)h.st, n, w->last, slot, tag);
         const hipError_t e = hipGetLastError();

@@ -74,6 +74,18 @@ int prepare_scan_state(uint32_t nblocks, ScanHandle *out, hipStream_t s, uint32_
 // (`size2_out`: of the second state).  `bits` > 0 additionally rejects a launch whose largest code does not fit.
 // NULL: returns at once, pkv_encode_status reads the outcome later.
 int finish_encode(ScanHandle &h, uint64_t *size_out, int bits, hipStream_t s, uint64_t *size2_out = nullptr, int bits2 = 0);
+// For a kernel whose last workgroup publishes the outcome and clears the state by itself: a pinned slot of eight words
+// that are valid one by one through their tag (value, 34 bits | tag << 34), and the two ends of its life.  Refused while
+// `s` is capturing (a graph's replays would write to a slot that has been given back).
+struct OutcomeSlot {
+    uint64_t *words = nullptr;
+    uint32_t tag = 0;
+    int take(hipStream_t s);
+    int wait(int n, hipStream_t s, uint64_t *values);      // the first `n` words, without their tags
+    ~OutcomeSlot();
+};
+// ... the launch that clears `h`'s state itself has been made.
+int scan_state_cleared(ScanHandle &h, hipStream_t s);
 // The block codec from a code matrix through the cells kernels (pkv_quant.hip): eight K / sixteen V blocks per group,
 // for hidden a multiple of 1024, the reference's block shapes, widths up to 6.  `st` holds one status word per group.
 int launch_code_cells(bool is_k, const uint8_t *codes, int ctx_len, int hidden, int bits, uint32_t bound, uint8_t *stream,

@@ -316,13 +316,24 @@ def quantize(x, scale, zero):
     """uint8 code matrix [T, B*H*128] (layout of evaluation/evaluation.py:406) and the largest code."""
     B, H, T = _check_x(x)
     _check_params(scale, zero, B, T, x.dtype, x.device)
-    codes = torch.empty(T, B * H * 128, dtype=torch.uint8, device=x.device)
     mx = torch.zeros(1, dtype=torch.int32, device=x.device)
+    codes = _quantize(x, scale, zero, B, H, T, mx)
+    return codes, int(mx.item())
+
+
+def _quantize(x, scale, zero, B, H, T, mx):
+    codes = torch.empty(T, B * H * 128, dtype=torch.uint8, device=x.device)
     with _on(x.device):
         rc = _lib.load().pkv_quantize(_ptr(x), _dtype_code(x), B, H, T, _ptr(scale), _ptr(zero), _ptr(codes),
                                       _ptr(mx), None, _stream(x.device))
     _lib.check(rc)
-    return codes, int(mx.item())
+    return codes
+
+
+def quant_codes(x, rel):
+    """(codes, scale, zero) of quant_params and quantize, without the largest code: nothing is waited for."""
+    scale, zero = quant_params(x, rel)
+    return _quantize(x, scale, zero, *_check_x(x), None), scale, zero
 
 
 def dequantize(codes, scale, zero, B, H):
@@ -566,12 +577,16 @@ def bit_pack_bytes(codes, pack_len, timed=False):
     """Analytic size of ONE code matrix [ctx_len, hidden] in bytes, as `bit_pack` prices each half
     (utils/compute.py:272-297): packs of `pack_len` consecutive tokens of one channel cost
     pack_len * bit_length(max - min) payload bits + W + ceil(log2(W + 1)) metadata bits, W = ceil(log2(#codes))."""
-    len_sum, n_unique, ms = code_stats(codes, pack_len, timed=True)
+    stats = code_stats(codes, pack_len, timed=timed)
+    size = _packed_bytes(codes, pack_len, *stats[:2])
+    return (size, stats[2]) if timed else size
+
+
+def _packed_bytes(codes, pack_len, len_sum, n_unique):
     ctx, hidden = codes.shape
     w = math.ceil(math.log2(n_unique))
     n_packs = (ctx // pack_len) * hidden
-    size = (len_sum * pack_len + n_packs * (w + math.ceil(math.log2(w + 1)))) // 8
-    return (size, ms) if timed else size
+    return (len_sum * pack_len + n_packs * (w + math.ceil(math.log2(w + 1)))) // 8
 
 
 def bit_pack(k_codes, v_codes, pack_len):
@@ -638,12 +653,19 @@ def greedy_order(k_codes, v_codes, pack_len=16, block_size=64):
 def repack_and_encode(k_codes, v_codes, pack_size, repack_method="none", block_size=64):
     """`repack_and_encode` (utils/compute.py:329-357) on code matrices: (k_size_pre, v_size_pre, k_size_aft,
     v_size_aft) in bytes.  repack_method: "none", "median" or "greedy"."""
-    k_pre, v_pre = bit_pack(k_codes, v_codes, pack_size)
+    return _repack_and_encode(k_codes, v_codes, pack_size, repack_method, block_size, bit_pack(k_codes, v_codes, pack_size))
+
+
+def _repack_and_encode(k_codes, v_codes, pack_size, repack_method, block_size, pre):
+    """repack_and_encode with the sizes before repacking at hand."""
+    k_pre, v_pre = pre
     if repack_method == "median":
         k_codes, v_codes, _ = median_repacking(k_codes, v_codes, block_size)
     elif repack_method == "greedy":
         k_codes, v_codes, _ = greedy_repacking(k_codes, v_codes, pack_size, block_size)
-    elif repack_method != "none":
+    elif repack_method == "none":
+        return k_pre, v_pre, k_pre, v_pre
+    else:
         raise ValueError("repack_method must be one of none, median, greedy")
     k_aft, v_aft = bit_pack(k_codes, v_codes, pack_size)
     return k_pre, v_pre, k_aft, v_aft

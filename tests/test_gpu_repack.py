@@ -52,6 +52,27 @@ def test_code_stats_shapes_against_closed_forms(cuda):
         assert ops.code_stats(torch.from_numpy(c).to(cuda), pack) == want
 
 
+@pytest.mark.parametrize("T,hid,pack,top", [(2, 16, 2, 255), (96, 48, 3, 63), (4200, 4096, 2, 64)])
+def test_code_stats_leave_their_state_clear_for_the_next_call(cuda, T, hid, pack, top):
+    """One workgroup, a part-filled one and more items than the largest grid has threads: the same answer from every call
+    in a row, on two streams in turn, whatever codes came before, and the sum of K and V in one bit_pack."""
+    g = torch.Generator().manual_seed(T)
+    mats = [torch.randint(0, hi + 1, (T, hid), generator=g, dtype=torch.uint8) for hi in (top, 1)]
+    want = []
+    for c in mats:
+        r = c.reshape(T // pack, pack, hid).int()
+        rng = (r.amax(1) - r.amin(1)).double()
+        want.append((int(torch.ceil(torch.log2(rng + 1)).sum()), int(c.unique().numel())))
+    dev = [c.to(cuda) for c in mats]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.current_stream(), torch.cuda.Stream()]
+    for i in range(8):
+        with torch.cuda.stream(streams[i % 2]):
+            _say("code_stats call", i, T, hid, pack)
+            assert ops.code_stats(dev[i // 2 % 2], pack) == want[i // 2 % 2]
+    assert ops.repack_and_encode(dev[0], dev[1], pack, "none") == ops.bit_pack(dev[0], dev[1], pack) * 2
+
+
 def test_median_repacking_matches_restatement(cuda):
     for (B, H, T, bs) in ((1, 2, 256, 64), (2, 8, 512, 64), (1, 1, 384, 128), (3, 2, 128, 16)):
         _say("repack case", B, H, T, bs)
