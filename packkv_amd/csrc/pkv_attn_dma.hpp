@@ -104,7 +104,11 @@ template <int KW, int VW>
 struct DmaGeom {
     static constexpr int kMaxBlock = k_block_bound(64, KW) > v_block_bound(64, VW) ? k_block_bound(64, KW) : v_block_bound(64, VW);
     // a block is copied from the 16-byte boundary below its start: up to 14 bytes of phase in front
-    static constexpr int kRegion = (kMaxBlock + 14 + 511) / 512 * 512;      // LDS bytes per block
+    // LDS bytes per block.  The copies up to 4 KiB are whole 1 KiB instructions without a lane test, and lanes past the
+    // block's end write zeroes: a region below 4 KiB is a multiple of 1 KiB, or a block that reaches into its last
+    // half would clear the start of the next one.  (At widths 2 and 3 the K tile is larger than the four regions anyway.)
+    static constexpr int kStep = kMaxBlock + 14 <= 4096 ? 1024 : 512;
+    static constexpr int kRegion = (kMaxBlock + 14 + kStep - 1) / kStep * kStep;
     static constexpr int kMaxInstr = (kRegion + 1023) / 1024;              // 64-lane copy instructions per block
     static constexpr int kKTile = 8 * 16 * 136;                            // the int8 K tile shares the block regions
     static constexpr int kParOff = 4 * kRegion > kKTile ? 4 * kRegion : kKTile;   // then 4 arrays x 128 tokens x 2 bytes

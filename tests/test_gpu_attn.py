@@ -528,3 +528,18 @@ def test_attn_decode_window_pieces(cuda, dtype, B, Hq, Hkv, T, Tw):
     assert bool(((got.cpu().double() - exact).abs() <= bound).all())
     got = ops.attn_decode(q.to(cuda), ke, ve, kw.to(cuda), vw.to(cuda))
     assert bool(((got.cpu().double() - exact).abs() <= bound + half_ulp).all())
+
+
+@pytest.mark.parametrize("rel,bits", [(0.2, 3), (0.34, 2)])
+@pytest.mark.parametrize("hq", [1, 2, 4, 8])
+def test_attn_decode_of_nearly_full_narrow_blocks(cuda, hq, rel, bits):
+    """V spread evenly over its range: every pack takes the whole width and the V blocks come close to their bound (over
+    3 KiB at 3 bits, 2 KiB at 2 bits)."""
+    for T in (128, 256, 1024, 2176):
+        k, _ = synth.make_kv(1, 1, T, seed=70 + T, dtype=torch.float16)
+        v = (2 * torch.rand(k.shape, generator=torch.Generator().manual_seed(T)) - 1).half()
+        q = synth.make_q(1, hq, seed=71, dtype=torch.float16)
+        ke, ve = ops.k_quant_encode(k.to(cuda), rel, bits=bits), ops.v_quant_encode(v.to(cuda), rel, bits=bits)
+        _say("narrow blocks: group", hq, "T", T, "bits", ke["bits"], ve["bits"], "largest V block", int(ve["info"].view(torch.int32)[:, 1].max()))
+        assert int(ve["info"].view(torch.int32)[:, 1].max()) > 1024 * bits
+        _parity(cuda, q, ke, ve, _reference(q, k, v, rel, rel), _exact(q, k, v, rel, rel), torch.float16, [0, 2], label="T=%d" % T)
