@@ -66,7 +66,9 @@ struct AttnParams {
     int direct_out;       // a single partial and a 16-bit result: the async-copy kernel writes `out` itself
     int dynamic;          // async-copy kernel: the members of a (sequence, KV head) take tiles from a common counter
     int batch_shift;      // ... in batches of (tiles left >> batch_shift), at least 1 and at most 4
-    uint32_t *counters;   // [B Hkv] tile counters, then [B Hkv] counts of members that are done; zero between launches
+    int merge;            // async-copy kernel: the last workgroup of a (sequence, KV head) to finish merges its partials
+    uint32_t *counters;   // [B Hkv] tile counters, [B Hkv] counts of members that are done with them, [B Hkv] workgroups that
+                          // have written their partials; zero between launches
 };
 
 // x rounded to the 16-bit storage type (nearest even), as fp32.
@@ -74,6 +76,10 @@ __device__ __forceinline__ float round16(float x, int dtype) {
     const uint32_t u = a_st16(x, dtype);
     return dtype == PKV_F16 ? __half2float(__ushort_as_half((unsigned short)u)) : __uint_as_float(u << 16);
 }
+
+// A partial is written through to memory: the workgroup that merges it may run on another XCD, behind another L2, in the
+// same launch (merge_head).
+__device__ __forceinline__ void part_store(float *p, float x) { __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
 // ---- variant 1: decode tiles into LDS, then plain VALU attention --------------------------
 // Straightforward and easy to audit; kept as the cross-check for the tuned kernel.
@@ -461,8 +467,8 @@ __device__ __forceinline__ void window_heads(const AttnParams &p, uint8_t *lds, 
             continue;
         }
         float *dst = p.part + (hq * p.nparts + part_idx) * kPartStride;
-        dst[2 + ch] = num;
-        if (ch == 0) { dst[0] = M; dst[1] = den; }
+        part_store(dst + 2 + ch, num);
+        if (ch == 0) { part_store(dst, M); part_store(dst + 1, den); }
     }
 }
 
@@ -486,6 +492,76 @@ __global__ void __launch_bounds__(256) attn_window_kernel(const AttnParams p) {
     __shared__ __attribute__((aligned(16))) uint8_t lds[kWinPieceLds];
     const int t0 = (int)blockIdx.z * p.win_piece;
     window_body<G, BF>(p, lds, blockIdx.x, blockIdx.y, t0, min(t0 + p.win_piece, p.T_w), p.nsplit + (int)blockIdx.z);
+}
+
+// ---- merge of a head's partials by the last of its `arrivals` workgroups to get here (async-copy kernel) ----
+// Saves the launch of the merge kernel, its run and the gap in front of it.  The price is three trips past the L2s -- a
+// workgroup's stores, its count, the last one's read of all partials -- and that the counts on one address retire one
+// after the other: a decode loop over 509 tokens (at most 6 workgroups a head) 1783 -> 1626 us, one over 32 x 8192
+// (4 workgroups) 4880 -> 4838, but one step of 32 heads x 4096 tokens (32 workgroups) 15.5 -> 16.5 us, one of
+// 3 x 8 heads x 11008 + 137 (24) 25.2 -> 27.2.  So: up to eight workgroups a head (kMergeArrivals).
+// Every workgroup has written its partials through to memory (part_store) and waited for that before it counts itself;
+// the reader's loads go past its own L2.  No workgroup waits for another.  Lane = two adjacent channels; a wavefront merges
+// a head of its own when the group has four or more, otherwise the wavefronts share a head's partials and meet in LDS.
+constexpr int kMergeArrivals = 8;
+template <int G>
+__device__ __forceinline__ void merge_head(const AttnParams &p, uint8_t *lds, int h, int b, uint32_t arrivals) {
+    constexpr int WPH = G >= 4 ? 1 : 4 / G;          // wavefronts per head
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    volatile uint32_t *last = reinterpret_cast<volatile uint32_t *>(lds);
+    float2v *sums = reinterpret_cast<float2v *>(lds + 16);        // [4 wavefronts][64 lanes]
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // this wavefront's partials have reached memory
+    __syncthreads();
+    if (tid == 0) {
+        uint32_t *count = p.counters + 2 * p.B * p.Hkv + b * p.Hkv + h;
+        const bool all = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == arrivals;
+        if (all) __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *last = all ? 1u : 0u;
+    }
+    __syncthreads();
+    if (*last == 0u) return;
+    const int sub = wave % WPH;
+    for (int g = wave / WPH; g < p.Gq; g += 4 / WPH) {
+        const size_t hq = (size_t)b * p.Hq + (size_t)h * p.Gq + g;
+        const float *base = p.part + hq * p.nparts * kPartStride;
+        // lane <-> partial (at most two per workgroup): maximum, weights, denominator
+        const uint64_t ml = __hip_atomic_load(reinterpret_cast<const uint64_t *>(base + (size_t)min(lane, p.nparts - 1) * kPartStride),
+                                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint64_t *col = reinterpret_cast<const uint64_t *>(base + 2) + lane;
+        constexpr int kRows = 2 * kMergeArrivals / WPH;
+        uint64_t v[kRows];
+#pragma unroll
+        for (int u = 0; u < kRows; u++)
+            v[u] = __hip_atomic_load(col + (size_t)min(sub + WPH * u, p.nparts - 1) * (kPartStride / 2), __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_AGENT);
+        const bool there = lane < p.nparts;
+        const float m = there ? __uint_as_float((uint32_t)ml) : -INFINITY, l = there ? __uint_as_float((uint32_t)(ml >> 32)) : 0.f;
+        const float w = __expf(m - wave_max(m));
+        const float den = wave_sum(w * l);
+        float2v num = {0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < kRows; u++) {
+            const int at = sub + WPH * u;
+            const float wu = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), at));
+            if (at < p.nparts) {
+                num[0] = fmaf(wu, __uint_as_float((uint32_t)v[u]), num[0]);
+                num[1] = fmaf(wu, __uint_as_float((uint32_t)(v[u] >> 32)), num[1]);
+            }
+        }
+        if constexpr (WPH > 1) {                     // (one pass of this loop: the group has G = 4 / WPH heads)
+            sums[tid] = num;
+            __syncthreads();
+            if (sub) return;
+#pragma unroll
+            for (int i = 1; i < WPH; i++) num += sums[tid + 64 * i];
+        }
+        if (p.out_f32) {
+            reinterpret_cast<float2v *>(reinterpret_cast<float *>(p.out) + hq * kHeadDim)[lane] = num / den;
+        } else {
+            const uint32_t lo = a_st16(num[0] / den, p.dtype), hi = a_st16(num[1] / den, p.dtype);
+            reinterpret_cast<uint32_t *>(p.out + hq * kHeadDim)[lane] = lo | (hi << 16);
+        }
+    }
 }
 
 // ---- merge of the per-split partials: grid (Hq, B), 256 threads, nparts floats of dynamic LDS ----
@@ -673,7 +749,8 @@ static int launch_attn(const AttnParams &p, int variant, bool aligned16, bool re
         else attn_window_kernel<G, false><<<grid, 256, 0, s>>>(p);
         PKV_HIP_CHECK(hipGetLastError());
     }
-    if (!((dma_path || p.T_c == 0) && p.direct_out)) {       // a single partial is the result: its kernel wrote it out itself
+    // (a single partial is the result, and the async-copy kernel merges short lists itself)
+    if (!((dma_path || p.T_c == 0) && p.direct_out) && !p.merge) {
         attn_merge_kernel<<<dim3((unsigned)p.Hq, (unsigned)p.B), 256, (size_t)p.nparts * sizeof(float), s>>>(
             p.part, out, p.Hq, p.nparts, p.dtype, p.out_f32);
         PKV_HIP_CHECK(hipGetLastError());
@@ -840,6 +917,8 @@ int pkv::attn_decode_impl(const pkv_attn_args *a, float *ms_out, hipStream_t s, 
     p.dynamic = PKV_DYNAMIC_TILES && dma_path && nsplit > 1 && nsplit <= 8 && tps >= 12 && 2 * a->B * a->Hkv <= kAttnCounters;
     p.batch_shift = 1;                     // a member asks for 1 / (2 nsplit) of what is left: ceil(log2(2 nsplit))
     while ((1 << p.batch_shift) < 2 * nsplit) p.batch_shift++;
+    // few workgroups a head: the last of them merges (merge_head)
+    p.merge = dma_path && p.nparts > 1 && nsplit + win_members <= kMergeArrivals && 3 * (int64_t)a->B * a->Hkv <= kAttnCounters;
     p.counters = nullptr;
     // Partials and counters: the stream's own scratch, or the static array -- for pkv_attn_decode_noalloc, and for a
     // stream that is capturing a graph before it has scratch of its own.
@@ -850,7 +929,10 @@ int pkv::attn_decode_impl(const pkv_attn_args *a, float *ms_out, hipStream_t s, 
     bool use_static = static_partials;
     if (!use_static) {
         rc = scratch_get(part_bytes, s, &part);
-        if (rc == PKV_OK && p.dynamic) rc = attn_counters_get(s, &p.counters);
+        if (rc == PKV_OK && (p.dynamic || p.merge)) {
+            rc = attn_counters_get(s, &p.counters);
+            if (rc == PKV_ERR_CAPTURING && !p.dynamic) { p.merge = 0; rc = PKV_OK; }     // a merge launch needs no counters
+        }
         if (rc == PKV_ERR_CAPTURING && part_bytes <= kStaticPartBytes) use_static = true;
         else if (rc) return rc == PKV_ERR_CAPTURING ? PKV_ERR_HIP : rc;
     }

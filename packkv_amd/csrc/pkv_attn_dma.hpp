@@ -300,6 +300,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PKV_DM
     if (split >= p.nsplit) {                                                  // a piece of the window, nothing else
         const int t0 = (split - p.nsplit) * p.win_piece;
         window_body<G, BF>(p, smem, h, b, t0, min(t0 + p.win_piece, p.T_w), split);
+        if (p.merge) merge_head<G>(p, smem, h, b, (uint32_t)(p.nsplit + p.win_members));
         return;
     }
     const int tid = threadIdx.x;
@@ -927,8 +928,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PKV_DM
                 continue;
             }
             float *dst = p.part + (hq * p.nparts + split) * kPartStride;
-            dst[2 + ch] = val;
-            if (ch == 0) { dst[0] = st_m[g]; dst[1] = st_l[g]; }
+            part_store(dst + 2 + ch, val);
+            if (ch == 0) { part_store(dst, st_m[g]); part_store(dst + 1, st_l[g]); }
         }
     }
     // this split's share of the 16-bit tail window, as a partial of its own (the slots are free: every
@@ -937,6 +938,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PKV_DM
         const int t0 = split * p.win_piece, t1 = min(t0 + p.win_piece, p.T_w);
         window_body<G, BF>(p, smem, h, b, t0, t1, p.nsplit + split);
     }
+    // (the merge reads the launch's parameters anew, through a pointer the compiler cannot see into: loaded with the others
+    // at the start of the kernel they held 17 more scalar registers through the loop than there are)
+    auto kernarg = __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(kernarg));
+    const AttnParams &late = *(const AttnParams *)kernarg;
+    if (late.merge) merge_head<G>(late, smem, h, b, (uint32_t)(late.nsplit + late.win_members));
 }
 
 }  // namespace pkv

@@ -318,7 +318,10 @@ int attn_counters_get(hipStream_t s, uint32_t **out) {
         }
         void *c = nullptr;
         PKV_HIP_CHECK(hipMalloc(&c, (size_t)kAttnCounters * sizeof(uint32_t)));
-        PKV_HIP_CHECK(hipMemset(c, 0, (size_t)kAttnCounters * sizeof(uint32_t)));
+        clear_state_kernel<<<kAttnCounters / 512, 256, 0, s>>>((uint64_t *)c, kAttnCounters / 2);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) (void)hipFree(c);
+        PKV_HIP_CHECK(e);
         w->counters = (uint32_t *)c;
     }
     *out = w->counters;

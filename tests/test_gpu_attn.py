@@ -543,3 +543,38 @@ def test_attn_decode_of_nearly_full_narrow_blocks(cuda, hq, rel, bits):
         _say("narrow blocks: group", hq, "T", T, "bits", ke["bits"], ve["bits"], "largest V block", int(ve["info"].view(torch.int32)[:, 1].max()))
         assert int(ve["info"].view(torch.int32)[:, 1].max()) > 1024 * bits
         _parity(cuda, q, ke, ve, _reference(q, k, v, rel, rel), _exact(q, k, v, rel, rel), torch.float16, [0, 2], label="T=%d" % T)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,Hq,Hkv,T,Tw,rel", [
+    (1, 2, 2, 256, 0, 0.1),            # one query head per KV head: four wavefronts share its partials
+    (1, 1, 1, 128 * 8, 0, 0.1),        # 8 workgroups a head: the most that are merged by the last of them
+    (1, 1, 1, 128 * 9, 0, 0.1),        # 9: a merge launch
+    (1, 1, 1, 128 * 7, 33, 0.1),       # 7 and one for the window
+    (2, 4, 2, 128 * 3, 300, 0.1),      # two per KV head, 3 and 5 for the window
+    (2, 12, 4, 128 * 6, 65, 0.1),      # three
+    (1, 8, 2, 128 * 5, 0, 0.1),        # four
+    (1, 8, 1, 128 * 6, 120, 0.2),      # eight
+    (1, 7, 1, 128 * 4, 200, 0.1),      # seven
+    (40, 8, 8, 128 * 6, 320, 0.1),     # the window shared by the splits: two partials a workgroup
+    (16, 32, 8, 128 * 8, 150, 0.1),    # ... 16 partials
+    (2, 8, 4, 128 * 5, 64, 0.05)])     # 5-bit codes
+def test_attn_decode_merged_by_its_last_workgroup(cuda, dtype, B, Hq, Hkv, T, Tw, rel):
+    """Partials merged inside the attention kernel, around its limits, against fp64 attention; again with fp32 output,
+    through the static scratch, and 20 times in a row: the counters are left clear and the result does not depend on which
+    workgroup comes last."""
+    _say("merge case", dtype, B, Hq, Hkv, T, Tw, rel)
+    k, v = synth.make_kv(B, Hkv, T + Tw, seed=70 + T, dtype=dtype)
+    q = synth.make_q(B, Hq, seed=71, dtype=dtype)
+    kc, vc = k[:, :, :T].contiguous(), v[:, :, :T].contiguous()
+    kw, vw = (k[:, :, T:].contiguous(), v[:, :, T:].contiguous()) if Tw else (None, None)
+    ke, ve = ops.k_quant_encode(kc.to(cuda), rel), ops.v_quant_encode(vc.to(cuda), rel)
+    win = (kw.to(cuda), vw.to(cuda)) if Tw else (None, None)
+    qd = q.to(cuda)
+    ref, exact = _reference(q, kc, vc, rel, rel, kw, vw), _exact(q, kc, vc, rel, rel, kw, vw)
+    got = ops.attn_decode(qd, ke, ve, *win)
+    check_fast(got, ref, exact, dtype, 0, label="merge")
+    for _ in range(20):
+        assert torch.equal(ops.attn_decode(qd, ke, ve, *win), got)
+    assert torch.equal(ops.attn_decode(qd, ke, ve, *win, noalloc=True), got)
+    assert torch.equal(ops.attn_decode(qd, ke, ve, *win, out_f32=True).to(dtype), got)
