@@ -159,7 +159,9 @@ int pkv_v_quant_encode_append(const void *x, int dtype, int B, int H, int T_new,
 /* pkv_kv_quant_encode_append: the two appends of a cut with one wait.  T_new (a multiple of 128) tokens of K and of V,
  * each read where it lies: element strides from one sequence, head and token to the next (multiples of 8, the rows on
  * 16-byte boundaries), so a cut needs no copy of the prompt it is taken from.  k_size / v_size receive the bytes in
- * use after the append; both encodes are launched before the call waits for either. */
+ * use after the append; both encodes are launched before the call waits for either.  With cos / sin (K only, five heads or
+ * more; [tokens, 128] of the data type, rot_stride_b elements from one sequence's table to the next, 0 for a shared one) the
+ * rows get the rotary embedding of row 0 .. T_new - 1 on the way, rounded as in pkv_window_append. */
 typedef struct pkv_append_side {
     const void *x;
     int64_t stride_b, stride_h, stride_t;
@@ -169,6 +171,8 @@ typedef struct pkv_append_side {
     void *scale_tail, *zero_tail;
     float rel;
     int bits;
+    const void *cos, *sin;
+    int64_t rot_stride_b;
 } pkv_append_side;
 int pkv_kv_quant_encode_append(const pkv_append_side *k, const pkv_append_side *v, int dtype, int B, int H, int T_new,
                                int par_stride, uint64_t *k_size, uint64_t *v_size, pkv_stream_t s);
@@ -191,7 +195,7 @@ int pkv_window_append(const void *k_new, const void *v_new, const void *cos, con
  * pend + buf - 1 of k_win / v_win, the n new tokens (strides and rotary embedding as in pkv_window_append, all strides
  * multiples of 8).  The first `stage` of them are written to k_stage / v_stage [B, H, stage, 128] for the encoder; a NULL
  * stage buffer leaves a side out, which is allowed where the encoder can read the new tokens as they are (nothing pending
- * or buffered; K: no rotary embedding).  The next pend_out (64 or 0) tokens are the new pending cut: originals to
+ * or buffered; K: no rotary embedding, or one that the encoder applies).  The next pend_out (64 or 0) tokens are the new pending cut: originals to
  * k_pend_out / v_pend_out, and rows 0 .. 63 of the new window receive them quantised at k_rel / v_rel and dequantised.
  * What remains fills the rows behind.  The new window k_win_out / v_win_out has the old one's shape and buffers of its
  * own.  All buffers 16-byte aligned. */

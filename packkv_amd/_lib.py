@@ -38,7 +38,8 @@ class AttnArgs(ctypes.Structure):
 
 class AppendSide(ctypes.Structure):
     _fields_ = [("x", _vp), ("stride_b", _i64), ("stride_h", _i64), ("stride_t", _i64), ("stream", _vp), ("capacity", _u64),
-                ("used", _u64), ("info_tail", _vp), ("scale_tail", _vp), ("zero_tail", _vp), ("rel", _f), ("bits", _i)]
+                ("used", _u64), ("info_tail", _vp), ("scale_tail", _vp), ("zero_tail", _vp), ("rel", _f), ("bits", _i),
+                ("cos", _vp), ("sin", _vp), ("rot_stride_b", _i64)]
 
 
 class CutArgs(ctypes.Structure):

@@ -175,9 +175,9 @@ int pkv_window_cut(const pkv_cut_args *a, pkv_stream_t s_) {
                 PKV_ERR_INVALID, "a pending cut needs buffers of its own and positive relative scales");
     PKV_REQUIRE(a->pend + a->buf == 0 || (a->k_win && a->v_win && a->k_win != a->k_win_out && a->v_win != a->v_win_out), PKV_ERR_INVALID,
                 "the new window is written into buffers of its own");
-    // what is encoded in place must be new tokens as they are
-    PKV_REQUIRE(a->stage == 0 || ((a->k_stage || (a->pend + a->buf == 0 && !a->cos)) && (a->v_stage || a->pend + a->buf == 0)), PKV_ERR_INVALID,
-                "staged tokens need a buffer unless they are new and have no rotary embedding");
+    // what is encoded in place must be new tokens (their rotary embedding is then the encoder's work)
+    PKV_REQUIRE(a->stage == 0 || ((a->k_stage && a->v_stage) || a->pend + a->buf == 0), PKV_ERR_INVALID,
+                "staged tokens need a buffer unless they are new");
     PKV_REQUIRE(a->stride_b >= 0 && a->stride_h >= 0 && a->stride_t >= 0 && a->rot_stride_b >= 0 &&
                     (a->stride_b | a->stride_h | a->stride_t | a->rot_stride_b) % 8 == 0, PKV_ERR_INVALID, "strides must be multiples of 8");
     const void *ptrs[] = {a->k_new, a->v_new, a->cos, a->sin, a->k_pend, a->v_pend, a->k_win, a->v_win, a->k_stage, a->v_stage,

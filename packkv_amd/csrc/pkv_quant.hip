@@ -449,6 +449,9 @@ __device__ __forceinline__ f16x2 pk_max_h(f16x2 a, f16x2 b) {
 // 16-byte boundary).  A cut of a prompt is encoded where it is, also as a transposed projection output.
 struct XRows { int64_t sb, sh, st; };
 
+// The rotary embedding of the rows, when the K encoder applies it: cos / sin [.., tokens, 128] by sequence (elements).
+struct Rot { const uint16_t *cos, *sin; int64_t sb; };
+
 // Token parameters of one round of the round-major encoders for a group of up to four heads (several of which share
 // a workgroup).  256 threads per 16 tokens: thread (tt = token, l16) reads 8 channels of every head; lane l16 == 0
 // writes the token's scale and zero and its constants for quant4.  `rows` is x at (sequence, head 0, the round's first
@@ -502,6 +505,48 @@ __device__ __forceinline__ void round_token_params_few(const uint16_t *rows, con
 __device__ __forceinline__ void cell_load(const char *rows, int64_t row_bytes, uint32_t lane_off, uint2 xr[16]) {
 #pragma unroll
     for (int k = 0; k < 16; k++) xr[k] = *reinterpret_cast<const uint2 *>(rows + k * row_bytes + lane_off);
+}
+
+// The rows of a cell with their rotary embedding, every product and the sum rounded to the storage type as the reference's
+// chain of elementwise ops does (utils/compute.py:35-43): channel d of the lower half becomes x[d] cos[d] - x[d + 64] sin[d],
+// of the upper half x[d] cos[d] + x[d - 64] sin[d].  A lane holds channels 4 t .. 4 t + 3, so the other factor of a pair is
+// in the same register of lane t ^ 16: one permlane16_swap and a select.  `cr` / `sr`: the first row's table entries,
+// uniform; eight rows of the tables at a time (they come from the caches: every head and sequence reads the same ones).
+template <int DT>
+__device__ __forceinline__ void cell_rotate(const char *cr, const char *sr, uint32_t lane_off, bool upper, uint2 xr[16]) {
+#pragma clang fp contract(off)
+    const uint32_t flip = upper ? 0u : 0x80008000u;
+#pragma unroll
+    for (int k0 = 0; k0 < 16; k0 += 8) {
+        uint2 c[8], s[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            c[k] = *reinterpret_cast<const uint2 *>(cr + (k0 + k) * (2 * kHeadDim) + lane_off);
+            s[k] = *reinterpret_cast<const uint2 *>(sr + (k0 + k) * (2 * kHeadDim) + lane_off);
+        }
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            uint32_t own[2] = {xr[k0 + k].x, xr[k0 + k].y}, cc[2] = {c[k].x, c[k].y}, ss[2] = {s[k].x, s[k].y};
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                const auto sw = __builtin_amdgcn_permlane16_swap(own[e], own[e], false, false);   // even rows' values, odd rows' values
+                const uint32_t other = (upper ? sw[0] : sw[1]) ^ flip;
+                if (DT == PKV_F16) {
+                    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+                    const h2 a = __builtin_bit_cast(h2, own[e]) * __builtin_bit_cast(h2, cc[e]);
+                    const h2 b = __builtin_bit_cast(h2, other) * __builtin_bit_cast(h2, ss[e]);
+                    own[e] = __builtin_bit_cast(uint32_t, (h2)(a + b));
+                } else {
+                    typedef float f2 __attribute__((ext_vector_type(2)));
+                    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+                    auto up = [](uint32_t v) -> f2 { return (f2){__uint_as_float(v << 16), __uint_as_float(v & 0xFFFF0000u)}; };
+                    auto rn = [](f2 v) -> uint32_t { return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, b2)); };
+                    own[e] = rn(up(rn(up(own[e]) * up(cc[e]))) + up(rn(up(other) * up(ss[e]))));
+                }
+            }
+            xr[k0 + k] = make_uint2(own[0], own[1]);
+        }
+    }
 }
 
 // The same where the lanes of a wavefront do not share a base (several groups to a workgroup).
@@ -907,12 +952,15 @@ __device__ __forceinline__ void cell_token_minmax_halves(const uint2 xr[16], flo
 // has one barrier), and the next round's cells are requested as soon as this round's are quantized -- into the same
 // registers -- so that they travel while the packs are formed and emitted.  For 5..8 heads (one group per
 // workgroup); PERM as in the round-major kernel.  Same stream, parameters and block_info as that kernel.
-template <int DT, bool WIDE, bool PERM, bool XCH = false, bool STRIDED = false>
+// ROT: the rows get their rotary embedding on the way (cell_rotate) -- a prompt's keys are then read once where they are,
+// instead of being rotated into a buffer of their own size first.  The arithmetic costs the encoder 90 us on 512 MiB of
+// bf16 (196 -> 287 us, bound by the vector units), the pass it saves took 190.
+template <int DT, bool WIDE, bool PERM, bool XCH = false, bool STRIDED = false, bool ROT = false>
 __global__ void __launch_bounds__(256) k_quant_encode_cells_kernel(
     const uint16_t *__restrict__ x, int B, int H, int T, const XRows xs, float rel, uint16_t *__restrict__ scale,
     uint16_t *__restrict__ zero, uint8_t *__restrict__ stream, uint64_t capacity, uint32_t *__restrict__ info,
     ScanState *st, int W, uint32_t ngroups, uint32_t bound, uint64_t base, int par_stride,
-    const uint32_t *__restrict__ perm, int perm_block, const Stagger stagger, int nsg = 1, uint64_t *xw = nullptr) {
+    const uint32_t *__restrict__ perm, int perm_block, const Stagger stagger, int nsg, uint64_t *xw, const Rot rot) {
     extern __shared__ __align__(16) uint8_t gbuf[];        // H block slots of `bound` bytes
     __shared__ uint32_t s_idx;
     __shared__ uint64_t s_off;
@@ -966,6 +1014,12 @@ __global__ void __launch_bounds__(256) k_quant_encode_cells_kernel(
             else cell_load(cells + r * 16 * row_bytes, row_bytes, cell_off, xr);
         }
         __builtin_amdgcn_s_setprio(PKV_EPRIO_STAT);
+        if (ROT) {
+            const int64_t row = (int64_t)b * rot.sb + (int64_t)(tok0 + 16 * (size_t)r) * kHeadDim;
+            uint32_t lt = (uint32_t)t;                     // (what follows from it is formed here, not kept through the loop: bf16 has 128
+            asm volatile("" : "+v"(lt));                   // registers in use)
+            cell_rotate<DT>(reinterpret_cast<const char *>(rot.cos + row), reinterpret_cast<const char *>(rot.sin + row), 8u * lt, lt >= 16u, xr);
+        }
         {
             float mn, mx;
             cell_token_minmax<DT>(xr, mn, mx);
@@ -2033,6 +2087,7 @@ struct EncodeJob {
     const uint32_t *perm = nullptr;
     int perm_block = 0;
     const void *scale_in = nullptr, *zero_in = nullptr;
+    Rot rot = {nullptr, nullptr, 0};       // K of five heads or more, in their own order
 };
 
 // 64-bit words of look-back state the job takes: status words (one per ticket), then, with more than eight heads, the
@@ -2084,22 +2139,24 @@ static int check_job(EncodeJob &job, int dtype, int B, int H, int T) {
     return PKV_OK;
 }
 
-// The cells kernel of a width, a type, a token order and a row stride.
+// The cells kernel of a width, a type, a token order, a row stride and (K) a rotary embedding.
 template <bool IS_K, bool WIDE, int DT>
-static auto cells_kernel_of(bool perm, bool xch, bool strided) {
+static auto cells_kernel_of(bool perm, bool xch, bool strided, bool rot) {
     if constexpr (IS_K)
         return perm ? k_quant_encode_cells_kernel<DT, WIDE, true>
-                    : xch ? (strided ? k_quant_encode_cells_kernel<DT, WIDE, false, true, true> : k_quant_encode_cells_kernel<DT, WIDE, false, true>)
-                          : (strided ? k_quant_encode_cells_kernel<DT, WIDE, false, false, true> : k_quant_encode_cells_kernel<DT, WIDE, false>);
+               : rot ? (xch ? k_quant_encode_cells_kernel<DT, WIDE, false, true, true, true> : k_quant_encode_cells_kernel<DT, WIDE, false, false, true, true>)
+               : xch ? (strided ? k_quant_encode_cells_kernel<DT, WIDE, false, true, true> : k_quant_encode_cells_kernel<DT, WIDE, false, true>)
+                     : (strided ? k_quant_encode_cells_kernel<DT, WIDE, false, false, true> : k_quant_encode_cells_kernel<DT, WIDE, false>);
     else
         return perm ? v_quant_encode_cells_kernel<DT, WIDE, true>
                     : xch ? (strided ? v_quant_encode_cells_kernel<DT, WIDE, false, true, true> : v_quant_encode_cells_kernel<DT, WIDE, false, true>)
                           : (strided ? v_quant_encode_cells_kernel<DT, WIDE, false, false, true> : v_quant_encode_cells_kernel<DT, WIDE, false>);
 }
 template <bool IS_K>
-static auto cells_kernel(int bits, int dtype, bool perm, bool xch, bool strided) {
-    if (bits > 4) return dtype == PKV_F16 ? cells_kernel_of<IS_K, true, PKV_F16>(perm, xch, strided) : cells_kernel_of<IS_K, true, PKV_BF16>(perm, xch, strided);
-    return dtype == PKV_F16 ? cells_kernel_of<IS_K, false, PKV_F16>(perm, xch, strided) : cells_kernel_of<IS_K, false, PKV_BF16>(perm, xch, strided);
+static auto cells_kernel(int bits, int dtype, bool perm, bool xch, bool strided, bool rot = false) {
+    if (bits > 4)
+        return dtype == PKV_F16 ? cells_kernel_of<IS_K, true, PKV_F16>(perm, xch, strided, rot) : cells_kernel_of<IS_K, true, PKV_BF16>(perm, xch, strided, rot);
+    return dtype == PKV_F16 ? cells_kernel_of<IS_K, false, PKV_F16>(perm, xch, strided, rot) : cells_kernel_of<IS_K, false, PKV_BF16>(perm, xch, strided, rot);
 }
 
 template <bool IS_K>
@@ -2167,10 +2224,10 @@ static int launch_quant_encode(const EncodeJob &job, int dtype, int B, int H, in
                                                       : k_quant_encode_rounds_kernel<PKV_BF16, false>);
             Stagger sg;
             if (gpw == 1) {                         // five to eight heads: x read once, as cells
-                auto cells = cells_kernel<true>(bits, dtype, perm != nullptr, false, xs.st != kHeadDim);
+                auto cells = cells_kernel<true>(bits, dtype, perm != nullptr, false, xs.st != kHeadDim, job.rot.cos != nullptr);
                 if ((rc = stagger_for(reinterpret_cast<const void *>(cells), 256, lds, nwg, &sg))) return rc;
                 cells<<<nwg, 256, lds, s>>>((const uint16_t *)x, B, H, T, xs, rel, (uint16_t *)scale, (uint16_t *)zero, stream,
-                                            capacity, info, st, bits, nwg, slot, base, par_stride, perm, perm_block, sg, 1, nullptr);
+                                            capacity, info, st, bits, nwg, slot, base, par_stride, perm, perm_block, sg, 1, nullptr, job.rot);
             } else {
                 if ((rc = stagger_for(reinterpret_cast<const void *>(kern), 256, lds, nwg, &sg))) return rc;
                 kern<<<nwg, 256, lds, s>>>((const uint16_t *)x, B, H, T, xs, rel, (uint16_t *)scale, (uint16_t *)zero, stream,
@@ -2180,12 +2237,12 @@ static int launch_quant_encode(const EncodeJob &job, int dtype, int B, int H, in
             const uint32_t slot = (bound + 15u) & ~15u;
             const uint32_t lds = (uint32_t)kSubBlocks * slot + 32u;
             const int nsg = (H + kSubBlocks - 1) / kSubBlocks;
-            auto kern = cells_kernel<true>(bits, dtype, false, true, xs.st != kHeadDim);
+            auto kern = cells_kernel<true>(bits, dtype, false, true, xs.st != kHeadDim, job.rot.cos != nullptr);
             Stagger sg;
             if ((rc = stagger_for(reinterpret_cast<const void *>(kern), 256, lds, nsub, &sg))) return rc;
             kern<<<nsub, 256, lds, s>>>((const uint16_t *)x, B, H, T, xs, rel, (uint16_t *)scale, (uint16_t *)zero, stream,
                                         capacity, info, st, bits, nsub, slot, base, par_stride, nullptr, 0, sg, nsg,
-                                        st->status + nsub);
+                                        st->status + nsub, job.rot);
         } else {                                     // V, more than eight heads: the same runs of eight
             const uint32_t unit_slot = (uint32_t)(((bound - 8u) / 4u + 15u) & ~15u);
             const uint32_t lds = 64u * unit_slot + 64u;
@@ -2377,6 +2434,13 @@ int pkv_kv_quant_encode_append(const pkv_append_side *k, const pkv_append_side *
                     PKV_ERR_INVALID, "rows must start on 16-byte boundaries (row stride below 2^25 elements)");
         job[i] = EncodeJob{a.x, XRows{a.stride_b, a.stride_h, a.stride_t}, a.rel, a.bits, a.stream, a.capacity, a.used, a.info_tail,
                            a.scale_tail, a.zero_tail, par_stride};
+        PKV_REQUIRE((a.cos == nullptr) == (a.sin == nullptr), PKV_ERR_INVALID, "cos and sin go together");
+        if (a.cos) {
+            PKV_REQUIRE(i == 0 && H > 4, PKV_ERR_UNSUPPORTED, "not supported: a rotary embedding other than of K with five heads or more");
+            PKV_REQUIRE(a.rot_stride_b >= 0 && a.rot_stride_b % 8 == 0 && ((reinterpret_cast<uintptr_t>(a.cos) | reinterpret_cast<uintptr_t>(a.sin)) & 15u) == 0,
+                        PKV_ERR_INVALID, "rows must start on 16-byte boundaries");
+            job[i].rot = Rot{(const uint16_t *)a.cos, (const uint16_t *)a.sin, a.rot_stride_b};
+        }
         rc = i == 0 ? check_job<true>(job[i], dtype, B, H, T_new) : check_job<false>(job[i], dtype, B, H, T_new);
         if (rc) return rc;
     }

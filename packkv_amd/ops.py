@@ -471,10 +471,21 @@ def _rows16(t):
     return t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(st % 8 == 0 for st in t.stride()[:-1])
 
 
-def kv_quant_encode_append(k, v, n, k_side, v_side, tokens):
+def _rotary_rows(cos, sin, like):
+    """cos / sin as [B, n, 128] tables the kernels read in place: (cos, sin, elements from one sequence's table to the next)."""
+    B, n = like.size(0), like.size(2)
+    cos, sin = cos.expand(B, n, 128), sin.expand(B, n, 128)
+    _require(cos.dtype == like.dtype and sin.dtype == like.dtype, "cos / sin must be [B, n, 128] of the tokens' dtype")
+    if cos.stride(2) != 1 or (n > 1 and cos.stride(1) != 128) or cos.stride() != sin.stride() or not _rows16(cos) or not _rows16(sin):
+        cos, sin = cos.contiguous(), sin.contiguous()
+    return cos, sin, cos.stride(0) if B > 1 else 0
+
+
+def kv_quant_encode_append(k, v, n, k_side, v_side, tokens, cos=None, sin=None):
     """quant_encode_append for the first n tokens (a multiple of 128) of k and of v [B, H, >= n, 128], with one wait for
     both.  The rows are read where they are (any strides whose rows start on 16-byte boundaries).  k_side / v_side:
-    (rel, bits, stream, used, info, scale, zero) as quant_encode_append takes them.  Returns the bytes in use of K and V."""
+    (rel, bits, stream, used, info, scale, zero) as quant_encode_append takes them.  With cos / sin (tables of k's rows;
+    five heads or more) the encoder applies the rotary embedding to K.  Returns the bytes in use of K and V."""
     B, H = k.size(0), k.size(1)
     _require(n % 128 == 0 and tokens % 128 == 0, "token counts must be multiples of the block length")
     sides, sizes = [], (ctypes.c_uint64(0), ctypes.c_uint64(0))
@@ -492,6 +503,9 @@ def kv_quant_encode_append(k, v, n, k_side, v_side, tokens):
         sides.append(_lib.AppendSide(x.data_ptr(), x.stride(0), x.stride(1), x.stride(2), stream.data_ptr(), stream.numel(), int(used),
                                      info.data_ptr() + 8 * (tokens // ctx_blk * per_tile), scale.data_ptr() + es * tokens,
                                      zero.data_ptr() + es * tokens, float(rel), int(bits)))
+    if cos is not None:
+        cos, sin, sides[0].rot_stride_b = _rotary_rows(cos, sin, k)
+        sides[0].cos, sides[0].sin = cos.data_ptr(), sin.data_ptr()
     with _on(k.device):
         rc = _lib.load().pkv_kv_quant_encode_append(ctypes.byref(sides[0]), ctypes.byref(sides[1]), _dtype_code(k), B, H, n,
                                                     k_side[5].size(1), ctypes.byref(sizes[0]), ctypes.byref(sizes[1]), _stream(k.device))
@@ -499,13 +513,15 @@ def kv_quant_encode_append(k, v, n, k_side, v_side, tokens):
     return int(sizes[0].value), int(sizes[1].value)
 
 
-def window_cut(k_new, v_new, cos, sin, k_pend, v_pend, k_win, v_win, win_len, stage, pend_out, k_rel, v_rel):
+def window_cut(k_new, v_new, cos, sin, k_pend, v_pend, k_win, v_win, win_len, stage, pend_out, k_rel, v_rel,
+               rotary_later=False):
     """The write into the cache's window when its first tokens leave for the streams (utils/compute.py:54-67,
     models/cache/packkv_quant.py:59-83).  Tokens in order: the pending cut's originals k_pend / v_pend [B, H, 64, 128] or
     None, the window rows behind them up to win_len, the new tokens [B, H, n, 128] (keys with their rotary embedding when
     cos / sin [B, n, 128] are given).  The first `stage` go to the encoder, `pend_out` (0 or 64) wait as the next pending
     cut, the rest are the new window.  Returns (k_stage, v_stage, k_pend, v_pend, k_win, v_win): what the encoder reads
-    (the new tokens themselves where nothing has to be done to them), the new pending originals or None, the new windows."""
+    (the new tokens themselves where nothing has to be done to them, or where, with nothing in the window, rotary_later
+    leaves the embedding of the staged keys to the encoder), the new pending originals or None, the new windows."""
     B, H, n, D = k_new.shape
     _require(D == 128 and v_new.shape == k_new.shape and k_new.is_cuda and v_new.is_cuda and v_new.dtype == k_new.dtype,
              "K and V must be device tensors [B, H, n, 128] of one dtype")
@@ -518,14 +534,11 @@ def window_cut(k_new, v_new, cos, sin, k_pend, v_pend, k_win, v_win, win_len, st
     buf = win_len - pend
     a = _lib.CutArgs()
     if cos is not None:
-        cos, sin = cos.expand(B, n, 128), sin.expand(B, n, 128)
-        _require(cos.dtype == k_new.dtype and sin.dtype == k_new.dtype, "cos / sin must be [B, n, 128] of the tokens' dtype")
-        if cos.stride(2) != 1 or (n > 1 and cos.stride(1) != 128) or cos.stride() != sin.stride() or not _rows16(cos) or not _rows16(sin):
-            cos, sin = cos.contiguous(), sin.contiguous()
-        a.cos, a.sin, a.rot_stride_b = cos.data_ptr(), sin.data_ptr(), cos.stride(0) if B > 1 else 0
+        cos, sin, a.rot_stride_b = _rotary_rows(cos, sin, k_new)
+        a.cos, a.sin = cos.data_ptr(), sin.data_ptr()
     empty = lambda rows: torch.empty(B, H, rows, 128, dtype=k_new.dtype, device=k_new.device)
     k_stage, v_stage = k_new, v_new
-    if stage and (pend + buf or cos is not None):
+    if stage and (pend + buf or (cos is not None and not rotary_later)):
         k_stage = empty(stage)
         a.k_stage = k_stage.data_ptr()
     if stage and pend + buf:

@@ -322,3 +322,33 @@ def test_window_cut_moves_every_row(cuda, dtype, pend, buf, n, rope):
             want = ops.dequantize(ops.quantize(cut, scale, zero)[0], scale, zero, B, H)
             assert torch.equal(w[:, :, :64], want)
         assert torch.equal(w[:, :, pend_out:x.size(2) - stage], x[:, :, stage + pend_out:])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,H,T,rel", [(1, 5, 128, 0.1), (2, 8, 256, 0.1), (3, 7, 128, 0.05), (1, 8, 384, 0.2), (2, 12, 256, 0.1), (1, 32, 128, 0.05)])
+def test_keys_rotated_by_the_encoder(cuda, dtype, B, H, T, rel):
+    """K appended with cos / sin tables -- one table for all sequences, one each, a prompt laid out [B, T, H, 128], and the
+    second half of a prompt's rows -- gives the stream, table and parameters of encoding the keys rotated by torch, a
+    negative zero and a subnormal among them (bit for bit: the roundings are the same)."""
+    from packkv_amd.cache import apply_rotary_pos_emb_single
+    k, v = synth.make_kv(B, H, T, seed=61, dtype=dtype, device=cuda)
+    k[:, :, 3, 5] = -0.0
+    k[:, :, 4, 70] = 6e-8
+    kt = k.transpose(1, 2).contiguous().transpose(1, 2)
+    for shared, x, lo in ((True, k, 0), (False, kt, 0), (True, kt, 128)):
+        n = T - lo
+        if n <= 0:
+            continue
+        _say("rotated keys", dtype, B, H, T, rel, "shared table", shared, "from", lo)
+        cos, sin = (t.to(cuda) for t in _rope_tables(1 if shared else B, 9, n, dtype))
+        cos, sin = cos.expand(B, n, 128), sin.expand(B, n, 128)
+        kr = apply_rotary_pos_emb_single(x[:, :, lo:], cos, sin).contiguous()
+        want = (ops.k_quant_encode(kr, rel), ops.v_quant_encode(v[:, :, lo:].contiguous(), rel))
+        sides = [[rel, w["bits"], torch.empty(w["stream"].numel() + 64, dtype=torch.uint8, device=cuda), 0, torch.empty_like(w["info"]),
+                  torch.empty_like(w["scale"]), torch.empty_like(w["zero"])] for w in want]
+        vx = v if x is k else v.transpose(1, 2).contiguous().transpose(1, 2)
+        sizes = ops.kv_quant_encode_append(x[:, :, lo:], vx[:, :, lo:], n, sides[0], sides[1], 0, cos, sin)
+        for w, s, size in zip(want, sides, sizes):
+            assert size == w["size"] and torch.equal(s[2][:size], w["stream"][:size])
+            assert torch.equal(s[4].view(torch.int32), w["info"].view(torch.int32))
+            assert torch.equal(s[5], w["scale"]) and torch.equal(s[6], w["zero"])
