@@ -682,12 +682,15 @@ struct PackSizeState {
     unsigned long long sum;             // workgroups that are done << kPackSizeDone | sum of the pack widths so far
     unsigned long long present[4];      // bit v: code v occurs
 };
-constexpr int kPackSizeDone = 52;       // 2^11 workgroups at most; 2^52 bits are 2^49 bytes of codes at the very least
+constexpr int kPackSizeDone = 52;       // fewer than 2^12 workgroups; 2^52 bits are 2^49 bytes of codes at the very least
 
-// 256 threads per workgroup, a grid-stride walk over the items (pack, 16 adjacent channels), the channel chunk
-// running fastest so that a wavefront reads whole rows; four rows in flight per thread; minima and maxima as packed
+// 256 or 1024 threads per workgroup, a grid-stride walk over the items (pack, 4 WORDS adjacent channels), the channel chunk
+// running fastest so that a wavefront reads whole rows; 16 / WORDS rows in flight per thread; minima and maxima as packed
 // 16-bit lanes (even and odd bytes of every dword apart).  One atomic per workgroup: same-address atomics retire
-// one after the other, so their number, not the bytes, would set the time of a grid with a workgroup per pack.
+// one after the other, so their number, not the bytes, would set the time of a grid with a workgroup per pack -- and the
+// wavefronts of a CU share a workgroup of 1024 (one presence table to clear, one atomic) rather than having one each of four.
+// Random 4-bit codes, packs of 16, a call's kernel time: 32768 x 16384 codes 113 us (174 with up to 2048 workgroups of 256
+// threads and 16 channels a thread), 16384 x 4096 37.6 (60.6), 16384 x 1024 19.6 (21.1), 256 x 512 9.4 (12.6).
 // Bound by instruction issue: 7 vector instructions per dword for the ranges and 8 for the presence flags (a
 // register bit mask for values below 32 instead of the LDS flags costs the same).
 // The last workgroup to finish hands the result to the waiting host thread (a tagged slot in pinned memory) and leaves
@@ -697,29 +700,37 @@ constexpr int kPackSizeDone = 52;       // 2^11 workgroups at most; 2^52 bits ar
 // addition to `sum` (which also counts it done): no fence, no cached read of another workgroup's data.
 typedef unsigned short pk_u16x2 __attribute__((ext_vector_type(2)));
 
-__global__ void __launch_bounds__(256) pack_size_kernel(const uint8_t *__restrict__ codes, int hidden, int pack_len,
+template <int WORDS>
+__global__ void __launch_bounds__(1024) pack_size_kernel(const uint8_t *__restrict__ codes, int hidden, int pack_len,
                                                         size_t n_items, PackSizeState *st, unsigned long long *slot,
                                                         uint32_t tag) {
     // a presence word per (code value, lane % 32): a lane marks its own column, so the marks of a wavefront never
     // share a bank however few values the matrix holds (one word per value made every mark a same-address conflict)
-    __shared__ uint32_t seen[256 * 32];
-    __shared__ unsigned long long wsum[4];
-    for (int i = threadIdx.x; i < 256 * 32; i += 256) seen[i] = 0u;
+    __shared__ __align__(16) uint32_t seen[256 * 32];
+    __shared__ unsigned long long wsum[16];
+    for (int i = threadIdx.x; i < 256 * 32 / 4; i += blockDim.x) reinterpret_cast<uint4 *>(seen)[i] = make_uint4(0u, 0u, 0u, 0u);
     __syncthreads();
     uint32_t *col = seen + (threadIdx.x & 31);
-    const uint32_t chunks = (uint32_t)hidden / 16u;
+    const uint32_t chunks = (uint32_t)hidden / (4u * WORDS);
+    struct Words { uint32_t w[WORDS]; };
+    constexpr int kRows = 16 / WORDS;
     unsigned long long lens = 0;
-    for (size_t item = (size_t)blockIdx.x * 256 + threadIdx.x; item < n_items; item += (size_t)gridDim.x * 256) {
+    for (size_t item = (size_t)blockIdx.x * blockDim.x + threadIdx.x; item < n_items; item += (size_t)gridDim.x * blockDim.x) {
         const size_t pack = item / chunks;
         const uint32_t chunk = (uint32_t)(item - pack * chunks);
-        const uint8_t *p = codes + pack * (size_t)pack_len * hidden + (size_t)chunk * 16;
-        pk_u16x2 mn[8], mx[8];
+        const uint8_t *p = codes + pack * (size_t)pack_len * hidden + (size_t)chunk * (4 * WORDS);
+        pk_u16x2 mn[2 * WORDS], mx[2 * WORDS];
 #pragma unroll
-        for (int i = 0; i < 8; i++) { mn[i] = (pk_u16x2){255, 255}; mx[i] = (pk_u16x2){0, 0}; }
-        auto take = [&](const uint4 v) {
-            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+        for (int i = 0; i < 2 * WORDS; i++) { mn[i] = (pk_u16x2){255, 255}; mx[i] = (pk_u16x2){0, 0}; }
+        auto load = [&](int row) -> Words {
+            const uint8_t *at = p + (size_t)row * hidden;
+            if constexpr (WORDS == 4) return __builtin_bit_cast(Words, *reinterpret_cast<const uint4 *>(at));
+            else return Words{{*reinterpret_cast<const uint32_t *>(at)}};
+        };
+        auto take = [&](const Words v) {
+            const uint32_t *w = v.w;
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
+            for (int i = 0; i < WORDS; i++) {
                 const pk_u16x2 e = __builtin_bit_cast(pk_u16x2, w[i] & 0x00FF00FFu);
                 const pk_u16x2 o = __builtin_bit_cast(pk_u16x2, (w[i] >> 8) & 0x00FF00FFu);
                 mn[2 * i] = __builtin_elementwise_min(mn[2 * i], e);
@@ -733,17 +744,17 @@ __global__ void __launch_bounds__(256) pack_size_kernel(const uint8_t *__restric
             }
         };
         int k = 0;
-        for (; k + 4 <= pack_len; k += 4) {
-            uint4 v[4];
+        for (; k + kRows <= pack_len; k += kRows) {
+            Words v[kRows];
 #pragma unroll
-            for (int u = 0; u < 4; u++) v[u] = *reinterpret_cast<const uint4 *>(p + (size_t)(k + u) * hidden);
+            for (int u = 0; u < kRows; u++) v[u] = load(k + u);
 #pragma unroll
-            for (int u = 0; u < 4; u++) take(v[u]);
+            for (int u = 0; u < kRows; u++) take(v[u]);
         }
-        for (; k < pack_len; k++) take(*reinterpret_cast<const uint4 *>(p + (size_t)k * hidden));
+        for (; k < pack_len; k++) take(load(k));
         uint32_t l = 0;
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
+        for (int i = 0; i < 2 * WORDS; i++) {
             const pk_u16x2 r = mx[i] - mn[i];
 #pragma unroll
             for (int hlf = 0; hlf < 2; hlf++)
@@ -755,7 +766,7 @@ __global__ void __launch_bounds__(256) pack_size_kernel(const uint8_t *__restric
     for (int d = 32; d >= 1; d >>= 1) lens += __shfl_xor(lens, d, 64);
     if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = lens;
     __syncthreads();
-    {   // value threadIdx.x: any of its 32 columns (read rotated, so that the threads of a wavefront spread over the banks)
+    if (threadIdx.x < 256) {   // value threadIdx.x: any of its 32 columns (read rotated, so that the threads of a wavefront spread over the banks)
         uint32_t any = 0u;
 #pragma unroll 8
         for (int c = 0; c < 32; c++) any |= seen[32 * threadIdx.x + ((c + threadIdx.x) & 31)];
@@ -770,7 +781,8 @@ __global__ void __launch_bounds__(256) pack_size_kernel(const uint8_t *__restric
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");            // this wavefront's marks have reached memory
     __syncthreads();
     if (threadIdx.x == 0) {
-        const unsigned long long mine = (1ull << kPackSizeDone) + (wsum[0] + wsum[1] + wsum[2] + wsum[3]);
+        unsigned long long mine = 1ull << kPackSizeDone;
+        for (uint32_t i = 0; i < blockDim.x / 64u; i++) mine += wsum[i];
         const unsigned long long all = __hip_atomic_fetch_add(&st->sum, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + mine;
         if ((all >> kPackSizeDone) == gridDim.x) {
             const unsigned long long total = all & ((1ull << kPackSizeDone) - 1ull), t = (unsigned long long)tag << 34;
@@ -807,9 +819,15 @@ int pkv_bit_pack_size(const uint8_t *codes, int ctx_len, int hidden_dim, int pac
     if ((rc = prepare_scan_state((uint32_t)(sizeof(PackSizeState) / 8), &sh, s))) return rc;
     LaunchTimer tm(s, ms_out != nullptr);
     if ((rc = tm.begin())) return rc;
-    const size_t n_items = (size_t)(ctx_len / pack_len) * (size_t)(hidden_dim / 16);
-    const size_t wanted = (n_items + 255) / 256;
-    pack_size_kernel<<<(unsigned)(wanted < 2048 ? wanted : 2048), 256, 0, s>>>(
+    // 16 channels to a thread once that fills the chip (two workgroups of 1024 per CU); below, 4 channels, and small
+    // workgroups while there is not one of 1024 for every CU (1024 x 1024 codes: 10.0 us, 12.8 with 16 channels a thread).
+    const size_t wide = (size_t)(ctx_len / pack_len) * (size_t)(hidden_dim / 16);
+    const bool large = wide >= 512u * 1024u;
+    const size_t n_items = large ? wide : 4 * wide;
+    const unsigned threads = n_items <= 256u * 256u ? 256u : 1024u;
+    const size_t wanted = (n_items + threads - 1) / threads;
+    auto kern = large ? pack_size_kernel<4> : pack_size_kernel<1>;
+    kern<<<(unsigned)(wanted < 512 ? wanted : 512), threads, 0, s>>>(
         codes, hidden_dim, pack_len, n_items, reinterpret_cast<PackSizeState *>(sh.st), (unsigned long long *)slot.words, slot.tag);
     PKV_HIP_CHECK(hipGetLastError());
     if ((rc = scan_state_cleared(sh, s))) return rc;

@@ -73,6 +73,19 @@ def test_code_stats_leave_their_state_clear_for_the_next_call(cuda, T, hid, pack
     assert ops.repack_and_encode(dev[0], dev[1], pack, "none") == ops.bit_pack(dev[0], dev[1], pack) * 2
 
 
+@pytest.mark.parametrize("packs,pack,top", [(16383, 17, 40), (16384, 16, 255), (16385, 33, 200), (524287, 3, 31), (524288, 5, 255), (524289, 2, 77)])
+def test_code_stats_on_both_sides_of_the_launch_rules(cuda, packs, pack, top):
+    """16 channels, one thread item (or four) a pack: the last size of the small workgroups and of the four-channel items and
+    the sizes beside them, pack lengths that leave a remainder of rows, against the definition on the same codes."""
+    _say("code_stats edges", packs, pack, top)
+    c = torch.randint(0, top + 1, (packs * pack, 16), generator=torch.Generator().manual_seed(packs), dtype=torch.uint8)
+    c[-pack:, 8:] = 0
+    c[-1, 15] = top                                       # the last channel's pack has a width of its own
+    r = c.reshape(packs, pack, 16)
+    rng = (r.amax(1).int() - r.amin(1).int()).double()
+    assert ops.code_stats(c.to(cuda), pack) == (int(torch.ceil(torch.log2(rng + 1)).sum()), int(c.unique().numel()))
+
+
 def test_median_repacking_matches_restatement(cuda):
     for (B, H, T, bs) in ((1, 2, 256, 64), (2, 8, 512, 64), (1, 1, 384, 128), (3, 2, 128, 16)):
         _say("repack case", B, H, T, bs)
