@@ -9,6 +9,7 @@
 #include <cstdarg>
 #include <cstddef>
 #include <cstdio>
+#include <cstring>
 #include <mutex>
 #include <vector>
 
@@ -219,6 +220,7 @@ static int slot_take(uint64_t **slot, uint32_t *tag) {       // caller holds g_w
             void *chunk = nullptr;
             PKV_HIP_CHECK(hipHostMalloc(&chunk, (size_t)kSlotsPerChunk * kSlotWords * 8,
                                         hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable));
+            std::memset(chunk, 0, (size_t)kSlotsPerChunk * kSlotWords * 8);     // (tags are never 0)
             g_chunks.push_back((uint64_t *)chunk);
             for (int i = 0; i < kSlotsPerChunk; i++) g_free_slots.push_back((uint64_t *)chunk + (size_t)i * kSlotWords);
         }
