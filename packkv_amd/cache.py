@@ -160,6 +160,14 @@ class PackKVCompressedCache:
                                                                 *((cos, sin) if later else ()))
                 L.k.tokens += whole
                 L.v.tokens += whole
+            if k_win is not L.k_win:
+                # the window the cut reads goes back to the allocator now, perhaps to another stream's pool (a prompt on one
+                # stream, decode steps on another), while the cut may still be queued: a cut that only makes a pending block
+                # waits for nothing.  (A second window per layer kept for life would do as well, at 320 more 16-bit rows a
+                # sequence and head.)
+                here = torch.cuda.current_stream(key_states.device)
+                L.k_win.record_stream(here)
+                L.v_win.record_stream(here)
             L.pend, L.k_pend, L.v_pend, L.k_win, L.v_win = cut - whole, k_pend, v_pend, k_win, v_win
             L.win_len = L.pend + left
             L.plan = None                  # token counts (and possibly the stream buffers) changed

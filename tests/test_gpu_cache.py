@@ -352,3 +352,37 @@ def test_keys_rotated_by_the_encoder(cuda, dtype, B, H, T, rel):
             assert size == w["size"] and torch.equal(s[2][:size], w["stream"][:size])
             assert torch.equal(s[4].view(torch.int32), w["info"].view(torch.int32))
             assert torch.equal(s[5], w["scale"]) and torch.equal(s[6], w["zero"])
+
+
+def test_a_cut_on_another_stream_keeps_the_window_it_reads(cuda):
+    """The prompt on one stream, a cut that waits for nothing queued on a second one: the first stream's next allocations
+    must not get the window that the cut has still to read (and may write to what they get)."""
+    B, H = 2, 4
+    k, v = synth.make_kv(B, H, 230, seed=17, device=cuda)
+    want = PackKVCompressedCache(B, H, 128, 1, max_tokens=512, device=cuda)
+    for lo, hi in ((0, 130), (130, 230)):
+        want.update(k[:, :, lo:hi], v[:, :, lo:hi], 0, return_dense=False)
+    want = want.materialize(0)
+    torch.cuda.synchronize()
+    prompt, decode = torch.cuda.Stream(), torch.cuda.Stream()
+    got = PackKVCompressedCache(B, H, 128, 1, max_tokens=512, device=cuda)
+    with torch.cuda.stream(prompt):
+        got.update(k[:, :, :130], v[:, :, :130], 0, return_dense=False)
+    L = got.layers[0]
+    old, shape = {L.k_win.data_ptr(), L.v_win.data_ptr()}, L.k_win.shape
+    decode.wait_stream(prompt)
+    with torch.cuda.stream(decode):
+        torch.cuda._sleep(50_000_000)
+        got.update(k[:, :, 130:], v[:, :, 130:], 0, return_dense=False)
+        done = decode.record_event()
+    assert L.k.tokens == 0 and L.pend == 64                   # a pending block only: nothing was waited for
+    with torch.cuda.stream(prompt):
+        others = [torch.full(shape, 7.0, dtype=torch.float16, device=cuda) for _ in range(4)]
+        early = not done.query()
+    assert early, "the cut had run before the other stream allocated"
+    assert not old & {t.data_ptr() for t in others}
+    prompt.wait_event(done)
+    with torch.cuda.stream(prompt):
+        dense = got.materialize(0)
+    torch.cuda.synchronize()
+    assert torch.equal(dense[0], want[0]) and torch.equal(dense[1], want[1])
