@@ -410,9 +410,14 @@ __device__ __forceinline__ void window_heads(const AttnParams &p, uint8_t *lds, 
                 l[g] += s[g][i];
             }
         }
+        // past the end V is zero as well: weight zero times an infinity of the last row would be NaN.  (The lanes compare
+        // again: the masks of the scores, kept until here, would take scalar registers the tiles' loop has not got.)
+        int rows = t1 - base - tt;
+        asm volatile("" : "+v"(rows));
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             float v8[8];
+            if (16 * i >= rows) vr[i] = make_uint4(0u, 0u, 0u, 0u);
             cvt8<BF>(vr[i], v8);
 #pragma unroll
             for (int g = 0; g < G; g++)

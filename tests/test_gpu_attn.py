@@ -578,3 +578,25 @@ def test_attn_decode_merged_by_its_last_workgroup(cuda, dtype, B, Hq, Hkv, T, Tw
         assert torch.equal(ops.attn_decode(qd, ke, ve, *win), got)
     assert torch.equal(ops.attn_decode(qd, ke, ve, *win, noalloc=True), got)
     assert torch.equal(ops.attn_decode(qd, ke, ve, *win, out_f32=True).to(dtype), got)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,Hq,Hkv,T,Tw", [(1, 2, 2, 0, 1), (2, 8, 4, 0, 63), (1, 12, 4, 128, 65), (2, 8, 1, 256, 130), (1, 8, 2, 256, 33),
+                                           (40, 16, 4, 128, 191)])
+def test_attn_decode_window_with_infinities(cuda, dtype, B, Hq, Hkv, T, Tw):
+    """V infinite in the newest and the oldest window row, one channel each (pieces of the window that are no multiple of 64
+    tokens, alone, beside tiles and shared by the splits): those channels are infinite with the row's sign, and no other
+    channel changes by a bit.  For that every weight has to be a positive fp32 number, so the queries are small: scores
+    (outlier keys of about 10 included) less than 40 apart, where exp reaches zero at 104."""
+    k, v = synth.make_kv(B, Hkv, T + Tw, seed=Tw, dtype=dtype)
+    q = synth.make_q(B, Hq, seed=3, dtype=dtype) * 0.125
+    scores = (q.float().reshape(B, Hkv, Hq // Hkv, 128) @ k.float().transpose(2, 3).contiguous()) * 128 ** -0.5
+    assert float((scores.amax(-1) - scores.amin(-1)).max()) < 40
+    q = q.to(cuda)
+    ke, ve = (ops.k_quant_encode(k[:, :, :T].contiguous().to(cuda), 0.1), ops.v_quant_encode(v[:, :, :T].contiguous().to(cuda), 0.1)) if T else (None, None)
+    kw, vw = k[:, :, T:].contiguous().to(cuda), v[:, :, T:].contiguous().to(cuda)
+    want = ops.attn_decode(q, ke, ve, kw, vw)
+    assert bool(want.isfinite().all())
+    vw[:, :, Tw - 1, 5], vw[:, :, 0, 77] = float("inf"), float("-inf")
+    want[:, :, 5], want[:, :, 77] = float("inf"), float("-inf")
+    assert torch.equal(ops.attn_decode(q, ke, ve, kw, vw), want)
