@@ -616,10 +616,11 @@ __global__ void __launch_bounds__(256) attn_merge_kernel(const float *__restrict
         for (int u = 0; u < 8; u++) {
             const int idx = min(s + 4 * u, nparts - 1);
             v[u] = col[(size_t)idx * (kPartStride / 2)];
-            w[u] = s + 4 * u < nparts ? w_s[idx] : 0.f;
+            w[u] = w_s[idx];
         }
 #pragma unroll
-        for (int u = 0; u < 8; u++) num += w[u] * v[u];
+        for (int u = 0; u < 8; u++)
+            if (s + 4 * u < nparts) num += w[u] * v[u];      // (not a weight of zero: the last partial may hold an infinity)
     }
     if (wave) reinterpret_cast<float2v *>(part_num + (wave - 1) * kHeadDim)[lane] = num;
     __syncthreads();

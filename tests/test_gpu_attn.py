@@ -582,12 +582,13 @@ def test_attn_decode_merged_by_its_last_workgroup(cuda, dtype, B, Hq, Hkv, T, Tw
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("B,Hq,Hkv,T,Tw", [(1, 2, 2, 0, 1), (2, 8, 4, 0, 63), (1, 12, 4, 128, 65), (2, 8, 1, 256, 130), (1, 8, 2, 256, 33),
-                                           (40, 16, 4, 128, 191)])
+                                           (40, 16, 4, 128, 191),
+                                           (1, 12, 4, 0, 65), (2, 8, 1, 0, 130), (1, 8, 2, 128 * 9, 33), (1, 2, 1, 128 * 40, 65)])
 def test_attn_decode_window_with_infinities(cuda, dtype, B, Hq, Hkv, T, Tw):
     """V infinite in the newest and the oldest window row, one channel each (pieces of the window that are no multiple of 64
-    tokens, alone, beside tiles and shared by the splits): those channels are infinite with the row's sign, and no other
-    channel changes by a bit.  For that every weight has to be a positive fp32 number, so the queries are small: scores
-    (outlier keys of about 10 included) less than 40 apart, where exp reaches zero at 104."""
+    tokens, alone, beside tiles, shared by the splits and merged by a launch of its own): those channels are infinite with
+    the row's sign, and no other channel changes by a bit.  For that every weight has to be a positive fp32 number, so the
+    queries are small: scores (outlier keys of about 10 included) less than 40 apart, where exp reaches zero at 104."""
     k, v = synth.make_kv(B, Hkv, T + Tw, seed=Tw, dtype=dtype)
     q = synth.make_q(B, Hq, seed=3, dtype=dtype) * 0.125
     scores = (q.float().reshape(B, Hkv, Hq // Hkv, 128) @ k.float().transpose(2, 3).contiguous()) * 128 ** -0.5
