@@ -466,9 +466,19 @@ def window_append(k_new, v_new, cos, sin, k_win, v_win, win_pos):
     _lib.check(rc)
 
 
+def _strides(t):
+    """Element strides, those of one-element dimensions as 0: they mean nothing and can be any number."""
+    return tuple(st if size > 1 else 0 for st, size in zip(t.stride(), t.shape))
+
+
 def _rows16(t):
     """Whether the rows of t [.., 128] can be read 16 bytes at a time where they are."""
-    return t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(st % 8 == 0 for st in t.stride()[:-1])
+    return t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(st % 8 == 0 for st in _strides(t)[:-1])
+
+
+def _copy(t):
+    """A contiguous copy in memory of its own (contiguous() hands back a tensor that is contiguous at any address)."""
+    return t.clone(memory_format=torch.contiguous_format)
 
 
 def _rotary_rows(cos, sin, like):
@@ -476,9 +486,9 @@ def _rotary_rows(cos, sin, like):
     B, n = like.size(0), like.size(2)
     cos, sin = cos.expand(B, n, 128), sin.expand(B, n, 128)
     _require(cos.dtype == like.dtype and sin.dtype == like.dtype, "cos / sin must be [B, n, 128] of the tokens' dtype")
-    if cos.stride(2) != 1 or (n > 1 and cos.stride(1) != 128) or cos.stride() != sin.stride() or not _rows16(cos) or not _rows16(sin):
-        cos, sin = cos.contiguous(), sin.contiguous()
-    return cos, sin, cos.stride(0) if B > 1 else 0
+    if (n > 1 and cos.stride(1) != 128) or _strides(cos) != _strides(sin) or not _rows16(cos) or not _rows16(sin):
+        cos, sin = _copy(cos), _copy(sin)
+    return cos, sin, _strides(cos)[0]
 
 
 def kv_quant_encode_append(k, v, n, k_side, v_side, tokens, cos=None, sin=None):
@@ -500,7 +510,7 @@ def kv_quant_encode_append(k, v, n, k_side, v_side, tokens, cos=None, sin=None):
         _require(stream.is_cuda and stream.dtype == torch.uint8 and stream.is_contiguous() and 0 <= used <= stream.numel(),
                  "compressed_buffer must be a contiguous device UInt8 tensor holding the bytes in use")
         es = scale.element_size()
-        sides.append(_lib.AppendSide(x.data_ptr(), x.stride(0), x.stride(1), x.stride(2), stream.data_ptr(), stream.numel(), int(used),
+        sides.append(_lib.AppendSide(x.data_ptr(), *_strides(x)[:3], stream.data_ptr(), stream.numel(), int(used),
                                      info.data_ptr() + 8 * (tokens // ctx_blk * per_tile), scale.data_ptr() + es * tokens,
                                      zero.data_ptr() + es * tokens, float(rel), int(bits)))
     if cos is not None:
@@ -528,8 +538,8 @@ def window_cut(k_new, v_new, cos, sin, k_pend, v_pend, k_win, v_win, win_len, st
     _require(k_win.is_contiguous() and v_win.is_contiguous() and k_win.shape == v_win.shape and k_win.dim() == 4
              and k_win.size(0) == B and k_win.size(1) == H and k_win.size(3) == 128 and k_win.dtype == k_new.dtype,
              "windows must be contiguous [B, H, cap, 128] of the tokens' dtype")
-    if k_new.stride() != v_new.stride() or not _rows16(k_new) or not _rows16(v_new):
-        k_new, v_new = k_new.contiguous(), v_new.contiguous()
+    if _strides(k_new) != _strides(v_new) or not _rows16(k_new) or not _rows16(v_new):
+        k_new, v_new = _copy(k_new), _copy(v_new)
     pend = 64 if k_pend is not None else 0
     buf = win_len - pend
     a = _lib.CutArgs()
@@ -547,7 +557,7 @@ def window_cut(k_new, v_new, cos, sin, k_pend, v_pend, k_win, v_win, win_len, st
     kp, vp = (empty(64), empty(64)) if pend_out else (None, None)
     kw, vw = (torch.empty_like(k_win), torch.empty_like(v_win)) if win_len else (k_win, v_win)
     a.k_new, a.v_new = k_new.data_ptr(), v_new.data_ptr()
-    a.stride_b, a.stride_h, a.stride_t = k_new.stride(0), k_new.stride(1), k_new.stride(2)
+    a.stride_b, a.stride_h, a.stride_t = _strides(k_new)[:3]
     if pend:
         a.k_pend, a.v_pend = k_pend.data_ptr(), v_pend.data_ptr()
     if win_len:

@@ -386,3 +386,42 @@ def test_a_cut_on_another_stream_keeps_the_window_it_reads(cuda):
         dense = got.materialize(0)
     torch.cuda.synchronize()
     assert torch.equal(dense[0], want[0]) and torch.equal(dense[1], want[1])
+
+
+def _placed(x, how):
+    """x where an encoder cannot read it in 16-byte rows: contiguous but 8 bytes past a 16-byte boundary, or with an odd
+    stride in a dimension of one element."""
+    if how == "offset":
+        out = torch.empty(x.numel() + 4, dtype=x.dtype, device=x.device)[4:].view(x.shape)
+    else:
+        out = torch.empty(x.numel(), dtype=x.dtype, device=x.device).as_strided(x.shape, (x.numel() // x.size(0) + 3,) + x.stride()[1:])
+    assert out.is_contiguous() and (out.data_ptr() % 16 == 8 or out.stride(0) % 8 == 3)
+    return out.copy_(x)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("B,how", [(2, "offset"), (1, "stride")])
+def test_cuts_take_tokens_and_tables_at_any_address(cuda, dtype, rope, B, how):
+    """A prompt that is encoded, a cut that makes a pending block, one that joins it and a prompt that ends in one, each
+    from tensors that are contiguous in torch's eyes only: the streams, pending originals and windows of a cache that was
+    given ordinary tensors."""
+    H, sizes = 5, (300, 1, 82, 64, 257)
+    k, v = synth.make_kv(B, H, sum(sizes), seed=51, dtype=dtype, device=cuda)
+    caches = [PackKVCompressedCache(B, H, 128, 1, max_tokens=1024, dtype=dtype, device=cuda) for _ in range(2)]
+    pos, states = 0, []
+    for n in sizes:
+        _say("tokens", pos, n, dtype, rope, B, how)
+        ks, vs = k[:, :, pos:pos + n].contiguous(), v[:, :, pos:pos + n].contiguous()
+        kw = dict(zip(("cos", "sin"), (t.to(cuda) for t in _rope_tables(B, pos, n, dtype)))) if rope else None
+        caches[0].update(ks, vs, 0, kw, return_dense=False)
+        caches[1].update(_placed(ks, how), _placed(vs, how), 0, kw and {a: _placed(t, how) for a, t in kw.items()}, return_dense=False)
+        pos += n
+        a, b = caches[0].layers[0], caches[1].layers[0]
+        states.append((b.k.tokens, b.pend))
+        assert (a.k.used, a.v.used, a.k.tokens, a.win_len, a.pend) == (b.k.used, b.v.used, b.k.tokens, b.win_len, b.pend)
+        for x, y in zip(caches[0].materialize(0), caches[1].materialize(0)):
+            assert torch.equal(x, y)
+        if a.pend:
+            assert torch.equal(a.k_pend, b.k_pend) and torch.equal(a.v_pend, b.v_pend)
+    assert states == [(128, 0), (128, 0), (128, 64), (256, 0), (512, 64)]
