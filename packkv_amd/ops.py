@@ -58,6 +58,12 @@ def _require(cond, msg):
         raise RuntimeError("PackKV Assertion failed: " + msg)
 
 
+def _on_device(dev, *tensors):
+    """The kernels get bare addresses: every tensor (None: not given) has to be on the device they run on."""
+    for t in tensors:
+        _require(t is None or t.device == dev, "all tensors must be on one device (%s)" % dev)
+
+
 def _device_of(*tensors):
     dev = None
     for t in tensors:
@@ -448,6 +454,7 @@ def window_append(k_new, v_new, cos, sin, k_win, v_win, win_pos):
     _require(k_win.is_contiguous() and v_win.is_contiguous() and k_win.shape == v_win.shape and k_win.dim() == 4
              and k_win.size(0) == B and k_win.size(1) == H and k_win.size(3) == 128 and k_win.dtype == k_new.dtype,
              "windows must be contiguous [B, H, cap, 128] of the tokens' dtype")
+    _on_device(k_new.device, v_new, cos, sin, k_win, v_win)
     if k_new.stride(3) != 1 or k_new.stride() != v_new.stride():
         k_new, v_new = k_new.contiguous(), v_new.contiguous()
     rot_sb = 0
@@ -484,6 +491,7 @@ def _copy(t):
 def _rotary_rows(cos, sin, like):
     """cos / sin as [B, n, 128] tables the kernels read in place: (cos, sin, elements from one sequence's table to the next)."""
     B, n = like.size(0), like.size(2)
+    _on_device(like.device, cos, sin)
     cos, sin = cos.expand(B, n, 128), sin.expand(B, n, 128)
     _require(cos.dtype == like.dtype and sin.dtype == like.dtype, "cos / sin must be [B, n, 128] of the tokens' dtype")
     if (n > 1 and cos.stride(1) != 128) or _strides(cos) != _strides(sin) or not _rows16(cos) or not _rows16(sin):
@@ -509,6 +517,7 @@ def kv_quant_encode_append(k, v, n, k_side, v_side, tokens, cos=None, sin=None):
                  "scale / zero must be contiguous [B, row] with room for the new tokens")
         _require(stream.is_cuda and stream.dtype == torch.uint8 and stream.is_contiguous() and 0 <= used <= stream.numel(),
                  "compressed_buffer must be a contiguous device UInt8 tensor holding the bytes in use")
+        _on_device(k.device, x, stream, info, scale, zero)
         es = scale.element_size()
         sides.append(_lib.AppendSide(x.data_ptr(), *_strides(x)[:3], stream.data_ptr(), stream.numel(), int(used),
                                      info.data_ptr() + 8 * (tokens // ctx_blk * per_tile), scale.data_ptr() + es * tokens,
@@ -538,6 +547,7 @@ def window_cut(k_new, v_new, cos, sin, k_pend, v_pend, k_win, v_win, win_len, st
     _require(k_win.is_contiguous() and v_win.is_contiguous() and k_win.shape == v_win.shape and k_win.dim() == 4
              and k_win.size(0) == B and k_win.size(1) == H and k_win.size(3) == 128 and k_win.dtype == k_new.dtype,
              "windows must be contiguous [B, H, cap, 128] of the tokens' dtype")
+    _on_device(k_new.device, v_new, k_pend, v_pend, k_win, v_win)
     if _strides(k_new) != _strides(v_new) or not _rows16(k_new) or not _rows16(v_new):
         k_new, v_new = _copy(k_new), _copy(v_new)
     pend = 64 if k_pend is not None else 0
@@ -931,6 +941,7 @@ def dense_view(k, v, k_win=None, v_win=None, win_len=None):
                  and k_win.shape[:2] == (B, H) and k_win.size(3) == 128 and 0 <= T_w <= k_win.size(2) and k_win.dtype == like.dtype
                  and v_win.dtype == like.dtype, "window tensors must be contiguous [B, H, cap, 128] of the cache's dtype")
         a.k_win, a.v_win, a.win_stride = _ptr(k_win), _ptr(v_win), k_win.size(2)
+    _on_device(like.device, k_win, v_win, *(d[f] for d in (k, v) if d is not None for f in ("stream", "info", "scale", "zero")))
     a.B, a.Hkv, a.T_c, a.T_w, a.dtype = B, H, T_c, T_w, _dtype_code(like)
     k_out = torch.empty(B, H, T_c + T_w, 128, dtype=like.dtype, device=like.device)
     v_out = torch.empty_like(k_out)

@@ -425,3 +425,30 @@ def test_cuts_take_tokens_and_tables_at_any_address(cuda, dtype, rope, B, how):
         if a.pend:
             assert torch.equal(a.k_pend, b.k_pend) and torch.equal(a.v_pend, b.v_pend)
     assert states == [(128, 0), (128, 0), (128, 64), (256, 0), (512, 64)]
+
+
+def test_tensors_on_another_device_are_refused_before_a_launch(cuda):
+    """Host tables, windows, parameters and streams beside device tokens: an error, on the append between cuts, on a cut, in
+    the encode and in the dense view."""
+    B, H = 1, 5
+    k, v = synth.make_kv(B, H, 256, seed=5, device=cuda)
+    host = torch.empty(B, H, 320, 128, dtype=torch.float16)
+    for n in (1, 256):                                        # an append, a cut
+        cos, sin = _rope_tables(B, 0, n, torch.float16)
+        for c, s in ((cos, sin), (cos.to(cuda), sin), (cos, sin.to(cuda))):
+            cache = PackKVCompressedCache(B, H, 128, 1, max_tokens=512, device=cuda)
+            with pytest.raises(RuntimeError, match="one device"):
+                cache.update(k[:, :, :n], v[:, :, :n], 0, {"cos": c, "sin": s}, return_dense=False)
+    win = host.to(cuda)
+    for kw, vw in ((host, win), (win, host)):
+        with pytest.raises(RuntimeError, match="one device"):
+            ops.window_append(k[:, :, :1], v[:, :, :1], None, None, kw, vw, 0)
+        with pytest.raises(RuntimeError, match="one device"):
+            ops.window_cut(k, v, None, None, None, None, kw, vw, 0, 128, 0, 0.1, 0.1)
+    ke, ve = ops.k_quant_encode(k, 0.1), ops.v_quant_encode(v, 0.1)
+    side = lambda e: [0.1, e["bits"], e["stream"], 0, e["info"], e["scale"], e["zero"]]
+    for f in (5, 6):
+        ks, vs = side(ke), side(ve)
+        vs[f] = vs[f].cpu()
+        with pytest.raises(RuntimeError, match="one device"):
+            ops.kv_quant_encode_append(k, v, 256, ks, vs, 0)
