@@ -298,9 +298,10 @@ int pkv_fused_wv(void *our_wv, const void *w, const void *v_zero, const void *v_
  *                     words as whole 8-byte words, so for it the buffer must extend at least 7 bytes
  *                     past the encoded size (size_out of the encoder) or the last block decodes wrongly
  *   k_scale..v_zero   [B, T_c] `dtype`
- *   q, out            [B, Hq, 128] `dtype`
- *   k_win, v_win      optional uncompressed tail [B, Hkv, T_w, 128] `dtype`, k_win 16-byte aligned (the residual
- *                     window the cache keeps in 16-bit, utils/compute.py:54-67); T_w may be 0
+ *   q, out            [B, Hq, 128] `dtype`, at any address of their elements
+ *   k_win, v_win      optional uncompressed tail [B, Hkv, T_w, 128] `dtype`, k_win 16-byte aligned, v_win at any
+ *                     address of its elements (the residual window the cache keeps in 16-bit, utils/compute.py:54-67);
+ *                     T_w may be 0
  *   T_c               compressed tokens, a multiple of 128 (may be 0 when T_w > 0)
  *   par_stride        tokens per row of the scale / zero arrays when they are allocated longer than
  *                     T_c (a cache that grows); 0 = T_c

@@ -27,6 +27,15 @@ namespace pkv {
 constexpr int kTile = 128;              // tokens per super-tile
 constexpr int kPartStride = 2 + kHeadDim;  // floats per partial: m, l, acc[128]
 typedef float float2v __attribute__((ext_vector_type(2)));
+// Rows of q and v_win and results are promised at their elements' alignment only.  The same wide instructions (global
+// accesses take any address), without telling the compiler more than that.
+typedef uint32_t uint4_at2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t uint_at2 __attribute__((aligned(2)));
+typedef float float2v_at4 __attribute__((ext_vector_type(2), aligned(4)));
+__device__ __forceinline__ uint4 load_uint4(const uint4_at2 *p) {
+    const uint4_at2 v = *p;
+    return make_uint4(v[0], v[1], v[2], v[3]);
+}
 
 __device__ __forceinline__ float a_ld16(const uint16_t *p, size_t i, int dtype) {
     const uint32_t u = p[i];
@@ -364,12 +373,13 @@ __device__ __forceinline__ void window_heads(const AttnParams &p, uint8_t *lds, 
     float *red_m = red + 4 * G * kHeadDim, *red_l = red_m + 4 * G;
     const int tid = threadIdx.x, tt = tid >> 4, c = tid & 15, wave = tid >> 6, lane = tid & 63;
     const size_t row0 = ((size_t)b * p.Hkv + h) * p.win_stride;
-    const uint4 *kbase = reinterpret_cast<const uint4 *>(p.k_win + row0 * kHeadDim) + c, *vbase = reinterpret_cast<const uint4 *>(p.v_win + row0 * kHeadDim) + c;
+    const uint4 *kbase = reinterpret_cast<const uint4 *>(p.k_win + row0 * kHeadDim) + c;
+    const uint4_at2 *vbase = reinterpret_cast<const uint4_at2 *>(p.v_win + row0 * kHeadDim) + c;
     float q[G][8], acc[G][8], m[G], l[G];
 #pragma unroll
     for (int g = 0; g < G; g++) {
         uint4 w = make_uint4(0u, 0u, 0u, 0u);                // an idle head slot (group of 3 in the kernel of 4, ...)
-        if (gb + g < p.Gq) w = reinterpret_cast<const uint4 *>(p.q + ((size_t)b * p.Hq + (size_t)h * p.Gq + gb + g) * kHeadDim)[c];
+        if (gb + g < p.Gq) w = load_uint4(reinterpret_cast<const uint4_at2 *>(p.q + ((size_t)b * p.Hq + (size_t)h * p.Gq + gb + g) * kHeadDim) + c);
         cvt8<BF>(w, q[g]);
         m[g] = -INFINITY; l[g] = 0.f;
 #pragma unroll
@@ -380,7 +390,7 @@ __device__ __forceinline__ void window_heads(const AttnParams &p, uint8_t *lds, 
 #pragma unroll
         for (int i = 0; i < 4; i++) kr[i] = kbase[(size_t)min(base + 16 * i + tt, t1 - 1) * 16];      // (past the end: the last row again, weight zero)
 #pragma unroll
-        for (int i = 0; i < 4; i++) vr[i] = vbase[(size_t)min(base + 16 * i + tt, t1 - 1) * 16];
+        for (int i = 0; i < 4; i++) vr[i] = load_uint4(vbase + (size_t)min(base + 16 * i + tt, t1 - 1) * 16);
         float s[G][4];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -561,10 +571,10 @@ __device__ __forceinline__ void merge_head(const AttnParams &p, uint8_t *lds, in
             for (int i = 1; i < WPH; i++) num += sums[tid + 64 * i];
         }
         if (p.out_f32) {
-            reinterpret_cast<float2v *>(reinterpret_cast<float *>(p.out) + hq * kHeadDim)[lane] = num / den;
+            reinterpret_cast<float2v_at4 *>(reinterpret_cast<float *>(p.out) + hq * kHeadDim)[lane] = num / den;
         } else {
             const uint32_t lo = a_st16(num[0] / den, p.dtype), hi = a_st16(num[1] / den, p.dtype);
-            reinterpret_cast<uint32_t *>(p.out + hq * kHeadDim)[lane] = lo | (hi << 16);
+            reinterpret_cast<uint_at2 *>(p.out + hq * kHeadDim)[lane] = lo | (hi << 16);
         }
     }
 }
@@ -628,10 +638,10 @@ __global__ void __launch_bounds__(256) attn_merge_kernel(const float *__restrict
 #pragma unroll
         for (int w = 0; w < 3; w++) num += reinterpret_cast<const float2v *>(part_num + w * kHeadDim)[lane];
         if (out_f32) {
-            reinterpret_cast<float2v *>(reinterpret_cast<float *>(out) + hq * kHeadDim)[lane] = num / den;
+            reinterpret_cast<float2v_at4 *>(reinterpret_cast<float *>(out) + hq * kHeadDim)[lane] = num / den;
         } else {
             const uint32_t lo = a_st16(num[0] / den, dtype), hi = a_st16(num[1] / den, dtype);
-            reinterpret_cast<uint32_t *>(out + hq * kHeadDim)[lane] = lo | (hi << 16);
+            reinterpret_cast<uint_at2 *>(out + hq * kHeadDim)[lane] = lo | (hi << 16);
         }
     }
 }

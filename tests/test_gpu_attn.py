@@ -601,3 +601,23 @@ def test_attn_decode_window_with_infinities(cuda, dtype, B, Hq, Hkv, T, Tw):
     vw[:, :, Tw - 1, 5], vw[:, :, 0, 77] = float("inf"), float("-inf")
     want[:, :, 5], want[:, :, 77] = float("inf"), float("-inf")
     assert torch.equal(ops.attn_decode(q, ke, ve, kw, vw), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,Hq,Hkv,T,Tw", [(1, 8, 2, 0, 33), (2, 6, 2, 256, 65), (1, 16, 2, 1280, 70), (40, 8, 4, 128, 191)])
+def test_attn_decode_takes_q_v_window_and_result_at_any_element(cuda, dtype, B, Hq, Hkv, T, Tw):
+    """q, v_win and out one element past a 16-byte boundary: the result of aligned tensors, bit for bit (the window alone,
+    merged in the attention kernel, by a launch of its own, and shared by the splits)."""
+    def shifted(x):
+        out = torch.empty(x.numel() + 1, dtype=x.dtype, device=cuda)[1:].view(x.shape)
+        assert out.data_ptr() % 16 == x.element_size()
+        return out.copy_(x)
+    k, v = synth.make_kv(B, Hkv, T + Tw, seed=Tw, dtype=dtype)
+    q = synth.make_q(B, Hq, seed=3, dtype=dtype).to(cuda)
+    ke, ve = (ops.k_quant_encode(k[:, :, :T].contiguous().to(cuda), 0.1), ops.v_quant_encode(v[:, :, :T].contiguous().to(cuda), 0.1)) if T else (None, None)
+    kw, vw = k[:, :, T:].contiguous().to(cuda), v[:, :, T:].contiguous().to(cuda)
+    for f32 in (False, True):
+        _say("any element", dtype, B, Hq, Hkv, T, Tw, "fp32 result" if f32 else "")
+        want = ops.attn_decode(q, ke, ve, kw, vw, out_f32=f32)
+        got = ops.attn_decode(shifted(q), ke, ve, kw, shifted(vw), out=shifted(torch.zeros_like(want)), out_f32=f32)
+        assert torch.equal(got, want)
