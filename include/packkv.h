@@ -158,7 +158,8 @@ int pkv_v_quant_encode_append(const void *x, int dtype, int B, int H, int T_new,
 
 /* pkv_kv_quant_encode_append: the two appends of a cut with one wait.  T_new (a multiple of 128) tokens of K and of V,
  * each read where it lies: element strides from one sequence, head and token to the next (multiples of 8, the rows on
- * 16-byte boundaries), so a cut needs no copy of the prompt it is taken from.  k_size / v_size receive the bytes in
+ * 16-byte boundaries; stride_t below 2^25, and stride_h of K below 2^31 - 128 with five heads or more whose rows are rotated
+ * or not 128 elements apart), so a cut needs no copy of the prompt it is taken from.  k_size / v_size receive the bytes in
  * use after the append; both encodes are launched before the call waits for either.  With cos / sin (K only, five heads or
  * more; [tokens, 128] of the data type, rot_stride_b elements from one sequence's table to the next, 0 for a shared one) the
  * rows get the rotary embedding of row 0 .. T_new - 1 on the way, rounded as in pkv_window_append. */

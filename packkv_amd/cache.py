@@ -150,7 +150,8 @@ class PackKVCompressedCache:
             # being rotated into a buffer of their own first: 32 x 8 heads x 8192 tokens (bf16, 512 MiB) 297 us against
             # 396.  A small one waits for the tables in every round: 2 x 8 x 2816 (11 MiB) 29.6 against 27.6.
             cos, sin = (cache_kwargs["cos"], cache_kwargs["sin"]) if rotary else (None, None)
-            later = (rotary and L.win_len == 0 and self.head_num > 4
+            # (The rotating encoder takes less than 4 GiB from head to head.)
+            later = (rotary and L.win_len == 0 and self.head_num > 4 and n < (1 << 24) - 1
                      and whole * self.batch_size * self.head_num * 128 * key_states.element_size() >= 32 << 20)
             k_enc, v_enc, k_pend, v_pend, k_win, v_win = ops.window_cut(
                 key_states, value_states, cos, sin, L.k_pend, L.v_pend, L.k_win, L.v_win, L.win_len, whole, cut - whole,

@@ -2132,8 +2132,10 @@ static int check_job(EncodeJob &job, int dtype, int B, int H, int T) {
     // that would grow past 4 GiB is reported as a full buffer instead of wrapping its offsets
     if (capacity > (1ull << 32)) capacity = 1ull << 32;
     PKV_REQUIRE(base <= capacity, PKV_ERR_CAPACITY, "stream offset beyond 4 GiB: block_info offsets are 32 bits");
-    // (the cells kernels reach the second head of a wavefront through a 32-bit byte offset)
-    PKV_REQUIRE((H <= 4 || job.xs.sh < (1ll << 31) - 128) && job.xs.st < (1 << 25), PKV_ERR_UNSUPPORTED,
+    // (the K cells kernels reach the second head of a wavefront through a 32-bit byte offset, unless the rows are 128 apart and
+    // not rotated: those hang off an address per lane)
+    const bool offset = IS_K && H > 4 && (job.xs.st != kHeadDim || job.rot.cos);
+    PKV_REQUIRE((!offset || job.xs.sh < (1ll << 31) - 128) && job.xs.st < (1 << 25), PKV_ERR_UNSUPPORTED,
                 "not supported: 4 GiB or more from one head to the next");
     PKV_REQUIRE(state_words(IS_K, B, H, T) < (1ull << 31), PKV_ERR_UNSUPPORTED, "batch x tokens too large");
     return PKV_OK;

@@ -483,6 +483,13 @@ def _rows16(t):
     return t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(st % 8 == 0 for st in _strides(t)[:-1])
 
 
+def _encodable(x):
+    """Whether the encoders can read the rows of x [B, H, n, 128] where they are: the limits of pkv_kv_quant_encode_append
+    (token stride; K's head stride for five heads or more, where rows 128 apart have none)."""
+    _, sh, st, _ = _strides(x)
+    return _rows16(x) and st < 1 << 25 and (x.size(1) <= 4 or st == 128 or sh < (1 << 31) - 128)
+
+
 def _copy(t):
     """A contiguous copy in memory of its own (contiguous() hands back a tensor that is contiguous at any address)."""
     return t.clone(memory_format=torch.contiguous_format)
@@ -548,7 +555,7 @@ def window_cut(k_new, v_new, cos, sin, k_pend, v_pend, k_win, v_win, win_len, st
              and k_win.size(0) == B and k_win.size(1) == H and k_win.size(3) == 128 and k_win.dtype == k_new.dtype,
              "windows must be contiguous [B, H, cap, 128] of the tokens' dtype")
     _on_device(k_new.device, v_new, k_pend, v_pend, k_win, v_win)
-    if _strides(k_new) != _strides(v_new) or not _rows16(k_new) or not _rows16(v_new):
+    if _strides(k_new) != _strides(v_new) or not _encodable(k_new) or not _encodable(v_new):
         k_new, v_new = _copy(k_new), _copy(v_new)
     pend = 64 if k_pend is not None else 0
     buf = win_len - pend

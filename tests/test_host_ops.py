@@ -1,8 +1,10 @@
 """Host side of packkv_amd/ops.py: checks that come before any launch, on tensors without a GPU."""
+import ctypes
+
 import pytest
 import torch
 
-from packkv_amd import ops
+from packkv_amd import _lib, ops
 
 
 def test_rotary_tables_on_another_device_than_the_tokens_are_refused():
@@ -12,3 +14,29 @@ def test_rotary_tables_on_another_device_than_the_tokens_are_refused():
     for cos, sin in ((there, there), (there, here), (here, there)):
         with pytest.raises(RuntimeError, match="one device"):
             ops._rotary_rows(cos, sin, like)
+
+
+def test_dense_rows_have_no_limit_from_head_to_head():
+    """2^24 tokens of five heads are 2^31 elements from head to head, which rows that lie 128 apart may have: the call comes
+    as far as the check behind that one (8192 sequences are too many; nothing is launched).  Strided K is refused."""
+    lib, at, size = _lib.load(), ctypes.c_void_p(4096), ctypes.c_uint64(0)
+    T, H, B = 1 << 24, 5, 8192
+    for fn in (lib.pkv_k_quant_encode, lib.pkv_v_quant_encode):
+        assert fn(at, _lib.F16, B, H, T, 0.1, 4, at, 1 << 20, at, at, at, ctypes.byref(size), None, None) != 0
+        assert b"batch x tokens too large" in lib.pkv_last_error()
+    side = lambda st, sh: _lib.AppendSide(4096, H * sh, sh, st, 4096, 1 << 20, 0, 4096, 4096, 4096, 0.1, 4)
+    for k, v, message in ((side(256, 1 << 31), side(256, 1 << 31), b"4 GiB or more"),
+                          (side(256, (1 << 31) - 256), side(256, 1 << 31), b"batch x tokens too large"),
+                          (side(128, 1 << 31), side(256, 1 << 31), b"batch x tokens too large")):
+        assert lib.pkv_kv_quant_encode_append(ctypes.byref(k), ctypes.byref(v), _lib.F16, B, H, T, T, ctypes.byref(size),
+                                              ctypes.byref(size), None) != 0
+        assert message in lib.pkv_last_error(), lib.pkv_last_error()
+
+
+def test_rows_that_the_encoders_cannot_reach_are_copied():
+    """What window_cut copies before the encode: the token and head strides that the entry point refuses, and no others."""
+    rows = lambda H, sh, st: torch.empty_strided((1, H, 256, 128), (0, sh, st, 1), dtype=torch.float16, device="meta")
+    for H, sh, st, want in ((5, 1 << 31, 128, True), (5, 1 << 31, 256, False), (4, 1 << 31, 256, True), (5, (1 << 31) - 136, 256, True),
+                            (5, (1 << 31) - 128, 256, False), (5, 128, 1 << 25, False), (4, 128, 1 << 25, False),
+                            (5, 128, (1 << 25) - 8, True), (5, 128, 1284, False), (1, 7, 256, True)):
+        assert ops._encodable(rows(H, sh, st)) == want, (H, sh, st)
