@@ -78,7 +78,8 @@ int pkv_v_encode(const uint8_t *codes, uint8_t *stream, uint64_t capacity, uint3
  * _append forms) -- for callers that passed size_out = NULL to keep the launch asynchronous: waits for the stream,
  * then returns what the encoder itself would have returned with size_out (PKV_ERR_CAPACITY when the stream did not
  * fit, PKV_ERR_INTERNAL, and with bits > 0 PKV_ERR_UNSUPPORTED when a code of a fused encode does not fit `bits`)
- * and stores the stream size.  No counterpart in the reference, whose encoders are synchronous host code. */
+ * and stores the stream size.  After pkv_kv_quant_encode_append: K's failure if K failed, else V's outcome.  No
+ * counterpart in the reference, whose encoders are synchronous host code. */
 int pkv_encode_status(pkv_stream_t s, int bits, uint64_t *size_out);
 int pkv_k_decode(const uint8_t *stream, uint64_t stream_bytes, const uint32_t *block_info, uint8_t *codes, int ctx_len,
                  int hidden_dim, int ctx_blk, int hid_blk, int bits, float *ms_out, pkv_stream_t s);

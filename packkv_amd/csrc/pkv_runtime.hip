@@ -101,22 +101,27 @@ int scratch_get(size_t bytes, hipStream_t s, void **out) {
 // ---- the encoders' look-back state and outcome ------------------------------------------------------------------
 // An outcome is two words, each valid by itself through its tag: total (34 bits) | tag << 34 and error (8 bits) |
 // largest code (16 bits) << 8 | tag << 34.
-__device__ __forceinline__ void publish_outcome(uint64_t *dst, const ScanState *st, uint64_t tag) {
+__device__ __forceinline__ void publish_outcome(uint64_t *dst, const ScanState *st, uint32_t error, uint64_t tag) {
     const uint64_t total = st->total & ((1ull << 34) - 1ull), code = min(st->max_code, 0xFFFFu);
     __hip_atomic_store(dst, total | (tag << 34), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    __hip_atomic_store(dst + 1, (uint64_t)(st->error & 0xFFu) | (code << 8) | (tag << 34), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(dst + 1, (uint64_t)(error & 0xFFu) | (code << 8) | (tag << 34), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // The outcome of the encode before it on the stream to `last` and, for a waiting caller, to `slot`; the state back to
-// zero.  Four words per thread: the state of 1 GiB of input (8192 tickets) is cleared by nine workgroups in 2 us.
+// zero.  Of two encodes `last` keeps the second's outcome unless the first one (codes of `bits` bits) failed.  Four words per thread: the state of 1 GiB of input (8192 tickets) is cleared by nine workgroups in 2 us.
 __global__ void __launch_bounds__(256) finish_encode_kernel(ScanState *st, ScanState *second, uint64_t *words, uint32_t n, uint64_t *last,
-                                                            uint64_t *slot, uint32_t tag) {
+                                                            uint64_t *slot, uint32_t tag, int bits) {
     constexpr uint32_t kHead = offsetof(ScanState, status) / 8;
     const uint32_t head2 = second ? (uint32_t)(reinterpret_cast<uint64_t *>(second) - words) : 0xFFFFFFFFu;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        if (slot) publish_outcome(slot, st, tag);
-        if (slot && second) publish_outcome(slot + kOutcomeWords, second, tag);
-        publish_outcome(last, second ? second : st, tag);
+        if (slot) publish_outcome(slot, st, st->error, tag);
+        if (slot && second) publish_outcome(slot + kOutcomeWords, second, second->error, tag);
+        if (second) {
+            const uint32_t first = st->error ? st->error : bits > 0 && st->max_code >= (1u << bits) ? (uint32_t)PKV_ERR_UNSUPPORTED : 0u;
+            publish_outcome(last, second, first ? first : second->error, tag);
+        } else {
+            publish_outcome(last, st, st->error, tag);
+        }
         for (uint32_t i = 0; i < kHead; i++) {
             words[i] = 0;
             if (second) words[head2 + i] = 0;
@@ -273,7 +278,7 @@ int finish_encode(ScanHandle &h, uint64_t *size_out, int bits, hipStream_t s, ui
         if (rc) return rc;
         if ((rc = slot_take(size_out ? &slot : nullptr, &tag))) return rc;
         const uint32_t n = (uint32_t)h.words64;
-        finish_encode_kernel<<<(n + 1023u) / 1024u, 256, 0, s>>>(h.st, h.second, (uint64_t *)h.st, n, w->last, slot, tag);
+        finish_encode_kernel<<<(n + 1023u) / 1024u, 256, 0, s>>>(h.st, h.second, (uint64_t *)h.st, n, w->last, slot, tag, bits);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) {
             if (slot) g_free_slots.push_back(slot);

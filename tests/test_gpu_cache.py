@@ -452,3 +452,23 @@ def test_tensors_on_another_device_are_refused_before_a_launch(cuda):
         vs[f] = vs[f].cpu()
         with pytest.raises(RuntimeError, match="one device"):
             ops.kv_quant_encode_append(k, v, 256, ks, vs, 0)
+
+
+@pytest.mark.parametrize("side", ["k", "v"])
+@pytest.mark.parametrize("why", ["capacity", "bits"])
+def test_encode_status_after_a_joint_append_that_failed(cuda, side, why):
+    """A stream of K or of V that does not fit its buffer, or codes that do not fit their width: the append raises, and so
+    does encode_status behind it.  After one that went well it gives V's size."""
+    k, v = synth.make_kv(1, 5, 256, seed=23, device=cuda)
+    enc = {"k": ops.k_quant_encode(k, 0.1), "v": ops.v_quant_encode(v, 0.1)}
+    sides = {s: [0.1, e["bits"], torch.empty_like(e["stream"]), 0, e["info"], e["scale"], e["zero"]] for s, e in enc.items()}
+    assert ops.kv_quant_encode_append(k, v, 256, sides["k"], sides["v"], 0) == (enc["k"]["size"], enc["v"]["size"])
+    assert ops.encode_status(cuda, bits=4) == enc["v"]["size"]
+    if why == "capacity":
+        sides[side][2] = sides[side][2][:1024]
+    else:
+        sides[side][1] = 2
+    for call in (lambda: ops.kv_quant_encode_append(k, v, 256, sides["k"], sides["v"], 0), lambda: ops.encode_status(cuda, bits=sides["v"][1])):
+        with pytest.raises(ops.PackKVError) as e:
+            call()
+        assert e.value.code == (4 if why == "capacity" else 1)
