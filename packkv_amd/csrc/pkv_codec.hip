@@ -345,7 +345,7 @@ static int run_pack(bool is_k, const uint8_t *codes, uint8_t *stream, uint64_t c
                        (is_k ? (ctx_blk == 64 && hid_blk == 128) : (ctx_blk == 128 && hid_blk == 64));
     if (cells) {
         const uint32_t ngroups = (uint32_t)cs.nblocks / (is_k ? 8u : 16u);
-        if ((rc = prepare_scan_state(ngroups, &sh, s))) return rc;
+        if ((rc = prepare_scan_state(ngroups, &sh, s, size_out || ms_out))) return rc;
         ScanState *st = sh.st;
         LaunchTimer tm(s, ms_out != nullptr);
         if ((rc = tm.begin())) return rc;
@@ -356,7 +356,7 @@ static int run_pack(bool is_k, const uint8_t *codes, uint8_t *stream, uint64_t c
     if (grouped) {
         const uint32_t ngroups = ((uint32_t)cs.nblocks + kPackGroup - 1) / kPackGroup;
         const uint32_t lds = 2u * (uint32_t)(ctx_blk * hid_blk) + (uint32_t)kPackGroup * cs.blk_cap + 32u;
-        if ((rc = prepare_scan_state(ngroups, &sh, s))) return rc;
+        if ((rc = prepare_scan_state(ngroups, &sh, s, size_out || ms_out))) return rc;
         ScanState *st = sh.st;
         auto kern = bits > 4 ? (is_k ? pack_group_kernel<true, true> : pack_group_kernel<false, true>)
                              : (is_k ? pack_group_kernel<true, false> : pack_group_kernel<false, false>);
@@ -372,7 +372,7 @@ static int run_pack(bool is_k, const uint8_t *codes, uint8_t *stream, uint64_t c
         if ((rc = tm.end(ms_out))) return rc;
         return finish_encode(sh, size_out, 0, s);
     }
-    if ((rc = prepare_scan_state((uint32_t)cs.nblocks, &sh, s))) return rc;
+    if ((rc = prepare_scan_state((uint32_t)cs.nblocks, &sh, s, size_out || ms_out))) return rc;
     ScanState *st = sh.st;
     LaunchTimer tm(s, ms_out != nullptr);
     if ((rc = tm.begin())) return rc;

@@ -894,7 +894,7 @@ static int run_pack_long(bool is_k, const uint8_t *codes, uint8_t *stream, uint6
     if (capacity > (1ull << 32)) capacity = 1ull << 32;          // block_info offsets are 32 bits: never wrapped
     const uint32_t nblocks = (uint32_t)(ctx_len / ((is_k ? 4 : 8) * P)) * (uint32_t)(hidden_dim / (is_k ? 128 : 64));
     ScanHandle sh;
-    if ((rc = prepare_scan_state(nblocks, &sh, s))) return rc;
+    if ((rc = prepare_scan_state(nblocks, &sh, s, size_out || ms_out))) return rc;
     ScanState *st = sh.st;
     LaunchTimer tm(s, ms_out != nullptr);
     if ((rc = tm.begin())) return rc;

@@ -2274,7 +2274,7 @@ static int run_quant_encode(const void *x, int dtype, int B, int H, int T, float
     int rc = check_job<IS_K>(job, dtype, B, H, T);
     if (rc) return rc;
     ScanHandle sh;
-    if ((rc = prepare_scan_state((uint32_t)state_words(IS_K, B, H, T), &sh, s))) return rc;
+    if ((rc = prepare_scan_state((uint32_t)state_words(IS_K, B, H, T), &sh, s, size_out || ms_out))) return rc;
     LaunchTimer tm(s, ms_out != nullptr);
     if ((rc = tm.begin())) return rc;
     if ((rc = launch_quant_encode<IS_K>(job, dtype, B, H, T, sh.st, s))) return rc;
@@ -2447,7 +2447,7 @@ int pkv_kv_quant_encode_append(const pkv_append_side *k, const pkv_append_side *
         if (rc) return rc;
     }
     ScanHandle sh;
-    if ((rc = prepare_scan_state((uint32_t)state_words(true, B, H, T_new), &sh, s, (uint32_t)state_words(false, B, H, T_new)))) return rc;
+    if ((rc = prepare_scan_state((uint32_t)state_words(true, B, H, T_new), &sh, s, true, (uint32_t)state_words(false, B, H, T_new)))) return rc;
     if ((rc = launch_quant_encode<true>(job[0], dtype, B, H, T_new, sh.st, s))) return rc;
     if ((rc = launch_quant_encode<false>(job[1], dtype, B, H, T_new, sh.second, s))) return rc;
     return finish_encode(sh, k_size, job[0].bits, s, v_size, job[1].bits);

@@ -816,7 +816,7 @@ int pkv_bit_pack_size(const uint8_t *codes, int ctx_len, int hidden_dim, int pac
     OutcomeSlot slot;
     if ((rc = slot.take(s))) return rc;
     ScanHandle sh;
-    if ((rc = prepare_scan_state((uint32_t)(sizeof(PackSizeState) / 8), &sh, s))) return rc;
+    if ((rc = prepare_scan_state((uint32_t)(sizeof(PackSizeState) / 8), &sh, s, true))) return rc;
     LaunchTimer tm(s, ms_out != nullptr);
     if ((rc = tm.begin())) return rc;
     // 16 channels to a thread once that fills the chip (two workgroups of 1024 per CU); below, 4 channels, and small
@@ -911,7 +911,7 @@ int pkv_greedy_repack(const uint8_t *k_codes, const uint8_t *v_codes, uint8_t *k
     int rc;
     if (groups > 0) {
         ScanHandle sh;
-        if ((rc = prepare_scan_state(groups * 2u * members * 128u, &sh, s))) return rc;
+        if ((rc = prepare_scan_state(groups * 2u * members * 128u, &sh, s, ms_out != nullptr))) return rc;
         ScanState *st = sh.st;
         LaunchTimer tm(s, ms_out != nullptr);
         if ((rc = tm.begin())) return rc;

@@ -76,6 +76,11 @@ static bool capturing(hipStream_t s) {
     return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
 }
 
+static int refuse_in_capture(hipStream_t s) {
+    PKV_REQUIRE(!capturing(s), PKV_ERR_HIP, "the result is waited for: not possible while the stream is capturing a graph");
+    return PKV_OK;
+}
+
 int scratch_get(size_t bytes, hipStream_t s, void **out) {
     std::lock_guard<std::mutex> lock(g_ws_mu);
     Workspace *w = nullptr;
@@ -138,7 +143,11 @@ __global__ void __launch_bounds__(256) clear_state_kernel(uint64_t *p, size_t n)
     if (i < n) p[i] = 0;
 }
 
-int prepare_scan_state(uint32_t nblocks, ScanHandle *out, hipStream_t s, uint32_t nblocks2) {
+int prepare_scan_state(uint32_t nblocks, ScanHandle *out, hipStream_t s, bool waited, uint32_t nblocks2) {
+    if (waited) {
+        const int rc = refuse_in_capture(s);
+        if (rc) return rc;
+    }
     constexpr size_t head = offsetof(ScanState, status) / 8;
     const size_t n1 = head + nblocks, n = n1 + (nblocks2 ? head + nblocks2 : 0);
     Workspace *w = nullptr;
@@ -239,7 +248,8 @@ static int slot_take(uint64_t **slot, uint32_t *tag) {       // caller holds g_w
 }
 
 int OutcomeSlot::take(hipStream_t s) {
-    PKV_REQUIRE(!capturing(s), PKV_ERR_HIP, "the result is waited for: not possible while the stream is capturing a graph");
+    const int rc = refuse_in_capture(s);
+    if (rc) return rc;
     std::lock_guard<std::mutex> lock(g_ws_mu);
     return slot_take(&words, &tag);
 }

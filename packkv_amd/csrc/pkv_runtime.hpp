@@ -68,8 +68,9 @@ struct ScanHandle {
     std::shared_ptr<std::mutex> mu;        // held from prepare_scan_state until finish_encode has launched its kernel:
     std::unique_lock<std::mutex> held;     // two host threads that encode on one stream take turns
 };
-// `nblocks` status words (and `nblocks2` for a second state when it is not zero).
-int prepare_scan_state(uint32_t nblocks, ScanHandle *out, hipStream_t s, uint32_t nblocks2 = 0);
+// `nblocks` status words (and `nblocks2` for a second state when it is not zero).  `waited`: the call will wait for its
+// outcome or its time, which is refused while `s` is capturing, before anything is recorded.
+int prepare_scan_state(uint32_t nblocks, ScanHandle *out, hipStream_t s, bool waited, uint32_t nblocks2 = 0);
 // Launches the kernel that publishes the outcome and clears the state; with `size_out` waits for it and reports it
 // (`size2_out`: of the second state).  `bits` > 0 additionally rejects a launch whose largest code does not fit.
 // NULL: returns at once, pkv_encode_status reads the outcome later.

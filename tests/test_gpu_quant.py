@@ -228,3 +228,40 @@ def test_asynchronous_encode_reports_through_encode_status(cuda):
     codes = torch.zeros(64, 128, dtype=torch.uint8, device=cuda)
     with pytest.raises(RuntimeError, match="even address"):
         ops.k_encode(codes, odd, torch.zeros(1, 2, dtype=torch.uint32, device=cuda))
+
+
+def test_encodes_that_wait_are_refused_while_their_stream_is_capturing(cuda):
+    """A call that hands a size or a time back is refused before it records anything, so the capture goes on: an encode
+    without them joins the graph, whose replays give what the eager call gives."""
+    B, H, T = 1, 5, 256
+    k, v = synth.make_kv(B, H, T, seed=630, device=cuda)
+    room = lambda: (torch.zeros(B * H * T * 128, dtype=torch.uint8, device=cuda), torch.zeros(T // 64 * B * H, 2, dtype=torch.uint32, device=cuda))
+    want, (stream, info), (other, oinfo) = ops.k_quant_encode(k, 0.1), room(), room()
+    codes, long_codes = ops.quantize(k, want["scale"], want["zero"])[0], torch.zeros(512, 128, dtype=torch.uint8, device=cuda)
+    side = lambda: [0.1, 4, other, 0, oinfo, torch.empty_like(want["scale"]), torch.empty_like(want["scale"])]
+    ksd, vsd = side(), side()
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        ops.k_quant_encode(k, 0.1, stream=stream, info=info)
+    g = torch.cuda.CUDAGraph()
+    calls = [lambda: ops.k_quant_encode(k, 0.1, stream=other, info=oinfo), lambda: ops.k_quant_encode(k, 0.1, stream=other, info=oinfo, want_size=False, timed=True),
+             lambda: ops.k_encode(codes, other, oinfo), lambda: ops.kv_quant_encode_append(k, v, T, ksd, vsd, 0),
+             lambda: ops.encode_p(True, long_codes, other, oinfo[:2], 64, 4), lambda: ops.code_stats(codes, 16)]
+    with torch.cuda.graph(g, stream=s):
+        for i, call in enumerate(calls):
+            _say("while capturing: call", i)
+            with pytest.raises(ops.PackKVError, match="capturing"):
+                call()
+        got = ops.k_quant_encode(k, 0.1, stream=stream, info=info, want_size=False)
+    for i in range(3):
+        for t in (stream, info.view(torch.int32), got["scale"], got["zero"]):
+            t.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(stream[:want["size"]], want["stream"][:want["size"]]) and torch.equal(info.view(torch.int32), want["info"].view(torch.int32))
+        assert torch.equal(got["scale"], want["scale"]) and torch.equal(got["zero"], want["zero"])
+        with torch.cuda.stream(s):
+            assert ops.encode_status(cuda, bits=4) == want["size"]
+            assert ops.k_quant_encode(k, 0.1)["size"] == want["size"]
