@@ -37,9 +37,8 @@ struct Workspace {
     uint32_t *counters;     // kAttnCounters tile counters of the attention kernel, zero between launches
     void *enc;              // the encoders' look-back state, zero between encodes
     size_t enc_bytes;
-    bool enc_dirty;         // between prepare_scan_state and the launch of the clearing kernel
-    uint64_t *last;         // pinned, host and device: outcome of the last encode on this stream (kOutcomeWords)
-    bool encoded;           // an encoder has run on this stream
+    bool enc_dirty;         // between prepare_scan_state and the launch of the kernel that clears the state
+    uint64_t *last;         // pinned, host and device: outcome of the last encode on this stream (kOutcomeWords), tag 0 before it
     std::shared_ptr<std::mutex> enc_mu;
 };
 constexpr int kOutcomeWords = 2, kSlotWords = 8;      // a slot: two outcomes (a cache line)
@@ -57,7 +56,7 @@ int workspace_for(hipStream_t s, Workspace **out) {     // caller holds g_ws_mu
     PKV_HIP_CHECK(hipGetDevice(&dev));
     for (Workspace &w : g_ws)
         if (w.dev == dev && w.stream == s) { *out = &w; return PKV_OK; }
-    g_ws.push_back(Workspace{dev, s, nullptr, 0, nullptr, nullptr, 0, false, nullptr, false, std::make_shared<std::mutex>()});
+    g_ws.push_back(Workspace{dev, s, nullptr, 0, nullptr, nullptr, 0, false, nullptr, std::make_shared<std::mutex>()});
     *out = &g_ws.back();
     return PKV_OK;
 }
@@ -143,6 +142,21 @@ __global__ void __launch_bounds__(256) clear_state_kernel(uint64_t *p, size_t n)
     if (i < n) p[i] = 0;
 }
 
+static hipError_t clear_state(const Workspace &w) {
+    const size_t all = w.enc_bytes / 8;
+    clear_state_kernel<<<(unsigned)((all + 255) / 256), 256, 0, w.stream>>>((uint64_t *)w.enc, all);
+    return hipGetLastError();
+}
+
+// A call that failed between its launches, with the encoder perhaps under way: the state is cleared behind it, for the
+// next encode and for the graphs that hold one.
+ScanHandle::~ScanHandle() {
+    if (!held.owns_lock() || !st) return;
+    std::lock_guard<std::mutex> lock(g_ws_mu);
+    Workspace *w = nullptr;
+    if (workspace_for(s, &w) == PKV_OK && clear_state(*w) == hipSuccess) w->enc_dirty = false;
+}
+
 int prepare_scan_state(uint32_t nblocks, ScanHandle *out, hipStream_t s, bool waited, uint32_t nblocks2) {
     if (waited) {
         const int rc = refuse_in_capture(s);
@@ -160,14 +174,24 @@ int prepare_scan_state(uint32_t nblocks, ScanHandle *out, hipStream_t s, bool wa
     out->held = std::unique_lock<std::mutex>(*out->mu);
     std::lock_guard<std::mutex> lock(g_ws_mu);
     if ((rc = workspace_for(s, &w))) return rc;            // (the list may have moved meanwhile)
-    bool clear = w->enc_dirty;                     // an earlier call failed between its two launches
+    // An earlier call failed and so did the clearing behind it (~ScanHandle): the state is cleared first.  Not inside a
+    // capture: that would only record it, and an eager encode before the first replay would find the state as it was left.
+    if (w->enc_dirty && capturing(s)) {
+        set_error("stream is capturing a graph and an encode on it has failed before: make one eager call on this stream first");
+        return PKV_ERR_CAPTURING;
+    }
     if (w->enc_bytes < n * 8 || !w->last) {
         if (capturing(s)) {
             set_error("stream is capturing a graph and has no scratch buffer of %zu bytes yet: make one eager call "
                       "of the same shape on this stream first", n * 8);
             return PKV_ERR_CAPTURING;
         }
-        if (!w->last) PKV_HIP_CHECK(hipHostMalloc((void **)&w->last, kOutcomeWords * 8, hipHostMallocMapped | hipHostMallocCoherent));
+        if (!w->last) {
+            void *last = nullptr;
+            PKV_HIP_CHECK(hipHostMalloc(&last, kOutcomeWords * 8, hipHostMallocMapped | hipHostMallocCoherent));
+            std::memset(last, 0, kOutcomeWords * 8);
+            w->last = (uint64_t *)last;
+        }
         if (w->enc_bytes < n * 8) {
             const size_t want = scratch_grown_size(w->enc_bytes, n * 8);
             void *fresh = nullptr;
@@ -175,15 +199,12 @@ int prepare_scan_state(uint32_t nblocks, ScanHandle *out, hipStream_t s, bool wa
             if (w->enc) g_retired.push_back(Retired{w->dev, s, w->enc});
             w->enc = fresh;
             w->enc_bytes = want;
-            clear = true;
+            w->enc_dirty = true;
         }
     }
-    if (clear) {
-        const size_t all = w->enc_bytes / 8;
-        clear_state_kernel<<<(unsigned)((all + 255) / 256), 256, 0, s>>>((uint64_t *)w->enc, all);
-        PKV_HIP_CHECK(hipGetLastError());
-    }
+    if (w->enc_dirty) PKV_HIP_CHECK(clear_state(*w));
     w->enc_dirty = true;
+    out->s = s;
     out->st = (ScanState *)w->enc;
     out->second = nblocks2 ? (ScanState *)((uint64_t *)w->enc + n1) : nullptr;
     out->words64 = n;
@@ -296,7 +317,6 @@ int finish_encode(ScanHandle &h, uint64_t *size_out, int bits, hipStream_t s, ui
             return PKV_ERR_HIP;
         }
         w->enc_dirty = false;
-        w->encoded = true;
     }
     h.held.unlock();
     if (!slot) return PKV_OK;
@@ -315,10 +335,10 @@ static int encode_status(hipStream_t s, int bits, uint64_t *size_out) {
         Workspace *w = nullptr;
         int rc = workspace_for(s, &w);
         if (rc) return rc;
-        PKV_REQUIRE(w->encoded && w->last, PKV_ERR_INVALID, "no encode has been launched on this stream");
         last = w->last;
     }
     PKV_HIP_CHECK(hipStreamSynchronize(s));
+    PKV_REQUIRE(last && (last[0] >> 34) != 0, PKV_ERR_INVALID, "no encode has run on this stream");
     return outcome(last, size_out, bits);
 }
 

@@ -67,6 +67,8 @@ struct ScanHandle {
     size_t words64 = 0;            // 64-bit words of the whole region
     std::shared_ptr<std::mutex> mu;        // held from prepare_scan_state until finish_encode has launched its kernel:
     std::unique_lock<std::mutex> held;     // two host threads that encode on one stream take turns
+    hipStream_t s = nullptr;
+    ~ScanHandle();
 };
 // `nblocks` status words (and `nblocks2` for a second state when it is not zero).  `waited`: the call will wait for its
 // outcome or its time, which is refused while `s` is capturing, before anything is recorded.

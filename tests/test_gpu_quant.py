@@ -1,11 +1,13 @@
 """GPU parity of the quantizer and the fused quantize+encode kernels: integer codes, scale, zero,
 dequantised values and the packed stream are bit-exact against the CPU oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 from oracle import quant as oq
-from packkv_amd import ops, synth
+from packkv_amd import _lib, ops, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -265,3 +267,67 @@ def test_encodes_that_wait_are_refused_while_their_stream_is_capturing(cuda):
         with torch.cuda.stream(s):
             assert ops.encode_status(cuda, bits=4) == want["size"]
             assert ops.k_quant_encode(k, 0.1)["size"] == want["size"]
+
+
+def test_an_encode_that_fails_after_its_launch_leaves_the_look_back_state_clear(cuda):
+    """The encoder is launched but the call fails behind it (an error that an earlier HIP call of the thread left is found
+    there): a graph that holds an encode, a capture made next and eager encodes give what they gave before.  Where the
+    clearing of a new state is what fails, nothing is captured before an eager call, and the stream has no status."""
+    B, H, T = 1, 5, 512
+    k, _ = synth.make_kv(B, H, T, seed=640, device=cuda)
+    want = ops.k_quant_encode(k, 0.1)
+    e = {n: torch.empty_like(want[n]) for n in ("stream", "info", "scale", "zero")}
+    lib, s = _lib.load(), torch.cuda.Stream()
+    with open("/proc/self/maps") as f:
+        hip = ctypes.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
+    torch.cuda.synchronize()
+
+    def fail():
+        assert hip.hipSetDevice(4096) != 0                    # no such device: the error stays for the thread
+        p = {n: ctypes.c_void_p(t.data_ptr()) for n, t in e.items()}
+        rc = lib.pkv_k_quant_encode(ctypes.c_void_p(k.data_ptr()), _lib.F16, B, H, T, 0.1, want["bits"], p["stream"], e["stream"].numel(), p["info"],
+                                    p["scale"], p["zero"], None, None, ctypes.c_void_p(s.cuda_stream))
+        assert rc == 3, (rc, lib.pkv_last_error())
+
+    def check():
+        torch.cuda.synchronize()
+        assert torch.equal(e["stream"][:want["size"]], want["stream"][:want["size"]])
+        for n in ("info", "scale", "zero"):
+            assert torch.equal(e[n].view(torch.int16), want[n].view(torch.int16))
+            e[n].zero_()
+        e["stream"].zero_()
+        torch.cuda.synchronize()
+
+    def capture():
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            got = ops.k_quant_encode(k, 0.1, stream=e["stream"], info=e["info"], want_size=False)
+            e["scale"].copy_(got["scale"])
+            e["zero"].copy_(got["zero"])
+        return g, got
+
+    fail()                                                    # the first call of the stream: its state is not even clear
+    with torch.cuda.stream(s), pytest.raises(ops.PackKVError, match="no encode has run"):
+        ops.encode_status(cuda)
+    with torch.cuda.graph(torch.cuda.CUDAGraph(), stream=s):
+        e["stream"].zero_()
+        with pytest.raises(ops.PackKVError, match="eager call"):
+            ops.k_quant_encode(k, 0.1, stream=e["stream"], info=e["info"], want_size=False)
+    with torch.cuda.stream(s):
+        assert ops.k_quant_encode(k, 0.1)["size"] == want["size"]
+    graphs = [capture()]
+    for i in range(3):
+        _say("after a failed call", i)
+        fail()
+        for g, _ in graphs:
+            with torch.cuda.stream(s):                        # (the state is the stream's: a replay elsewhere would race with it)
+                g.replay()
+            check()
+        fail()
+        graphs.append(capture())
+        with torch.cuda.stream(s):
+            got = ops.k_quant_encode(k, 0.1, stream=e["stream"], info=e["info"])
+            e["scale"].copy_(got["scale"])
+            e["zero"].copy_(got["zero"])
+        assert got["size"] == want["size"]
+        check()
