@@ -37,14 +37,14 @@ def _ptr(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
 
 
-_raw_stream = torch._C._cuda_getCurrentRawStream
-_current_device = torch._C._cuda_getDevice
+# Every op makes `dev` current and passes on its current stream.  A stream object and a device context that is entered
+# although the device is current take 3.5 us of host time a call -- a decode step is two calls and 13 us of GPU time --
+# these two take 0.5.  (They are not part of torch's public surface: without them the public functions serve.)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda index: torch.cuda.current_stream(index).cuda_stream)
+_current_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
 _here = contextlib.nullcontext()
 
 
-# Every op makes `dev` current and passes on its current stream.  A stream object and a device context that is entered
-# although the device is current take 3.5 us of host time a call -- a decode step is two calls and 13 us of GPU time --
-# these two take 0.5.
 def _stream(dev):
     return _raw_stream(_current_device() if dev.index is None else dev.index)
 

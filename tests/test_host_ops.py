@@ -1,5 +1,8 @@
 """Host side of packkv_amd/ops.py: checks that come before any launch, on tensors without a GPU."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -40,3 +43,17 @@ def test_rows_that_the_encoders_cannot_reach_are_copied():
                             (5, (1 << 31) - 128, 256, False), (5, 128, 1 << 25, False), (4, 128, 1 << 25, False),
                             (5, 128, (1 << 25) - 8, True), (5, 128, 1284, False), (1, 7, 256, True)):
         assert ops._encodable(rows(H, sh, st)) == want, (H, sh, st)
+
+
+def test_import_without_the_private_torch_functions():
+    """The two look-ups that torch does not promise: without them the module imports and asks torch.cuda instead."""
+    code = """
+import types, torch
+del torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
+torch.cuda.current_device = lambda: 3
+torch.cuda.current_stream = lambda device=None: types.SimpleNamespace(cuda_stream=100 + device)
+from packkv_amd import ops
+assert ops._stream(torch.device("cuda")) == 103 and ops._stream(torch.device("cuda", 1)) == 101
+assert ops._on(torch.device("cuda", 3)) is ops._here
+"""
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))), timeout=300)
