@@ -101,6 +101,12 @@ class _Layer:
         self.plan = None                   # checked arguments of the decode step, valid until the next cut
 
 
+# A prompt whose keys are at least so many bytes has them rotated by the encoder as it reads them (kernels for five heads or
+# more) instead of being rotated into a buffer of their own first: 32 x 8 heads x 8192 tokens (bf16, 512 MiB) 297 us against
+# 396.  A small one waits for the tables in every round: 2 x 8 x 2816 (11 MiB) 29.6 against 27.6.
+ROTATE_IN_ENCODER = 32 << 20
+
+
 class PackKVCompressedCache:
     """``update`` / ``get_seq_length`` as in the reference's cache classes, plus ``attend``."""
 
@@ -146,13 +152,10 @@ class PackKVCompressedCache:
             if whole:
                 L.k.reserve(whole // 128)
                 L.v.reserve(whole // 128)
-            # A large prompt's keys are rotated by the encoder as it reads them (kernels for five heads or more) instead of
-            # being rotated into a buffer of their own first: 32 x 8 heads x 8192 tokens (bf16, 512 MiB) 297 us against
-            # 396.  A small one waits for the tables in every round: 2 x 8 x 2816 (11 MiB) 29.6 against 27.6.
             cos, sin = (cache_kwargs["cos"], cache_kwargs["sin"]) if rotary else (None, None)
             # (The rotating encoder takes less than 4 GiB from head to head.)
             later = (rotary and L.win_len == 0 and self.head_num > 4 and n < (1 << 24) - 1
-                     and whole * self.batch_size * self.head_num * 128 * key_states.element_size() >= 32 << 20)
+                     and whole * self.batch_size * self.head_num * 128 * key_states.element_size() >= ROTATE_IN_ENCODER)
             k_enc, v_enc, k_pend, v_pend, k_win, v_win = ops.window_cut(
                 key_states, value_states, cos, sin, L.k_pend, L.v_pend, L.k_win, L.v_win, L.win_len, whole, cut - whole,
                 cfg.k_quant_scale_rel, cfg.v_quant_scale_rel, rotary_later=later)

@@ -472,3 +472,48 @@ def test_encode_status_after_a_joint_append_that_failed(cuda, side, why):
         with pytest.raises(ops.PackKVError) as e:
             call()
         assert e.value.code == (4 if why == "capacity" else 1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,H,n,layout,shared", [(1, 5, 320, "bhnd", True), (2, 5, 363, "bnhd", True), (2, 8, 300, "bnhd", False),
+                                                 (2, 8, 512, "bhnd", False), (1, 12, 380, "bnhd", True), (2, 12, 447, "bhnd", False)])
+def test_prompt_rotated_in_the_encoder_or_before_it(cuda, monkeypatch, dtype, B, H, n, layout, shared):
+    """A first prompt by both routes, with a whole number of tiles and with a pending cut behind them, as [B, H, n, 128] and
+    as a transposed [B, n, H, 128], one rotary table for all sequences and one each: the same streams, tables, parameters,
+    pending originals and window, and the dense view of the restated reference cache."""
+    from packkv_amd import cache as cache_mod
+    k, v = synth.make_kv(B, H, n, seed=71, dtype=dtype)
+    cos, sin = _rope_tables(1 if shared else B, 5, n, dtype)
+    if not shared:
+        for b in range(1, B):
+            cos[b], sin[b] = (t[0] for t in _rope_tables(1, 5 + 40 * b, n, dtype))
+    cos, sin = cos.expand(B, n, 128), sin.expand(B, n, 128)
+    want = oc.SimulatedCache(1, 64, 192, 0.1, 0.1).update(k, v, 0, cos, sin)
+    place = (lambda x: x.to(cuda)) if layout == "bhnd" else (lambda x: x.to(cuda).transpose(1, 2).contiguous().transpose(1, 2))
+    dev = [place(k), place(v), (cos[:1] if shared else cos).to(cuda).expand(B, n, 128), (sin[:1] if shared else sin).to(cuda).expand(B, n, 128)]
+    cut, routes = ops.window_cut, []
+
+    def spy(*args, rotary_later=False, **kw):
+        routes.append(rotary_later)
+        return cut(*args, rotary_later=rotary_later, **kw)
+
+    monkeypatch.setattr(ops, "window_cut", spy)
+    layers = []
+    for limit in (0, 1 << 62):
+        monkeypatch.setattr(cache_mod, "ROTATE_IN_ENCODER", limit)
+        cache = PackKVCompressedCache(B, H, 128, 1, max_tokens=512, dtype=dtype, device=cuda)
+        _say("prompt", dtype, B, H, n, layout, "one table" if shared else "a table each", "limit", limit)
+        dense = cache.update(dev[0], dev[1], 0, {"cos": dev[2], "sin": dev[3]})
+        for g, w in zip(dense, want):
+            assert torch.equal(g.cpu().view(torch.int16), w.view(torch.int16))
+        layers.append(cache.layers[0])
+    assert routes == [True, False]
+    a, b = layers
+    assert a.k.tokens and (a.k.tokens, a.pend, a.win_len) == (b.k.tokens, b.pend, b.win_len)
+    for x, y in ((a.k, b.k), (a.v, b.v)):
+        blocks = x.tokens // 128 * x.blocks_per_tile
+        assert x.used == y.used and torch.equal(x.stream[:x.used], y.stream[:x.used])
+        assert torch.equal(x.info[:blocks].view(torch.int32), y.info[:blocks].view(torch.int32))
+        assert torch.equal(x.scale[:, :x.tokens], y.scale[:, :x.tokens]) and torch.equal(x.zero[:, :x.tokens], y.zero[:, :x.tokens])
+    assert (a.k_pend is None) == (a.pend == 0) and (a.pend == 0 or torch.equal(a.k_pend, b.k_pend) and torch.equal(a.v_pend, b.v_pend))
+    assert torch.equal(a.k_win[:, :, :a.win_len], b.k_win[:, :, :a.win_len]) and torch.equal(a.v_win[:, :, :a.win_len], b.v_win[:, :, :a.win_len])
