@@ -58,10 +58,9 @@ def _require(cond, msg):
         raise RuntimeError("PackKV Assertion failed: " + msg)
 
 
-def _on_device(dev, *tensors):
-    """The kernels get bare addresses: every tensor (None: not given) has to be on the device they run on."""
-    for t in tensors:
-        _require(t is None or t.device == dev, "all tensors must be on one device (%s)" % dev)
+# The kernels get bare addresses: a tensor on another device than the one they run on must not get that far.  (Compared as
+# get_device() of tensors that are on a GPU: -1 on the host; two torch.device objects take three times as long.)
+_ONE_DEVICE = "all tensors must be on one device"
 
 
 def _device_of(*tensors):
@@ -449,45 +448,49 @@ def window_append(k_new, v_new, cos, sin, k_win, v_win, win_pos):
     chain of 16-bit elementwise ops (utils/compute.py:35-43).  One launch; strided views (a transposed projection
     output, an expanded cos / sin table) are read in place."""
     B, H, n, D = k_new.shape
-    _require(D == 128 and v_new.shape == k_new.shape and k_new.is_cuda and v_new.dtype == k_new.dtype,
+    dev, at, dtype, win = k_new.device, k_new.get_device(), k_new.dtype, k_win.shape
+    _require(D == 128 and v_new.shape == k_new.shape and k_new.is_cuda and v_new.dtype == dtype,
              "K and V must be device tensors [B, H, n, 128] of one dtype")
-    _require(k_win.is_contiguous() and v_win.is_contiguous() and k_win.shape == v_win.shape and k_win.dim() == 4
-             and k_win.size(0) == B and k_win.size(1) == H and k_win.size(3) == 128 and k_win.dtype == k_new.dtype,
+    _require(k_win.is_contiguous() and v_win.is_contiguous() and v_win.shape == win and len(win) == 4
+             and win[0] == B and win[1] == H and win[3] == 128 and k_win.dtype == dtype,
              "windows must be contiguous [B, H, cap, 128] of the tokens' dtype")
-    _on_device(k_new.device, v_new, cos, sin, k_win, v_win)
-    if k_new.stride(3) != 1 or k_new.stride() != v_new.stride():
+    _require(v_new.get_device() == at and k_win.get_device() == at and v_win.get_device() == at, _ONE_DEVICE)
+    ks = k_new.stride()
+    if ks[3] != 1 or ks != v_new.stride():
         k_new, v_new = k_new.contiguous(), v_new.contiguous()
+        ks = k_new.stride()
     rot_sb = 0
     if cos is not None:
-        _require(cos.shape == (B, n, 128) and sin.shape == (B, n, 128) and cos.dtype == k_new.dtype
-                 and sin.dtype == k_new.dtype, "cos / sin must be [B, n, 128] of the tokens' dtype")
-        if cos.stride(2) != 1 or (n > 1 and cos.stride(1) != 128) or cos.stride() != sin.stride():
+        _require(cos.shape == (B, n, 128) and sin.shape == (B, n, 128) and cos.dtype == dtype
+                 and sin.dtype == dtype, "cos / sin must be [B, n, 128] of the tokens' dtype")
+        _require(cos.get_device() == at and sin.get_device() == at, _ONE_DEVICE)
+        cs = cos.stride()
+        if cs[2] != 1 or (n > 1 and cs[1] != 128) or cs != sin.stride():
             cos, sin = cos.contiguous(), sin.contiguous()
-        rot_sb = cos.stride(0) if B > 1 else 0
-    sb, sh, st, _ = k_new.stride()
-    with _on(k_new.device):
+            cs = cos.stride()
+        rot_sb = cs[0] if B > 1 else 0
+    with _on(dev):
         rc = _lib.load().pkv_window_append(k_new.data_ptr(), v_new.data_ptr(), cos.data_ptr() if cos is not None else None,
-                                           sin.data_ptr() if cos is not None else None, _dtype_code(k_new), B, H, n, sb, sh, st,
-                                           rot_sb, k_win.data_ptr(), v_win.data_ptr(), int(win_pos), k_win.size(2),
-                                           _stream(k_new.device))
+                                           sin.data_ptr() if cos is not None else None, _dtype_code(k_new), B, H, n, ks[0], ks[1],
+                                           ks[2], rot_sb, k_win.data_ptr(), v_win.data_ptr(), int(win_pos), win[2], _stream(dev))
     _lib.check(rc)
 
 
 def _strides(t):
     """Element strides, those of one-element dimensions as 0: they mean nothing and can be any number."""
-    return tuple(st if size > 1 else 0 for st, size in zip(t.stride(), t.shape))
+    st, shape = t.stride(), t.shape
+    return tuple(s if size > 1 else 0 for s, size in zip(st, shape)) if 1 in shape else st
 
 
-def _rows16(t):
-    """Whether the rows of t [.., 128] can be read 16 bytes at a time where they are."""
-    return t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(st % 8 == 0 for st in _strides(t)[:-1])
+def _rows16(t, st):
+    """Whether the rows of t [B, n, 128] or [B, H, n, 128] (strides `st`) can be read 16 bytes at a time where they are."""
+    return st[-1] == 1 and t.data_ptr() % 16 == 0 and (st[0] | st[-3] | st[-2]) % 8 == 0
 
 
-def _encodable(x):
-    """Whether the encoders can read the rows of x [B, H, n, 128] where they are: the limits of pkv_kv_quant_encode_append
-    (token stride; K's head stride for five heads or more, where rows 128 apart have none)."""
-    _, sh, st, _ = _strides(x)
-    return _rows16(x) and st < 1 << 25 and (x.size(1) <= 4 or st == 128 or sh < (1 << 31) - 128)
+def _encodable(x, st):
+    """Whether the encoders can read the rows of x [B, H, n, 128] (strides `st`) where they are: the limits of
+    pkv_kv_quant_encode_append (token stride; K's head stride for five heads or more, where rows 128 apart have none)."""
+    return _rows16(x, st) and st[2] < 1 << 25 and (x.size(1) <= 4 or st[2] == 128 or st[1] < (1 << 31) - 128)
 
 
 def _copy(t):
@@ -497,13 +500,15 @@ def _copy(t):
 
 def _rotary_rows(cos, sin, like):
     """cos / sin as [B, n, 128] tables the kernels read in place: (cos, sin, elements from one sequence's table to the next)."""
-    B, n = like.size(0), like.size(2)
-    _on_device(like.device, cos, sin)
+    B, n, dev, dtype = like.size(0), like.size(2), like.device, like.dtype
+    _require(cos.device == dev and sin.device == dev, _ONE_DEVICE)
     cos, sin = cos.expand(B, n, 128), sin.expand(B, n, 128)
-    _require(cos.dtype == like.dtype and sin.dtype == like.dtype, "cos / sin must be [B, n, 128] of the tokens' dtype")
-    if (n > 1 and cos.stride(1) != 128) or _strides(cos) != _strides(sin) or not _rows16(cos) or not _rows16(sin):
+    _require(cos.dtype == dtype and sin.dtype == dtype, "cos / sin must be [B, n, 128] of the tokens' dtype")
+    cs = _strides(cos)
+    if (n > 1 and cs[1] != 128) or cs != _strides(sin) or not _rows16(cos, cs) or not _rows16(sin, cs):
         cos, sin = _copy(cos), _copy(sin)
-    return cos, sin, _strides(cos)[0]
+        cs = _strides(cos)
+    return cos, sin, cs[0]
 
 
 def kv_quant_encode_append(k, v, n, k_side, v_side, tokens, cos=None, sin=None):
@@ -511,30 +516,31 @@ def kv_quant_encode_append(k, v, n, k_side, v_side, tokens, cos=None, sin=None):
     both.  The rows are read where they are (any strides whose rows start on 16-byte boundaries).  k_side / v_side:
     (rel, bits, stream, used, info, scale, zero) as quant_encode_append takes them.  With cos / sin (tables of k's rows;
     five heads or more) the encoder applies the rotary embedding to K.  Returns the bytes in use of K and V."""
-    B, H = k.size(0), k.size(1)
+    B, H, dev, at = k.size(0), k.size(1), k.device, k.get_device()
     _require(n % 128 == 0 and tokens % 128 == 0, "token counts must be multiples of the block length")
     sides, sizes = [], (ctypes.c_uint64(0), ctypes.c_uint64(0))
     for x, (rel, bits, stream, used, info, scale, zero), per_tile, ctx_blk in ((k, k_side, B * H, 64), (v, v_side, 2 * B * H, 128)):
-        _require(x.is_cuda and x.dim() == 4 and x.size(0) == B and x.size(1) == H and x.size(2) >= n and x.size(3) == 128 and _rows16(x),
+        st = _strides(x)
+        _require(x.is_cuda and x.dim() == 4 and x.size(0) == B and x.size(1) == H and x.size(2) >= n and x.size(3) == 128 and _rows16(x, st),
                  "x must be a device tensor [B, H, n, 128] with rows on 16-byte boundaries")
-        _require(info.is_cuda and info.dtype == torch.uint32 and info.is_contiguous()
+        _require(x.get_device() == at and stream.get_device() == at and info.get_device() == at and scale.get_device() == at and zero.get_device() == at, _ONE_DEVICE)
+        _require(info.dtype == torch.uint32 and info.is_contiguous()
                  and info.numel() >= 2 * ((tokens + n) // ctx_blk * per_tile), "block_info_buffer too small")
         _require(scale.shape == zero.shape == k_side[5].shape and scale.dim() == 2 and scale.size(0) == B and scale.dtype == x.dtype
                  and zero.dtype == x.dtype and scale.is_contiguous() and zero.is_contiguous() and scale.size(1) >= tokens + n,
                  "scale / zero must be contiguous [B, row] with room for the new tokens")
-        _require(stream.is_cuda and stream.dtype == torch.uint8 and stream.is_contiguous() and 0 <= used <= stream.numel(),
+        _require(stream.dtype == torch.uint8 and stream.is_contiguous() and 0 <= used <= stream.numel(),
                  "compressed_buffer must be a contiguous device UInt8 tensor holding the bytes in use")
-        _on_device(k.device, x, stream, info, scale, zero)
         es = scale.element_size()
-        sides.append(_lib.AppendSide(x.data_ptr(), *_strides(x)[:3], stream.data_ptr(), stream.numel(), int(used),
+        sides.append(_lib.AppendSide(x.data_ptr(), *st[:3], stream.data_ptr(), stream.numel(), int(used),
                                      info.data_ptr() + 8 * (tokens // ctx_blk * per_tile), scale.data_ptr() + es * tokens,
                                      zero.data_ptr() + es * tokens, float(rel), int(bits)))
     if cos is not None:
         cos, sin, sides[0].rot_stride_b = _rotary_rows(cos, sin, k)
         sides[0].cos, sides[0].sin = cos.data_ptr(), sin.data_ptr()
-    with _on(k.device):
+    with _on(dev):
         rc = _lib.load().pkv_kv_quant_encode_append(ctypes.byref(sides[0]), ctypes.byref(sides[1]), _dtype_code(k), B, H, n,
-                                                    k_side[5].size(1), ctypes.byref(sizes[0]), ctypes.byref(sizes[1]), _stream(k.device))
+                                                    k_side[5].size(1), ctypes.byref(sizes[0]), ctypes.byref(sizes[1]), _stream(dev))
     _lib.check(rc)
     return int(sizes[0].value), int(sizes[1].value)
 
@@ -554,16 +560,20 @@ def window_cut(k_new, v_new, cos, sin, k_pend, v_pend, k_win, v_win, win_len, st
     _require(k_win.is_contiguous() and v_win.is_contiguous() and k_win.shape == v_win.shape and k_win.dim() == 4
              and k_win.size(0) == B and k_win.size(1) == H and k_win.size(3) == 128 and k_win.dtype == k_new.dtype,
              "windows must be contiguous [B, H, cap, 128] of the tokens' dtype")
-    _on_device(k_new.device, v_new, k_pend, v_pend, k_win, v_win)
-    if _strides(k_new) != _strides(v_new) or not _encodable(k_new) or not _encodable(v_new):
+    dev, at = k_new.device, k_new.get_device()
+    _require(v_new.get_device() == at and k_win.get_device() == at and v_win.get_device() == at
+             and (k_pend is None or k_pend.get_device() == at and v_pend.get_device() == at), _ONE_DEVICE)
+    ks = _strides(k_new)
+    if ks != _strides(v_new) or not _encodable(k_new, ks) or not _encodable(v_new, ks):
         k_new, v_new = _copy(k_new), _copy(v_new)
+        ks = _strides(k_new)
     pend = 64 if k_pend is not None else 0
     buf = win_len - pend
     a = _lib.CutArgs()
     if cos is not None:
         cos, sin, a.rot_stride_b = _rotary_rows(cos, sin, k_new)
         a.cos, a.sin = cos.data_ptr(), sin.data_ptr()
-    empty = lambda rows: torch.empty(B, H, rows, 128, dtype=k_new.dtype, device=k_new.device)
+    empty = lambda rows: torch.empty(B, H, rows, 128, dtype=k_new.dtype, device=dev)
     k_stage, v_stage = k_new, v_new
     if stage and (pend + buf or (cos is not None and not rotary_later)):
         k_stage = empty(stage)
@@ -574,7 +584,7 @@ def window_cut(k_new, v_new, cos, sin, k_pend, v_pend, k_win, v_win, win_len, st
     kp, vp = (empty(64), empty(64)) if pend_out else (None, None)
     kw, vw = (torch.empty_like(k_win), torch.empty_like(v_win)) if win_len else (k_win, v_win)
     a.k_new, a.v_new = k_new.data_ptr(), v_new.data_ptr()
-    a.stride_b, a.stride_h, a.stride_t = _strides(k_new)[:3]
+    a.stride_b, a.stride_h, a.stride_t = ks[:3]
     if pend:
         a.k_pend, a.v_pend = k_pend.data_ptr(), v_pend.data_ptr()
     if win_len:
@@ -584,8 +594,8 @@ def window_cut(k_new, v_new, cos, sin, k_pend, v_pend, k_win, v_win, win_len, st
     a.k_win_out, a.v_win_out, a.win_stride = kw.data_ptr(), vw.data_ptr(), k_win.size(2)
     a.dtype, a.B, a.H, a.n, a.pend, a.buf, a.stage, a.pend_out = _dtype_code(k_new), B, H, n, pend, buf, stage, pend_out
     a.k_rel, a.v_rel = float(k_rel), float(v_rel)
-    with _on(k_new.device):
-        rc = _lib.load().pkv_window_cut(ctypes.byref(a), _stream(k_new.device))
+    with _on(dev):
+        rc = _lib.load().pkv_window_cut(ctypes.byref(a), _stream(dev))
     _lib.check(rc)
     return k_stage, v_stage, kp, vp, kw, vw
 
@@ -927,6 +937,8 @@ def dense_view(k, v, k_win=None, v_win=None, win_len=None):
     by the `win_len` rows in use of the 16-bit windows k_win / v_win [B, H, cap, 128].  One launch."""
     a = AttnArgs()
     like = k["scale"] if k is not None else k_win
+    dev, at = like.device, like.get_device()
+    _require(like.is_cuda, "a compressed cache is on a GPU")
     if k is not None:
         T_c, B = int(k.get("tokens", k["scale"].size(1))), k["scale"].size(0)
         H = int(k["heads"]) if "heads" in k else k["info"].numel() // 2 // (T_c // 64) // B
@@ -936,24 +948,23 @@ def dense_view(k, v, k_win=None, v_win=None, win_len=None):
         a.k_bits, a.v_bits, a.par_stride = int(k["bits"]), int(v["bits"]), k["scale"].size(1)
         for d in (k, v):
             _require(d["scale"].shape == k["scale"].shape and d["zero"].shape == k["scale"].shape and d["scale"].size(1) >= T_c
-                     and d["info"].numel() // 2 >= T_c // 64 * B * H and all(d[f].is_cuda and d[f].is_contiguous()
+                     and d["info"].numel() // 2 >= T_c // 64 * B * H and all(d[f].get_device() == at and d[f].is_contiguous()
                                                                              for f in ("stream", "info", "scale", "zero")),
-                     "stream, info, scale and zero must be contiguous device tensors that hold the tokens in use")
+                     "stream, info, scale and zero must be contiguous tensors on one device that hold the tokens in use")
     else:
         T_c, H, B = 0, k_win.size(1), k_win.size(0)
     T_w = 0
     if k_win is not None:
         T_w = k_win.size(2) if win_len is None else int(win_len)
-        _require(k_win.is_cuda and v_win.is_cuda and k_win.is_contiguous() and v_win.is_contiguous() and k_win.shape == v_win.shape
+        _require(k_win.get_device() == at and v_win.get_device() == at and k_win.is_contiguous() and v_win.is_contiguous() and k_win.shape == v_win.shape
                  and k_win.shape[:2] == (B, H) and k_win.size(3) == 128 and 0 <= T_w <= k_win.size(2) and k_win.dtype == like.dtype
-                 and v_win.dtype == like.dtype, "window tensors must be contiguous [B, H, cap, 128] of the cache's dtype")
+                 and v_win.dtype == like.dtype, "window tensors must be contiguous [B, H, cap, 128] of the cache's dtype, all on one device")
         a.k_win, a.v_win, a.win_stride = _ptr(k_win), _ptr(v_win), k_win.size(2)
-    _on_device(like.device, k_win, v_win, *(d[f] for d in (k, v) if d is not None for f in ("stream", "info", "scale", "zero")))
     a.B, a.Hkv, a.T_c, a.T_w, a.dtype = B, H, T_c, T_w, _dtype_code(like)
-    k_out = torch.empty(B, H, T_c + T_w, 128, dtype=like.dtype, device=like.device)
+    k_out = torch.empty(B, H, T_c + T_w, 128, dtype=like.dtype, device=dev)
     v_out = torch.empty_like(k_out)
-    with _on(like.device):
-        rc = _lib.load().pkv_dense_view(ctypes.byref(a), _ptr(k_out), _ptr(v_out), _stream(like.device))
+    with _on(dev):
+        rc = _lib.load().pkv_dense_view(ctypes.byref(a), _ptr(k_out), _ptr(v_out), _stream(dev))
     _lib.check(rc)
     return k_out, v_out
 

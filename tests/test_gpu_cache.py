@@ -452,6 +452,11 @@ def test_tensors_on_another_device_are_refused_before_a_launch(cuda):
         vs[f] = vs[f].cpu()
         with pytest.raises(RuntimeError, match="one device"):
             ops.kv_quant_encode_append(k, v, 256, ks, vs, 0)
+        with pytest.raises(RuntimeError, match="one device"):
+            ops.dense_view(ke, dict(ve, **{("scale", "zero")[f - 5]: vs[f]}))
+    for kw, vw in ((win, host), (host, win)):
+        with pytest.raises(RuntimeError, match="one device"):
+            ops.dense_view(ke, ve, kw, vw, 1)
 
 
 @pytest.mark.parametrize("side", ["k", "v"])

@@ -42,7 +42,8 @@ def test_rows_that_the_encoders_cannot_reach_are_copied():
     for H, sh, st, want in ((5, 1 << 31, 128, True), (5, 1 << 31, 256, False), (4, 1 << 31, 256, True), (5, (1 << 31) - 136, 256, True),
                             (5, (1 << 31) - 128, 256, False), (5, 128, 1 << 25, False), (4, 128, 1 << 25, False),
                             (5, 128, (1 << 25) - 8, True), (5, 128, 1284, False), (1, 7, 256, True)):
-        assert ops._encodable(rows(H, sh, st)) == want, (H, sh, st)
+        x = rows(H, sh, st)
+        assert ops._encodable(x, ops._strides(x)) == want, (H, sh, st)
 
 
 def test_import_without_the_private_torch_functions():
