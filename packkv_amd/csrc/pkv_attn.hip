@@ -512,13 +512,24 @@ __global__ void __launch_bounds__(256) attn_window_kernel(const AttnParams p) {
 // ---- merge of a head's partials by the last of its `arrivals` workgroups to get here (async-copy kernel) ----
 // Saves the launch of the merge kernel, its run and the gap in front of it.  The price is three trips past the L2s -- a
 // workgroup's stores, its count, the last one's read of all partials -- and that the counts on one address retire one
-// after the other: a decode loop over 509 tokens (at most 6 workgroups a head) 1783 -> 1626 us, one over 32 x 8192
-// (4 workgroups) 4880 -> 4838, but one step of 32 heads x 4096 tokens (32 workgroups) 15.5 -> 16.5 us, one of
-// 3 x 8 heads x 11008 + 137 (24) 25.2 -> 27.2.  So: up to eight workgroups a head (kMergeArrivals).
+// after the other.  merge_pays says where the price is lower.  4-bit fp16 steps, us per step in a graph of 40 (and launched
+// one by one), with the merge launch -> merged here; `pairs` = sequences x KV heads:
+//   several tiles a workgroup, 4 to 8 workgroups a head: always.  Groups of 4: 128 pairs x 256 tiles 112.5 -> 111.2, x 32
+//     26.3 -> 25.3 (25.4 -> 24.5), 256 x 32 39.7 -> 38.2 (39.0 -> 37.6); groups of 8: 128 x 16 24.9 -> 24.4, 256 x 64 87.4 -> 86.1
+//   one tile each, when all workgroups of a head arrive at once and nothing hides the trips: groups of 8 never (two heads a
+//     wavefront one after the other: 8 pairs x 6 tiles 12.2 -> 12.9, 128 x 2 12.8 -> 13.2); else up to 14 pairs (14 x 8 10.2 ->
+//     10.5 (10.7 -> 10.5), 8 x 4 9.9 -> 9.7 (10.5 -> 10.0)) and from 72 on (72 x 8 12.7 -> 12.7 (13.0 -> 12.6), 128 x 4 11.5 -> 11.3);
+//     in between up to four workgroups (32 x 4 10.0 -> 10.2 (10.7 -> 10.5), but 32 x 8 10.2 -> 10.9 (10.7 -> 11.2), 64 x 8 11.2 -> 12.2
+//     (11.8 -> 12.3)), with groups of 4 and more than 32 pairs three (64 x 3 10.2 -> 10.5 (10.6 -> 10.6), x 4 10.2 -> 10.7 (10.7 -> 10.8)).
+//   32 workgroups a head (32 heads x 4096 tokens) 15.5 -> 16.5, 24 (3 x 8 x 11008 + 137) 25.2 -> 27.2: hence at most eight.
 // Every workgroup has written its partials through to memory (part_store) and waited for that before it counts itself;
 // the reader's loads go past its own L2.  No workgroup waits for another.  Lane = two adjacent channels; a wavefront merges
 // a head of its own when the group has four or more, otherwise the wavefronts share a head's partials and meet in LDS.
 constexpr int kMergeArrivals = 8;
+static bool merge_pays(int G, int pairs, int nsplit, int tiles_per_split) {
+    if (tiles_per_split > 1) return true;
+    return G <= 4 && (pairs <= 14 || pairs >= 72 || nsplit <= (G == 4 && pairs > 32 ? 3 : 4));
+}
 template <int G>
 __device__ __forceinline__ void merge_head(const AttnParams &p, uint8_t *lds, int h, int b, uint32_t arrivals) {
     constexpr int WPH = G >= 4 ? 1 : 4 / G;          // wavefronts per head
@@ -934,7 +945,8 @@ int pkv::attn_decode_impl(const pkv_attn_args *a, float *ms_out, hipStream_t s, 
     p.batch_shift = 1;                     // a member asks for 1 / (2 nsplit) of what is left: ceil(log2(2 nsplit))
     while ((1 << p.batch_shift) < 2 * nsplit) p.batch_shift++;
     // few workgroups a head: the last of them merges (merge_head)
-    p.merge = dma_path && p.nparts > 1 && nsplit + win_members <= kMergeArrivals && 3 * (int64_t)a->B * a->Hkv <= kAttnCounters;
+    p.merge = dma_path && p.nparts > 1 && nsplit + win_members <= kMergeArrivals && merge_pays(G, pairs, nsplit, tps) &&
+              3 * (int64_t)a->B * a->Hkv <= kAttnCounters;
     p.counters = nullptr;
     // Partials and counters: the stream's own scratch, or the static array -- for pkv_attn_decode_noalloc, and for a
     // stream that is capturing a graph before it has scratch of its own.

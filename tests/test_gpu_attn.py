@@ -558,7 +558,17 @@ def test_attn_decode_of_nearly_full_narrow_blocks(cuda, hq, rel, bits):
     (1, 7, 1, 128 * 4, 200, 0.1),      # seven
     (40, 8, 8, 128 * 6, 320, 0.1),     # the window shared by the splits: two partials a workgroup
     (16, 32, 8, 128 * 8, 150, 0.1),    # ... 16 partials
-    (2, 8, 4, 128 * 5, 64, 0.05)])     # 5-bit codes
+    (2, 8, 4, 128 * 5, 64, 0.05),      # 5-bit codes
+    (128, 8, 1, 128 * 8, 0, 0.1),      # eight query heads, two tiles a workgroup: merged by the last of four
+    (128, 5, 1, 128 * 8, 90, 0.1),     # ... of five in eight slots
+    (14, 4, 1, 128 * 5, 0, 0.1),       # one tile each, five workgroups a head: up to 14 (sequence, KV head) pairs merged so,
+    (15, 4, 1, 128 * 5, 33, 0.1),      # from 15 on by a launch;
+    (32, 4, 1, 128 * 4, 0, 0.1),       # four up to 32 pairs merged so,
+    (33, 4, 1, 128 * 4, 0, 0.1),       # with more by a launch,
+    (33, 2, 1, 128 * 4, 0, 0.1),       # but not with two query heads
+    (33, 4, 1, 128 * 3, 33, 0.1),      # or three workgroups;
+    (71, 4, 1, 128 * 4, 0, 0.1),       # by a launch
+    (72, 4, 1, 128 * 4, 0, 0.1)])      # and from 72 pairs on by the last workgroup again
 def test_attn_decode_merged_by_its_last_workgroup(cuda, dtype, B, Hq, Hkv, T, Tw, rel):
     """Partials merged inside the attention kernel, around its limits, against fp64 attention; again with fp32 output,
     through the static scratch, and 20 times in a row: the counters are left clear and the result does not depend on which
