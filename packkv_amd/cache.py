@@ -102,9 +102,12 @@ class _Layer:
 
 
 # A prompt whose keys are at least so many bytes has them rotated by the encoder as it reads them (kernels for five heads or
-# more) instead of being rotated into a buffer of their own first: 32 x 8 heads x 8192 tokens (bf16, 512 MiB) 297 us against
-# 396.  A small one waits for the tables in every round: 2 x 8 x 2816 (11 MiB) 29.6 against 27.6.
-ROTATE_IN_ENCODER = 32 << 20
+# more) instead of being rotated into a buffer of their own first.  That saves the keys one trip to memory and back, and costs
+# the encoder a wait for the tables in every round, which a prompt that the caches hold does not pay back.  First update of a
+# layer, us, in the encoder / before it: 2 x 8 heads x 8342 tokens (fp16, 33 MiB of keys) 119 / 109, 2 x 32 x 2198 (bf16, 34 MiB)
+# 148 / 134, 8 x 32 x 1174 (bf16, 73 MiB) 151 / 146, 8 x 8 x 5270 (82 MiB) fp16 137 / 149, bf16 158 / 163, 8 x 8 x 16534 (258 MiB,
+# bf16) 339 / 402, 32 x 8 x 8192 (bf16, 512 MiB; the encode alone) 297 / 396.
+ROTATE_IN_ENCODER = 80 << 20
 
 
 class PackKVCompressedCache:
