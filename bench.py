@@ -2,7 +2,7 @@
 """Benchmark of the PackKV hot path on one MI355X.
 
 A step = one fused decompress-attention decode (one layer, one query token per sequence) over a
-compressed KV cache resident in HBM.  Workload (BASELINE.json configs[1]): batch 16, 32 query /
+compressed KV cache resident in HBM.  Workload: batch 16, 32 query /
 8 KV heads, head_dim 128, 32768 cached tokens per sequence, fp16, K ~ N(0,1) with four outlier
 channels x10, V ~ N(0,1), per-token quantisation at relative step 0.1, 64-token quant blocks.
 
@@ -54,16 +54,16 @@ def parse():
                     help="do not stop when the kernel disagrees with the plain kernel (development builds that switch "
                          "parts of the kernel off, -DPKV_ATTN_PROBE: their results are wrong by design)")
     ap.add_argument("--no-config-legs", action="store_true",
-                    help="skip the configs[4] loop and the configs[3] decoder legs of the default run")
+                    help="skip the 32-layer loop and the decoder legs of the default run")
     ap.add_argument("--layers", type=int, default=0,
                     help="instead of the single-layer step: a decode loop over this many layers through the growing "
-                         "compressed cache (configs[4] is --layers 32 --batch 4 --ctx 131072); prints its own JSON line")
+                         "compressed cache (--layers 32 --batch 4 --ctx 131072, say); prints its own JSON line")
     ap.add_argument("--e2e", action="store_true",
                     help="instead of the single-layer step: greedy decoding on a random-init decoder of Qwen3-8B shape "
-                         "through the compressed cache (configs[3]: --e2e --batch 32 --ctx 8192 --steps 256); --e2e-layers "
+                         "through the compressed cache (--e2e --batch 32 --ctx 8192 --steps 256, say); --e2e-layers "
                          "and --e2e-dense-steps scale it; prints its own JSON line")
     ap.add_argument("--sweep", action="store_true",
-                    help="instead of the single-layer step: the repack + bit-pack sweep of configs[2] (--sweep --hkv 8 "
+                    help="instead of the single-layer step: the repack + bit-pack sweep of one layer (--sweep --hkv 8 "
                          "--ctx 16384): compression ratios over pack sizes 16..256, code widths 2..8 bits and the three "
                          "repacking methods, and the block codec's encode / decode rates per width; prints its own JSON line")
     ap.add_argument("--e2e-layers", type=int, default=36)
@@ -88,7 +88,7 @@ def event_time_ms(torch, fn, iters):
 
 
 def cpu_baseline(torch, args, k1, v1, q1, threads=None, passes=5, warm=2):
-    """Decompress-then-attend for a sample of the sequences in PyTorch CPU ops (the checker's restatement of
+    """Decompress-then-attend for a sample of the sequences in PyTorch CPU ops (the oracle's restatement of
     utils/compute.py:173-179 + models/llama.py:189-212), median of `passes` after `warm` warm-ups, scaled to the
     batch: about ten seconds of host work at the default workload.  threads: torch's thread count for the
     measurement (None = all the cores torch uses by default)."""
@@ -208,7 +208,7 @@ def decode_loop(torch, args, dev):
 
 
 def e2e_decode(torch, args, dev):
-    """a random-init decoder of Qwen3-8B shape (bf16 weights ~ N(0, 0.02)), a random-token prompt of
+    """A random-init decoder of Qwen3-8B shape (bf16 weights ~ N(0, 0.02)), a random-token prompt of
     --ctx tokens per sequence, --steps greedy tokens; the cache compresses a 64-token cut whenever its 16-bit buffer
     reaches 192 tokens.  Reports decode tokens/s of the fused path, the prompt pass, the bytes the caches hold, and
     a few steps of the reference's decompress-then-attend on the same cache for scale."""
@@ -270,7 +270,7 @@ SWEEP_PACKS = (16, 32, 64, 128, 256)
 
 
 def pack_sweep(torch, H, T, dev, rels=SWEEP_RELS, packs=SWEEP_PACKS, time_codec=True, kv=None):
-    """one layer of H KV heads x 128 x T tokens, K with a per-channel scale drawn log-uniform in
+    """One layer of H KV heads x 128 x T tokens, K with a per-channel scale drawn log-uniform in
     [0.1, 10], V ~ N(0, 1).  For every error bound (one per code width) the tensors are quantised once; every
     (pack size, repacking method) is then priced with the reference's size model (`repack_and_encode`,
     utils/compute.py:329-357: integers, so the ratios are the reference's wherever its token order is defined),
@@ -296,7 +296,7 @@ def pack_sweep(torch, H, T, dev, rels=SWEEP_RELS, packs=SWEEP_PACKS, time_codec=
                 rows.append({"rel": rel, "bits": bits, "pack": pack, "method": method, "block": bs,
                              "k_bytes": k_aft, "v_bytes": v_aft, "k_cr": fp16 / k_aft, "v_cr": fp16 / v_aft})
         if time_codec:
-            # the real block codec at every pack length (16 = the reference's format; longer packs = this build's
+            # the real block codec at every pack length (16 = the reference's format; longer packs = an
             # extension of it): stream bytes - 8 per block equal the size model's bytes of the "none" rows above
             back = torch.empty_like(kc)
             gbs = lambda ms: T * hid / (ms * 1e-3) / 1e9
@@ -367,7 +367,7 @@ def gemv_surface(torch, ops, synth, dev):
 def main():
     args = parse()
     if args.gpus != 1:
-        print("bench.py measures one GPU: this build has no multi-GPU path (--gpus %d refused)" % args.gpus,
+        print("bench.py measures one GPU: this library has no multi-GPU path (--gpus %d refused)" % args.gpus,
               file=sys.stderr)
         sys.exit(2)
     import torch
@@ -499,7 +499,7 @@ def main():
             "median_repack_ms": rp_ms, "median_repack_gbs": 5 * Tc * hidden / (rp_ms * 1e-3) / 1e9,   # V read twice, K once, both written
             "bit_pack_size_ms": bp_ms, "bit_pack_size_gbs": Tc * hidden / (bp_ms * 1e-3) / 1e9,
         }
-        # packs longer than 16 tokens (this build's extension of the format) on the same 2 x 512 MiB of codes: the real
+        # packs longer than 16 tokens (an extension of the format) on the same 2 x 512 MiB of codes: the real
         # codec at every pack length, beside the 16-token codec's figures above (K decode 1.0 = as fast as that one)
         long_packs = {}
         back = torch.empty_like(codes)
@@ -577,8 +577,8 @@ def main():
         del dst
 
     if not args.no_extras and default_workload:
-        # configs[1] names three error bounds; the line above is the middle one.  The other two on the same tensors:
-        # fused encode, unpack and the decode step (5-bit codes at 0.05 are this build's extension of the format)
+        # Three error bounds are of use; the line above is the middle one.  The other two on the same tensors:
+        # fused encode, unpack and the decode step (5-bit codes at 0.05 are an extension of the format)
         other = {}
         for rel2 in (0.05, 0.2):
             b2 = ops.bits_for_rel(rel2)
@@ -600,7 +600,7 @@ def main():
                 "ratio_k": fp16_bytes / 2 / ke2["size"], "ratio_v": fp16_bytes / 2 / ve2["size"]}
             del ke2, ve2, codes2
         result["other_error_bounds"] = other
-        # the same bytes as fewer, longer sequences (one layer of configs[4] is 4 x 131072 tokens): the tensors read as
+        # the same bytes as fewer, longer sequences (4 x 131072 tokens among them): the tensors read as
         # [B / f, Hkv, f * Tc, 128], encoded and attended at that shape -- more members share a KV head there
         longer = {}
         for f in (4, 16):
@@ -634,8 +634,8 @@ def main():
         result["cpu_baseline"] = None
 
     if not args.no_extras and not args.no_config_legs and default_workload:
-        # the two configurations that run more than one layer, at their own sizes and in this same run: configs[4]'s
-        # loop over 32 layers of the growing cache and configs[3]'s greedy decode through the decoder (both have flags
+        # the two configurations that run more than one layer, at their own sizes and in this same run: the
+        # loop over 32 layers of the growing cache and the greedy decode through the decoder (both have flags
         # of their own for longer runs: --layers / --e2e).  A leg that fails reports its error instead of a figure.
         del k, v, kc, vc, ke, ve, q, out
         import copy

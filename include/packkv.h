@@ -222,7 +222,7 @@ int pkv_window_cut(const pkv_cut_args *args, pkv_stream_t s);
  *   of the token's V codes over all hidden_dim channels.  Equal medians keep their original order
  *   (the reference leaves that order to torch.sort's backend).  perm[blk * block_size + r] is
  *   the index inside the block of the token that moves to position r. */
-/* Median repacking inside the fused encode (north-star "quantize, token repack, bit-pack" as one encode; reference
+/* Median repacking inside the fused encode (quantize, token repack and bit-pack as one encode; reference
  * order utils/compute.py:329-357: quantise, repack, bit-pack): no code matrix is formed.
  * pkv_median_order: the permutation pkv_median_repack would produce for V [B, H, T, 128] quantised at `rel` -- the
  *   medians are counted straight from V (every value quantised in registers).  H <= 8, bits 2..6.  scale_out /

@@ -26,7 +26,7 @@ _u32p = ctypes.POINTER(ctypes.c_uint32)
 
 
 def build(with_ref=True):
-    """Compile the checker libraries (the restated C codec, and the reference build
+    """Compile the oracle's libraries (the restated C codec, and the reference build
     when the reference checkout is present)."""
     subprocess.check_call(["make", "-s", "-C", _HERE, "oracle"])
     if with_ref:
@@ -52,7 +52,7 @@ class _Codec:
         ctx_len, hidden = codes.shape
         nblk = (ctx_len // ctx_blk) * (hidden // hid_blk)
         # the reference sizes the buffer like the code matrix (evaluation/evaluation.py:426); widths above 4
-        # (this build's extension) can exceed that, so take the worst case when it is larger
+        # (an extension of the format) can exceed that, so take the worst case when it is larger
         bound = int(self.bound(int(is_k), ctx_blk, hid_blk, W)) if self.bound is not None else 0
         stream = np.zeros(max(ctx_len * hidden, nblk * bound), dtype=np.uint8)
         info = np.zeros((nblk, 2), dtype=np.uint32)
@@ -101,7 +101,7 @@ def block_bound(is_k, ctx_blk, hid_blk, W):
     return int(oracle().lib.pkv_oracle_block_bound(int(is_k), ctx_blk, hid_blk, W))
 
 
-# ---- packs longer than 16 tokens (this build's extension of the format; see packkv_oracle.c) ----
+# ---- packs longer than 16 tokens (this library's extension of the format; see packkv_oracle.c) ----
 
 def long_block_bound(pack_len, W):
     lib = oracle().lib

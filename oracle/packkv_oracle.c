@@ -20,7 +20,7 @@
  * stream + block_info for W in {2,3,4}), the committed golden vectors made
  * from that build, and closed-form block sizes / byte patterns in the tests.
  *
- * W in 5..8 is a FORMAT EXTENSION of this build (the reference stops at 16 * W <= 64 bits
+ * W in 5..8 is a FORMAT EXTENSION of this library (the reference stops at 16 * W <= 64 bits
  * per pack word, k_encode_cpu.cpp:211): the same layout rules with pack words of up to 128
  * bits.  No reference exists for it -- parity unpinned; it is pinned by encode -> decode round
  * trips, by the closed-form block sizes and by the reference's analytic size model
@@ -295,7 +295,7 @@ int pkv_oracle_decode(int is_k, const uint8_t *stream, const uint32_t *block_inf
 
 /* ------------------------------------------------- packs longer than 16 tokens --
  *
- * FORMAT EXTENSION of this build (the reference fixes PACK_ELE_NUM = 16, include/static_def.h:6, and only its
+ * FORMAT EXTENSION of this library (the reference fixes PACK_ELE_NUM = 16, include/static_def.h:6, and only its
  * analytic size model, utils/compute.py:272-297, knows other pack lengths).  No reference exists for it -- parity
  * unpinned; it is pinned by the definition below restated with big integers in the tests, by the closed-form size
  * (stream bytes - 8 per block == the size model's bytes), by round trips, and by P = 16 reproducing the format above.

@@ -199,7 +199,7 @@ __device__ __forceinline__ void pair_windows(const UnitPairs &u, uint32_t win01[
     }
 }
 
-// Widths 5 and 6 (this build's extension of the format): a quarter of a pack no longer fits a 16-bit lane, so the
+// Widths 5 and 6 (this library's extension of the format): a quarter of a pack no longer fits a 16-bit lane, so the
 // windows hold TWO tokens each.  e01[e] = tokens 2e, 2e+1 of packs 0 and 1 in the low / high 16 bits (token 2e on
 // top), e23 likewise; bits above 2*len in a half are other tokens' fields, every consumer masks.
 struct UnitWide {

@@ -3,7 +3,7 @@
 K ~ N(0,1) with four fixed outlier channels per head scaled x10 (or a per-channel log-uniform
 scale), V ~ N(0,1), q ~ N(0,1); 16-bit storage.  Generated on the requested device with a
 seeded torch.Generator so that a run is reproducible; small test cases generate on the CPU and
-copy, so that the CPU checker and the GPU see identical bits.
+copy, so that the CPU oracle and the GPU see identical bits.
 """
 import math
 

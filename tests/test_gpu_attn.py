@@ -379,7 +379,7 @@ def test_stream_release_gives_the_scratch_back(cuda):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_attn_decode_wide_codes(cuda, rel, bits, dtype):
     """rel 0.05 gives 22 code levels, rel 0.03 gives 35: 5- and 6-bit codes, outside the reference's format and
-    inside this build's extension (three-kernel encode).  The asynchronous-copy kernel takes them with two-token
+    inside this library's extension (three-kernel encode).  The asynchronous-copy kernel takes them with two-token
     windows (variant 0); the plain kernel (variant 1) is the cross-check.  Same contract against
     decompress-then-attend, with a tail window and a context that is not a multiple of the split size."""
     B, Hq, Hkv, T, Tw = 2, 16, 4, 1152, 70

@@ -192,7 +192,7 @@ def test_round_trip_at_bench_scale(cuda):
 
 @pytest.mark.parametrize("W", [5, 6, 7, 8])
 def test_wide_codes_stream_matches_restatement(cuda, oracle_codec, W):
-    """Widths 5..8 are this build's extension of the format (pack words of up to 128 bits; the reference's
+    """Widths 5..8 are this library's extension of the format (pack words of up to 128 bits; the reference's
     templates stop at 4).  There is no reference for them: the device codec is held to the restated C codec byte for
     byte, to an exact round trip, and the stream size to the closed form (payload 2 * len bytes per pack, W + LB bits
     of metadata per pack, 8 header bytes per block)."""
@@ -222,7 +222,7 @@ def test_wide_codes_stream_matches_restatement(cuda, oracle_codec, W):
         assert torch.equal(back, d)
 
 
-# ---- packs longer than 16 tokens (this build's extension of the format; the oracle's restatement of it is pinned
+# ---- packs longer than 16 tokens (this library's extension of the format; the oracle's restatement of it is pinned
 # on the CPU by tests/test_oracle_codec.py) ---------------------------------------------------------------------
 
 def _gpu_encode_p(cuda, is_k, c, P, W):

@@ -126,7 +126,7 @@ def test_repacked_codes_encode_and_round_trip(cuda):
 
 
 def test_full_size_properties(cuda):
-    """configs[2] shape (8 KV heads x 128 x 16384 tokens): the oracle is slow there, so check what must hold:
+    """The sweep's shape (8 KV heads x 128 x 16384 tokens): the oracle is slow there, so check what must hold:
     perm is a permutation inside every block, rows move with it, medians come out non-increasing, and repacking
     leaves the multiset of codes (hence the histogram and W) unchanged."""
     T, hid, bs = 16384, 1024, 64

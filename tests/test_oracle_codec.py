@@ -122,7 +122,7 @@ def test_unsupported_shapes_raise(oracle_codec):
         oracle_codec.encode(0, c, 64, 64, 3)
 
 
-# ---- packs longer than 16 tokens: this build's extension of the format (no reference: parity unpinned) ----------
+# ---- packs longer than 16 tokens: this library's extension of the format (no reference: parity unpinned) ----------
 # Pinned by (i) the definition restated here with Python integers (a different formulation from the C restatement's
 # bit writes), (ii) the reference's size model, (iii) P = 16 reproducing the reference-pinned format, (iv) round trips.
 
