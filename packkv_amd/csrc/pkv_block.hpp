@@ -167,6 +167,51 @@ __device__ __forceinline__ void unit_codes(const uint8_t *blk, uint32_t unit_off
     }
 }
 
+// The same for a width known at compile time (2..4), for consumers that multiply: `sink(k, c01, c23)` gets the codes of
+// slots 0 | 1 and 2 | 3 at token k as 16-bit lanes.  Such a lane read as a half is the code times 2^-24 (a subnormal), which
+// v_fma_mix_f32 multiplies exactly: no conversion.  (Not the offsets alone with the minima multiplied apart: a factor that is
+// infinite would meet an offset of zero.)
+template <int W, class Sink>
+__device__ __forceinline__ void unit_fields(const uint8_t *blk, uint32_t unit_off, int t, Sink sink) {
+    static_assert(W >= 2 && W <= 4, "pack words of up to 64 bits");
+    typedef unsigned short u16pair __attribute__((ext_vector_type(2)));
+    constexpr int LB = len_field_bits(W);
+    const uint32_t minsw = lds_meta_word(blk + unit_off, t, W);
+    const uint32_t lensw = lds_meta_word(blk + unit_off + 16 * W, t, LB);
+    uint32_t len[4], mn[4], off[4], payload;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        len[i] = (lensw >> (i * LB)) & ((1u << LB) - 1u);
+        mn[i] = (minsw >> (i * W)) & ((1u << W) - 1u);
+    }
+    pack_offsets(len, off, payload);
+    uint32_t hlf[4][2];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint64_t w = lds_load64(blk, unit_off + 16u * (W + LB) + off[i]);
+        hlf[i][0] = W < 4 ? __builtin_amdgcn_alignbit((uint32_t)(w >> 32), (uint32_t)w, 8u * len[i]) : (uint32_t)(w >> (8u * len[i]));   // tokens 0..7
+        hlf[i][1] = (uint32_t)w;                                                                                                         // tokens 8..15
+    }
+    const uint32_t len01 = len[0] | (len[1] << 16), len23 = len[2] | (len[3] << 16);
+    const u16pair mask01 = __builtin_bit_cast(u16pair, ((1u << len[0]) - 1u) | (((1u << len[1]) - 1u) << 16));
+    const u16pair mask23 = __builtin_bit_cast(u16pair, ((1u << len[2]) - 1u) | (((1u << len[3]) - 1u) << 16));
+    const u16pair mn01 = __builtin_bit_cast(u16pair, mn[0] | (mn[1] << 16)), mn23 = __builtin_bit_cast(u16pair, mn[2] | (mn[3] << 16));
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        uint32_t qd[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) qd[i] = (q & 1) ? hlf[i][q >> 1] : hlf[i][q >> 1] >> (4u * len[i]);
+        const u16pair w01 = __builtin_bit_cast(u16pair, __builtin_amdgcn_perm(qd[1], qd[0], 0x05040100u));       // tokens 4q..4q+3 of packs 0 | 1
+        const u16pair w23 = __builtin_bit_cast(u16pair, __builtin_amdgcn_perm(qd[3], qd[2], 0x05040100u));
+#pragma unroll
+        for (int pp = 0; pp < 4; pp++) {
+            const u16pair s01 = __builtin_bit_cast(u16pair, len01 * (uint32_t)(3 - pp)), s23 = __builtin_bit_cast(u16pair, len23 * (uint32_t)(3 - pp));
+            const u16pair d01 = (w01 >> s01) & mask01, d23 = (w23 >> s23) & mask23;
+            sink(4 * q + pp, __builtin_bit_cast(uint32_t, (u16pair)(d01 + mn01)), __builtin_bit_cast(uint32_t, (u16pair)(d23 + mn23)));
+        }
+    }
+}
+
 // Decode one unit whose bytes start at blk[unit_off] into the LDS tile.
 template <bool IS_K>
 __device__ __forceinline__ void unit_decode(const uint8_t *blk, uint32_t unit_off, int unit, int t,

@@ -23,94 +23,140 @@ __device__ __forceinline__ uint16_t st16(float x, int dtype) {
     return (uint16_t)(u >> 16);
 }
 
-// grid = number of K blocks, threads = 2 * ctx_blk (one half-wavefront per round).  (Padding the tile rows so
-// that the dot product's reads spread over the LDS banks changes nothing measurable: the kernel's time is the
-// latency chain stage -> decode -> dot of many small workgroups.)
-__global__ void kq_kernel(const uint8_t *__restrict__ stream, uint64_t stream_bytes, const uint32_t *__restrict__ info,
-                          const uint16_t *__restrict__ q, uint16_t *__restrict__ kq_out, int ctx_len,
-                          int hidden_dim, int ctx_blk, int nunits, int W, uint32_t blk_cap, int dtype,
-                          int q_interleaved) {
-    extern __shared__ __align__(16) uint8_t lds[];
-    __shared__ float qs[kHeadDim];
-    uint8_t *tile = lds;
-    uint8_t *blk = lds + ctx_blk * kHeadDim;
-    const int n_hid = hidden_dim / kHeadDim;
-    const uint32_t b = blockIdx.x;
-    const uint32_t cb = b / n_hid, hb = b % n_hid;
-    uint32_t off, size;
-    block_span(info, b, blk_cap, stream_bytes, off, size);
-    const uint32_t phase = stage_to_lds(stream + off, size, blk, threadIdx.x, blockDim.x);
-    for (int c = threadIdx.x; c < kHeadDim; c += blockDim.x) {
-        int src = c;
-        if (q_interleaved) {   // evaluation/evaluation.py:465-468
-            const int l = c >> 2, i = c & 3;
-            src = i < 2 ? 2 * l + i : 64 + 2 * l + (i - 2);
-        }
-        qs[c] = ld16(q, (size_t)hb * kHeadDim + src, dtype);
-    }
-    __syncthreads();
-    block_decode<true>(blk, phase, nunits, W, tile, kHeadDim);
-    __syncthreads();
-    const int r = threadIdx.x >> 1, half = threadIdx.x & 1;
-    float acc = 0.f;
-    if (r < ctx_blk) {
-        const uint32_t *row = reinterpret_cast<const uint32_t *>(tile + r * kHeadDim + half * 64);
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const uint32_t w = row[i];
-            const float *qq = qs + half * 64 + 4 * i;
-            acc += qq[0] * (float)(w & 0xFFu) + qq[1] * (float)((w >> 8) & 0xFFu) +
-                   qq[2] * (float)((w >> 16) & 0xFFu) + qq[3] * (float)(w >> 24);
-        }
-    }
-    acc += __shfl_xor(acc, 1, 64);
-    if (half == 0 && r < ctx_blk)
-        kq_out[(size_t)hb * ctx_len + (size_t)cb * ctx_blk + r] = st16(acc, dtype);
+// A wavefront decodes a block by itself: the block's bytes go to an LDS slot of its own, its two halves parse a unit each
+// (unit_fields) and the codes meet q or w in registers as they come out -- no code tile, no barrier.  What bounds both
+// kernels is instruction issue (about 300 vector instructions per wavefront and pair of units: windows, shifts and masks
+// 1.75 per code pair, minima 0.5, products 1 per code) behind the chain block_info -> block bytes -> parse; with a workgroup
+// of two wavefronts per block the chain had a barrier between its links, the tile was written and read back, and a code
+// cost a conversion.
+__device__ __forceinline__ void wave_lds_order() {         // LDS serves a wavefront's accesses in order
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// grid = number of V blocks, threads = 2 * hid_blk (one half-wavefront per segment; 8 * hid_blk / 4 in the dot product).
-__global__ void wv_kernel(const uint8_t *__restrict__ stream, uint64_t stream_bytes, const uint32_t *__restrict__ info,
-                          const uint16_t *__restrict__ w, float *__restrict__ wv_out, int ctx_len,
-                          int hidden_dim, int hid_blk, int nunits, int W, uint32_t blk_cap, int dtype) {
+// f.x .. f.w times the four codes c01 | c23 (unit_fields) times 2^-24: products exact, fp32 sums.  The sum is scaled
+// back and not the factors: 2^24 times a large bf16 value would overflow.
+constexpr float kFieldUnit = 16777216.f;                   // 2^24
+typedef _Float16 half_pair __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float dot4(uint32_t c01, uint32_t c23, const float4 f) {
+    const half_pair a = __builtin_bit_cast(half_pair, c01), b = __builtin_bit_cast(half_pair, c23);
+    float s = (float)a[1] * f.y;
+    s = fmaf((float)a[0], f.x, s);
+    s = fmaf((float)b[0], f.z, s);
+    return fmaf((float)b[1], f.w, s);
+}
+__device__ __forceinline__ float dot4(uint32_t c01, uint32_t c23, const float4 f, float acc) {
+    const half_pair a = __builtin_bit_cast(half_pair, c01), b = __builtin_bit_cast(half_pair, c23);
+    acc = fmaf((float)a[0], f.x, acc);
+    acc = fmaf((float)a[1], f.y, acc);
+    acc = fmaf((float)b[0], f.z, acc);
+    return fmaf((float)b[1], f.w, acc);
+}
+
+// K . q: wavefront per K block (`wpw` of them to a workgroup, `slot` bytes of LDS each), a half per round, lane = four
+// channels.  A token's 32 sums of four channels are turned through LDS so that a lane adds sixteen of them, one after the
+// other from the lowest channel on: kq comes out of sums that nearly cancel (q . code against the zero points), so a last
+// bit here that changed with the order of the sum would show there.
+// 65536 tokens x 8 heads at 4 bits: 12.3 us, 15.3 with a workgroup and a code tile per block.
+constexpr int kKqTok = 20, kKqRow = 16 * kKqTok + 16;      // floats from token to token and from row of lanes to row: no bank conflicts
+template <int W>
+__global__ void __launch_bounds__(256) kq_kernel(const uint8_t *__restrict__ stream, uint64_t stream_bytes, const uint32_t *__restrict__ info,
+                                                 const uint16_t *__restrict__ q, uint16_t *__restrict__ kq_out, int ctx_len,
+                                                 int hidden_dim, int ctx_blk, int nunits, uint32_t blk_cap, uint32_t slot,
+                                                 uint32_t nblocks, int dtype, int q_interleaved) {
     extern __shared__ __align__(16) uint8_t lds[];
-    __shared__ float ws[128];
-    uint8_t *tile = lds;
-    uint8_t *blk = lds + 128 * hid_blk;
-    const int n_hid = hidden_dim / hid_blk;
-    const uint32_t b = blockIdx.x;
-    const uint32_t cb = b / n_hid, hb = b % n_hid;
-    const uint32_t head = (hb * (uint32_t)hid_blk) / kHeadDim;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t b = blockIdx.x * (blockDim.x >> 6) + wave;
+    if (b >= nblocks) return;
+    uint8_t *blk = lds + wave * slot;
+    const int lane = threadIdx.x & 63, t = lane & 31, half = lane >> 5, l16 = lane & 15;
+    float *turn = reinterpret_cast<float *>(blk + slot - 4 * 4 * kKqRow) + (lane >> 4) * kKqRow;
+    const uint32_t n_hid = (uint32_t)hidden_dim / kHeadDim, cb = b / n_hid, hb = b % n_hid;
     uint32_t off, size;
     block_span(info, b, blk_cap, stream_bytes, off, size);
-    const uint32_t phase = stage_to_lds(stream + off, size, blk, threadIdx.x, blockDim.x);
-    for (int t = threadIdx.x; t < 128; t += blockDim.x)
-        ws[t] = ld16(w, (size_t)head * ctx_len + (size_t)cb * 128 + t, dtype);
-    __syncthreads();
-    block_decode<false>(blk, phase, nunits, W, tile, hid_blk);
-    __syncthreads();
-    // thread = 4 adjacent channels x 16 tokens (one dword of the tile per token); the eight token slices meet in
-    // LDS, over the staged block, which nobody reads any more (it holds at least 32 * hid_blk bytes at 2 bits)
-    const int ncg = hid_blk >> 2;
-    const int cg = threadIdx.x % ncg, ts = threadIdx.x / ncg;
-    const uint32_t *col = reinterpret_cast<const uint32_t *>(tile) + (ts * 16) * ncg + cg;
-    float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
+    const uint32_t phase = stage_to_lds(stream + off, size, blk, lane, 64);
+    float qf[4];
 #pragma unroll
-    for (int t = 0; t < 16; t++) {
-        const uint32_t c = col[t * ncg];
-        const float wt = ws[ts * 16 + t];
-        a0 += wt * (float)(c & 0xFFu);
-        a1 += wt * (float)((c >> 8) & 0xFFu);
-        a2 += wt * (float)((c >> 16) & 0xFFu);
-        a3 += wt * (float)(c >> 24);
+    for (int i = 0; i < 4; i++) {      // (interleaved as in evaluation/evaluation.py:465-468)
+        const int src = !q_interleaved ? 4 * t + i : i < 2 ? 2 * t + i : 64 + 2 * t + (i - 2);
+        qf[i] = ld16(q, (size_t)hb * kHeadDim + src, dtype);
     }
-    float *part = reinterpret_cast<float *>(blk);
-    *reinterpret_cast<float4 *>(part + ts * hid_blk + 4 * cg) = make_float4(a0, a1, a2, a3);
+    const float4 q4 = make_float4(qf[0], qf[1], qf[2], qf[3]);
+    wave_lds_order();
+    const uint16_t *cum = reinterpret_cast<const uint16_t *>(blk + phase);      // (phase is even)
+#pragma unroll 1
+    for (int u0 = 0; u0 < nunits; u0 += 2) {
+        const int unit = min(u0 + half, nunits - 1);      // (an odd last round: both halves decode it, the first one writes)
+        const uint32_t start = phase + 2u * (uint32_t)nunits + (unit ? (uint32_t)cum[unit - 1] : 0u);
+        unit_fields<W>(blk, start, t, [&](int k, uint32_t c01, uint32_t c23) { turn[kKqTok * k + l16] = dot4(c01, c23, q4); });
+        wave_lds_order();
+        float s = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float4 v = *reinterpret_cast<const float4 *>(turn + kKqTok * l16 + 4 * i);
+            s = ((s + v.x) + v.y) + v.z;
+            s += v.w;
+        }
+        wave_lds_order();
+        s = kFieldUnit * (s + __shfl_xor(s, 16, 64));
+        if ((lane & 16) == 0 && u0 + half < nunits) kq_out[(size_t)hb * ctx_len + (size_t)cb * ctx_blk + 16 * unit + l16] = st16(s, dtype);
+    }
+}
+
+// w . V: wavefront per V block, four context blocks of one column of blocks to a workgroup; a half per 64-token segment,
+// lane = channel, so a channel's sum over the tokens stays in its lane.  The weights lie in LDS as floats, [segment][token of
+// the pack][round], one 16-byte broadcast per four codes.  The halves and then the workgroup's blocks are added before the
+// one atomic per channel.
+// 65536 tokens x 8 heads at 3 bits: 10.7 us, 18.6 with a code tile per block and an atomic per channel and block.
+constexpr int kWvWaves = 4;
+template <int W>
+__global__ void __launch_bounds__(64 * kWvWaves) wv_kernel(const uint8_t *__restrict__ stream, uint64_t stream_bytes, const uint32_t *__restrict__ info,
+                                                           const uint16_t *__restrict__ w, float *__restrict__ wv_out, int ctx_len,
+                                                           int hidden_dim, int hid_blk, uint32_t blk_cap, uint32_t slot, int dtype) {
+    extern __shared__ __align__(16) uint8_t lds[];
+    __shared__ __align__(16) float ws[kWvWaves][128];
+    __shared__ float part[kWvWaves][kHeadDim];
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63, t = lane & 31, seg = lane >> 5;
+    const uint32_t n_hid = (uint32_t)(hidden_dim / hid_blk), n_ctx = (uint32_t)(ctx_len / 128);
+    const uint32_t hb = blockIdx.x % n_hid, cb = blockIdx.x / n_hid * kWvWaves + wave;
+    const int npair = hid_blk / kLanes;                    // unit = 2 * pair + segment
+    if (cb < n_ctx) {
+        uint8_t *blk = lds + wave * slot;
+        const uint32_t head = (hb * (uint32_t)hid_blk) / kHeadDim;
+        uint32_t off, size;
+        block_span(info, cb * n_hid + hb, blk_cap, stream_bytes, off, size);
+        const uint32_t phase = stage_to_lds(stream + off, size, blk, lane, 64);
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int tok = lane + 64 * i;                 // segment i, round lane / 16, token lane % 16 of the pack
+            ws[wave][64 * i + 4 * (lane & 15) + (lane >> 4)] = ld16(w, (size_t)head * ctx_len + (size_t)cb * 128 + tok, dtype);
+        }
+        wave_lds_order();
+        const uint16_t *cum = reinterpret_cast<const uint16_t *>(blk + phase);  // (phase is even)
+#pragma unroll 1
+        for (int p = 0; p < npair; p++) {
+            uint32_t at = 64u * (uint32_t)seg;
+            asm volatile("" : "+v"(at));                   // (the weights are read where they are used: kept in registers they would take 64)
+            const float4 *w4 = reinterpret_cast<const float4 *>(ws[wave] + at);
+            const int unit = 2 * p + seg;
+            const uint32_t start = phase + 4u * (uint32_t)npair + (unit ? (uint32_t)cum[unit - 1] : 0u);
+            float acc[4] = {0.f, 0.f, 0.f, 0.f};
+            unit_fields<W>(blk, start, t, [&](int k, uint32_t c01, uint32_t c23) { acc[k & 3] = dot4(c01, c23, w4[k], acc[k & 3]); });
+            const float s = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+            const float both = kFieldUnit * (s + __shfl_xor(s, 32, 64));
+            if (seg == 0) part[wave][kLanes * p + t] = both;
+        }
+    } else {
+        for (int c = lane; c < hid_blk; c += 64) part[wave][c] = 0.f;
+    }
     __syncthreads();
     if ((int)threadIdx.x < hid_blk) {
-        float acc = 0.f;
+        float s = 0.f;
 #pragma unroll
-        for (int i = 0; i < 8; i++) acc += part[i * hid_blk + threadIdx.x];
-        atomicAdd(wv_out + (size_t)hb * hid_blk + threadIdx.x, acc);
+        for (int i = 0; i < kWvWaves; i++) s += part[i][threadIdx.x];
+        atomicAdd(wv_out + (size_t)hb * hid_blk + threadIdx.x, s);
     }
 }
 
@@ -202,13 +248,14 @@ int pkv_kq_mat_vec_mul(const uint8_t *stream, uint64_t stream_bytes, const uint3
     const int nunits = ctx_blk / kPackTok;
     const uint32_t cap = (uint32_t)k_block_bound(ctx_blk, bits);
     const int nblocks = (ctx_len / ctx_blk) * (hidden_dim / hid_blk);
-    const uint32_t lds_bytes = (uint32_t)(ctx_blk * kHeadDim) + ((cap + 15u) & ~15u) + 32u;
-    const int threads = ((2 * ctx_blk + 63) / 64) * 64;
+    const uint32_t slot = ((cap + 15u) & ~15u) + 32u + 4u * 4u * kKqRow;      // at most 23.7 KB: 256 tokens at 4 bits
+    const uint32_t wpw = slot * 4u <= 65536u ? 4u : 65536u / slot;
     LaunchTimer tm(s, ms_out != nullptr);
     if ((rc = tm.begin())) return rc;
-    kq_kernel<<<nblocks, threads, lds_bytes, s>>>(stream, stream_bytes, block_info, (const uint16_t *)q, (uint16_t *)kq_out,
-                                                   ctx_len, hidden_dim, ctx_blk, nunits, bits, cap, dtype,
-                                                   q_interleaved);
+    auto kern = bits == 2 ? kq_kernel<2> : bits == 3 ? kq_kernel<3> : kq_kernel<4>;
+    kern<<<((uint32_t)nblocks + wpw - 1u) / wpw, 64u * wpw, wpw * slot, s>>>(
+        stream, stream_bytes, block_info, (const uint16_t *)q, (uint16_t *)kq_out, ctx_len, hidden_dim, ctx_blk, nunits, cap,
+        slot, (uint32_t)nblocks, dtype, q_interleaved);
     PKV_HIP_CHECK(hipGetLastError());
     return tm.end(ms_out);
 }
@@ -225,14 +272,14 @@ int pkv_wv_mat_vec_mul(const uint8_t *stream, uint64_t stream_bytes, const uint3
     PKV_REQUIRE(bits >= 2 && bits <= 4 && ctx_blk == 128 && (hid_blk == 32 || hid_blk == 64 || hid_blk == 128) &&
                     ctx_len > 0 && ctx_len % ctx_blk == 0 && hidden_dim > 0 && hidden_dim % kHeadDim == 0,
                 PKV_ERR_UNSUPPORTED, "no such case");
-    const int nunits = 2 * (hid_blk / kLanes);
     const uint32_t cap = (uint32_t)v_block_bound(hid_blk, bits);
-    const int nblocks = (ctx_len / ctx_blk) * (hidden_dim / hid_blk);
-    const uint32_t lds_bytes = (uint32_t)(128 * hid_blk) + ((cap + 15u) & ~15u) + 32u;
+    const uint32_t slot = ((cap + 15u) & ~15u) + 32u;           // at most 9.2 KB: 128 channels at 4 bits
+    const uint32_t rows = (uint32_t)(ctx_len / ctx_blk + kWvWaves - 1) / kWvWaves;
     LaunchTimer tm(s, ms_out != nullptr);
     if ((rc = tm.begin())) return rc;
-    wv_kernel<<<nblocks, 2 * hid_blk, lds_bytes, s>>>(stream, stream_bytes, block_info, (const uint16_t *)w, wv_out, ctx_len,
-                                                      hidden_dim, hid_blk, nunits, bits, cap, dtype);
+    auto kern = bits == 2 ? wv_kernel<2> : bits == 3 ? wv_kernel<3> : wv_kernel<4>;
+    kern<<<rows * (uint32_t)(hidden_dim / hid_blk), 64 * kWvWaves, kWvWaves * slot, s>>>(
+        stream, stream_bytes, block_info, (const uint16_t *)w, wv_out, ctx_len, hidden_dim, hid_blk, cap, slot, dtype);
     PKV_HIP_CHECK(hipGetLastError());
     return tm.end(ms_out);
 }

@@ -143,3 +143,47 @@ def test_damaged_block_info_is_survived(cuda):
     ops.wv_mat_vec_mul(comp, torch.from_numpy(bad_info.astype(np.uint32)).to(cuda), w, out, T, H * 128, cb, hb, W)
     torch.cuda.synchronize()
     assert out.shape == (H, 128)
+
+
+# Blocks of other lengths and widths, odd round counts, blocks and context blocks that do not fill the last workgroup.
+KQ_SHAPES = [(1, 16, 16, 2), (3, 48, 48, 3), (8, 768, 48, 4), (2, 1024, 256, 4), (5, 192, 64, 2), (1, 64, 64, 4)]
+WV_SHAPES = [(1, 128, 32, 2), (3, 384, 64, 3), (2, 640, 128, 4), (5, 1152, 64, 2), (1, 512, 128, 3)]
+
+
+def _block_codec(cuda, is_k, H, T, cb, hb, bits, seed):
+    g = torch.Generator().manual_seed(seed)
+    codes = torch.randint(0, 1 << bits, (T, H * 128), generator=g, dtype=torch.uint8)
+    codes[:, ::5] = codes[0, ::5]                                   # packs of width 0 among them
+    codes = codes.to(cuda)
+    n = (T // cb) * (H * 128 // hb)
+    stream = torch.zeros(n * ops.block_bound(is_k, cb, hb, bits) + 16, dtype=torch.uint8, device=cuda)
+    info = torch.zeros(n, 2, dtype=torch.uint32, device=cuda)
+    (ops.k_encode if is_k else ops.v_encode)(codes, stream, info, cb, hb, bits)
+    return codes.cpu().double().view(T, H, 128), stream, info
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("H,T,cb,bits", KQ_SHAPES)
+def test_kq_block_shapes(cuda, H, T, cb, bits, dtype):
+    codes, stream, info = _block_codec(cuda, True, H, T, cb, 128, bits, 5)
+    q = torch.randn(H, 128, generator=torch.Generator().manual_seed(6)).to(dtype)
+    t = torch.full((H, T), float("nan"), dtype=dtype, device=cuda)
+    ops.kq_mat_vec_mul(stream, info, q.to(cuda), t, T, H * 128, cb, 128, bits, q_interleaved=False)
+    want = torch.einsum("thd,hd->ht", codes, q.double())
+    # fp32 sums of 128 exact products (at most 128 roundings of 2^-24 of the sum of magnitudes), one rounding to dtype
+    mag = torch.einsum("thd,hd->ht", codes, q.double().abs())
+    half_ulp = 2 ** -11 if dtype == torch.float16 else 2 ** -8
+    assert bool(((t.cpu().double() - want).abs() <= half_ulp * want.abs() * 1.01 + 2 ** -17 * mag).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("H,T,hb,bits", WV_SHAPES)
+def test_wv_block_shapes(cuda, H, T, hb, bits, dtype):
+    codes, stream, info = _block_codec(cuda, False, H, T, 128, hb, bits, 7)
+    w = torch.rand(H, T, generator=torch.Generator().manual_seed(8)).to(dtype)
+    out = torch.ones(H, 128, dtype=torch.float32, device=cuda)      # the sums are added to what is there
+    ops.wv_mat_vec_mul(stream, info, w.to(cuda), out, T, H * 128, 128, hb, bits)
+    want = 1.0 + torch.einsum("ht,thd->hd", w.double(), codes)
+    # every term is non-negative: at most T + 8 roundings of 2^-24 of the result
+    assert bool(((out.cpu().double() - want).abs() <= (T + 8) * 2 ** -24 * want).all())
+
