@@ -8,6 +8,8 @@
 #include "pkv_block.hpp"
 #include "pkv_runtime.hpp"
 
+#include <initializer_list>
+
 namespace pkv {
 
 __device__ __forceinline__ float ld16(const uint16_t *p, size_t i, int dtype) {
@@ -166,43 +168,73 @@ __device__ __forceinline__ float wave_sum_f32(float x) {
     return x;
 }
 
-// grid = (ceil(N / 2048), M), 256 threads: every workgroup forms the row's sum of q itself (K values) and then
-// finishes 2048 columns, eight per thread.
+// Four adjacent 16-bit values from `i` on, as they lie: one 8-byte load where `vec` says that every row starts on an 8-byte
+// boundary and ends on a multiple of four (uniform), else one by one, zero past the end.
+struct Raw4 {
+    uint16_t u[4];
+};
+__device__ __forceinline__ Raw4 ld4(const uint16_t *p, size_t row, int i, int n, bool vec) {
+    Raw4 r = {{0, 0, 0, 0}};
+    if (vec) {
+        if (i < n) *reinterpret_cast<uint2 *>(r.u) = *reinterpret_cast<const uint2 *>(p + row + i);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (i + k < n) r.u[k] = p[row + i + k];
+    }
+    return r;
+}
+static bool rows_of_fours(int n, std::initializer_list<const void *> ptrs) {
+    uintptr_t a = 0;
+    for (const void *p : ptrs) a |= reinterpret_cast<uintptr_t>(p);
+    return n % 4 == 0 && (a & 7u) == 0;
+}
+
+// grid = (ceil(N / 1024), M), 256 threads: every workgroup forms the row's sum of q itself (K values) and finishes 1024
+// columns, four per thread, which are on their way meanwhile.
 __global__ void __launch_bounds__(256) fused_kq_kernel(uint16_t *__restrict__ out, const uint16_t *__restrict__ q,
                                                        const uint16_t *__restrict__ zero, const uint16_t *__restrict__ scale,
-                                                       const uint16_t *__restrict__ t, int K, int N, int dtype) {
+                                                       const uint16_t *__restrict__ t, int K, int N, int dtype, bool vec) {
     __shared__ float red[4];
     const int m = blockIdx.y;
+    const int n = blockIdx.x * 1024 + 4 * (int)threadIdx.x;
+    const size_t row = (size_t)m * N;
+    const Raw4 z = ld4(zero, 0, n, N, vec), tt = ld4(t, row, n, N, vec), sc = ld4(scale, 0, n, N, vec);
     float s = 0.f;
     for (int d = threadIdx.x; d < K; d += 256) s += ld16(q, (size_t)m * K + d, dtype);
     s = wave_sum_f32(s);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
     __syncthreads();
     const float sm = (red[0] + red[1]) + (red[2] + red[3]);
-    const int n0 = blockIdx.x * 2048;
+    Raw4 o;
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const int n = n0 + threadIdx.x + 256 * i;
-        if (n < N) {
-            const float u = sm * ld16(zero, n, dtype) + ld16(t, (size_t)m * N + n, dtype);
-            out[(size_t)m * N + n] = st16(u * ld16(scale, n, dtype), dtype);
-        }
+    for (int i = 0; i < 4; i++) {
+        const float u = sm * ld16(z.u, i, dtype) + ld16(tt.u, i, dtype);
+        o.u[i] = st16(u * ld16(sc.u, i, dtype), dtype);
+    }
+    if (vec) {
+        if (n < N) *reinterpret_cast<uint2 *>(out + row + n) = *reinterpret_cast<const uint2 *>(o.u);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (n + i < N) out[row + n + i] = o.u[i];
     }
 }
 
-// Row sums of w * zero * scale in two steps: grid (ceil(N / 4096), M) partial sums, then one workgroup per row
-// adds the partials and finishes the D outputs.
+// Row sums of w * zero * scale in two steps: grid (ceil(N / 1024), M) partial sums, then one workgroup per row
+// adds the partials and finishes the D outputs.  (65536 columns x 8 rows: 3.5 us for the partial sums; 7.9 with 4096 columns
+// a workgroup, read one value at a time.)
+constexpr int kWvPart = 1024;
 __global__ void __launch_bounds__(256) fused_wv_partial_kernel(const uint16_t *__restrict__ w, const uint16_t *__restrict__ zero,
                                                                const uint16_t *__restrict__ scale, float *__restrict__ part,
-                                                               int N, int dtype) {
+                                                               int N, int dtype, bool vec) {
     __shared__ float red[4];
-    const int m = blockIdx.y, n0 = blockIdx.x * 4096;
+    const int m = blockIdx.y, n = blockIdx.x * kWvPart + 4 * (int)threadIdx.x;
+    const Raw4 a = ld4(w, (size_t)m * N, n, N, vec), z = ld4(zero, 0, n, N, vec), sc = ld4(scale, 0, n, N, vec);
     float s = 0.f;
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-        const int n = n0 + threadIdx.x + 256 * i;
-        if (n < N) s += ld16(w, (size_t)m * N + n, dtype) * ld16(zero, n, dtype) * ld16(scale, n, dtype);
-    }
+    for (int i = 0; i < 4; i++)
+        if (n + i < N) s += ld16(a.u, i, dtype) * ld16(z.u, i, dtype) * ld16(sc.u, i, dtype);
     s = wave_sum_f32(s);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
     __syncthreads();
@@ -295,9 +327,9 @@ int pkv_fused_kq(void *our_kq, const void *q, const void *k_zero, const void *k_
     PKV_REQUIRE(M <= 65535, PKV_ERR_UNSUPPORTED, "more than 65535 rows");
     LaunchTimer tm(s, ms_out != nullptr);
     if ((rc = tm.begin())) return rc;
-    fused_kq_kernel<<<dim3((unsigned)((N + 2047) / 2048), (unsigned)M), 256, 0, s>>>(
+    fused_kq_kernel<<<dim3((unsigned)((N + 1023) / 1024), (unsigned)M), 256, 0, s>>>(
         (uint16_t *)our_kq, (const uint16_t *)q, (const uint16_t *)k_zero, (const uint16_t *)k_scale,
-        (const uint16_t *)t, K, N, dtype);
+        (const uint16_t *)t, K, N, dtype, rows_of_fours(N, {our_kq, k_zero, k_scale, t}));
     PKV_HIP_CHECK(hipGetLastError());
     return tm.end(ms_out);
 }
@@ -311,13 +343,14 @@ int pkv_fused_wv(void *our_wv, const void *w, const void *v_zero, const void *v_
     PKV_REQUIRE(our_wv && w && v_zero && v_scale && term1, PKV_ERR_INVALID, "null pointer argument");
     PKV_REQUIRE(M > 0 && N > 0 && D > 0, PKV_ERR_INVALID, "sizes must be positive");
     PKV_REQUIRE(M <= 65535, PKV_ERR_UNSUPPORTED, "more than 65535 rows");
-    const int nparts = (N + 4095) / 4096;
+    const int nparts = (N + kWvPart - 1) / kWvPart;
     void *scratch = nullptr;
     if ((rc = scratch_get((size_t)M * nparts * sizeof(float), s, &scratch))) return rc;
     LaunchTimer tm(s, ms_out != nullptr);
     if ((rc = tm.begin())) return rc;
     fused_wv_partial_kernel<<<dim3((unsigned)nparts, (unsigned)M), 256, 0, s>>>(
-        (const uint16_t *)w, (const uint16_t *)v_zero, (const uint16_t *)v_scale, (float *)scratch, N, dtype);
+        (const uint16_t *)w, (const uint16_t *)v_zero, (const uint16_t *)v_scale, (float *)scratch, N, dtype,
+        rows_of_fours(N, {w, v_zero, v_scale}));
     fused_wv_kernel<<<M, 256, 0, s>>>((uint16_t *)our_wv, (const float *)scratch, nparts, (const uint16_t *)term1,
                                       D, dtype);
     PKV_HIP_CHECK(hipGetLastError());

@@ -187,3 +187,29 @@ def test_wv_block_shapes(cuda, H, T, hb, bits, dtype):
     # every term is non-negative: at most T + 8 roundings of 2^-24 of the result
     assert bool(((out.cpu().double() - want).abs() <= (T + 8) * 2 ** -24 * want).all())
 
+
+@pytest.mark.parametrize("N,off", [(1, 0), (1023, 0), (1024, 1), (1028, 0), (4100, 3), (2050, 0)])
+def test_fused_fixups_any_length_and_alignment(cuda, N, off):
+    """Rows that start off an 8-byte boundary or are no multiple of four long are read one value at a time."""
+    g = torch.Generator().manual_seed(N)
+    M, K, D = 3, 128, 100
+
+    def rows(shape, fn):
+        n = int(np.prod(shape))
+        return fn(n + off).to(torch.float16).to(cuda)[off:].view(shape)
+    q, t = rows((M, K), lambda n: torch.randn(n, generator=g)), rows((M, N), lambda n: torch.randn(n, generator=g))
+    zero, scale = rows((N,), lambda n: torch.randn(n, generator=g).round()), rows((N,), lambda n: torch.rand(n, generator=g) + 0.5)
+    w, term1 = rows((M, N), lambda n: torch.rand(n, generator=g)), rows((M, D), lambda n: torch.randn(n, generator=g))
+    guard = torch.full((M * N + off + 8,), 7.0, dtype=torch.float16, device=cuda)
+    kq = guard[off:off + M * N].view(M, N)
+    packkv_cuda.fused_kq(kq, q, zero, scale, t)
+    want = (q.double().sum(1, keepdim=True) * zero.double() + t.double()) * scale.double()
+    mag = (q.double().abs().sum(1, keepdim=True) * zero.double().abs() + t.double().abs()) * scale.double()
+    assert bool(((kq.double() - want).abs() <= 2 ** -11 * want.abs() * 1.01 + 2 ** -17 * mag + 2 ** -24).all())
+    assert bool((guard[:off] == 7.0).all()) and bool((guard[off + M * N:] == 7.0).all())
+    wv = torch.empty(M, D, dtype=torch.float16, device=cuda)
+    packkv_cuda.fused_wv(wv, w, zero, scale, term1)
+    c = w.double() * zero.double() * scale.double()
+    want = c.sum(1, keepdim=True) + term1.double()
+    mag = c.abs().sum(1, keepdim=True) + term1.double().abs()
+    assert bool(((wv.double() - want).abs() <= 2 ** -11 * want.abs() * 1.01 + 2 ** -14 * mag + 2 ** -24).all())
