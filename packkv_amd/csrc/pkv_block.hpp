@@ -501,6 +501,7 @@ __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
 // stores that publish them.  A window's aggregates (sizes of single tickets, far below 2^32) are summed in 32 bits
 // on the DPP path; the one inclusive prefix that ends the walk is read from its lane.
 constexpr int kLookWindows = 1;
+template <int SLEEP = PKV_LOOKBACK_SLEEP>
 __device__ __forceinline__ uint64_t lookback_offset(ScanState *st, uint32_t idx, uint32_t my_bytes, bool published = false) {
     const int lane = threadIdx.x & 63;
     uint64_t *status = st->status;
@@ -530,7 +531,7 @@ __device__ __forceinline__ uint64_t lookback_offset(ScanState *st, uint32_t idx,
             const int64_t j = base - 64 * w - lane;
             int spins = 0;
             while ((s[w] >> 62) == 0 && spins < kSpinLimit) {
-                __builtin_amdgcn_s_sleep(PKV_LOOKBACK_SLEEP);
+                __builtin_amdgcn_s_sleep(SLEEP);
                 s[w] = __hip_atomic_load(&status[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 spins++;
             }

@@ -344,12 +344,11 @@ static int run_pack(bool is_k, const uint8_t *codes, uint8_t *stream, uint64_t c
     const bool cells = bits <= 6 && hidden_dim % 1024 == 0 && (reinterpret_cast<uintptr_t>(codes) & 3u) == 0 &&
                        (is_k ? (ctx_blk == 64 && hid_blk == 128) : (ctx_blk == 128 && hid_blk == 64));
     if (cells) {
-        const uint32_t ngroups = (uint32_t)cs.nblocks / (is_k ? 8u : 16u);
-        if ((rc = prepare_scan_state(ngroups, &sh, s, size_out || ms_out))) return rc;
+        if ((rc = prepare_scan_state(code_cells_words(is_k, ctx_len, hidden_dim), &sh, s, size_out || ms_out))) return rc;
         ScanState *st = sh.st;
         LaunchTimer tm(s, ms_out != nullptr);
         if ((rc = tm.begin())) return rc;
-        if ((rc = launch_code_cells(is_k, codes, ctx_len, hidden_dim, bits, cs.blk_cap, stream, capacity, info, st, ngroups, s))) return rc;
+        if ((rc = launch_code_cells(is_k, codes, ctx_len, hidden_dim, bits, cs.blk_cap, stream, capacity, info, st, s))) return rc;
         if ((rc = tm.end(ms_out))) return rc;
         return finish_encode(sh, size_out, 0, s);
     }

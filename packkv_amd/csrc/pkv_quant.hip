@@ -8,6 +8,8 @@
 #include "pkv_block.hpp"
 #include "pkv_runtime.hpp"
 
+#include <algorithm>
+
 namespace pkv {
 
 template <int DT> struct T16;
@@ -789,15 +791,16 @@ constexpr int kSubBlocks = 8;
 #endif
 
 // Copy n bytes (even) from LDS (src 4-byte aligned, readable up to 20 bytes past n) to global memory (dst 2-byte
-// aligned) with the 32 lanes of a half-wavefront: head to the first 16-byte boundary and tail in 2-byte pieces, the
+// aligned) with `N` threads, t = 0 .. N - 1 of them: head to the first 16-byte boundary and tail in 2-byte pieces, the
 // body as aligned 16-byte stores fed by aligned LDS reads and byte funnel shifts.
-__device__ __forceinline__ void copy_out32(uint8_t *dst, const uint8_t *src, uint32_t n, int t) {
+template <int N>
+__device__ __forceinline__ void copy_out(uint8_t *dst, const uint8_t *src, uint32_t n, int t) {
     const uint32_t head = min(n, (uint32_t)((16u - (uint32_t)(reinterpret_cast<uintptr_t>(dst) & 15u)) & 15u));
     const uint32_t nq = (n - head) >> 4;
-    for (uint32_t i = t; i < (head >> 1); i += 32)
+    for (uint32_t i = t; i < (head >> 1); i += N)
         reinterpret_cast<uint16_t *>(dst)[i] = reinterpret_cast<const uint16_t *>(src)[i];
     const uint32_t *src32 = reinterpret_cast<const uint32_t *>(src + (head & ~3u));
-    for (uint32_t i = t; i < nq; i += 32) {
+    for (uint32_t i = t; i < nq; i += N) {
         const uint32_t *q = src32 + 4 * i;
         const uint32_t d0 = q[0], d1 = q[1], d2 = q[2], d3 = q[3], d4 = q[4];
         uint4 v;
@@ -808,9 +811,10 @@ __device__ __forceinline__ void copy_out32(uint8_t *dst, const uint8_t *src, uin
         *reinterpret_cast<uint4 *>(dst + head + 16 * (size_t)i) = v;
     }
     const uint32_t done = head + 16u * nq;
-    for (uint32_t i = t; i < ((n - done) >> 1); i += 32)
+    for (uint32_t i = t; i < ((n - done) >> 1); i += N)
         reinterpret_cast<uint16_t *>(dst + done)[i] = reinterpret_cast<const uint16_t *>(src + done)[i];
 }
+__device__ __forceinline__ void copy_out32(uint8_t *dst, const uint8_t *src, uint32_t n, int t) { copy_out<32>(dst, src, n, t); }
 
 // Minimum and maximum of every token of a round over a wavefront's cells.  Lane's cell: rows xr[k] = token
 // k, four channels.  The 16 per-token values of a lane are reduced and transposed at once: each step exchanges half
@@ -1683,14 +1687,6 @@ __global__ void __launch_bounds__(512) v_quant_encode_cells_kernel(
     }
 }
 
-// ---- the block codec from a code matrix, as cells --------------------------------------------------------------
-// The cells encoders with nothing to quantize: the input is the uint8 code matrix [ctx_len, hidden] of pkv_k_encode /
-// pkv_v_encode.  Eight consecutive K blocks (64 x 128) or sixteen consecutive V blocks (128 x 64) of the stream are
-// 1024 adjacent channels of one context block, i.e. exactly the group a cells workgroup owns, with the "heads" being
-// 128-channel slices of the matrix.  A thread reads its cell as sixteen dwords (four codes of one token each; the 32
-// lanes of a half-wavefront one 128-byte line per token), asks for the next round's while it forms and emits this
-// round's packs, and no code tile is staged in LDS.  For hidden a multiple of 1024, the reference's block shapes and
-// widths up to 6; pack_group_kernel takes everything else.
 // `rows` (uniform: scalar registers) is the first of the 16 token rows, `lane_off` the lane's byte offset inside a
 // row, so that a load is one 32-bit lane offset on a scalar base
 __device__ __forceinline__ void code_cell_load(const uint8_t *rows, size_t row_bytes, uint32_t lane_off, uint32_t w[16]) {
@@ -1706,6 +1702,20 @@ __device__ __forceinline__ void code_cell_pairs(const uint32_t w[16], uint32_t c
     }
 }
 
+}  // namespace pkv
+
+#include "pkv_quant_once.hpp"
+
+namespace pkv {
+
+// ---- the block codec from a code matrix, as cells --------------------------------------------------------------
+// The cells encoders with nothing to quantize: the input is the uint8 code matrix [ctx_len, hidden] of pkv_k_encode /
+// pkv_v_encode.  Eight consecutive K blocks (64 x 128) or sixteen consecutive V blocks (128 x 64) of the stream are
+// 1024 adjacent channels of one context block, i.e. exactly the group a cells workgroup owns, with the "heads" being
+// 128-channel slices of the matrix.  A thread reads its cell as sixteen dwords (four codes of one token each; the 32
+// lanes of a half-wavefront one 128-byte line per token), asks for the next round's while it forms and emits this
+// round's packs, and no code tile is staged in LDS.  For hidden a multiple of 1024, the reference's block shapes and
+// widths up to 6; pack_group_kernel takes everything else.
 template <bool WIDE>
 __global__ void __launch_bounds__(256) k_code_cells_kernel(
     const uint8_t *__restrict__ codes, int hidden, uint8_t *__restrict__ stream, uint64_t capacity,
@@ -1882,13 +1892,25 @@ __global__ void __launch_bounds__(512) v_code_cells_kernel(
     }
 }
 
-// Launch of the two kernels above (pkv_codec.hip decides when they apply): `st` is a prepared scan state with one
-// status word per group, `bound` the worst-case bytes of a block.
+// Launch of the two kernels above (pkv_codec.hip decides when they apply): `st` is a prepared scan state of
+// code_cells_words status words, `bound` the worst-case bytes of a block.
+static OncePlan code_plan(bool is_k, int ctx_len, int hidden) { return once_plan(is_k, (uint64_t)(ctx_len / (is_k ? 64 : 128)), hidden / kHeadDim, kOnceSmallCodes); }
+uint32_t code_cells_words(bool is_k, int ctx_len, int hidden) {
+    const OncePlan p = code_plan(is_k, ctx_len, hidden);
+    return p.threads ? p.nwg : (uint32_t)(ctx_len / (is_k ? 64 : 128)) * (uint32_t)(hidden / 1024);
+}
 int launch_code_cells(bool is_k, const uint8_t *codes, int ctx_len, int hidden, int bits, uint32_t bound, uint8_t *stream,
-                      uint64_t capacity, uint32_t *info, ScanState *st, uint32_t ngroups, hipStream_t s) {
+                      uint64_t capacity, uint32_t *info, ScanState *st, hipStream_t s) {
+    const uint32_t ngroups = code_cells_words(is_k, ctx_len, hidden);
     int rc;
     Stagger sg;
-    if (is_k) {
+    if (const OncePlan p = code_plan(is_k, ctx_len, hidden); p.threads) {
+        OnceSide a{};
+        a.codes = codes; a.hidden = hidden;
+        a.stream = stream; a.capacity = capacity; a.info = info; a.st = st; a.W = bits;
+        a.nruns = p.nruns; a.nwg = p.nwg; a.slot = once_slot(is_k, bits);
+        return p.threads == 256 ? once_launch_codes<256>(is_k, a, p.run, s) : once_launch_codes<1024>(is_k, a, p.run, s);
+    } else if (is_k) {
         const uint32_t slot = (bound + 15u) & ~15u;
         const uint32_t lds = (uint32_t)kSubBlocks * slot + 32u;
         auto kern = bits > 4 ? k_code_cells_kernel<true> : k_code_cells_kernel<false>;
@@ -1902,7 +1924,6 @@ int launch_code_cells(bool is_k, const uint8_t *codes, int ctx_len, int hidden, 
         if ((rc = stagger_for(reinterpret_cast<const void *>(kern), 512, lds, ngroups, &sg))) return rc;
         kern<<<ngroups, 512, lds, s>>>(codes, hidden, stream, capacity, info, st, bits, ngroups, unit_slot, sg);
     }
-    (void)ctx_len;
     PKV_HIP_CHECK(hipGetLastError());
     return PKV_OK;
 }
@@ -2090,12 +2111,14 @@ struct EncodeJob {
     Rot rot = {nullptr, nullptr, 0};       // K of five heads or more, in their own order
 };
 
-// 64-bit words of look-back state the job takes: status words (one per ticket), then, with more than eight heads, the
-// words the runs of a group exchange: one per (run, token).
+// 64-bit words of look-back state the job takes: status words (one per ticket), then the words the runs of a group
+// exchange: one per (run, token), where a group has more than one.
 static uint64_t state_words(bool is_k, int B, int H, int T) {
     const uint64_t ctx_blk = is_k ? 64 : 128, groups = (uint64_t)T / ctx_blk * (uint64_t)B;
     const uint64_t nsub = groups * (uint64_t)(((is_k ? H : 2 * H) + kSubBlocks - 1) / kSubBlocks);
-    return nsub + (H <= kSubBlocks ? 0 : groups * (uint64_t)((H + kSubBlocks - 1) / kSubBlocks) * ctx_blk);
+    const uint64_t n = nsub + (H <= kSubBlocks ? 0 : groups * (uint64_t)((H + kSubBlocks - 1) / kSubBlocks) * ctx_blk);
+    const OncePlan p = once_plan(is_k, groups, H, kOnceSmall);
+    return p.threads ? std::max(n, p.nwg * (p.nruns > 1 ? 1 + ctx_blk : 1)) : n;
 }
 
 template <bool IS_K>
@@ -2161,6 +2184,26 @@ static auto cells_kernel(int bits, int dtype, bool perm, bool xch, bool strided,
     return dtype == PKV_F16 ? cells_kernel_of<IS_K, false, PKV_F16>(perm, xch, strided, rot) : cells_kernel_of<IS_K, false, PKV_BF16>(perm, xch, strided, rot);
 }
 
+// The kernels that take a group's tokens at once (pkv_quant_once.hpp), where they serve the job.  (K reaches the second head of
+// a wavefront through a 32-bit byte offset.  Groups of up to four heads in bf16 stay with the round-major kernels: those leave a
+// NaN out of a token's minimum and maximum, the order keys of the cells do not.)
+static OncePlan once_plan_of(bool is_k, const EncodeJob &job, int dtype, int B, int H, int T) {
+    if (job.rot.cos || job.xs.sh >= (1ll << 31) - 128 || (H <= 4 && dtype != PKV_F16 && !job.perm)) return OncePlan{0, 0, 0, 0};
+    return once_plan(is_k, (uint64_t)T / (is_k ? 64 : 128) * (uint64_t)B, H, kOnceSmall);
+}
+static OnceSide once_side(bool is_k, const EncodeJob &job, const OncePlan &p, int B, int H, int T, ScanState *st) {
+    OnceSide a{};
+    a.x = (const uint16_t *)job.x; a.xs = job.xs; a.rel = job.rel;
+    a.scale = (uint16_t *)job.scale; a.zero = (uint16_t *)job.zero;
+    a.stream = job.stream; a.capacity = job.capacity; a.base = job.base; a.info = job.info;
+    a.st = st; a.xw = st->status + p.nwg;
+    a.B = B; a.H = H; a.T = T; a.W = job.bits; a.par_stride = job.par_stride; a.nruns = p.nruns;
+    a.nwg = p.nwg; a.slot = once_slot(is_k, job.bits);
+    a.perm = job.perm; a.perm_block = job.perm_block;
+    a.scale_in = (const uint16_t *)job.scale_in; a.zero_in = (const uint16_t *)job.zero_in;
+    return a;
+}
+
 template <bool IS_K>
 static int launch_quant_encode(const EncodeJob &job, int dtype, int B, int H, int T, ScanState *st, hipStream_t s) {
     const void *x = job.x;
@@ -2175,6 +2218,10 @@ static int launch_quant_encode(const EncodeJob &job, int dtype, int B, int H, in
     const void *scale_in = job.scale_in, *zero_in = job.zero_in;
     const int ctx_blk = IS_K ? 64 : 128, hid_blk = IS_K ? 128 : 64;
     int rc;
+    if (const OncePlan p = once_plan_of(IS_K, job, dtype, B, H, T); p.threads) {
+        const OnceSide a = once_side(IS_K, job, p, B, H, T, st), none{};
+        return p.threads == 256 ? once_launch<256>(IS_K ? a : none, IS_K ? none : a, dtype, s) : once_launch<1024>(IS_K ? a : none, IS_K ? none : a, dtype, s);
+    }
     // One workgroup per run of up to eight heads of a (context block, sequence) group -- K: its up to eight blocks;
     // V: its up to sixteen -- or, with fewer than five heads, per 8 / H groups.
     {
@@ -2448,8 +2495,14 @@ int pkv_kv_quant_encode_append(const pkv_append_side *k, const pkv_append_side *
     }
     ScanHandle sh;
     if ((rc = prepare_scan_state((uint32_t)state_words(true, B, H, T_new), &sh, s, true, (uint32_t)state_words(false, B, H, T_new)))) return rc;
-    if ((rc = launch_quant_encode<true>(job[0], dtype, B, H, T_new, sh.st, s))) return rc;
-    if ((rc = launch_quant_encode<false>(job[1], dtype, B, H, T_new, sh.second, s))) return rc;
+    const OncePlan pk = once_plan_of(true, job[0], dtype, B, H, T_new), pv = once_plan_of(false, job[1], dtype, B, H, T_new);
+    if (pk.threads && pk.threads == pv.threads && (job[0].bits > 4) == (job[1].bits > 4)) {      // both sides in one launch
+        const OnceSide ks = once_side(true, job[0], pk, B, H, T_new, sh.st), vs = once_side(false, job[1], pv, B, H, T_new, sh.second);
+        if ((rc = pk.threads == 256 ? once_launch<256>(ks, vs, dtype, s) : once_launch<1024>(ks, vs, dtype, s))) return rc;
+    } else {
+        if ((rc = launch_quant_encode<true>(job[0], dtype, B, H, T_new, sh.st, s))) return rc;
+        if ((rc = launch_quant_encode<false>(job[1], dtype, B, H, T_new, sh.second, s))) return rc;
+    }
     return finish_encode(sh, k_size, job[0].bits, s, v_size, job[1].bits);
 }
 

@@ -367,3 +367,21 @@ def test_damaged_block_info_is_survived(cuda, is_k):
             continue
         r, h = b // n_hid, b % n_hid
         assert np.array_equal(got[r * cb:(r + 1) * cb, h * hb:(h + 1) * hb], c[r * cb:(r + 1) * cb, h * hb:(h + 1) * hb]), b
+
+
+@pytest.mark.parametrize("bits", [2, 4, 5, 6])
+@pytest.mark.parametrize("heads,T", [(8, 128), (8, 2048), (16, 1152), (8, 16384), (8, 16512)])
+def test_code_matrix_encode_by_group_count(cuda, oracle_codec, heads, T, bits):
+    """Either side of the lines between the kernels: 128 workgroups of 256 threads, 256 of 1024, the kernels that walk."""
+    codes = torch.randint(0, 1 << bits, (T, heads * 128), generator=torch.Generator().manual_seed(T + bits), dtype=torch.uint8)
+    codes[:, ::3] >>= 1
+    codes[:, ::7] = codes[0, ::7]
+    for is_k in (True, False):
+        cb, hb = (64, 128) if is_k else (128, 64)
+        so, io, zo = oracle_codec.encode(int(is_k), codes.numpy(), cb, hb, bits)
+        n = codes.numel() // 8192
+        stream = torch.zeros(n * ops.block_bound(is_k, cb, hb, bits) + 16, dtype=torch.uint8, device=cuda)
+        info = torch.zeros(n, 2, dtype=torch.uint32, device=cuda)
+        size = (ops.k_encode if is_k else ops.v_encode)(codes.to(cuda), stream, info, cb, hb, bits)
+        assert size == zo and np.array_equal(info.cpu().numpy(), io)
+        assert np.array_equal(stream[:zo].cpu().numpy(), so[:zo]) and not bool(stream[zo:].any())

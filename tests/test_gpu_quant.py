@@ -331,3 +331,41 @@ def test_an_encode_that_fails_after_its_launch_leaves_the_look_back_state_clear(
             e["zero"].copy_(got["zero"])
         assert got["size"] == want["size"]
         check()
+
+
+# Either side of the lines between the kernels: 256 workgroups of 256 threads, 256 of 1024 threads, the kernels that walk.
+@pytest.mark.parametrize("B,H,T,rel", [(1, 8, 4096, 0.1), (1, 8, 4224, 0.05), (1, 8, 16384, 0.1), (1, 8, 16512, 0.1), (3, 3, 2816, 0.1),
+                                       (2, 1, 16384, 0.2), (1, 20, 1536, 0.1), (1, 9, 3712, 0.05), (5, 7, 128, 0.03)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_fused_quant_encode_by_group_count(cuda, oracle_codec, B, H, T, rel, dtype):
+    k, v = synth.make_kv(B, H, T, seed=H + T, dtype=dtype)
+    W = ops.bits_for_rel(rel)
+    for is_k, x in ((1, k), (0, v)):
+        _say("fused quant+encode by groups", "K" if is_k else "V", dtype, B, H, T, rel)
+        c, z, s = oq.quant_ints(x, 64, rel)
+        so, io, zo = oracle_codec.encode(is_k, oq.code_matrix(c).numpy(), *((64, 128) if is_k else (128, 64)), W)
+        for rep in range(2):                      # (twice: nothing of the first call's exchange may be left)
+            r = (ops.k_quant_encode if is_k else ops.v_quant_encode)(x.to(cuda), rel, W)
+            assert r["size"] == zo
+            assert np.array_equal(r["info"].cpu().numpy(), io)
+            assert np.array_equal(r["stream"][:zo].cpu().numpy(), so[:zo])
+            assert torch.equal(r["scale"].cpu().view(torch.int16), s.reshape(B, T).view(torch.int16))
+            assert torch.equal(r["zero"].cpu().view(torch.int16), z.reshape(B, T).view(torch.int16))
+
+
+@pytest.mark.parametrize("T", [128, 4096, 4224, 16512])
+def test_encodes_at_once_report_codes_and_capacity(cuda, T):
+    """A code wider than the stream's width and a stream that does not fit are reported, and the next encode is right."""
+    k, v = synth.make_kv(1, 8, T, seed=T, device=cuda)
+    for fn, x in ((ops.k_quant_encode, k), (ops.v_quant_encode, v)):
+        good = fn(x, 0.1)
+        with pytest.raises(RuntimeError, match="does not fit bits_len"):
+            fn(x, 0.03, bits=4)
+        small = torch.full((good["size"] + 62,), 77, dtype=torch.uint8, device=cuda)
+        with pytest.raises(RuntimeError, match="does not fit the output buffer"):
+            fn(x, 0.1, stream=small[:good["size"] - 2])
+        torch.cuda.synchronize()
+        assert bool((small[good["size"] - 2:] == 77).all())
+        again = fn(x, 0.1, stream=small[:good["size"]])
+        assert again["size"] == good["size"] and torch.equal(again["stream"], good["stream"][:good["size"]])
+        assert torch.equal(again["info"].view(torch.int32), good["info"].view(torch.int32)) and bool((small[good["size"]:] == 77).all())
