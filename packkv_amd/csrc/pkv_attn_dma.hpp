@@ -98,7 +98,7 @@ __device__ __forceinline__ u32x4 dma_rsrc_at(u32x4 r, uint32_t add, uint32_t byt
     return (u32x4){(uint32_t)a, (uint32_t)(a >> 32), bytes, r[3]};
 }
 
-template <int N> struct IntC { static constexpr int value = N; };
+template <int N> struct IntC { static constexpr int value = N; __device__ constexpr operator int() const { return N; } };
 
 template <int KW, int VW>
 struct DmaGeom {
@@ -304,9 +304,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PKV_DM
         return;
     }
     const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     __builtin_assume(wave >= 0 && wave < 4);
-    const int t = tid & 31, hw = tid >> 5;
+    int lane = tid & 63, t = tid & 31, hw = tid >> 5;
     const int bh = b * p.Hkv + h;
     const int n_hid_k = p.B * p.Hkv;
 
@@ -413,9 +413,22 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PKV_DM
         if (l16p < 256u) dma_b128(rs_p, dst_p, lane16);
     };
 
+    // this wave's query rows, there before the first copy goes out (the compiler's wait for them would wait for the copies too):
+    // splitting them into digits then lies under the copy's flight
+    float q_row[GW][2];
+#pragma unroll
+    for (int gi = 0; gi < GW; gi++) {
+        const int g = min(wave + 4 * gi, p.Gq - 1);
+        const size_t qoff = ((size_t)b * p.Hq + (size_t)h * p.Gq + g) * kHeadDim;
+        q_row[gi][0] = a_ld16(p.q, qoff + lane, p.dtype);
+        q_row[gi][1] = a_ld16(p.q, qoff + 64 + lane, p.dtype);
+    }
+
     // tile 0 starts its way into slot 0 now, under the prologue's arithmetic
     int t_cur = first_tiles(0), t1 = first_tiles(1), t2 = first_tiles(2), t3 = first_tiles(3);
     TileInfo i0 = pack_info(load_info(t_cur)), i1 = pack_info(load_info(t1)), i2 = pack_info(load_info(t2));
+#pragma unroll
+    for (int gi = 0; gi < GW; gi++) asm volatile("" : "+v"(q_row[gi][0]), "+v"(q_row[gi][1]));
     dma_issue(IntC<0>{}, t_cur, i0);
 
     auto cvt2 = [&](uint32_t w, float &lo, float &hi) {
@@ -437,13 +450,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PKV_DM
     if (tid < 8) { st_m[tid] = -INFINITY; st_l[tid] = 0.f; st_z[tid] = 0.f; st_a[tid] = 1.f; st_a[8 + tid] = 1.f; resc[tid] = 0u; }
     __builtin_amdgcn_s_waitcnt(0xC07F);       // lgkmcnt(0): the zeroes are written; the copy in flight is not waited for
     __builtin_amdgcn_s_barrier();
-    for (int g = wave; g < G; g += 4) {
+#pragma unroll
+    for (int gi = 0; gi < GW; gi++) {
+        const int g = wave + 4 * gi;
+        if (g >= G) continue;
         if (g >= p.Gq) {                       // an idle head slot (group of 3 in the kernel of 4, ...): a query of zeros
             if (lane == 0) { qsum[g] = 0.f; qs[g] = 0.f; }
             continue;
         }
-        const size_t qoff = ((size_t)b * p.Hq + (size_t)h * p.Gq + g) * kHeadDim;
-        const float q0 = a_ld16(p.q, qoff + lane, p.dtype), q1 = a_ld16(p.q, qoff + 64 + lane, p.dtype);
+        const float q0 = q_row[gi][0], q1 = q_row[gi][1];
         const float mx = wave_max(fmaxf(fabsf(q0), fabsf(q1)));
         const float sm = wave_sum(q0 + q1);
         const float inv = mx > 0.f ? 1048576.f / mx : 0.f;
@@ -625,7 +640,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PKV_DM
     uint32_t ethr_pair = 0u;
     int stale_factors = 0;           // this wave published factors != 1 in the previous step: put them back to 1
     auto softmax_stage = [&](auto slot_c, const uint8_t *kt) {
-        constexpr int slot = decltype(slot_c)::value;
+        const int slot = slot_c;
         const uint32_t *par = reinterpret_cast<const uint32_t *>(ring + slot * Geo::kSlot + Geo::kParOff) + lane;
         const uint32_t vs_raw = par[128];
         float ks0, ks1, kz0, kz1, vs0, vs1, vz0, vz1;
@@ -738,7 +753,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PKV_DM
     const lds_half4_ptr aw_ptr = (lds_half4_ptr)aw_addr;
 #pragma clang diagnostic pop
     auto v_stage = [&](auto slot_c, const VUnit &vr) {
-        constexpr int slot = decltype(slot_c)::value;
+        const int slot = slot_c;
         constexpr int TPW = VTPW, NWIN = VNWIN;
         const int seg = hw & 1;
         uint32_t w01[NWIN], w23[NWIN];
@@ -803,7 +818,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PKV_DM
     VUnit v_a, v_b;               // the two sets; the loop below is written out twice so that nothing is copied
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // tile 0 (issued before the prologue's arithmetic)
     PKV_LDS_BARRIER();                                    // ... and every wave has its q operands out of slot 1
-    dma_issue(IntC<1>{}, t1, i1);
+    if ((uint32_t)t1 < (uint32_t)tile_end) dma_issue(IntC<1>{}, t1, i1);
     parse(IntC<0>{}, i0, k_a, v_a);
     // the head's counter: tiles 5 nsplit + [old value, old value + size) belong to whoever added `size`
     const int n_dyn = n_tiles - 5 * p.nsplit;                   // tiles that are handed out by counter
@@ -874,7 +889,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PKV_DM
         __builtin_amdgcn_s_setprio(0);
         PKV_LDS_BARRIER();                                    // publishes the weights; slot s is free, tile t1 is parsed
         __builtin_amdgcn_s_setprio(Prio::D);
-        if (!(PKV_ATTN_PROBE & 1)) dma_issue(slot_c, t2, i2);
+        if (!(PKV_ATTN_PROBE & 1) && (uint32_t)t2 < (uint32_t)tile_end) dma_issue(slot_c, t2, i2);
         if (take) request(batch_of(cur_base));                // collected at the wait above, a step or more from now
         __builtin_amdgcn_s_setprio(Prio::V);
         if (!(PKV_ATTN_PROBE & 8)) v_stage(slot_c, vcur);
@@ -883,12 +898,31 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PKV_DM
         i1 = i2; i2 = pack_info(i3);
         s++;
     };
-    while ((uint32_t)t_cur < (uint32_t)tile_end) {
-        step(IntC<0>{}, k_a, v_a, k_b, v_b);
-        if (!((uint32_t)t_cur < (uint32_t)tile_end)) break;
-        step(IntC<1>{}, k_b, v_b, k_a, v_a);
+    // The last tile is a step of its own without the copy, the wait and the parse of a next one, and tiles past the end are
+    // not copied: a member's first step used to bring two tiles that nobody reads.  (One tile a member: 1 x 32 heads x 4096
+    // tokens 13.0 -> 11.2 us, 1 x 8 x 1024 9.9 -> 8.8; two: 4 x 8 x 8192 18.4 -> 16.7; four of 5-bit codes 24.3 -> 23.4; 32 tiles: no
+    // difference; steps of a graph, with their merge.)  Its slot is a run-time value: one copy of the code serves both.
+    if ((uint32_t)t_cur < (uint32_t)tile_end) {
+        int slot = 0;
+        while ((uint32_t)t1 < (uint32_t)tile_end) {
+            step(IntC<0>{}, k_a, v_a, k_b, v_b);
+            if (!((uint32_t)t1 < (uint32_t)tile_end)) { slot = 1; k_a = k_b; v_a = v_b; break; }
+            step(IntC<1>{}, k_b, v_b, k_a, v_a);
+        }
+        // (what the last step derives from the lane number is formed here: kept through the loop it was spilled)
+        asm volatile("" : "+v"(lane), "+v"(t), "+v"(hw));
+        uint8_t *kt = ring + slot * Geo::kSlot;
+        __builtin_amdgcn_s_setprio(Prio::K);
+        if (!(PKV_ATTN_PROBE & 2)) k_stage(k_a, kt);
+        PKV_LDS_BARRIER();
+        __builtin_amdgcn_s_setprio(Prio::S);
+        if (!(PKV_ATTN_PROBE & 4)) softmax_stage(slot, kt);
+        PKV_LDS_BARRIER();
+        __builtin_amdgcn_s_setprio(Prio::V);
+        if (!(PKV_ATTN_PROBE & 8)) v_stage(slot, v_a);
+        __builtin_amdgcn_s_setprio(0);
     }
-    // drain: the copy issued in the last step must land before the workgroup's LDS is released
+    // drain: a request for tiles that is still under way
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     // the last member of the head to get here (every request of the others has been answered) zeroes the head's two
     // counters for the next launch

@@ -631,3 +631,21 @@ def test_attn_decode_takes_q_v_window_and_result_at_any_element(cuda, dtype, B, 
         want = ops.attn_decode(q, ke, ve, kw, vw, out_f32=f32)
         got = ops.attn_decode(shifted(q), ke, ve, kw, shifted(vw), out=shifted(torch.zeros_like(want)), out_f32=f32)
         assert torch.equal(got, want)
+
+
+# One member per head with 1..4 tiles (the last one in either slot), members that draw their tiles from a counter.
+@pytest.mark.parametrize("B,Hkv,tiles", [(64, 16, 1), (64, 16, 2), (64, 16, 3), (64, 16, 4), (32, 16, 25), (32, 16, 26)])
+@pytest.mark.parametrize("Hq_per,rel,dtype", [(1, 0.1, torch.float16), (4, 0.1, torch.bfloat16), (4, 0.05, torch.float16), (8, 0.2, torch.float16)])
+def test_attn_decode_last_tile_of_a_member(cuda, B, Hkv, tiles, Hq_per, rel, dtype):
+    if tiles > 4 and Hq_per == 8:
+        B //= 2
+    k, v = synth.make_kv(B, Hkv, 128 * tiles, seed=tiles, dtype=dtype, device=cuda)
+    q = synth.make_q(B, Hq_per * Hkv, seed=9, dtype=dtype, device=cuda)
+    ke, ve = ops.k_quant_encode(k, rel), ops.v_quant_encode(v, rel)
+    plain = ops.attn_decode(q, ke, ve, variant=1, out_f32=True)
+    # weights rounded to 11 bits (each side's error at most 2^-11 of the weights' sum times the largest value); scores from
+    # q split to 2^-21 of its row's maximum
+    bound = 2 ** -10 * v.float().abs().amax(dim=(2, 3)).repeat_interleave(Hq_per, 1).unsqueeze(-1)
+    for _ in range(2):                            # (twice: counters and flags are left as they were found)
+        fast = ops.attn_decode(q, ke, ve, out_f32=True)
+        assert bool(((fast - plain).abs() <= bound).all())
