@@ -385,3 +385,34 @@ def test_code_matrix_encode_by_group_count(cuda, oracle_codec, heads, T, bits):
         size = (ops.k_encode if is_k else ops.v_encode)(codes.to(cuda), stream, info, cb, hb, bits)
         assert size == zo and np.array_equal(info.cpu().numpy(), io)
         assert np.array_equal(stream[:zo].cpu().numpy(), so[:zo]) and not bool(stream[zo:].any())
+
+
+@pytest.mark.parametrize("stage", [1 << 25, 70000, 4097])
+@pytest.mark.parametrize("is_k", [True, False])
+def test_host_tensors_in_pieces(cuda, monkeypatch, is_k, stage):
+    """The host round trip in one, some and many pieces; what lies behind the stream in the caller's buffer stays, and a
+    block_info that points past the buffer reads no further than the buffer."""
+    monkeypatch.setattr(ops, "_STAGE_BYTES", stage)
+    codes = torch.randint(0, 16, (384, 1024), generator=torch.Generator().manual_seed(3), dtype=torch.uint8)
+    cb, hb = (64, 128) if is_k else (128, 64)
+    n = codes.numel() // 8192
+    enc, dec = (ops.k_encode_cpu, ops.k_decode_cpu) if is_k else (ops.v_encode_cpu, ops.v_decode_cpu)
+    room = n * ops.block_bound(is_k, cb, hb, 4) + 5000
+    d_stream, d_info = torch.zeros(room, dtype=torch.uint8, device=cuda), torch.zeros(n, 2, dtype=torch.uint32, device=cuda)
+    want = enc(codes.to(cuda), d_stream, d_info, 384, 1024, cb, hb, 4)
+    stream, info = torch.full((room,), 99, dtype=torch.uint8), torch.zeros(n, 2, dtype=torch.uint32)
+    assert enc(codes, stream, info, 384, 1024, cb, hb, 4) == want
+    assert torch.equal(stream[:want], d_stream[:want].cpu()) and bool((stream[want:] == 99).all())
+    assert torch.equal(info.view(torch.int32), d_info.cpu().view(torch.int32))
+    back = torch.zeros_like(codes)
+    dec(stream, info, back, 384, 1024, cb, hb, 4)
+    assert torch.equal(back, codes)
+    exact = stream[:want].clone()                             # a buffer that ends with the stream
+    back.zero_()
+    dec(exact, info, back, 384, 1024, cb, hb, 4)
+    assert torch.equal(back, codes)
+    bad = info.view(torch.int32).clone()
+    bad[n - 1] = torch.tensor([-16, 4000], dtype=torch.int32)       # 4 GiB - 16: outside
+    back.zero_()
+    dec(exact, bad.view(torch.uint32), back, 384, 1024, cb, hb, 4)
+    assert torch.equal(back[:256], codes[:256])
