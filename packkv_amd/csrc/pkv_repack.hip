@@ -662,6 +662,194 @@ greedy_order_sliced_kernel(const uint8_t *__restrict__ k_codes, const uint8_t *_
     }
 }
 
+// ---- the same for rows of up to 2048 channels, K and V together: one workgroup holds a block by itself ----
+// Four channels to a thread, kept as 16-bit lanes (even and odd bytes apart: two registers a token, nothing to unpack at
+// a pick), so that a block is priced by two wavefronts a SIMD instead of one, 3.0 vector instructions a channel instead of
+// 3.7; and with nobody to exchange sums with there is no state, no ticket and no closing launch.  What is left of a step
+// is the chain price -> sums -> winner -> move.
+// 256 blocks of 64 tokens x 2048 channels: 193 us, 223 with eight channels to a thread; x 1024 channels (256 threads) 149 us, 218
+// with half of 256 threads idle.
+__device__ __forceinline__ void price4x2(uint32_t ea, uint32_t oa, uint32_t eb, uint32_t ob, const uint32_t (&mn)[2], const uint32_t (&mx)[2],
+                                         uint32_t &sum_a, uint32_t &sum_b) {
+    const uint32_t v[4] = {ea, eb, oa, ob};
+    ushort2v hi[4], lo[4];
+    uint32_t e[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) hi[i] = __builtin_elementwise_max(__builtin_bit_cast(ushort2v, v[i]), __builtin_bit_cast(ushort2v, mx[i >> 1]));
+#pragma unroll
+    for (int i = 0; i < 4; i++) lo[i] = __builtin_elementwise_min(__builtin_bit_cast(ushort2v, v[i]), __builtin_bit_cast(ushort2v, mn[i >> 1]));
+#pragma unroll
+    for (int i = 0; i < 4; i++) hi[i] -= lo[i];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const half2v f = __builtin_elementwise_fma(__builtin_bit_cast(half2v, hi[i]), (half2v){(_Float16)32768.0f, (_Float16)32768.0f},
+                                                   (half2v){(_Float16)0.0009765625f, (_Float16)0.0009765625f});
+        e[i] = __builtin_bit_cast(uint32_t, f);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) e[i] &= 0x7C007C00u;
+    sum_a = __builtin_amdgcn_sad_u16(e[2], 0u, __builtin_amdgcn_sad_u16(e[0], 0u, 0u));
+    sum_b = __builtin_amdgcn_sad_u16(e[3], 0u, __builtin_amdgcn_sad_u16(e[1], 0u, 0u));
+}
+
+template <int THREADS>
+__global__ void __launch_bounds__(THREADS, 2)
+greedy_order_block_kernel(const uint8_t *__restrict__ k_codes, const uint8_t *__restrict__ v_codes, int hidden, int N, int pack_len,
+                          uint32_t *__restrict__ perm) {
+    constexpr int kRuns = THREADS / 32, kPartStride = kRuns * 36 + 4, kSeedParts = THREADS / 128;
+    __shared__ __attribute__((aligned(16))) uint32_t s_part[32 * kPartStride];   // picks: [pair of slots][thread], padded
+    __shared__ uint32_t s_seed[128 * 32];            // seeds: [2 * slot + (0: dot, 1: squared norm)][adder]
+    __shared__ uint32_t s_tot[64];
+    __shared__ uint32_t s_key[128];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int ch = tid * 4;
+    const uint8_t *col = ch < hidden ? k_codes + ch : v_codes + (ch - hidden);
+    const bool have = ch < 2 * hidden;
+    const int adder = (tid >> 2) & 31;               // the LDS word that takes the sums of the thread's four lanes
+    const bool quad_first = (tid & 3) == 0;
+    const int part_word = (tid >> 5) * 36 + (tid & 31), part_read = (tid / kRuns) * kPartStride + (tid % kRuns) * 36;
+    const size_t row0 = (size_t)blockIdx.x * N;
+    u32x32 ev[2], ov[2];
+#define xe(t) ev[(t) >> 5][(t) & 31]
+#define xo(t) ov[(t) >> 5][(t) & 31]
+#pragma unroll
+    for (int t = 0; t < kSlicedTokens; t++) {
+        uint32_t v = 0u;
+        if (t < N && have) v = *reinterpret_cast<const uint32_t *>(col + (row0 + t) * (size_t)hidden);
+        xe(t) = bytes_even(v);
+        xo(t) = bytes_odd(v);
+    }
+    uint32_t orig = (uint32_t)lane;                  // the token in slot `lane`
+    int n_alive = N, picked = 0;
+    uint32_t mn[2], mx[2];
+    for (int step = 0; step < N / pack_len * pack_len; step++) {
+        const bool seed = step % pack_len == 0;
+        int sel = -1;
+        if (seed) {
+            // ---- seed: rounded mean of the remaining tokens, then the best cosine ----
+            uint32_t sum[2] = {0u, 0u};
+#pragma unroll
+            for (int t8 = 0; t8 < kSlicedTokens; t8 += 8) {
+                if (t8 < n_alive) {
+#pragma unroll
+                    for (int t = t8; t < t8 + 8; t++)
+                        if (t < n_alive) { sum[0] += xe(t); sum[1] += xo(t); }
+                }
+            }
+            const float na = (float)n_alive;           // mean(dim=1).round(): fp32 quotient, round half to even
+            const uint32_t mean = (uint32_t)rintf((float)(sum[0] & 0xFFFFu) / na) | ((uint32_t)rintf((float)(sum[1] & 0xFFFFu) / na) << 8) |
+                                  ((uint32_t)rintf((float)(sum[0] >> 16) / na) << 16) | ((uint32_t)rintf((float)(sum[1] >> 16) / na) << 24);
+            for (int i = tid; i < 128 * 32; i += THREADS) s_seed[i] = 0u;
+            __syncthreads();
+#pragma unroll
+            for (int t8 = 0; t8 < kSlicedTokens; t8 += 8) {
+                if (t8 < n_alive) {
+#pragma unroll
+                    for (int t = t8; t < t8 + 8; t++)
+                        if (t < n_alive) {
+                            const uint32_t x = xe(t) | (xo(t) << 8);
+                            const uint32_t dot = quad_sum(__builtin_amdgcn_udot4(x, mean, 0u, false)), nx = quad_sum(__builtin_amdgcn_udot4(x, x, 0u, false));
+                            if (quad_first) {
+                                atomicAdd(&s_seed[(2 * t) * 32 + adder], dot);
+                                atomicAdd(&s_seed[(2 * t + 1) * 32 + adder], nx);
+                            }
+                        }
+                }
+            }
+            __syncthreads();
+            {   // value v: two or four adjacent threads add 16 or 8 adders each
+                const int v = tid / kSeedParts, part = tid % kSeedParts;
+                uint32_t a = 0u;
+#pragma unroll
+                for (int i = 0; i < 32 / kSeedParts; i++) a += s_seed[v * 32 + part * (32 / kSeedParts) + i];
+                a += lane_move<0xB1, 0xF, false>(0u, a);
+                if (kSeedParts == 4) a += lane_move<0x4E, 0xF, false>(0u, a);
+                if (part == 0) s_key[v] = a;
+            }
+            __syncthreads();
+            unsigned long long bd = 0, bn = 0;
+            uint32_t bo = orig;
+            if (lane < n_alive) {
+                sel = lane;
+                bd = s_key[2 * lane];
+                bn = s_key[2 * lane + 1];
+            }
+#pragma unroll
+            for (int d = 32; d >= 1; d >>= 1) {        // equal cosines: the earlier token
+                const int os = __shfl_xor(sel, d, 64);
+                const uint32_t oo = __shfl_xor(bo, d, 64);
+                const unsigned long long od = __shfl_xor(bd, d, 64), on = __shfl_xor(bn, d, 64);
+                if (os >= 0 && (sel < 0 || cos_greater(od, on, bd, bn) || (!cos_greater(bd, bn, od, on) && oo < bo))) {
+                    sel = os; bo = oo; bd = od; bn = on;
+                }
+            }
+            sel = __builtin_amdgcn_readfirstlane(sel);
+        } else {
+            // ---- the pack's other tokens: fewest bits after the pick ----
+#pragma unroll
+            for (int k4 = 0; k4 < kSlicedTokens / 2; k4 += 4) {
+                if (2 * k4 < n_alive) {
+#pragma unroll
+                    for (int k = k4; k < k4 + 4; k++)
+                        if (2 * k < n_alive) {
+                            // (with an odd count the slot past the last one is priced as well: a bounded sum nobody reads)
+                            uint32_t a0, a1;
+                            price4x2(xe(2 * k), xo(2 * k), xe(2 * k + 1), xo(2 * k + 1), mn, mx, a0, a1);
+                            s_part[k * kPartStride + part_word] = (a0 >> 10) | (a1 << 6);   // sums of fields at bit 10: a 16-bit lane per slot
+                        }
+                }
+            }
+            __syncthreads();
+            {   // pair k: kRuns adjacent threads add 32 words each
+                const int k = tid / kRuns, part = tid % kRuns;
+                const uint4 *src = reinterpret_cast<const uint4 *>(s_part + part_read);
+                uint32_t a = 0u;
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    const uint4 w = src[i];
+                    a += w.x + w.y + w.z + w.w;
+                }
+                a = sum8_down(a);
+                if (kRuns == 16) a += lane_move<0x108, 0xF, true>(0u, a);
+                if (part == 0 && 2 * k < n_alive) {
+                    s_tot[2 * k] = a & 0xFFFFu;
+                    s_tot[2 * k + 1] = a >> 16;
+                }
+            }
+            __syncthreads();
+            // (cost, token) in one word: the minimum is the first cheapest token
+            const uint32_t key = lane < n_alive ? (s_tot[lane] << 8) | orig : 0xFFFFFFFFu;
+            const uint32_t best = wave_min_u32(key);
+            sel = (int)__builtin_ctzll(__ballot(key == best));
+        }
+        // the winner in slot `sel` leaves: its rows widen the pack's ranges and the last slot moves into `sel`
+        const int last = n_alive - 1;
+        const uint32_t tok = (uint32_t)__builtin_amdgcn_readlane((int)orig, sel);
+        const uint32_t moved = (uint32_t)__builtin_amdgcn_readlane((int)orig, last);
+        if (lane == sel) orig = moved;
+        // (both halves of the slot arrays are read and written at the index modulo 32, with what they hold unless
+        // the slot lies in them: no branch, so the arrays stay where they are)
+        const int li = last & 31, si = sel & 31;
+        const uint32_t la0 = ev[0][li], la1 = ov[0][li], lb0 = ev[1][li], lb1 = ov[1][li];
+        const uint32_t l0 = last < 32 ? la0 : lb0, l1 = last < 32 ? la1 : lb1;
+        const uint32_t sa0 = ev[0][si], sa1 = ov[0][si], sb0 = ev[1][si], sb1 = ov[1][si];
+        const uint32_t w0 = sel < 32 ? sa0 : sb0, w1 = sel < 32 ? sa1 : sb1;
+        ev[0][si] = sel < 32 ? l0 : sa0;
+        ov[0][si] = sel < 32 ? l1 : sa1;
+        ev[1][si] = sel < 32 ? sb0 : l0;
+        ov[1][si] = sel < 32 ? sb1 : l1;
+        if (tid == 0) perm[row0 + picked] = tok;
+        picked++;
+        n_alive--;
+        mn[0] = seed ? w0 : pk_min_u16(mn[0], w0);
+        mx[0] = seed ? w0 : pk_max_u16(mx[0], w0);
+        mn[1] = seed ? w1 : pk_min_u16(mn[1], w1);
+        mx[1] = seed ? w1 : pk_max_u16(mx[1], w1);
+    }
+#undef xe
+#undef xo
+}
+
 // ---- out row r = in row perm[r], for K and V at once: grid (ctx_len), 256 threads ----
 __global__ void __launch_bounds__(256) gather_rows_kernel(const uint8_t *__restrict__ k_in, const uint8_t *__restrict__ v_in,
                                                           uint8_t *__restrict__ k_out, uint8_t *__restrict__ v_out,
@@ -882,6 +1070,22 @@ int pkv_greedy_repack(const uint8_t *k_codes, const uint8_t *v_codes, uint8_t *k
                 "block_size must be a multiple of pack_len (the reference drops the tokens of an incomplete pack)");
     const uint32_t nblocks = (uint32_t)(ctx_len / block_size);
     // blocks of up to 64 tokens: register-resident channel slices, as many groups of workgroups as fit the device;
+    int rc;
+    // K and V rows of up to 1024 channels together: a workgroup of 256 threads to a block.  Up to 2048: one of 512, while the blocks do
+    // not outnumber the CUs (256 blocks 235 -> 204 us, the gather included; 512 blocks 345 against 390: two workgroups of the sliced
+    // kernel on a CU fill each other's gaps).
+    const bool small = 2 * (size_t)hidden_dim <= 4u * kSlicedThreadsNarrow;
+    if (block_size <= kSlicedTokens && (small || (2 * (size_t)hidden_dim <= 4u * kSlicedThreadsWide && nblocks <= 256u))) {
+        LaunchTimer tm(s, ms_out != nullptr);
+        if ((rc = tm.begin())) return rc;
+        if (small)
+            greedy_order_block_kernel<kSlicedThreadsNarrow><<<nblocks, kSlicedThreadsNarrow, 0, s>>>(k_codes, v_codes, hidden_dim, block_size, pack_len, perm);
+        else
+            greedy_order_block_kernel<kSlicedThreadsWide><<<nblocks, kSlicedThreadsWide, 0, s>>>(k_codes, v_codes, hidden_dim, block_size, pack_len, perm);
+        if (rows) gather_rows_kernel<<<(unsigned)ctx_len, 256, 0, s>>>(k_codes, v_codes, k_out, v_out, perm, block_size, hidden_dim);
+        PKV_HIP_CHECK(hipGetLastError());
+        return tm.end(ms_out);
+    }
     // rows of more than one narrow slice go to the wide workgroups, which have a CU to themselves: two members of a
     // group on one CU, or another group's member in the same phase, would price at half speed and hold up their group
     const bool wide = 2 * (size_t)hidden_dim > 8u * kSlicedThreadsNarrow;
@@ -908,7 +1112,6 @@ int pkv_greedy_repack(const uint8_t *k_codes, const uint8_t *v_codes, uint8_t *k
         groups = it->second / members;
         if (groups > nblocks) groups = nblocks;
     }
-    int rc;
     if (groups > 0) {
         ScanHandle sh;
         if ((rc = prepare_scan_state(groups * 2u * members * 128u, &sh, s, ms_out != nullptr))) return rc;

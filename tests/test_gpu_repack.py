@@ -389,3 +389,22 @@ def test_fused_median_repack_at_the_benchmark_shape(cuda):
             m = med.view(-1, 64)
             assert bool((m[:, 1:] <= m[:, :-1]).all())
         del cf, cn
+
+
+@pytest.mark.parametrize("hid,T,bs,pack,top", [(16, 128, 64, 16, 256), (512, 128, 64, 16, 12), (528, 96, 48, 16, 16), (1024, 64, 64, 64, 24),
+                                               (1024, 64, 32, 8, 2), (992, 80, 16, 16, 200)])
+def test_greedy_order_with_a_block_to_a_workgroup(cuda, hid, T, bs, pack, top):
+    g = torch.Generator().manual_seed(hid + T)
+    kc, vc = (torch.randint(0, top, (T, hid), dtype=torch.uint8, generator=g) for _ in range(2))
+    _, order = orp.greedy_repacking(orp.blocks_from_code_matrices(kc.numpy(), vc.numpy(), bs), pack)
+    perm = ops.greedy_order(kc.to(cuda), vc.to(cuda), pack, bs)
+    assert (perm.cpu().numpy().reshape(-1, bs) == order).all()
+
+
+def test_greedy_order_does_not_depend_on_the_number_of_blocks(cuda):
+    """256 blocks of 2048 channels take a workgroup each, 257 the workgroups that walk several blocks."""
+    g = torch.Generator(device=cuda)
+    g.manual_seed(4)
+    kc, vc = (torch.randint(0, 12, (257 * 64, 1024), dtype=torch.uint8, generator=g, device=cuda) for _ in range(2))
+    many = ops.greedy_order(kc, vc, 16, 64)
+    assert torch.equal(many[:256 * 64], ops.greedy_order(kc[:256 * 64], vc[:256 * 64], 16, 64))
