@@ -217,11 +217,14 @@ int pkv_window_cut(const pkv_cut_args *args, pkv_stream_t s);
  *   `pack_len` consecutive tokens of one channel; returns  len_sum = sum over packs of
  *   bit_length(max - min)  and the number of distinct code values, from which the caller forms
  *   bytes = (len_sum * pack_len + n_packs * (W + ceil(log2(W + 1)))) / 8,  W = ceil(log2(n_unique)).
+ * pkv_bit_pack_size_pair: the same for K and V with one wait; with `perm` (else NULL, block_size ignored) for the matrices a
+ *   repacking of blocks of `block_size` tokens (a multiple of pack_len that divides ctx_len) in that order would give,
+ *   without writing them.
  * pkv_median_repack (utils/compute.py:262-270, `median_repacking`): inside every block of
  *   `block_size` tokens the tokens of K and V are reordered together by descending lower median
  *   of the token's V codes over all hidden_dim channels.  Equal medians keep their original order
  *   (the reference leaves that order to torch.sort's backend).  perm[blk * block_size + r] is
- *   the index inside the block of the token that moves to position r. */
+ *   the index inside the block of the token that moves to position r.  k_out = v_out = NULL: the order only. */
 /* Median repacking inside the fused encode (quantize, token repack and bit-pack as one encode; reference
  * order utils/compute.py:329-357: quantise, repack, bit-pack): no code matrix is formed.
  * pkv_median_order: the permutation pkv_median_repack would produce for V [B, H, T, 128] quantised at `rel` -- the
@@ -243,6 +246,8 @@ int pkv_v_quant_encode_perm(const void *x, int dtype, int B, int H, int T, float
                             uint32_t *block_info, void *scale, void *zero, uint64_t *size_out, float *ms_out, pkv_stream_t s);
 int pkv_bit_pack_size(const uint8_t *codes, int ctx_len, int hidden_dim, int pack_len, uint64_t *len_sum_out,
                       uint32_t *n_unique_out, float *ms_out, pkv_stream_t s);
+int pkv_bit_pack_size_pair(const uint8_t *k_codes, const uint8_t *v_codes, const uint32_t *perm, int block_size, int ctx_len,
+                           int hidden_dim, int pack_len, uint64_t len_sum_out[2], uint32_t n_unique_out[2], pkv_stream_t s);
 int pkv_median_repack(const uint8_t *k_codes, const uint8_t *v_codes, uint8_t *k_out, uint8_t *v_out, uint32_t *perm,
                       int ctx_len, int hidden_dim, int block_size, float *ms_out, pkv_stream_t s);
 /* pkv_greedy_repack (utils/compute.py:210-260, `greedy_repacking`, with `_batched_pick` :186-208): every block of

@@ -70,16 +70,18 @@ def crs_evaluation_with_data(config, key_caches, value_caches, device="cuda"):
     for k, v in zip(key_caches, value_caches):
         if k.shape != v.shape or k.dim() != 4 or k.size(2) % config.block_size:
             raise RuntimeError("K and V must be [B, H, T, D] of one shape with T a multiple of block_size")
-        codes, orig, before = {}, {}, {}
+        codes, pars, orig, before = {}, {}, {}, {}
         for side, x, rel in (("k", k, config.k_quant_scale_rel), ("v", v, config.v_quant_scale_rel)):
             xd = x.to(device).contiguous()
-            c, scale, zero = ops.quant_codes(xd, rel)
-            codes[side] = c
+            codes[side], scale, zero = ops.quant_codes(xd, rel)
+            pars[side] = zero.numel() + scale.numel()
             orig[side] = x.numel() * x.element_size()
+        stats = ops.code_stats_pair(codes["k"], codes["v"], config.pack_size)
+        for side, x, (len_sum, n_unique) in (("k", k, stats[0]), ("v", v, stats[1])):
+            c = codes[side]
             # every code at quant_bit_num bits plus one zero and one scale per (batch, token) in the storage dtype
-            len_sum, n_unique = ops.code_stats(c, config.pack_size)
             before[side] = ops._packed_bytes(c, config.pack_size, len_sum, n_unique)
-            quant_size = c.numel() * _bit_num(n_unique) // 8 + (zero.numel() + scale.numel()) * x.element_size()
+            quant_size = c.numel() * _bit_num(n_unique) // 8 + pars[side] * x.element_size()
             res[side + "_original_size"].append(orig[side])
             res[side + "_quant_size"].append(quant_size)
             res[side + "_quant_cr"].append(orig[side] / quant_size)

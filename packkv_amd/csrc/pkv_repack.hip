@@ -878,7 +878,7 @@ constexpr int kPackSizeDone = 52;       // fewer than 2^12 workgroups; 2^52 bits
 // one after the other, so their number, not the bytes, would set the time of a grid with a workgroup per pack -- and the
 // wavefronts of a CU share a workgroup of 1024 (one presence table to clear, one atomic) rather than having one each of four.
 // Random 4-bit codes, packs of 16, a call's kernel time: 32768 x 16384 codes 113 us (174 with up to 2048 workgroups of 256
-// threads and 16 channels a thread), 16384 x 4096 37.6 (60.6), 16384 x 1024 19.6 (21.1), 256 x 512 9.4 (12.6).
+// threads and 16 channels a thread), 16384 x 4096 31 (60.6), 16384 x 1024 19.6 (21.1), 256 x 512 9.4 (12.6).
 // Bound by instruction issue: 7 vector instructions per dword for the ranges and 8 for the presence flags (a
 // register bit mask for values below 32 instead of the LDS flags costs the same).
 // The last workgroup to finish hands the result to the waiting host thread (a tagged slot in pinned memory) and leaves
@@ -888,10 +888,21 @@ constexpr int kPackSizeDone = 52;       // fewer than 2^12 workgroups; 2^52 bits
 // addition to `sum` (which also counts it done): no fence, no cached read of another workgroup's data.
 typedef unsigned short pk_u16x2 __attribute__((ext_vector_type(2)));
 
-template <int WORDS>
-__global__ void __launch_bounds__(1024) pack_size_kernel(const uint8_t *__restrict__ codes, int hidden, int pack_len,
-                                                        size_t n_items, PackSizeState *st, unsigned long long *slot,
-                                                        uint32_t tag) {
+// One or two matrices of one shape (K and V: blockIdx.y), whose last workgroups report apart; with PERM the rows of a block of
+// `block_size` tokens (a multiple of the pack) in the order of a repacking: row r of block b is row perm[b * block_size + r] of it, so that
+// a repacked matrix need not be written to be priced (16384 x 2 x 1024 codes: 27.1 us a call; written first, 25.5 and 11 for the gather).
+struct PackSizeJob {
+    const uint8_t *codes[2];
+    PackSizeState *st;                   // one for each matrix
+    unsigned long long *slot;            // three words for each matrix
+    const uint32_t *perm;
+    int block_size;
+};
+template <int WORDS, bool PERM>
+__global__ void __launch_bounds__(1024) pack_size_kernel(const PackSizeJob job, int hidden, int pack_len, size_t n_items, uint32_t tag) {
+    const uint8_t *__restrict__ codes = job.codes[blockIdx.y];
+    PackSizeState *st = job.st + blockIdx.y;
+    unsigned long long *slot = job.slot + 3 * blockIdx.y;
     // a presence word per (code value, lane % 32): a lane marks its own column, so the marks of a wavefront never
     // share a bank however few values the matrix holds (one word per value made every mark a same-address conflict)
     __shared__ __align__(16) uint32_t seen[256 * 32];
@@ -906,12 +917,16 @@ __global__ void __launch_bounds__(1024) pack_size_kernel(const uint8_t *__restri
     for (size_t item = (size_t)blockIdx.x * blockDim.x + threadIdx.x; item < n_items; item += (size_t)gridDim.x * blockDim.x) {
         const size_t pack = item / chunks;
         const uint32_t chunk = (uint32_t)(item - pack * chunks);
-        const uint8_t *p = codes + pack * (size_t)pack_len * hidden + (size_t)chunk * (4 * WORDS);
+        const size_t tok0 = pack * (size_t)pack_len;
+        // PERM: the block's first row; the pack's entries of the order
+        const size_t row0 = PERM ? tok0 / (size_t)job.block_size * (size_t)job.block_size : tok0;
+        const uint8_t *p = codes + row0 * hidden + (size_t)chunk * (4 * WORDS);
+        const uint32_t *order = PERM ? job.perm + tok0 : nullptr;
         pk_u16x2 mn[2 * WORDS], mx[2 * WORDS];
 #pragma unroll
         for (int i = 0; i < 2 * WORDS; i++) { mn[i] = (pk_u16x2){255, 255}; mx[i] = (pk_u16x2){0, 0}; }
         auto load = [&](int row) -> Words {
-            const uint8_t *at = p + (size_t)row * hidden;
+            const uint8_t *at = p + (size_t)(PERM ? (int)min(order[row], (uint32_t)job.block_size - 1u) : row) * hidden;
             if constexpr (WORDS == 4) return __builtin_bit_cast(Words, *reinterpret_cast<const uint4 *>(at));
             else return Words{{*reinterpret_cast<const uint32_t *>(at)}};
         };
@@ -987,51 +1002,69 @@ __global__ void __launch_bounds__(1024) pack_size_kernel(const uint8_t *__restri
     }
 }
 
+static int pack_sizes(const uint8_t *const *codes, int n, const uint32_t *perm, int block_size, int ctx_len, int hidden_dim, int pack_len,
+                      uint64_t *len_sum_out, uint32_t *n_unique_out, float *ms_out, hipStream_t s) {
+    PKV_REQUIRE(len_sum_out && n_unique_out, PKV_ERR_INVALID, "null pointer argument");
+    for (int i = 0; i < n; i++) PKV_REQUIRE(codes[i], PKV_ERR_INVALID, "null pointer argument");
+    PKV_REQUIRE(ctx_len > 0 && hidden_dim > 0 && pack_len > 0, PKV_ERR_INVALID, "sizes must be positive");
+    for (int i = 0; i < n; i++)
+        PKV_REQUIRE(hidden_dim % 16 == 0 && (reinterpret_cast<uintptr_t>(codes[i]) & 15u) == 0, PKV_ERR_INVALID,
+                    "hidden_dim must be a multiple of 16 and the code matrix 16-byte aligned");
+    PKV_REQUIRE(ctx_len % pack_len == 0, PKV_ERR_INVALID, "ctx_len must be divisible by the pack length");
+    PKV_REQUIRE(!perm || (block_size > 0 && block_size % pack_len == 0 && ctx_len % block_size == 0), PKV_ERR_INVALID,
+                "with a token order, ctx_len must be divisible by the block size and that by the pack length");
+    int rc;
+    OutcomeSlot slot;
+    if ((rc = slot.take(s))) return rc;
+    ScanHandle sh;
+    if ((rc = prepare_scan_state((uint32_t)(n * sizeof(PackSizeState) / 8), &sh, s, true))) return rc;
+    LaunchTimer tm(s, ms_out != nullptr);
+    if ((rc = tm.begin())) return rc;
+    // 16 channels to a thread once that fills the chip (two workgroups of 1024 per CU); below, 4 channels, and small
+    // workgroups while there is not one of 1024 for every CU (1024 x 1024 codes: 10.0 us, 12.8 with 16 channels a thread).  At
+    // most one of 1024 a CU: a second one clears and scans a presence table of its own and adds once more to the one sum (K and V
+    // of 16384 tokens, a call: 1024 channels 25.5 us, 28.4 with twice the workgroups; 2048 33.6, 40.7; 4096 43.4, 45.7; 16384 112, 117).
+    const size_t wide = (size_t)(ctx_len / pack_len) * (size_t)(hidden_dim / 16);
+    const bool large = n * wide >= 512u * 1024u;
+    const size_t n_items = large ? wide : 4 * wide;
+    const unsigned threads = n * n_items <= 256u * 256u ? 256u : 1024u;
+    const size_t wanted = (n_items + threads - 1) / threads, most = 256u / (unsigned)n;
+    PackSizeJob job{{codes[0], codes[n - 1]}, reinterpret_cast<PackSizeState *>(sh.st), (unsigned long long *)slot.words, perm, block_size};
+    auto kern = perm ? (large ? pack_size_kernel<4, true> : pack_size_kernel<1, true>) : (large ? pack_size_kernel<4, false> : pack_size_kernel<1, false>);
+    kern<<<dim3((unsigned)(wanted < most ? wanted : most), (unsigned)n), threads, 0, s>>>(job, hidden_dim, pack_len, n_items, slot.tag);
+    PKV_HIP_CHECK(hipGetLastError());
+    if ((rc = scan_state_cleared(sh, s))) return rc;
+    if ((rc = tm.end(ms_out))) return rc;
+    uint64_t v[6];
+    if ((rc = slot.wait(3 * n, s, v))) return rc;
+    for (int i = 0; i < n; i++) {
+        len_sum_out[i] = v[3 * i] | v[3 * i + 1] << 32;
+        n_unique_out[i] = (uint32_t)v[3 * i + 2];
+    }
+    return PKV_OK;
+}
+
 }  // namespace pkv
 
 extern "C" {
 
 int pkv_bit_pack_size(const uint8_t *codes, int ctx_len, int hidden_dim, int pack_len, uint64_t *len_sum_out,
-                      uint32_t *n_unique_out, float *ms_out, pkv_stream_t s_) {
-    using namespace pkv;
-    hipStream_t s = (hipStream_t)s_;
-    PKV_REQUIRE(codes && len_sum_out && n_unique_out, PKV_ERR_INVALID, "null pointer argument");
-    PKV_REQUIRE(ctx_len > 0 && hidden_dim > 0 && pack_len > 0, PKV_ERR_INVALID, "sizes must be positive");
-    PKV_REQUIRE(hidden_dim % 16 == 0 && (reinterpret_cast<uintptr_t>(codes) & 15u) == 0, PKV_ERR_INVALID,
-                "hidden_dim must be a multiple of 16 and the code matrix 16-byte aligned");
-    PKV_REQUIRE(ctx_len % pack_len == 0, PKV_ERR_INVALID, "ctx_len must be divisible by the pack length");
-    int rc;
-    OutcomeSlot slot;
-    if ((rc = slot.take(s))) return rc;
-    ScanHandle sh;
-    if ((rc = prepare_scan_state((uint32_t)(sizeof(PackSizeState) / 8), &sh, s, true))) return rc;
-    LaunchTimer tm(s, ms_out != nullptr);
-    if ((rc = tm.begin())) return rc;
-    // 16 channels to a thread once that fills the chip (two workgroups of 1024 per CU); below, 4 channels, and small
-    // workgroups while there is not one of 1024 for every CU (1024 x 1024 codes: 10.0 us, 12.8 with 16 channels a thread).
-    const size_t wide = (size_t)(ctx_len / pack_len) * (size_t)(hidden_dim / 16);
-    const bool large = wide >= 512u * 1024u;
-    const size_t n_items = large ? wide : 4 * wide;
-    const unsigned threads = n_items <= 256u * 256u ? 256u : 1024u;
-    const size_t wanted = (n_items + threads - 1) / threads;
-    auto kern = large ? pack_size_kernel<4> : pack_size_kernel<1>;
-    kern<<<(unsigned)(wanted < 512 ? wanted : 512), threads, 0, s>>>(
-        codes, hidden_dim, pack_len, n_items, reinterpret_cast<PackSizeState *>(sh.st), (unsigned long long *)slot.words, slot.tag);
-    PKV_HIP_CHECK(hipGetLastError());
-    if ((rc = scan_state_cleared(sh, s))) return rc;
-    if ((rc = tm.end(ms_out))) return rc;
-    uint64_t v[3];
-    if ((rc = slot.wait(3, s, v))) return rc;
-    *len_sum_out = v[0] | v[1] << 32;
-    *n_unique_out = (uint32_t)v[2];
-    return PKV_OK;
+                      uint32_t *n_unique_out, float *ms_out, pkv_stream_t s) {
+    const uint8_t *one[1] = {codes};
+    return pkv::pack_sizes(one, 1, nullptr, 0, ctx_len, hidden_dim, pack_len, len_sum_out, n_unique_out, ms_out, (hipStream_t)s);
+}
+
+int pkv_bit_pack_size_pair(const uint8_t *k_codes, const uint8_t *v_codes, const uint32_t *perm, int block_size, int ctx_len, int hidden_dim,
+                           int pack_len, uint64_t len_sum_out[2], uint32_t n_unique_out[2], pkv_stream_t s) {
+    const uint8_t *both[2] = {k_codes, v_codes};
+    return pkv::pack_sizes(both, 2, perm, block_size, ctx_len, hidden_dim, pack_len, len_sum_out, n_unique_out, nullptr, (hipStream_t)s);
 }
 
 int pkv_median_repack(const uint8_t *k_codes, const uint8_t *v_codes, uint8_t *k_out, uint8_t *v_out, uint32_t *perm,
                       int ctx_len, int hidden_dim, int block_size, float *ms_out, pkv_stream_t s_) {
     using namespace pkv;
     hipStream_t s = (hipStream_t)s_;
-    PKV_REQUIRE(k_codes && v_codes && k_out && v_out && perm, PKV_ERR_INVALID, "null pointer argument");
+    PKV_REQUIRE(k_codes && v_codes && perm && (k_out != nullptr) == (v_out != nullptr), PKV_ERR_INVALID, "null pointer argument");
     PKV_REQUIRE(k_codes != k_out && v_codes != v_out, PKV_ERR_INVALID, "repacking cannot run in place");
     PKV_REQUIRE(ctx_len > 0 && hidden_dim > 0 && block_size > 0, PKV_ERR_INVALID, "sizes must be positive");
     PKV_REQUIRE(hidden_dim % 16 == 0 && ((reinterpret_cast<uintptr_t>(k_codes) | reinterpret_cast<uintptr_t>(v_codes) |
@@ -1048,7 +1081,7 @@ int pkv_median_repack(const uint8_t *k_codes, const uint8_t *v_codes, uint8_t *k
     token_median_kernel<<<(unsigned)((ctx_len + 3) / 4), 256, 0, s>>>(v_codes, ctx_len, hidden_dim, median);
     const int threads = (block_size + 63) / 64 * 64;
     block_order_kernel<<<(unsigned)(ctx_len / block_size), threads, (size_t)block_size, s>>>(median, block_size, perm);
-    gather_rows_kernel<<<(unsigned)ctx_len, 256, 0, s>>>(k_codes, v_codes, k_out, v_out, perm, block_size, hidden_dim);
+    if (k_out) gather_rows_kernel<<<(unsigned)ctx_len, 256, 0, s>>>(k_codes, v_codes, k_out, v_out, perm, block_size, hidden_dim);
     PKV_HIP_CHECK(hipGetLastError());
     return tm.end(ms_out);
 }

@@ -684,6 +684,24 @@ def code_stats(codes, pack_len, timed=False):
     return out + (float(ms.value),) if timed else out
 
 
+def code_stats_pair(k_codes, v_codes, pack_len, perm=None, block_size=0):
+    """code_stats of K and of V (one shape) with one wait; with `perm` [ctx_len] (32 bits, as the repackings return it) of the
+    matrices in that order, which are not written: blocks of `block_size` tokens, a multiple of pack_len."""
+    _check_code_matrix(k_codes, "k_codes")
+    _check_code_matrix(v_codes, "v_codes")
+    _require(k_codes.shape == v_codes.shape, "K and V code matrices must have one shape")
+    _require(k_codes.get_device() == v_codes.get_device(), _ONE_DEVICE)
+    ctx, hidden = k_codes.shape
+    _require(perm is None or (perm.get_device() == k_codes.get_device() and perm.dtype in (torch.int32, torch.uint32) and perm.numel() == ctx
+                              and perm.is_contiguous()), "perm must hold one 32-bit index per token")
+    len_sum, n_unique = (ctypes.c_uint64 * 2)(), (ctypes.c_uint32 * 2)()
+    with _on(k_codes.device):
+        rc = _lib.load().pkv_bit_pack_size_pair(_ptr(k_codes), _ptr(v_codes), None if perm is None else _ptr(perm), int(block_size), ctx, hidden,
+                                                int(pack_len), len_sum, n_unique, _stream(k_codes.device))
+    _lib.check(rc)
+    return (len_sum[0], n_unique[0]), (len_sum[1], n_unique[1])
+
+
 def bit_pack_bytes(codes, pack_len, timed=False):
     """Analytic size of ONE code matrix [ctx_len, hidden] in bytes, as `bit_pack` prices each half
     (utils/compute.py:272-297): packs of `pack_len` consecutive tokens of one channel cost
@@ -703,7 +721,10 @@ def _packed_bytes(codes, pack_len, len_sum, n_unique):
 def bit_pack(k_codes, v_codes, pack_len):
     """(k_bytes, v_bytes) of `bit_pack(blocks, pack_len)` (utils/compute.py:272-297) for blocks = K and V codes
     side by side."""
-    return bit_pack_bytes(k_codes, pack_len), bit_pack_bytes(v_codes, pack_len)
+    if k_codes.shape != v_codes.shape or k_codes.get_device() != v_codes.get_device():
+        return bit_pack_bytes(k_codes, pack_len), bit_pack_bytes(v_codes, pack_len)
+    k, v = code_stats_pair(k_codes, v_codes, pack_len)
+    return _packed_bytes(k_codes, pack_len, *k), _packed_bytes(v_codes, pack_len, *v)
 
 
 def median_repacking(k_codes, v_codes, block_size=64, timed=False):
@@ -746,6 +767,20 @@ def greedy_repacking(k_codes, v_codes, pack_len=16, block_size=64, timed=False):
     return (k_out, v_out, perm, float(ms.value)) if timed else (k_out, v_out, perm)
 
 
+def _median_code_order(k_codes, v_codes, block_size):
+    """perm [ctx] int32 of median_repacking without the repacked matrices."""
+    _check_code_matrix(k_codes, "k_codes")
+    _check_code_matrix(v_codes, "v_codes")
+    _require(k_codes.shape == v_codes.shape, "K and V code matrices must have one shape")
+    ctx, hidden = k_codes.shape
+    perm = torch.empty(ctx, dtype=torch.int32, device=k_codes.device)
+    with _on(k_codes.device):
+        rc = _lib.load().pkv_median_repack(_ptr(k_codes), _ptr(v_codes), None, None, _ptr(perm), ctx, hidden, int(block_size), None,
+                                           _stream(k_codes.device))
+    _lib.check(rc)
+    return perm
+
+
 def greedy_order(k_codes, v_codes, pack_len=16, block_size=64):
     """perm [ctx] int32 of greedy_repacking without the repacked matrices (for the fused encoders, which gather the
     rows of K and V themselves)."""
@@ -770,6 +805,10 @@ def repack_and_encode(k_codes, v_codes, pack_size, repack_method="none", block_s
 def _repack_and_encode(k_codes, v_codes, pack_size, repack_method, block_size, pre):
     """repack_and_encode with the sizes before repacking at hand."""
     k_pre, v_pre = pre
+    if repack_method in ("median", "greedy") and block_size % pack_size == 0:       # priced where they lie
+        order = greedy_order(k_codes, v_codes, pack_size, block_size) if repack_method == "greedy" else _median_code_order(k_codes, v_codes, block_size)
+        k_aft, v_aft = code_stats_pair(k_codes, v_codes, pack_size, order, block_size)
+        return k_pre, v_pre, _packed_bytes(k_codes, pack_size, *k_aft), _packed_bytes(v_codes, pack_size, *v_aft)
     if repack_method == "median":
         k_codes, v_codes, _ = median_repacking(k_codes, v_codes, block_size)
     elif repack_method == "greedy":

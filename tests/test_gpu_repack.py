@@ -408,3 +408,18 @@ def test_greedy_order_does_not_depend_on_the_number_of_blocks(cuda):
     kc, vc = (torch.randint(0, 12, (257 * 64, 1024), dtype=torch.uint8, generator=g, device=cuda) for _ in range(2))
     many = ops.greedy_order(kc, vc, 16, 64)
     assert torch.equal(many[:256 * 64], ops.greedy_order(kc[:256 * 64], vc[:256 * 64], 16, 64))
+
+
+@pytest.mark.parametrize("hid,T,bs,pack", [(16, 64, 64, 64), (1024, 1024, 64, 16), (528, 96, 48, 16), (1024, 8192, 64, 32), (4096, 4096, 128, 16), (48, 60, 20, 5)])
+def test_sizes_of_both_matrices_and_in_an_order(cuda, hid, T, bs, pack):
+    """K and V in one call, natural and repacked, against each matrix on its own with its rows written out."""
+    g = torch.Generator(device=cuda)
+    g.manual_seed(hid + T)
+    kc, vc = (torch.randint(0, top, (T, hid), dtype=torch.uint8, generator=g, device=cuda) for top in (12, 256))
+    assert ops.code_stats_pair(kc, vc, pack) == (ops.code_stats(kc, pack), ops.code_stats(vc, pack))
+    perm = torch.stack([torch.randperm(bs, generator=g, device=cuda) for _ in range(T // bs)]).to(torch.int32).reshape(-1)
+    rows = perm.long() + torch.arange(T, device=cuda) // bs * bs
+    for _ in range(2):                            # (twice: the state is left clear)
+        assert ops.code_stats_pair(kc, vc, pack, perm, bs) == (ops.code_stats(kc[rows].contiguous(), pack), ops.code_stats(vc[rows].contiguous(), pack))
+    with pytest.raises(RuntimeError, match="divisible"):
+        ops.code_stats_pair(kc, vc, pack, perm, bs + 1)
