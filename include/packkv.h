@@ -178,6 +178,11 @@ typedef struct pkv_append_side {
 } pkv_append_side;
 int pkv_kv_quant_encode_append(const pkv_append_side *k, const pkv_append_side *v, int dtype, int B, int H, int T_new,
                                int par_stride, uint64_t *k_size, uint64_t *v_size, pkv_stream_t s);
+/* pkv_kv_quant_encode_perm: pkv_k_quant_encode_perm and pkv_v_quant_encode_perm of one order with one wait.  Of the sides x
+ * (contiguous [B, H, T, 128]), stream, capacity, info_tail, scale_tail / zero_tail ([B, T]), rel and bits count. */
+int pkv_kv_quant_encode_perm(const pkv_append_side *k, const pkv_append_side *v, int dtype, int B, int H, int T, const uint32_t *perm,
+                             int perm_block, const void *v_scale_in, const void *v_zero_in, uint64_t *k_size, uint64_t *v_size, pkv_stream_t s);
+
 
 /* ---- the decode step's write into a cache's 16-bit window ------------------------------
  * pkv_window_append: rows win_pos .. win_pos + n - 1 of the windows k_win / v_win [B, H, win_stride, 128] receive the

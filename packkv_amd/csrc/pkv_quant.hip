@@ -2329,6 +2329,22 @@ static int run_quant_encode(const void *x, int dtype, int B, int H, int T, float
     return finish_encode(sh, size_out, bits, s);
 }
 
+// K and V (checked jobs) with one wait; in one launch where both take a group's tokens at once.
+static int encode_both(const EncodeJob job[2], int dtype, int B, int H, int T, uint64_t *k_size, uint64_t *v_size, hipStream_t s) {
+    int rc;
+    ScanHandle sh;
+    if ((rc = prepare_scan_state((uint32_t)state_words(true, B, H, T), &sh, s, true, (uint32_t)state_words(false, B, H, T)))) return rc;
+    const OncePlan pk = once_plan_of(true, job[0], dtype, B, H, T), pv = once_plan_of(false, job[1], dtype, B, H, T);
+    if (pk.threads && pk.threads == pv.threads && (job[0].bits > 4) == (job[1].bits > 4)) {
+        const OnceSide ks = once_side(true, job[0], pk, B, H, T, sh.st), vs = once_side(false, job[1], pv, B, H, T, sh.second);
+        if ((rc = pk.threads == 256 ? once_launch<256>(ks, vs, dtype, s) : once_launch<1024>(ks, vs, dtype, s))) return rc;
+    } else {
+        if ((rc = launch_quant_encode<true>(job[0], dtype, B, H, T, sh.st, s))) return rc;
+        if ((rc = launch_quant_encode<false>(job[1], dtype, B, H, T, sh.second, s))) return rc;
+    }
+    return finish_encode(sh, k_size, job[0].bits, s, v_size, job[1].bits);
+}
+
 }  // namespace pkv
 
 extern "C" {
@@ -2373,6 +2389,24 @@ int pkv_v_quant_encode_perm(const void *x, int dtype, int B, int H, int T, float
                 "the known parameters (order of x) and the written ones (order of the stream) are different arrays");
     return pkv::run_quant_encode<false>(x, dtype, B, H, T, rel, bits, stream, capacity, 0, block_info, scale, zero, T,
                                         size_out, ms_out, (hipStream_t)s, perm, perm_block, scale_in, zero_in);
+}
+
+int pkv_kv_quant_encode_perm(const pkv_append_side *k, const pkv_append_side *v, int dtype, int B, int H, int T, const uint32_t *perm, int perm_block,
+                             const void *v_scale_in, const void *v_zero_in, uint64_t *k_size, uint64_t *v_size, pkv_stream_t s_) {
+    using namespace pkv;
+    PKV_REQUIRE(k && v && k_size && v_size && perm, PKV_ERR_INVALID, "null pointer argument");
+    PKV_REQUIRE((v_scale_in == nullptr) == (v_zero_in == nullptr), PKV_ERR_INVALID, "scale_in and zero_in go together");
+    PKV_REQUIRE(v_scale_in == nullptr || (v_scale_in != v->scale_tail && v_zero_in != v->zero_tail), PKV_ERR_INVALID,
+                "the known parameters (order of x) and the written ones (order of the stream) are different arrays");
+    EncodeJob job[2];
+    for (int i = 0; i < 2; i++) {
+        const pkv_append_side &a = i ? *v : *k;
+        job[i] = EncodeJob{a.x, dense_rows(H, T), a.rel, a.bits, a.stream, a.capacity, 0, a.info_tail, a.scale_tail, a.zero_tail, T, perm, perm_block,
+                           i ? v_scale_in : nullptr, i ? v_zero_in : nullptr};
+        const int rc = i ? check_job<false>(job[i], dtype, B, H, T) : check_job<true>(job[i], dtype, B, H, T);
+        if (rc) return rc;
+    }
+    return encode_both(job, dtype, B, H, T, k_size, v_size, (hipStream_t)s_);
 }
 
 int pkv_quant_params(const void *x, int dtype, int B, int H, int T, float rel, void *scale, void *zero,
@@ -2493,17 +2527,7 @@ int pkv_kv_quant_encode_append(const pkv_append_side *k, const pkv_append_side *
         rc = i == 0 ? check_job<true>(job[i], dtype, B, H, T_new) : check_job<false>(job[i], dtype, B, H, T_new);
         if (rc) return rc;
     }
-    ScanHandle sh;
-    if ((rc = prepare_scan_state((uint32_t)state_words(true, B, H, T_new), &sh, s, true, (uint32_t)state_words(false, B, H, T_new)))) return rc;
-    const OncePlan pk = once_plan_of(true, job[0], dtype, B, H, T_new), pv = once_plan_of(false, job[1], dtype, B, H, T_new);
-    if (pk.threads && pk.threads == pv.threads && (job[0].bits > 4) == (job[1].bits > 4)) {      // both sides in one launch
-        const OnceSide ks = once_side(true, job[0], pk, B, H, T_new, sh.st), vs = once_side(false, job[1], pv, B, H, T_new, sh.second);
-        if ((rc = pk.threads == 256 ? once_launch<256>(ks, vs, dtype, s) : once_launch<1024>(ks, vs, dtype, s))) return rc;
-    } else {
-        if ((rc = launch_quant_encode<true>(job[0], dtype, B, H, T_new, sh.st, s))) return rc;
-        if ((rc = launch_quant_encode<false>(job[1], dtype, B, H, T_new, sh.second, s))) return rc;
-    }
-    return finish_encode(sh, k_size, job[0].bits, s, v_size, job[1].bits);
+    return encode_both(job, dtype, B, H, T_new, k_size, v_size, s);
 }
 
 }  // extern "C"

@@ -464,6 +464,42 @@ def _quant_encode(is_k, x, rel, bits, stream, info, want_size, timed, perm=None,
             "ms": float(ms.value), "bits": bits}
 
 
+def _stream_and_info(is_k, x, bits):
+    """A stream buffer and block_info for x [B, H, T, 128]: sized like the code matrix as the reference does; the extension
+    widths can need more."""
+    B, H, T = x.size(0), x.size(1), x.size(2)
+    hidden = B * H * 128
+    ctx_blk, hid_blk = (64, 128) if is_k else (128, 64)
+    nblk = (T // ctx_blk) * (hidden // hid_blk)
+    room = max(T * hidden, nblk * block_bound(is_k, ctx_blk, hid_blk, bits) + 16) if bits > 4 else T * hidden
+    return torch.empty(room, dtype=torch.uint8, device=x.device), torch.empty(nblk, 2, dtype=torch.uint32, device=x.device)
+
+
+def _kv_quant_encode_perm(k, v, k_rel, v_rel, k_bits, v_bits, perm, perm_block, v_scale, v_zero):
+    """Both sides of a repacked encode with one wait: dicts like k_quant_encode / v_quant_encode.  v_scale / v_zero: V's
+    parameters [B, T] in the order of v."""
+    B, H, T = _check_x(k)
+    _require(k.get_device() == v.get_device() == perm.get_device() == v_scale.get_device() == v_zero.get_device(), _ONE_DEVICE)
+    sides, out = [], []
+    for is_k, x, rel, bits in ((True, k, k_rel, k_bits), (False, v, v_rel, v_bits)):
+        stream, info = _stream_and_info(is_k, x, bits)
+        scale = torch.empty(B, T, dtype=x.dtype, device=x.device)
+        zero = torch.empty(B, T, dtype=x.dtype, device=x.device)
+        a = _lib.AppendSide()
+        a.x, a.stream, a.capacity, a.info_tail = x.data_ptr(), stream.data_ptr(), stream.numel(), info.data_ptr()
+        a.scale_tail, a.zero_tail, a.rel, a.bits = scale.data_ptr(), zero.data_ptr(), float(rel), int(bits)
+        sides.append(a)
+        out.append({"stream": stream, "info": info, "scale": scale, "zero": zero, "size": 0, "ms": 0.0, "bits": bits})
+    ks, vs = ctypes.c_uint64(0), ctypes.c_uint64(0)
+    with _on(k.device):
+        rc = _lib.load().pkv_kv_quant_encode_perm(ctypes.byref(sides[0]), ctypes.byref(sides[1]), _dtype_code(k), B, H, T, _ptr(perm),
+                                                  int(perm_block), _ptr(v_scale), _ptr(v_zero), ctypes.byref(ks), ctypes.byref(vs),
+                                                  _stream(k.device))
+    _lib.check(rc)
+    out[0]["size"], out[1]["size"] = int(ks.value), int(vs.value)
+    return out[0], out[1]
+
+
 def k_quant_encode(x, rel, bits=None, stream=None, info=None, want_size=True, timed=False):
     """Fused quantize + K encode of x [B, H, T, 128]; returns a dict with stream, info (block_info),
     scale, zero [B, T], size (bytes), ms and bits."""
@@ -864,18 +900,11 @@ def repack_quant_encode(k, v, k_rel, v_rel, repack_method="median", block_size=6
         if repack_method == "median":
             perm, vs, vz = median_order(v, v_rel, v_bits, block_size, want_params=True)
         else:
-            ks, kz = quant_params(k, k_rel)
-            vs, vz = quant_params(v, v_rel)
-            kc, kmx = quantize(k, ks, kz)
-            vc, vmx = quantize(v, vs, vz)
-            for mx, bits in ((kmx, k_bits), (vmx, v_bits)):
-                if mx >= (1 << bits):
-                    raise PackKVError(1, "not supported: code %d does not fit bits_len %d" % (mx, bits))
+            kc = quant_codes(k, k_rel)[0]
+            vc, vs, vz = quant_codes(v, v_rel)
             perm = greedy_order(kc, vc, 16, block_size)      # the codecs' packs are 16 tokens
-            del kc, vc
-        ke = _quant_encode(True, k, k_rel, k_bits, None, None, True, False, perm, block_size)
-        ve = _quant_encode(False, v, v_rel, v_bits, None, None, True, False, perm, block_size, (vs, vz))
-        return ke, ve, perm
+            del kc, vc                                       # (codes too wide for the stream are the encoders' to report)
+        return _kv_quant_encode_perm(k, v, k_rel, v_rel, k_bits, v_bits, perm, block_size, vs, vz) + (perm,)
     ks, kz = quant_params(k, k_rel)
     vs, vz = quant_params(v, v_rel)
     kc, kmx = quantize(k, ks, kz)

@@ -423,3 +423,17 @@ def test_sizes_of_both_matrices_and_in_an_order(cuda, hid, T, bs, pack):
         assert ops.code_stats_pair(kc, vc, pack, perm, bs) == (ops.code_stats(kc[rows].contiguous(), pack), ops.code_stats(vc[rows].contiguous(), pack))
     with pytest.raises(RuntimeError, match="divisible"):
         ops.code_stats_pair(kc, vc, pack, perm, bs + 1)
+
+
+@pytest.mark.parametrize("method", ["median", "greedy"])
+@pytest.mark.parametrize("B,H,T", [(1, 8, 256), (2, 3, 4224), (1, 8, 20480)])
+def test_repacked_encode_of_both_sides_reports_codes_and_equals_one_side_at_a_time(cuda, B, H, T, method):
+    k, v = synth.make_kv(B, H, T, seed=T, device=cuda)
+    for kb, vb in ((3, 4), (4, 3)):
+        with pytest.raises(RuntimeError, match="does not fit bits_len 3"):
+            ops.repack_quant_encode(k, v, 0.1, 0.1, method, k_bits=kb, v_bits=vb)
+    ke, ve, perm = ops.repack_quant_encode(k, v, 0.1, 0.05, method)
+    for e, x, is_k, rel in ((ke, k, True, 0.1), (ve, v, False, 0.05)):
+        one = ops._quant_encode(is_k, x, rel, e["bits"], None, None, True, False, perm, 64)
+        assert one["size"] == e["size"] and torch.equal(one["stream"][:e["size"]], e["stream"][:e["size"]])
+        assert all(torch.equal(one[f].view(torch.int16), e[f].view(torch.int16)) for f in ("info", "scale", "zero"))
