@@ -89,38 +89,47 @@ __device__ __forceinline__ void unit_parse2(const uint8_t *blk_a, uint32_t off_a
 // unit_codes hands lane t's four packs to `sink(k, c4)` token by token: c4 holds the codes of slots 0..3 at token k of
 // the pack, one per byte, slot 0 lowest.
 
-// Widths 5..8 (format extension): pack words of up to 128 bits, the four slots' words shifted down one field at a time
-// (token 15 sits in the lowest field).
+// Widths 5..8 (format extension): a pack word is up to 16 bytes long and is not assembled.  Each quarter of it (four
+// tokens, 4 * len bits that start (3 - q) * 4 * len bits into the word, at a byte or a nibble) is the 32 bits at its byte
+// address, two aligned dwords and a funnel shift, cut into two 16-bit windows of two tokens; from there as below, one
+// instruction a code.  (Codes of 5 bits, kernel time: 16384 x 1024 take 9.2 us for K and 9.0 for V, 11.1 and 10.4 with
+// 128-bit words that were shifted down a field at a time; calls at 65536 x 1024 20.8 and 19.0 us against 28.1 and 22.2.)
 template <class Sink>
 __device__ __forceinline__ void unit_codes_wide(const uint8_t *blk, uint32_t unit_off, int t, const UnitGeom g, Sink sink) {
+    typedef unsigned short u16pair __attribute__((ext_vector_type(2)));
     const uint32_t minsw = lds_meta_word(blk + unit_off, t, g.W);
     const uint32_t lensw = lds_meta_word(blk + unit_off + g.mins_bytes, t, g.LB);
     const uint32_t pay0 = unit_off + g.mins_bytes + g.lens_bytes;
-    uint32_t len[4], mn[4], off[4], mask[4], d[4][4], payload;
+    uint32_t len[4], off[4], payload, mq = 0u, minq = 0u;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         len[i] = (lensw >> (i * g.LB)) & ((1u << g.LB) - 1u);
-        mn[i] = (minsw >> (i * g.W)) & ((1u << g.W) - 1u);
-        mask[i] = (1u << len[i]) - 1u;
+        minq |= ((minsw >> (i * g.W)) & ((1u << g.W) - 1u)) << (8 * i);
+        mq |= (((1u << len[i]) - 1u) & 0xFFu) << (8 * i);
     }
     pack_offsets(len, off, payload);
+    const u16pair len01 = __builtin_bit_cast(u16pair, len[0] | (len[1] << 16)), len23 = __builtin_bit_cast(u16pair, len[2] | (len[3] << 16));
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const uint64_t lo = lds_load64(blk, pay0 + off[i]), hi = lds_load64(blk, pay0 + off[i] + 8u);
-        d[i][0] = (uint32_t)lo; d[i][1] = (uint32_t)(lo >> 32); d[i][2] = (uint32_t)hi; d[i][3] = (uint32_t)(hi >> 32);
-    }
-#pragma unroll
-    for (int k = kPackTok - 1; k >= 0; k--) {
-        uint32_t c4 = 0;
+    for (int q = 0; q < 4; q++) {
+        uint32_t lo[4], hi[4];                               // tokens 4q + 2, 4q + 3 and 4q, 4q + 1
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            c4 |= (((d[i][0] & mask[i]) + mn[i]) & 0xFFu) << (8 * i);
-            d[i][0] = __builtin_amdgcn_alignbit(d[i][1], d[i][0], len[i]);
-            d[i][1] = __builtin_amdgcn_alignbit(d[i][2], d[i][1], len[i]);
-            d[i][2] = __builtin_amdgcn_alignbit(d[i][3], d[i][2], len[i]);
-            d[i][3] >>= len[i];
+            const uint32_t bit = (uint32_t)(3 - q) * 4u * len[i], at = pay0 + off[i] + (bit >> 3);
+            const uint32_t *d = reinterpret_cast<const uint32_t *>(blk + (at & ~3u));
+            lo[i] = __builtin_amdgcn_alignbyte(d[1], d[0], at) >> (bit & 4u);
+            hi[i] = lo[i] >> (2u * len[i]);
         }
-        sink(k, c4);
+#pragma unroll
+        for (int half = 0; half < 2; half++) {
+            const uint32_t *e = half ? lo : hi;
+            const u16pair w01 = __builtin_bit_cast(u16pair, __builtin_amdgcn_perm(e[1], e[0], 0x05040100u));
+            const u16pair w23 = __builtin_bit_cast(u16pair, __builtin_amdgcn_perm(e[3], e[2], 0x05040100u));
+#pragma unroll
+            for (int pp = 0; pp < 2; pp++) {
+                const uint32_t x01 = __builtin_bit_cast(uint32_t, pp ? w01 : (u16pair)(w01 >> len01)), x23 = __builtin_bit_cast(uint32_t, pp ? w23 : (u16pair)(w23 >> len23));
+                sink(4 * q + 2 * half + pp, (__builtin_amdgcn_perm(x23, x01, 0x06040200u) & mq) + minq);
+            }
+        }
     }
 }
 

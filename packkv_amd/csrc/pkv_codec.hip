@@ -54,6 +54,9 @@ __global__ void unpack_kernel(const uint8_t *__restrict__ stream, uint64_t strea
 // V blocks of 64 channels, two adjacent ones (the two halves of a head) per workgroup of 256 threads: the pair
 // decodes into one tile of 128 tokens x 128 channels, so the write-back stores whole 128-byte lines.  In tile
 // addressing the pair is a V block of 128 channels whose units 4 j + u are the units u of block j.
+// A lane's four codes at a token are one channel in four rounds; four lanes turn theirs into four channels of one round
+// each, so that the tile takes dwords instead of bytes (64 byte stores a lane).  The 16-byte pieces of a row lie at their
+// number xor the round's: the rounds are 2 KB apart and would meet in the same banks.
 __global__ void __launch_bounds__(256) unpack_v_pair_kernel(const uint8_t *__restrict__ stream, uint64_t stream_bytes,
                                                             const uint32_t *__restrict__ info,
                                                             uint8_t *__restrict__ codes, int hidden_dim, int W,
@@ -77,7 +80,14 @@ __global__ void __launch_bounds__(256) unpack_v_pair_kernel(const uint8_t *__res
         const int t = tid & 31, u = (tid >> 5) & 3;
         const uint16_t *cum = reinterpret_cast<const uint16_t *>(blk + phase);
         const uint32_t start = phase + 8u + (u ? (uint32_t)cum[u - 1] : 0u);
-        unit_decode<false>(blk, min(start, blk_cap), 4 * j + u, t, g, tile, kPairHid);
+        const int warp = 2 * j + (u >> 1), round = 4 * (u & 1) + (t & 3);
+        const uint32_t sel1 = (t & 1) ? 0x03070105u : 0x06020400u, sel2 = (t & 2) ? 0x03020706u : 0x05040100u;
+        uint32_t *dst = reinterpret_cast<uint32_t *>(tile) + round * (kPackTok * kPairHid / 4) + 4 * ((2 * warp + (t >> 4)) ^ round) + ((t >> 2) & 3);
+        unit_codes(blk, min(start, blk_cap), t, g, [&](int k, uint32_t c4) {
+            c4 = __builtin_amdgcn_perm((uint32_t)__builtin_amdgcn_update_dpp(0, (int)c4, 0xB1, 0xF, 0xF, true), c4, sel1);      // lane ^ 1
+            c4 = __builtin_amdgcn_perm((uint32_t)__builtin_amdgcn_update_dpp(0, (int)c4, 0x4E, 0xF, 0xF, true), c4, sel2);      // lane ^ 2
+            dst[k * (kPairHid / 4)] = c4;
+        });
     }
     __syncthreads();
     const uint4 *t16 = reinterpret_cast<const uint4 *>(tile);
@@ -85,7 +95,7 @@ __global__ void __launch_bounds__(256) unpack_v_pair_kernel(const uint8_t *__res
 #pragma unroll
     for (int i = 0; i < kCtx * kPairHid / 16 / 256; i++) {     // 8 rows of 128 bytes per step, 16 bytes per thread
         const int idx = tid + 256 * i;
-        *reinterpret_cast<uint4 *>(base + (size_t)(idx >> 3) * hidden_dim + 16 * (idx & 7)) = t16[idx];
+        *reinterpret_cast<uint4 *>(base + (size_t)(idx >> 3) * hidden_dim + 16 * (idx & 7)) = t16[idx ^ (idx >> 7)];
     }
 }
 
