@@ -116,8 +116,11 @@ def _check_codec_args(codes, stream, info, ctx_len, hidden_dim, ctx_blk, hid_blk
 
 # Host tensors go through page-locked memory from torch's host allocator, at most two pieces of this size at a time: the
 # link moves 8 MiB between it and the device in 155 us, where a copy from or to pageable memory takes 246 and 460 us (574
-# into a fresh tensor); the copy on the host is 16 us.
+# into a fresh tensor); the copy on the host is 16 us.  Smaller tensors are copied as they are, the buffer and the event cost
+# more than they save there.  Up / down in us, as they are and staged: 128 KiB 17 / 18 and 30 / 42, 512 KiB 28 / 34 and
+# 37 / 51, 1 MiB 57 / 66 and 47 / 63, 8 MiB 250 / 523 and 201 / 235.
 _STAGE_BYTES = 32 << 20
+_STAGE_FROM = 1 << 20
 
 
 def _bytes(t):
@@ -143,6 +146,9 @@ def _staged(n, pieces, step):
 
 def _upload(dst, src):
     """Device bytes dst = host bytes src, on the current stream of dst's device; src may be reused at once."""
+    if src.numel() < _STAGE_FROM:
+        dst.copy_(src)
+        return
     last = src.numel() <= _STAGE_BYTES
 
     def step(buf, a, b):
@@ -156,6 +162,10 @@ def _upload(dst, src):
 
 def _download(dst, src):
     """Host bytes dst = device bytes src, there when this returns."""
+    if src.numel() < _STAGE_FROM:
+        dst.copy_(src)
+        return
+
     def step(buf, a, b):
         buf.copy_(src[a:b], non_blocking=True)
         there = torch.cuda.current_stream(src.device).record_event()
@@ -204,9 +214,9 @@ def _decode(is_k, stream, info, codes, ctx_len, hidden_dim, ctx_blk, hid_blk, bi
     ms = ctypes.c_float(0.0)
     fn = lib.pkv_k_decode if is_k else lib.pkv_v_decode
     with _on(dev):
-        if on_host:          # the part of the buffer that block_info points into
+        if on_host:          # the part of the buffer that block_info points into, where that is worth its sum (9 us)
             used = stream.numel()
-            if info.numel():
+            if info.numel() and used >= _STAGE_FROM:
                 used = min(used, max(1, int(info.view(torch.int32).to(torch.int64).bitwise_and_(0xFFFFFFFF).sum(1).max())))
             d_stream = torch.empty(used, dtype=torch.uint8, device=dev)
             d_info, d_codes = torch.empty_like(info, device=dev), torch.empty_like(codes, device=dev)

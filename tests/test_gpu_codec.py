@@ -387,12 +387,13 @@ def test_code_matrix_encode_by_group_count(cuda, oracle_codec, heads, T, bits):
         assert np.array_equal(stream[:zo].cpu().numpy(), so[:zo]) and not bool(stream[zo:].any())
 
 
-@pytest.mark.parametrize("stage", [1 << 25, 70000, 4097])
+@pytest.mark.parametrize("stage,staged_from", [(1 << 25, 1 << 20), (1 << 25, 0), (70000, 0), (4097, 0)])
 @pytest.mark.parametrize("is_k", [True, False])
-def test_host_tensors_in_pieces(cuda, monkeypatch, is_k, stage):
-    """The host round trip in one, some and many pieces; what lies behind the stream in the caller's buffer stays, and a
+def test_host_tensors_in_pieces(cuda, monkeypatch, is_k, stage, staged_from):
+    """The host round trip copied as it is and in one, some and many pieces; what lies behind the stream in the caller's buffer stays, and a
     block_info that points past the buffer reads no further than the buffer."""
     monkeypatch.setattr(ops, "_STAGE_BYTES", stage)
+    monkeypatch.setattr(ops, "_STAGE_FROM", staged_from)
     codes = torch.randint(0, 16, (384, 1024), generator=torch.Generator().manual_seed(3), dtype=torch.uint8)
     cb, hb = (64, 128) if is_k else (128, 64)
     n = codes.numel() // 8192
