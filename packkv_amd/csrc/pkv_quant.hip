@@ -2186,9 +2186,11 @@ static auto cells_kernel(int bits, int dtype, bool perm, bool xch, bool strided,
 
 // The kernels that take a group's tokens at once (pkv_quant_once.hpp), where they serve the job.  (K reaches the second head of
 // a wavefront through a 32-bit byte offset.  Groups of up to four heads in bf16 stay with the round-major kernels: those leave a
-// NaN out of a token's minimum and maximum, the order keys of the cells do not.)
+// NaN out of a token's minimum and maximum, the order keys of the cells do not.  So does V of more than eight heads for the
+// other runs of eight, where the keys of all heads meet here.)
 static OncePlan once_plan_of(bool is_k, const EncodeJob &job, int dtype, int B, int H, int T) {
-    if (job.rot.cos || job.xs.sh >= (1ll << 31) - 128 || (H <= 4 && dtype != PKV_F16 && !job.perm)) return OncePlan{0, 0, 0, 0};
+    if (job.rot.cos || job.xs.sh >= (1ll << 31) - 128 || (H <= 4 && dtype != PKV_F16 && !job.perm) ||
+        (!is_k && H > kSubBlocks && dtype != PKV_F16 && !job.scale_in)) return OncePlan{0, 0, 0, 0};
     return once_plan(is_k, (uint64_t)T / (is_k ? 64 : 128) * (uint64_t)B, H, kOnceSmall);
 }
 static OnceSide once_side(bool is_k, const EncodeJob &job, const OncePlan &p, int B, int H, int T, ScanState *st) {

@@ -203,7 +203,8 @@ __device__ __forceinline__ void k_encode_once(const OnceSide &a, OnceLds<NT> &l,
     }
     if (a.nruns > 1) {
         const uint32_t mine = T16<DT>::to_bits(mn) << 16 | T16<DT>::to_bits(mx);
-        mn = INFINITY, mx = -INFINITY;
+        // (NaN drops out of minima and maxima; a token that is nothing else keeps what the cells kernels make of it)
+        mn = a.H <= 8 ? NAN : INFINITY, mx = a.H <= 8 ? NAN : -INFINITY;
         once_exchange<4>(a.xw + (size_t)grp * a.nruns * 64 + 16 * r, 64, run, a.nruns, wr == 0, mine, a.st, [&](uint32_t w) {
             mn = fminf(mn, T16<DT>::from_bits(w >> 16));
             mx = fmaxf(mx, T16<DT>::from_bits(w & 0xFFFFu));
@@ -334,6 +335,7 @@ __device__ __forceinline__ void v_encode_once(const OnceSide &a, OnceLds<NT> &l,
             pw = pk_sel_x<false, DT != PKV_F16>(pw, (uint32_t)__shfl_xor((int)pw, 1, 64));
         }
         minmax_unword<DT>(pw, mn, mx);
+        if (a.H > 8) mn = fminf(mn, INFINITY), mx = fmaxf(mx, -INFINITY);      // (a token of NaN only, as above)
         const TokPar tp = once_params<DT>(mn, mx, a.rel, write, a.scale, a.zero, ptok);
         if ((lane & 1) == 0) par[lane >> 1] = tp;
     }

@@ -369,3 +369,26 @@ def test_encodes_at_once_report_codes_and_capacity(cuda, T):
         again = fn(x, 0.1, stream=small[:good["size"]])
         assert again["size"] == good["size"] and torch.equal(again["stream"], good["stream"][:good["size"]])
         assert torch.equal(again["info"].view(torch.int32), good["info"].view(torch.int32)) and bool((small[good["size"]:] == 77).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("H", [3, 8, 12])
+def test_nan_parameters_do_not_depend_on_the_launch(cuda, dtype, H):
+    """Tokens with NaN and infinities get the same scale and zero from a launch of one group and from one that fills the
+    chip (257 groups of V: other kernels)."""
+    g = torch.Generator(device=cuda).manual_seed(5)
+    big = torch.randn(1, H, 128 * 257, 128, generator=g, device=cuda).to(dtype)
+    nan, inf = float("nan"), float("inf")
+    big[0, 1, 5, 7] = nan                                # one value
+    big[0, :, 9] = nan                                   # a whole token
+    big[0, 0, 20] = nan                                  # a whole head of a token
+    big[0, H - 1, 40, 3], big[0, 0, 41, 100] = inf, -inf
+    big[0, 2, 50, 1], big[0, 1, 50, 2] = nan, inf
+    big[0, H - 1, 77, 64:] = -torch.tensor(nan)
+    for enc in (ops.k_quant_encode, ops.v_quant_encode):
+        small, whole = enc(big[:, :, :128].contiguous(), 0.1, want_size=False), enc(big, 0.1, want_size=False)
+        torch.cuda.synchronize()
+        for name in ("scale", "zero"):
+            a, b = small[name].cpu(), whole[name][:, :128].cpu()
+            same = (a.view(torch.int16) == b.view(torch.int16)) | (a.isnan() & b.isnan())
+            assert bool(same.all()), (enc.__name__, name, (~same).nonzero().tolist())
