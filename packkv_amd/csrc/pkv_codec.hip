@@ -350,9 +350,12 @@ static int run_pack(bool is_k, const uint8_t *codes, uint8_t *stream, uint64_t c
     const bool grouped = cs.nunits == 4 && bits <= 7 && hid_blk % 16 == 0 && hidden_dim % 16 == 0 &&
                          (reinterpret_cast<uintptr_t>(codes) & 15u) == 0;
     // the reference's block shapes over rows that are whole groups of 1024 channels: the cells kernels (no code tile
-    // in LDS, the next round in flight while packs are formed)
-    const bool cells = bits <= 6 && hidden_dim % 1024 == 0 && (reinterpret_cast<uintptr_t>(codes) & 3u) == 0 &&
-                       (is_k ? (ctx_blk == 64 && hid_blk == 128) : (ctx_blk == 128 && hid_blk == 64));
+    // in LDS, the next round in flight while packs are formed); other rows while the launch is small enough for all
+    // tokens of a group at once (both sides, encode and decode of 512 channels, a pass; pack_group_kernel in brackets: 1024 rows
+    // of 4 bits 55 us [67], 4096 of 5 bits 58 [80]; V alone: 12288 of 4 bits 64 [69], 32768 of 5 bits 79 [90])
+    const bool cells = bits <= 6 && (reinterpret_cast<uintptr_t>(codes) & 3u) == 0 &&
+                       (is_k ? (ctx_blk == 64 && hid_blk == 128) : (ctx_blk == 128 && hid_blk == 64)) &&
+                       code_cells_serve(is_k, ctx_len, hidden_dim);
     if (cells) {
         if ((rc = prepare_scan_state(code_cells_words(is_k, ctx_len, hidden_dim), &sh, s, size_out || ms_out))) return rc;
         ScanState *st = sh.st;

@@ -1895,6 +1895,11 @@ __global__ void __launch_bounds__(512) v_code_cells_kernel(
 // Launch of the two kernels above (pkv_codec.hip decides when they apply): `st` is a prepared scan state of
 // code_cells_words status words, `bound` the worst-case bytes of a block.
 static OncePlan code_plan(bool is_k, int ctx_len, int hidden) { return once_plan(is_k, (uint64_t)(ctx_len / (is_k ? 64 : 128)), hidden / kHeadDim, kOnceSmallCodes); }
+bool code_cells_serve(bool is_k, int ctx_len, int hidden) {
+    if (hidden % 1024 == 0) return true;
+    const OncePlan p = hidden % kHeadDim ? OncePlan{0, 0, 0, 0} : code_plan(is_k, ctx_len, hidden);
+    return p.threads && hidden / kHeadDim % p.run == 0;    // (code_encode_once_kernel knows whole runs only)
+}
 uint32_t code_cells_words(bool is_k, int ctx_len, int hidden) {
     const OncePlan p = code_plan(is_k, ctx_len, hidden);
     return p.threads ? p.nwg : (uint32_t)(ctx_len / (is_k ? 64 : 128)) * (uint32_t)(hidden / 1024);

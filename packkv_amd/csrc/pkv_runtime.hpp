@@ -89,8 +89,9 @@ struct OutcomeSlot {
 };
 // ... the launch that clears `h`'s state itself has been made.
 int scan_state_cleared(ScanHandle &h, hipStream_t s);
-// The block codec from a code matrix through the cells kernels (pkv_quant.hip): for hidden a multiple of 1024, the
-// reference's block shapes, widths up to 6.  `st` holds code_cells_words status words.
+// The block codec from a code matrix through the cells kernels (pkv_quant.hip): where code_cells_serve says so, for the
+// reference's block shapes and widths up to 6.  `st` holds code_cells_words status words.
+bool code_cells_serve(bool is_k, int ctx_len, int hidden);
 uint32_t code_cells_words(bool is_k, int ctx_len, int hidden);
 int launch_code_cells(bool is_k, const uint8_t *codes, int ctx_len, int hidden, int bits, uint32_t bound, uint8_t *stream,
                       uint64_t capacity, uint32_t *info, ScanState *st, hipStream_t s);

@@ -370,9 +370,10 @@ def test_damaged_block_info_is_survived(cuda, is_k):
 
 
 @pytest.mark.parametrize("bits", [2, 4, 5, 6])
-@pytest.mark.parametrize("heads,T", [(8, 128), (8, 2048), (16, 1152), (8, 16384), (8, 16512)])
+@pytest.mark.parametrize("heads,T", [(8, 128), (8, 2048), (16, 1152), (8, 16384), (8, 16512), (4, 256), (4, 4096), (4, 4224), (3, 256), (12, 2048)])
 def test_code_matrix_encode_by_group_count(cuda, oracle_codec, heads, T, bits):
-    """Either side of the lines between the kernels: 128 workgroups of 256 threads, 256 of 1024, the kernels that walk."""
+    """Either side of the lines between the kernels: 128 workgroups of 256 threads, 256 of 1024, the kernels that walk;
+    rows that are no multiple of 1024 channels, in whole runs of heads and not."""
     codes = torch.randint(0, 1 << bits, (T, heads * 128), generator=torch.Generator().manual_seed(T + bits), dtype=torch.uint8)
     codes[:, ::3] >>= 1
     codes[:, ::7] = codes[0, ::7]
