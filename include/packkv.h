@@ -178,6 +178,12 @@ typedef struct pkv_append_side {
 } pkv_append_side;
 int pkv_kv_quant_encode_append(const pkv_append_side *k, const pkv_append_side *v, int dtype, int B, int H, int T_new,
                                int par_stride, uint64_t *k_size, uint64_t *v_size, pkv_stream_t s);
+/* pkv_kv_quant_encode_alone: the same encode, with a token order if perm is not NULL (the rows are then contiguous).  In launches
+ * of few groups the workgroups that share a group's heads tell each other the minima and maxima of its tokens; one that has
+ * looked for another's in vain for a while -- it may not have started, if another stream holds the CUs -- reads the group's
+ * rows itself.  Here every one does so at once: slower, with the same result to the bit. */
+int pkv_kv_quant_encode_alone(const pkv_append_side *k, const pkv_append_side *v, int dtype, int B, int H, int T_new, int par_stride,
+                              const uint32_t *perm, int perm_block, uint64_t *k_size, uint64_t *v_size, pkv_stream_t s);
 /* pkv_kv_quant_encode_perm: pkv_k_quant_encode_perm and pkv_v_quant_encode_perm of one order with one wait.  Of the sides x
  * (contiguous [B, H, T, 128]), stream, capacity, info_tail, scale_tail / zero_tail ([B, T]), rel and bits count. */
 int pkv_kv_quant_encode_perm(const pkv_append_side *k, const pkv_append_side *v, int dtype, int B, int H, int T, const uint32_t *perm,

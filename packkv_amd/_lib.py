@@ -77,6 +77,7 @@ SIGNATURES = {
     "pkv_k_quant_encode_append": (_i, [_vp, _i, _i, _i, _i, _f, _i, _vp, _u64, _u64, _vp, _vp, _vp, _i, _u64p, _fp, _vp]),
     "pkv_v_quant_encode_append": (_i, [_vp, _i, _i, _i, _i, _f, _i, _vp, _u64, _u64, _vp, _vp, _vp, _i, _u64p, _fp, _vp]),
     "pkv_kv_quant_encode_append": (_i, [ctypes.POINTER(AppendSide), ctypes.POINTER(AppendSide), _i, _i, _i, _i, _i, _u64p, _u64p, _vp]),
+    "pkv_kv_quant_encode_alone": (_i, [ctypes.POINTER(AppendSide), ctypes.POINTER(AppendSide), _i, _i, _i, _i, _i, _vp, _i, _u64p, _u64p, _vp]),
     "pkv_kv_quant_encode_perm": (_i, [ctypes.POINTER(AppendSide), ctypes.POINTER(AppendSide), _i, _i, _i, _i, _vp, _i, _vp, _vp, _u64p, _u64p, _vp]),
     "pkv_window_cut": (_i, [ctypes.POINTER(CutArgs), _vp]),
     "pkv_window_append": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64,

@@ -465,7 +465,8 @@ __device__ __forceinline__ void stagger_first_generation(const Stagger sg) {
 constexpr uint64_t kFlagAgg = 1ull << 62;
 constexpr uint64_t kFlagIncl = 2ull << 62;
 constexpr uint64_t kValueMask = (1ull << 62) - 1ull;
-constexpr int kSpinLimit = 1 << 18;          // polls before a wait gives up with PKV_ERR_INTERNAL: well under a second at the look-back's back-off
+constexpr int kSpinLimit = 1 << 18;          // polls before a wait gives up with PKV_ERR_INTERNAL: about a second at a back-off of
+                                             // PKV_LOOKBACK_SLEEP; a look-back with a shorter one polls as many times more
 
 struct ScanState {
     uint32_t ticket;      // next block index to hand out
@@ -513,6 +514,7 @@ constexpr int kLookWindows = 1;
 template <int SLEEP = PKV_LOOKBACK_SLEEP>
 __device__ __forceinline__ uint64_t lookback_offset(ScanState *st, uint32_t idx, uint32_t my_bytes, bool published = false) {
     const int lane = threadIdx.x & 63;
+    constexpr int kLimit = SLEEP < PKV_LOOKBACK_SLEEP ? kSpinLimit * (PKV_LOOKBACK_SLEEP / SLEEP) : kSpinLimit;
     uint64_t *status = st->status;
     if (idx == 0) {
         if (lane == 0 && !published)
@@ -539,7 +541,7 @@ __device__ __forceinline__ uint64_t lookback_offset(ScanState *st, uint32_t idx,
             if (done || failed) break;
             const int64_t j = base - 64 * w - lane;
             int spins = 0;
-            while ((s[w] >> 62) == 0 && spins < kSpinLimit) {
+            while ((s[w] >> 62) == 0 && spins < kLimit) {
                 __builtin_amdgcn_s_sleep(SLEEP);
                 s[w] = __hip_atomic_load(&status[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 spins++;

@@ -2114,6 +2114,7 @@ struct EncodeJob {
     int perm_block = 0;
     const void *scale_in = nullptr, *zero_in = nullptr;
     Rot rot = {nullptr, nullptr, 0};       // K of five heads or more, in their own order
+    int polls = kOncePolls;                // (pkv_quant_once.hpp)
 };
 
 // 64-bit words of look-back state the job takes: status words (one per ticket), then the words the runs of a group
@@ -2208,6 +2209,7 @@ static OnceSide once_side(bool is_k, const EncodeJob &job, const OncePlan &p, in
     a.nwg = p.nwg; a.slot = once_slot(is_k, job.bits);
     a.perm = job.perm; a.perm_block = job.perm_block;
     a.scale_in = (const uint16_t *)job.scale_in; a.zero_in = (const uint16_t *)job.zero_in;
+    a.polls = job.polls;
     return a;
 }
 
@@ -2350,6 +2352,30 @@ static int encode_both(const EncodeJob job[2], int dtype, int B, int H, int T, u
         if ((rc = launch_quant_encode<false>(job[1], dtype, B, H, T, sh.second, s))) return rc;
     }
     return finish_encode(sh, k_size, job[0].bits, s, v_size, job[1].bits);
+}
+
+// The jobs of two sides, checked.  With a token order the rows are dense.
+static int append_jobs(EncodeJob job[2], const pkv_append_side *k, const pkv_append_side *v, int dtype, int B, int H, int T, int par_stride,
+                       const uint32_t *perm, int perm_block, bool sizes) {
+    PKV_REQUIRE(k && v && sizes, PKV_ERR_INVALID, "null pointer argument");
+    for (int i = 0; i < 2; i++) {
+        const pkv_append_side &a = i ? *v : *k;
+        PKV_REQUIRE(a.stride_b >= 0 && a.stride_h >= 0 && a.stride_t >= 0 && a.stride_t < (1 << 25) &&
+                        (a.stride_b | a.stride_h | a.stride_t) % 8 == 0 && (reinterpret_cast<uintptr_t>(a.x) & 15u) == 0,
+                    PKV_ERR_INVALID, "rows must start on 16-byte boundaries (row stride below 2^25 elements)");
+        job[i] = EncodeJob{a.x, perm ? dense_rows(H, T) : XRows{a.stride_b, a.stride_h, a.stride_t}, a.rel, a.bits, a.stream, a.capacity, a.used,
+                           a.info_tail, a.scale_tail, a.zero_tail, par_stride, perm, perm_block};
+        PKV_REQUIRE((a.cos == nullptr) == (a.sin == nullptr), PKV_ERR_INVALID, "cos and sin go together");
+        if (a.cos) {
+            PKV_REQUIRE(i == 0 && H > 4 && !perm, PKV_ERR_UNSUPPORTED, "not supported: a rotary embedding other than of K with five heads or more");
+            PKV_REQUIRE(a.rot_stride_b >= 0 && a.rot_stride_b % 8 == 0 && ((reinterpret_cast<uintptr_t>(a.cos) | reinterpret_cast<uintptr_t>(a.sin)) & 15u) == 0,
+                        PKV_ERR_INVALID, "rows must start on 16-byte boundaries");
+            job[i].rot = Rot{(const uint16_t *)a.cos, (const uint16_t *)a.sin, a.rot_stride_b};
+        }
+        const int rc = i ? check_job<false>(job[i], dtype, B, H, T) : check_job<true>(job[i], dtype, B, H, T);
+        if (rc) return rc;
+    }
+    return PKV_OK;
 }
 
 }  // namespace pkv
@@ -2510,31 +2536,21 @@ int pkv_v_quant_encode_append(const void *x, int dtype, int B, int H, int T_new,
 }
 
 int pkv_kv_quant_encode_append(const pkv_append_side *k, const pkv_append_side *v, int dtype, int B, int H, int T_new,
-                               int par_stride, uint64_t *k_size, uint64_t *v_size, pkv_stream_t s_) {
+                               int par_stride, uint64_t *k_size, uint64_t *v_size, pkv_stream_t s) {
     using namespace pkv;
-    hipStream_t s = (hipStream_t)s_;
-    PKV_REQUIRE(k && v && k_size && v_size, PKV_ERR_INVALID, "null pointer argument");
-    const pkv_append_side *sides[2] = {k, v};
     EncodeJob job[2];
-    int rc;
-    for (int i = 0; i < 2; i++) {
-        const pkv_append_side &a = *sides[i];
-        PKV_REQUIRE(a.stride_b >= 0 && a.stride_h >= 0 && a.stride_t >= 0 && a.stride_t < (1 << 25) &&
-                        (a.stride_b | a.stride_h | a.stride_t) % 8 == 0 && (reinterpret_cast<uintptr_t>(a.x) & 15u) == 0,
-                    PKV_ERR_INVALID, "rows must start on 16-byte boundaries (row stride below 2^25 elements)");
-        job[i] = EncodeJob{a.x, XRows{a.stride_b, a.stride_h, a.stride_t}, a.rel, a.bits, a.stream, a.capacity, a.used, a.info_tail,
-                           a.scale_tail, a.zero_tail, par_stride};
-        PKV_REQUIRE((a.cos == nullptr) == (a.sin == nullptr), PKV_ERR_INVALID, "cos and sin go together");
-        if (a.cos) {
-            PKV_REQUIRE(i == 0 && H > 4, PKV_ERR_UNSUPPORTED, "not supported: a rotary embedding other than of K with five heads or more");
-            PKV_REQUIRE(a.rot_stride_b >= 0 && a.rot_stride_b % 8 == 0 && ((reinterpret_cast<uintptr_t>(a.cos) | reinterpret_cast<uintptr_t>(a.sin)) & 15u) == 0,
-                        PKV_ERR_INVALID, "rows must start on 16-byte boundaries");
-            job[i].rot = Rot{(const uint16_t *)a.cos, (const uint16_t *)a.sin, a.rot_stride_b};
-        }
-        rc = i == 0 ? check_job<true>(job[i], dtype, B, H, T_new) : check_job<false>(job[i], dtype, B, H, T_new);
-        if (rc) return rc;
-    }
-    return encode_both(job, dtype, B, H, T_new, k_size, v_size, s);
+    const int rc = append_jobs(job, k, v, dtype, B, H, T_new, par_stride, nullptr, 0, k_size && v_size);
+    return rc ? rc : encode_both(job, dtype, B, H, T_new, k_size, v_size, (hipStream_t)s);
+}
+
+int pkv_kv_quant_encode_alone(const pkv_append_side *k, const pkv_append_side *v, int dtype, int B, int H, int T_new, int par_stride,
+                              const uint32_t *perm, int perm_block, uint64_t *k_size, uint64_t *v_size, pkv_stream_t s) {
+    using namespace pkv;
+    EncodeJob job[2];
+    const int rc = append_jobs(job, k, v, dtype, B, H, T_new, par_stride, perm, perm_block, k_size && v_size);
+    if (rc) return rc;
+    job[0].polls = job[1].polls = 0;
+    return encode_both(job, dtype, B, H, T_new, k_size, v_size, (hipStream_t)s);
 }
 
 }  // extern "C"

@@ -14,6 +14,11 @@
 namespace pkv {
 
 constexpr int kOnceSleep = 4;  // back-off of the waits, in units of 64 cycles: a few hundred workgroups at most poll
+// Polls before a wavefront stops waiting for the other runs of its group.  They take tickets after its own too and may not
+// have started -- another stream's kernel can hold the CUs that they need, for as long as it likes -- so it then reads the
+// rows of the whole group itself (once_exchange).  A few tenths of a millisecond; where nothing else runs a run's words are
+// there after a few microseconds.
+constexpr int kOncePolls = 512;
 
 // One side of a launch.
 struct OnceSide {
@@ -31,6 +36,7 @@ struct OnceSide {
     const uint32_t *perm;
     int perm_block;
     const uint16_t *scale_in, *zero_in;
+    int polls;                 // kOncePolls; 0: never wait for another run
     const uint8_t *codes;      // the block codec: a code matrix [T, hidden] instead of x
     int hidden;
 };
@@ -62,25 +68,33 @@ __device__ __forceinline__ uint32_t once_ticket(OnceLds<NT> &l, ScanState *st) {
 }
 
 // A 32-bit value per token of a wavefront (token lane / LANES, the same value in the LANES lanes) combined over all runs of the
-// group: `words` holds [run][stride] of them.  The wavefronts that `publish` store their run's; waits are bounded like the
-// look-back's.  `add(value)` is called for one run after the other, a LANES-th of them in each lane.
+// group: `words` holds [run][stride] of them.  The wavefronts that `publish` store their run's.  `add(value)` is called for one run
+// after the other, a LANES-th of them in each lane.  False (uniform) where a run was not there after `polls` looks: what was
+// added is then no result, and the caller forms the value from the rows of all runs.
 template <int LANES, class Add>
-__device__ __forceinline__ void once_exchange(uint64_t *words, uint32_t stride, uint32_t run, int nruns, bool publish, uint32_t mine, ScanState *st, Add add) {
+__device__ __forceinline__ bool once_exchange(uint64_t *words, uint32_t stride, uint32_t run, int nruns, bool publish, uint32_t mine, int polls, Add add) {
     const int lane = threadIdx.x & 63, tk = lane / LANES, part = lane % LANES;
     if (publish && part == 0)
         __hip_atomic_store(words + (size_t)run * stride + tk, (1ull << 63) | (uint64_t)mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (int q = part; q < nruns; q += LANES) {
+    bool there = polls > 0;
+    for (int q = part; q < nruns && there; q += LANES) {
         const uint64_t *wp = words + (size_t)q * stride + tk;
         uint64_t w = __hip_atomic_load(wp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        int spins = 0;
-        while ((w >> 63) == 0 && spins < kSpinLimit) {
+        while ((w >> 63) == 0 && polls > 0) {
             __builtin_amdgcn_s_sleep(kOnceSleep);
             w = __hip_atomic_load(wp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            spins++;
+            polls--;
         }
-        if ((w >> 63) == 0) atomicExch(&st->error, (uint32_t)PKV_ERR_INTERNAL);     // (bounded wait: the host reports it)
-        add((uint32_t)w);
+        there = (w >> 63) != 0;
+        if (there) add((uint32_t)w);
     }
+    return __all(there);
+}
+
+// (the sixteen row addresses are formed where they are used: kept for the rare path they took 30 registers)
+__device__ __forceinline__ int once_opaque(int head) {
+    asm volatile("" : "+s"(head));
+    return head;
 }
 
 // Token parameters from the minimum and maximum; the lanes that `write` store them.
@@ -179,16 +193,19 @@ __device__ __forceinline__ void k_encode_once(const OnceSide &a, OnceLds<NT> &l,
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = wave / WPR, wr = wave % WPR;
     const int lane = tid & 63, t = tid & 31;
     const size_t tok0 = (size_t)cb * 64 + 16 * (size_t)r;
-    const int jc = min(2 * wr + (lane >> 5), H - 1), j0 = min(2 * wr, H - 1);      // (a repeated head changes no minimum or maximum)
     uint2 xr[16];
-    if (PERM) {
-        const size_t blk0 = (size_t)cb * 64 / (size_t)a.perm_block * (size_t)a.perm_block;
-        cell_load_rows(a.x + ((size_t)b * a.H * a.T + blk0) * kHeadDim, a.perm + tok0, (uint32_t)a.perm_block - 1u,
-                       (uint32_t)(((size_t)(hbase + jc) * a.T * kHeadDim + 4 * t) * 2), xr);
-    } else {
-        cell_load(reinterpret_cast<const char *>(a.x + b * a.xs.sb + (hbase + j0) * a.xs.sh + (int64_t)tok0 * a.xs.st), 2 * a.xs.st,
-                  ((uint32_t)(jc - j0) * (uint32_t)a.xs.sh + 4u * (uint32_t)t) * 2u, xr);
-    }
+    auto load = [&](int head) {                            // heads `head` and the one after it in the halves (a repeated head changes no minimum or maximum)
+        const int j0 = min(head, a.H - 1), jc = min(head + (lane >> 5), a.H - 1);
+        if (PERM) {
+            const size_t blk0 = (size_t)cb * 64 / (size_t)a.perm_block * (size_t)a.perm_block;
+            cell_load_rows(a.x + ((size_t)b * a.H * a.T + blk0) * kHeadDim, a.perm + tok0, (uint32_t)a.perm_block - 1u,
+                           (uint32_t)(((size_t)jc * a.T * kHeadDim + 4 * t) * 2), xr);
+        } else {
+            cell_load(reinterpret_cast<const char *>(a.x + b * a.xs.sb + j0 * a.xs.sh + (int64_t)tok0 * a.xs.st), 2 * a.xs.st,
+                      ((uint32_t)(jc - j0) * (uint32_t)a.xs.sh + 4u * (uint32_t)t) * 2u, xr);
+        }
+    };
+    load(hbase + 2 * wr);
     float mn, mx;                                          // of token lane / 4
     cell_token_minmax<DT>(xr, mn, mx);
     if (WPR > 1) {
@@ -204,15 +221,28 @@ __device__ __forceinline__ void k_encode_once(const OnceSide &a, OnceLds<NT> &l,
     if (a.nruns > 1) {
         const uint32_t mine = T16<DT>::to_bits(mn) << 16 | T16<DT>::to_bits(mx);
         // (NaN drops out of minima and maxima; a token that is nothing else keeps what the cells kernels make of it)
-        mn = a.H <= 8 ? NAN : INFINITY, mx = a.H <= 8 ? NAN : -INFINITY;
-        once_exchange<4>(a.xw + (size_t)grp * a.nruns * 64 + 16 * r, 64, run, a.nruns, wr == 0, mine, a.st, [&](uint32_t w) {
-            mn = fminf(mn, T16<DT>::from_bits(w >> 16));
-            mx = fmaxf(mx, T16<DT>::from_bits(w & 0xFFFFu));
-        });
+        const float mn0 = a.H <= 8 ? NAN : INFINITY, mx0 = a.H <= 8 ? NAN : -INFINITY;
+        mn = mn0, mx = mx0;
+        if (once_exchange<4>(a.xw + (size_t)grp * a.nruns * 64 + 16 * r, 64, run, a.nruns, wr == 0, mine, a.polls, [&](uint32_t w) {
+                mn = fminf(mn, T16<DT>::from_bits(w >> 16));
+                mx = fmaxf(mx, T16<DT>::from_bits(w & 0xFFFFu));
+            })) {
 #pragma unroll
-        for (int d = 1; d < 4; d <<= 1) {
-            mn = fminf(mn, __shfl_xor(mn, d, 64));
-            mx = fmaxf(mx, __shfl_xor(mx, d, 64));
+            for (int d = 1; d < 4; d <<= 1) {
+                mn = fminf(mn, __shfl_xor(mn, d, 64));
+                mx = fmaxf(mx, __shfl_xor(mx, d, 64));
+            }
+        } else {
+            mn = mn0, mx = mx0;
+#pragma unroll 1
+            for (int h = 0; h < a.H; h += 2) {
+                load(once_opaque(h));
+                float hmn, hmx;
+                cell_token_minmax<DT>(xr, hmn, hmx);
+                mn = fminf(mn, hmn);
+                mx = fmaxf(mx, hmx);
+            }
+            load(once_opaque(hbase + 2 * wr));
         }
     }
     TokPar *par = l.par + 32 * wave;
@@ -294,17 +324,19 @@ __device__ __forceinline__ void v_encode_once(const OnceSide &a, OnceLds<NT> &l,
     const int hbase = R * (int)run, H = min(R, a.H - hbase);
     const uint32_t cb = grp / (uint32_t)a.B, b = grp % (uint32_t)a.B;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), it = wave / R, j = wave % R;
-    const int lane = tid & 63, rp = lane >> 5, t = lane & 31, jc = min(j, H - 1);
+    const int lane = tid & 63, rp = lane >> 5, t = lane & 31;
     const size_t tok = (size_t)cb * 128 + 32 * (size_t)it;
     const size_t rb = PERM ? tok / (size_t)a.perm_block * (size_t)a.perm_block : 0;      // (32 tokens lie in one repacking block)
     uint2 xr[16];
-    if (PERM) {
-        cell_load_rows_lanes(a.x + ((size_t)b * a.H * a.T + rb) * kHeadDim, a.perm + tok + 16 * rp, (uint32_t)a.perm_block - 1u,
-                             (uint32_t)(((size_t)(hbase + jc) * a.T * kHeadDim + 4 * t) * 2), xr);
-    } else {
-        cell_load(reinterpret_cast<const char *>(a.x + b * a.xs.sb + (hbase + jc) * a.xs.sh + (int64_t)tok * a.xs.st), 2 * a.xs.st,
-                  (16u * (uint32_t)rp * (uint32_t)a.xs.st + 4u * (uint32_t)t) * 2u, xr);
-    }
+    auto load = [&](int head) {
+        if (PERM)
+            cell_load_rows_lanes(a.x + ((size_t)b * a.H * a.T + rb) * kHeadDim, a.perm + tok + 16 * rp, (uint32_t)a.perm_block - 1u,
+                                 (uint32_t)(((size_t)head * a.T * kHeadDim + 4 * t) * 2), xr);
+        else
+            cell_load(reinterpret_cast<const char *>(a.x + b * a.xs.sb + head * a.xs.sh + (int64_t)tok * a.xs.st), 2 * a.xs.st,
+                      (16u * (uint32_t)rp * (uint32_t)a.xs.st + 4u * (uint32_t)t) * 2u, xr);
+    };
+    load(hbase + min(j, H - 1));
     TokPar *par = l.par + 32 * wave;
     const size_t ptok = (size_t)b * a.par_stride + tok + (lane >> 1);                    // of token lane / 2
     const bool write = (lane & 1) == 0 && j == 0 && run == 0;
@@ -330,9 +362,19 @@ __device__ __forceinline__ void v_encode_once(const OnceSide &a, OnceLds<NT> &l,
         }
         if (a.nruns > 1) {
             const uint32_t mine = pw;
-            once_exchange<2>(a.xw + (size_t)grp * a.nruns * 128 + 32 * it, 128, run, a.nruns, j == 0, mine, a.st,
-                             [&](uint32_t w) { pw = pk_sel_x<false, DT != PKV_F16>(pw, w); });
-            pw = pk_sel_x<false, DT != PKV_F16>(pw, (uint32_t)__shfl_xor((int)pw, 1, 64));
+            if (once_exchange<2>(a.xw + (size_t)grp * a.nruns * 128 + 32 * it, 128, run, a.nruns, j == 0, mine, a.polls,
+                                 [&](uint32_t w) { pw = pk_sel_x<false, DT != PKV_F16>(pw, w); })) {
+                pw = pk_sel_x<false, DT != PKV_F16>(pw, (uint32_t)__shfl_xor((int)pw, 1, 64));
+            } else {
+                pw = mine;
+#pragma unroll 1
+                for (int h = 0; h < a.H; h++) {
+                    load(once_opaque(h));
+                    cell_token_minmax_halves<DT>(xr, mn, mx);
+                    pw = pk_sel_x<false, DT != PKV_F16>(pw, minmax_word<DT>(mn, mx));
+                }
+                load(once_opaque(hbase + min(j, H - 1)));
+            }
         }
         minmax_unword<DT>(pw, mn, mx);
         if (a.H > 8) mn = fminf(mn, INFINITY), mx = fmaxf(mx, -INFINITY);      // (a token of NaN only, as above)

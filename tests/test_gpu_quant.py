@@ -392,3 +392,37 @@ def test_nan_parameters_do_not_depend_on_the_launch(cuda, dtype, H):
             a, b = small[name].cpu(), whole[name][:, :128].cpu()
             same = (a.view(torch.int16) == b.view(torch.int16)) | (a.isnan() & b.isnan())
             assert bool(same.all()), (enc.__name__, name, (~same).nonzero().tolist())
+
+
+# Runs of two heads of K and one of V (256 threads), of eight and four (1024), one launch for both sides and two.
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,H,T,rels,block", [(1, 8, 512, (0.1, 0.1), 0), (2, 3, 256, (0.05, 0.1), 0), (1, 32, 128, (0.1, 0.1), 0), (1, 8, 4224, (0.05, 0.05), 0),
+                                              (1, 20, 4096, (0.1, 0.2), 0), (1, 8, 512, (0.1, 0.1), 64), (3, 5, 256, (0.05, 0.05), 128)])
+def test_a_run_that_waits_for_no_other_gives_the_same_stream(cuda, dtype, B, H, T, rels, block):
+    """The encode of few groups with no look at what the other runs of a group found, as when they do not start."""
+    x = list(synth.make_kv(B, H, T, seed=H + T, dtype=dtype, device=cuda))
+    for i in range(2):
+        x[i][0, 1, 5, 7], x[i][0, :, 9], x[i][0, H - 1, 40, 3], x[i][0, 0, 41, 100] = float("nan"), float("nan"), float("inf"), -float("inf")
+    perm = None
+    if block:
+        perm = torch.stack([torch.randperm(block, generator=torch.Generator().manual_seed(i)) for i in range(T // block)]).to(torch.int32).reshape(-1).to(cuda)
+    want = [ops._quant_encode(i == 0, x[i], rels[i], ops.bits_for_rel(rels[i]), None, None, False, False, perm, block) for i in range(2)]
+    got, sides = [], []
+    for i in range(2):
+        stream, info = ops._stream_and_info(i == 0, x[i], want[i]["bits"])
+        scale, zero = torch.zeros(B, T, dtype=dtype, device=cuda), torch.zeros(B, T, dtype=dtype, device=cuda)
+        got.append({"stream": stream, "info": info, "scale": scale, "zero": zero})
+        sides.append(_lib.AppendSide(x[i].data_ptr(), *x[i].stride()[:3], stream.data_ptr(), stream.numel(), 0, info.data_ptr(), scale.data_ptr(),
+                                     zero.data_ptr(), rels[i], want[i]["bits"]))
+    sizes = [ctypes.c_uint64(0), ctypes.c_uint64(0)]
+    rc = _lib.load().pkv_kv_quant_encode_alone(ctypes.byref(sides[0]), ctypes.byref(sides[1]), _lib.F16 if dtype == torch.float16 else _lib.BF16, B, H, T, T,
+                                               None if perm is None else ctypes.c_void_p(perm.data_ptr()), block, ctypes.byref(sizes[0]),
+                                               ctypes.byref(sizes[1]), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert rc in (0, 1), _lib.load().pkv_last_error()         # (1: codes of the tokens with infinities that are too wide)
+    for i in range(2):
+        end = want[i]["info"].view(torch.int32)[-1].cpu().sum().item()
+        assert end > 0 and (rc or sizes[i].value == end)
+        assert torch.equal(got[i]["stream"][:end], want[i]["stream"][:end])
+        for name in ("info", "scale", "zero"):
+            assert torch.equal(got[i][name].view(torch.int16), want[i][name].view(torch.int16)), name
