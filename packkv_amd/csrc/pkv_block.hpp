@@ -178,7 +178,7 @@ __device__ __forceinline__ void unit_codes(const uint8_t *blk, uint32_t unit_off
 
 // The same for a width known at compile time (2..4), for consumers that multiply: `sink(k, c01, c23)` gets the codes of
 // slots 0 | 1 and 2 | 3 at token k as 16-bit lanes.  Such a lane read as a half is the code times 2^-24 (a subnormal), which
-// v_fma_mix_f32 multiplies exactly: no conversion.  (Not the offsets alone with the minima multiplied apart: a factor that is
+// v_fma_mix_f32 multiplies exactly where the product is no subnormal: no conversion.  (Not the offsets alone with the minima multiplied apart: a factor that is
 // infinite would meet an offset of zero.)
 template <int W, class Sink>
 __device__ __forceinline__ void unit_fields(const uint8_t *blk, uint32_t unit_off, int t, Sink sink) {

@@ -37,23 +37,37 @@ __device__ __forceinline__ void wave_lds_order() {         // LDS serves a wavef
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// f.x .. f.w times the four codes c01 | c23 (unit_fields) times 2^-24: products exact, fp32 sums.  The sum is scaled
-// back and not the factors: 2^24 times a large bf16 value would overflow.
-constexpr float kFieldUnit = 16777216.f;                   // 2^24
+// f.x .. f.w times the four codes c01 | c23 as unit_fields hands them out, i.e. codes times 2^-24 read from halves: products
+// exact, fp32 sums.  The factors come 2^24 times as large, so that the products are those of the codes: with the sum scaled
+// back instead, products of bf16 factors below 2^-102 fell among the subnormals and lost bits.  Factors of 2^100 and more
+// could overflow: where a row holds one (or a NaN), a code is scaled instead, one more instruction each (BIG).
+constexpr float kFieldUnit = 16777216.f, kFieldMost = 0x1p100f;      // 2^24
 typedef _Float16 half_pair __attribute__((ext_vector_type(2)));
+template <bool BIG>
+__device__ __forceinline__ float field(_Float16 c) { return BIG ? (float)c * kFieldUnit : (float)c; }
+template <bool BIG>
 __device__ __forceinline__ float dot4(uint32_t c01, uint32_t c23, const float4 f) {
     const half_pair a = __builtin_bit_cast(half_pair, c01), b = __builtin_bit_cast(half_pair, c23);
-    float s = (float)a[1] * f.y;
-    s = fmaf((float)a[0], f.x, s);
-    s = fmaf((float)b[0], f.z, s);
-    return fmaf((float)b[1], f.w, s);
+    float s = field<BIG>(a[1]) * f.y;
+    s = fmaf(field<BIG>(a[0]), f.x, s);
+    s = fmaf(field<BIG>(b[0]), f.z, s);
+    return fmaf(field<BIG>(b[1]), f.w, s);
 }
+template <bool BIG>
 __device__ __forceinline__ float dot4(uint32_t c01, uint32_t c23, const float4 f, float acc) {
     const half_pair a = __builtin_bit_cast(half_pair, c01), b = __builtin_bit_cast(half_pair, c23);
-    acc = fmaf((float)a[0], f.x, acc);
-    acc = fmaf((float)a[1], f.y, acc);
-    acc = fmaf((float)b[0], f.z, acc);
-    return fmaf((float)b[1], f.w, acc);
+    acc = fmaf(field<BIG>(a[0]), f.x, acc);
+    acc = fmaf(field<BIG>(a[1]), f.y, acc);
+    acc = fmaf(field<BIG>(b[0]), f.z, acc);
+    return fmaf(field<BIG>(b[1]), f.w, acc);
+}
+// True (uniform) when one of the wavefront's factors, `N` a lane, is too large for 2^24 times itself, or NaN.
+template <int N>
+__device__ __forceinline__ bool factors_big(const float (&f)[N]) {
+    bool big = false;
+#pragma unroll
+    for (int i = 0; i < N; i++) big = big || !(fabsf(f[i]) < kFieldMost);
+    return __any(big);
 }
 
 // K . q: wavefront per K block (`wpw` of them to a workgroup, `slot` bytes of LDS each), a half per round, lane = four
@@ -84,14 +98,17 @@ __global__ void __launch_bounds__(256) kq_kernel(const uint8_t *__restrict__ str
         const int src = !q_interleaved ? 4 * t + i : i < 2 ? 2 * t + i : 64 + 2 * t + (i - 2);
         qf[i] = ld16(q, (size_t)hb * kHeadDim + src, dtype);
     }
-    const float4 q4 = make_float4(qf[0], qf[1], qf[2], qf[3]);
+    const bool big = factors_big(qf);
+    const float unit_q = big ? 1.f : kFieldUnit;
+    const float4 q4 = make_float4(qf[0] * unit_q, qf[1] * unit_q, qf[2] * unit_q, qf[3] * unit_q);
     wave_lds_order();
     const uint16_t *cum = reinterpret_cast<const uint16_t *>(blk + phase);      // (phase is even)
 #pragma unroll 1
     for (int u0 = 0; u0 < nunits; u0 += 2) {
         const int unit = min(u0 + half, nunits - 1);      // (an odd last round: both halves decode it, the first one writes)
         const uint32_t start = phase + 2u * (uint32_t)nunits + (unit ? (uint32_t)cum[unit - 1] : 0u);
-        unit_fields<W>(blk, start, t, [&](int k, uint32_t c01, uint32_t c23) { turn[kKqTok * k + l16] = dot4(c01, c23, q4); });
+        if (big) unit_fields<W>(blk, start, t, [&](int k, uint32_t c01, uint32_t c23) { turn[kKqTok * k + l16] = dot4<true>(c01, c23, q4); });
+        else unit_fields<W>(blk, start, t, [&](int k, uint32_t c01, uint32_t c23) { turn[kKqTok * k + l16] = dot4<false>(c01, c23, q4); });
         wave_lds_order();
         float s = 0.f;
 #pragma unroll
@@ -101,7 +118,7 @@ __global__ void __launch_bounds__(256) kq_kernel(const uint8_t *__restrict__ str
             s += v.w;
         }
         wave_lds_order();
-        s = kFieldUnit * (s + __shfl_xor(s, 16, 64));
+        s += __shfl_xor(s, 16, 64);
         if ((lane & 16) == 0 && u0 + half < nunits) kq_out[(size_t)hb * ctx_len + (size_t)cb * ctx_blk + 16 * unit + l16] = st16(s, dtype);
     }
 }
@@ -130,11 +147,13 @@ __global__ void __launch_bounds__(64 * kWvWaves) wv_kernel(const uint8_t *__rest
         uint32_t off, size;
         block_span(info, cb * n_hid + hb, blk_cap, stream_bytes, off, size);
         const uint32_t phase = stage_to_lds(stream + off, size, blk, lane, 64);
+        float wf[2];
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const int tok = lane + 64 * i;                 // segment i, round lane / 16, token lane % 16 of the pack
-            ws[wave][64 * i + 4 * (lane & 15) + (lane >> 4)] = ld16(w, (size_t)head * ctx_len + (size_t)cb * 128 + tok, dtype);
-        }
+        for (int i = 0; i < 2; i++) wf[i] = ld16(w, (size_t)head * ctx_len + (size_t)cb * 128 + lane + 64 * i, dtype);
+        const bool big = factors_big(wf);
+#pragma unroll
+        for (int i = 0; i < 2; i++)                        // segment i, round lane / 16, token lane % 16 of the pack
+            ws[wave][64 * i + 4 * (lane & 15) + (lane >> 4)] = wf[i] * (big ? 1.f : kFieldUnit);
         wave_lds_order();
         const uint16_t *cum = reinterpret_cast<const uint16_t *>(blk + phase);  // (phase is even)
 #pragma unroll 1
@@ -145,9 +164,10 @@ __global__ void __launch_bounds__(64 * kWvWaves) wv_kernel(const uint8_t *__rest
             const int unit = 2 * p + seg;
             const uint32_t start = phase + 4u * (uint32_t)npair + (unit ? (uint32_t)cum[unit - 1] : 0u);
             float acc[4] = {0.f, 0.f, 0.f, 0.f};
-            unit_fields<W>(blk, start, t, [&](int k, uint32_t c01, uint32_t c23) { acc[k & 3] = dot4(c01, c23, w4[k], acc[k & 3]); });
+            if (big) unit_fields<W>(blk, start, t, [&](int k, uint32_t c01, uint32_t c23) { acc[k & 3] = dot4<true>(c01, c23, w4[k], acc[k & 3]); });
+            else unit_fields<W>(blk, start, t, [&](int k, uint32_t c01, uint32_t c23) { acc[k & 3] = dot4<false>(c01, c23, w4[k], acc[k & 3]); });
             const float s = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-            const float both = kFieldUnit * (s + __shfl_xor(s, 32, 64));
+            const float both = s + __shfl_xor(s, 32, 64);
             if (seg == 0) part[wave][kLanes * p + t] = both;
         }
     } else {

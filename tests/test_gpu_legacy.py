@@ -213,3 +213,43 @@ def test_fused_fixups_any_length_and_alignment(cuda, N, off):
     want = c.sum(1, keepdim=True) + term1.double()
     mag = c.abs().sum(1, keepdim=True) + term1.double().abs()
     assert bool(((wv.double() - want).abs() <= 2 ** -11 * want.abs() * 1.01 + 2 ** -14 * mag + 2 ** -24).all())
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4])
+@pytest.mark.parametrize("low,high", [(-126, -116), (-126, 110), (100, 115)])
+def test_bf16_factors_of_any_size(cuda, low, high, bits):
+    """bf16 q and weights near the ends of the exponent range, and both ends in one row (the large ones over channels and
+    tokens whose codes are zero, so that the small ones make the result)."""
+    H, T = 3, 256
+    g = torch.Generator().manual_seed(bits)
+    codes = torch.randint(1, 1 << bits, (T, H * 128), generator=g, dtype=torch.uint8)
+    mixed = high - low > 100
+    if mixed:
+        codes[:, ::8], codes[::8] = 0, 0
+
+    def factors(n, zero):
+        e = torch.randint(low, low + 10, (H, n), generator=g).double()
+        f = (1 + torch.rand(H, n, generator=g).double()) * 2 ** e
+        if mixed:
+            f[:, zero] = 2.0 ** high
+        return f.to(torch.bfloat16)
+    q, w = factors(128, slice(0, None, 8)), factors(T, slice(0, None, 8))
+    c = codes.double().view(T, H, 128)
+    for is_k, cb, hb in ((True, 64, 128), (False, 128, 64)):
+        n = codes.numel() // (cb * hb)
+        stream = torch.zeros(n * ops.block_bound(is_k, cb, hb, bits) + 16, dtype=torch.uint8, device=cuda)
+        info = torch.zeros(n, 2, dtype=torch.uint32, device=cuda)
+        (ops.k_encode if is_k else ops.v_encode)(codes.to(cuda), stream, info, cb, hb, bits)
+        # all terms are non-negative: the fp32 sums of exact products are off by at most a rounding of 2^-24 a term; bf16 rounds
+            # to 8 bits
+        if is_k:
+            got = torch.empty(H, T, dtype=torch.bfloat16, device=cuda)
+            ops.kq_mat_vec_mul(stream, info, q.to(cuda), got, T, H * 128, cb, hb, bits, q_interleaved=False)
+            want = torch.einsum("thd,hd->ht", c, q.double())
+            bound = (2 ** -8 + 136 * 2 ** -24) * 1.01
+        else:
+            got = torch.zeros(H, 128, dtype=torch.float32, device=cuda)
+            ops.wv_mat_vec_mul(stream, info, w.to(cuda), got, T, H * 128, cb, hb, bits)
+            want = torch.einsum("ht,thd->hd", w.double(), c)
+            bound = (T + 8) * 2 ** -24
+        assert bool(((got.cpu().double() - want).abs() <= bound * want).all()), is_k
