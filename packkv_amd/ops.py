@@ -118,7 +118,9 @@ def _check_codec_args(codes, stream, info, ctx_len, hidden_dim, ctx_blk, hid_blk
 # link moves 8 MiB between it and the device in 155 us, where a copy from or to pageable memory takes 246 and 460 us (574
 # into a fresh tensor); the copy on the host is 16 us.  Smaller tensors are copied as they are, the buffer and the event cost
 # more than they save there.  Up / down in us, as they are and staged: 128 KiB 17 / 18 and 30 / 42, 512 KiB 28 / 34 and
-# 37 / 51, 1 MiB 57 / 66 and 47 / 63, 8 MiB 250 / 523 and 201 / 235.
+# 37 / 51, 1 MiB 57 / 66 and 47 / 63, 8 MiB 250 / 523 and 201 / 235.  Tensors that the caller holds in page-locked memory go
+# over the link as they are (8 MiB 160 / 160, staged 191 / 244).  The allocator keeps the pieces, at most 2 x 32 MiB of them for
+# each host thread that copies at a time.
 _STAGE_BYTES = 32 << 20
 _STAGE_FROM = 1 << 20
 
@@ -146,7 +148,7 @@ def _staged(n, pieces, step):
 
 def _upload(dst, src):
     """Device bytes dst = host bytes src, on the current stream of dst's device; src may be reused at once."""
-    if src.numel() < _STAGE_FROM:
+    if src.numel() < _STAGE_FROM or src.is_pinned():
         dst.copy_(src)
         return
     last = src.numel() <= _STAGE_BYTES
@@ -162,7 +164,7 @@ def _upload(dst, src):
 
 def _download(dst, src):
     """Host bytes dst = device bytes src, there when this returns."""
-    if src.numel() < _STAGE_FROM:
+    if src.numel() < _STAGE_FROM or dst.is_pinned():
         dst.copy_(src)
         return
 

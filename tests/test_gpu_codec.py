@@ -418,3 +418,29 @@ def test_host_tensors_in_pieces(cuda, monkeypatch, is_k, stage, staged_from):
     back.zero_()
     dec(exact, bad.view(torch.uint32), back, 384, 1024, cb, hb, 4)
     assert torch.equal(back[:256], codes[:256])
+
+
+@pytest.mark.parametrize("is_k", [True, False])
+def test_page_locked_host_tensors_go_over_the_link_as_they_are(cuda, monkeypatch, is_k):
+    """Nothing of a caller's page-locked tensors, whole or a part of a larger one, is copied on the host first; pageable ones are."""
+    staged, real = [], ops._staged
+    monkeypatch.setattr(ops, "_staged", lambda n, pieces, step: (staged.append(n), real(n, pieces, step)))
+    codes = torch.randint(0, 16, (2048, 1024), generator=torch.Generator().manual_seed(3), dtype=torch.uint8)
+    cb, hb = (64, 128) if is_k else (128, 64)
+    n = codes.numel() // 8192
+    enc, dec = (ops.k_encode_cpu, ops.k_decode_cpu) if is_k else (ops.v_encode_cpu, ops.v_decode_cpu)
+    room = n * ops.block_bound(is_k, cb, hb, 4) + 16
+    sizes = []
+    for pin, part in ((False, 0), (True, 0), (True, 2)):
+        staged.clear()
+
+        def host(values):
+            t = torch.empty(values.numel() * values.element_size() + 4 * part, dtype=torch.uint8, pin_memory=pin)[4 * part:]
+            t = t.view(values.dtype).view(values.shape)
+            return t.copy_(values)
+        src, back = host(codes), host(torch.zeros_like(codes))
+        stream, info = host(torch.zeros(room, dtype=torch.uint8)), host(torch.zeros(n, 2, dtype=torch.int32)).view(torch.uint32)
+        sizes.append(enc(src, stream, info, 2048, 1024, cb, hb, 4))
+        dec(stream, info, back, 2048, 1024, cb, hb, 4)
+        assert torch.equal(back, codes) and sizes[-1] == sizes[0]
+        assert (staged == []) == pin
