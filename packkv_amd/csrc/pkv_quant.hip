@@ -1715,7 +1715,8 @@ namespace pkv {
 // 128-channel slices of the matrix.  A thread reads its cell as sixteen dwords (four codes of one token each; the 32
 // lanes of a half-wavefront one 128-byte line per token), asks for the next round's while it forms and emits this
 // round's packs, and no code tile is staged in LDS.  For hidden a multiple of 1024, the reference's block shapes and
-// widths up to 6; pack_group_kernel takes everything else.
+// widths up to 6.  Launches of few groups take all tokens of a group at once (code_encode_once_kernel), also with other
+// rows of whole runs; pack_group_kernel takes everything else.
 template <bool WIDE>
 __global__ void __launch_bounds__(256) k_code_cells_kernel(
     const uint8_t *__restrict__ codes, int hidden, uint8_t *__restrict__ stream, uint64_t capacity,

@@ -329,7 +329,8 @@ __global__ void __launch_bounds__(kGreedyThreads) greedy_order_kernel(const uint
 // workgroups takes ~6.5 us on an MI355X: 3.8 us of pricing at the full rate of the vector ALUs, the rest the sums,
 // the exchange, the winner and the slot move, which nothing overlaps.
 constexpr int kSlicedThreadsWide = 512;                 // one workgroup per CU, two wavefronts per SIMD: rows of two or more slices
-constexpr int kSlicedThreadsNarrow = 256;               // two workgroups per CU: rows of up to 2048 channels
+constexpr int kSlicedThreadsNarrow = 256;               // two workgroups per CU: rows of up to 2048 channels in more than 256 blocks
+                                                        // (fewer blocks, and rows of up to 1024: greedy_order_block_kernel)
 constexpr int kSlicedTokens = 64;
 constexpr int kGreedySpinLimit = 1 << 22;
 // words per row of the per-thread sums: runs of 32 threads, each + 4, then + 4
@@ -891,10 +892,12 @@ typedef unsigned short pk_u16x2 __attribute__((ext_vector_type(2)));
 // One or two matrices of one shape (K and V: blockIdx.y), whose last workgroups report apart; with PERM the rows of a block of
 // `block_size` tokens (a multiple of the pack) in the order of a repacking: row r of block b is row perm[b * block_size + r] of it, so that
 // a repacked matrix need not be written to be priced (16384 x 2 x 1024 codes: 27.1 us a call; written first, 25.5 and 11 for the gather).
+constexpr int kPackSizeMost = 2, kPackSizeWords = 3;       // matrices of a launch, words of a slot for each
+static_assert(kPackSizeMost * kPackSizeWords <= kSlotWords, "a slot holds the results of a launch: the next one is another thread's");
 struct PackSizeJob {
-    const uint8_t *codes[2];
+    const uint8_t *codes[kPackSizeMost];
     PackSizeState *st;                   // one for each matrix
-    unsigned long long *slot;            // three words for each matrix
+    unsigned long long *slot;            // kPackSizeWords words for each matrix
     const uint32_t *perm;
     int block_size;
 };
@@ -902,7 +905,7 @@ template <int WORDS, bool PERM>
 __global__ void __launch_bounds__(1024) pack_size_kernel(const PackSizeJob job, int hidden, int pack_len, size_t n_items, uint32_t tag) {
     const uint8_t *__restrict__ codes = job.codes[blockIdx.y];
     PackSizeState *st = job.st + blockIdx.y;
-    unsigned long long *slot = job.slot + 3 * blockIdx.y;
+    unsigned long long *slot = job.slot + kPackSizeWords * blockIdx.y;
     // a presence word per (code value, lane % 32): a lane marks its own column, so the marks of a wavefront never
     // share a bank however few values the matrix holds (one word per value made every mark a same-address conflict)
     __shared__ __align__(16) uint32_t seen[256 * 32];
@@ -1004,6 +1007,7 @@ __global__ void __launch_bounds__(1024) pack_size_kernel(const PackSizeJob job, 
 
 static int pack_sizes(const uint8_t *const *codes, int n, const uint32_t *perm, int block_size, int ctx_len, int hidden_dim, int pack_len,
                       uint64_t *len_sum_out, uint32_t *n_unique_out, float *ms_out, hipStream_t s) {
+    PKV_REQUIRE(n >= 1 && n <= kPackSizeMost, PKV_ERR_INVALID, "one or two matrices");
     PKV_REQUIRE(len_sum_out && n_unique_out, PKV_ERR_INVALID, "null pointer argument");
     for (int i = 0; i < n; i++) PKV_REQUIRE(codes[i], PKV_ERR_INVALID, "null pointer argument");
     PKV_REQUIRE(ctx_len > 0 && hidden_dim > 0 && pack_len > 0, PKV_ERR_INVALID, "sizes must be positive");
@@ -1035,11 +1039,12 @@ static int pack_sizes(const uint8_t *const *codes, int n, const uint32_t *perm, 
     PKV_HIP_CHECK(hipGetLastError());
     if ((rc = scan_state_cleared(sh, s))) return rc;
     if ((rc = tm.end(ms_out))) return rc;
-    uint64_t v[6];
-    if ((rc = slot.wait(3 * n, s, v))) return rc;
+    uint64_t v[kPackSizeMost * kPackSizeWords];
+    if ((rc = slot.wait(kPackSizeWords * n, s, v))) return rc;
     for (int i = 0; i < n; i++) {
-        len_sum_out[i] = v[3 * i] | v[3 * i + 1] << 32;
-        n_unique_out[i] = (uint32_t)v[3 * i + 2];
+        const uint64_t *r = v + kPackSizeWords * i;
+        len_sum_out[i] = r[0] | r[1] << 32;
+        n_unique_out[i] = (uint32_t)r[2];
     }
     return PKV_OK;
 }

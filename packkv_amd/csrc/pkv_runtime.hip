@@ -41,7 +41,8 @@ struct Workspace {
     uint64_t *last;         // pinned, host and device: outcome of the last encode on this stream (kOutcomeWords), tag 0 before it
     std::shared_ptr<std::mutex> enc_mu;
 };
-constexpr int kOutcomeWords = 2, kSlotWords = 8;      // a slot: two outcomes (a cache line)
+constexpr int kOutcomeWords = 2;
+static_assert(2 * kOutcomeWords <= kSlotWords, "a slot (a cache line) holds the outcomes of two encodes");
 constexpr int kSlotsPerChunk = 64;
 std::vector<uint64_t *> g_chunks;                     // pinned slots of the encodes that are waited for (any device)
 std::vector<uint64_t *> g_free_slots;                 // as many as host threads have waited at once, in chunks of 64

@@ -77,9 +77,10 @@ int prepare_scan_state(uint32_t nblocks, ScanHandle *out, hipStream_t s, bool wa
 // (`size2_out`: of the second state).  `bits` > 0 additionally rejects a launch whose largest code does not fit.
 // NULL: returns at once, pkv_encode_status reads the outcome later.
 int finish_encode(ScanHandle &h, uint64_t *size_out, int bits, hipStream_t s, uint64_t *size2_out = nullptr, int bits2 = 0);
-// For a kernel whose last workgroup publishes the outcome and clears the state by itself: a pinned slot of eight words
+// For a kernel whose last workgroup publishes the outcome and clears the state by itself: a pinned slot of kSlotWords words
 // that are valid one by one through their tag (value, 34 bits | tag << 34), and the two ends of its life.  Refused while
 // `s` is capturing (a graph's replays would write to a slot that has been given back).
+constexpr int kSlotWords = 8;
 struct OutcomeSlot {
     uint64_t *words = nullptr;
     uint32_t tag = 0;
