@@ -639,7 +639,9 @@ __device__ __forceinline__ void cell_build(const uint32_t c01[16], const uint32_
     u.len[0] = len01 & 0xFFFFu; u.len[1] = len01 >> 16; u.len[2] = len23 & 0xFFFFu; u.len[3] = len23 >> 16;
 }
 
-// The four packs of a loaded cell (rows xr, the 16 tokens' constants at par): words, minima, widths.
+// The four packs of a loaded cell (rows xr, the 16 tokens' constants at par): words, minima, widths.  For the round-major
+// encoders: with one or three heads the halves of a wavefront serve different groups, hence different tokens, so each lane takes
+// its own token's sequence.
 template <int DT>
 __device__ __forceinline__ void cell_packs(const uint2 xr[16], const TokPar *par, UnitPacks &u, uint32_t &cmax) {
     uint32_t c01[16], c23[16];
@@ -648,7 +650,7 @@ __device__ __forceinline__ void cell_packs(const uint2 xr[16], const TokPar *par
         for (int k = 0; k < 16; k++) quant4_f16_fast(xr[k], par[k], c01[k], c23[k]);
     } else {
 #pragma unroll
-        for (int k = 0; k < 16; k++) quant4<DT>(xr[k], par[k], c01[k], c23[k]);
+        for (int k = 0; k < 16; k++) quant4<DT, false>(xr[k], par[k], c01[k], c23[k]);
     }
     uint32_t mn01, mn23, len01, len23, mx01, mx23;
     build_pair(c01, mn01, len01, mx01, u.word[0], u.word[1]);
@@ -727,7 +729,7 @@ __device__ __forceinline__ void cell_packs(const uint2 xr[16], const TokPar *par
         for (int k = 0; k < 16; k++) quant4_f16_fast(xr[k], par[k], c01[k], c23[k]);
     } else {
 #pragma unroll
-        for (int k = 0; k < 16; k++) quant4<DT>(xr[k], par[k], c01[k], c23[k]);
+        for (int k = 0; k < 16; k++) quant4<DT, false>(xr[k], par[k], c01[k], c23[k]);
     }
     uint32_t mn01, mn23, len01, len23, mx01, mx23;
     build_pair_wide(c01, mn01, len01, mx01, u.lo[0], u.hi[0], u.lo[1], u.hi[1]);

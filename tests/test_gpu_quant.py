@@ -374,8 +374,8 @@ def test_encodes_at_once_report_codes_and_capacity(cuda, T):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("H", [3, 8, 12])
 def test_nan_parameters_do_not_depend_on_the_launch(cuda, dtype, H):
-    """Tokens with NaN and infinities get the same scale and zero from a launch of one group and from one that fills the
-    chip (257 groups of V: other kernels)."""
+    """Tokens with NaN and infinities get the same scale, zero and codes from a launch of one group and from one that fills
+    the chip (257 groups of V: other kernels)."""
     g = torch.Generator(device=cuda).manual_seed(5)
     big = torch.randn(1, H, 128 * 257, 128, generator=g, device=cuda).to(dtype)
     nan, inf = float("nan"), float("inf")
@@ -392,6 +392,11 @@ def test_nan_parameters_do_not_depend_on_the_launch(cuda, dtype, H):
             a, b = small[name].cpu(), whole[name][:, :128].cpu()
             same = (a.view(torch.int16) == b.view(torch.int16)) | (a.isnan() & b.isnan())
             assert bool(same.all()), (enc.__name__, name, (~same).nonzero().tolist())
+        info = small["info"].view(torch.int32)                # the same blocks at the same place: the group comes first in both streams
+        assert torch.equal(info, whole["info"].view(torch.int32)[:info.size(0)]), enc.__name__
+        end = int(info[-1].sum())
+        differ = (small["stream"][:end] != whole["stream"][:end]).nonzero().flatten().tolist()
+        assert not differ, (enc.__name__, len(differ), differ[:8])
 
 
 # Runs of two heads of K and one of V (256 threads), of eight and four (1024), one launch for both sides and two.
@@ -426,3 +431,20 @@ def test_a_run_that_waits_for_no_other_gives_the_same_stream(cuda, dtype, B, H, 
         assert torch.equal(got[i]["stream"][:end], want[i]["stream"][:end])
         for name in ("info", "scale", "zero"):
             assert torch.equal(got[i][name].view(torch.int16), want[i][name].view(torch.int16)), name
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("H,T", [(1, 128), (3, 128), (2, 128), (1, 16640), (3, 16640)])
+def test_padding_of_one_sequence_leaves_the_others_alone(cuda, dtype, H, T):
+    """Tokens of zeros (scale 0) and tokens far below zero in one sequence: the codes of the other one are those of its own
+    parameters, whichever groups share a wavefront."""
+    for is_k in (True, False):
+        x = torch.randn(2, H, T, 128, generator=torch.Generator(device=cuda).manual_seed(H + T), device=cuda).to(dtype)
+        x[0, :, T // 2 + 3:] = 0
+        x[0, :, 2:T // 2:3] -= 100
+        enc, dec = (ops.k_quant_encode, ops.k_decode) if is_k else (ops.v_quant_encode, ops.v_decode)
+        e = enc(x, 0.1, want_size=False)
+        codes = torch.zeros(T, 2 * H * 128, dtype=torch.uint8, device=cuda)
+        dec(e["stream"], e["info"], codes, bits=4)
+        c, z, s = oq.quant_ints(x[1:].cpu(), 64, 0.1)
+        assert torch.equal(codes[:, H * 128:].cpu(), oq.code_matrix(c)), "K" if is_k else "V"
