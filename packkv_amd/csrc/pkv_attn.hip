@@ -512,16 +512,18 @@ __global__ void __launch_bounds__(256) attn_window_kernel(const AttnParams p) {
 // ---- merge of a head's partials by the last of its `arrivals` workgroups to get here (async-copy kernel) ----
 // Saves the launch of the merge kernel, its run and the gap in front of it.  The price is three trips past the L2s -- a
 // workgroup's stores, its count, the last one's read of all partials -- and that the counts on one address retire one
-// after the other.  merge_pays says where the price is lower.  4-bit fp16 steps, us per step in a graph of 40 (and launched
-// one by one), with the merge launch -> merged here; `pairs` = sequences x KV heads:
-//   several tiles a workgroup, 4 to 8 workgroups a head: always.  Groups of 4: 128 pairs x 256 tiles 112.5 -> 111.2, x 32
-//     26.3 -> 25.3 (25.4 -> 24.5), 256 x 32 39.7 -> 38.2 (39.0 -> 37.6); groups of 8: 128 x 16 24.9 -> 24.4, 256 x 64 87.4 -> 86.1
+// after the other.  merge_pays says where the price is lower.  4-bit fp16 steps, us per step in a graph of 40 (launched
+// one by one the host takes about 12.7 us for two launches and 10 for one, so that there every step below that gains),
+// with the merge launch -> merged here; `pairs` = sequences x KV heads:
+//   several tiles a workgroup, 4 to 8 workgroups a head: always.  Groups of 4: 128 pairs x 256 tiles 116.0 -> 114.7, x 32
+//     24.7 -> 23.8, 256 x 32 38.6 -> 37.1; groups of 8: 128 x 16 22.9 -> 22.5, 256 x 64 86.4 -> 84.8
 //   one tile each, when all workgroups of a head arrive at once and nothing hides the trips: groups of 8 never (two heads a
-//     wavefront one after the other: 8 pairs x 6 tiles 12.2 -> 12.9, 128 x 2 12.8 -> 13.2); else up to 14 pairs (14 x 8 10.2 ->
-//     10.5 (10.7 -> 10.5), 8 x 4 9.9 -> 9.7 (10.5 -> 10.0)) and from 72 on (72 x 8 12.7 -> 12.7 (13.0 -> 12.6), 128 x 4 11.5 -> 11.3);
-//     in between up to four workgroups (32 x 4 10.0 -> 10.2 (10.7 -> 10.5), but 32 x 8 10.2 -> 10.9 (10.7 -> 11.2), 64 x 8 11.2 -> 12.2
-//     (11.8 -> 12.3)), with groups of 4 and more than 32 pairs three (64 x 3 10.2 -> 10.5 (10.6 -> 10.6), x 4 10.2 -> 10.7 (10.7 -> 10.8)).
-//   32 workgroups a head (32 heads x 4096 tokens) 15.5 -> 16.5, 24 (3 x 8 x 11008 + 137) 25.2 -> 27.2: hence at most eight.
+//     wavefront one after the other: 8 pairs x 6 tiles 10.8 -> 11.5, 128 x 2 11.2 -> 11.8); else up to 14 pairs (14 x 8 9.0 ->
+//     9.3, but 12.6 -> 9.9 one by one; 8 x 4 8.8 -> 8.7) and from 72 on (72 x 8 11.2 -> 11.0, 128 x 4 10.3 -> 9.9; groups of
+//     1: 128 x 8 11.3 -> 10.8); in between up to four workgroups (32 x 4 9.0 -> 9.2, groups of 1 8.3 -> 8.1, but 32 x 8 9.0 ->
+//     10.0, 64 x 8 10.0 -> 11.0), with groups of 4 and more than 32 pairs three (64 x 3 9.0 -> 9.4, x 4 9.1 -> 9.7).
+//   32 workgroups a head (32 heads x 4096 tokens) 15.5 -> 16.5, 24 (3 x 8 x 11008 + 137) 25.2 -> 27.2 (both before a member's
+//     last tile became a step of its own): hence at most eight.
 // Every workgroup has written its partials through to memory (part_store) and waited for that before it counts itself;
 // the reader's loads go past its own L2.  No workgroup waits for another.  Lane = two adjacent channels; a wavefront merges
 // a head of its own when the group has four or more, otherwise the wavefronts share a head's partials and meet in LDS.

@@ -26,6 +26,14 @@ __host__ __device__ inline UnitGeom unit_geom(int W) {
 
 #ifdef __HIPCC__
 
+// Between a wavefront's writes to LDS and its own reads of what other lanes wrote: LDS serves a wavefront's accesses in
+// order, so nothing waits, only the compiler must not move them.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Tile addressing: the uint8 code tile in LDS is row-major [tokens][hid_blk].
 template <bool IS_K>
 __device__ __forceinline__ int tile_index(int unit, int slot, int k, int t, int hid_blk) {
@@ -347,9 +355,7 @@ __device__ __forceinline__ uint32_t unit_encode_wide(const uint8_t *tile, int hi
     if (blk == nullptr) return meta + payload;
     uint16_t *m16 = reinterpret_cast<uint16_t *>(blk + unit_off);
     for (uint32_t i = t; i < meta / 2u; i += 32) m16[i] = 0;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");      // LDS serves a wavefront's accesses in order
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_lds_order();
     uint32_t minsw = 0, lensw = 0;
 #pragma unroll
     for (int i = 0; i < 4; i++) {

@@ -430,15 +430,11 @@ __global__ void __launch_bounds__(512 * NB) pack_long_v_kernel(const uint8_t *__
         uint4 t2 = t1;
         if (j + 2 < NSUB) t2 = *reinterpret_cast<const uint4 *>(rows + (size_t)(16 * (j + 2)) * hidden_dim);
         *reinterpret_cast<uint4 *>(mine + (c >> 2) * kRow + 16 * (c & 3)) = t0;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_order();
         uint32_t e[16];
 #pragma unroll
         for (int k = 0; k < 16; k++) e[k] = mine[k * kRow + c];
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_order();
 #pragma unroll
         for (int k = 0; k < 16; k++) { lo = min(lo, e[k]); hi = max(hi, e[k]); }
 #pragma unroll

@@ -31,12 +31,6 @@ __device__ __forceinline__ uint16_t st16(float x, int dtype) {
 // 1.75 per code pair, minima 0.5, products 1 per code) behind the chain block_info -> block bytes -> parse; with a workgroup
 // of two wavefronts per block the chain had a barrier between its links, the tile was written and read back, and a code
 // cost a conversion.
-__device__ __forceinline__ void wave_lds_order() {         // LDS serves a wavefront's accesses in order
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // f.x .. f.w times the four codes c01 | c23 as unit_fields hands them out, i.e. codes times 2^-24 read from halves: products
 // exact, fp32 sums.  The factors come 2^24 times as large, so that the products are those of the codes: with the sum scaled
 // back instead, products of bf16 factors below 2^-102 fell among the subnormals and lost bits.  Factors of 2^100 and more
@@ -74,7 +68,8 @@ __device__ __forceinline__ bool factors_big(const float (&f)[N]) {
 // channels.  A token's 32 sums of four channels are turned through LDS so that a lane adds sixteen of them, one after the
 // other from the lowest channel on: kq comes out of sums that nearly cancel (q . code against the zero points), so a last
 // bit here that changed with the order of the sum would show there.
-// 65536 tokens x 8 heads at 4 bits: 12.3 us, 15.3 with a workgroup and a code tile per block.
+// 65536 tokens x 8 heads at 4 bits: 15.4 us, 17.4 with a workgroup and a code tile per block (medians of 300 launches in
+// kernel traces, in the reference's sequence of four ops with two inputs in turn; these and those below).
 constexpr int kKqTok = 20, kKqRow = 16 * kKqTok + 16;      // floats from token to token and from row of lanes to row: no bank conflicts
 template <int W>
 __global__ void __launch_bounds__(256) kq_kernel(const uint8_t *__restrict__ stream, uint64_t stream_bytes, const uint32_t *__restrict__ info,
@@ -127,7 +122,7 @@ __global__ void __launch_bounds__(256) kq_kernel(const uint8_t *__restrict__ str
 // lane = channel, so a channel's sum over the tokens stays in its lane.  The weights lie in LDS as floats, [segment][token of
 // the pack][round], one 16-byte broadcast per four codes.  The halves and then the workgroup's blocks are added before the
 // one atomic per channel.
-// 65536 tokens x 8 heads at 3 bits: 10.7 us, 18.6 with a code tile per block and an atomic per channel and block.
+// 65536 tokens x 8 heads at 3 bits: 14.8 us, 21.2 with a code tile per block and an atomic per channel and block.
 constexpr int kWvWaves = 4;
 template <int W>
 __global__ void __launch_bounds__(64 * kWvWaves) wv_kernel(const uint8_t *__restrict__ stream, uint64_t stream_bytes, const uint32_t *__restrict__ info,
@@ -242,7 +237,7 @@ __global__ void __launch_bounds__(256) fused_kq_kernel(uint16_t *__restrict__ ou
 }
 
 // Row sums of w * zero * scale in two steps: grid (ceil(N / 1024), M) partial sums, then one workgroup per row
-// adds the partials and finishes the D outputs.  (65536 columns x 8 rows: 3.5 us for the partial sums; 7.9 with 4096 columns
+// adds the partials and finishes the D outputs.  (65536 columns x 8 rows: 3.4 us for the partial sums; 8.0 with 4096 columns
 // a workgroup, read one value at a time.)
 constexpr int kWvPart = 1024;
 __global__ void __launch_bounds__(256) fused_wv_partial_kernel(const uint16_t *__restrict__ w, const uint16_t *__restrict__ zero,

@@ -1087,9 +1087,7 @@ __global__ void __launch_bounds__(256) k_quant_encode_cells_kernel(
             }
             s_par[16 * wave + lane] = token_par<DT>(sc, zb, false);
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_order();
         __builtin_amdgcn_s_setprio(PKV_EPRIO_PACK);
         uint32_t c01[16], c23[16];
         cell_quant<DT>(xr, my_par, c01, c23);
@@ -1604,9 +1602,7 @@ __global__ void __launch_bounds__(512) v_quant_encode_cells_kernel(
             s_par[32 * wave + lane] = token_par<DT>(sc, zb, false);
         }
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_order();
         __builtin_amdgcn_s_setprio(PKV_EPRIO_PACK);
         uint32_t c01[16], c23[16];
         cell_quant<DT, false>(xr, my_par, c01, c23);          // (the halves of the wavefront hold different tokens)

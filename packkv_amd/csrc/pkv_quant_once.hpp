@@ -53,12 +53,6 @@ template <int NT> struct OnceLds {
     __attribute__((aligned(16))) TokPar par[NT / 64 * 32];              // [wavefront][token of its rounds]
 };
 
-__device__ __forceinline__ void once_order() {             // LDS serves a wavefront's accesses in order
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // The workgroup's ticket; every thread of it calls.
 template <int NT>
 __device__ __forceinline__ uint32_t once_ticket(OnceLds<NT> &l, ScanState *st) {
@@ -248,7 +242,7 @@ __device__ __forceinline__ void k_encode_once(const OnceSide &a, OnceLds<NT> &l,
     TokPar *par = l.par + 32 * wave;
     const TokPar tp = once_params<DT>(mn, mx, a.rel, (lane & 3) == 0 && wr == 0 && run == 0, a.scale, a.zero, (size_t)b * a.par_stride + tok0 + (lane >> 2));
     if ((lane & 3) == 0) par[lane >> 2] = tp;
-    once_order();
+    wave_lds_order();
     uint32_t c01[16], c23[16];
     cell_quant<DT>(xr, par, c01, c23);
     k_write_once<NT, WIDE>(a, l, gbuf, idx, H, grp * (uint32_t)a.H + (uint32_t)hbase, c01, c23, true);      // block index = group * heads + head
@@ -284,7 +278,7 @@ __device__ __forceinline__ void v_write_once(const OnceSide &a, OnceLds<NT> &l, 
         l.usz[q][un] = (uint16_t)(meta + l.tot[2 * sg][q >> 1][at] + l.tot[2 * sg + 1][q >> 1][at]);
     }
     if (tid < 64) {
-        once_order();
+        wave_lds_order();
         once_sizes(l, a.st, idx, nblk);
     }
     if (j < H) {
@@ -381,7 +375,7 @@ __device__ __forceinline__ void v_encode_once(const OnceSide &a, OnceLds<NT> &l,
         const TokPar tp = once_params<DT>(mn, mx, a.rel, write, a.scale, a.zero, ptok);
         if ((lane & 1) == 0) par[lane >> 1] = tp;
     }
-    once_order();
+    wave_lds_order();
     uint32_t c01[16], c23[16];
     cell_quant<DT, false>(xr, par + 16 * rp, c01, c23);    // (the halves of the wavefront hold different tokens)
     v_write_once<NT, WIDE>(a, l, gbuf, idx, H, grp * (uint32_t)(2 * a.H) + (uint32_t)(2 * hbase), c01, c23, true);      // block index = group * 2 heads + 2 head + half

@@ -63,9 +63,7 @@ __global__ void __launch_bounds__(256) token_median_kernel(const uint8_t *__rest
     }
     uint32_t *h = hist[wave];
     for (int i = lane; i < 256; i += 64) h[i] = 0u;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_lds_order();
     for (int c = lane; c < nchunks; c += 64) {
         const uint4 v = row[c];
         const uint32_t w[4] = {v.x, v.y, v.z, v.w};
@@ -74,9 +72,7 @@ __global__ void __launch_bounds__(256) token_median_kernel(const uint8_t *__rest
 #pragma unroll
             for (int kk = 0; kk < 4; kk++) atomicAdd(&h[(w[i] >> (8 * kk)) & 0xFFu], 1u);
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_lds_order();
     // lane l owns bins 4l..4l+3
     const uint32_t c0 = h[4 * lane], c1 = h[4 * lane + 1], c2 = h[4 * lane + 2], c3 = h[4 * lane + 3];
     const uint32_t mine = c0 + c1 + c2 + c3;
