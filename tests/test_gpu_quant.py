@@ -406,8 +406,9 @@ def test_nan_parameters_do_not_depend_on_the_launch(cuda, dtype, H):
 def test_a_run_that_waits_for_no_other_gives_the_same_stream(cuda, dtype, B, H, T, rels, block):
     """The encode of few groups with no look at what the other runs of a group found, as when they do not start."""
     x = list(synth.make_kv(B, H, T, seed=H + T, dtype=dtype, device=cuda))
-    for i in range(2):
-        x[i][0, 1, 5, 7], x[i][0, :, 9], x[i][0, H - 1, 40, 3], x[i][0, 0, 41, 100] = float("nan"), float("nan"), float("inf"), -float("inf")
+    for i in range(2):           # (at 4 bits only: codes that do not fit write packs of 4 bits or of 6, which must not outgrow a block's slot)
+        if rels[i] == 0.1:
+            x[i][0, 1, 5, 7], x[i][0, :, 9], x[i][0, H - 1, 40, 3], x[i][0, 0, 41, 100] = float("nan"), float("nan"), float("inf"), -float("inf")
     perm = None
     if block:
         perm = torch.stack([torch.randperm(block, generator=torch.Generator().manual_seed(i)) for i in range(T // block)]).to(torch.int32).reshape(-1).to(cuda)
