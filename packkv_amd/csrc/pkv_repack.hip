@@ -660,12 +660,11 @@ greedy_order_sliced_kernel(const uint8_t *__restrict__ k_codes, const uint8_t *_
 }
 
 // ---- the same for rows of up to 2048 channels, K and V together: one workgroup holds a block by itself ----
-// Four channels to a thread, kept as 16-bit lanes (even and odd bytes apart: two registers a token, nothing to unpack at
-// a pick), so that a block is priced by two wavefronts a SIMD instead of one, 3.0 vector instructions a channel instead of
-// 3.7; and with nobody to exchange sums with there is no state, no ticket and no closing launch.  What is left of a step
-// is the chain price -> sums -> winner -> move.
-// 256 blocks of 64 tokens x 2048 channels: 193 us, 223 with eight channels to a thread; x 1024 channels (256 threads) 149 us, 218
-// with half of 256 threads idle.
+// Four channels to a thread, and with nobody to exchange sums with there is no state, no ticket and no closing launch.  What a
+// step consists of is the chain price -> sums -> winner -> move.  Codes of any width are priced as 16-bit lanes (greedy_block_wide:
+// even and odd bytes apart, two registers a token, 3.0 vector instructions a channel and token), codes of four bits by looking
+// them up (greedy_block_narrow).  256 blocks of 64 tokens, a launch: x 2048 channels 182 us wide and 99 narrow, x 1024 channels
+// (256 threads) 142 and 70; 1024 blocks of the latter 342 and 182.
 __device__ __forceinline__ void price4x2(uint32_t ea, uint32_t oa, uint32_t eb, uint32_t ob, const uint32_t (&mn)[2], const uint32_t (&mx)[2],
                                          uint32_t &sum_a, uint32_t &sum_b) {
     const uint32_t v[4] = {ea, eb, oa, ob};
@@ -690,31 +689,27 @@ __device__ __forceinline__ void price4x2(uint32_t ea, uint32_t oa, uint32_t eb, 
 }
 
 template <int THREADS>
-__global__ void __launch_bounds__(THREADS, 2)
-greedy_order_block_kernel(const uint8_t *__restrict__ k_codes, const uint8_t *__restrict__ v_codes, int hidden, int N, int pack_len,
-                          uint32_t *__restrict__ perm) {
+constexpr int greedy_block_words() { return 32 * (THREADS / 32 * 36 + 4) + 128 * 32 + 64 + 128; }
+
+// Codes of any width: `raw` = the thread's four channels of every token, as loaded; `perm` = the block's order.
+template <int THREADS>
+__device__ __forceinline__ void greedy_block_wide(const uint32_t (&raw)[kSlicedTokens], uint32_t *lds, int N, int pack_len, uint32_t *__restrict__ perm) {
     constexpr int kRuns = THREADS / 32, kPartStride = kRuns * 36 + 4, kSeedParts = THREADS / 128;
-    __shared__ __attribute__((aligned(16))) uint32_t s_part[32 * kPartStride];   // picks: [pair of slots][thread], padded
-    __shared__ uint32_t s_seed[128 * 32];            // seeds: [2 * slot + (0: dot, 1: squared norm)][adder]
-    __shared__ uint32_t s_tot[64];
-    __shared__ uint32_t s_key[128];
+    uint32_t *s_part = lds;                          // picks: [pair of slots][thread], padded
+    uint32_t *s_seed = s_part + 32 * kPartStride;    // seeds: [2 * slot + (0: dot, 1: squared norm)][adder]
+    uint32_t *s_tot = s_seed + 128 * 32, *s_key = s_tot + 64;
+    static_assert(32 * kPartStride + 128 * 32 + 64 + 128 == greedy_block_words<THREADS>(), "LDS");
     const int tid = threadIdx.x, lane = tid & 63;
-    const int ch = tid * 4;
-    const uint8_t *col = ch < hidden ? k_codes + ch : v_codes + (ch - hidden);
-    const bool have = ch < 2 * hidden;
     const int adder = (tid >> 2) & 31;               // the LDS word that takes the sums of the thread's four lanes
     const bool quad_first = (tid & 3) == 0;
     const int part_word = (tid >> 5) * 36 + (tid & 31), part_read = (tid / kRuns) * kPartStride + (tid % kRuns) * 36;
-    const size_t row0 = (size_t)blockIdx.x * N;
     u32x32 ev[2], ov[2];
 #define xe(t) ev[(t) >> 5][(t) & 31]
 #define xo(t) ov[(t) >> 5][(t) & 31]
 #pragma unroll
     for (int t = 0; t < kSlicedTokens; t++) {
-        uint32_t v = 0u;
-        if (t < N && have) v = *reinterpret_cast<const uint32_t *>(col + (row0 + t) * (size_t)hidden);
-        xe(t) = bytes_even(v);
-        xo(t) = bytes_odd(v);
+        xe(t) = bytes_even(raw[t]);
+        xo(t) = bytes_odd(raw[t]);
     }
     uint32_t orig = (uint32_t)lane;                  // the token in slot `lane`
     int n_alive = N, picked = 0;
@@ -835,7 +830,7 @@ greedy_order_block_kernel(const uint8_t *__restrict__ k_codes, const uint8_t *__
         ov[0][si] = sel < 32 ? l1 : sa1;
         ev[1][si] = sel < 32 ? sb0 : l0;
         ov[1][si] = sel < 32 ? sb1 : l1;
-        if (tid == 0) perm[row0 + picked] = tok;
+        if (tid == 0) perm[picked] = tok;
         picked++;
         n_alive--;
         mn[0] = seed ? w0 : pk_min_u16(mn[0], w0);
@@ -845,6 +840,254 @@ greedy_order_block_kernel(const uint8_t *__restrict__ k_codes, const uint8_t *__
     }
 #undef xe
 #undef xo
+}
+
+// Codes of at most four bits, where every one of a block is below 16.  A channel's four codes of four tokens lie in one register,
+// and what a code costs -- bit_length of the pack's range once it has joined -- is looked up there: a channel's table of 16
+// bytes (one of 136 for its minimum and maximum so far, read from LDS after every pick) serves four tokens with two byte
+// permutes, one vector instruction a token and channel against 3.0.  A code c >= 8 is kept as 0x80 | (c - 8): as a selector
+// that is out of the lower half's range, and 0xFF comes out; with its top bit flipped it selects from the upper half, and the
+// codes below 8 are out of range.  So each lookup finds one cost and one 0xFF, which is a constant -1 of the whole register,
+// carries included.
+__device__ __forceinline__ uint32_t code_selectors(uint32_t x) { return (x & 0x07070707u) | ((x & 0x08080808u) << 4); }
+__device__ __forceinline__ uint32_t selector_codes(uint32_t s) { return (s & 0x07070707u) | ((s >> 4) & 0x08080808u); }
+// Bytes [row][column] of four registers the other way round.
+__device__ __forceinline__ void transpose4(const uint32_t a0, const uint32_t a1, const uint32_t a2, const uint32_t a3, uint32_t (&x)[4]) {
+    const uint32_t l01 = __builtin_amdgcn_perm(a1, a0, 0x05010400u), h01 = __builtin_amdgcn_perm(a1, a0, 0x07030602u);
+    const uint32_t l23 = __builtin_amdgcn_perm(a3, a2, 0x05010400u), h23 = __builtin_amdgcn_perm(a3, a2, 0x07030602u);
+    x[0] = __builtin_amdgcn_perm(l23, l01, 0x05040100u);
+    x[1] = __builtin_amdgcn_perm(l23, l01, 0x07060302u);
+    x[2] = __builtin_amdgcn_perm(h23, h01, 0x05040100u);
+    x[3] = __builtin_amdgcn_perm(h23, h01, 0x07060302u);
+}
+// Half of a reduction that shares its results out: lanes l and l ^ 32 (16, or by a move within a row) each give away one of two values
+// and keep the sum of the other.  a's sum ends up where the lane's bit is clear (`upper` false), b's where it is set.
+__device__ __forceinline__ uint32_t halve32(uint32_t a, uint32_t b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    return (uint32_t)r[0] + (uint32_t)r[1];
+}
+__device__ __forceinline__ uint32_t halve16(uint32_t a, uint32_t b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    return (uint32_t)r[0] + (uint32_t)r[1];
+}
+template <int CTRL>
+__device__ __forceinline__ uint32_t halve_row(uint32_t a, uint32_t b, bool upper) {
+    return (upper ? b : a) + lane_move<CTRL, 0xF, true>(0u, upper ? a : b);
+}
+constexpr int kRor8 = 0x128, kHalfMirror = 0x141, kXor2 = 0x4E, kXor1 = 0xB1;     // lanes l ^ 8, l ^ 7, l ^ 2, l ^ 1
+
+// The better of this lane's vector and of the one a move brings (none: its own again): larger dot^2 / norm, then lower tag.
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ void best_cosine(uint32_t &dot, uint32_t &norm, uint32_t &tag) {
+    const uint32_t d = lane_move<CTRL, ROW_MASK, false>(dot, dot), n = lane_move<CTRL, ROW_MASK, false>(norm, norm),
+                   t = lane_move<CTRL, ROW_MASK, false>(tag, tag);
+    const unsigned long long theirs = (unsigned long long)d * d * norm, own = (unsigned long long)dot * dot * n;
+    const bool take = theirs > own || (theirs == own && t < tag);
+    dot = take ? d : dot;
+    norm = take ? n : norm;
+    tag = take ? t : tag;
+}
+
+typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
+
+// One barrier a step: a wavefront adds its channels up by itself -- 64 tokens in sixteen registers of byte sums, halved six
+// times -- and leaves a sum per token; behind the barrier every wavefront adds the wavefronts' sums of all tokens (lane = token
+// slot) and finds the winner.  The sums of two steps in turn lie in two buffers.  About 1.5 us a step of 2048 channels, half of it
+// vector instructions of two wavefronts a SIMD, the rest the latency of that chain; tables read only where a range has changed
+// were slower (104 us a launch against 98), cosines compared in 128 bits by shuffles 108.
+template <int THREADS>
+__device__ __forceinline__ void greedy_block_narrow(const uint32_t (&raw)[kSlicedTokens], uint32_t *lds, int N, int pack_len, uint32_t *__restrict__ perm) {
+    constexpr int kWaves = THREADS / 64;
+    static_assert(kWaves == 4 || kWaves == 8, "a lane reads the wavefronts' sums 16 bytes at a time");
+    uint4 *table = reinterpret_cast<uint4 *>(lds);             // [minimum][maximum]: the cost of every code
+    uint32_t *sums = lds + 256 * 4;                            // [2][64 tokens or 32 pairs][wavefront]
+    static_assert(256 * 4 + 2 * 64 * kWaves <= greedy_block_words<THREADS>(), "LDS");
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool bit1 = lane & 2, bit2 = lane & 4, bit3 = lane & 8;
+    if (tid < 256) {
+        const int lo = tid >> 4, hi = max(tid & 15, lo);
+        uint32_t w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int v = 0; v < 16; v++) w[v >> 2] |= (32u - (uint32_t)__clz(max(hi, v) - min(lo, v))) << (8 * (v & 3));
+        table[tid] = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+    u32x16 x[4];                                               // x[c][q]: channel c of the tokens in slots 4 q .. 4 q + 3
+#pragma unroll
+    for (int q = 0; q < kSlicedTokens / 4; q++) {
+        uint32_t by_channel[4];
+        transpose4(raw[4 * q], raw[4 * q + 1], raw[4 * q + 2], raw[4 * q + 3], by_channel);
+#pragma unroll
+        for (int c = 0; c < 4; c++) x[c][q] = code_selectors(by_channel[c]);
+    }
+    __syncthreads();
+    // where a lane leaves its wavefront's sums and which it reads (lane = slot): see the halvings below
+    const int pick_quad = (lane >> 5) | ((lane >> 3) & 2) | ((lane >> 1) & 4) | ((lane << 2) & 8);
+    const int pick_word = (2 * pick_quad + ((lane >> 2) & 1)) * kWaves + wave;
+    const int seed_word = (int)(__brev((uint32_t)lane) >> 26) * kWaves + wave;
+    const int pick_read = (2 * (lane >> 2) + (lane & 1)) * kWaves, pick_half = (lane & 2) << 3;
+    uint32_t orig = (uint32_t)lane, order = 0u;                // the token in slot `lane`; the token picked as number `lane`
+    int n_alive = N, in_pack = 0;
+    uint32_t mn[2], mx[2];                                     // ranges of channels (0, 2) and (1, 3), as 16-bit lanes
+    uint32_t cost[4][4];                                       // [channel]: its table
+    for (int step = 0; step < N; step++) {
+        const bool seed = in_pack == 0;
+        in_pack = in_pack + 1 == pack_len ? 0 : in_pack + 1;
+        uint32_t *buf = sums + (step & 1) * 64 * kWaves;
+        int sel;
+        if (seed) {
+            // ---- seed: rounded mean of the remaining tokens, then the best cosine ----
+            uint32_t sum[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int q = 0; q < kSlicedTokens / 4; q++) {
+                if (4 * q < n_alive) {
+                    const uint32_t live = n_alive - 4 * q >= 4 ? 0x01010101u : 0x01010101u >> (8 * (4 * q + 4 - n_alive));
+#pragma unroll
+                    for (int c = 0; c < 4; c++) sum[c] = __builtin_amdgcn_udot4(selector_codes(x[c][q]), live, sum[c], false);
+                }
+            }
+            const float na = (float)n_alive;                   // mean(dim=1).round(): fp32 quotient, round half to even
+            const uint32_t mean = (uint32_t)rintf((float)sum[0] / na) | ((uint32_t)rintf((float)sum[1] / na) << 8) |
+                                  ((uint32_t)rintf((float)sum[2] / na) << 16) | ((uint32_t)rintf((float)sum[3] / na) << 24);
+            // dot product and squared norm as 16-bit lanes: at most 4 x 15 x 15 a lane, 57600 a wavefront
+            uint32_t g8[8];
+#pragma unroll
+            for (int g = 0; g < 8; g++) {
+                g8[g] = 0u;
+                if (8 * g < n_alive) {
+                    uint32_t v[8];
+#pragma unroll
+                    for (int q = 0; q < 2; q++) {
+                        uint32_t by_token[4];
+                        transpose4(selector_codes(x[0][2 * g + q]), selector_codes(x[1][2 * g + q]), selector_codes(x[2][2 * g + q]),
+                                   selector_codes(x[3][2 * g + q]), by_token);
+#pragma unroll
+                        for (int t = 0; t < 4; t++)
+                            v[4 * q + t] = __builtin_amdgcn_udot4(by_token[t], mean, 0u, false) | (__builtin_amdgcn_udot4(by_token[t], by_token[t], 0u, false) << 16);
+                    }
+                    const uint32_t a = halve16(halve32(v[0], v[1]), halve32(v[2], v[3])), b = halve16(halve32(v[4], v[5]), halve32(v[6], v[7]));
+                    g8[g] = halve_row<kRor8>(a, b, bit3);
+                }
+            }
+            uint32_t g4[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) g4[i] = halve_row<kHalfMirror>(g8[2 * i], g8[2 * i + 1], bit2);
+            const uint32_t g2a = halve_row<kXor2>(g4[0], g4[1], bit1), g2b = halve_row<kXor2>(g4[2], g4[3], bit1);
+            buf[seed_word] = halve_row<kXor1>(g2a, g2b, lane & 1);     // slot: the lane's number with its bits in reverse
+            __syncthreads();
+            // dot^2 / norm by cross products: dot and norm stay below 2^19 (2048 channels), so they fit 64 bits.  A zero vector has
+            // cosine 0; slots that are empty as well, and lose every tie.
+            uint32_t dot = 0u, norm = 0u, tag = 0x8000u | (uint32_t)lane;
+            if (lane < n_alive) {
+#pragma unroll
+                for (int i = 0; i < kWaves; i += 4) {
+                    const uint4 w = *reinterpret_cast<const uint4 *>(buf + lane * kWaves + i);
+                    dot += (w.x & 0xFFFFu) + (w.y & 0xFFFFu) + (w.z & 0xFFFFu) + (w.w & 0xFFFFu);
+                    norm += (w.x >> 16) + (w.y >> 16) + (w.z >> 16) + (w.w >> 16);
+                }
+                tag = (orig << 8) | (uint32_t)lane;            // equal cosines: the earlier token
+            }
+            norm = max(norm, 1u);
+            best_cosine<0x111, 0xF>(dot, norm, tag);
+            best_cosine<0x112, 0xF>(dot, norm, tag);
+            best_cosine<0x114, 0xF>(dot, norm, tag);
+            best_cosine<0x118, 0xF>(dot, norm, tag);
+            best_cosine<0x142, 0xA>(dot, norm, tag);
+            best_cosine<0x143, 0xC>(dot, norm, tag);
+            sel = __builtin_amdgcn_readlane((int)tag, 63) & 0xFF;
+        } else {
+            // ---- the pack's other tokens: fewest bits after the pick ----
+            uint32_t h32[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                h32[i] = 0u;
+                if (8 * i < n_alive) {
+                    // (slots past the last one are priced as well: bounded sums nobody reads)
+                    uint32_t s[2];
+#pragma unroll
+                    for (int q = 0; q < 2; q++) {
+                        s[q] = 4u;                             // four channels' 0xFFs
+#pragma unroll
+                        for (int c = 0; c < 4; c++) {
+                            const uint32_t at = x[c][2 * i + q];
+                            s[q] += __builtin_amdgcn_perm(cost[c][1], cost[c][0], at) + __builtin_amdgcn_perm(cost[c][3], cost[c][2], at ^ 0x80808080u);
+                        }
+                    }
+                    h32[i] = halve32(s[0], s[1]);
+                }
+            }
+            // bytes: 16 a lane at most, 32, 64 and 128 after these halvings, then 16-bit lanes
+            uint32_t h16[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) h16[j] = halve16(h32[2 * j], h32[2 * j + 1]);
+            const uint32_t za = halve_row<kRor8>(h16[0], h16[1], bit3), zb = halve_row<kRor8>(h16[2], h16[3], bit3);
+            const uint32_t wa = halve_row<kHalfMirror>(bytes_even(za), bytes_odd(za), bit2), wb = halve_row<kHalfMirror>(bytes_even(zb), bytes_odd(zb), bit2);
+            uint32_t u = halve_row<kXor2>(wa, wb, bit1);
+            u += lane_move<kXor1, 0xF, true>(0u, u);
+            if ((lane & 1) == 0) buf[pick_word] = u;           // slots 4 quad + (lane bit 2) and, in the upper half, + 2
+            __syncthreads();
+            uint32_t a = 0u;
+#pragma unroll
+            for (int i = 0; i < kWaves; i += 4) {
+                const uint4 w = *reinterpret_cast<const uint4 *>(buf + pick_read + i);
+                a += w.x + w.y + w.z + w.w;
+            }
+            // (cost, token) in one word: the minimum is the first cheapest token
+            const uint32_t key = lane < n_alive ? (((a >> pick_half) & 0xFFFFu) << 8) | orig : 0xFFFFFFFFu;
+            const uint32_t best = wave_min_u32(key);
+            sel = (int)__builtin_ctzll(__ballot(key == best));
+        }
+        // the winner in slot `sel` leaves: its codes widen the pack's ranges and the last slot moves into `sel`
+        const int last = n_alive - 1;
+        const uint32_t tok = (uint32_t)__builtin_amdgcn_readlane((int)orig, sel);
+        const uint32_t moved = (uint32_t)__builtin_amdgcn_readlane((int)orig, last);
+        if (lane == sel) orig = moved;
+        if (lane == step) order = tok;
+        const int lq = last >> 2, sq = sel >> 2;
+        const uint32_t sb = (uint32_t)sel & 3u, keep = ~(0xFFu << (8 * sb));
+        const uint32_t take = (0x07060504u & keep) | (((uint32_t)last & 3u) << (8 * sb)), pair = sb | ((4u + sb) << 16) | 0x0C000C00u;
+        uint32_t w[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const uint32_t l = x[c][lq];
+            w[c] = x[c][sq];
+            x[c][sq] = __builtin_amdgcn_perm(w[c], l, take);
+        }
+        n_alive--;
+        const uint32_t we = selector_codes(__builtin_amdgcn_perm(w[2], w[0], pair));
+        const uint32_t wo = selector_codes(__builtin_amdgcn_perm(w[3], w[1], pair));
+        mn[0] = seed ? we : pk_min_u16(mn[0], we);
+        mx[0] = seed ? we : pk_max_u16(mx[0], we);
+        mn[1] = seed ? wo : pk_min_u16(mn[1], wo);
+        mx[1] = seed ? wo : pk_max_u16(mx[1], wo);
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const uint32_t at = (mn[c & 1] << 8) | (mx[c & 1] << 4);      // bytes into the table, a 16-bit lane a channel
+            const uint4 t = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint8_t *>(table) + ((at >> (c >> 1) * 16) & 0xFF0u));
+            cost[c][0] = t.x; cost[c][1] = t.y; cost[c][2] = t.z; cost[c][3] = t.w;
+        }
+    }
+    if (wave == 0 && lane < N) perm[lane] = order;
+}
+
+template <int THREADS>
+__global__ void __launch_bounds__(THREADS, 2)
+greedy_order_block_kernel(const uint8_t *__restrict__ k_codes, const uint8_t *__restrict__ v_codes, int hidden, int N, int pack_len,
+                          uint32_t *__restrict__ perm) {
+    __shared__ __attribute__((aligned(16))) uint32_t lds[greedy_block_words<THREADS>()];
+    const int ch = (int)threadIdx.x * 4;
+    const uint8_t *col = ch < hidden ? k_codes + ch : v_codes + (ch - hidden);
+    const bool have = ch < 2 * hidden;
+    const size_t row0 = (size_t)blockIdx.x * N;
+    uint32_t raw[kSlicedTokens], any = 0u;
+#pragma unroll
+    for (int t = 0; t < kSlicedTokens; t++) {
+        raw[t] = 0u;
+        if (t < N && have) raw[t] = *reinterpret_cast<const uint32_t *>(col + (row0 + t) * (size_t)hidden);
+    }
+#pragma unroll
+    for (int t = 0; t < kSlicedTokens; t++) any |= raw[t];
+    if (__syncthreads_or((any & 0xF0F0F0F0u) != 0u)) greedy_block_wide<THREADS>(raw, lds, N, pack_len, perm + row0);
+    else greedy_block_narrow<THREADS>(raw, lds, N, pack_len, perm + row0);
 }
 
 // ---- out row r = in row perm[r], for K and V at once: grid (ctx_len), 256 threads ----

@@ -401,6 +401,23 @@ def test_greedy_order_with_a_block_to_a_workgroup(cuda, hid, T, bs, pack, top):
     assert (perm.cpu().numpy().reshape(-1, bs) == order).all()
 
 
+@pytest.mark.parametrize("hid,bs,pack", [(1024, 64, 16), (512, 64, 32), (1024, 36, 12), (272, 64, 16), (16, 4, 2)])
+def test_greedy_order_at_the_four_bit_edge(cuda, hid, bs, pack):
+    """Blocks whose codes all lie below 16 look their costs up (four tokens to a register), others compute them: codes at the
+    ends of the range (the largest sums a wavefront can meet), equal tokens, zero tokens, one code of 16 in one of the blocks."""
+    g = torch.Generator().manual_seed(hid + bs)
+    ends = lambda: torch.randint(0, 2, (5 * bs, hid), dtype=torch.uint8, generator=g) * 15
+    kc, vc = ends(), ends()
+    kc[bs:2 * bs], vc[bs:2 * bs] = 15, 15
+    kc[bs + 1], vc[bs + 1] = 0, 0
+    kc[2 * bs:3 * bs], vc[2 * bs:3 * bs] = 0, 0
+    kc[3 * bs:], vc[3 * bs:] = (torch.randint(0, 16, (2 * bs, hid), dtype=torch.uint8, generator=g) for _ in range(2))
+    vc[5 * bs - 1, hid - 1] = 16
+    _, order = orp.greedy_repacking(orp.blocks_from_code_matrices(kc.numpy(), vc.numpy(), bs), pack)
+    perm = ops.greedy_order(kc.to(cuda), vc.to(cuda), pack, bs)
+    assert (perm.cpu().numpy().reshape(-1, bs) == order).all()
+
+
 def test_greedy_order_does_not_depend_on_the_number_of_blocks(cuda):
     """256 blocks of 2048 channels take a workgroup each, 257 the workgroups that walk several blocks."""
     g = torch.Generator(device=cuda)
