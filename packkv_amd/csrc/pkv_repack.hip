@@ -324,6 +324,10 @@ __global__ void __launch_bounds__(kGreedyThreads) greedy_order_kernel(const uint
 // constant bias of the exponent (5 per channel) is common to all tokens.  A step of a group of eight wide
 // workgroups takes ~6.5 us on an MI355X: 3.8 us of pricing at the full rate of the vector ALUs, the rest the sums,
 // the exchange, the winner and the slot move, which nothing overlaps.
+// A member whose slice of a block holds no code above 15 looks its costs up instead (greedy_narrow, eight channels to a thread; its
+// sums lack the bias, which is common to all tokens and so may differ from member to member).  us a launch, codes of 5 bits and
+// of 4: 128 blocks x 4096 channels 306 and 159, 512 x 2048 (256 threads) 319 and 170, 32 x 8192 365 and 223 (two members), 128 x 32768 1590
+// and 960 (eight).  Before there was a second path both took the time of the first.
 constexpr int kSlicedThreadsWide = 512;                 // one workgroup per CU, two wavefronts per SIMD: rows of two or more slices
 constexpr int kSlicedThreadsNarrow = 256;               // two workgroups per CU: rows of up to 2048 channels in more than 256 blocks
                                                         // (fewer blocks, and rows of up to 1024: greedy_order_block_kernel)
@@ -426,6 +430,375 @@ __device__ __forceinline__ void gather_words(const uint64_t *words, uint32_t idx
 // index (register-indexed moves); every other access is by constant.
 typedef uint32_t u32x32 __attribute__((ext_vector_type(32)));
 
+template <int THREADS, int CHANNELS>
+constexpr int greedy_narrow_words() { return 256 * 4 + 2 * 64 * (THREADS / 64) * (CHANNELS / 4); }
+
+// Codes of at most four bits, where every one of a block is below 16.  A channel's four codes of four tokens lie in one register,
+// and what a code costs -- bit_length of the pack's range once it has joined -- is looked up there: a channel's table of 16
+// bytes (one of 136 for its minimum and maximum so far, read from LDS after every pick) serves four tokens with two byte
+// permutes, one vector instruction a token and channel against 3.0.  A code c >= 8 is kept as 0x80 | (c - 8): as a selector
+// that is out of the lower half's range, and 0xFF comes out; with its top bit flipped it selects from the upper half, and the
+// codes below 8 are out of range.  So each lookup finds one cost and one 0xFF, which is a constant -1 of the whole register,
+// carries included.
+__device__ __forceinline__ uint32_t code_selectors(uint32_t x) { return (x & 0x07070707u) | ((x & 0x08080808u) << 4); }
+__device__ __forceinline__ uint32_t selector_codes(uint32_t s, uint32_t low = 0x07070707u, uint32_t shift = 4u) { return (s & low) | ((s >> shift) & 0x08080808u); }
+// Bytes [row][column] of four registers the other way round.
+__device__ __forceinline__ void transpose4(const uint32_t a0, const uint32_t a1, const uint32_t a2, const uint32_t a3, uint32_t (&x)[4]) {
+    const uint32_t l01 = __builtin_amdgcn_perm(a1, a0, 0x05010400u), h01 = __builtin_amdgcn_perm(a1, a0, 0x07030602u);
+    const uint32_t l23 = __builtin_amdgcn_perm(a3, a2, 0x05010400u), h23 = __builtin_amdgcn_perm(a3, a2, 0x07030602u);
+    x[0] = __builtin_amdgcn_perm(l23, l01, 0x05040100u);
+    x[1] = __builtin_amdgcn_perm(l23, l01, 0x07060302u);
+    x[2] = __builtin_amdgcn_perm(h23, h01, 0x05040100u);
+    x[3] = __builtin_amdgcn_perm(h23, h01, 0x07060302u);
+}
+// Half of a reduction that shares its results out: lanes l and l ^ 32 (16, or by a move within a row) each give away one of two values
+// and keep the sum of the other.  a's sum ends up where the lane's bit is clear (`upper` false), b's where it is set.
+__device__ __forceinline__ uint32_t halve32(uint32_t a, uint32_t b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    return (uint32_t)r[0] + (uint32_t)r[1];
+}
+__device__ __forceinline__ uint32_t halve16(uint32_t a, uint32_t b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    return (uint32_t)r[0] + (uint32_t)r[1];
+}
+template <int CTRL>
+__device__ __forceinline__ uint32_t halve_row(uint32_t a, uint32_t b, bool upper) {
+    return (upper ? b : a) + lane_move<CTRL, 0xF, true>(0u, upper ? a : b);
+}
+constexpr int kRor8 = 0x128, kHalfMirror = 0x141, kXor2 = 0x4E, kXor1 = 0xB1;     // lanes l ^ 8, l ^ 7, l ^ 2, l ^ 1
+
+// The better of this lane's vector and of the one a move brings (none: its own again): larger dot^2 / norm, by cross products,
+// then lower tag.  32 bits: dot and norm stay below 2^19 (2048 channels), the products below 2^57.
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ void best_cosine(uint32_t &dot, uint32_t &norm, uint32_t &tag) {
+    const uint32_t d = lane_move<CTRL, ROW_MASK, false>(dot, dot), n = lane_move<CTRL, ROW_MASK, false>(norm, norm),
+                   t = lane_move<CTRL, ROW_MASK, false>(tag, tag);
+    const unsigned long long theirs = (unsigned long long)d * d * norm, own = (unsigned long long)dot * dot * n;
+    const bool take = theirs > own || (theirs == own && t < tag);
+    dot = take ? d : dot;
+    norm = take ? n : norm;
+    tag = take ? t : tag;
+}
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ unsigned long long lane_move64(unsigned long long x) {
+    const uint32_t lo = lane_move<CTRL, ROW_MASK, false>((uint32_t)x, (uint32_t)x),
+                   hi = lane_move<CTRL, ROW_MASK, false>((uint32_t)(x >> 32), (uint32_t)(x >> 32));
+    return ((unsigned long long)hi << 32) | lo;
+}
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ void best_cosine(unsigned long long &dot, unsigned long long &norm, uint32_t &tag) {
+    const unsigned long long d = lane_move64<CTRL, ROW_MASK>(dot), n = lane_move64<CTRL, ROW_MASK>(norm);
+    const uint32_t t = lane_move<CTRL, ROW_MASK, false>(tag, tag);
+    const unsigned __int128 theirs = (unsigned __int128)(d * d) * norm, own = (unsigned __int128)(dot * dot) * n;
+    const bool take = theirs > own || (theirs == own && t < tag);
+    dot = take ? d : dot;
+    norm = take ? n : norm;
+    tag = take ? t : tag;
+}
+
+typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
+
+// CHANNELS adjacent channels to a thread, 4 or 8; `rows(q, v)`: v[i][t] = dword i of token 4 q + t's, called in order.  One barrier a step: a wavefront adds its
+// channels up by itself -- 64 tokens in sixteen registers of byte sums, halved six times -- and leaves a sum per token; behind
+// the barrier every wavefront adds the wavefronts' sums of all tokens (lane = token slot) and finds the winner.  The sums of two
+// steps in turn lie in two buffers.  Where several workgroups hold a block the sums go through GROUP, with a second barrier.  About 1.5 us a step of 2048 channels, half of it
+// vector instructions of two wavefronts a SIMD, the rest the latency of that chain; tables read only where a range has changed
+// were slower (104 us a launch against 98), cosines compared in 128 bits by shuffles 108.
+struct NoGroup {
+    static constexpr bool kMany = false;
+};
+template <int THREADS, int CHANNELS, typename ROWS, typename GROUP>
+__device__ __forceinline__ void greedy_narrow(ROWS &&rows, uint32_t *lds, int N, int pack_len, GROUP &&group, uint32_t *__restrict__ perm) {
+    constexpr int kWaves = THREADS / 64, kDwords = CHANNELS / 4;
+    typedef typename std::remove_reference<GROUP>::type Group;
+    static_assert(CHANNELS == 4 || CHANNELS == 8, "byte sums of a lane's channels");
+    static_assert(kWaves == 4 || kWaves == 8, "a lane reads the wavefronts' sums 16 bytes at a time");
+    uint4 *table = reinterpret_cast<uint4 *>(lds);             // [minimum][maximum]: the cost of every code
+    uint32_t *sums = lds + 256 * 4;                            // [2][64 tokens or 32 pairs][wavefront][kDwords]
+    static_assert(greedy_narrow_words<THREADS, CHANNELS>() == 256 * 4 + 2 * 64 * kWaves * kDwords, "LDS");
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool bit1 = lane & 2, bit2 = lane & 4, bit3 = lane & 8;
+    if (tid < 256) {
+        const int lo = tid >> 4, hi = max(tid & 15, lo);
+        uint32_t w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int v = 0; v < 16; v++) w[v >> 2] |= (32u - (uint32_t)__clz(max(hi, v) - min(lo, v))) << (8 * (v & 3));
+        table[tid] = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+    u32x16 x[CHANNELS];                                        // x[c][q]: channel c of the tokens in slots 4 q .. 4 q + 3
+#pragma unroll
+    for (int q = 0; q < kSlicedTokens / 4; q++) {
+        uint32_t v[kDwords][4];
+        rows(q, v);
+#pragma unroll
+        for (int i = 0; i < kDwords; i++) {
+            uint32_t by_channel[4];
+            transpose4(v[i][0], v[i][1], v[i][2], v[i][3], by_channel);
+#pragma unroll
+            for (int c = 0; c < 4; c++) x[4 * i + c][q] = code_selectors(by_channel[c]);
+        }
+    }
+    __syncthreads();
+    // where a lane leaves its wavefront's sums and which it reads (lane = slot): see the halvings below
+    const int pick_quad = (lane >> 5) | ((lane >> 3) & 2) | (kDwords == 1 ? (lane >> 1) & 4 : lane & 4) | ((lane << 2) & 8);
+    const int pick_odd = kDwords == 1 ? (lane >> 2) & 1 : (lane >> 3) & 1, pick_word = (2 * pick_quad + pick_odd) * kWaves + wave;
+    const int seed_word = ((int)(__brev((uint32_t)lane) >> 26) * kWaves + wave) * kDwords;
+    const int pick_read = (2 * (lane >> 2) + (lane & 1)) * kWaves, pick_half = (lane & 2) << 3;
+    uint32_t orig = (uint32_t)lane, order = 0u;                // the token in slot `lane`; the token picked as number `lane`
+    int n_alive = N, in_pack = 0;
+    uint32_t mn[2 * kDwords], mx[2 * kDwords];                 // ranges of channels (0, 2), (1, 3), (4, 6), (5, 7), as 16-bit lanes
+    uint32_t cost[CHANNELS][4];                                // [channel]: its table
+    for (int step = 0; step < N; step++) {
+        const bool seed = in_pack == 0;
+        in_pack = in_pack + 1 == pack_len ? 0 : in_pack + 1;
+        uint32_t *buf = sums + (step & 1) * 64 * kWaves * kDwords;
+        int sel;
+        if (seed) {
+            // ---- seed: rounded mean of the remaining tokens, then the best cosine ----
+            uint32_t sum[CHANNELS] = {};
+#pragma unroll
+            for (int q = 0; q < kSlicedTokens / 4; q++) {
+                if (4 * q < n_alive) {
+                    const uint32_t live = n_alive - 4 * q >= 4 ? 0x01010101u : 0x01010101u >> (8 * (4 * q + 4 - n_alive));
+#pragma unroll
+                    for (int c = 0; c < CHANNELS; c++) sum[c] = __builtin_amdgcn_udot4(selector_codes(x[c][q]), live, sum[c], false);
+                }
+            }
+            const float na = (float)n_alive;                   // mean(dim=1).round(): fp32 quotient, round half to even
+            uint32_t mean[kDwords];
+#pragma unroll
+            for (int i = 0; i < kDwords; i++)
+                mean[i] = (uint32_t)rintf((float)sum[4 * i] / na) | ((uint32_t)rintf((float)sum[4 * i + 1] / na) << 8) |
+                          ((uint32_t)rintf((float)sum[4 * i + 2] / na) << 16) | ((uint32_t)rintf((float)sum[4 * i + 3] / na) << 24);
+            // dot product and squared norm as 16-bit lanes: at most 4 x 15 x 15 a lane and four channels, 57600 a wavefront
+            uint32_t g8[8], low = 0x07070707u, shift = 4u;
+            asm volatile("" : "+s"(low), "+s"(shift));         // (the codes anew: those of the mean's sums would be kept in registers)
+#pragma unroll
+            for (int g = 0; g < 8; g++) {
+                g8[g] = 0u;
+                if (8 * g < n_alive) {
+                    uint32_t v[8];
+#pragma unroll
+                    for (int q = 0; q < 2; q++) {
+                        uint32_t dot[4] = {}, norm[4] = {};
+#pragma unroll
+                        for (int i = 0; i < kDwords; i++) {
+                            uint32_t by_token[4];
+                            transpose4(selector_codes(x[4 * i][2 * g + q], low, shift), selector_codes(x[4 * i + 1][2 * g + q], low, shift),
+                                       selector_codes(x[4 * i + 2][2 * g + q], low, shift), selector_codes(x[4 * i + 3][2 * g + q], low, shift), by_token);
+#pragma unroll
+                            for (int t = 0; t < 4; t++) {
+                                dot[t] = __builtin_amdgcn_udot4(by_token[t], mean[i], dot[t], false);
+                                norm[t] = __builtin_amdgcn_udot4(by_token[t], by_token[t], norm[t], false);
+                            }
+                        }
+#pragma unroll
+                        for (int t = 0; t < 4; t++) v[4 * q + t] = dot[t] | (norm[t] << 16);
+                    }
+                    const uint32_t a = halve16(halve32(v[0], v[1]), halve32(v[2], v[3])), b = halve16(halve32(v[4], v[5]), halve32(v[6], v[7]));
+                    g8[g] = halve_row<kRor8>(a, b, bit3);
+                }
+            }
+            uint32_t g4[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) g4[i] = halve_row<kHalfMirror>(g8[2 * i], g8[2 * i + 1], bit2);
+            const uint32_t g2a = halve_row<kXor2>(g4[0], g4[1], bit1), g2b = halve_row<kXor2>(g4[2], g4[3], bit1);
+            // (slot: the lane's number with its bits in reverse)
+            if constexpr (kDwords == 1) {
+                buf[seed_word] = halve_row<kXor1>(g2a, g2b, lane & 1);
+            } else {                                           // half a wavefront's sums fill 16 bits: the last halving in 32
+                const uint32_t own = lane & 1 ? g2b : g2a, got = lane_move<kXor1, 0xF, true>(0u, lane & 1 ? g2a : g2b);
+                *reinterpret_cast<uint2 *>(buf + seed_word) = make_uint2((own & 0xFFFFu) + (got & 0xFFFFu), (own >> 16) + (got >> 16));
+            }
+            __syncthreads();
+            uint32_t dot = 0u, norm = 0u;
+            if (lane < n_alive) {
+#pragma unroll
+                for (int i = 0; i < kWaves * kDwords; i += 4) {
+                    const uint4 w = *reinterpret_cast<const uint4 *>(buf + lane * kWaves * kDwords + i);
+                    if constexpr (kDwords == 1) {
+                        dot += (w.x & 0xFFFFu) + (w.y & 0xFFFFu) + (w.z & 0xFFFFu) + (w.w & 0xFFFFu);
+                        norm += (w.x >> 16) + (w.y >> 16) + (w.z >> 16) + (w.w >> 16);
+                    } else {
+                        dot += w.x + w.z;
+                        norm += w.y + w.w;
+                    }
+                }
+            }
+            // equal cosines: the earlier token.  A zero vector has cosine 0; slots that are empty as well, and lose every tie.
+            uint32_t tag = lane < n_alive ? (orig << 8) | (uint32_t)lane : 0x8000u | (uint32_t)lane;
+            if constexpr (Group::kMany) {
+                unsigned long long all_dot = dot, all_norm = norm;
+                group.seeds(lane, wave, n_alive, all_dot, all_norm);
+                all_norm = all_norm ? all_norm : 1ull;
+                best_cosine<0x111, 0xF>(all_dot, all_norm, tag);
+                best_cosine<0x112, 0xF>(all_dot, all_norm, tag);
+                best_cosine<0x114, 0xF>(all_dot, all_norm, tag);
+                best_cosine<0x118, 0xF>(all_dot, all_norm, tag);
+                best_cosine<0x142, 0xA>(all_dot, all_norm, tag);
+                best_cosine<0x143, 0xC>(all_dot, all_norm, tag);
+            } else {
+                norm = max(norm, 1u);
+                best_cosine<0x111, 0xF>(dot, norm, tag);
+                best_cosine<0x112, 0xF>(dot, norm, tag);
+                best_cosine<0x114, 0xF>(dot, norm, tag);
+                best_cosine<0x118, 0xF>(dot, norm, tag);
+                best_cosine<0x142, 0xA>(dot, norm, tag);
+                best_cosine<0x143, 0xC>(dot, norm, tag);
+            }
+            sel = __builtin_amdgcn_readlane((int)tag, 63) & 0xFF;
+        } else {
+            // ---- the pack's other tokens: fewest bits after the pick ----
+            uint32_t h32[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                h32[i] = 0u;
+                if (8 * i < n_alive) {
+                    // (slots past the last one are priced as well: bounded sums nobody reads)
+                    uint32_t s[2];
+#pragma unroll
+                    for (int q = 0; q < 2; q++) {
+                        s[q] = CHANNELS;                       // the channels' 0xFFs
+#pragma unroll
+                        for (int c = 0; c < CHANNELS; c++) {
+                            const uint32_t at = x[c][2 * i + q];
+                            s[q] += __builtin_amdgcn_perm(cost[c][1], cost[c][0], at) + __builtin_amdgcn_perm(cost[c][3], cost[c][2], at ^ 0x80808080u);
+                        }
+                    }
+                    h32[i] = halve32(s[0], s[1]);
+                }
+            }
+            // bytes of at most 4 CHANNELS a lane, twice as much after each halving up to 128, then 16-bit lanes
+            uint32_t h16[4], wa, wb;
+#pragma unroll
+            for (int j = 0; j < 4; j++) h16[j] = halve16(h32[2 * j], h32[2 * j + 1]);
+            if constexpr (kDwords == 1) {
+                const uint32_t za = halve_row<kRor8>(h16[0], h16[1], bit3), zb = halve_row<kRor8>(h16[2], h16[3], bit3);
+                wa = halve_row<kHalfMirror>(bytes_even(za), bytes_odd(za), bit2);
+                wb = halve_row<kHalfMirror>(bytes_even(zb), bytes_odd(zb), bit2);
+            } else {
+                uint32_t z[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) z[j] = halve_row<kRor8>(bytes_even(h16[j]), bytes_odd(h16[j]), bit3);
+                wa = halve_row<kHalfMirror>(z[0], z[1], bit2);
+                wb = halve_row<kHalfMirror>(z[2], z[3], bit2);
+            }
+            uint32_t u = halve_row<kXor2>(wa, wb, bit1);
+            u += lane_move<kXor1, 0xF, true>(0u, u);
+            if ((lane & 1) == 0) buf[pick_word] = u;           // slots 4 quad + odd and, in the upper half, + 2
+            __syncthreads();
+            uint32_t a = 0u;
+#pragma unroll
+            for (int i = 0; i < kWaves; i += 4) {
+                const uint4 w = *reinterpret_cast<const uint4 *>(buf + pick_read + i);
+                a += w.x + w.y + w.z + w.w;
+            }
+            a = (a >> pick_half) & 0xFFFFu;
+            if constexpr (Group::kMany) group.picks(lane, wave, n_alive, a);
+            // (cost, token) in one word: the minimum is the first cheapest token
+            const uint32_t key = lane < n_alive ? (a << 8) | orig : 0xFFFFFFFFu;
+            const uint32_t best = wave_min_u32(key);
+            sel = (int)__builtin_ctzll(__ballot(key == best));
+        }
+        // the winner in slot `sel` leaves: its codes widen the pack's ranges and the last slot moves into `sel`
+        const int last = n_alive - 1;
+        const uint32_t tok = (uint32_t)__builtin_amdgcn_readlane((int)orig, sel);
+        const uint32_t moved = (uint32_t)__builtin_amdgcn_readlane((int)orig, last);
+        if (lane == sel) orig = moved;
+        if (lane == step) order = tok;
+        const int lq = last >> 2, sq = sel >> 2;
+        const uint32_t sb = (uint32_t)sel & 3u, keep = ~(0xFFu << (8 * sb));
+        const uint32_t take = (0x07060504u & keep) | (((uint32_t)last & 3u) << (8 * sb)), pair = sb | ((4u + sb) << 16) | 0x0C000C00u;
+        uint32_t w[CHANNELS];
+#pragma unroll
+        for (int c = 0; c < CHANNELS; c++) {
+            const uint32_t l = x[c][lq];
+            w[c] = x[c][sq];
+            x[c][sq] = __builtin_amdgcn_perm(w[c], l, take);
+        }
+        n_alive--;
+#pragma unroll
+        for (int i = 0; i < 2 * kDwords; i++) {
+            const int c = 4 * (i >> 1) + (i & 1);
+            const uint32_t codes = selector_codes(__builtin_amdgcn_perm(w[c + 2], w[c], pair));
+            mn[i] = seed ? codes : pk_min_u16(mn[i], codes);
+            mx[i] = seed ? codes : pk_max_u16(mx[i], codes);
+        }
+#pragma unroll
+        for (int c = 0; c < CHANNELS; c++) {
+            const int i = 2 * (c >> 2) + (c & 1);
+            const uint32_t at = (mn[i] << 8) | (mx[i] << 4);              // bytes into the table, a 16-bit lane a channel
+            const uint4 t = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint8_t *>(table) + ((at >> (c & 2) * 8) & 0xFF0u));
+            cost[c][0] = t.x; cost[c][1] = t.y; cost[c][2] = t.z; cost[c][3] = t.w;
+        }
+    }
+    if (perm && wave == 0 && lane < N) perm[lane] = order;
+}
+
+// The sums of a group's members: published and gathered as greedy_order_sliced_kernel's comment says, by members that look costs
+// up and by those that compute them alike.
+template <int THREADS>
+struct SliceGroup {
+    static constexpr bool kMany = true;
+    static constexpr int kRuns = THREADS / 32, kSeedParts = THREADS / 128;
+    uint64_t *xw;
+    uint32_t members, mem, seq;
+    int flip;
+    ScanState *st;
+    uint32_t (*s_tot)[64];                           // [kRuns]
+    unsigned long long (*s_tot64)[128];              // [kSeedParts]
+    __device__ __forceinline__ void publish(uint32_t word, uint32_t value) const {
+        __hip_atomic_store(xw + ((size_t)flip * members + mem) * 128 + word, ((uint64_t)seq << 32) | value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    // value v = tid & 127 of the members q = tid >> 7, q + kSeedParts, ..
+    __device__ __forceinline__ void gather_seeds(int n_alive) {
+        const int v = threadIdx.x & 127, q = threadIdx.x >> 7;
+        unsigned long long a = 0ull;
+        if (v < 2 * n_alive)
+            gather_words(xw + (size_t)flip * members * 128, (uint32_t)v, (uint32_t)q, (uint32_t)kSeedParts, members, seq, st,
+                         [&](uint32_t w) { a += w; });
+        s_tot64[q][v] = a;
+        flip ^= 1;
+    }
+    // pair k = tid & 31 of the members q = tid >> 5, q + kRuns, ..
+    __device__ __forceinline__ void gather_picks(int n_alive) {
+        const int k = threadIdx.x & 31, q = threadIdx.x >> 5;
+        uint32_t a_lo = 0u, a_hi = 0u;
+        if (2 * k < n_alive)
+            gather_words(xw + (size_t)flip * members * 128, (uint32_t)k, (uint32_t)q, (uint32_t)kRuns, members, seq, st,
+                         [&](uint32_t w) { a_lo += w & 0xFFFFu; a_hi += w >> 16; });
+        s_tot[q][2 * k] = a_lo;
+        s_tot[q][2 * k + 1] = a_hi;
+        flip ^= 1;
+    }
+    // this member's sums of the token in slot `lane` -> the group's
+    __device__ __forceinline__ void seeds(int lane, int wave, int n_alive, unsigned long long &dot, unsigned long long &norm) {
+        seq++;
+        if (members == 1) return;
+        if (wave == 0 && lane < n_alive) {
+            publish(2 * lane, (uint32_t)dot);
+            publish(2 * lane + 1, (uint32_t)norm);
+        }
+        gather_seeds(n_alive);
+        __syncthreads();
+        dot = norm = 0ull;
+        if (lane < n_alive) {
+#pragma unroll
+            for (int q = 0; q < kSeedParts; q++) { dot += s_tot64[q][2 * lane]; norm += s_tot64[q][2 * lane + 1]; }
+        }
+    }
+    __device__ __forceinline__ void picks(int lane, int wave, int n_alive, uint32_t &cost) {
+        seq++;
+        if (members == 1) return;
+        const uint32_t next = lane_move<0xB1, 0xF, true>(0u, cost);
+        if (wave == 0 && (lane & 1) == 0 && lane < n_alive) publish(lane >> 1, cost | (next << 16));
+        gather_picks(n_alive);
+        __syncthreads();
+        cost = 0u;
+        for (int q = 0; q < (int)min(members, (uint32_t)kRuns); q++) cost += s_tot[q][lane];
+    }
+};
+
 template <int THREADS>
 __global__ void __launch_bounds__(THREADS, 2)
 greedy_order_sliced_kernel(const uint8_t *__restrict__ k_codes, const uint8_t *__restrict__ v_codes, int hidden, int N,
@@ -446,25 +819,67 @@ greedy_order_sliced_kernel(const uint8_t *__restrict__ k_codes, const uint8_t *_
     uint64_t *xw = st->status + (size_t)grp * 2 * members * 128;      // [buffer][member][128]
     const int D2 = 2 * hidden;
     const int ch = ((int)mem * THREADS + tid) * 8;                    // first of the thread's 8 channels
-    const uint8_t *col = ch < hidden ? k_codes + ch : v_codes + (ch - hidden);
     const bool have = ch < D2;
-    const int adder = (tid >> 2) & 31;               // the LDS word that takes the sums of the thread's four lanes
-    const bool quad_first = (tid & 3) == 0;
-    uint32_t seq = 0;
-    int flip = 0;
-    // a thread's word in a row of s_part and, as a reader, where the 32 words it adds start: rows and runs of 32 are
-    // padded so that the 16-byte reads of a wavefront spread over all banks
-    const int part_word = (tid >> 5) * 36 + (tid & 31), part_read = (tid / kRuns) * kPartStride + (tid % kRuns) * 36;
+    const uint8_t *col = ch < hidden ? k_codes + ch : v_codes + (have ? ch - hidden : 0);
+    const uint32_t channels = have ? ~0u : 0u;
+    SliceGroup<THREADS> group{xw, members, mem, 0u, 0, st, s_tot, s_tot64};
 
     for (uint32_t blk = grp; blk < nblocks; blk += groups) {
         const size_t row0 = (size_t)blk * N;
+        // codes of at most four bits are looked up, by each member as its own slice allows
+        // (the rows are gone through twice, each time with an address that moves on: 64 of them kept would be spilled.  Slots past
+        // the block hold its last row, which is never alive there; threads without channels read some and drop it: no branch)
+        const uint8_t *at;
+        int left;
+        auto from_the_top = [&]() {
+            uint64_t first = row0 * (size_t)hidden;
+            left = N;
+            asm volatile("" : "+s"(first), "+s"(left));
+            at = col + first;
+        };
+        auto next_row = [&]() {
+            uint2 v = *reinterpret_cast<const uint2 *>(at);
+            v.x &= channels;
+            v.y &= channels;
+            left--;
+            at += left > 0 ? hidden : 0;
+            return v;
+        };
+        uint32_t any = 0u;
+        from_the_top();
+#pragma unroll 16
+        for (int t = 0; t < N; t++) {
+            const uint2 v = next_row();
+            any |= v.x | v.y;
+        }
+        from_the_top();
+        if (!__syncthreads_or((any & 0xF0F0F0F0u) != 0u)) {
+            greedy_narrow<THREADS, 8>(
+                [&](int q, uint32_t (&v)[2][4]) {
+#pragma unroll
+                    for (int t = 0; t < 4; t++) {
+                        const uint2 r = next_row();
+                        v[0][t] = r.x;
+                        v[1][t] = r.y;
+                    }
+                    if (q & 1) __builtin_amdgcn_sched_barrier(0);      // (no more than eight rows on their way: there are no registers for all)
+                }, s_part, N, pack_len, group,
+                                      mem == 0 ? perm + row0 : nullptr);
+            continue;
+        }
+        int own = tid;                               // (what follows from it is formed here: kept through the other path it was spilled)
+        asm volatile("" : "+v"(own));
+        const int adder = (own >> 2) & 31;           // the LDS word that takes the sums of the thread's four lanes
+        const bool quad_first = (own & 3) == 0;
+        // a thread's word in a row of s_part and, as a reader, where the 32 words it adds start: rows and runs of 32 are
+        // padded so that the 16-byte reads of a wavefront spread over all banks
+        const int part_word = (own >> 5) * 36 + (own & 31), part_read = (own / kRuns) * kPartStride + (own % kRuns) * 36;
         u32x32 x0v[2], x1v[2];
 #define x0(t) x0v[(t) >> 5][(t) & 31]
 #define x1(t) x1v[(t) >> 5][(t) & 31]
 #pragma unroll
         for (int t = 0; t < kSlicedTokens; t++) {
-            uint2 v = make_uint2(0u, 0u);
-            if (t < N && have) v = *reinterpret_cast<const uint2 *>(col + (row0 + t) * (size_t)hidden);
+            const uint2 v = next_row();
             x0(t) = v.x;
             x1(t) = v.y;
         }
@@ -517,7 +932,7 @@ greedy_order_sliced_kernel(const uint8_t *__restrict__ k_codes, const uint8_t *_
                 }
             }
             __syncthreads();
-            seq++;
+            group.seq++;
             {   // value v: two or four adjacent threads add 16 or 8 adders each
                 const int v = tid / kSeedParts, part = tid % kSeedParts;
                 uint32_t a = 0u;
@@ -526,22 +941,11 @@ greedy_order_sliced_kernel(const uint8_t *__restrict__ k_codes, const uint8_t *_
                 a += lane_move<0xB1, 0xF, false>(0u, a);
                 if (kSeedParts == 4) a += lane_move<0x4E, 0xF, false>(0u, a);
                 if (part == 0 && v < 2 * n_alive) {
-                    if (members > 1)
-                        __hip_atomic_store(xw + ((size_t)flip * members + mem) * 128 + v, ((uint64_t)seq << 32) | a,
-                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    else
-                        s_tot64[0][v] = a;
+                    if (members > 1) group.publish((uint32_t)v, a);
+                    else s_tot64[0][v] = a;
                 }
             }
-            if (members > 1) {
-                const int v = tid & 127, q = tid >> 7;
-                unsigned long long a = 0ull;
-                if (v < 2 * n_alive)
-                    gather_words(xw + (size_t)flip * members * 128, (uint32_t)v, (uint32_t)q, (uint32_t)kSeedParts, members, seq, st,
-                                 [&](uint32_t w) { a += w; });
-                s_tot64[q][v] = a;
-                flip ^= 1;
-            }
+            if (members > 1) group.gather_seeds(n_alive);
             __syncthreads();
             {
                 unsigned long long bd = 0, bn = 0;
@@ -582,7 +986,7 @@ greedy_order_sliced_kernel(const uint8_t *__restrict__ k_codes, const uint8_t *_
                     }
                 }
                 __syncthreads();
-                seq++;
+                group.seq++;
                 {   // pair k: kRuns adjacent threads add 32 words each
                     const int k = tid / kRuns, part = tid % kRuns;
                     const uint4 *src = reinterpret_cast<const uint4 *>(s_part + part_read);
@@ -596,24 +1000,14 @@ greedy_order_sliced_kernel(const uint8_t *__restrict__ k_codes, const uint8_t *_
                     if (kRuns == 16) a += lane_move<0x108, 0xF, true>(0u, a);
                     if (part == 0 && 2 * k < n_alive) {
                         if (members > 1) {      // both slots of the pair in one word
-                            __hip_atomic_store(xw + ((size_t)flip * members + mem) * 128 + k, ((uint64_t)seq << 32) | a, __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_AGENT);
+                            group.publish((uint32_t)k, a);
                         } else {
                             s_tot[0][2 * k] = a & 0xFFFFu;
                             s_tot[0][2 * k + 1] = a >> 16;
                         }
                     }
                 }
-                if (members > 1) {       // pair k = tid & 31 of the members q, q + kRuns, ..
-                    const int k = tid & 31, q = tid >> 5;
-                    uint32_t a_lo = 0u, a_hi = 0u;
-                    if (2 * k < n_alive)
-                        gather_words(xw + (size_t)flip * members * 128, (uint32_t)k, (uint32_t)q, (uint32_t)kRuns, members, seq, st,
-                                     [&](uint32_t w) { a_lo += w & 0xFFFFu; a_hi += w >> 16; });
-                    s_tot[q][2 * k] = a_lo;
-                    s_tot[q][2 * k + 1] = a_hi;
-                    flip ^= 1;
-                }
+                if (members > 1) group.gather_picks(n_alive);
                 __syncthreads();
                 uint32_t key = 0xFFFFFFFFu;            // (cost, token) in one word: the minimum is the first cheapest token
                 if (lane < n_alive) {
@@ -663,7 +1057,7 @@ greedy_order_sliced_kernel(const uint8_t *__restrict__ k_codes, const uint8_t *_
 // Four channels to a thread, and with nobody to exchange sums with there is no state, no ticket and no closing launch.  What a
 // step consists of is the chain price -> sums -> winner -> move.  Codes of any width are priced as 16-bit lanes (greedy_block_wide:
 // even and odd bytes apart, two registers a token, 3.0 vector instructions a channel and token), codes of four bits by looking
-// them up (greedy_block_narrow).  256 blocks of 64 tokens, a launch: x 2048 channels 182 us wide and 99 narrow, x 1024 channels
+// them up (greedy_narrow).  256 blocks of 64 tokens, a launch: x 2048 channels 182 us wide and 99 narrow, x 1024 channels
 // (256 threads) 142 and 70; 1024 blocks of the latter 342 and 182.
 __device__ __forceinline__ void price4x2(uint32_t ea, uint32_t oa, uint32_t eb, uint32_t ob, const uint32_t (&mn)[2], const uint32_t (&mx)[2],
                                          uint32_t &sum_a, uint32_t &sum_b) {
@@ -842,233 +1236,6 @@ __device__ __forceinline__ void greedy_block_wide(const uint32_t (&raw)[kSlicedT
 #undef xo
 }
 
-// Codes of at most four bits, where every one of a block is below 16.  A channel's four codes of four tokens lie in one register,
-// and what a code costs -- bit_length of the pack's range once it has joined -- is looked up there: a channel's table of 16
-// bytes (one of 136 for its minimum and maximum so far, read from LDS after every pick) serves four tokens with two byte
-// permutes, one vector instruction a token and channel against 3.0.  A code c >= 8 is kept as 0x80 | (c - 8): as a selector
-// that is out of the lower half's range, and 0xFF comes out; with its top bit flipped it selects from the upper half, and the
-// codes below 8 are out of range.  So each lookup finds one cost and one 0xFF, which is a constant -1 of the whole register,
-// carries included.
-__device__ __forceinline__ uint32_t code_selectors(uint32_t x) { return (x & 0x07070707u) | ((x & 0x08080808u) << 4); }
-__device__ __forceinline__ uint32_t selector_codes(uint32_t s) { return (s & 0x07070707u) | ((s >> 4) & 0x08080808u); }
-// Bytes [row][column] of four registers the other way round.
-__device__ __forceinline__ void transpose4(const uint32_t a0, const uint32_t a1, const uint32_t a2, const uint32_t a3, uint32_t (&x)[4]) {
-    const uint32_t l01 = __builtin_amdgcn_perm(a1, a0, 0x05010400u), h01 = __builtin_amdgcn_perm(a1, a0, 0x07030602u);
-    const uint32_t l23 = __builtin_amdgcn_perm(a3, a2, 0x05010400u), h23 = __builtin_amdgcn_perm(a3, a2, 0x07030602u);
-    x[0] = __builtin_amdgcn_perm(l23, l01, 0x05040100u);
-    x[1] = __builtin_amdgcn_perm(l23, l01, 0x07060302u);
-    x[2] = __builtin_amdgcn_perm(h23, h01, 0x05040100u);
-    x[3] = __builtin_amdgcn_perm(h23, h01, 0x07060302u);
-}
-// Half of a reduction that shares its results out: lanes l and l ^ 32 (16, or by a move within a row) each give away one of two values
-// and keep the sum of the other.  a's sum ends up where the lane's bit is clear (`upper` false), b's where it is set.
-__device__ __forceinline__ uint32_t halve32(uint32_t a, uint32_t b) {
-    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
-    return (uint32_t)r[0] + (uint32_t)r[1];
-}
-__device__ __forceinline__ uint32_t halve16(uint32_t a, uint32_t b) {
-    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
-    return (uint32_t)r[0] + (uint32_t)r[1];
-}
-template <int CTRL>
-__device__ __forceinline__ uint32_t halve_row(uint32_t a, uint32_t b, bool upper) {
-    return (upper ? b : a) + lane_move<CTRL, 0xF, true>(0u, upper ? a : b);
-}
-constexpr int kRor8 = 0x128, kHalfMirror = 0x141, kXor2 = 0x4E, kXor1 = 0xB1;     // lanes l ^ 8, l ^ 7, l ^ 2, l ^ 1
-
-// The better of this lane's vector and of the one a move brings (none: its own again): larger dot^2 / norm, then lower tag.
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ void best_cosine(uint32_t &dot, uint32_t &norm, uint32_t &tag) {
-    const uint32_t d = lane_move<CTRL, ROW_MASK, false>(dot, dot), n = lane_move<CTRL, ROW_MASK, false>(norm, norm),
-                   t = lane_move<CTRL, ROW_MASK, false>(tag, tag);
-    const unsigned long long theirs = (unsigned long long)d * d * norm, own = (unsigned long long)dot * dot * n;
-    const bool take = theirs > own || (theirs == own && t < tag);
-    dot = take ? d : dot;
-    norm = take ? n : norm;
-    tag = take ? t : tag;
-}
-
-typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
-
-// One barrier a step: a wavefront adds its channels up by itself -- 64 tokens in sixteen registers of byte sums, halved six
-// times -- and leaves a sum per token; behind the barrier every wavefront adds the wavefronts' sums of all tokens (lane = token
-// slot) and finds the winner.  The sums of two steps in turn lie in two buffers.  About 1.5 us a step of 2048 channels, half of it
-// vector instructions of two wavefronts a SIMD, the rest the latency of that chain; tables read only where a range has changed
-// were slower (104 us a launch against 98), cosines compared in 128 bits by shuffles 108.
-template <int THREADS>
-__device__ __forceinline__ void greedy_block_narrow(const uint32_t (&raw)[kSlicedTokens], uint32_t *lds, int N, int pack_len, uint32_t *__restrict__ perm) {
-    constexpr int kWaves = THREADS / 64;
-    static_assert(kWaves == 4 || kWaves == 8, "a lane reads the wavefronts' sums 16 bytes at a time");
-    uint4 *table = reinterpret_cast<uint4 *>(lds);             // [minimum][maximum]: the cost of every code
-    uint32_t *sums = lds + 256 * 4;                            // [2][64 tokens or 32 pairs][wavefront]
-    static_assert(256 * 4 + 2 * 64 * kWaves <= greedy_block_words<THREADS>(), "LDS");
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const bool bit1 = lane & 2, bit2 = lane & 4, bit3 = lane & 8;
-    if (tid < 256) {
-        const int lo = tid >> 4, hi = max(tid & 15, lo);
-        uint32_t w[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int v = 0; v < 16; v++) w[v >> 2] |= (32u - (uint32_t)__clz(max(hi, v) - min(lo, v))) << (8 * (v & 3));
-        table[tid] = make_uint4(w[0], w[1], w[2], w[3]);
-    }
-    u32x16 x[4];                                               // x[c][q]: channel c of the tokens in slots 4 q .. 4 q + 3
-#pragma unroll
-    for (int q = 0; q < kSlicedTokens / 4; q++) {
-        uint32_t by_channel[4];
-        transpose4(raw[4 * q], raw[4 * q + 1], raw[4 * q + 2], raw[4 * q + 3], by_channel);
-#pragma unroll
-        for (int c = 0; c < 4; c++) x[c][q] = code_selectors(by_channel[c]);
-    }
-    __syncthreads();
-    // where a lane leaves its wavefront's sums and which it reads (lane = slot): see the halvings below
-    const int pick_quad = (lane >> 5) | ((lane >> 3) & 2) | ((lane >> 1) & 4) | ((lane << 2) & 8);
-    const int pick_word = (2 * pick_quad + ((lane >> 2) & 1)) * kWaves + wave;
-    const int seed_word = (int)(__brev((uint32_t)lane) >> 26) * kWaves + wave;
-    const int pick_read = (2 * (lane >> 2) + (lane & 1)) * kWaves, pick_half = (lane & 2) << 3;
-    uint32_t orig = (uint32_t)lane, order = 0u;                // the token in slot `lane`; the token picked as number `lane`
-    int n_alive = N, in_pack = 0;
-    uint32_t mn[2], mx[2];                                     // ranges of channels (0, 2) and (1, 3), as 16-bit lanes
-    uint32_t cost[4][4];                                       // [channel]: its table
-    for (int step = 0; step < N; step++) {
-        const bool seed = in_pack == 0;
-        in_pack = in_pack + 1 == pack_len ? 0 : in_pack + 1;
-        uint32_t *buf = sums + (step & 1) * 64 * kWaves;
-        int sel;
-        if (seed) {
-            // ---- seed: rounded mean of the remaining tokens, then the best cosine ----
-            uint32_t sum[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-            for (int q = 0; q < kSlicedTokens / 4; q++) {
-                if (4 * q < n_alive) {
-                    const uint32_t live = n_alive - 4 * q >= 4 ? 0x01010101u : 0x01010101u >> (8 * (4 * q + 4 - n_alive));
-#pragma unroll
-                    for (int c = 0; c < 4; c++) sum[c] = __builtin_amdgcn_udot4(selector_codes(x[c][q]), live, sum[c], false);
-                }
-            }
-            const float na = (float)n_alive;                   // mean(dim=1).round(): fp32 quotient, round half to even
-            const uint32_t mean = (uint32_t)rintf((float)sum[0] / na) | ((uint32_t)rintf((float)sum[1] / na) << 8) |
-                                  ((uint32_t)rintf((float)sum[2] / na) << 16) | ((uint32_t)rintf((float)sum[3] / na) << 24);
-            // dot product and squared norm as 16-bit lanes: at most 4 x 15 x 15 a lane, 57600 a wavefront
-            uint32_t g8[8];
-#pragma unroll
-            for (int g = 0; g < 8; g++) {
-                g8[g] = 0u;
-                if (8 * g < n_alive) {
-                    uint32_t v[8];
-#pragma unroll
-                    for (int q = 0; q < 2; q++) {
-                        uint32_t by_token[4];
-                        transpose4(selector_codes(x[0][2 * g + q]), selector_codes(x[1][2 * g + q]), selector_codes(x[2][2 * g + q]),
-                                   selector_codes(x[3][2 * g + q]), by_token);
-#pragma unroll
-                        for (int t = 0; t < 4; t++)
-                            v[4 * q + t] = __builtin_amdgcn_udot4(by_token[t], mean, 0u, false) | (__builtin_amdgcn_udot4(by_token[t], by_token[t], 0u, false) << 16);
-                    }
-                    const uint32_t a = halve16(halve32(v[0], v[1]), halve32(v[2], v[3])), b = halve16(halve32(v[4], v[5]), halve32(v[6], v[7]));
-                    g8[g] = halve_row<kRor8>(a, b, bit3);
-                }
-            }
-            uint32_t g4[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) g4[i] = halve_row<kHalfMirror>(g8[2 * i], g8[2 * i + 1], bit2);
-            const uint32_t g2a = halve_row<kXor2>(g4[0], g4[1], bit1), g2b = halve_row<kXor2>(g4[2], g4[3], bit1);
-            buf[seed_word] = halve_row<kXor1>(g2a, g2b, lane & 1);     // slot: the lane's number with its bits in reverse
-            __syncthreads();
-            // dot^2 / norm by cross products: dot and norm stay below 2^19 (2048 channels), so they fit 64 bits.  A zero vector has
-            // cosine 0; slots that are empty as well, and lose every tie.
-            uint32_t dot = 0u, norm = 0u, tag = 0x8000u | (uint32_t)lane;
-            if (lane < n_alive) {
-#pragma unroll
-                for (int i = 0; i < kWaves; i += 4) {
-                    const uint4 w = *reinterpret_cast<const uint4 *>(buf + lane * kWaves + i);
-                    dot += (w.x & 0xFFFFu) + (w.y & 0xFFFFu) + (w.z & 0xFFFFu) + (w.w & 0xFFFFu);
-                    norm += (w.x >> 16) + (w.y >> 16) + (w.z >> 16) + (w.w >> 16);
-                }
-                tag = (orig << 8) | (uint32_t)lane;            // equal cosines: the earlier token
-            }
-            norm = max(norm, 1u);
-            best_cosine<0x111, 0xF>(dot, norm, tag);
-            best_cosine<0x112, 0xF>(dot, norm, tag);
-            best_cosine<0x114, 0xF>(dot, norm, tag);
-            best_cosine<0x118, 0xF>(dot, norm, tag);
-            best_cosine<0x142, 0xA>(dot, norm, tag);
-            best_cosine<0x143, 0xC>(dot, norm, tag);
-            sel = __builtin_amdgcn_readlane((int)tag, 63) & 0xFF;
-        } else {
-            // ---- the pack's other tokens: fewest bits after the pick ----
-            uint32_t h32[8];
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-                h32[i] = 0u;
-                if (8 * i < n_alive) {
-                    // (slots past the last one are priced as well: bounded sums nobody reads)
-                    uint32_t s[2];
-#pragma unroll
-                    for (int q = 0; q < 2; q++) {
-                        s[q] = 4u;                             // four channels' 0xFFs
-#pragma unroll
-                        for (int c = 0; c < 4; c++) {
-                            const uint32_t at = x[c][2 * i + q];
-                            s[q] += __builtin_amdgcn_perm(cost[c][1], cost[c][0], at) + __builtin_amdgcn_perm(cost[c][3], cost[c][2], at ^ 0x80808080u);
-                        }
-                    }
-                    h32[i] = halve32(s[0], s[1]);
-                }
-            }
-            // bytes: 16 a lane at most, 32, 64 and 128 after these halvings, then 16-bit lanes
-            uint32_t h16[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) h16[j] = halve16(h32[2 * j], h32[2 * j + 1]);
-            const uint32_t za = halve_row<kRor8>(h16[0], h16[1], bit3), zb = halve_row<kRor8>(h16[2], h16[3], bit3);
-            const uint32_t wa = halve_row<kHalfMirror>(bytes_even(za), bytes_odd(za), bit2), wb = halve_row<kHalfMirror>(bytes_even(zb), bytes_odd(zb), bit2);
-            uint32_t u = halve_row<kXor2>(wa, wb, bit1);
-            u += lane_move<kXor1, 0xF, true>(0u, u);
-            if ((lane & 1) == 0) buf[pick_word] = u;           // slots 4 quad + (lane bit 2) and, in the upper half, + 2
-            __syncthreads();
-            uint32_t a = 0u;
-#pragma unroll
-            for (int i = 0; i < kWaves; i += 4) {
-                const uint4 w = *reinterpret_cast<const uint4 *>(buf + pick_read + i);
-                a += w.x + w.y + w.z + w.w;
-            }
-            // (cost, token) in one word: the minimum is the first cheapest token
-            const uint32_t key = lane < n_alive ? (((a >> pick_half) & 0xFFFFu) << 8) | orig : 0xFFFFFFFFu;
-            const uint32_t best = wave_min_u32(key);
-            sel = (int)__builtin_ctzll(__ballot(key == best));
-        }
-        // the winner in slot `sel` leaves: its codes widen the pack's ranges and the last slot moves into `sel`
-        const int last = n_alive - 1;
-        const uint32_t tok = (uint32_t)__builtin_amdgcn_readlane((int)orig, sel);
-        const uint32_t moved = (uint32_t)__builtin_amdgcn_readlane((int)orig, last);
-        if (lane == sel) orig = moved;
-        if (lane == step) order = tok;
-        const int lq = last >> 2, sq = sel >> 2;
-        const uint32_t sb = (uint32_t)sel & 3u, keep = ~(0xFFu << (8 * sb));
-        const uint32_t take = (0x07060504u & keep) | (((uint32_t)last & 3u) << (8 * sb)), pair = sb | ((4u + sb) << 16) | 0x0C000C00u;
-        uint32_t w[4];
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const uint32_t l = x[c][lq];
-            w[c] = x[c][sq];
-            x[c][sq] = __builtin_amdgcn_perm(w[c], l, take);
-        }
-        n_alive--;
-        const uint32_t we = selector_codes(__builtin_amdgcn_perm(w[2], w[0], pair));
-        const uint32_t wo = selector_codes(__builtin_amdgcn_perm(w[3], w[1], pair));
-        mn[0] = seed ? we : pk_min_u16(mn[0], we);
-        mx[0] = seed ? we : pk_max_u16(mx[0], we);
-        mn[1] = seed ? wo : pk_min_u16(mn[1], wo);
-        mx[1] = seed ? wo : pk_max_u16(mx[1], wo);
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const uint32_t at = (mn[c & 1] << 8) | (mx[c & 1] << 4);      // bytes into the table, a 16-bit lane a channel
-            const uint4 t = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint8_t *>(table) + ((at >> (c >> 1) * 16) & 0xFF0u));
-            cost[c][0] = t.x; cost[c][1] = t.y; cost[c][2] = t.z; cost[c][3] = t.w;
-        }
-    }
-    if (wave == 0 && lane < N) perm[lane] = order;
-}
-
 template <int THREADS>
 __global__ void __launch_bounds__(THREADS, 2)
 greedy_order_block_kernel(const uint8_t *__restrict__ k_codes, const uint8_t *__restrict__ v_codes, int hidden, int N, int pack_len,
@@ -1087,7 +1254,11 @@ greedy_order_block_kernel(const uint8_t *__restrict__ k_codes, const uint8_t *__
 #pragma unroll
     for (int t = 0; t < kSlicedTokens; t++) any |= raw[t];
     if (__syncthreads_or((any & 0xF0F0F0F0u) != 0u)) greedy_block_wide<THREADS>(raw, lds, N, pack_len, perm + row0);
-    else greedy_block_narrow<THREADS>(raw, lds, N, pack_len, perm + row0);
+    else greedy_narrow<THREADS, 4>(
+        [&](int q, uint32_t (&v)[1][4]) {
+#pragma unroll
+            for (int t = 0; t < 4; t++) v[0][t] = raw[4 * q + t];
+        }, lds, N, pack_len, NoGroup{}, perm + row0);
 }
 
 // ---- out row r = in row perm[r], for K and V at once: grid (ctx_len), 256 threads ----
@@ -1349,8 +1520,8 @@ int pkv_greedy_repack(const uint8_t *k_codes, const uint8_t *v_codes, uint8_t *k
     // blocks of up to 64 tokens: register-resident channel slices, as many groups of workgroups as fit the device;
     int rc;
     // K and V rows of up to 1024 channels together: a workgroup of 256 threads to a block.  Up to 2048: one of 512, while the blocks do
-    // not outnumber the CUs (256 blocks 235 -> 204 us, the gather included; 512 blocks 345 against 390: two workgroups of the sliced
-    // kernel on a CU fill each other's gaps).
+    // not outnumber the CUs (5-bit codes: 256 blocks 235 -> 204 us, the gather included; 512 blocks 345 against 390: two workgroups of the
+    // sliced kernel on a CU fill each other's gaps; 4-bit codes, without a gather: 256 blocks 102, 512 in the sliced kernel 170).
     const bool small = 2 * (size_t)hidden_dim <= 4u * kSlicedThreadsNarrow;
     if (block_size <= kSlicedTokens && (small || (2 * (size_t)hidden_dim <= 4u * kSlicedThreadsWide && nblocks <= 256u))) {
         LaunchTimer tm(s, ms_out != nullptr);

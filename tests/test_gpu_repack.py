@@ -401,10 +401,12 @@ def test_greedy_order_with_a_block_to_a_workgroup(cuda, hid, T, bs, pack, top):
     assert (perm.cpu().numpy().reshape(-1, bs) == order).all()
 
 
-@pytest.mark.parametrize("hid,bs,pack", [(1024, 64, 16), (512, 64, 32), (1024, 36, 12), (272, 64, 16), (16, 4, 2)])
+@pytest.mark.parametrize("hid,bs,pack", [(1024, 64, 16), (512, 64, 32), (1024, 36, 12), (272, 64, 16), (16, 4, 2), (2048, 64, 16),
+                                         (1040, 48, 16), (2064, 64, 32), (4096, 64, 16), (4624, 12, 4)])
 def test_greedy_order_at_the_four_bit_edge(cuda, hid, bs, pack):
     """Blocks whose codes all lie below 16 look their costs up (four tokens to a register), others compute them: codes at the
-    ends of the range (the largest sums a wavefront can meet), equal tokens, zero tokens, one code of 16 in one of the blocks."""
+    ends of the range (the largest sums a wavefront can meet), equal tokens, zero tokens, one code of 16 in one of the blocks -- from
+    2064 channels on in the slice of one of several workgroups, which meet the others' sums."""
     g = torch.Generator().manual_seed(hid + bs)
     ends = lambda: torch.randint(0, 2, (5 * bs, hid), dtype=torch.uint8, generator=g) * 15
     kc, vc = ends(), ends()
