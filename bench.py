@@ -329,8 +329,8 @@ def gemv_surface(torch, ops, synth, dev):
     """The reference's own GPU ops at the shape its throughput script runs (one sequence of Llama-3.1-8B shape:
     8 KV heads, 65536 cached tokens, K at rel 0.1 = 4-bit codes, V at rel 0.2 = 3-bit codes) and by its definition:
     fp16 bytes of the uncompressed tensor / kernel time, K = kq_mat_vec_mul + fused_kq, V = wv_mat_vec_mul +
-    fused_wv, every op timed by the events inside its launcher (scripts/figure/throughput.py:124-138), beside
-    torch.matmul on the fp16 tensor."""
+    fused_wv, every op timed inside its launcher (scripts/figure/throughput.py:124-138), beside torch.matmul on the
+    fp16 tensor."""
     H, T = 8, 65536
     hid = H * 128
     k, v = synth.make_kv(1, H, T, seed=5, device=dev)

@@ -10,7 +10,9 @@
  *   - `ms_out` (host, may be NULL): when non-NULL the call brackets its kernels with HIP
  *     events, waits for them and stores the elapsed milliseconds -- the reference's
  *     launchers are synchronous and return milliseconds the same way
- *     (packkv_cuda_ext/src/kernels.cu:560-608, src/fused_kernels.cu:118-168);
+ *     (packkv_cuda_ext/src/kernels.cu:560-608, src/fused_kernels.cu:118-168).  The four ops of
+ *     the reference's GPU surface, which are always timed there, read the device's wall clock
+ *     instead: from the start of the first workgroup to a marker behind the last kernel;
  *   - return value 0 = success, otherwise a PKV_ERR_* code with text in pkv_last_error();
  *     the library never aborts the process (the reference's CPU codec aborts on a failed
  *     precondition, include/utils.h:8-16, and throws "not supported" for shapes outside

@@ -75,7 +75,8 @@ template <int W>
 __global__ void __launch_bounds__(256) kq_kernel(const uint8_t *__restrict__ stream, uint64_t stream_bytes, const uint32_t *__restrict__ info,
                                                  const uint16_t *__restrict__ q, uint16_t *__restrict__ kq_out, int ctx_len,
                                                  int hidden_dim, int ctx_blk, int nunits, uint32_t blk_cap, uint32_t slot,
-                                                 uint32_t nblocks, int dtype, int q_interleaved) {
+                                                 uint32_t nblocks, int dtype, int q_interleaved, LaunchStamp started) {
+    launch_started(started);
     extern __shared__ __align__(16) uint8_t lds[];
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t b = blockIdx.x * (blockDim.x >> 6) + wave;
@@ -127,7 +128,9 @@ constexpr int kWvWaves = 4;
 template <int W>
 __global__ void __launch_bounds__(64 * kWvWaves) wv_kernel(const uint8_t *__restrict__ stream, uint64_t stream_bytes, const uint32_t *__restrict__ info,
                                                            const uint16_t *__restrict__ w, float *__restrict__ wv_out, int ctx_len,
-                                                           int hidden_dim, int hid_blk, uint32_t blk_cap, uint32_t slot, int dtype) {
+                                                           int hidden_dim, int hid_blk, uint32_t blk_cap, uint32_t slot, int dtype,
+                                                           LaunchStamp started) {
+    launch_started(started);
     extern __shared__ __align__(16) uint8_t lds[];
     __shared__ __align__(16) float ws[kWvWaves][128];
     __shared__ float part[kWvWaves][kHeadDim];
@@ -209,7 +212,8 @@ static bool rows_of_fours(int n, std::initializer_list<const void *> ptrs) {
 // columns, four per thread, which are on their way meanwhile.
 __global__ void __launch_bounds__(256) fused_kq_kernel(uint16_t *__restrict__ out, const uint16_t *__restrict__ q,
                                                        const uint16_t *__restrict__ zero, const uint16_t *__restrict__ scale,
-                                                       const uint16_t *__restrict__ t, int K, int N, int dtype, bool vec) {
+                                                       const uint16_t *__restrict__ t, int K, int N, int dtype, bool vec, LaunchStamp started) {
+    launch_started(started);
     __shared__ float red[4];
     const int m = blockIdx.y;
     const int n = blockIdx.x * 1024 + 4 * (int)threadIdx.x;
@@ -242,7 +246,8 @@ __global__ void __launch_bounds__(256) fused_kq_kernel(uint16_t *__restrict__ ou
 constexpr int kWvPart = 1024;
 __global__ void __launch_bounds__(256) fused_wv_partial_kernel(const uint16_t *__restrict__ w, const uint16_t *__restrict__ zero,
                                                                const uint16_t *__restrict__ scale, float *__restrict__ part,
-                                                               int N, int dtype, bool vec) {
+                                                               int N, int dtype, bool vec, LaunchStamp started) {
+    launch_started(started);
     __shared__ float red[4];
     const int m = blockIdx.y, n = blockIdx.x * kWvPart + 4 * (int)threadIdx.x;
     const Raw4 a = ld4(w, (size_t)m * N, n, N, vec), z = ld4(zero, 0, n, N, vec), sc = ld4(scale, 0, n, N, vec);
@@ -297,12 +302,12 @@ int pkv_kq_mat_vec_mul(const uint8_t *stream, uint64_t stream_bytes, const uint3
     const int nblocks = (ctx_len / ctx_blk) * (hidden_dim / hid_blk);
     const uint32_t slot = ((cap + 15u) & ~15u) + 32u + 4u * 4u * kKqRow;      // at most 23.7 KB: 256 tokens at 4 bits
     const uint32_t wpw = slot * 4u <= 65536u ? 4u : 65536u / slot;
-    LaunchTimer tm(s, ms_out != nullptr);
+    StampedLaunch tm(s, ms_out != nullptr);
     if ((rc = tm.begin())) return rc;
     auto kern = bits == 2 ? kq_kernel<2> : bits == 3 ? kq_kernel<3> : kq_kernel<4>;
     kern<<<((uint32_t)nblocks + wpw - 1u) / wpw, 64u * wpw, wpw * slot, s>>>(
         stream, stream_bytes, block_info, (const uint16_t *)q, (uint16_t *)kq_out, ctx_len, hidden_dim, ctx_blk, nunits, cap,
-        slot, (uint32_t)nblocks, dtype, q_interleaved);
+        slot, (uint32_t)nblocks, dtype, q_interleaved, tm.stamp());
     PKV_HIP_CHECK(hipGetLastError());
     return tm.end(ms_out);
 }
@@ -322,11 +327,11 @@ int pkv_wv_mat_vec_mul(const uint8_t *stream, uint64_t stream_bytes, const uint3
     const uint32_t cap = (uint32_t)v_block_bound(hid_blk, bits);
     const uint32_t slot = ((cap + 15u) & ~15u) + 32u;           // at most 9.2 KB: 128 channels at 4 bits
     const uint32_t rows = (uint32_t)(ctx_len / ctx_blk + kWvWaves - 1) / kWvWaves;
-    LaunchTimer tm(s, ms_out != nullptr);
+    StampedLaunch tm(s, ms_out != nullptr);
     if ((rc = tm.begin())) return rc;
     auto kern = bits == 2 ? wv_kernel<2> : bits == 3 ? wv_kernel<3> : wv_kernel<4>;
     kern<<<rows * (uint32_t)(hidden_dim / hid_blk), 64 * kWvWaves, kWvWaves * slot, s>>>(
-        stream, stream_bytes, block_info, (const uint16_t *)w, wv_out, ctx_len, hidden_dim, hid_blk, cap, slot, dtype);
+        stream, stream_bytes, block_info, (const uint16_t *)w, wv_out, ctx_len, hidden_dim, hid_blk, cap, slot, dtype, tm.stamp());
     PKV_HIP_CHECK(hipGetLastError());
     return tm.end(ms_out);
 }
@@ -340,11 +345,11 @@ int pkv_fused_kq(void *our_kq, const void *q, const void *k_zero, const void *k_
     PKV_REQUIRE(our_kq && q && k_zero && k_scale && t, PKV_ERR_INVALID, "null pointer argument");
     PKV_REQUIRE(M > 0 && K > 0 && N > 0, PKV_ERR_INVALID, "sizes must be positive");
     PKV_REQUIRE(M <= 65535, PKV_ERR_UNSUPPORTED, "more than 65535 rows");
-    LaunchTimer tm(s, ms_out != nullptr);
+    StampedLaunch tm(s, ms_out != nullptr);
     if ((rc = tm.begin())) return rc;
     fused_kq_kernel<<<dim3((unsigned)((N + 1023) / 1024), (unsigned)M), 256, 0, s>>>(
         (uint16_t *)our_kq, (const uint16_t *)q, (const uint16_t *)k_zero, (const uint16_t *)k_scale,
-        (const uint16_t *)t, K, N, dtype, rows_of_fours(N, {our_kq, k_zero, k_scale, t}));
+        (const uint16_t *)t, K, N, dtype, rows_of_fours(N, {our_kq, k_zero, k_scale, t}), tm.stamp());
     PKV_HIP_CHECK(hipGetLastError());
     return tm.end(ms_out);
 }
@@ -361,11 +366,11 @@ int pkv_fused_wv(void *our_wv, const void *w, const void *v_zero, const void *v_
     const int nparts = (N + kWvPart - 1) / kWvPart;
     void *scratch = nullptr;
     if ((rc = scratch_get((size_t)M * nparts * sizeof(float), s, &scratch))) return rc;
-    LaunchTimer tm(s, ms_out != nullptr);
+    StampedLaunch tm(s, ms_out != nullptr);
     if ((rc = tm.begin())) return rc;
     fused_wv_partial_kernel<<<dim3((unsigned)nparts, (unsigned)M), 256, 0, s>>>(
         (const uint16_t *)w, (const uint16_t *)v_zero, (const uint16_t *)v_scale, (float *)scratch, N, dtype,
-        rows_of_fours(N, {w, v_zero, v_scale}));
+        rows_of_fours(N, {w, v_zero, v_scale}), tm.stamp());
     fused_wv_kernel<<<M, 256, 0, s>>>((uint16_t *)our_wv, (const float *)scratch, nparts, (const uint16_t *)term1,
                                       D, dtype);
     PKV_HIP_CHECK(hipGetLastError());

@@ -424,6 +424,29 @@ LaunchTimer::~LaunchTimer() {
     if (stop) (void)hipEventDestroy(stop);
 }
 
+__global__ void launch_ended_kernel(const LaunchStamp st) {
+    if (threadIdx.x == 0) stamp_now(st.word + 1, st.tag);
+}
+
+int StampedLaunch::end(float *ms_out) {
+    if (!enabled) return PKV_OK;
+    launch_ended_kernel<<<1, 64, 0, stream>>>(stamp());
+    PKV_HIP_CHECK(hipGetLastError());
+    uint64_t clock[2];
+    int rc = slot.wait(2, stream, clock), dev = 0, khz = 0;
+    if (rc) return rc;
+    waited = true;
+    PKV_HIP_CHECK(hipGetDevice(&dev));
+    PKV_HIP_CHECK(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
+    PKV_REQUIRE(khz > 0, PKV_ERR_HIP, "the device reports no wall clock rate");
+    *ms_out = (float)((clock[1] - clock[0]) & ((1ull << 34) - 1ull)) / (float)khz;
+    return PKV_OK;
+}
+
+StampedLaunch::~StampedLaunch() {
+    if (slot.words && !waited) (void)hipStreamSynchronize(stream);
+}
+
 int stagger_for(const void *kernel, int threads, uint32_t lds, uint32_t nwg, Stagger *out) {
     out->cus = out->slots = 0u;
     if (nwg < 1024u) return PKV_OK;                         // the appends of a growing cache: a handful of workgroups

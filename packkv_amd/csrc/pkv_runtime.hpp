@@ -88,6 +88,32 @@ struct OutcomeSlot {
     int wait(int n, hipStream_t s, uint64_t *values);      // the first `n` words, without their tags
     ~OutcomeSlot();
 };
+// The time of an op that is always timed, without events: its first kernel leaves the device's wall clock as it starts
+// (launch_started in workgroup 0) and a kernel of one wavefront behind the last one leaves it again, both in a pinned slot
+// that the host polls.  A pair of events recorded around the launch, waited for and read costs the host 17 us, this 10, around a
+// kernel of 4 us; events attached to the launch itself (hipExtLaunchKernel) 27.
+struct LaunchStamp {
+    uint64_t *word;                // NULL: not timed
+    uint64_t tag;                  // << 34
+};
+struct StampedLaunch {
+    OutcomeSlot slot;
+    hipStream_t stream;
+    bool enabled, waited = false;
+    StampedLaunch(hipStream_t s, bool on) : stream(s), enabled(on) {}
+    int begin() { return enabled ? slot.take(stream) : PKV_OK; }
+    ~StampedLaunch();              // a call that failed in between: its stamps have arrived before the slot goes back
+    LaunchStamp stamp() const { return LaunchStamp{enabled ? slot.words : nullptr, (uint64_t)slot.tag << 34}; }
+    int end(float *ms_out);        // behind the last launch: marks the end and waits when enabled
+};
+#ifdef __HIPCC__
+__device__ __forceinline__ void stamp_now(uint64_t *word, uint64_t tag) {
+    __hip_atomic_store(word, ((uint64_t)wall_clock64() & ((1ull << 34) - 1ull)) | tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ __forceinline__ void launch_started(const LaunchStamp st) {
+    if (st.word && (blockIdx.x | blockIdx.y | blockIdx.z | threadIdx.x) == 0) stamp_now(st.word, st.tag);
+}
+#endif
 // ... the launch that clears `h`'s state itself has been made.
 int scan_state_cleared(ScanHandle &h, hipStream_t s);
 // The block codec from a code matrix through the cells kernels (pkv_quant.hip): where code_cells_serve says so, for the

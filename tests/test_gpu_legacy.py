@@ -253,3 +253,47 @@ def test_bf16_factors_of_any_size(cuda, low, high, bits):
             want = torch.einsum("ht,thd->hd", w.double(), c)
             bound = (T + 8) * 2 ** -24
         assert bool(((got.cpu().double() - want).abs() <= bound * want).all()), is_k
+
+
+def test_times_and_results_of_ops_on_several_streams_at_once(cuda):
+    """Each op waits for its own kernel and returns its own time, whoever else is waiting; while a stream is capturing there is
+    no time to wait for, and the op is refused before it records anything."""
+    import threading
+    H, T = 8, 4096
+    g = torch.Generator(device=cuda)
+    g.manual_seed(3)
+    z, sc = (torch.randn(T, generator=g, device=cuda).half() for _ in range(2))
+    jobs = [(torch.randn(H, 128, generator=g, device=cuda).half(), torch.randn(H, T, generator=g, device=cuda).half()) for _ in range(4)]
+    want = [torch.empty(H, T, dtype=torch.float16, device=cuda) for _ in jobs]
+    for (q, t), out in zip(jobs, want):
+        assert ops.fused_kq(out, q, z, sc, t) > 0
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(i):
+        st, (q, t) = torch.cuda.Stream(), jobs[i]
+        with torch.cuda.stream(st):
+            for _ in range(50):
+                out = torch.zeros_like(want[i])
+                ms = ops.fused_kq(out, q, z, sc, t)
+                if not (0 < ms < 20 and torch.equal(out, want[i])):
+                    bad.append((i, ms))
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    assert not bad
+    st, graph, out = torch.cuda.Stream(), torch.cuda.CUDAGraph(), torch.empty_like(want[0])
+    with torch.cuda.stream(st):
+        graph.capture_begin()
+        try:
+            with pytest.raises(ops.PackKVError, match="capturing"):
+                ops.fused_kq(out, jobs[0][0], z, sc, jobs[0][1])
+            out.zero_()
+        finally:
+            graph.capture_end()
+    graph.replay()
+    torch.cuda.synchronize()
+    assert not out.any()
+    assert ops.fused_kq(out, jobs[0][0], z, sc, jobs[0][1]) > 0 and torch.equal(out, want[0])
