@@ -483,6 +483,32 @@ struct ScanState {
     uint64_t status[1];   // one per block
 };
 
+// An outcome is two words, each valid by itself through its tag: total (34 bits) | tag << 34 and error (8 bits) |
+// largest code (16 bits) << 8 | tag << 34.
+constexpr int kOutcomeWords = 2;
+__device__ __forceinline__ void publish_outcome(uint64_t *dst, uint64_t total, uint32_t max_code, uint32_t error, uint64_t tag) {
+    const uint64_t code = min(max_code, 0xFFFFu);
+    __hip_atomic_store(dst, (total & ((1ull << 34) - 1ull)) | (tag << 34), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(dst + 1, (uint64_t)(error & 0xFFu) | (code << 8) | (tag << 34), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// The outcome of an encode, or of two, to `last` and, for a waiting caller, to `slot`.  Of two encodes `last` keeps the second's
+// outcome unless the first one (codes of `bits` bits) failed.
+__device__ __forceinline__ void publish_outcomes(const ScanState *st, const ScanState *second, uint64_t *last, uint64_t *slot, uint64_t tag, int bits) {
+    auto get = [](const auto *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    const uint64_t total = get(&st->total);
+    const uint32_t error = get(&st->error), code = get(&st->max_code);
+    if (slot) publish_outcome(slot, total, code, error, tag);
+    if (!second) {
+        publish_outcome(last, total, code, error, tag);
+        return;
+    }
+    const uint64_t total2 = get(&second->total);
+    const uint32_t error2 = get(&second->error), code2 = get(&second->max_code);
+    if (slot) publish_outcome(slot + kOutcomeWords, total2, code2, error2, tag);
+    const uint32_t first = error ? error : bits > 0 && code >= (1u << bits) ? (uint32_t)PKV_ERR_UNSUPPORTED : 0u;
+    publish_outcome(last, total2, code2, first ? first : error2, tag);
+}
+
 // Called by every lane of the FIRST wavefront of the workgroup that owns block `idx`.
 // Returns the byte offset of the block in the stream.
 // Back-off between two polls of a status word that is still empty, in units of 64 cycles.  Hundreds of workgroups

@@ -1899,13 +1899,15 @@ bool code_cells_serve(bool is_k, int ctx_len, int hidden) {
     const OncePlan p = hidden % kHeadDim ? OncePlan{0, 0, 0, 0} : code_plan(is_k, ctx_len, hidden);
     return p.threads && hidden / kHeadDim % p.run == 0;    // (code_encode_once_kernel knows whole runs only)
 }
+uint32_t code_cells_closes(bool is_k, int ctx_len, int hidden) { return code_plan(is_k, ctx_len, hidden).nwg; }
+static uint32_t code_cells_groups(bool is_k, int ctx_len, int hidden) { return (uint32_t)(ctx_len / (is_k ? 64 : 128)) * (uint32_t)(hidden / 1024); }
 uint32_t code_cells_words(bool is_k, int ctx_len, int hidden) {
     const OncePlan p = code_plan(is_k, ctx_len, hidden);
-    return p.threads ? p.nwg : (uint32_t)(ctx_len / (is_k ? 64 : 128)) * (uint32_t)(hidden / 1024);
+    return p.threads ? p.nwg + close_words(p.nwg) : code_cells_groups(is_k, ctx_len, hidden);
 }
 int launch_code_cells(bool is_k, const uint8_t *codes, int ctx_len, int hidden, int bits, uint32_t bound, uint8_t *stream,
-                      uint64_t capacity, uint32_t *info, ScanState *st, hipStream_t s) {
-    const uint32_t ngroups = code_cells_words(is_k, ctx_len, hidden);
+                      uint64_t capacity, uint32_t *info, ScanState *st, const EncodeClose &close, hipStream_t s) {
+    const uint32_t ngroups = code_cells_groups(is_k, ctx_len, hidden);
     int rc;
     Stagger sg;
     if (const OncePlan p = code_plan(is_k, ctx_len, hidden); p.threads) {
@@ -1913,7 +1915,7 @@ int launch_code_cells(bool is_k, const uint8_t *codes, int ctx_len, int hidden, 
         a.codes = codes; a.hidden = hidden;
         a.stream = stream; a.capacity = capacity; a.info = info; a.st = st; a.W = bits;
         a.nruns = p.nruns; a.nwg = p.nwg; a.slot = once_slot(is_k, bits);
-        return p.threads == 256 ? once_launch_codes<256>(is_k, a, p.run, s) : once_launch_codes<1024>(is_k, a, p.run, s);
+        return p.threads == 256 ? once_launch_codes<256>(is_k, a, p.run, close, s) : once_launch_codes<1024>(is_k, a, p.run, close, s);
     } else if (is_k) {
         const uint32_t slot = (bound + 15u) & ~15u;
         const uint32_t lds = (uint32_t)kSubBlocks * slot + 32u;
@@ -2213,7 +2215,7 @@ static OnceSide once_side(bool is_k, const EncodeJob &job, const OncePlan &p, in
 }
 
 template <bool IS_K>
-static int launch_quant_encode(const EncodeJob &job, int dtype, int B, int H, int T, ScanState *st, hipStream_t s) {
+static int launch_quant_encode(const EncodeJob &job, int dtype, int B, int H, int T, ScanState *st, const EncodeClose &close, hipStream_t s) {
     const void *x = job.x;
     const XRows xs = job.xs;
     const float rel = job.rel;
@@ -2228,7 +2230,7 @@ static int launch_quant_encode(const EncodeJob &job, int dtype, int B, int H, in
     int rc;
     if (const OncePlan p = once_plan_of(IS_K, job, dtype, B, H, T); p.threads) {
         const OnceSide a = once_side(IS_K, job, p, B, H, T, st), none{};
-        return p.threads == 256 ? once_launch<256>(IS_K ? a : none, IS_K ? none : a, dtype, s) : once_launch<1024>(IS_K ? a : none, IS_K ? none : a, dtype, s);
+        return p.threads == 256 ? once_launch<256>(IS_K ? a : none, IS_K ? none : a, dtype, close, s) : once_launch<1024>(IS_K ? a : none, IS_K ? none : a, dtype, close, s);
     }
     // One workgroup per run of up to eight heads of a (context block, sequence) group -- K: its up to eight blocks;
     // V: its up to sixteen -- or, with fewer than five heads, per 8 / H groups.
@@ -2328,28 +2330,38 @@ static int run_quant_encode(const void *x, int dtype, int B, int H, int T, float
     EncodeJob job{x, dense_rows(H, T), rel, bits, stream, capacity, base, info, scale, zero, par_stride, perm, perm_block, scale_in, zero_in};
     int rc = check_job<IS_K>(job, dtype, B, H, T);
     if (rc) return rc;
+    const uint32_t closes = once_plan_of(IS_K, job, dtype, B, H, T).nwg;       // workgroups of a launch that closes by itself
+    ClosedEncode ce;
     ScanHandle sh;
-    if ((rc = prepare_scan_state((uint32_t)state_words(IS_K, B, H, T), &sh, s, size_out || ms_out))) return rc;
+    if ((rc = prepare_scan_state((uint32_t)state_words(IS_K, B, H, T) + (closes ? close_words(closes) : 0u), &sh, s, size_out || ms_out))) return rc;
+    if (closes && (rc = ce.begin(sh, closes, size_out ? 1 : 0, bits, s))) return rc;
     LaunchTimer tm(s, ms_out != nullptr);
     if ((rc = tm.begin())) return rc;
-    if ((rc = launch_quant_encode<IS_K>(job, dtype, B, H, T, sh.st, s))) return rc;
+    if ((rc = launch_quant_encode<IS_K>(job, dtype, B, H, T, sh.st, ce.close, s))) return rc;
+    if (closes && (rc = ce.launched(sh))) return rc;
     if ((rc = tm.end(ms_out))) return rc;
-    return finish_encode(sh, size_out, bits, s);
+    return closes ? ce.wait(size_out, bits) : finish_encode(sh, size_out, bits, s);
 }
 
 // K and V (checked jobs) with one wait; in one launch where both take a group's tokens at once.
 static int encode_both(const EncodeJob job[2], int dtype, int B, int H, int T, uint64_t *k_size, uint64_t *v_size, hipStream_t s) {
     int rc;
-    ScanHandle sh;
-    if ((rc = prepare_scan_state((uint32_t)state_words(true, B, H, T), &sh, s, true, (uint32_t)state_words(false, B, H, T)))) return rc;
     const OncePlan pk = once_plan_of(true, job[0], dtype, B, H, T), pv = once_plan_of(false, job[1], dtype, B, H, T);
-    if (pk.threads && pk.threads == pv.threads && (job[0].bits > 4) == (job[1].bits > 4)) {
+    const bool one_launch = pk.threads && pk.threads == pv.threads && (job[0].bits > 4) == (job[1].bits > 4);
+    const uint32_t closes = one_launch ? pk.nwg + pv.nwg : 0u;
+    ClosedEncode ce;
+    ScanHandle sh;
+    if ((rc = prepare_scan_state((uint32_t)state_words(true, B, H, T), &sh, s, true,
+                                 (uint32_t)state_words(false, B, H, T) + (closes ? close_words(closes) : 0u)))) return rc;
+    if (one_launch) {
         const OnceSide ks = once_side(true, job[0], pk, B, H, T, sh.st), vs = once_side(false, job[1], pv, B, H, T, sh.second);
-        if ((rc = pk.threads == 256 ? once_launch<256>(ks, vs, dtype, s) : once_launch<1024>(ks, vs, dtype, s))) return rc;
-    } else {
-        if ((rc = launch_quant_encode<true>(job[0], dtype, B, H, T, sh.st, s))) return rc;
-        if ((rc = launch_quant_encode<false>(job[1], dtype, B, H, T, sh.second, s))) return rc;
+        if ((rc = ce.begin(sh, closes, 2, job[0].bits, s))) return rc;
+        if ((rc = pk.threads == 256 ? once_launch<256>(ks, vs, dtype, ce.close, s) : once_launch<1024>(ks, vs, dtype, ce.close, s))) return rc;
+        if ((rc = ce.launched(sh))) return rc;
+        return ce.wait(k_size, job[0].bits, v_size, job[1].bits);
     }
+    if ((rc = launch_quant_encode<true>(job[0], dtype, B, H, T, sh.st, EncodeClose{}, s))) return rc;
+    if ((rc = launch_quant_encode<false>(job[1], dtype, B, H, T, sh.second, EncodeClose{}, s))) return rc;
     return finish_encode(sh, k_size, job[0].bits, s, v_size, job[1].bits);
 }
 

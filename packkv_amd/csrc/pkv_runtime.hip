@@ -41,7 +41,6 @@ struct Workspace {
     uint64_t *last;         // pinned, host and device: outcome of the last encode on this stream (kOutcomeWords), tag 0 before it
     std::shared_ptr<std::mutex> enc_mu;
 };
-constexpr int kOutcomeWords = 2;
 static_assert(2 * kOutcomeWords <= kSlotWords, "a slot (a cache line) holds the outcomes of two encodes");
 constexpr int kSlotsPerChunk = 64;
 std::vector<uint64_t *> g_chunks;                     // pinned slots of the encodes that are waited for (any device)
@@ -104,14 +103,6 @@ int scratch_get(size_t bytes, hipStream_t s, void **out) {
 }
 
 // ---- the encoders' look-back state and outcome ------------------------------------------------------------------
-// An outcome is two words, each valid by itself through its tag: total (34 bits) | tag << 34 and error (8 bits) |
-// largest code (16 bits) << 8 | tag << 34.
-__device__ __forceinline__ void publish_outcome(uint64_t *dst, const ScanState *st, uint32_t error, uint64_t tag) {
-    const uint64_t total = st->total & ((1ull << 34) - 1ull), code = min(st->max_code, 0xFFFFu);
-    __hip_atomic_store(dst, total | (tag << 34), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    __hip_atomic_store(dst + 1, (uint64_t)(error & 0xFFu) | (code << 8) | (tag << 34), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
 // The outcome of the encode before it on the stream to `last` and, for a waiting caller, to `slot`; the state back to
 // zero.  Of two encodes `last` keeps the second's outcome unless the first one (codes of `bits` bits) failed.  Four words
 // per thread: the state of 1 GiB of input (8192 tickets) is cleared by nine workgroups.  Latency is all there is to it: 4.2 us
@@ -121,14 +112,7 @@ __global__ void __launch_bounds__(256) finish_encode_kernel(ScanState *st, ScanS
     constexpr uint32_t kHead = offsetof(ScanState, status) / 8;
     const uint32_t head2 = second ? (uint32_t)(reinterpret_cast<uint64_t *>(second) - words) : 0xFFFFFFFFu;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        if (slot) publish_outcome(slot, st, st->error, tag);
-        if (slot && second) publish_outcome(slot + kOutcomeWords, second, second->error, tag);
-        if (second) {
-            const uint32_t first = st->error ? st->error : bits > 0 && st->max_code >= (1u << bits) ? (uint32_t)PKV_ERR_UNSUPPORTED : 0u;
-            publish_outcome(last, second, first ? first : second->error, tag);
-        } else {
-            publish_outcome(last, st, st->error, tag);
-        }
+        publish_outcomes(st, second, last, slot, tag, bits);
         for (uint32_t i = 0; i < kHead; i++) {
             words[i] = 0;
             if (second) words[head2 + i] = 0;
@@ -288,6 +272,44 @@ OutcomeSlot::~OutcomeSlot() {
     if (!words) return;
     std::lock_guard<std::mutex> lock(g_ws_mu);
     g_free_slots.push_back(words);
+}
+
+int ClosedEncode::begin(ScanHandle &h, uint32_t total, int sizes, int bits, hipStream_t stream) {
+    std::lock_guard<std::mutex> lock(g_ws_mu);
+    Workspace *w = nullptr;
+    int rc = workspace_for(stream, &w);
+    if (rc) return rc;
+    uint32_t tag = 0;
+    if ((rc = slot_take(sizes ? &close.slot : nullptr, &tag))) return rc;
+    s = stream;
+    close.words = (uint64_t *)h.st;
+    close.n = (uint32_t)h.words64;
+    close.total = total;
+    close.count = close.words + (h.words64 - close_words(total));
+    close.st = h.st;
+    close.second = h.second;
+    close.last = w->last;
+    close.tag = tag;
+    close.bits = bits;
+    return PKV_OK;
+}
+
+int ClosedEncode::launched(ScanHandle &h) { return scan_state_cleared(h, s); }
+
+int ClosedEncode::wait(uint64_t *size_out, int bits, uint64_t *size2_out, int bits2) {
+    if (!close.slot) return PKV_OK;
+    int rc = wait_words(close.slot, close.second ? 2 * kOutcomeWords : kOutcomeWords, (uint32_t)close.tag, s);
+    waited = true;
+    if (!rc && size_out) rc = outcome(close.slot, size_out, bits);
+    if (!rc && close.second && size2_out) rc = outcome(close.slot + kOutcomeWords, size2_out, bits2);
+    return rc;
+}
+
+ClosedEncode::~ClosedEncode() {
+    if (!close.slot) return;
+    if (!waited) (void)hipStreamSynchronize(s);
+    std::lock_guard<std::mutex> lock(g_ws_mu);
+    g_free_slots.push_back(close.slot);
 }
 
 int scan_state_cleared(ScanHandle &h, hipStream_t s) {

@@ -449,3 +449,45 @@ def test_padding_of_one_sequence_leaves_the_others_alone(cuda, dtype, H, T):
         dec(e["stream"], e["info"], codes, bits=4)
         c, z, s = oq.quant_ints(x[1:].cpu(), 64, 0.1)
         assert torch.equal(codes[:, H * 128:].cpu(), oq.code_matrix(c)), "K" if is_k else "V"
+
+
+@pytest.mark.parametrize("H,T", [(2, 128), (2, 1920), (2, 2048), (2, 2176), (8, 2048), (16, 1024), (8, 16384), (40, 640)])
+def test_encoders_that_close_by_themselves(cuda, H, T):
+    """Launches of up to 256 workgroups hand their outcome over and clear the look-back state without a kernel behind them,
+    counted in sixteens: one workgroup, counts around a multiple of sixteen, the most there are.  Each encode finds the state
+    clear, whatever the one before was -- fused K and V, K and V in one launch, codes, with and without a size, a stream that does
+    not fit -- and gives what encodes of 64 and 128 tokens appended one by one give."""
+    k, v = synth.make_kv(1, H, T, seed=H + T, device=cuda)
+
+    def side(x, is_k):
+        nblk = T // (64 if is_k else 128) * H * (1 if is_k else 2)
+        return [0.1, 4, torch.zeros(T * H * 128 + 16, dtype=torch.uint8, device=cuda), 0, torch.zeros(nblk, 2, dtype=torch.uint32, device=cuda),
+                torch.zeros(1, T, dtype=x.dtype, device=cuda), torch.zeros(1, T, dtype=x.dtype, device=cuda)]
+    want = {}
+    for is_k, x in ((True, k), (False, v)):
+        s, step = side(x, is_k), 64 if is_k else 128
+        for t in range(0, T, step):
+            s[3] = ops.quant_encode_append(is_k, x[:, :, t:t + step].contiguous(), 0.1, 4, s[2], s[3], s[4], t, s[5], s[6])
+        want[is_k] = s
+
+    def check(is_k, size, stream, info, what):
+        w = want[is_k]
+        assert size == w[3], (what, is_k)
+        assert torch.equal(stream[:size], w[2][:size]) and torch.equal(info.view(torch.int32), w[4].view(torch.int32)), (what, is_k)
+    for turn in range(3):
+        ks, vs = side(k, True), side(v, False)
+        kn, vn = ops.kv_quant_encode_append(k, v, T, ks, vs, 0)
+        check(True, kn, ks[2], ks[4], "both")
+        check(False, vn, vs[2], vs[4], "both")
+        for is_k, x, enc, code_enc in ((True, k, ops.k_quant_encode, ops.k_encode), (False, v, ops.v_quant_encode, ops.v_encode)):
+            e = enc(x, 0.1)
+            check(is_k, e["size"], e["stream"], e["info"], "alone")
+            u = enc(x, 0.1, want_size=False)
+            check(is_k, ops.encode_status(cuda, bits=4), u["stream"], u["info"], "no size")
+            codes = ops.quantize(x, e["scale"], e["zero"])[0]
+            s = side(x, is_k)
+            check(is_k, code_enc(codes, s[2], s[4]), s[2], s[4], "codes")
+            with pytest.raises(ops.PackKVError, match="fit"):
+                code_enc(codes, s[2][:e["size"] - 2], s[4])
+            with pytest.raises(ops.PackKVError, match="fit"):
+                enc(x, 0.1, stream=s[2][:e["size"] - 2], info=s[4])
