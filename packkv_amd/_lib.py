@@ -10,6 +10,9 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # PACKKV_HIP_LIB names another build of the same library (kernel development: A/B runs of two builds)
 LIB_PATH = os.environ.get("PACKKV_HIP_LIB") or os.path.join(_HERE, "libpackkv_hip.so")
+HOST_PATH = os.path.join(_HERE, "_host.so")
+HOST_SYMBOLS = ("pkv_attn_decode", "pkv_window_append", "pkv_dense_view", "pkv_kq_mat_vec_mul", "pkv_wv_mat_vec_mul", "pkv_fused_kq",
+                "pkv_fused_wv")
 
 F16, BF16 = 0, 1
 OK, ERR_UNSUPPORTED, ERR_INVALID, ERR_HIP, ERR_CAPACITY, ERR_INTERNAL = range(6)
@@ -97,6 +100,7 @@ SIGNATURES = {
 }
 
 _lib = None
+host = None        # the native host side of the repeated calls (csrc/pkv_host.cpp), bound to the library once that is loaded
 
 
 class PackKVError(RuntimeError):
@@ -109,13 +113,16 @@ class PackKVError(RuntimeError):
 
 def load():
     """Load the library once and attach prototypes.  Raises ImportError when it is missing."""
-    global _lib
+    global _lib, host
     if _lib is not None:
         return _lib
-    if not os.path.exists(LIB_PATH):
-        raise ImportError(
-            "libpackkv_hip.so is not built (%s). Build it with `python -m packkv_amd.build` "
-            "(needs hipcc, targets gfx950); there is no CPU fallback." % LIB_PATH)
+    for path in (LIB_PATH, HOST_PATH):
+        if not os.path.exists(path):
+            raise ImportError(
+                "%s is not built (%s). Build it with `python -m packkv_amd.build` "
+                "(needs hipcc, targets gfx950); there is no CPU fallback." % (os.path.basename(path), path))
+    import torch  # noqa: F401  (the libraries that _host.so needs)
+    from . import _host
     try:
         lib = ctypes.CDLL(LIB_PATH)
     except OSError as e:  # pragma: no cover - depends on the machine
@@ -124,7 +131,8 @@ def load():
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
-    _lib = lib
+    _host.bind(*(ctypes.cast(getattr(lib, name), _vp).value for name in HOST_SYMBOLS))
+    host, _lib = _host, lib
     return lib
 
 

@@ -1,6 +1,7 @@
 """Builds libpackkv_hip.so (hand-written HIP for gfx950) in-tree with hipcc.
 
     python -m packkv_amd.build          # compile every kernel source and link
+                                        # (and _host.so, the host side of the repeated calls: C++ against torch's headers)
     python -m packkv_amd.build --changed   # recompile only what is older than its sources
     python -m packkv_amd.build --define PKV_ATTN_PROBE=30 --out /tmp/libpackkv_probe.so
                                         # a development build with extra -D flags under another name (objects in a
@@ -18,6 +19,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libpackkv_hip.so")
+HOST = os.path.join(HERE, "_host.so")
 SOURCES = ["pkv_runtime.hip", "pkv_codec.hip", "pkv_codec_long.hip", "pkv_quant.hip", "pkv_legacy.hip", "pkv_attn.hip", "pkv_repack.hip", "pkv_cache.hip", "pkv_dense.hip"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -59,6 +61,21 @@ def _compile(src, only_stale=False, defines=(), obj_dir=OBJ):
     return obj
 
 
+def _build_host(only_stale=False):
+    if only_stale and os.path.exists(HOST) and not _stale("pkv_host.cpp", HOST):
+        return HOST
+    import sysconfig
+    from torch.utils import cpp_extension
+    torch_lib = os.path.join(os.path.dirname(os.path.dirname(cpp_extension.include_paths()[0])), "torch", "lib")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"]
+    cmd += ["-I" + d for d in [sysconfig.get_paths()["include"]] + cpp_extension.include_paths()] + ["-I/opt/rocm/include"]
+    cmd += [os.path.join(CSRC, "pkv_host.cpp"), "-o", HOST, "-L" + torch_lib, "-ltorch_python", "-ltorch_cpu", "-lc10_hip", "-lc10"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed for pkv_host.cpp:\n" + r.stderr)
+    return HOST
+
+
 def build(verbose=True, only_stale=False, defines=(), out=None):
     """Compile and link.  only_stale=True (``--changed`` on the command line) recompiles only the sources whose
     object file is older than the source or a header.  `defines` / `out`: a development build with extra -D flags,
@@ -66,8 +83,11 @@ def build(verbose=True, only_stale=False, defines=(), out=None):
     lib = out or LIB
     obj_dir = OBJ if not defines else OBJ + "_" + "_".join(d.replace("=", "-") for d in defines)
     os.makedirs(obj_dir, exist_ok=True)
-    with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as ex:
+    with ThreadPoolExecutor(max_workers=8) as ex:
+        host = ex.submit(_build_host, only_stale) if out is None else None
         objs = list(ex.map(lambda src: _compile(src, only_stale, defines, obj_dir), SOURCES))
+        if host is not None:
+            host.result()
     cmd = [_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", lib] + objs
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:

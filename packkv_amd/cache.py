@@ -191,8 +191,12 @@ class PackKVCompressedCache:
         """One decode step: query_states [B, Hq, 128] (or [B, Hq, 1, 128]) against everything cached in the
         layer; returns [B, Hq, 128] (same rank as given).  variant / ref_rounding / out_f32 select the checking
         kernels of ops.attn_decode (not cached as a plan)."""
-        L = self._layer(layer_idx)
+        L = self.layers[layer_idx] or self._layer(layer_idx)
         q = query_states
+        if L.plan is not None and L.plan.sm_scale_arg == sm_scale and L.win_len and out is None and not (variant or ref_rounding or out_f32):
+            res = L.plan.step(q, L.win_len)
+            if res is not None:
+                return res
         squeeze = q.dim() == 4
         if squeeze:
             q = q[:, :, 0]

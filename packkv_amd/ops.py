@@ -37,6 +37,12 @@ def _ptr(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
 
 
+def _host():
+    """The native side of the calls a decode loop repeats (csrc/pkv_host.cpp): its functions return None for a call that they do
+    not serve, which then takes the general code below them."""
+    return _lib.host or (_lib.load() and _lib.host)
+
+
 # Every op makes `dev` current and passes on its current stream.  A stream object and a device context that is entered
 # although the device is current take 3.5 us of host time a call -- a decode step is two calls and 13 us of GPU time --
 # these two take 0.5.  (They are not part of torch's public surface: without them the public functions serve.)
@@ -558,6 +564,9 @@ def window_append(k_new, v_new, cos, sin, k_win, v_win, win_pos):
     [B, H, cap, 128]; with cos / sin [B, n, 128] the keys get the rotary embedding first, rounded like the reference's
     chain of 16-bit elementwise ops (utils/compute.py:35-43).  One launch; strided views (a transposed projection
     output, an expanded cos / sin table) are read in place."""
+    rc = _host().window_append(k_new, v_new, cos, sin, k_win, v_win, win_pos)
+    if rc is not None:
+        return _lib.check(rc)
     B, H, n, D = k_new.shape
     dev, at, dtype, win = k_new.device, k_new.get_device(), k_new.dtype, k_win.shape
     _require(D == 128 and v_new.shape == k_new.shape and k_new.is_cuda and v_new.dtype == dtype,
@@ -953,6 +962,16 @@ def repack_quant_encode(k, v, k_rel, v_rel, repack_method="median", block_size=6
 
 # ------------------------------------------------------- reference GEMV surface ------
 
+def _timed(served, raises=False):
+    """What the native side of a timed op returned: milliseconds, or a status -- an unsupported shape prints and takes no time."""
+    if type(served) is float:
+        return served
+    if served == _lib.ERR_UNSUPPORTED and not raises:
+        print("no such case")
+        return 0.0
+    return _lib.check(served)
+
+
 def _require_cuda(*ts):
     for t in ts:
         if not t.is_cuda:
@@ -966,6 +985,10 @@ def kq_mat_vec_mul(compressed_buffer, block_info_buffer, q, kq_out, ctx_len, hid
     reference's lane-interleaved layout (evaluation/evaluation.py:465-468) unless
     q_interleaved=False.  Like the reference, an unsupported shape or dtype prints a message
     and returns 0.0 (src/kernels.cu:586-589, :626-629)."""
+    served = _host().mat_vec(True, compressed_buffer, block_info_buffer, q, kq_out, ctx_len, hidden_dim, ctx_len_block_size, hidden_dim_block_size,
+                             bits_len, q_interleaved)
+    if served is not None:
+        return _timed(served)
     _require_cuda(compressed_buffer, block_info_buffer, q, kq_out)
     if q.dtype not in (torch.float16, torch.bfloat16):
         print("Unsupported data type")
@@ -987,6 +1010,10 @@ def wv_mat_vec_mul(compressed_buffer, block_info_buffer, w, wv_out, ctx_len, hid
                    ctx_len_block_size, hidden_dim_block_size, bits_len):
     """Drop-in for packkv_cuda.wv_mat_vec_mul (packkv_cuda.pyi:60-70): wv_out (fp32, caller-zeroed,
     [hidden_dim] or [H, 128]) += sum_tok w[c // 128, tok] * code[tok, c]; returns milliseconds."""
+    served = _host().mat_vec(False, compressed_buffer, block_info_buffer, w, wv_out, ctx_len, hidden_dim, ctx_len_block_size, hidden_dim_block_size,
+                             bits_len, False)
+    if served is not None:
+        return _timed(served)
     _require_cuda(compressed_buffer, block_info_buffer, w, wv_out)
     if w.dtype not in (torch.float16, torch.bfloat16):
         print("Unsupported data type")
@@ -1009,6 +1036,9 @@ def wv_mat_vec_mul(compressed_buffer, block_info_buffer, w, wv_out, ctx_len, hid
 def fused_kq(our_kq, q, k_quant_zero, k_quant_scale, t):
     """Drop-in for packkv_cuda.fused_kq (packkv_cuda.pyi:72-78; checks of
     src/fused_kernels.cu:90-108): our_kq[m, n] = (sum(q[m]) * zero[n] + t[m, n]) * scale[n]."""
+    served = _host().fused(True, our_kq, q, k_quant_zero, k_quant_scale, t)
+    if served is not None:
+        return _timed(served, raises=True)
     if q.dtype not in (torch.float16, torch.bfloat16):
         raise RuntimeError("Unsupported data type for fused_kq_launcher")
     if q.dim() != 2: raise RuntimeError("q must be a 2D tensor")
@@ -1043,6 +1073,9 @@ def fused_kq(our_kq, q, k_quant_zero, k_quant_scale, t):
 def fused_wv(our_wv, w, v_quant_zero, v_quant_scale, term1):
     """Drop-in for packkv_cuda.fused_wv (packkv_cuda.pyi:80-86; checks of
     src/fused_kernels.cu:275-293): our_wv[m, d] = sum_n w[m, n] * zero[n] * scale[n] + term1[m, d]."""
+    served = _host().fused(False, our_wv, w, v_quant_zero, v_quant_scale, term1)
+    if served is not None:
+        return _timed(served, raises=True)
     if w.dtype not in (torch.float16, torch.bfloat16):
         raise RuntimeError("Unsupported data type for fused_wv_launcher")
     if w.dim() != 2: raise RuntimeError("w must be a 2D tensor")
@@ -1078,6 +1111,9 @@ def dense_view(k, v, k_win=None, v_win=None, win_len=None):
     """(K, V) [B, H, T, 128] behind a compressed cache: k and v as attn_decode takes them (stream, info, scale, zero,
     bits, ``tokens``, ``heads``) or None, dequantised as the reference stores them (utils/compute.py:173-179), followed
     by the `win_len` rows in use of the 16-bit windows k_win / v_win [B, H, cap, 128].  One launch."""
+    served = _host().dense_view(k, v, k_win, v_win, win_len)
+    if served is not None:
+        return served if type(served) is tuple else _lib.check(served)
     a = AttnArgs()
     like = k["scale"] if k is not None else k_win
     dev, at = like.device, like.get_device()
@@ -1182,6 +1218,13 @@ class AttnPlan:
         self._fn = _lib.load().pkv_attn_decode
         self._fn_noalloc = _lib.load().pkv_attn_decode_noalloc if noalloc else None
         self._ref = ctypes.byref(a)
+        self._where = (ctypes.addressof(a), q.get_device())
+
+    def step(self, q, win_len):
+        """The result of the step for `q` -- [B, Hq, 128], or [B, Hq, 1, 128] -- with `win_len` window rows in use, in q's shape;
+        None where q is not what the plan was made for as it lies."""
+        served = _host().plan_step(*self._where, win_len, q)
+        return _lib.check(served) if type(served) is int else served
 
     def set_window_rows(self, win_len):
         """Window rows in use (the window tensors are allocated longer and fill up between cuts)."""
@@ -1227,4 +1270,8 @@ def attn_decode(q, k, v, k_win=None, v_win=None, sm_scale=None, out=None, varian
     mode -- every K and V element is formed as the reference stores it, dtype(dtype(code + zero) * scale)
     (utils/compute.py:173-179), before the fp32 dot products.  noalloc: go through pkv_attn_decode_noalloc (the
     partial results in the library's fixed 8 MiB device array; the caller passes `out`, or torch allocates it)."""
+    if out is None and not (variant or timed or ref_rounding or out_f32 or noalloc):
+        served = _host().attn_decode(q, k, v, k_win, v_win, sm_scale, win_len)
+        if served is not None:
+            return _lib.check(served) if type(served) is int else served
     return AttnPlan(q, k, v, k_win, v_win, sm_scale, out, variant, win_len, ref_rounding, out_f32, noalloc)(timed=timed)
