@@ -348,43 +348,60 @@ int launch_quant_dequant(const void *k, const void *v, void *k_out, void *v_out,
     return PKV_OK;
 }
 
-// bit_length of both 16-bit halves, clamped to 4 (values above 15 mean the codes overflow the
-// format; the launch reports that through max_code)
-__device__ __forceinline__ uint32_t pk_bitlen4(uint32_t d) {
-    const u16x2 v = as_u16x2(d), one = {1, 1};
-    const u16x2 l = __builtin_elementwise_min(v, one) + __builtin_elementwise_min((u16x2)(v >> 1), one) +
-                    __builtin_elementwise_min((u16x2)(v >> 2), one) + __builtin_elementwise_min((u16x2)(v >> 3), one);
-    return pk_u16(l);
+// bit_length of both 16-bit halves, clamped to MOST (larger values mean the codes overflow the format; the launch reports that
+// through max_code): the exponent of (2 r + 1) 2^-10 as a half, r read as a subnormal half (r 2^-24 times 2^15, exact).  Four
+// instructions; sums of min(r >> k, 1) came out of the compiler as compares and selects of single halves, 24.
+template <int MOST>
+__device__ __forceinline__ uint32_t pk_bitlen(uint32_t r) {
+    const f16x2 f = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, r), (f16x2){(_Float16)32768.f, (_Float16)32768.f},
+                                              (f16x2){(_Float16)0.0009765625f, (_Float16)0.0009765625f});
+    const u16x2 e = (__builtin_bit_cast(u16x2, f) >> 10) - (u16x2){5, 5};
+    return pk_u16(__builtin_elementwise_min(e, (u16x2){MOST, MOST}));
+}
+// Minimum or maximum of 16 words of two codes each, as unsigned integers: what NaN makes of a code may have its top bit set, and
+// the packs of such tokens are to be the same in every kernel (v_pk_minimum3_f16 would take three at a time, but by their sign).
+template <bool MAX>
+__device__ __forceinline__ uint32_t pk_side16(const uint32_t c[16]) {
+    auto of = [](u16x2 a, u16x2 b) { return MAX ? __builtin_elementwise_max(a, b) : __builtin_elementwise_min(a, b); };
+    u16x2 m[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) m[j] = as_u16x2(c[j]);
+#pragma unroll
+    for (int k = 4; k < 16; k++) m[k & 3] = of(m[k & 3], as_u16x2(c[k]));
+    return pk_u16(of(of(m[0], m[1]), of(m[2], m[3])));
+}
+// 2^len of both halves, as a factor the compiler does not see through: it would make a shift and an addition of every
+// multiply-add by it.
+__device__ __forceinline__ u16x2 pk_power(uint32_t len2) {
+    uint32_t p = pk_u16((u16x2)((u16x2){1, 1} << as_u16x2(len2)));
+    asm("" : "+v"(p));
+    return as_u16x2(p);
 }
 
 // The two packs held in one register pair column: codes c[k] (k = token, two channels per word)
 // -> minima, widths and the two 64-bit pack words  sum (c_k - min) << ((15 - k) * len).
 __device__ __forceinline__ void build_pair(const uint32_t c[16], uint32_t &mn2, uint32_t &len2, uint32_t &mx2,
                                            uint64_t &w_lo, uint64_t &w_hi) {
-    u16x2 mn = as_u16x2(c[0]), mx = as_u16x2(c[0]);
-#pragma unroll
-    for (int k = 1; k < 16; k++) {
-        mn = __builtin_elementwise_min(mn, as_u16x2(c[k]));
-        mx = __builtin_elementwise_max(mx, as_u16x2(c[k]));
-    }
-    mn2 = pk_u16(mn);
-    mx2 = pk_u16(mx);
-    len2 = pk_bitlen4(pk_u16((u16x2)(mx - mn)));
-    const u16x2 one = {1, 1};
-    const u16x2 p = one << as_u16x2(len2);                       // 2^len per half
+    mn2 = pk_side16<false>(c);
+    mx2 = pk_side16<true>(c);
+    const u16x2 mn = as_u16x2(mn2), mx = as_u16x2(mx2), one = {1, 1};
+    len2 = pk_bitlen<4>(pk_u16((u16x2)(mx - mn)));
+    const u16x2 p = pk_power(len2);
     // quarter windows (4 tokens, 4 * len <= 16 bits), all arithmetic modulo 2^16 per half:
     //   sum c_k p^(3-k) - min (1 + p + p^2 + p^3)
     const u16x2 rep = ((p + one) * p + one) * p + one;
     const u16x2 mnrep = mn * rep;
+    // (the four windows side by side: each step waits for the one before)
+    u16x2 w[4];
     uint32_t qw[4];
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        u16x2 w = as_u16x2(c[4 * j]);
-        w = w * p + as_u16x2(c[4 * j + 1]);
-        w = w * p + as_u16x2(c[4 * j + 2]);
-        w = w * p + as_u16x2(c[4 * j + 3]);
-        qw[j] = pk_u16((u16x2)(w - mnrep));
-    }
+    for (int j = 0; j < 4; j++) w[j] = as_u16x2(c[4 * j]) * p + as_u16x2(c[4 * j + 1]);
+#pragma unroll
+    for (int j = 0; j < 4; j++) w[j] = w[j] * p + as_u16x2(c[4 * j + 2]);
+#pragma unroll
+    for (int j = 0; j < 4; j++) w[j] = w[j] * p + as_u16x2(c[4 * j + 3]);
+#pragma unroll
+    for (int j = 0; j < 4; j++) qw[j] = pk_u16((u16x2)(w[j] - mnrep));
     // 64-bit words: tokens 0..7 above tokens 8..15
     const uint32_t l0 = len2 & 0xFFFFu, l1 = len2 >> 16;
     const uint32_t a0 = ((qw[0] & 0xFFFFu) << (4u * l0)) | (qw[1] & 0xFFFFu), b0 = ((qw[2] & 0xFFFFu) << (4u * l0)) | (qw[3] & 0xFFFFu);
@@ -674,32 +691,18 @@ struct UnitPacksW {
     uint32_t payload;
 };
 
-// bit_length of both 16-bit halves, clamped to 6
-__device__ __forceinline__ uint32_t pk_bitlen6(uint32_t d) {
-    const u16x2 v = as_u16x2(d), one = {1, 1};
-    u16x2 l = __builtin_elementwise_min(v, one);
-#pragma unroll
-    for (int k = 1; k < 6; k++) l += __builtin_elementwise_min((u16x2)(v >> (uint16_t)k), one);
-    return pk_u16(l);
-}
-
+// four windows of l2 = 2 * len <= 12 bits
 __device__ __forceinline__ uint64_t join4(uint32_t e0, uint32_t e1, uint32_t e2, uint32_t e3, uint32_t l2) {
-    return ((((((uint64_t)e0 << l2) | e1) << l2) | e2) << l2) | e3;      // l2 = 2 * len
+    return ((uint64_t)((e0 << l2) | e1) << (2u * l2)) | ((e2 << l2) | e3);
 }
 
 __device__ __forceinline__ void build_pair_wide(const uint32_t c[16], uint32_t &mn2, uint32_t &len2, uint32_t &mx2,
                                                 uint64_t &lo_a, uint64_t &hi_a, uint64_t &lo_b, uint64_t &hi_b) {
-    u16x2 mn = as_u16x2(c[0]), mx = as_u16x2(c[0]);
-#pragma unroll
-    for (int k = 1; k < 16; k++) {
-        mn = __builtin_elementwise_min(mn, as_u16x2(c[k]));
-        mx = __builtin_elementwise_max(mx, as_u16x2(c[k]));
-    }
-    mn2 = pk_u16(mn);
-    mx2 = pk_u16(mx);
-    len2 = pk_bitlen6(pk_u16((u16x2)(mx - mn)));
-    const u16x2 one = {1, 1};
-    const u16x2 p = one << as_u16x2(len2);                       // 2^len per half
+    mn2 = pk_side16<false>(c);
+    mx2 = pk_side16<true>(c);
+    const u16x2 mn = as_u16x2(mn2), mx = as_u16x2(mx2), one = {1, 1};
+    len2 = pk_bitlen<6>(pk_u16((u16x2)(mx - mn)));
+    const u16x2 p = pk_power(len2);
     const u16x2 mnrep = mn * (p + one);
     uint32_t ew[8];                                              // tokens 2j, 2j+1: (c - min) p + (c' - min) < 2^12
 #pragma unroll
@@ -743,25 +746,59 @@ __device__ __forceinline__ void cell_packs(const uint2 xr[16], const TokPar *par
 template <bool WIDE> struct PacksOf { typedef UnitPacks type; };
 template <> struct PacksOf<true> { typedef UnitPacksW type; };
 
-// the 2 * len bytes of pack k at dst (2-byte aligned): one predicated 16-bit store per piece, written out (a loop
-// over the lane's own length costs a shift, a compare and the loop's control flow per piece)
+// the 2 * len bytes of pack k at dst (2-byte aligned, in LDS): one 16-bit store per piece by the lanes whose pack has that piece.
+// A longer pack has the pieces of a shorter one, so every compare narrows the execution mask of the one before and the mask
+// is put back once per pack.  Written as instructions: the compiler made a branch to a block of its own and one back
+// out of every predicated store, 32 of them a round.  It does not see these stores either: packs_put() stands before the barrier behind
+// the last ones.  (Behind a lane's last pack the s_nop fills up the five wait states that an exchange between lanes needs after a
+// vector instruction wrote the mask.)
+// The encoders are bound by the instructions they issue: these stores, the widths and windows above and the minima and maxima
+// below (fewer wait states) took 4 % off K, 4 % off V on 16 x 8 x 32768 tokens (fp16, rel 0.1: 322 -> 309, 352 -> 339 us), 3 and 7 % at
+// rel 0.05 with its wide packs (329 -> 318, 508 -> 475).
+__device__ __forceinline__ uint32_t lds_offset(const void *p) {
+    return (uint32_t)reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) void *)p);
+}
 __device__ __forceinline__ void put_pack(uint16_t *dst, const UnitPacks &u, int k) {
-    const uint32_t lo = (uint32_t)u.word[k], hi = (uint32_t)(u.word[k] >> 32), len = u.len[k];
-    if (len > 0u) dst[0] = (uint16_t)lo;
-    if (len > 1u) dst[1] = (uint16_t)(lo >> 16);
-    if (len > 2u) dst[2] = (uint16_t)hi;
-    if (len > 3u) dst[3] = (uint16_t)(hi >> 16);
+    uint64_t mask;
+    asm volatile("s_mov_b64 %0, exec\n\t"
+                 "v_cmpx_lt_u32_e32 vcc, 0, %4\n\t"
+                 "ds_write_b16 %1, %2\n\t"
+                 "v_cmpx_lt_u32_e32 vcc, 1, %4\n\t"
+                 "ds_write_b16_d16_hi %1, %2 offset:2\n\t"
+                 "v_cmpx_lt_u32_e32 vcc, 2, %4\n\t"
+                 "ds_write_b16 %1, %3 offset:4\n\t"
+                 "v_cmpx_lt_u32_e32 vcc, 3, %4\n\t"
+                 "ds_write_b16_d16_hi %1, %3 offset:6\n\t"
+                 "s_mov_b64 exec, %0"
+                 : "=&s"(mask)
+                 : "v"(lds_offset(dst)), "v"((uint32_t)u.word[k]), "v"((uint32_t)(u.word[k] >> 32)), "v"(u.len[k])
+                 : "vcc", "memory");
+    if (k == 3) asm volatile("s_nop 2");
 }
 __device__ __forceinline__ void put_pack(uint16_t *dst, const UnitPacksW &u, int k) {
-    const unsigned __int128 wd = ((unsigned __int128)u.hi[k] << (8u * u.len[k])) | u.lo[k];
-    const uint32_t d0 = (uint32_t)wd, d1 = (uint32_t)(wd >> 32), d2 = (uint32_t)(wd >> 64), len = u.len[k];
-    if (len > 0u) dst[0] = (uint16_t)d0;
-    if (len > 1u) dst[1] = (uint16_t)(d0 >> 16);
-    if (len > 2u) dst[2] = (uint16_t)d1;
-    if (len > 3u) dst[3] = (uint16_t)(d1 >> 16);
-    if (len > 4u) dst[4] = (uint16_t)d2;
-    if (len > 5u) dst[5] = (uint16_t)(d2 >> 16);
+    const uint32_t s = 8u * u.len[k];                            // (at most 48; without pieces nothing is stored)
+    const uint64_t w = u.lo[k] | (u.hi[k] << s);
+    uint64_t mask;
+    asm volatile("s_mov_b64 %0, exec\n\t"
+                 "v_cmpx_lt_u32_e32 vcc, 0, %5\n\t"
+                 "ds_write_b16 %1, %2\n\t"
+                 "v_cmpx_lt_u32_e32 vcc, 1, %5\n\t"
+                 "ds_write_b16_d16_hi %1, %2 offset:2\n\t"
+                 "v_cmpx_lt_u32_e32 vcc, 2, %5\n\t"
+                 "ds_write_b16 %1, %3 offset:4\n\t"
+                 "v_cmpx_lt_u32_e32 vcc, 3, %5\n\t"
+                 "ds_write_b16_d16_hi %1, %3 offset:6\n\t"
+                 "v_cmpx_lt_u32_e32 vcc, 4, %5\n\t"
+                 "ds_write_b16 %1, %4 offset:8\n\t"
+                 "v_cmpx_lt_u32_e32 vcc, 5, %5\n\t"
+                 "ds_write_b16_d16_hi %1, %4 offset:10\n\t"
+                 "s_mov_b64 exec, %0"
+                 : "=&s"(mask)
+                 : "v"(lds_offset(dst)), "v"((uint32_t)w), "v"((uint32_t)(w >> 32)), "v"((uint32_t)(u.hi[k] >> ((64u - s) & 63u))), "v"(u.len[k])
+                 : "vcc", "memory");
+    if (k == 3) asm volatile("s_nop 2");
 }
+__device__ __forceinline__ void packs_put() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 // Emit one analysed unit at blk[unit_off] (the K layout: lane t's packs sit where they were computed).
 template <class U>
@@ -826,7 +863,8 @@ __device__ __forceinline__ void copy_out32(uint8_t *dst, const uint8_t *src, uin
 // token l / 4 (all four lanes of a quad the same): ~120 vector instructions instead of a second pass over the rows.
 // (The packed min / max are written as instructions, see pk_min_h; a lane exchange must not read a register that a
 // vector instruction wrote less than two instructions earlier, and the compiler does not see into the assembly, so
-// these carry their own two wait states.)
+// these carry their own two wait states, one for four of them where four are independent: with two behind each of the 62 a round
+// they held a wavefront for 250 cycles.)
 // KEYS: the operands are order keys of bf16 values (bf16_keys), compared as signed 16-bit integers.
 template <bool MAX, bool KEYS>
 __device__ __forceinline__ uint32_t pk_sel_x(uint32_t a, uint32_t b) {
@@ -862,15 +900,52 @@ __device__ __forceinline__ void minmax_unword(uint32_t w, float &mn, float &mx) 
     mn = T16<DT>::from_bits(w & 0xFFFFu);
     mx = T16<DT>::from_bits(w >> 16);
 }
+// Four of them with the wait states once, behind the last: a[i] = min / max(a[i], b[i]).
 template <bool MAX, bool KEYS>
-__device__ __forceinline__ uint32_t swap32_sel(uint32_t a, uint32_t b) {
-    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
-    return pk_sel_x<MAX, KEYS>((uint32_t)r[0], (uint32_t)r[1]);
+__device__ __forceinline__ void pk_sel4(uint32_t &a0, uint32_t &a1, uint32_t &a2, uint32_t &a3, uint32_t b0, uint32_t b1, uint32_t b2, uint32_t b3) {
+#define PKV_SEL4(op)                                                                                                                      \
+    asm(op " %0, %0, %4\n\t" op " %1, %1, %5\n\t" op " %2, %2, %6\n\t" op " %3, %3, %7\n\ts_nop 1"                                         \
+        : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3) : "v"(b0), "v"(b1), "v"(b2), "v"(b3))
+    if (KEYS) {
+        if (MAX) PKV_SEL4("v_pk_max_i16");
+        else PKV_SEL4("v_pk_min_i16");
+    } else {
+        if (MAX) PKV_SEL4("v_pk_max_f16");
+        else PKV_SEL4("v_pk_min_f16");
+    }
+#undef PKV_SEL4
 }
-template <bool MAX, bool KEYS>
-__device__ __forceinline__ uint32_t swap16_sel(uint32_t a, uint32_t b) {
-    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
-    return pk_sel_x<MAX, KEYS>((uint32_t)r[0], (uint32_t)r[1]);
+// v[i] = min / max over the two dwords of row xr[first + i], rows first .. first + 3
+template <int DT, bool MAX>
+__device__ __forceinline__ void rows_sel4(const uint2 xr[16], int first, uint32_t (&v)[4]) {
+    constexpr bool KEYS = DT != PKV_F16;
+    if (KEYS) {
+        uint32_t b[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = bf16_keys(xr[first + i].x), b[i] = bf16_keys(xr[first + i].y);
+        pk_sel4<MAX, true>(v[0], v[1], v[2], v[3], b[0], b[1], b[2], b[3]);
+    } else {
+#define PKV_ROWS4(op)                                                                                                                     \
+    asm(op " %0, %4, %5\n\t" op " %1, %6, %7\n\t" op " %2, %8, %9\n\t" op " %3, %10, %11\n\ts_nop 1"                                       \
+        : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])                                                                               \
+        : "v"(xr[first].x), "v"(xr[first].y), "v"(xr[first + 1].x), "v"(xr[first + 1].y), "v"(xr[first + 2].x), "v"(xr[first + 2].y),        \
+          "v"(xr[first + 3].x), "v"(xr[first + 3].y))
+        if (MAX) PKV_ROWS4("v_pk_max_f16");
+        else PKV_ROWS4("v_pk_min_f16");
+#undef PKV_ROWS4
+    }
+}
+// a[i] = min / max after halves of the wavefront (rows of 16) of a[i] and b[i] have changed places
+template <bool MAX, bool KEYS, bool HALVES>
+__device__ __forceinline__ void swap_sel4(uint32_t (&a)[4], const uint32_t (&b)[4]) {
+    uint32_t o[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const auto r = HALVES ? __builtin_amdgcn_permlane32_swap(a[i], b[i], false, false) : __builtin_amdgcn_permlane16_swap(a[i], b[i], false, false);
+        a[i] = (uint32_t)r[0];
+        o[i] = (uint32_t)r[1];
+    }
+    pk_sel4<MAX, KEYS>(a[0], a[1], a[2], a[3], o[0], o[1], o[2], o[3]);
 }
 // lanes whose bank is in HI_BANKS keep b and meet the partner's b, the others keep a and meet the partner's a;
 // CTRL_LO / CTRL_HI: how the low / high banks read their partner
@@ -885,14 +960,14 @@ __device__ __forceinline__ uint32_t row_step_sel(uint32_t a, uint32_t b) {
 template <int DT, bool MAX>
 __device__ __forceinline__ uint32_t cell_token_side(const uint2 xr[16]) {
     constexpr bool KEYS = DT != PKV_F16;
-    uint32_t v[16];
-#pragma unroll
-    for (int k = 0; k < 16; k++)
-        v[k] = KEYS ? pk_sel_x<MAX, true>(bf16_keys(xr[k].x), bf16_keys(xr[k].y)) : pk_sel_x<MAX, false>(xr[k].x, xr[k].y);
-#pragma unroll
-    for (int k = 0; k < 8; k++) v[k] = swap32_sel<MAX, KEYS>(v[k], v[k + 8]);          // lanes 0..31: token k, lanes 32..63: token k + 8
-#pragma unroll
-    for (int k = 0; k < 4; k++) v[k] = swap16_sel<MAX, KEYS>(v[k], v[k + 4]);          // row rho: token k + 4 rho
+    uint32_t v[4], w[4], q[4];
+    rows_sel4<DT, MAX>(xr, 0, v);
+    rows_sel4<DT, MAX>(xr, 8, q);
+    swap_sel4<MAX, KEYS, true>(v, q);                      // lanes 0..31: token k, lanes 32..63: token k + 8
+    rows_sel4<DT, MAX>(xr, 4, w);
+    rows_sel4<DT, MAX>(xr, 12, q);
+    swap_sel4<MAX, KEYS, true>(w, q);
+    swap_sel4<MAX, KEYS, false>(v, w);                     // row rho: token k + 4 rho
 #pragma unroll
     for (int k = 0; k < 2; k++) v[k] = row_step_sel<MAX, KEYS, 0x128, 0x128, 0xC>(v[k], v[k + 2]);   // lanes 8..15 of a row: token k + 2 + 4 rho
     const uint32_t r = row_step_sel<MAX, KEYS, 0x104, 0x114, 0xA>(v[0], v[1]);         // banks 1, 3: the odd token; token = lane / 4
@@ -920,14 +995,15 @@ __device__ __forceinline__ void cell_token_minmax(const uint2 xr[16], float &mn,
 template <int DT, bool MAX>
 __device__ __forceinline__ uint32_t cell_token_side_halves(const uint2 xr[16], bool odd_pair) {
     constexpr bool KEYS = DT != PKV_F16;
-    uint32_t v[16];
+    uint32_t v[4], w[4], q[4];
+    rows_sel4<DT, MAX>(xr, 0, v);
+    rows_sel4<DT, MAX>(xr, 8, q);
+    swap_sel4<MAX, KEYS, false>(v, q);                     // odd rows: token k + 8
+    rows_sel4<DT, MAX>(xr, 4, w);
+    rows_sel4<DT, MAX>(xr, 12, q);
+    swap_sel4<MAX, KEYS, false>(w, q);
 #pragma unroll
-    for (int k = 0; k < 16; k++)
-        v[k] = KEYS ? pk_sel_x<MAX, true>(bf16_keys(xr[k].x), bf16_keys(xr[k].y)) : pk_sel_x<MAX, false>(xr[k].x, xr[k].y);
-#pragma unroll
-    for (int k = 0; k < 8; k++) v[k] = swap16_sel<MAX, KEYS>(v[k], v[k + 8]);          // odd rows: token k + 8
-#pragma unroll
-    for (int k = 0; k < 4; k++) v[k] = row_step_sel<MAX, KEYS, 0x128, 0x128, 0xC>(v[k], v[k + 4]);   // lanes 8..15 of a row: + 4
+    for (int k = 0; k < 4; k++) v[k] = row_step_sel<MAX, KEYS, 0x128, 0x128, 0xC>(v[k], w[k]);       // lanes 8..15 of a row: + 4
 #pragma unroll
     for (int k = 0; k < 2; k++) v[k] = row_step_sel<MAX, KEYS, 0x104, 0x114, 0xA>(v[k], v[k + 2]);   // banks 1, 3: + 2
     // lanes 2, 3 of a quad: + 1 (no bank mask reaches inside a quad: selects, and the exchange as a quad permute)
@@ -1123,6 +1199,7 @@ __global__ void __launch_bounds__(256) k_quant_encode_cells_kernel(
         for (int d = 32; d >= 1; d >>= 1) cmax_all = max(cmax_all, __shfl_xor(cmax_all, d, 64));
         if ((tid & 63) == 0) atomicMax(&st->max_code, cmax_all);
     }
+    packs_put();
     __syncthreads();
     const uint32_t bytes = blk_off[H];
     if (tid < 64) {
@@ -1234,6 +1311,7 @@ __global__ void __launch_bounds__(256) k_quant_encode_rounds_kernel(
         for (int d = 32; d >= 1; d >>= 1) cmax_all = max(cmax_all, __shfl_xor(cmax_all, d, 64));
         if ((tid & 63) == 0) atomicMax(&st->max_code, cmax_all);
     }
+    packs_put();
     __syncthreads();
     const uint32_t bytes = blk_off[nblk];
     if (tid < 64) {
@@ -1424,6 +1502,7 @@ __global__ void __launch_bounds__(512) v_quant_encode_rounds_kernel(
         for (int d = 32; d >= 1; d >>= 1) cmax_all = max(cmax_all, __shfl_xor(cmax_all, d, 64));
         if ((tid & 63) == 0) atomicMax(&st->max_code, cmax_all);
     }
+    packs_put();
     __syncthreads();
     const int nblk = 2 * nheads;
     const uint32_t bytes = blk_off[nblk];
@@ -1652,6 +1731,7 @@ __global__ void __launch_bounds__(512) v_quant_encode_cells_kernel(
         for (int d = 32; d >= 1; d >>= 1) cmax_all = max(cmax_all, __shfl_xor(cmax_all, d, 64));
         if ((tid & 63) == 0) atomicMax(&st->max_code, cmax_all);
     }
+    packs_put();
     __syncthreads();
     const int nblk = 2 * H;
     const uint32_t bytes = blk_off[nblk];
@@ -1764,6 +1844,7 @@ __global__ void __launch_bounds__(256) k_code_cells_kernel(
         unit_emit_any(blk, my_off, t, g, u);
         my_off += usz;
     }
+    packs_put();
     __syncthreads();
     const uint32_t bytes = blk_off[kSubBlocks];
     if (tid < 64) {
@@ -1862,6 +1943,7 @@ __global__ void __launch_bounds__(512) v_code_cells_kernel(
             run_off = 0;
         }
     }
+    packs_put();
     __syncthreads();
     const uint32_t bytes = blk_off[16];
     if (tid < 64) {

@@ -210,6 +210,7 @@ __device__ __forceinline__ void k_write_once(const OnceSide &a, OnceLds<NT> &l, 
         unit_emit_any(blk, at, t, g, u);
     }
     if (checked) once_max_code(a.st, j < nblk ? cmax : 0u, a.W);
+    packs_put();
     __syncthreads();
     if (!once_place(l, a, c, counted, idx, first, nblk)) return;
     const int q = tid >> 7;                                // 128 threads copy a block
@@ -333,6 +334,7 @@ __device__ __forceinline__ void v_write_once(const OnceSide &a, OnceLds<NT> &l, 
         }
     }
     if (checked) once_max_code(a.st, j < H ? cmax : 0u, a.W);
+    packs_put();
     __syncthreads();
     if (!once_place(l, a, c, counted, idx, first, nblk)) return;
     // a half-wavefront copies a unit, the first of a block its header of cumulative unit sizes
