@@ -900,20 +900,26 @@ int pkv::attn_decode_impl(const pkv_attn_args *a, float *ms_out, hipStream_t s, 
         // only start once others have finished, each with a full share of tiles (12 sequences x 8 heads: 11 members,
         // 1056 workgroups, 115 us per step against 99 us with 10 members); so both roundings are priced as
         // generations x tiles per member and the cheaper one is taken, the finer cut on a tie.
-        // (as many members as are resident at once: widths 5 and 6 run two workgroups per CU -- 193 us per step with
-        // 512 members against 199 us with 1024 in two generations, 6 bits 201 against 218 us -- and groups of eight
-        // query heads three: 156 against 165 us)
-        const int resident = PKV_SPLIT_TARGET / 4 * PKV_DMA_WAVES((a->k_bits > a->v_bits ? a->k_bits : a->v_bits), G);
-        if (dma_path && 4 * (int64_t)pairs * win_members > resident) win_members = 0;
-        const int target = resident - (dma_path ? pairs * win_members : 0);
+        // (as many members as are resident at once; groups of eight query heads run three workgroups per CU: 156 against
+        // 165 us with four.)  Width 5 runs three, but two when that is the cheaper cut: with three a tile takes 1.3 times as
+        // long and a member's start half a tile more, and up to eight members merge by themselves (merge_head).  5-bit
+        // steps, three -> two: 32 pairs x 64 tiles (22 members of three tiles, 16 of four) 19.95 -> 19.0 us, 64 x 64 (six, eight)
+        // 30.8 -> 29.3; the other way round 24 x 86 with a window (three, five) 20.3 and 21.7, 256 x 64 83 and 94, 128 x 256 149 and 168.
+        const int bits = a->k_bits > a->v_bits ? a->k_bits : a->v_bits;
+        const int most = !dma_path && bits == 5 && G <= 4 ? 2 : PKV_DMA_RESIDENT(bits, G), least = bits == 5 && most == 3 ? 2 : most;
+        if (dma_path && 4 * (int64_t)pairs * win_members > PKV_SPLIT_TARGET / 4 * most) win_members = 0;
         long best_cost = -1;
-        for (int up = 1; up >= 0; up--) {
-            int want = up ? (target + pairs - 1) / pairs : target / pairs;
-            if (want < 1) want = 1;
-            if (want > n_tiles) want = n_tiles;
-            const int t = (n_tiles + want - 1) / want, n = (n_tiles + t - 1) / t;
-            const long cost = (((long)pairs * n + target - 1) / target) * (long)t;
-            if (best_cost < 0 || cost < best_cost) { best_cost = cost; tps = t; nsplit = n; }
+        for (int per_cu = most; per_cu >= least; per_cu--) {
+            const int target = PKV_SPLIT_TARGET / 4 * per_cu - (dma_path ? pairs * win_members : 0);
+            for (int up = 1; up >= 0; up--) {
+                int want = up ? (target + pairs - 1) / pairs : target / pairs;
+                if (want < 1) want = 1;
+                if (want > n_tiles) want = n_tiles;
+                const int t = (n_tiles + want - 1) / want, n = (n_tiles + t - 1) / t;
+                const long each = per_cu > least ? 13l * t + 5 : 10l * t;
+                const long cost = (((long)pairs * n + target - 1) / target) * each;
+                if (best_cost < 0 || cost < best_cost) { best_cost = cost; tps = t; nsplit = n; }
+            }
         }
     }
     const bool shared_window = dma_path && win_members == 0 && a->T_w > 0;      // every split writes a piece, empty or not

@@ -32,8 +32,8 @@ namespace pkv {
 // drift apart instead of competing stage for stage -- wavefronts reach their barriers earlier and the vector ALUs
 // idle less: 142.5 us with equal priorities, 129.5 us with (K 1, softmax 2, copy issue 0, V 3) on the 16 x 8 x
 // 32768-token workload (a sweep over the 2-bit range; copy issue lowest was best).  The setting does not carry over
-// to fewer resident workgroups: with three (groups of 8) equal priorities are best (197 us against 218), with two
-// (widths 5 and 6) the K stage first (211 us against 218).
+// to fewer resident workgroups: with three (groups of 8) equal priorities are best (197 us against 218); with three or
+// two of widths 5 and 6 the K stage first (5 bits: 148 us; equal ones 159, those of four per CU 150 to 153).
 template <int G, bool WIDE> struct StagePrio {                       // 4 workgroups per CU
     static constexpr int K = 1, S = 2, D = 0, V = 3;                 // K stage, parse + softmax, copy issue and waits, V stage
 };
@@ -199,48 +199,64 @@ __device__ __forceinline__ void pair_windows(const UnitPairs &u, uint32_t win01[
     }
 }
 
-// Widths 5 and 6 (this library's extension of the format): a quarter of a pack no longer fits a 16-bit lane, so the
-// windows hold TWO tokens each.  e01[e] = tokens 2e, 2e+1 of packs 0 and 1 in the low / high 16 bits (token 2e on
-// top), e23 likewise; bits above 2*len in a half are other tokens' fields, every consumer masks.
+// Widths 5 and 6 (this library's extension of the format): a pack's word is up to 12 bytes long and a quarter of it no
+// longer fits a 16-bit lane, so the words stay as they are until a stage uses them and its windows hold TWO tokens each.
 struct UnitWide {
-    uint32_t e01[8], e23[8];
+    uint32_t word[4][3];
     uint32_t len01, len23;
     uint32_t mins;
 };
 
-// The eight two-token windows of the four packs whose words start at byte pay0 + 2 * off2[i] of `base`.  A word is
-// up to 12 bytes long, so it is not assembled: each quarter (four tokens, 4 * len bits starting (3 - q) * 4 * len
-// bits into the word, i.e. at a byte or a nibble boundary) is fetched on its own as the 32 bits at its byte
-// address -- two aligned dwords and a byte funnel shift -- and moved down by the odd nibble.
-__device__ __forceinline__ void wide_windows(const uint8_t *base, uint32_t pay0, const uint32_t off2[4], UnitWide &u) {
-    const uint32_t len[4] = {u.len01 & 0xFFFFu, u.len01 >> 16, u.len23 & 0xFFFFu, u.len23 >> 16};
+// 96 bits at byte offset `off` (even) of an LDS array whose base is 4-byte aligned, like lds_word64.
+__device__ __forceinline__ void lds_word96(const uint8_t *base, uint32_t off, uint32_t word[3]) {
+    const uint32_t *q = reinterpret_cast<const uint32_t *>(base + (off & ~3u));
+    const uint32_t d0 = q[0], d1 = q[1], d2 = q[2], d3 = q[3];
+    word[0] = __builtin_amdgcn_alignbyte(d1, d0, off);
+    word[1] = __builtin_amdgcn_alignbyte(d2, d1, off);
+    word[2] = __builtin_amdgcn_alignbyte(d3, d2, off);
+}
+
+// e01[e] = tokens 2e, 2e+1 of packs 0 and 1 in the low / high 16 bits (token 2e on top), e23 likewise; bits above 2 len
+// in a half are other tokens' fields, every consumer masks.  A quarter (four tokens) is 4 len <= 24 bits; the lower two
+// lie in the word's first 8 len <= 48 bits, the upper two as far into the word moved down by 8 len bits = len bytes.
+__device__ __forceinline__ void wide_windows(const UnitWide &u, uint32_t e01[8], uint32_t e23[8]) {
+    const uint32_t s2[2] = {u.len01 << 1, u.len23 << 1}, s4[2] = {u.len01 << 2, u.len23 << 2};
     uint32_t hi[4][4], lo[4][4];       // [pack][quarter]: tokens 4q, 4q+1 and 4q+2, 4q+3
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        const uint32_t a = pay0 + 2u * off2[i], L = len[i], nib = (L & 1u) * 4u;
-        const uint32_t at[4] = {a + ((3u * L) >> 1), a + L, a + (L >> 1), a};      // byte address of quarter q
+        const uint32_t L = (i & 1) ? (i < 2 ? u.len01 : u.len23) >> 16 : (i < 2 ? u.len01 : u.len23) & 0xFFFFu;
+        const uint32_t a4 = (i & 1) ? s4[i >> 1] >> 16 : s4[i >> 1], a2 = (i & 1) ? s2[i >> 1] >> 16 : s2[i >> 1];
+        const uint32_t *w = u.word[i];
+        const bool far = L >= 4u;      // the upper half starts in the second dword
+        const uint32_t u0 = __builtin_amdgcn_alignbyte(far ? w[2] : w[1], far ? w[1] : w[0], L);
+        const uint32_t u1 = w[2] >> ((8u * L) & 31u);      // (below width 4 the upper half is in u0 altogether)
+        const uint32_t v[4] = {__builtin_amdgcn_alignbit(u1, u0, a4), u0, __builtin_amdgcn_alignbit(w[1], w[0], a4), w[0]};
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const uint32_t *dq = reinterpret_cast<const uint32_t *>(base + (at[q] & ~3u));
-            uint32_t v = __builtin_amdgcn_alignbyte(dq[1], dq[0], at[q]);
-            if (q == 0 || q == 2) v >>= nib;
-            lo[i][q] = v;
-            hi[i][q] = v >> (2u * L);
+            lo[i][q] = v[q];
+            hi[i][q] = v[q] >> (a2 & 31u);
         }
     }
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-        u.e01[2 * q] = __builtin_amdgcn_perm(hi[1][q], hi[0][q], 0x05040100u);
-        u.e01[2 * q + 1] = __builtin_amdgcn_perm(lo[1][q], lo[0][q], 0x05040100u);
-        u.e23[2 * q] = __builtin_amdgcn_perm(hi[3][q], hi[2][q], 0x05040100u);
-        u.e23[2 * q + 1] = __builtin_amdgcn_perm(lo[3][q], lo[2][q], 0x05040100u);
+        e01[2 * q] = __builtin_amdgcn_perm(hi[1][q], hi[0][q], 0x05040100u);
+        e01[2 * q + 1] = __builtin_amdgcn_perm(lo[1][q], lo[0][q], 0x05040100u);
+        e23[2 * q] = __builtin_amdgcn_perm(hi[3][q], hi[2][q], 0x05040100u);
+        e23[2 * q + 1] = __builtin_amdgcn_perm(lo[3][q], lo[2][q], 0x05040100u);
     }
 }
 
 // Wavefronts per SIMD the register allocation aims for: four workgroups per CU for the reference's widths (three for
-// groups of 8 query heads); the two-token windows of widths 5 and 6 need about 210 VGPRs, two workgroups per CU
-// (at three, 168 VGPRs, the compiler spills 47 of them and the kernel is 2.4 times slower).
-#define PKV_DMA_WAVES(KW, G) ((KW) > 4 ? ((G) <= 4 ? 2 : 1) : ((G) <= 4 ? 4 : 3))
+// groups of 8 query heads), two for widths 5 and 6.  With their words kept as they lie these take 137 to 160 registers (184
+// for groups of 8), so that three workgroups of width 5 fit a CU all the same; told to aim for three the compiler comes to
+// 152 of them, but with three times the spilled scalars, and every step is 0.4 us longer.  (While a tile's windows were formed
+// with its parse, a tile ahead, the 5-bit kernel held 206 registers and fetched each quarter of a word on its own, eight
+// reads of LDS a pack instead of four dwords: 199 us a step of 16 x 8 x 32768 tokens, now 148; 32 x 8 x 8192 with a window 110,
+// now 83.)
+#define PKV_DMA_WAVES(KW, G) ((KW) > 4 ? 2 : ((G) <= 4 ? 4 : 3))
+// Workgroups per CU that the cache is cut for (three of width 5 take 53 KB of its LDS each, width 6 takes 61; groups of 8 of
+// both keep the cut, and with it the size of their partials, that they had while one of them filled a CU's registers).
+#define PKV_DMA_RESIDENT(KW, G) ((KW) > 4 ? ((G) > 4 ? 1 : (KW) == 5 ? 3 : 2) : ((G) <= 4 ? 4 : 3))
 template <bool WIDE> struct UnitOf { typedef UnitPairs type; };
 template <> struct UnitOf<true> { typedef UnitWide type; };
 
@@ -541,13 +557,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PKV_DM
         const uint32_t kabs = (uint32_t)(slot * Geo::kSlot + kj * Geo::kRegion) + kpay0;
         const uint32_t vabs = (uint32_t)(slot * Geo::kSlot + (2 + kj) * Geo::kRegion) + vpay0;
         if constexpr (KWIDE) {
-            wide_windows(kb, kpay0, koff, kr);
+#pragma unroll
+            for (int i = 0; i < 4; i++) lds_word96(ring, kabs + 2u * koff[i], kr.word[i]);
         } else {
 #pragma unroll
             for (int i = 0; i < 4; i++) kr.word[i] = lds_word64(ring, kabs + 2u * koff[i]);
         }
         if constexpr (VWIDE) {
-            wide_windows(vb, vpay0, voff, vr);
+#pragma unroll
+            for (int i = 0; i < 4; i++) lds_word96(ring, vabs + 2u * voff[i], vr.word[i]);
         } else {
 #pragma unroll
             for (int i = 0; i < 4; i++) vr.word[i] = lds_word64(ring, vabs + 2u * voff[i]);
@@ -568,8 +586,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PKV_DM
             constexpr int TPW = KTPW, NWIN = KNWIN;
             uint32_t w01[NWIN], w23[NWIN];
             if constexpr (KWIDE) {
-#pragma unroll
-                for (int e = 0; e < NWIN; e++) { w01[e] = kr.e01[e]; w23[e] = kr.e23[e]; }
+                wide_windows(kr, w01, w23);
             } else {
                 pair_windows(kr, w01, w23);
             }
@@ -758,8 +775,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PKV_DM
         const int seg = hw & 1;
         uint32_t w01[NWIN], w23[NWIN];
         if constexpr (VWIDE) {
-#pragma unroll
-            for (int e = 0; e < NWIN; e++) { w01[e] = vr.e01[e]; w23[e] = vr.e23[e]; }
+            wide_windows(vr, w01, w23);
         } else {
             pair_windows(vr, w01, w23);
         }
@@ -878,13 +894,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PKV_DM
         if (!(PKV_ATTN_PROBE & 4)) softmax_stage(slot_c, kt);
         // the pack words of tile t1 are put together here, not wherever the compiler finds room before their first
         // use: it kept the three raw dwords of every word alive through the V stage (24 registers instead of 16)
-        if constexpr (!KWIDE) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) asm volatile("" : "+v"(knext.word[i]));
+        for (int i = 0; i < 4; i++) {
+            if constexpr (KWIDE) asm volatile("" : "+v"(knext.word[i][0]), "+v"(knext.word[i][1]), "+v"(knext.word[i][2]));
+            else asm volatile("" : "+v"(knext.word[i]));
         }
-        if constexpr (!VWIDE) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) asm volatile("" : "+v"(vnext.word[i]));
+        for (int i = 0; i < 4; i++) {
+            if constexpr (VWIDE) asm volatile("" : "+v"(vnext.word[i][0]), "+v"(vnext.word[i][1]), "+v"(vnext.word[i][2]));
+            else asm volatile("" : "+v"(vnext.word[i]));
         }
         __builtin_amdgcn_s_setprio(0);
         PKV_LDS_BARRIER();                                    // publishes the weights; slot s is free, tile t1 is parsed

@@ -402,6 +402,28 @@ def test_attn_decode_wide_codes(cuda, rel, bits, dtype):
     _say("  fast vs plain kernel: max diff", (outs[0] - outs[1]).abs().max().item())
 
 
+@pytest.mark.parametrize("rel,bits", [(0.05, 5), (0.03, 6)])
+@pytest.mark.parametrize("B,Hkv,T,Tw", [(1, 1, 128, 0), (1, 3, 384, 1), (2, 8, 2176, 64), (4, 8, 8192, 0), (3, 8, 11008, 137)])
+def test_attn_decode_wide_words_of_every_width(cuda, rel, bits, B, Hkv, T, Tw):
+    """Packs of every width from 0 to 6 side by side (channels from constant to full range): the halves and quarters of a
+    word start at every byte and nibble that they can.  From one tile up to the cuts of two and of three workgroups a CU;
+    the fast kernel against the plain one, which decodes codes one by one."""
+    g = torch.Generator(device=cuda).manual_seed(189)
+    x = torch.randn(2, B, Hkv, T + Tw, 128, generator=g, device=cuda)
+    x *= torch.tensor([0.0, 0.02, 0.05, 0.1, 0.2, 0.4, 1.0, 1.0], device=cuda).repeat(16)
+    k, v = x.to(torch.float16)
+    q = torch.randn(B, 4 * Hkv, 128, generator=g, device=cuda).to(torch.float16)
+    ke = ops.k_quant_encode(k[:, :, :T].contiguous(), rel)
+    ve = ops.v_quant_encode(v[:, :, :T].contiguous(), rel)
+    assert ke["bits"] == bits and ve["bits"] == bits
+    kw, vw = (k[:, :, T:].contiguous(), v[:, :, T:].contiguous()) if Tw else (None, None)
+    _say("every width", bits, B, Hkv, T, Tw)
+    fast = ops.attn_decode(q, ke, ve, kw, vw).float()
+    plain = ops.attn_decode(q, ke, ve, kw, vw, variant=1).float()
+    # as between the kernels above: twice the allowance of the faster one + an output rounding
+    assert (fast - plain).abs().max().item() <= 2 * 5e-4 + 2 ** -10 * plain.abs().max().item()
+
+
 @pytest.mark.parametrize("hq", [4, 8, 32])
 def test_attn_decode_wide_codes_group_sizes(cuda, hq):
     """The 5-bit path for groups of 1, 2 and 8 query heads per KV head (the case above has 4), no tail window."""
