@@ -1549,20 +1549,26 @@ __global__ void __launch_bounds__(512) v_quant_encode_rounds_kernel(
 // PERM: the tokens in the order of a repacking, as in the round-major kernel; with scale_in / zero_in (the tokens'
 // parameters in the order of x, known from the pass that made the order) nothing is left to exchange and an
 // iteration has no barrier at all.
+// Wide packs: the sixteen blocks' worst cases fill more than half of a CU's LDS, so that one workgroup is resident, and takes
+// the two 64-token segments of its blocks side by side, sixteen wavefronts in two iterations instead of eight in four: eight
+// wavefronts a CU left it waiting for its loads.  16 x 8 x 32768 tokens of fp16 V at rel 0.05: 475 -> 425 us (bf16 521 -> 463, rel 0.03
+// 487 -> 436), from a code matrix 284 -> 225, 3 x 8 x 11008 70.6 -> 60.7 and 44.9 -> 38.2.
+__host__ __device__ constexpr int v_cell_segs(bool wide) { return wide ? 2 : 1; }
 template <int DT, bool WIDE, bool PERM, bool XCH = false, bool STRIDED = false>
-__global__ void __launch_bounds__(512) v_quant_encode_cells_kernel(
+__global__ void __launch_bounds__(512 * v_cell_segs(WIDE)) v_quant_encode_cells_kernel(
     const uint16_t *__restrict__ x, int B, int H, int T, const XRows xs, float rel, uint16_t *__restrict__ scale,
     uint16_t *__restrict__ zero, uint8_t *__restrict__ stream, uint64_t capacity, uint32_t *__restrict__ info,
     ScanState *st, int W, uint32_t ngroups, uint32_t unit_slot, uint64_t base, int par_stride,
     const uint32_t *__restrict__ perm, int perm_block, const uint16_t *__restrict__ scale_in,
     const uint16_t *__restrict__ zero_in, const Stagger stagger, int nsg = 1, uint64_t *xw = nullptr) {
+    constexpr int SEGS = v_cell_segs(WIDE), ITS = 4 / SEGS;
     extern __shared__ __align__(16) uint8_t gbuf[];        // 16 blocks x 4 units x unit_slot bytes
     __shared__ uint32_t s_idx;
     __shared__ uint64_t s_off;
     __shared__ uint32_t blk_off[17];
     __shared__ uint16_t s_usz[16][4];
-    __shared__ __attribute__((aligned(16))) TokPar s_par[8 * 32];       // [wavefront][token of the iteration]
-    __shared__ uint32_t s_mm[2][8][32];                                  // [iteration parity][wavefront][token]: minmax_word
+    __shared__ __attribute__((aligned(16))) TokPar s_par[SEGS * 8 * 32];       // [wavefront][token of the iteration]
+    __shared__ uint32_t s_mm[2][SEGS * 8][32];                           // [iteration parity][wavefront][token]: minmax_word
     const int tid = threadIdx.x;
     stagger_first_generation(stagger);
     if (tid == 0) s_idx = atomicAdd(&st->ticket, 1u);
@@ -1575,7 +1581,7 @@ __global__ void __launch_bounds__(512) v_quant_encode_cells_kernel(
     const uint32_t sgi = XCH ? gidx % (uint32_t)nsg : 0u;
     const int hbase = XCH ? 8 * (int)sgi : 0;
     if (XCH) H = min(8, H_all - hbase);
-    const int j = tid >> 6, rp = (tid >> 5) & 1, t = tid & 31, wave = j, lane = tid & 63;
+    const int wave = tid >> 6, j = wave & 7, seg = wave >> 3, rp = (tid >> 5) & 1, t = tid & 31, lane = tid & 63;
     const uint32_t grp = XCH ? gidx / (uint32_t)nsg : gidx;
     const uint32_t cb = grp / (uint32_t)B, b = grp % (uint32_t)B;
     const size_t tok0 = (size_t)cb * 128;
@@ -1583,9 +1589,9 @@ __global__ void __launch_bounds__(512) v_quant_encode_cells_kernel(
     const uint32_t meta = (uint32_t)(g.mins_bytes + g.lens_bytes);
     const bool active = j < H;
     const int jc = min(j, H - 1);
-    const TokPar *my_par = (XCH ? s_par : s_par + 32 * wave) + 16 * rp;
+    const TokPar *my_par = s_par + 32 * (XCH ? seg : wave) + 16 * rp;
     const int blkid = 2 * j + (t >> 4), w = (t >> 3) & 1, m = t & 7;
-    for (uint32_t i = tid; i < 64u * (meta / 4u); i += 512)                 // metadata areas start as zeros
+    for (uint32_t i = tid; i < 64u * (meta / 4u); i += 512 * SEGS)                 // metadata areas start as zeros
         reinterpret_cast<uint32_t *>(gbuf + (size_t)(i / (meta / 4u)) * unit_slot)[i % (meta / 4u)] = 0u;
     uint32_t run_off = 0;
     uint32_t cmax_all = 0;
@@ -1596,7 +1602,8 @@ __global__ void __launch_bounds__(512) v_quant_encode_cells_kernel(
     const bool known = PERM && scale_in != nullptr;              // uniform
     if (known) __syncthreads();                                  // the metadata zeros are in place before the first OR (no barrier below)
 #pragma unroll 1
-    for (int it = 0; it < 4; it++) {
+    for (int step = 0; step < ITS; step++) {
+        const int it = SEGS == 1 ? step : step + 2 * __builtin_amdgcn_readfirstlane(seg);      // 32 tokens each
         // (no request ahead as in the K kernel: placing the packs holds too many registers to keep 16 rows in flight)
         uint2 xr[16];
         // PERM: (the 32 tokens of an iteration lie in one repacking block: perm_block is a multiple of 64)
@@ -1608,7 +1615,7 @@ __global__ void __launch_bounds__(512) v_quant_encode_cells_kernel(
             if (lane < 32) {
                 const uint32_t src = min(perm[tok0 + 32 * it + lane], (uint32_t)perm_block - 1u);
                 const uint32_t sb = scale_in[(size_t)b * T + rb + src], zb = zero_in[(size_t)b * T + rb + src];
-                if (wave == 0) {
+                if (j == 0) {
                     const size_t tok = (size_t)b * par_stride + tok0 + 32 * it + lane;
                     scale[tok] = (uint16_t)sb;
                     zero[tok] = (uint16_t)zb;
@@ -1623,11 +1630,11 @@ __global__ void __launch_bounds__(512) v_quant_encode_cells_kernel(
         }
         __syncthreads();
         if (XCH) {
-            if (wave == 0) {
+            if (j == 0) {
                 const int tk = lane & 31;
-                uint32_t pw = s_mm[it & 1][0][tk];
+                uint32_t pw = s_mm[it & 1][8 * seg][tk];
 #pragma unroll
-                for (int q = 1; q < 8; q++) pw = pk_sel_x<false, DT != PKV_F16>(pw, s_mm[it & 1][q][tk]);
+                for (int q = 1; q < 8; q++) pw = pk_sel_x<false, DT != PKV_F16>(pw, s_mm[it & 1][8 * seg + q][tk]);
                 float rmn, rmx;
                 minmax_unword<DT>(pw, rmn, rmx);
                 uint64_t *words = xw + (size_t)(gidx - sgi) * 128 + 32 * it;      // [run][iteration][token] of this group
@@ -1659,21 +1666,21 @@ __global__ void __launch_bounds__(512) v_quant_encode_cells_kernel(
                         scale[tok] = (uint16_t)T16<DT>::to_bits(sc);
                         zero[tok] = (uint16_t)zb;
                     }
-                    s_par[lane] = token_par<DT>(sc, zb, false);
+                    s_par[32 * seg + lane] = token_par<DT>(sc, zb, false);
                 }
             }
             __syncthreads();
         } else
         if (lane < 32) {
-            uint32_t pw = s_mm[it & 1][0][lane];             // the eight heads' words, combined by packed minima
+            uint32_t pw = s_mm[it & 1][8 * seg][lane];             // the eight heads' words, combined by packed minima
 #pragma unroll
-            for (int q = 1; q < 8; q++) pw = pk_sel_x<false, DT != PKV_F16>(pw, s_mm[it & 1][q][lane]);
+            for (int q = 1; q < 8; q++) pw = pk_sel_x<false, DT != PKV_F16>(pw, s_mm[it & 1][8 * seg + q][lane]);
             float mn, mx;
             minmax_unword<DT>(pw, mn, mx);
             const float range = round_t<DT>(mx - mn);
             const float sc = round_t<DT>(range * rel);
             const uint32_t zb = T16<DT>::to_bits(rintf(round_t<DT>(__fdiv_rn(mn, sc))));
-            if (wave == 0) {
+            if (j == 0) {
                 const size_t tok = (size_t)b * par_stride + tok0 + 32 * it + lane;
                 scale[tok] = (uint16_t)T16<DT>::to_bits(sc);
                 zero[tok] = (uint16_t)zb;
@@ -1694,8 +1701,8 @@ __global__ void __launch_bounds__(512) v_quant_encode_cells_kernel(
         __builtin_amdgcn_s_setprio(PKV_EPRIO_EMIT);
         const auto halves = __builtin_amdgcn_permlane32_swap(tot, tot, false, false);      // the even round's total, the odd round's
         const uint32_t tot_even = halves[0], tot_odd = halves[1];
-        if (it == 3) {
-            if (active && rp == 0 && m == 0) s_usz[blkid][2 * w + 1] = (uint16_t)(meta + run_off + tot_even + tot_odd);
+        if (step == ITS - 1) {
+            if (active && rp == 0 && m == 0) s_usz[blkid][2 * w + (it >> 1)] = (uint16_t)(meta + run_off + tot_even + tot_odd);
             __syncthreads();
             if (tid == 0) {
                 uint32_t run = 0;
@@ -1722,7 +1729,7 @@ __global__ void __launch_bounds__(512) v_quant_encode_cells_kernel(
         }
         run_off += tot_even + tot_odd;
         if (it & 1) {
-            if (it == 1 && active && rp == 0 && m == 0) s_usz[blkid][2 * w] = (uint16_t)(meta + run_off);
+            if (SEGS == 1 && it == 1 && active && rp == 0 && m == 0) s_usz[blkid][2 * w] = (uint16_t)(meta + run_off);
             run_off = 0;
         }
     }
@@ -1751,16 +1758,17 @@ __global__ void __launch_bounds__(512) v_quant_encode_cells_kernel(
         info[2 * (size_t)(first + tid)] = (uint32_t)(off + blk_off[tid]);
         info[2 * (size_t)(first + tid) + 1] = blk_off[tid + 1] - blk_off[tid];
     }
-    const int q = tid >> 5;
+    const int q = (tid >> 5) & 15;
     if (q < nblk) {
         uint8_t *dst = stream + off + blk_off[q];
         uint32_t cum = 0;
 #pragma unroll
         for (int un = 0; un < 4; un++) {
             const uint32_t n = s_usz[q][un];
-            copy_out32(dst + 8 + cum, gbuf + (size_t)(q * 4 + un) * unit_slot, n, t);
+            const bool mine = SEGS == 1 || un >> 1 == seg;
+            if (mine) copy_out32(dst + 8 + cum, gbuf + (size_t)(q * 4 + un) * unit_slot, n, t);
             cum += n;
-            if (t == un) reinterpret_cast<uint16_t *>(dst)[un] = (uint16_t)cum;
+            if (mine && t == un) reinterpret_cast<uint16_t *>(dst)[un] = (uint16_t)cum;
         }
     }
 }
@@ -1868,7 +1876,7 @@ __global__ void __launch_bounds__(256) k_code_cells_kernel(
 // V: the thread roles of v_quant_encode_cells_kernel (a wavefront = one 128-channel slice with both rounds of an
 // iteration in its halves), no barrier inside an iteration.
 template <bool WIDE>
-__global__ void __launch_bounds__(512) v_code_cells_kernel(
+__global__ void __launch_bounds__(512 * v_cell_segs(WIDE)) v_code_cells_kernel(
     const uint8_t *__restrict__ codes, int hidden, uint8_t *__restrict__ stream, uint64_t capacity,
     uint32_t *__restrict__ info, ScanState *st, int W, uint32_t ngroups, uint32_t unit_slot, const Stagger stagger) {
     extern __shared__ __align__(16) uint8_t gbuf[];        // 16 blocks x 4 units x unit_slot bytes
@@ -1876,26 +1884,28 @@ __global__ void __launch_bounds__(512) v_code_cells_kernel(
     __shared__ uint64_t s_off;
     __shared__ uint32_t blk_off[17];
     __shared__ uint16_t s_usz[16][4];
+    constexpr int SEGS = v_cell_segs(WIDE), ITS = 4 / SEGS;
     const int tid = threadIdx.x;
     stagger_first_generation(stagger);
     if (tid == 0) s_idx = atomicAdd(&st->ticket, 1u);
     __syncthreads();
     const uint32_t gidx = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_idx);      // uniform: the rows' addresses become scalar
     if (gidx >= ngroups) return;
-    const int j = tid >> 6, rp = (tid >> 5) & 1, t = tid & 31;
+    const int j = (tid >> 6) & 7, seg = tid >> 9, rp = (tid >> 5) & 1, t = tid & 31;
     const uint32_t per_row = (uint32_t)hidden / 1024u;
     const uint32_t cb = gidx / per_row, hg = gidx % per_row;
     const UnitGeom g = unit_geom(W);
     const uint32_t meta = (uint32_t)(g.mins_bytes + g.lens_bytes);
     const int blkid = 2 * j + (t >> 4), wq = (t >> 3) & 1, m = t & 7;
-    for (uint32_t i = tid; i < 64u * (meta / 4u); i += 512)                 // metadata areas start as zeros
+    for (uint32_t i = tid; i < 64u * (meta / 4u); i += 512 * SEGS)                 // metadata areas start as zeros
         reinterpret_cast<uint32_t *>(gbuf + (size_t)(i / (meta / 4u)) * unit_slot)[i % (meta / 4u)] = 0u;
     uint32_t run_off = 0;
     const uint8_t *rows = codes + (size_t)cb * 128 * (size_t)hidden + (size_t)hg * 1024;      // uniform
     const uint32_t lane_off = (uint32_t)(16 * rp) * (uint32_t)hidden + (uint32_t)(j * 128 + 4 * t);
     __syncthreads();                                       // the metadata zeros are in place before the first OR
 #pragma unroll 1
-    for (int it = 0; it < 4; it++) {
+    for (int step = 0; step < ITS; step++) {
+        const int it = SEGS == 1 ? step : step + 2 * __builtin_amdgcn_readfirstlane(seg);      // 32 tokens each
         // (no request ahead: with sixteen more registers in flight while the packs are placed the kernel needs 142
         // and a CU holds one workgroup instead of two)
         uint32_t w[16];
@@ -1912,8 +1922,8 @@ __global__ void __launch_bounds__(512) v_code_cells_kernel(
         __builtin_amdgcn_s_setprio(PKV_EPRIO_EMIT);
         const auto halves = __builtin_amdgcn_permlane32_swap(tot, tot, false, false);      // the even round's total, the odd round's
         const uint32_t tot_even = halves[0], tot_odd = halves[1];
-        if (it == 3) {
-            if (rp == 0 && m == 0) s_usz[blkid][2 * wq + 1] = (uint16_t)(meta + run_off + tot_even + tot_odd);
+        if (step == ITS - 1) {
+            if (rp == 0 && m == 0) s_usz[blkid][2 * wq + (it >> 1)] = (uint16_t)(meta + run_off + tot_even + tot_odd);
             __syncthreads();
             if (tid == 0) {
                 uint32_t run = 0;
@@ -1939,7 +1949,7 @@ __global__ void __launch_bounds__(512) v_code_cells_kernel(
         }
         run_off += tot_even + tot_odd;
         if (it & 1) {
-            if (it == 1 && rp == 0 && m == 0) s_usz[blkid][2 * wq] = (uint16_t)(meta + run_off);
+            if (SEGS == 1 && it == 1 && rp == 0 && m == 0) s_usz[blkid][2 * wq] = (uint16_t)(meta + run_off);
             run_off = 0;
         }
     }
@@ -1961,15 +1971,16 @@ __global__ void __launch_bounds__(512) v_code_cells_kernel(
         info[2 * (size_t)(gidx * 16u + tid)] = (uint32_t)(off + blk_off[tid]);
         info[2 * (size_t)(gidx * 16u + tid) + 1] = blk_off[tid + 1] - blk_off[tid];
     }
-    const int q = tid >> 5;                                // half-wavefront q copies block q
+    const int q = (tid >> 5) & 15;                         // half-wavefront q copies block q (of two segments each its own)
     uint8_t *dst = stream + off + blk_off[q];
     uint32_t cum = 0;
 #pragma unroll
     for (int un = 0; un < 4; un++) {
         const uint32_t n = s_usz[q][un];
-        copy_out32(dst + 8 + cum, gbuf + (size_t)(q * 4 + un) * unit_slot, n, t);
+        const bool mine = SEGS == 1 || un >> 1 == seg;
+        if (mine) copy_out32(dst + 8 + cum, gbuf + (size_t)(q * 4 + un) * unit_slot, n, t);
         cum += n;
-        if (t == un) reinterpret_cast<uint16_t *>(dst)[un] = (uint16_t)cum;
+        if (mine && t == un) reinterpret_cast<uint16_t *>(dst)[un] = (uint16_t)cum;
     }
 }
 
@@ -2009,8 +2020,9 @@ int launch_code_cells(bool is_k, const uint8_t *codes, int ctx_len, int hidden, 
         const uint32_t lds = 64u * unit_slot + 64u;
         auto kern = bits > 4 ? v_code_cells_kernel<true> : v_code_cells_kernel<false>;
         PKV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        if ((rc = stagger_for(reinterpret_cast<const void *>(kern), 512, lds, ngroups, &sg))) return rc;
-        kern<<<ngroups, 512, lds, s>>>(codes, hidden, stream, capacity, info, st, bits, ngroups, unit_slot, sg);
+        const unsigned threads = 512u * v_cell_segs(bits > 4);
+        if ((rc = stagger_for(reinterpret_cast<const void *>(kern), (int)threads, lds, ngroups, &sg))) return rc;
+        kern<<<ngroups, threads, lds, s>>>(codes, hidden, stream, capacity, info, st, bits, ngroups, unit_slot, sg);
     }
     PKV_HIP_CHECK(hipGetLastError());
     return PKV_OK;
@@ -2341,8 +2353,9 @@ static int launch_quant_encode(const EncodeJob &job, int dtype, int B, int H, in
                 auto cells = cells_kernel<false>(bits, dtype, perm != nullptr, false, xs.st != kHeadDim);
                 PKV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(cells),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-                if ((rc = stagger_for(reinterpret_cast<const void *>(cells), 512, lds, ngroups, &sg))) return rc;
-                cells<<<ngroups, 512, lds, s>>>((const uint16_t *)x, B, H, T, xs, rel, (uint16_t *)scale, (uint16_t *)zero,
+                const unsigned threads = 512u * v_cell_segs(bits > 4);
+                if ((rc = stagger_for(reinterpret_cast<const void *>(cells), (int)threads, lds, ngroups, &sg))) return rc;
+                cells<<<ngroups, threads, lds, s>>>((const uint16_t *)x, B, H, T, xs, rel, (uint16_t *)scale, (uint16_t *)zero,
                                                 stream, capacity, info, st, bits, ngroups, unit_slot, base, par_stride, perm, perm_block,
                                                 (const uint16_t *)scale_in, (const uint16_t *)zero_in, sg, 1, nullptr);
             } else {
@@ -2391,8 +2404,9 @@ static int launch_quant_encode(const EncodeJob &job, int dtype, int B, int H, in
             PKV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
             Stagger sg;
-            if ((rc = stagger_for(reinterpret_cast<const void *>(kern), 512, lds, nruns_all, &sg))) return rc;
-            kern<<<nruns_all, 512, lds, s>>>((const uint16_t *)x, B, H, T, xs, rel, (uint16_t *)scale, (uint16_t *)zero,
+            const unsigned threads = 512u * v_cell_segs(bits > 4);
+            if ((rc = stagger_for(reinterpret_cast<const void *>(kern), (int)threads, lds, nruns_all, &sg))) return rc;
+            kern<<<nruns_all, threads, lds, s>>>((const uint16_t *)x, B, H, T, xs, rel, (uint16_t *)scale, (uint16_t *)zero,
                                              stream, capacity, info, st, bits, nruns_all, unit_slot, base, par_stride, nullptr, 0,
                                              nullptr, nullptr, sg, nruns, st->status + nruns_all);
         }

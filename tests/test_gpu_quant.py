@@ -491,3 +491,35 @@ def test_encoders_that_close_by_themselves(cuda, H, T):
                 code_enc(codes, s[2][:e["size"] - 2], s[4])
             with pytest.raises(ops.PackKVError, match="fit"):
                 enc(x, 0.1, stream=s[2][:e["size"] - 2], info=s[4])
+
+
+# V of 5 and 6 bits beyond the encodes at once: two segments of a block side by side; idle head slots, runs of eight heads.
+@pytest.mark.parametrize("B,H,T,rel", [(1, 8, 16512, 0.05), (3, 5, 5632, 0.03), (1, 12, 11136, 0.05), (129, 8, 128, 0.05)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_wide_v_with_both_segments_at_once(cuda, oracle_codec, B, H, T, rel, dtype):
+    k, v = synth.make_kv(B, H, T, seed=H + T, dtype=dtype)
+    W = ops.bits_for_rel(rel)
+    c, z, s = oq.quant_ints(v, 64, rel)
+    codes = oq.code_matrix(c)
+    so, io, zo = oracle_codec.encode(0, codes.numpy(), 128, 64, W)
+    _say("wide V", B, H, T, rel, dtype)
+    vd = v.to(cuda)
+    r = ops.v_quant_encode(vd, rel, W)
+    assert r["size"] == zo
+    assert np.array_equal(r["info"].cpu().numpy(), io)
+    assert np.array_equal(r["stream"][:zo].cpu().numpy(), so[:zo])
+    assert torch.equal(r["scale"].cpu().view(torch.int16), s.reshape(B, T).view(torch.int16))
+    assert torch.equal(r["zero"].cpu().view(torch.int16), z.reshape(B, T).view(torch.int16))
+    if H % 8 == 0:                                     # the same from the code matrix
+        stream, info = torch.zeros_like(r["stream"]), torch.zeros_like(r["info"])
+        assert ops.encode_p(False, codes.to(cuda), stream, info, 16, W) == zo
+        assert torch.equal(stream[:zo], r["stream"][:zo]) and torch.equal(info.view(torch.int32), r["info"].view(torch.int32))
+    if H <= 8:                                         # in the order of a repacking: as the rows in that order
+        _, ve, perm = ops.repack_quant_encode(k.to(cuda), vd, rel, rel, "median")
+        block = 64
+        src = torch.arange(T, device=cuda) // block * block + perm.view(torch.int32).long()
+        want = ops.v_quant_encode(vd[:, :, src].contiguous(), rel, W)
+        n = want["size"]
+        assert ve["size"] == n and torch.equal(ve["stream"][:n], want["stream"][:n])
+        for name in ("info", "scale", "zero"):
+            assert torch.equal(ve[name].view(torch.int16), want[name].view(torch.int16)), name
