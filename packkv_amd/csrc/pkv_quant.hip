@@ -1037,23 +1037,28 @@ __device__ __forceinline__ void cell_token_minmax_halves(const uint2 xr[16], flo
 // ROT: the rows get their rotary embedding on the way (cell_rotate) -- a prompt's keys are then read once where they are,
 // instead of being rotated into a buffer of their own size first.  The arithmetic costs the encoder 90 us on 512 MiB of
 // bf16 (196 -> 287 us, bound by the vector units), the pass it saves took 190.
-template <int DT, bool WIDE, bool PERM, bool XCH = false, bool STRIDED = false, bool ROT = false>
-__global__ void __launch_bounds__(256) k_quant_encode_cells_kernel(
-    const uint16_t *__restrict__ x, int B, int H, int T, const XRows xs, float rel, uint16_t *__restrict__ scale,
+// The 256 threads `tid` of a workgroup of their own, or of one that holds two such groups (both have one: they meet at the barriers).
+struct KCellsLds {
+    uint32_t idx;
+    uint64_t off;
+    uint32_t blk_off[kSubBlocks + 1];
+    __attribute__((aligned(16))) TokPar par[4 * 16];       // [wavefront][token of the round]
+    float2 mm[2][4][16];                                   // [round parity][wavefront][token]: (min, max)
+};
+template <int DT, bool WIDE, bool PERM, bool XCH, bool STRIDED, bool ROT>
+__device__ __forceinline__ void k_quant_encode_cells(
+    const int tid, uint8_t *const gbuf, KCellsLds &lds, const uint16_t *__restrict__ x, int B, int H, int T, const XRows xs, float rel, uint16_t *__restrict__ scale,
     uint16_t *__restrict__ zero, uint8_t *__restrict__ stream, uint64_t capacity, uint32_t *__restrict__ info,
     ScanState *st, int W, uint32_t ngroups, uint32_t bound, uint64_t base, int par_stride,
     const uint32_t *__restrict__ perm, int perm_block, const Stagger stagger, int nsg, uint64_t *xw, const Rot rot) {
-    extern __shared__ __align__(16) uint8_t gbuf[];        // H block slots of `bound` bytes
-    __shared__ uint32_t s_idx;
-    __shared__ uint64_t s_off;
-    __shared__ uint32_t blk_off[kSubBlocks + 1];
-    __shared__ __attribute__((aligned(16))) TokPar s_par[4 * 16];       // [wavefront][token of the round]
-    __shared__ float2 s_mm[2][4][16];                                    // [round parity][wavefront][token]: (min, max)
-    const int tid = threadIdx.x;
+    uint64_t &s_off = lds.off;
+    uint32_t *const blk_off = lds.blk_off;
+    TokPar *const s_par = lds.par;
+    auto &s_mm = lds.mm;
     stagger_first_generation(stagger);
-    if (tid == 0) s_idx = atomicAdd(&st->ticket, 1u);
+    if (tid == 0) lds.idx = atomicAdd(&st->ticket, 1u);
     __syncthreads();
-    const uint32_t gidx = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_idx);
+    const uint32_t gidx = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds.idx);
     if (gidx >= ngroups) return;
     // XCH (more than eight heads): runs of eight heads, one workgroup and one ticket each, as in the round-major
     // kernel: a run forms the minima and maxima over its own heads, publishes them per token and collects the others'.
@@ -1219,6 +1224,19 @@ __global__ void __launch_bounds__(256) k_quant_encode_cells_kernel(
         info[2 * (size_t)(first + tid) + 1] = blk_off[tid + 1] - blk_off[tid];
     }
     if (active) copy_out32(stream + off + blk_off[j], blk, my_off, t);
+}
+
+template <int DT, bool WIDE, bool PERM, bool XCH = false, bool STRIDED = false, bool ROT = false>
+__global__ void __launch_bounds__(256) k_quant_encode_cells_kernel(
+    const uint16_t *__restrict__ x, int B, int H, int T, const XRows xs, float rel, uint16_t *__restrict__ scale,
+    uint16_t *__restrict__ zero, uint8_t *__restrict__ stream, uint64_t capacity, uint32_t *__restrict__ info,
+    ScanState *st, int W, uint32_t ngroups, uint32_t bound, uint64_t base, int par_stride,
+    const uint32_t *__restrict__ perm, int perm_block, const Stagger stagger, int nsg, uint64_t *xw, const Rot rot) {
+    extern __shared__ __align__(16) uint8_t gbuf[];        // H block slots of `bound` bytes
+    __shared__ KCellsLds lds;
+    k_quant_encode_cells<DT, WIDE, PERM, XCH, STRIDED, ROT>(threadIdx.x, gbuf, lds, x, B, H, T, xs, rel, scale, zero, stream, capacity,
+                                                                   info, st, W, ngroups, bound, base, par_stride, perm, perm_block, stagger,
+                                                                   nsg, xw, rot);
 }
 
 // ---- K, up to four heads: round-major, several groups to a workgroup ---------------------------
@@ -1554,26 +1572,33 @@ __global__ void __launch_bounds__(512) v_quant_encode_rounds_kernel(
 // wavefronts a CU left it waiting for its loads.  16 x 8 x 32768 tokens of fp16 V at rel 0.05: 475 -> 425 us (bf16 521 -> 463, rel 0.03
 // 487 -> 436), from a code matrix 284 -> 225, 3 x 8 x 11008 70.6 -> 60.7 and 44.9 -> 38.2.
 __host__ __device__ constexpr int v_cell_segs(bool wide) { return wide ? 2 : 1; }
-template <int DT, bool WIDE, bool PERM, bool XCH = false, bool STRIDED = false>
-__global__ void __launch_bounds__(512 * v_cell_segs(WIDE)) v_quant_encode_cells_kernel(
-    const uint16_t *__restrict__ x, int B, int H, int T, const XRows xs, float rel, uint16_t *__restrict__ scale,
+template <bool WIDE>
+struct VCellsLds {
+    uint32_t idx;
+    uint64_t off;
+    uint32_t blk_off[17];
+    uint16_t usz[16][4];
+    __attribute__((aligned(16))) TokPar par[v_cell_segs(WIDE) * 8 * 32];       // [wavefront][token of the iteration]
+    uint32_t mm[2][v_cell_segs(WIDE) * 8][32];                                 // [iteration parity][wavefront][token]: minmax_word
+};
+template <int DT, bool WIDE, bool PERM, bool XCH, bool STRIDED>
+__device__ __forceinline__ void v_quant_encode_cells(
+    uint8_t *const gbuf, VCellsLds<WIDE> &lds, const uint16_t *__restrict__ x, int B, int H, int T, const XRows xs, float rel, uint16_t *__restrict__ scale,
     uint16_t *__restrict__ zero, uint8_t *__restrict__ stream, uint64_t capacity, uint32_t *__restrict__ info,
     ScanState *st, int W, uint32_t ngroups, uint32_t unit_slot, uint64_t base, int par_stride,
     const uint32_t *__restrict__ perm, int perm_block, const uint16_t *__restrict__ scale_in,
-    const uint16_t *__restrict__ zero_in, const Stagger stagger, int nsg = 1, uint64_t *xw = nullptr) {
+    const uint16_t *__restrict__ zero_in, const Stagger stagger, int nsg, uint64_t *xw) {
     constexpr int SEGS = v_cell_segs(WIDE), ITS = 4 / SEGS;
-    extern __shared__ __align__(16) uint8_t gbuf[];        // 16 blocks x 4 units x unit_slot bytes
-    __shared__ uint32_t s_idx;
-    __shared__ uint64_t s_off;
-    __shared__ uint32_t blk_off[17];
-    __shared__ uint16_t s_usz[16][4];
-    __shared__ __attribute__((aligned(16))) TokPar s_par[SEGS * 8 * 32];       // [wavefront][token of the iteration]
-    __shared__ uint32_t s_mm[2][SEGS * 8][32];                           // [iteration parity][wavefront][token]: minmax_word
+    uint64_t &s_off = lds.off;
+    uint32_t *const blk_off = lds.blk_off;
+    auto &s_usz = lds.usz;
+    TokPar *const s_par = lds.par;
+    auto &s_mm = lds.mm;
     const int tid = threadIdx.x;
     stagger_first_generation(stagger);
-    if (tid == 0) s_idx = atomicAdd(&st->ticket, 1u);
+    if (tid == 0) lds.idx = atomicAdd(&st->ticket, 1u);
     __syncthreads();
-    const uint32_t gidx = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_idx);
+    const uint32_t gidx = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds.idx);
     if (gidx >= ngroups) return;
     // XCH (more than eight heads): runs of eight heads that exchange the minima and maxima of their heads per token,
     // as in the K kernel; a run's words are [iteration][token of the iteration]
@@ -1770,6 +1795,57 @@ __global__ void __launch_bounds__(512 * v_cell_segs(WIDE)) v_quant_encode_cells_
             cum += n;
             if (mine && t == un) reinterpret_cast<uint16_t *>(dst)[un] = (uint16_t)cum;
         }
+    }
+}
+
+template <int DT, bool WIDE, bool PERM, bool XCH = false, bool STRIDED = false>
+__global__ void __launch_bounds__(512 * v_cell_segs(WIDE)) v_quant_encode_cells_kernel(
+    const uint16_t *__restrict__ x, int B, int H, int T, const XRows xs, float rel, uint16_t *__restrict__ scale,
+    uint16_t *__restrict__ zero, uint8_t *__restrict__ stream, uint64_t capacity, uint32_t *__restrict__ info,
+    ScanState *st, int W, uint32_t ngroups, uint32_t unit_slot, uint64_t base, int par_stride,
+    const uint32_t *__restrict__ perm, int perm_block, const uint16_t *__restrict__ scale_in,
+    const uint16_t *__restrict__ zero_in, const Stagger stagger, int nsg = 1, uint64_t *xw = nullptr) {
+    extern __shared__ __align__(16) uint8_t gbuf[];        // 16 blocks x 4 units x unit_slot bytes
+    __shared__ VCellsLds<WIDE> lds;
+    v_quant_encode_cells<DT, WIDE, PERM, XCH, STRIDED>(gbuf, lds, x, B, H, T, xs, rel, scale, zero, stream, capacity, info, st, W, ngroups,
+                                                       unit_slot, base, par_stride, perm, perm_block, scale_in, zero_in, stagger, nsg, xw);
+}
+
+// ---- K and V in one launch -----------------------------------------------------------------------
+// Workgroups of 512 threads, two resident on a CU: one in two takes a group of V as the kernel above, the other two groups of K
+// (T is a multiple of 128, so there are twice as many of those).  A launch of its own leaves the chip partly empty at its end or,
+// when it is small, all the time, and all its workgroups go through their phases together.  V and K go in turns of 256 (`turns` of
+// them each, then the rest of V, the rest of K), so that a CU starts with one of each.
+struct CellsSide {
+    const uint16_t *x;
+    XRows xs;
+    float rel;
+    uint16_t *scale, *zero;
+    uint8_t *stream;
+    uint64_t capacity, base;
+    uint32_t *info;
+    ScanState *st;
+    int W;
+    uint32_t ngroups, slot;                // K: bytes of a block's slot, V: of a unit's
+    const uint16_t *scale_in, *zero_in;
+};
+template <int DT, bool PERM, bool ROT>
+__global__ void __launch_bounds__(512) kv_quant_encode_cells_kernel(const CellsSide k, const CellsSide v, int B, int H, int T, int par_stride,
+                                                                    const uint32_t *__restrict__ perm, int perm_block, uint32_t turns, const Rot rot) {
+    extern __shared__ __align__(16) uint8_t gbuf[];
+    const Stagger stagger{0u, 0u};
+    __shared__ union Lds { __device__ Lds() {} VCellsLds<false> v; KCellsLds k[2]; } lds;
+    const uint32_t turn = blockIdx.x >> 8;
+    if (turn < 2u * turns ? (turn & 1u) == 0u : blockIdx.x - (turns << 9) < v.ngroups - (turns << 8)) {
+        v_quant_encode_cells<DT, false, PERM, false, !PERM>(gbuf, lds.v, v.x, B, H, T, v.xs, v.rel, v.scale, v.zero, v.stream, v.capacity, v.info,
+                                                            v.st, v.W, v.ngroups, v.slot, v.base, par_stride, perm, perm_block, v.scale_in,
+                                                            v.zero_in, stagger, 1, nullptr);
+    } else {
+        const int half = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8);
+        k_quant_encode_cells<DT, false, PERM, false, !PERM, ROT>((int)threadIdx.x & 255, gbuf + (size_t)half * H * k.slot, lds.k[half], k.x,
+                                                                       B, H, T, k.xs, k.rel, k.scale, k.zero, k.stream, k.capacity, k.info, k.st,
+                                                                       k.W, k.ngroups, k.slot, k.base, par_stride, perm, perm_block, stagger, 1,
+                                                                       nullptr, rot);
     }
 }
 
@@ -2439,6 +2515,41 @@ static int run_quant_encode(const void *x, int dtype, int B, int H, int T, float
     return closes ? ce.wait(size_out, bits) : finish_encode(sh, size_out, bits, s);
 }
 
+// K and V by the cells kernels in one launch: five to eight heads and codes of up to four bits on both sides, below the four
+// generations of V from which the launches of their own are staggered.  B x 8 heads x 8192 tokens, us for a median repacking's
+// order and encodes and for the first update of a growing cache (rotary keys), two launches -> one: fp16 B = 4 99.2 -> 84.9 and 130.5 ->
+// 118.0, 6 122 -> 117 and 153 -> 140, 8 146 -> 145 and 175 -> 172, 12 227 -> 199 and 259 -> 217, 24 384 -> 347 and 376 -> 347, 32 (8192 and
+// 8064 tokens) 435 -> 437 and 449 -> 427; bf16 B = 4 115 -> 93 and 144 -> 126, 8 166 -> 158 and 196 -> 195, 24 428 -> 387 and 434 -> 401, 32 522 ->
+// 493; at 8192 tokens, staggered, 414 -> 429 and 484 -> 497.  In turns up to 1024 groups of V, V first beyond (fp16 B = 16 269 -> 259 us in
+// turns, but 24 347 -> 359 and 32 427 -> 445).
+constexpr uint64_t kBothGroups = 2048, kBothTurns = 1024;
+static bool cells_in_one_launch(const EncodeJob job[2], const OncePlan &pk, const OncePlan &pv, int B, int H, int T) {
+    return !pk.threads && !pv.threads && H > 4 && H <= kSubBlocks && job[0].bits <= 4 && job[1].bits <= 4 &&
+           job[0].xs.sh < (1ll << 31) - 128 && (uint64_t)(T / 128) * (uint64_t)B < kBothGroups;
+}
+static int launch_cells_both(const EncodeJob job[2], int dtype, int B, int H, int T, ScanState *k_st, ScanState *v_st, hipStream_t s) {
+    CellsSide side[2];
+    for (int i = 0; i < 2; i++) {
+        const EncodeJob &a = job[i];
+        const uint32_t bound = i ? ((uint32_t)v_block_bound(64, a.bits) - 8u) / 4u : (uint32_t)k_block_bound(64, a.bits);
+        side[i] = CellsSide{(const uint16_t *)a.x, a.xs, a.rel, (uint16_t *)a.scale, (uint16_t *)a.zero, a.stream, a.capacity, a.base, a.info,
+                            i ? v_st : k_st, a.bits, (uint32_t)(T / (i ? 128 : 64)) * (uint32_t)B, (bound + 15u) & ~15u,
+                            (const uint16_t *)a.scale_in, (const uint16_t *)a.zero_in};
+    }
+    const uint32_t lds_k = 2u * (uint32_t)H * side[0].slot + 32u, lds_v = 64u * side[1].slot + 64u, lds = lds_k > lds_v ? lds_k : lds_v;
+    const bool perm = job[0].perm != nullptr, rot = job[0].rot.cos != nullptr;
+    auto pick = [&](auto f16, auto bf16) { return dtype == PKV_F16 ? f16 : bf16; };
+    auto kern = perm ? pick(kv_quant_encode_cells_kernel<PKV_F16, true, false>, kv_quant_encode_cells_kernel<PKV_BF16, true, false>)
+                : rot ? pick(kv_quant_encode_cells_kernel<PKV_F16, false, true>, kv_quant_encode_cells_kernel<PKV_BF16, false, true>)
+                      : pick(kv_quant_encode_cells_kernel<PKV_F16, false, false>, kv_quant_encode_cells_kernel<PKV_BF16, false, false>);
+    PKV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    const uint32_t vg = side[1].ngroups;
+    kern<<<2u * vg, 512, lds, s>>>(side[0], side[1], B, H, T, job[0].par_stride, job[0].perm, job[0].perm_block,
+                                   vg <= kBothTurns ? vg >> 8 : 0u, job[0].rot);
+    PKV_HIP_CHECK(hipGetLastError());
+    return PKV_OK;
+}
+
 // K and V (checked jobs) with one wait; in one launch where both take a group's tokens at once.
 static int encode_both(const EncodeJob job[2], int dtype, int B, int H, int T, uint64_t *k_size, uint64_t *v_size, hipStream_t s) {
     int rc;
@@ -2455,6 +2566,10 @@ static int encode_both(const EncodeJob job[2], int dtype, int B, int H, int T, u
         if ((rc = pk.threads == 256 ? once_launch<256>(ks, vs, dtype, ce.close, s) : once_launch<1024>(ks, vs, dtype, ce.close, s))) return rc;
         if ((rc = ce.launched(sh))) return rc;
         return ce.wait(k_size, job[0].bits, v_size, job[1].bits);
+    }
+    if (cells_in_one_launch(job, pk, pv, B, H, T)) {
+        if ((rc = launch_cells_both(job, dtype, B, H, T, sh.st, sh.second, s))) return rc;
+        return finish_encode(sh, k_size, job[0].bits, s, v_size, job[1].bits);
     }
     if ((rc = launch_quant_encode<true>(job[0], dtype, B, H, T, sh.st, EncodeClose{}, s))) return rc;
     if ((rc = launch_quant_encode<false>(job[1], dtype, B, H, T, sh.second, EncodeClose{}, s))) return rc;

@@ -523,3 +523,47 @@ def test_wide_v_with_both_segments_at_once(cuda, oracle_codec, B, H, T, rel, dty
         assert ve["size"] == n and torch.equal(ve["stream"][:n], want["stream"][:n])
         for name in ("info", "scale", "zero"):
             assert torch.equal(ve[name].view(torch.int16), want[name].view(torch.int16)), name
+
+
+# K and V of five to eight heads in one launch: idle head slots, V first and in turns of 256 groups with a rest, one type and both
+# kinds of rows, each as the encodes of one side.
+@pytest.mark.parametrize("B,H,T", [(1, 8, 17408), (2, 5, 17280), (9, 7, 4864), (21, 6, 6272)])
+@pytest.mark.parametrize("form", ["order", "rows", "rotary"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_both_sides_in_one_launch(cuda, B, H, T, form, dtype):
+    k, v = synth.make_kv(B, H, T, seed=H + T, dtype=dtype, device=cuda)
+    rels = (0.1, 0.2)
+    _say("both sides", B, H, T, form, dtype)
+    if form == "order":
+        ke, ve, perm = ops.repack_quant_encode(k, v, *rels, "median")
+        for e, x, is_k in ((ke, k, True), (ve, v, False)):
+            want = ops._quant_encode(is_k, x, rels[not is_k], e["bits"], None, None, True, False, perm, 64)
+            n = want["size"]
+            assert e["size"] == n and torch.equal(e["stream"][:n], want["stream"][:n])
+            assert all(torch.equal(e[f].view(torch.int16), want[f].view(torch.int16)) for f in ("info", "scale", "zero"))
+        return
+    used, before = 1002, 128
+    cos = sin = None
+    kr = k
+    if form == "rotary":
+        cos, sin = (torch.randn(1, T, 128, device=cuda).to(dtype).expand(B, -1, -1) for _ in range(2))
+        kr = (k * cos.unsqueeze(1)) + (torch.cat((-k[..., 64:], k[..., :64]), dim=-1) * sin.unsqueeze(1))
+    want = [ops.k_quant_encode(kr, rels[0]), ops.v_quant_encode(v, rels[1])]
+    sides, blocks = [], []
+    for i in range(2):
+        per_tile, ctx = (B * H, 64) if i == 0 else (2 * B * H, 128)
+        blocks.append(before // ctx * per_tile)
+        sides.append((rels[i], want[i]["bits"], torch.zeros(used + want[i]["stream"].numel(), dtype=torch.uint8, device=cuda), used,
+                      torch.zeros((before + T) // ctx * per_tile, 2, dtype=torch.uint32, device=cuda),
+                      torch.zeros(B, before + T + 64, dtype=dtype, device=cuda), torch.zeros(B, before + T + 64, dtype=dtype, device=cuda)))
+    rows = [x.transpose(1, 2).contiguous().transpose(1, 2) for x in (k, v)] if form == "rows" else [k, v]
+    for rep in range(2):                               # (twice: nothing of the first call's look-back may be left)
+        sizes = ops.kv_quant_encode_append(*rows, T, *sides, before, cos, sin)
+        for i in range(2):
+            n = want[i]["size"]
+            _, _, stream, _, info, scale, zero = sides[i]
+            assert sizes[i] == used + n and torch.equal(stream[used:used + n], want[i]["stream"][:n])
+            got, ref = info.view(torch.int32)[blocks[i]:], want[i]["info"].view(torch.int32)
+            assert torch.equal(got[:, 0], ref[:, 0] + used) and torch.equal(got[:, 1], ref[:, 1])
+            assert torch.equal(scale[:, before:before + T], want[i]["scale"]) and torch.equal(zero[:, before:before + T], want[i]["zero"])
+            assert not scale[:, :before].any() and not scale[:, before + T:].any() and not stream[:used].any()
