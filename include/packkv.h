@@ -117,11 +117,14 @@ uint64_t pkv_block_bound_p(int pack_len, int bits);
  * `dtype`; scale and zero are [B, T] in `dtype` (one pair per batch and token, shared by
  * all heads and channels); every intermediate is rounded to `dtype` exactly where the
  * PyTorch op chain rounds it.  `codes` is the uint8 code matrix [T, B*H*128].
- * `max_code_out` (device uint32, may be NULL) receives the largest code produced. */
+ * `max_code_out` (device uint32, may be NULL) receives the largest code produced.
+ * pkv_quant_codes: parameters and codes in one pass over k and, unless it is NULL, over v of the same shape. */
 int pkv_quant_params(const void *x, int dtype, int B, int H, int T, float rel, void *scale, void *zero,
                      float *ms_out, pkv_stream_t s);
 int pkv_quantize(const void *x, int dtype, int B, int H, int T, const void *scale, const void *zero,
                  uint8_t *codes, uint32_t *max_code_out, float *ms_out, pkv_stream_t s);
+int pkv_quant_codes(const void *k, const void *v, int dtype, int B, int H, int T, float k_rel, float v_rel, void *k_scale, void *k_zero,
+                    uint8_t *k_codes, void *v_scale, void *v_zero, uint8_t *v_codes, pkv_stream_t s);
 int pkv_dequantize(const uint8_t *codes, int dtype, int B, int H, int T, const void *scale,
                    const void *zero, void *x_out, float *ms_out, pkv_stream_t s);
 

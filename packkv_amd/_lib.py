@@ -70,6 +70,7 @@ SIGNATURES = {
     "pkv_k_decode": (_i, [_vp, _u64, _vp, _vp, _i, _i, _i, _i, _i, _fp, _vp]),
     "pkv_v_decode": (_i, [_vp, _u64, _vp, _vp, _i, _i, _i, _i, _i, _fp, _vp]),
     "pkv_quant_params": (_i, [_vp, _i, _i, _i, _i, _f, _vp, _vp, _fp, _vp]),
+    "pkv_quant_codes": (_i, [_vp, _vp, _i, _i, _i, _i, _f, _f, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "pkv_quantize": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _fp, _vp]),
     "pkv_dequantize": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _fp, _vp]),
     "pkv_median_order": (_i, [_vp, _i, _i, _i, _i, _f, _i, _i, _vp, _vp, _vp, _fp, _vp]),

@@ -71,9 +71,9 @@ def crs_evaluation_with_data(config, key_caches, value_caches, device="cuda"):
         if k.shape != v.shape or k.dim() != 4 or k.size(2) % config.block_size:
             raise RuntimeError("K and V must be [B, H, T, D] of one shape with T a multiple of block_size")
         codes, pars, orig, before = {}, {}, {}, {}
-        for side, x, rel in (("k", k, config.k_quant_scale_rel), ("v", v, config.v_quant_scale_rel)):
-            xd = x.to(device).contiguous()
-            codes[side], scale, zero = ops.quant_codes(xd, rel)
+        quantised = ops.quant_codes_pair(k.to(device).contiguous(), v.to(device).contiguous(), config.k_quant_scale_rel, config.v_quant_scale_rel)
+        for side, x, (c, scale, zero) in zip("kv", (k, v), quantised):
+            codes[side] = c
             pars[side] = zero.numel() + scale.numel()
             orig[side] = x.numel() * x.element_size()
         stats = ops.code_stats_pair(codes["k"], codes["v"], config.pack_size)
@@ -104,9 +104,9 @@ def crs_evaluation_detail(config, key_caches, value_caches, device="cuda"):
     res = {s + "_" + k: [] for k in keys for s in ("k", "v")}
     for k, v in zip(key_caches, value_caches):
         codes, pars = {}, {}
-        for side, x, rel in (("k", k, config.k_quant_scale_rel), ("v", v, config.v_quant_scale_rel)):
-            xd = x.to(device).contiguous()
-            codes[side], scale, zero = ops.quant_codes(xd, rel)
+        quantised = ops.quant_codes_pair(k.to(device).contiguous(), v.to(device).contiguous(), config.k_quant_scale_rel, config.v_quant_scale_rel)
+        for side, x, (c, scale, zero) in zip("kv", (k, v), quantised):
+            codes[side] = c
             pars[side] = (zero.numel() * x.element_size(), scale.numel() * x.element_size())
             res[side + "_original_size"].append(x.numel() * x.element_size())
         kc, vc, _ = ops.median_repacking(codes["k"], codes["v"], config.block_size)

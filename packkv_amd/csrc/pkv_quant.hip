@@ -252,6 +252,78 @@ __global__ void __launch_bounds__(256) quantize_kernel(const uint16_t *__restric
     }
 }
 
+// ---- parameters and codes in one pass over x, of one tensor or of K and V ---------------
+// quant_params_kernel and quantize_kernel in one: grid (T/16, B, tensors), 256 threads, 16 lanes per token, 8 channels per lane.  The
+// rows of up to eight heads stay in registers between the two; with more heads the last eight do and the others come again, from
+// the L2.  Bound by the memory system, where the pair read x twice in four launches for K and V.
+struct QuantSide {
+    const uint16_t *x;
+    float rel;
+    uint16_t *scale, *zero;
+    uint8_t *codes;
+};
+template <int DT>
+__global__ void __launch_bounds__(256) quant_codes_kernel(const QuantSide k, const QuantSide v, int H, int T) {
+    constexpr int kHeads = 8;
+    const QuantSide &sd = blockIdx.z == 0 ? k : v;
+    const int b = blockIdx.y, B = gridDim.y;
+    const int tok = blockIdx.x * 16 + (threadIdx.x >> 4), l16 = threadIdx.x & 15;
+    const int at = min(tok, T - 1);                        // (lanes past the end go along for the exchanges)
+    const uint16_t *rows = sd.x + ((size_t)b * H * T + at) * kHeadDim + l16 * 8;
+    const size_t head = (size_t)T * kHeadDim;
+    uint4 r[kHeads];
+    auto load = [&](int h0) {
+#pragma unroll
+        for (int i = 0; i < kHeads; i++)
+            if (h0 + i < H) r[i] = *reinterpret_cast<const uint4 *>(rows + (size_t)(h0 + i) * head);
+    };
+    const int last = (H - 1) / kHeads * kHeads;
+    float mn = INFINITY, mx = -INFINITY;
+    for (int h0 = 0; h0 <= last; h0 += kHeads) {
+        load(h0);
+#pragma unroll
+        for (int i = 0; i < kHeads; i++) {
+            if (h0 + i < H) {
+                float f[8];
+                unpack8<DT>(r[i], f);
+#pragma unroll
+                for (int c = 0; c < 8; c++) {
+                    mn = fminf(mn, f[c]);
+                    mx = fmaxf(mx, f[c]);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int d = 8; d >= 1; d >>= 1) {
+        mn = fminf(mn, __shfl_xor(mn, d, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, d, 16));
+    }
+    const float range = round_t<DT>(mx - mn);
+    const float sc = round_t<DT>(range * sd.rel);
+    const uint32_t zb = T16<DT>::to_bits(rintf(round_t<DT>(__fdiv_rn(mn, sc))));
+    const bool in = tok < T;
+    if (in && l16 == 0) {
+        sd.scale[(size_t)b * T + tok] = (uint16_t)T16<DT>::to_bits(sc);
+        sd.zero[(size_t)b * T + tok] = (uint16_t)zb;
+    }
+    const TokPar tp = token_par<DT>(sc, zb, false);
+    uint8_t *row = sd.codes + ((size_t)at * B + b) * (size_t)H * kHeadDim + l16 * 8;
+    for (int h0 = last; h0 >= 0; h0 -= kHeads) {
+        if (h0 != last) load(h0);
+#pragma unroll
+        for (int i = 0; i < kHeads; i++) {
+            if (in && h0 + i < H) {
+                uint32_t a01, a23, b01, b23;
+                quant4<DT, false>(make_uint2(r[i].x, r[i].y), tp, a01, a23);
+                quant4<DT, false>(make_uint2(r[i].z, r[i].w), tp, b01, b23);
+                *reinterpret_cast<uint2 *>(row + (size_t)(h0 + i) * kHeadDim) =
+                    make_uint2(__builtin_amdgcn_perm(a23, a01, 0x06040200u), __builtin_amdgcn_perm(b23, b01, 0x06040200u));
+            }
+        }
+    }
+}
+
 // ---- uint8 code matrix -> x_hat [B, H, T, 128] -----------------------------------------
 // the same grid and thread roles
 template <int DT>
@@ -2703,6 +2775,23 @@ int pkv_quantize(const void *x, int dtype, int B, int H, int T, const void *scal
                                                        (const uint16_t *)zero, codes, max_code_out);
     PKV_HIP_CHECK(hipGetLastError());
     return tm.end(ms_out);
+}
+
+int pkv_quant_codes(const void *k, const void *v, int dtype, int B, int H, int T, float k_rel, float v_rel, void *k_scale, void *k_zero,
+                    uint8_t *k_codes, void *v_scale, void *v_zero, uint8_t *v_codes, pkv_stream_t s_) {
+    using namespace pkv;
+    hipStream_t s = (hipStream_t)s_;
+    int rc = check_xshape(k, dtype, B, H, T);
+    if (rc || (v && (rc = check_xshape(v, dtype, B, H, T)))) return rc;
+    PKV_REQUIRE(k_scale && k_zero && k_codes && (!v || (v_scale && v_zero && v_codes)), PKV_ERR_INVALID, "null pointer argument");
+    PKV_REQUIRE(k_rel > 0.f && (!v || v_rel > 0.f), PKV_ERR_INVALID, "quant_scale_rel must be positive");
+    const QuantSide ks{(const uint16_t *)k, k_rel, (uint16_t *)k_scale, (uint16_t *)k_zero, k_codes},
+                    vs{(const uint16_t *)v, v_rel, (uint16_t *)v_scale, (uint16_t *)v_zero, v_codes};
+    const dim3 grid((unsigned)((T + 15) / 16), (unsigned)B, v ? 2u : 1u);
+    if (dtype == PKV_F16) quant_codes_kernel<PKV_F16><<<grid, 256, 0, s>>>(ks, vs, H, T);
+    else quant_codes_kernel<PKV_BF16><<<grid, 256, 0, s>>>(ks, vs, H, T);
+    PKV_HIP_CHECK(hipGetLastError());
+    return PKV_OK;
 }
 
 int pkv_dequantize(const uint8_t *codes, int dtype, int B, int H, int T, const void *scale,

@@ -418,8 +418,30 @@ def _quantize(x, scale, zero, B, H, T, mx):
 
 def quant_codes(x, rel):
     """(codes, scale, zero) of quant_params and quantize, without the largest code: nothing is waited for."""
-    scale, zero = quant_params(x, rel)
-    return _quantize(x, scale, zero, *_check_x(x), None), scale, zero
+    return _quant_codes((x,), (rel,))[0]
+
+
+def quant_codes_pair(k, v, k_rel, v_rel):
+    """quant_codes of K and of V, in one launch where they are alike."""
+    if v.shape == k.shape and v.dtype == k.dtype and v.device == k.device:
+        return _quant_codes((k, v), (k_rel, v_rel))
+    return [quant_codes(k, k_rel), quant_codes(v, v_rel)]
+
+
+def _quant_codes(xs, rels):
+    out, args = [], []
+    for x in xs:
+        B, H, T = _check_x(x)
+        codes = torch.empty(T, B * H * 128, dtype=torch.uint8, device=x.device)
+        scale, zero = (torch.empty(B, T, dtype=x.dtype, device=x.device) for _ in range(2))
+        out.append((codes, scale, zero))
+        args += [_ptr(scale), _ptr(zero), _ptr(codes)]
+    both, dev = len(xs) == 2, xs[0].device
+    with _on(dev):
+        rc = _lib.load().pkv_quant_codes(_ptr(xs[0]), _ptr(xs[1]) if both else None, _dtype_code(xs[0]), B, H, T, float(rels[0]),
+                                         float(rels[-1]), *args, *(() if both else (None,) * 3), _stream(dev))
+    _lib.check(rc)
+    return out
 
 
 def dequantize(codes, scale, zero, B, H):
@@ -923,8 +945,7 @@ def repack_quant_encode(k, v, k_rel, v_rel, repack_method="median", block_size=6
         if repack_method == "median":
             perm, vs, vz = median_order(v, v_rel, v_bits, block_size, want_params=True)
         else:
-            kc = quant_codes(k, k_rel)[0]
-            vc, vs, vz = quant_codes(v, v_rel)
+            (kc, _, _), (vc, vs, vz) = quant_codes_pair(k, v, k_rel, v_rel)
             perm = greedy_order(kc, vc, 16, block_size)      # the codecs' packs are 16 tokens
             del kc, vc                                       # (codes too wide for the stream are the encoders' to report)
         return _kv_quant_encode_perm(k, v, k_rel, v_rel, k_bits, v_bits, perm, block_size, vs, vz) + (perm,)

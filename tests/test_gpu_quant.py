@@ -38,6 +38,25 @@ def test_quantizer_bit_exact(cuda, dtype, rel):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,H,T", [(1, 1, 1), (2, 8, 37), (3, 9, 64), (1, 20, 100)])
+def test_parameters_and_codes_in_one_pass(cuda, dtype, B, H, T):
+    """As quant_params and quantize give them, bit for bit: rows in registers, more heads than those hold, a last workgroup
+    of fewer than 16 tokens, and tokens with NaN and infinities."""
+    k, v = synth.make_kv(B, H, T, seed=22, dtype=dtype, device=cuda)
+    if T > 3:
+        k[0, 0, 1, 5], v[0, H - 1, 2], v[0, :, 3], k[B - 1, 0, T - 1, 127] = float("nan"), float("nan"), float("inf"), -float("inf")
+    rels = (0.1, 0.03)
+    for (codes, scale, zero), x, rel in zip(ops.quant_codes_pair(k, v, *rels), (k, v), rels):
+        _say("one pass", dtype, B, H, T, rel)
+        ws, wz = ops.quant_params(x, rel)
+        want, _ = ops.quantize(x, ws, wz)
+        one = ops.quant_codes(x, rel)
+        for c, s, z in ((codes, scale, zero), one):
+            assert torch.equal(s.view(torch.int16), ws.view(torch.int16)) and torch.equal(z.view(torch.int16), wz.view(torch.int16))
+            assert torch.equal(c, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_fused_quant_encode_stream_bit_exact(cuda, oracle_codec, dtype):
     for (B, H, T, rel) in ((1, 2, 128, 0.1), (2, 8, 256, 0.1), (1, 32, 128, 0.1), (2, 4, 256, 0.2), (1, 8, 128, 0.34),
                            (1, 3, 128, 0.1), (2, 5, 256, 0.14), (3, 1, 128, 0.1),
