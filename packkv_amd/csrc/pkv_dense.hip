@@ -79,12 +79,12 @@ __global__ void __launch_bounds__(256) dense_view_kernel(const DenseParams p) {
     uint16_t *rows = sd.out + (size_t)bh * (size_t)(p.T_c + p.T_w) * kHeadDim;
     if (item >= (uint32_t)p.n_tiles) {                       // a piece of the window
         const int r0 = (int)(item - (uint32_t)p.n_tiles) * kDenseWinRows, n16 = min(kDenseWinRows, p.T_w - r0) * (kHeadDim / 8);
-        const uint4 *src = reinterpret_cast<const uint4 *>(sd.win + ((size_t)bh * p.win_stride + r0) * kHeadDim);
-        uint4 *dst = reinterpret_cast<uint4 *>(rows + (size_t)(p.T_c + r0) * kHeadDim);
-        uint4 v[4];
+        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+        const u32x4 *src = reinterpret_cast<const u32x4 *>(sd.win + ((size_t)bh * p.win_stride + r0) * kHeadDim);
+        u32x4 *dst = reinterpret_cast<u32x4 *>(rows + (size_t)(p.T_c + r0) * kHeadDim);
+        u32x4 v[4];      // (filled whatever n16 is: an array filled under conditions went through scratch memory)
 #pragma unroll
-        for (int i = 0; i < 4; i++)
-            if (tid + 256 * i < n16) v[i] = src[tid + 256 * i];
+        for (int i = 0; i < 4; i++) v[i] = src[min(tid + 256 * i, n16 - 1)];
 #pragma unroll
         for (int i = 0; i < 4; i++)
             if (tid + 256 * i < n16) dst[tid + 256 * i] = v[i];
