@@ -1283,7 +1283,7 @@ __device__ __forceinline__ void k_quant_encode_cells(
         const uint64_t off = base + lookback_offset(st, gidx, bytes, true);
         if (tid == 0) {
             s_off = off;
-            if (gidx == ngroups - 1) st->total = off + bytes;
+            if (gidx == ngroups - 1) __hip_atomic_store(&st->total, off + bytes, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (off + bytes > capacity) atomicExch(&st->error, (uint32_t)PKV_ERR_CAPACITY);
         }
     }
@@ -1843,7 +1843,7 @@ __device__ __forceinline__ void v_quant_encode_cells(
         const uint64_t off = base + lookback_offset(st, gidx, bytes, true);
         if (tid == 0) {
             s_off = off;
-            if (gidx == ngroups - 1) st->total = off + bytes;
+            if (gidx == ngroups - 1) __hip_atomic_store(&st->total, off + bytes, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (off + bytes > capacity) atomicExch(&st->error, (uint32_t)PKV_ERR_CAPACITY);
         }
     }
@@ -1901,9 +1901,28 @@ struct CellsSide {
     uint32_t ngroups, slot;                // K: bytes of a block's slot, V: of a unit's
     const uint16_t *scale_in, *zero_in;
 };
+// The end of the launch, which closes by itself (as once_close does it): every workgroup counts itself out, sixteen to a counter and
+// the sixteens on one, and the last one hands the outcome over and clears the state.  Against a kernel for that behind it, median
+// repacking's order and encodes of B x 8 heads x 8192 fp16 tokens: B = 4 83.8 -> 81.4 us, 8 145 -> 138, 12 192 -> 184, 16 243 -> 235, 24 348 -> 343, 32 the same.
+__device__ __forceinline__ void cells_close(const EncodeClose &c, uint32_t &last_of_all) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // what this wavefront wrote into the state has arrived
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const uint32_t group = blockIdx.x / kCloseGroup, groups = (c.total + kCloseGroup - 1u) / kCloseGroup;
+        auto count = [&](uint32_t at) { return __hip_atomic_fetch_add(reinterpret_cast<uint32_t *>(c.count + kCloseStride * at), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u; };
+        const bool last = count(1u + group) == min(kCloseGroup, c.total - group * kCloseGroup) && count(0u) == groups;
+        if (last) publish_outcomes(c.st, c.second, c.last, c.slot, c.tag, c.bits);
+        last_of_all = last ? 1u : 0u;
+    }
+    __syncthreads();
+    if (last_of_all == 0u) return;
+    // (ordinary stores: nothing reads the state any more before the launch has ended)
+    for (uint32_t i = threadIdx.x; i < c.n / 2u; i += blockDim.x) reinterpret_cast<uint4 *>(c.words)[i] = make_uint4(0u, 0u, 0u, 0u);
+    if (threadIdx.x == 0 && (c.n & 1u)) c.words[c.n - 1u] = 0;
+}
 template <int DT, bool PERM, bool ROT>
 __global__ void __launch_bounds__(512) kv_quant_encode_cells_kernel(const CellsSide k, const CellsSide v, int B, int H, int T, int par_stride,
-                                                                    const uint32_t *__restrict__ perm, int perm_block, uint32_t turns, const Rot rot) {
+                                                                    const uint32_t *__restrict__ perm, int perm_block, uint32_t turns, const Rot rot, const EncodeClose c) {
     extern __shared__ __align__(16) uint8_t gbuf[];
     const Stagger stagger{0u, 0u};
     __shared__ union Lds { __device__ Lds() {} VCellsLds<false> v; KCellsLds k[2]; } lds;
@@ -1919,6 +1938,7 @@ __global__ void __launch_bounds__(512) kv_quant_encode_cells_kernel(const CellsS
                                                                        k.W, k.ngroups, k.slot, k.base, par_stride, perm, perm_block, stagger, 1,
                                                                        nullptr, rot);
     }
+    cells_close(c, lds.v.idx);
 }
 
 // `rows` (uniform: scalar registers) is the first of the 16 token rows, `lane_off` the lane's byte offset inside a
@@ -2599,7 +2619,7 @@ static bool cells_in_one_launch(const EncodeJob job[2], const OncePlan &pk, cons
     return !pk.threads && !pv.threads && H > 4 && H <= kSubBlocks && job[0].bits <= 4 && job[1].bits <= 4 &&
            job[0].xs.sh < (1ll << 31) - 128 && (uint64_t)(T / 128) * (uint64_t)B < kBothGroups;
 }
-static int launch_cells_both(const EncodeJob job[2], int dtype, int B, int H, int T, ScanState *k_st, ScanState *v_st, hipStream_t s) {
+static int launch_cells_both(const EncodeJob job[2], int dtype, int B, int H, int T, ScanState *k_st, ScanState *v_st, const EncodeClose &close, hipStream_t s) {
     CellsSide side[2];
     for (int i = 0; i < 2; i++) {
         const EncodeJob &a = job[i];
@@ -2617,7 +2637,7 @@ static int launch_cells_both(const EncodeJob job[2], int dtype, int B, int H, in
     PKV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     const uint32_t vg = side[1].ngroups;
     kern<<<2u * vg, 512, lds, s>>>(side[0], side[1], B, H, T, job[0].par_stride, job[0].perm, job[0].perm_block,
-                                   vg <= kBothTurns ? vg >> 8 : 0u, job[0].rot);
+                                   vg <= kBothTurns ? vg >> 8 : 0u, job[0].rot, close);
     PKV_HIP_CHECK(hipGetLastError());
     return PKV_OK;
 }
@@ -2627,7 +2647,8 @@ static int encode_both(const EncodeJob job[2], int dtype, int B, int H, int T, u
     int rc;
     const OncePlan pk = once_plan_of(true, job[0], dtype, B, H, T), pv = once_plan_of(false, job[1], dtype, B, H, T);
     const bool one_launch = pk.threads && pk.threads == pv.threads && (job[0].bits > 4) == (job[1].bits > 4);
-    const uint32_t closes = one_launch ? pk.nwg + pv.nwg : 0u;
+    const bool both = cells_in_one_launch(job, pk, pv, B, H, T);
+    const uint32_t closes = one_launch ? pk.nwg + pv.nwg : both ? 2u * (uint32_t)(T / 128) * (uint32_t)B : 0u;
     ClosedEncode ce;
     ScanHandle sh;
     if ((rc = prepare_scan_state((uint32_t)state_words(true, B, H, T), &sh, s, true,
@@ -2639,9 +2660,11 @@ static int encode_both(const EncodeJob job[2], int dtype, int B, int H, int T, u
         if ((rc = ce.launched(sh))) return rc;
         return ce.wait(k_size, job[0].bits, v_size, job[1].bits);
     }
-    if (cells_in_one_launch(job, pk, pv, B, H, T)) {
-        if ((rc = launch_cells_both(job, dtype, B, H, T, sh.st, sh.second, s))) return rc;
-        return finish_encode(sh, k_size, job[0].bits, s, v_size, job[1].bits);
+    if (both) {
+        if ((rc = ce.begin(sh, closes, 2, job[0].bits, s))) return rc;
+        if ((rc = launch_cells_both(job, dtype, B, H, T, sh.st, sh.second, ce.close, s))) return rc;
+        if ((rc = ce.launched(sh))) return rc;
+        return ce.wait(k_size, job[0].bits, v_size, job[1].bits);
     }
     if ((rc = launch_quant_encode<true>(job[0], dtype, B, H, T, sh.st, EncodeClose{}, s))) return rc;
     if ((rc = launch_quant_encode<false>(job[1], dtype, B, H, T, sh.second, EncodeClose{}, s))) return rc;
