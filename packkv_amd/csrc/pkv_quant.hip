@@ -1098,6 +1098,27 @@ __device__ __forceinline__ void cell_token_minmax_halves(const uint2 xr[16], flo
         : "+v"(mn), "+v"(mx));
 }
 
+// The end of the launch, which closes by itself (as once_close does it): every workgroup counts itself out, sixteen to a counter and
+// the sixteens on one, and the last one hands the outcome over and clears the state.  Against a kernel for that behind it, median
+// repacking's order and encodes of B x 8 heads x 8192 fp16 tokens: B = 4 83.8 -> 81.4 us, 8 145 -> 138, 12 192 -> 184, 16 243 -> 235, 24 348 -> 343, 32 the same.
+__device__ __forceinline__ void cells_close(const EncodeClose &c, uint32_t &last_of_all) {
+    if (c.total == 0) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // what this wavefront wrote into the state has arrived
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const uint32_t group = blockIdx.x / kCloseGroup, groups = (c.total + kCloseGroup - 1u) / kCloseGroup;
+        auto count = [&](uint32_t at) { return __hip_atomic_fetch_add(reinterpret_cast<uint32_t *>(c.count + kCloseStride * at), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u; };
+        const bool last = count(1u + group) == min(kCloseGroup, c.total - group * kCloseGroup) && count(0u) == groups;
+        if (last) publish_outcomes(c.st, c.second, c.last, c.slot, c.tag, c.bits);
+        last_of_all = last ? 1u : 0u;
+    }
+    __syncthreads();
+    if (last_of_all == 0u) return;
+    // (ordinary stores: nothing reads the state any more before the launch has ended)
+    for (uint32_t i = threadIdx.x; i < c.n / 2u; i += blockDim.x) reinterpret_cast<uint4 *>(c.words)[i] = make_uint4(0u, 0u, 0u, 0u);
+    if (threadIdx.x == 0 && (c.n & 1u)) c.words[c.n - 1u] = 0;
+}
+
 // ---- K, all heads in one workgroup, x read ONCE as cells ----------------------------------------
 // The round-major encoder above reads a round's rows twice: once row-wise for the token parameters (the trip that
 // goes to HBM and whose latency every round waits out) and again as cells.  Here a round is read as cells only; the
@@ -1303,12 +1324,13 @@ __global__ void __launch_bounds__(256) k_quant_encode_cells_kernel(
     const uint16_t *__restrict__ x, int B, int H, int T, const XRows xs, float rel, uint16_t *__restrict__ scale,
     uint16_t *__restrict__ zero, uint8_t *__restrict__ stream, uint64_t capacity, uint32_t *__restrict__ info,
     ScanState *st, int W, uint32_t ngroups, uint32_t bound, uint64_t base, int par_stride,
-    const uint32_t *__restrict__ perm, int perm_block, const Stagger stagger, int nsg, uint64_t *xw, const Rot rot) {
+    const uint32_t *__restrict__ perm, int perm_block, const Stagger stagger, int nsg, uint64_t *xw, const Rot rot, const EncodeClose c) {
     extern __shared__ __align__(16) uint8_t gbuf[];        // H block slots of `bound` bytes
     __shared__ KCellsLds lds;
     k_quant_encode_cells<DT, WIDE, PERM, XCH, STRIDED, ROT>(threadIdx.x, gbuf, lds, x, B, H, T, xs, rel, scale, zero, stream, capacity,
                                                                    info, st, W, ngroups, bound, base, par_stride, perm, perm_block, stagger,
                                                                    nsg, xw, rot);
+    if (!XCH) cells_close(c, lds.idx);                     // (runs that wait for each other are closed by finish_encode)
 }
 
 // ---- K, up to four heads: round-major, several groups to a workgroup ---------------------------
@@ -1876,11 +1898,12 @@ __global__ void __launch_bounds__(512 * v_cell_segs(WIDE)) v_quant_encode_cells_
     uint16_t *__restrict__ zero, uint8_t *__restrict__ stream, uint64_t capacity, uint32_t *__restrict__ info,
     ScanState *st, int W, uint32_t ngroups, uint32_t unit_slot, uint64_t base, int par_stride,
     const uint32_t *__restrict__ perm, int perm_block, const uint16_t *__restrict__ scale_in,
-    const uint16_t *__restrict__ zero_in, const Stagger stagger, int nsg = 1, uint64_t *xw = nullptr) {
+    const uint16_t *__restrict__ zero_in, const Stagger stagger, int nsg, uint64_t *xw, const EncodeClose c) {
     extern __shared__ __align__(16) uint8_t gbuf[];        // 16 blocks x 4 units x unit_slot bytes
     __shared__ VCellsLds<WIDE> lds;
     v_quant_encode_cells<DT, WIDE, PERM, XCH, STRIDED>(gbuf, lds, x, B, H, T, xs, rel, scale, zero, stream, capacity, info, st, W, ngroups,
                                                        unit_slot, base, par_stride, perm, perm_block, scale_in, zero_in, stagger, nsg, xw);
+    if (!XCH) cells_close(c, lds.idx);                     // (runs that wait for each other are closed by finish_encode)
 }
 
 // ---- K and V in one launch -----------------------------------------------------------------------
@@ -1901,25 +1924,6 @@ struct CellsSide {
     uint32_t ngroups, slot;                // K: bytes of a block's slot, V: of a unit's
     const uint16_t *scale_in, *zero_in;
 };
-// The end of the launch, which closes by itself (as once_close does it): every workgroup counts itself out, sixteen to a counter and
-// the sixteens on one, and the last one hands the outcome over and clears the state.  Against a kernel for that behind it, median
-// repacking's order and encodes of B x 8 heads x 8192 fp16 tokens: B = 4 83.8 -> 81.4 us, 8 145 -> 138, 12 192 -> 184, 16 243 -> 235, 24 348 -> 343, 32 the same.
-__device__ __forceinline__ void cells_close(const EncodeClose &c, uint32_t &last_of_all) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // what this wavefront wrote into the state has arrived
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const uint32_t group = blockIdx.x / kCloseGroup, groups = (c.total + kCloseGroup - 1u) / kCloseGroup;
-        auto count = [&](uint32_t at) { return __hip_atomic_fetch_add(reinterpret_cast<uint32_t *>(c.count + kCloseStride * at), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u; };
-        const bool last = count(1u + group) == min(kCloseGroup, c.total - group * kCloseGroup) && count(0u) == groups;
-        if (last) publish_outcomes(c.st, c.second, c.last, c.slot, c.tag, c.bits);
-        last_of_all = last ? 1u : 0u;
-    }
-    __syncthreads();
-    if (last_of_all == 0u) return;
-    // (ordinary stores: nothing reads the state any more before the launch has ended)
-    for (uint32_t i = threadIdx.x; i < c.n / 2u; i += blockDim.x) reinterpret_cast<uint4 *>(c.words)[i] = make_uint4(0u, 0u, 0u, 0u);
-    if (threadIdx.x == 0 && (c.n & 1u)) c.words[c.n - 1u] = 0;
-}
 template <int DT, bool PERM, bool ROT>
 __global__ void __launch_bounds__(512) kv_quant_encode_cells_kernel(const CellsSide k, const CellsSide v, int B, int H, int T, int par_stride,
                                                                     const uint32_t *__restrict__ perm, int perm_block, uint32_t turns, const Rot rot, const EncodeClose c) {
@@ -2476,6 +2480,18 @@ static OnceSide once_side(bool is_k, const EncodeJob &job, const OncePlan &p, in
     return a;
 }
 
+// Workgroups of a launch that closes by itself; 0: finish_encode follows.  The cells kernels of up to eight heads do so up to 2048
+// workgroups (B x 8 heads x 8192 fp16 tokens, K and V, us: B = 3 40.8 -> 39.5 and 42.3 -> 40.6, 6 54.5 -> 52.5 and 57 -> 54.4, 16 102 -> 99.8 and 120 ->
+// 108; bf16 B = 8 71.6 -> 69.0 and 65.7 -> 62.7); beyond, what a workgroup waits for at its end costs as much or more (K of 32 161.3 and 161.1,
+// of 8 x 65536 tokens 304 -> 308), and runs of eight heads that wait for each other lose (4 x 32 heads x 16384 179.4 -> 183.2 and 197 -> 199).
+constexpr uint64_t kCloseCells = 2048;
+static uint32_t encode_closes(bool is_k, const EncodeJob &job, int dtype, int B, int H, int T) {
+    if (const OncePlan p = once_plan_of(is_k, job, dtype, B, H, T); p.threads) return p.nwg;
+    if ((H <= 4 && !job.perm) || H > kSubBlocks) return 0;
+    const uint64_t n = (uint64_t)(T / (is_k ? 64 : 128)) * (uint64_t)B;
+    return n <= kCloseCells ? (uint32_t)n : 0u;
+}
+
 template <bool IS_K>
 static int launch_quant_encode(const EncodeJob &job, int dtype, int B, int H, int T, ScanState *st, const EncodeClose &close, hipStream_t s) {
     const void *x = job.x;
@@ -2525,7 +2541,7 @@ static int launch_quant_encode(const EncodeJob &job, int dtype, int B, int H, in
                 if ((rc = stagger_for(reinterpret_cast<const void *>(cells), (int)threads, lds, ngroups, &sg))) return rc;
                 cells<<<ngroups, threads, lds, s>>>((const uint16_t *)x, B, H, T, xs, rel, (uint16_t *)scale, (uint16_t *)zero,
                                                 stream, capacity, info, st, bits, ngroups, unit_slot, base, par_stride, perm, perm_block,
-                                                (const uint16_t *)scale_in, (const uint16_t *)zero_in, sg, 1, nullptr);
+                                                (const uint16_t *)scale_in, (const uint16_t *)zero_in, sg, 1, nullptr, close);
             } else {
                 if ((rc = stagger_for(reinterpret_cast<const void *>(kern), 512, lds, ngroups, &sg))) return rc;
                 kern<<<ngroups, 512, lds, s>>>((const uint16_t *)x, B, H, T, xs, rel, (uint16_t *)scale, (uint16_t *)zero,
@@ -2549,7 +2565,7 @@ static int launch_quant_encode(const EncodeJob &job, int dtype, int B, int H, in
                 auto cells = cells_kernel<true>(bits, dtype, perm != nullptr, false, xs.st != kHeadDim, job.rot.cos != nullptr);
                 if ((rc = stagger_for(reinterpret_cast<const void *>(cells), 256, lds, nwg, &sg))) return rc;
                 cells<<<nwg, 256, lds, s>>>((const uint16_t *)x, B, H, T, xs, rel, (uint16_t *)scale, (uint16_t *)zero, stream,
-                                            capacity, info, st, bits, nwg, slot, base, par_stride, perm, perm_block, sg, 1, nullptr, job.rot);
+                                            capacity, info, st, bits, nwg, slot, base, par_stride, perm, perm_block, sg, 1, nullptr, job.rot, close);
             } else {
                 if ((rc = stagger_for(reinterpret_cast<const void *>(kern), 256, lds, nwg, &sg))) return rc;
                 kern<<<nwg, 256, lds, s>>>((const uint16_t *)x, B, H, T, xs, rel, (uint16_t *)scale, (uint16_t *)zero, stream,
@@ -2564,7 +2580,7 @@ static int launch_quant_encode(const EncodeJob &job, int dtype, int B, int H, in
             if ((rc = stagger_for(reinterpret_cast<const void *>(kern), 256, lds, nsub, &sg))) return rc;
             kern<<<nsub, 256, lds, s>>>((const uint16_t *)x, B, H, T, xs, rel, (uint16_t *)scale, (uint16_t *)zero, stream,
                                         capacity, info, st, bits, nsub, slot, base, par_stride, nullptr, 0, sg, nsg,
-                                        st->status + nsub, job.rot);
+                                        st->status + nsub, job.rot, EncodeClose{});
         } else {                                     // V, more than eight heads: the same runs of eight
             const uint32_t unit_slot = (uint32_t)(((bound - 8u) / 4u + 15u) & ~15u);
             const uint32_t lds = 64u * unit_slot + 64u;
@@ -2576,7 +2592,7 @@ static int launch_quant_encode(const EncodeJob &job, int dtype, int B, int H, in
             if ((rc = stagger_for(reinterpret_cast<const void *>(kern), (int)threads, lds, nruns_all, &sg))) return rc;
             kern<<<nruns_all, threads, lds, s>>>((const uint16_t *)x, B, H, T, xs, rel, (uint16_t *)scale, (uint16_t *)zero,
                                              stream, capacity, info, st, bits, nruns_all, unit_slot, base, par_stride, nullptr, 0,
-                                             nullptr, nullptr, sg, nruns, st->status + nruns_all);
+                                             nullptr, nullptr, sg, nruns, st->status + nruns_all, EncodeClose{});
         }
         PKV_HIP_CHECK(hipGetLastError());
     }
@@ -2594,7 +2610,7 @@ static int run_quant_encode(const void *x, int dtype, int B, int H, int T, float
     EncodeJob job{x, dense_rows(H, T), rel, bits, stream, capacity, base, info, scale, zero, par_stride, perm, perm_block, scale_in, zero_in};
     int rc = check_job<IS_K>(job, dtype, B, H, T);
     if (rc) return rc;
-    const uint32_t closes = once_plan_of(IS_K, job, dtype, B, H, T).nwg;       // workgroups of a launch that closes by itself
+    const uint32_t closes = encode_closes(IS_K, job, dtype, B, H, T);
     ClosedEncode ce;
     ScanHandle sh;
     if ((rc = prepare_scan_state((uint32_t)state_words(IS_K, B, H, T) + (closes ? close_words(closes) : 0u), &sh, s, size_out || ms_out))) return rc;

@@ -586,3 +586,21 @@ def test_both_sides_in_one_launch(cuda, B, H, T, form, dtype):
             assert torch.equal(got[:, 0], ref[:, 0] + used) and torch.equal(got[:, 1], ref[:, 1])
             assert torch.equal(scale[:, before:before + T], want[i]["scale"]) and torch.equal(zero[:, before:before + T], want[i]["zero"])
             assert not scale[:, :before].any() and not scale[:, before + T:].any() and not stream[:used].any()
+
+
+# Either side of the sizes up to which the encoders that walk close by themselves: 2048 workgroups of K, 2048 of V.
+@pytest.mark.parametrize("H,T", [(5, 131072), (5, 131200), (6, 262144), (6, 262272)])
+def test_encoders_that_walk_and_close_by_themselves(cuda, H, T):
+    k, v = synth.make_kv(1, H, T, seed=T, device=cuda)
+    for is_k, x, enc in ((True, k, ops.k_quant_encode), (False, v, ops.v_quant_encode)):
+        _say("closing", H, T, is_k)
+        first = enc(x, 0.1)
+        with pytest.raises(RuntimeError, match="does not fit bits_len 3"):
+            enc(x, 0.1, 3)
+        for rep in range(2):                           # (after an error, and after a launch of its own: the state is clear)
+            r = enc(x, 0.1)
+            assert r["size"] == first["size"] and torch.equal(r["stream"][:r["size"]], first["stream"][:r["size"]])
+            assert all(torch.equal(r[f].view(torch.int16), first[f].view(torch.int16)) for f in ("info", "scale", "zero"))
+        codes = torch.empty(T, H * 128, dtype=torch.uint8, device=cuda)
+        (ops.k_decode if is_k else ops.v_decode)(r["stream"], r["info"], codes, *((64, 128) if is_k else (128, 64)), r["bits"])
+        assert torch.equal(codes, ops.quant_codes(x, 0.1)[0])
