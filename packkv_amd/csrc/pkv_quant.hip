@@ -1098,6 +1098,7 @@ __device__ __forceinline__ void cell_token_minmax_halves(const uint2 xr[16], flo
         : "+v"(mn), "+v"(mx));
 }
 
+constexpr uint64_t kCloseCells = 2048;       // workgroups of one side's launch, at most (encode_closes)
 // The end of the launch, which closes by itself (as once_close does it): every workgroup counts itself out, sixteen to a counter and
 // the sixteens on one, and the last one hands the outcome over and clears the state.  Against a kernel for that behind it, median
 // repacking's order and encodes of B x 8 heads x 8192 fp16 tokens: B = 4 83.8 -> 81.4 us, 8 145 -> 138, 12 192 -> 184, 16 243 -> 235, 24 348 -> 343, 32 the same.
@@ -1978,7 +1979,7 @@ namespace pkv {
 template <bool WIDE>
 __global__ void __launch_bounds__(256) k_code_cells_kernel(
     const uint8_t *__restrict__ codes, int hidden, uint8_t *__restrict__ stream, uint64_t capacity,
-    uint32_t *__restrict__ info, ScanState *st, int W, uint32_t ngroups, uint32_t bound, const Stagger stagger) {
+    uint32_t *__restrict__ info, ScanState *st, int W, uint32_t ngroups, uint32_t bound, const Stagger stagger, const EncodeClose c) {
     extern __shared__ __align__(16) uint8_t gbuf[];        // 8 block slots of `bound` bytes
     __shared__ uint32_t s_idx;
     __shared__ uint64_t s_off;
@@ -1988,7 +1989,10 @@ __global__ void __launch_bounds__(256) k_code_cells_kernel(
     if (tid == 0) s_idx = atomicAdd(&st->ticket, 1u);
     __syncthreads();
     const uint32_t gidx = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_idx);
-    if (gidx >= ngroups) return;
+    if (gidx >= ngroups) {
+        cells_close(c, s_idx);
+        return;
+    }
     const int j = tid >> 5, t = tid & 31;                 // block of the group, lane of the unit
     const uint32_t per_row = (uint32_t)hidden / 1024u;    // groups per context block
     const uint32_t cb = gidx / per_row, hg = gidx % per_row;
@@ -2031,18 +2035,20 @@ __global__ void __launch_bounds__(256) k_code_cells_kernel(
         const uint64_t off = lookback_offset(st, gidx, bytes, true);
         if (tid == 0) {
             s_off = off;
-            if (gidx == ngroups - 1) st->total = off + bytes;
+            if (gidx == ngroups - 1) __hip_atomic_store(&st->total, off + bytes, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (off + bytes > capacity) atomicExch(&st->error, (uint32_t)PKV_ERR_CAPACITY);
         }
     }
     __syncthreads();
     const uint64_t off = s_off;
-    if (off + bytes > capacity) return;
-    if (tid < kSubBlocks) {
-        info[2 * (size_t)(gidx * (uint32_t)kSubBlocks + tid)] = (uint32_t)(off + blk_off[tid]);
-        info[2 * (size_t)(gidx * (uint32_t)kSubBlocks + tid) + 1] = blk_off[tid + 1] - blk_off[tid];
+    if (off + bytes <= capacity) {
+        if (tid < kSubBlocks) {
+            info[2 * (size_t)(gidx * (uint32_t)kSubBlocks + tid)] = (uint32_t)(off + blk_off[tid]);
+            info[2 * (size_t)(gidx * (uint32_t)kSubBlocks + tid) + 1] = blk_off[tid + 1] - blk_off[tid];
+        }
+        copy_out32(stream + off + blk_off[j], blk, my_off, t);
     }
-    copy_out32(stream + off + blk_off[j], blk, my_off, t);
+    cells_close(c, s_idx);
 }
 
 // V: the thread roles of v_quant_encode_cells_kernel (a wavefront = one 128-channel slice with both rounds of an
@@ -2050,7 +2056,7 @@ __global__ void __launch_bounds__(256) k_code_cells_kernel(
 template <bool WIDE>
 __global__ void __launch_bounds__(512 * v_cell_segs(WIDE)) v_code_cells_kernel(
     const uint8_t *__restrict__ codes, int hidden, uint8_t *__restrict__ stream, uint64_t capacity,
-    uint32_t *__restrict__ info, ScanState *st, int W, uint32_t ngroups, uint32_t unit_slot, const Stagger stagger) {
+    uint32_t *__restrict__ info, ScanState *st, int W, uint32_t ngroups, uint32_t unit_slot, const Stagger stagger, const EncodeClose c) {
     extern __shared__ __align__(16) uint8_t gbuf[];        // 16 blocks x 4 units x unit_slot bytes
     __shared__ uint32_t s_idx;
     __shared__ uint64_t s_off;
@@ -2062,7 +2068,10 @@ __global__ void __launch_bounds__(512 * v_cell_segs(WIDE)) v_code_cells_kernel(
     if (tid == 0) s_idx = atomicAdd(&st->ticket, 1u);
     __syncthreads();
     const uint32_t gidx = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_idx);      // uniform: the rows' addresses become scalar
-    if (gidx >= ngroups) return;
+    if (gidx >= ngroups) {
+        cells_close(c, s_idx);
+        return;
+    }
     const int j = (tid >> 6) & 7, seg = tid >> 9, rp = (tid >> 5) & 1, t = tid & 31;
     const uint32_t per_row = (uint32_t)hidden / 1024u;
     const uint32_t cb = gidx / per_row, hg = gidx % per_row;
@@ -2132,28 +2141,30 @@ __global__ void __launch_bounds__(512 * v_cell_segs(WIDE)) v_code_cells_kernel(
         const uint64_t off = lookback_offset(st, gidx, bytes, true);
         if (tid == 0) {
             s_off = off;
-            if (gidx == ngroups - 1) st->total = off + bytes;
+            if (gidx == ngroups - 1) __hip_atomic_store(&st->total, off + bytes, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (off + bytes > capacity) atomicExch(&st->error, (uint32_t)PKV_ERR_CAPACITY);
         }
     }
     __syncthreads();
     const uint64_t off = s_off;
-    if (off + bytes > capacity) return;
-    if (tid < 16) {
-        info[2 * (size_t)(gidx * 16u + tid)] = (uint32_t)(off + blk_off[tid]);
-        info[2 * (size_t)(gidx * 16u + tid) + 1] = blk_off[tid + 1] - blk_off[tid];
-    }
-    const int q = (tid >> 5) & 15;                         // half-wavefront q copies block q (of two segments each its own)
-    uint8_t *dst = stream + off + blk_off[q];
-    uint32_t cum = 0;
+    if (off + bytes <= capacity) {
+        if (tid < 16) {
+            info[2 * (size_t)(gidx * 16u + tid)] = (uint32_t)(off + blk_off[tid]);
+            info[2 * (size_t)(gidx * 16u + tid) + 1] = blk_off[tid + 1] - blk_off[tid];
+        }
+        const int q = (tid >> 5) & 15;                         // half-wavefront q copies block q (of two segments each its own)
+        uint8_t *dst = stream + off + blk_off[q];
+        uint32_t cum = 0;
 #pragma unroll
-    for (int un = 0; un < 4; un++) {
-        const uint32_t n = s_usz[q][un];
-        const bool mine = SEGS == 1 || un >> 1 == seg;
-        if (mine) copy_out32(dst + 8 + cum, gbuf + (size_t)(q * 4 + un) * unit_slot, n, t);
-        cum += n;
-        if (mine && t == un) reinterpret_cast<uint16_t *>(dst)[un] = (uint16_t)cum;
+        for (int un = 0; un < 4; un++) {
+            const uint32_t n = s_usz[q][un];
+            const bool mine = SEGS == 1 || un >> 1 == seg;
+            if (mine) copy_out32(dst + 8 + cum, gbuf + (size_t)(q * 4 + un) * unit_slot, n, t);
+            cum += n;
+            if (mine && t == un) reinterpret_cast<uint16_t *>(dst)[un] = (uint16_t)cum;
+        }
     }
+    cells_close(c, s_idx);
 }
 
 // Launch of the two kernels above (pkv_codec.hip decides when they apply): `st` is a prepared scan state of
@@ -2164,11 +2175,18 @@ bool code_cells_serve(bool is_k, int ctx_len, int hidden) {
     const OncePlan p = hidden % kHeadDim ? OncePlan{0, 0, 0, 0} : code_plan(is_k, ctx_len, hidden);
     return p.threads && hidden / kHeadDim % p.run == 0;    // (code_encode_once_kernel knows whole runs only)
 }
-uint32_t code_cells_closes(bool is_k, int ctx_len, int hidden) { return code_plan(is_k, ctx_len, hidden).nwg; }
 static uint32_t code_cells_groups(bool is_k, int ctx_len, int hidden) { return (uint32_t)(ctx_len / (is_k ? 64 : 128)) * (uint32_t)(hidden / 1024); }
+// (the kernels that walk close by themselves up to 2048 workgroups, K and V of 8 x 128 channels of 4-bit codes, us: 32768 rows 32.4 -> 31.0
+// and 29.9 -> 28.6, 65536 47.4 -> 45.2 and 39.0 -> 36.8, 131072 69.5 -> 68.7 and 61.8 -> 59.4; 262144 rows 118.4 and 119.0 for K)
+uint32_t code_cells_closes(bool is_k, int ctx_len, int hidden) {
+    if (const OncePlan p = code_plan(is_k, ctx_len, hidden); p.threads) return p.nwg;
+    const uint32_t n = code_cells_groups(is_k, ctx_len, hidden);
+    return n <= kCloseCells ? n : 0u;
+}
 uint32_t code_cells_words(bool is_k, int ctx_len, int hidden) {
     const OncePlan p = code_plan(is_k, ctx_len, hidden);
-    return p.threads ? p.nwg + close_words(p.nwg) : code_cells_groups(is_k, ctx_len, hidden);
+    const uint32_t closes = code_cells_closes(is_k, ctx_len, hidden);
+    return (p.threads ? p.nwg : code_cells_groups(is_k, ctx_len, hidden)) + (closes ? close_words(closes) : 0u);
 }
 int launch_code_cells(bool is_k, const uint8_t *codes, int ctx_len, int hidden, int bits, uint32_t bound, uint8_t *stream,
                       uint64_t capacity, uint32_t *info, ScanState *st, const EncodeClose &close, hipStream_t s) {
@@ -2186,7 +2204,7 @@ int launch_code_cells(bool is_k, const uint8_t *codes, int ctx_len, int hidden, 
         const uint32_t lds = (uint32_t)kSubBlocks * slot + 32u;
         auto kern = bits > 4 ? k_code_cells_kernel<true> : k_code_cells_kernel<false>;
         if ((rc = stagger_for(reinterpret_cast<const void *>(kern), 256, lds, ngroups, &sg))) return rc;
-        kern<<<ngroups, 256, lds, s>>>(codes, hidden, stream, capacity, info, st, bits, ngroups, slot, sg);
+        kern<<<ngroups, 256, lds, s>>>(codes, hidden, stream, capacity, info, st, bits, ngroups, slot, sg, close);
     } else {
         const uint32_t unit_slot = (uint32_t)(((bound - 8u) / 4u + 15u) & ~15u);
         const uint32_t lds = 64u * unit_slot + 64u;
@@ -2194,7 +2212,7 @@ int launch_code_cells(bool is_k, const uint8_t *codes, int ctx_len, int hidden, 
         PKV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         const unsigned threads = 512u * v_cell_segs(bits > 4);
         if ((rc = stagger_for(reinterpret_cast<const void *>(kern), (int)threads, lds, ngroups, &sg))) return rc;
-        kern<<<ngroups, threads, lds, s>>>(codes, hidden, stream, capacity, info, st, bits, ngroups, unit_slot, sg);
+        kern<<<ngroups, threads, lds, s>>>(codes, hidden, stream, capacity, info, st, bits, ngroups, unit_slot, sg, close);
     }
     PKV_HIP_CHECK(hipGetLastError());
     return PKV_OK;
@@ -2484,7 +2502,6 @@ static OnceSide once_side(bool is_k, const EncodeJob &job, const OncePlan &p, in
 // workgroups (B x 8 heads x 8192 fp16 tokens, K and V, us: B = 3 40.8 -> 39.5 and 42.3 -> 40.6, 6 54.5 -> 52.5 and 57 -> 54.4, 16 102 -> 99.8 and 120 ->
 // 108; bf16 B = 8 71.6 -> 69.0 and 65.7 -> 62.7); beyond, what a workgroup waits for at its end costs as much or more (K of 32 161.3 and 161.1,
 // of 8 x 65536 tokens 304 -> 308), and runs of eight heads that wait for each other lose (4 x 32 heads x 16384 179.4 -> 183.2 and 197 -> 199).
-constexpr uint64_t kCloseCells = 2048;
 static uint32_t encode_closes(bool is_k, const EncodeJob &job, int dtype, int B, int H, int T) {
     if (const OncePlan p = once_plan_of(is_k, job, dtype, B, H, T); p.threads) return p.nwg;
     if ((H <= 4 && !job.perm) || H > kSubBlocks) return 0;

@@ -604,3 +604,23 @@ def test_encoders_that_walk_and_close_by_themselves(cuda, H, T):
         codes = torch.empty(T, H * 128, dtype=torch.uint8, device=cuda)
         (ops.k_decode if is_k else ops.v_decode)(r["stream"], r["info"], codes, *((64, 128) if is_k else (128, 64)), r["bits"])
         assert torch.equal(codes, ops.quant_codes(x, 0.1)[0])
+
+
+@pytest.mark.parametrize("T", [32768, 131072, 131200])
+@pytest.mark.parametrize("bits", [4, 5])
+def test_code_encoders_that_walk_and_close_by_themselves(cuda, T, bits):
+    g = torch.Generator(device=cuda).manual_seed(T + bits)
+    codes = torch.randint(0, 1 << bits, (T, 1024), generator=g, dtype=torch.uint8, device=cuda)
+    codes[T // 2:] &= 3
+    stream, info = torch.zeros(T * 1024, dtype=torch.uint8, device=cuda), torch.zeros(T // 8, 2, dtype=torch.uint32, device=cuda)
+    back = torch.empty_like(codes)
+    for is_k in (True, False):
+        _say("codes, closing", T, bits, is_k)
+        size = ops.encode_p(is_k, codes, stream, info, 16, bits)
+        ops.decode_p(is_k, stream, info, back, 16, bits)
+        assert torch.equal(back, codes)
+        want, table = stream[:size].clone(), info.clone()
+        with pytest.raises(RuntimeError):              # (a stream that does not fit; the state is clear behind it)
+            ops.encode_p(is_k, codes, stream[:size - 2], info, 16, bits)
+        assert ops.encode_p(is_k, codes, stream, info, 16, bits) == size
+        assert torch.equal(stream[:size], want) and torch.equal(info.view(torch.int32), table.view(torch.int32))
