@@ -174,17 +174,17 @@ PyObject *plan_step(PyObject *, PyObject *const *o, Py_ssize_t n) {
     int plan_dev = -1, rows = 0;
     const int dev = here();
     if (!q || !PyLong_CheckExact(o[0]) || !integer(o[1], &plan_dev) || !integer(o[2], &rows) || plan_dev != dev || !dense(*q, dev)) Py_RETURN_NONE;
-    pkv_attn_args *a = (pkv_attn_args *)PyLong_AsVoidPtr(o[0]);
+    // (a copy: the plan's own q, out and rows stay what its owner has set, and keeps alive)
+    pkv_attn_args a = *(const pkv_attn_args *)PyLong_AsVoidPtr(o[0]);
     const int64_t d = q->dim();
-    if ((d != 3 && (d != 4 || q->size(2) != 1)) || q->size(0) != a->B || q->size(1) != a->Hq || q->size(d - 1) != 128 ||
-        !half(*q) || code(*q) != a->dtype || rows < 1 || rows > a->win_stride) Py_RETURN_NONE;
+    if ((d != 3 && (d != 4 || q->size(2) != 1)) || q->size(0) != a.B || q->size(1) != a.Hq || q->size(d - 1) != 128 ||
+        !half(*q) || code(*q) != a.dtype || a.flags || rows < 1 || rows > a.win_stride) Py_RETURN_NONE;
     at::Tensor out = at::empty(q->sizes(), q->options());
-    a->q = at_ptr<void>(*q);
-    a->out = at_ptr<void>(out);
-    a->T_w = rows;
-    const pkv_attn_args args = *a;
+    a.q = at_ptr<void>(*q);
+    a.out = at_ptr<void>(out);
+    a.T_w = rows;
     const pkv_stream_t s = stream(dev);
-    const int rc = call([&] { return lib.attn_decode(&args, nullptr, s); });
+    const int rc = call([&] { return lib.attn_decode(&a, nullptr, s); });
     return rc ? status(rc) : THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
 }

@@ -1243,7 +1243,10 @@ class AttnPlan:
 
     def step(self, q, win_len):
         """The result of the step for `q` -- [B, Hq, 128], or [B, Hq, 1, 128] -- with `win_len` window rows in use, in q's shape;
-        None where q is not what the plan was made for as it lies."""
+        None where q is not what the plan was made for as it lies, and for plans of the checking kernels (flags, noalloc).  The
+        plan's own query, output and window rows stay as they are."""
+        if self._fn_noalloc is not None:
+            return None
         served = _host().plan_step(*self._where, win_len, q)
         return _lib.check(served) if type(served) is int else served
 

@@ -174,6 +174,21 @@ def test_on_a_side_stream_and_while_capturing(cuda):
         assert (ops.attn_decode(q, ke, ve, kw, vw).float() - want.float()).abs().max() <= 2e-3
 
 
+def test_a_step_leaves_the_plan_as_it_is(cuda):
+    ke, ve, kw, vw, q = _cache(cuda, torch.float16)
+    other = q.flip(0).contiguous()
+    for form in ({"out_f32": True}, {"ref_rounding": True, "variant": 1}, {"noalloc": True}):
+        assert ops.AttnPlan(q, ke, ve, kw, vw, win_len=33, **form).step(q, 33) is None
+    plan = ops.AttnPlan(q, ke, ve, kw, vw, win_len=33)
+    want = plan().clone()
+    before, out = bytes(plan.args), plan.out
+    got = plan.step(other, 70)
+    assert bytes(plan.args) == before and (got.float() - ops.attn_decode(other, ke, ve, kw, vw, win_len=70).float()).abs().max() <= 2e-3
+    out.zero_()
+    again = plan()
+    assert again is out and (again.float() - want.float()).abs().max() <= 2e-3
+
+
 def test_a_function_mode_sees_the_general_code(cuda):
     ke, ve, _, _, q = _cache(cuda, torch.float16)
 
