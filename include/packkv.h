@@ -65,7 +65,8 @@ uint64_t pkv_block_bound(int is_k, int ctx_blk, int hid_blk, int bits);
  * up to 128 bits and a 4-bit length field at bits = 8.  A stream of such codes can be larger
  * than the code matrix: size the buffer with pkv_block_bound.
  * `capacity` = bytes available at `stream` (which must start at an even address); `size_out` (host, may be NULL)
- * receives the stream size and makes the call synchronous.  With size_out = NULL nothing is reported by the call
+ * receives the stream size and makes the call synchronous: the stream, block_info and the parameters are there, for work on
+ * any stream of the device.  With size_out = NULL nothing is reported by the call
  * itself, not even a stream that did not fit: ask pkv_encode_status afterwards.
  * The decoders (and the kq / wv products further down) take `stream_bytes`, the size of the buffer at `stream` --
  * what the reference's binding knows as compressed_buffer.numel(): a block whose block_info entry points outside

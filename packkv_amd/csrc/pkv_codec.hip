@@ -357,16 +357,16 @@ static int run_pack(bool is_k, const uint8_t *codes, uint8_t *stream, uint64_t c
                        (is_k ? (ctx_blk == 64 && hid_blk == 128) : (ctx_blk == 128 && hid_blk == 64)) &&
                        code_cells_serve(is_k, ctx_len, hidden_dim);
     if (cells) {
-        const uint32_t closes = code_cells_closes(is_k, ctx_len, hidden_dim);
-        if ((rc = prepare_scan_state(code_cells_words(is_k, ctx_len, hidden_dim), &sh, s, size_out || ms_out))) return rc;
+        const uint32_t closes = size_out ? 0u : code_cells_closes(is_k, ctx_len, hidden_dim);
+        if ((rc = prepare_scan_state(code_cells_words(is_k, ctx_len, hidden_dim) + (closes ? close_words(closes) : 0u), &sh, s, size_out || ms_out))) return rc;
         ClosedEncode ce;
-        if (closes && (rc = ce.begin(sh, closes, size_out ? 1 : 0, 0, s))) return rc;
+        if (closes && (rc = ce.begin(sh, closes, s))) return rc;
         LaunchTimer tm(s, ms_out != nullptr);
         if ((rc = tm.begin())) return rc;
         if ((rc = launch_code_cells(is_k, codes, ctx_len, hidden_dim, bits, cs.blk_cap, stream, capacity, info, sh.st, ce.close, s))) return rc;
         if (closes && (rc = ce.launched(sh))) return rc;
         if ((rc = tm.end(ms_out))) return rc;
-        return closes ? ce.wait(size_out, 0) : finish_encode(sh, size_out, 0, s);
+        return closes ? PKV_OK : finish_encode(sh, size_out, 0, s);
     }
     if (grouped) {
         const uint32_t ngroups = ((uint32_t)cs.nblocks + kPackGroup - 1) / kPackGroup;

@@ -1099,25 +1099,26 @@ __device__ __forceinline__ void cell_token_minmax_halves(const uint2 xr[16], flo
 }
 
 constexpr uint64_t kCloseCells = 2048;       // workgroups of one side's launch, at most (encode_closes)
-// The end of the launch, which closes by itself (as once_close does it): every workgroup counts itself out, sixteen to a counter and
-// the sixteens on one, and the last one hands the outcome over and clears the state.  Against a kernel for that behind it, median
-// repacking's order and encodes of B x 8 heads x 8192 fp16 tokens: B = 4 83.8 -> 81.4 us, 8 145 -> 138, 12 192 -> 184, 16 243 -> 235, 24 348 -> 343, 32 the same.
-__device__ __forceinline__ void cells_close(const EncodeClose &c, uint32_t &last_of_all) {
+// The end of a launch that closes by itself (ClosedEncode): every workgroup counts itself out, sixteen to a counter and the sixteens on
+// one (adding to one address takes 13 ns each, one after the other), and the last one leaves the outcome and clears the state.
+// Behind `waitcnt` this wavefront's accesses to the state have arrived.  The output has not: its lines may stay in this XCD's L2 until
+// the launch ends, so a host that learned of the end from here could read the stream's old bytes through another stream.
+__device__ __forceinline__ void encode_close(const EncodeClose &c, uint32_t &last_of_all) {
     if (c.total == 0) return;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // what this wavefront wrote into the state has arrived
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (threadIdx.x == 0) {
         const uint32_t group = blockIdx.x / kCloseGroup, groups = (c.total + kCloseGroup - 1u) / kCloseGroup;
         auto count = [&](uint32_t at) { return __hip_atomic_fetch_add(reinterpret_cast<uint32_t *>(c.count + kCloseStride * at), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u; };
         const bool last = count(1u + group) == min(kCloseGroup, c.total - group * kCloseGroup) && count(0u) == groups;
-        if (last) publish_outcomes(c.st, c.second, c.last, c.slot, c.tag, c.bits);
+        if (last) publish_outcomes(c.st, nullptr, c.last, nullptr, c.tag, 0);
         last_of_all = last ? 1u : 0u;
     }
     __syncthreads();
     if (last_of_all == 0u) return;
     // (ordinary stores: nothing reads the state any more before the launch has ended)
-    for (uint32_t i = threadIdx.x; i < c.n / 2u; i += blockDim.x) reinterpret_cast<uint4 *>(c.words)[i] = make_uint4(0u, 0u, 0u, 0u);
-    if (threadIdx.x == 0 && (c.n & 1u)) c.words[c.n - 1u] = 0;
+    for (uint32_t i = threadIdx.x; i < c.n / 2u; i += blockDim.x) reinterpret_cast<uint4 *>(c.st)[i] = make_uint4(0u, 0u, 0u, 0u);
+    if (threadIdx.x == 0 && (c.n & 1u)) reinterpret_cast<uint64_t *>(c.st)[c.n - 1u] = 0;
 }
 
 // ---- K, all heads in one workgroup, x read ONCE as cells ----------------------------------------
@@ -1331,7 +1332,7 @@ __global__ void __launch_bounds__(256) k_quant_encode_cells_kernel(
     k_quant_encode_cells<DT, WIDE, PERM, XCH, STRIDED, ROT>(threadIdx.x, gbuf, lds, x, B, H, T, xs, rel, scale, zero, stream, capacity,
                                                                    info, st, W, ngroups, bound, base, par_stride, perm, perm_block, stagger,
                                                                    nsg, xw, rot);
-    if (!XCH) cells_close(c, lds.idx);                     // (runs that wait for each other are closed by finish_encode)
+    if (!XCH) encode_close(c, lds.idx);                     // (runs that wait for each other are closed by finish_encode)
 }
 
 // ---- K, up to four heads: round-major, several groups to a workgroup ---------------------------
@@ -1904,7 +1905,7 @@ __global__ void __launch_bounds__(512 * v_cell_segs(WIDE)) v_quant_encode_cells_
     __shared__ VCellsLds<WIDE> lds;
     v_quant_encode_cells<DT, WIDE, PERM, XCH, STRIDED>(gbuf, lds, x, B, H, T, xs, rel, scale, zero, stream, capacity, info, st, W, ngroups,
                                                        unit_slot, base, par_stride, perm, perm_block, scale_in, zero_in, stagger, nsg, xw);
-    if (!XCH) cells_close(c, lds.idx);                     // (runs that wait for each other are closed by finish_encode)
+    if (!XCH) encode_close(c, lds.idx);                     // (runs that wait for each other are closed by finish_encode)
 }
 
 // ---- K and V in one launch -----------------------------------------------------------------------
@@ -1927,7 +1928,7 @@ struct CellsSide {
 };
 template <int DT, bool PERM, bool ROT>
 __global__ void __launch_bounds__(512) kv_quant_encode_cells_kernel(const CellsSide k, const CellsSide v, int B, int H, int T, int par_stride,
-                                                                    const uint32_t *__restrict__ perm, int perm_block, uint32_t turns, const Rot rot, const EncodeClose c) {
+                                                                    const uint32_t *__restrict__ perm, int perm_block, uint32_t turns, const Rot rot) {
     extern __shared__ __align__(16) uint8_t gbuf[];
     const Stagger stagger{0u, 0u};
     __shared__ union Lds { __device__ Lds() {} VCellsLds<false> v; KCellsLds k[2]; } lds;
@@ -1943,7 +1944,6 @@ __global__ void __launch_bounds__(512) kv_quant_encode_cells_kernel(const CellsS
                                                                        k.W, k.ngroups, k.slot, k.base, par_stride, perm, perm_block, stagger, 1,
                                                                        nullptr, rot);
     }
-    cells_close(c, lds.v.idx);
 }
 
 // `rows` (uniform: scalar registers) is the first of the 16 token rows, `lane_off` the lane's byte offset inside a
@@ -1990,7 +1990,7 @@ __global__ void __launch_bounds__(256) k_code_cells_kernel(
     __syncthreads();
     const uint32_t gidx = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_idx);
     if (gidx >= ngroups) {
-        cells_close(c, s_idx);
+        encode_close(c, s_idx);
         return;
     }
     const int j = tid >> 5, t = tid & 31;                 // block of the group, lane of the unit
@@ -2048,7 +2048,7 @@ __global__ void __launch_bounds__(256) k_code_cells_kernel(
         }
         copy_out32(stream + off + blk_off[j], blk, my_off, t);
     }
-    cells_close(c, s_idx);
+    encode_close(c, s_idx);
 }
 
 // V: the thread roles of v_quant_encode_cells_kernel (a wavefront = one 128-channel slice with both rounds of an
@@ -2069,7 +2069,7 @@ __global__ void __launch_bounds__(512 * v_cell_segs(WIDE)) v_code_cells_kernel(
     __syncthreads();
     const uint32_t gidx = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_idx);      // uniform: the rows' addresses become scalar
     if (gidx >= ngroups) {
-        cells_close(c, s_idx);
+        encode_close(c, s_idx);
         return;
     }
     const int j = (tid >> 6) & 7, seg = tid >> 9, rp = (tid >> 5) & 1, t = tid & 31;
@@ -2164,7 +2164,7 @@ __global__ void __launch_bounds__(512 * v_cell_segs(WIDE)) v_code_cells_kernel(
             if (mine && t == un) reinterpret_cast<uint16_t *>(dst)[un] = (uint16_t)cum;
         }
     }
-    cells_close(c, s_idx);
+    encode_close(c, s_idx);
 }
 
 // Launch of the two kernels above (pkv_codec.hip decides when they apply): `st` is a prepared scan state of
@@ -2176,8 +2176,8 @@ bool code_cells_serve(bool is_k, int ctx_len, int hidden) {
     return p.threads && hidden / kHeadDim % p.run == 0;    // (code_encode_once_kernel knows whole runs only)
 }
 static uint32_t code_cells_groups(bool is_k, int ctx_len, int hidden) { return (uint32_t)(ctx_len / (is_k ? 64 : 128)) * (uint32_t)(hidden / 1024); }
-// (the kernels that walk close by themselves up to 2048 workgroups, K and V of 8 x 128 channels of 4-bit codes, us: 32768 rows 32.4 -> 31.0
-// and 29.9 -> 28.6, 65536 47.4 -> 45.2 and 39.0 -> 36.8, 131072 69.5 -> 68.7 and 61.8 -> 59.4; 262144 rows 118.4 and 119.0 for K)
+// (as encode_closes: K of 1024 channels of 4-bit codes, calls without a size one after the other, us: 4096 rows 13.1 -> 9.8, 16384 13.4 -> 12.7, 32768
+// 22.1 -> 21.8, 65536 37.0 -> 36.4, 131072 60.3 -> 60.8; beyond, 262144 rows, 118.4 and 119.0)
 uint32_t code_cells_closes(bool is_k, int ctx_len, int hidden) {
     if (const OncePlan p = code_plan(is_k, ctx_len, hidden); p.threads) return p.nwg;
     const uint32_t n = code_cells_groups(is_k, ctx_len, hidden);
@@ -2185,8 +2185,7 @@ uint32_t code_cells_closes(bool is_k, int ctx_len, int hidden) {
 }
 uint32_t code_cells_words(bool is_k, int ctx_len, int hidden) {
     const OncePlan p = code_plan(is_k, ctx_len, hidden);
-    const uint32_t closes = code_cells_closes(is_k, ctx_len, hidden);
-    return (p.threads ? p.nwg : code_cells_groups(is_k, ctx_len, hidden)) + (closes ? close_words(closes) : 0u);
+    return p.threads ? p.nwg : code_cells_groups(is_k, ctx_len, hidden);
 }
 int launch_code_cells(bool is_k, const uint8_t *codes, int ctx_len, int hidden, int bits, uint32_t bound, uint8_t *stream,
                       uint64_t capacity, uint32_t *info, ScanState *st, const EncodeClose &close, hipStream_t s) {
@@ -2499,9 +2498,11 @@ static OnceSide once_side(bool is_k, const EncodeJob &job, const OncePlan &p, in
 }
 
 // Workgroups of a launch that closes by itself; 0: finish_encode follows.  The cells kernels of up to eight heads do so up to 2048
-// workgroups (B x 8 heads x 8192 fp16 tokens, K and V, us: B = 3 40.8 -> 39.5 and 42.3 -> 40.6, 6 54.5 -> 52.5 and 57 -> 54.4, 16 102 -> 99.8 and 120 ->
-// 108; bf16 B = 8 71.6 -> 69.0 and 65.7 -> 62.7); beyond, what a workgroup waits for at its end costs as much or more (K of 32 161.3 and 161.1,
-// of 8 x 65536 tokens 304 -> 308), and runs of eight heads that wait for each other lose (4 x 32 heads x 16384 179.4 -> 183.2 and 197 -> 199).
+// workgroups.  Calls without a size one after the other, a kernel behind -> by itself, 8 heads, fp16, us: K and V of 512 tokens 16.0 -> 12.7 and
+// 15.9 -> 12.7 (the host's launch), 4096 15.6 -> 14.4 and 16.0 -> 16.8, 2 x 8192 19.5 -> 19.3 and 21.5 -> 23.0 (what the runs have exchanged is cleared by
+// one workgroup), 4 x 8192 32.2 -> 31.5 and 31.3 -> 30.9, 8 x 8192 53.1 -> 52.6 and 47.1 -> 46.4, 16 x 8192 90.1 -> 90.5 and 108.4 -> 97.8.  Beyond, what a
+// workgroup waits for at its end costs as much or more (K of 32 x 8192 161.3 and 161.1, of 8 x 65536 304 -> 308), and runs of eight heads
+// that wait for each other lose (4 x 32 heads x 16384 179.4 -> 183.2 and 197 -> 199).
 static uint32_t encode_closes(bool is_k, const EncodeJob &job, int dtype, int B, int H, int T) {
     if (const OncePlan p = once_plan_of(is_k, job, dtype, B, H, T); p.threads) return p.nwg;
     if ((H <= 4 && !job.perm) || H > kSubBlocks) return 0;
@@ -2627,17 +2628,17 @@ static int run_quant_encode(const void *x, int dtype, int B, int H, int T, float
     EncodeJob job{x, dense_rows(H, T), rel, bits, stream, capacity, base, info, scale, zero, par_stride, perm, perm_block, scale_in, zero_in};
     int rc = check_job<IS_K>(job, dtype, B, H, T);
     if (rc) return rc;
-    const uint32_t closes = encode_closes(IS_K, job, dtype, B, H, T);
+    const uint32_t closes = size_out ? 0u : encode_closes(IS_K, job, dtype, B, H, T);
     ClosedEncode ce;
     ScanHandle sh;
     if ((rc = prepare_scan_state((uint32_t)state_words(IS_K, B, H, T) + (closes ? close_words(closes) : 0u), &sh, s, size_out || ms_out))) return rc;
-    if (closes && (rc = ce.begin(sh, closes, size_out ? 1 : 0, bits, s))) return rc;
+    if (closes && (rc = ce.begin(sh, closes, s))) return rc;
     LaunchTimer tm(s, ms_out != nullptr);
     if ((rc = tm.begin())) return rc;
     if ((rc = launch_quant_encode<IS_K>(job, dtype, B, H, T, sh.st, ce.close, s))) return rc;
     if (closes && (rc = ce.launched(sh))) return rc;
     if ((rc = tm.end(ms_out))) return rc;
-    return closes ? ce.wait(size_out, bits) : finish_encode(sh, size_out, bits, s);
+    return closes ? PKV_OK : finish_encode(sh, size_out, bits, s);
 }
 
 // K and V by the cells kernels in one launch: five to eight heads and codes of up to four bits on both sides, below the four
@@ -2652,7 +2653,7 @@ static bool cells_in_one_launch(const EncodeJob job[2], const OncePlan &pk, cons
     return !pk.threads && !pv.threads && H > 4 && H <= kSubBlocks && job[0].bits <= 4 && job[1].bits <= 4 &&
            job[0].xs.sh < (1ll << 31) - 128 && (uint64_t)(T / 128) * (uint64_t)B < kBothGroups;
 }
-static int launch_cells_both(const EncodeJob job[2], int dtype, int B, int H, int T, ScanState *k_st, ScanState *v_st, const EncodeClose &close, hipStream_t s) {
+static int launch_cells_both(const EncodeJob job[2], int dtype, int B, int H, int T, ScanState *k_st, ScanState *v_st, hipStream_t s) {
     CellsSide side[2];
     for (int i = 0; i < 2; i++) {
         const EncodeJob &a = job[i];
@@ -2670,7 +2671,7 @@ static int launch_cells_both(const EncodeJob job[2], int dtype, int B, int H, in
     PKV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     const uint32_t vg = side[1].ngroups;
     kern<<<2u * vg, 512, lds, s>>>(side[0], side[1], B, H, T, job[0].par_stride, job[0].perm, job[0].perm_block,
-                                   vg <= kBothTurns ? vg >> 8 : 0u, job[0].rot, close);
+                                   vg <= kBothTurns ? vg >> 8 : 0u, job[0].rot);
     PKV_HIP_CHECK(hipGetLastError());
     return PKV_OK;
 }
@@ -2678,29 +2679,18 @@ static int launch_cells_both(const EncodeJob job[2], int dtype, int B, int H, in
 // K and V (checked jobs) with one wait; in one launch where both take a group's tokens at once.
 static int encode_both(const EncodeJob job[2], int dtype, int B, int H, int T, uint64_t *k_size, uint64_t *v_size, hipStream_t s) {
     int rc;
-    const OncePlan pk = once_plan_of(true, job[0], dtype, B, H, T), pv = once_plan_of(false, job[1], dtype, B, H, T);
-    const bool one_launch = pk.threads && pk.threads == pv.threads && (job[0].bits > 4) == (job[1].bits > 4);
-    const bool both = cells_in_one_launch(job, pk, pv, B, H, T);
-    const uint32_t closes = one_launch ? pk.nwg + pv.nwg : both ? 2u * (uint32_t)(T / 128) * (uint32_t)B : 0u;
-    ClosedEncode ce;
     ScanHandle sh;
-    if ((rc = prepare_scan_state((uint32_t)state_words(true, B, H, T), &sh, s, true,
-                                 (uint32_t)state_words(false, B, H, T) + (closes ? close_words(closes) : 0u)))) return rc;
-    if (one_launch) {
+    if ((rc = prepare_scan_state((uint32_t)state_words(true, B, H, T), &sh, s, true, (uint32_t)state_words(false, B, H, T)))) return rc;
+    const OncePlan pk = once_plan_of(true, job[0], dtype, B, H, T), pv = once_plan_of(false, job[1], dtype, B, H, T);
+    if (pk.threads && pk.threads == pv.threads && (job[0].bits > 4) == (job[1].bits > 4)) {
         const OnceSide ks = once_side(true, job[0], pk, B, H, T, sh.st), vs = once_side(false, job[1], pv, B, H, T, sh.second);
-        if ((rc = ce.begin(sh, closes, 2, job[0].bits, s))) return rc;
-        if ((rc = pk.threads == 256 ? once_launch<256>(ks, vs, dtype, ce.close, s) : once_launch<1024>(ks, vs, dtype, ce.close, s))) return rc;
-        if ((rc = ce.launched(sh))) return rc;
-        return ce.wait(k_size, job[0].bits, v_size, job[1].bits);
+        if ((rc = pk.threads == 256 ? once_launch<256>(ks, vs, dtype, EncodeClose{}, s) : once_launch<1024>(ks, vs, dtype, EncodeClose{}, s))) return rc;
+    } else if (cells_in_one_launch(job, pk, pv, B, H, T)) {
+        if ((rc = launch_cells_both(job, dtype, B, H, T, sh.st, sh.second, s))) return rc;
+    } else {
+        if ((rc = launch_quant_encode<true>(job[0], dtype, B, H, T, sh.st, EncodeClose{}, s))) return rc;
+        if ((rc = launch_quant_encode<false>(job[1], dtype, B, H, T, sh.second, EncodeClose{}, s))) return rc;
     }
-    if (both) {
-        if ((rc = ce.begin(sh, closes, 2, job[0].bits, s))) return rc;
-        if ((rc = launch_cells_both(job, dtype, B, H, T, sh.st, sh.second, ce.close, s))) return rc;
-        if ((rc = ce.launched(sh))) return rc;
-        return ce.wait(k_size, job[0].bits, v_size, job[1].bits);
-    }
-    if ((rc = launch_quant_encode<true>(job[0], dtype, B, H, T, sh.st, EncodeClose{}, s))) return rc;
-    if ((rc = launch_quant_encode<false>(job[1], dtype, B, H, T, sh.second, EncodeClose{}, s))) return rc;
     return finish_encode(sh, k_size, job[0].bits, s, v_size, job[1].bits);
 }
 

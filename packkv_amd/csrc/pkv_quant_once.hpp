@@ -6,10 +6,6 @@
 // 16 (K) or 32 (V) tokens of a group have wavefronts of their own, and a group's heads are dealt to workgroups in runs of
 // `R`, so that the chain is gone through once and the work spreads over the CUs.  The runs exchange the minima and maxima of
 // their tokens through memory, as the runs of eight heads do in the cells kernels.  Same stream, parameters and block_info.
-// The last workgroup to be done with the look-back state hands the outcome over and clears the state (once_close): a kernel of
-// its own behind the encoder is 4 us and a gap of 1.5, which a waiting host sees, and a launch.  Inside, the encoders get 0.3 (codes)
-// to 2.5 us (V's exchanged words to clear) longer: codes of 16384 tokens x 8 heads, both sides encoded and decoded, 67.7 -> 64.9 us;
-// a prompt of 3001 tokens and six decode steps 290 -> 285.
 //
 // Two sizes: 256 threads, two heads of K or one of V, and 1024 threads, eight heads of K or four of V.  K and V of one call
 // share a launch, K's workgroups first.
@@ -120,43 +116,9 @@ __device__ __forceinline__ void once_sizes(OnceLds<NT> &l, ScanState *st, uint32
     if (lane == nblk - 1) lookback_publish(st, idx, incl);
 }
 
-// ---- the end of the launch ----
-// Counts the workgroup out: nothing of it reads or writes the state any more, and what it wrote has arrived there.  Called by the
-// first wavefront, behind a barrier that every wavefront reached with its own accesses complete; the first thread gets the
-// answer, which it needs only after the copy.  Two steps -- sixteen workgroups to a counter, then one for all: adding
-// to one address takes 13 ns each, one after the other.
-constexpr uint32_t kNotCounted = 0xFFFFFFFFu;
-__device__ __forceinline__ void once_count(const EncodeClose &c, uint32_t &counted) {
-    if (c.total == 0) return;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (threadIdx.x == 0) {
-        uint32_t at = kCloseStride * (1u + blockIdx.x / kCloseGroup);
-        asm volatile("" : "+v"(at));                       // (not as one address for all lanes: the compiler then waits for the answer here)
-        counted = __hip_atomic_fetch_add(reinterpret_cast<uint32_t *>(c.count + at), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-}
+// The workgroup's place in the stream, by its first wavefront; then block_info.  False where the stream does not fit.
 template <int NT>
-__device__ __forceinline__ void once_close(const EncodeClose &c, OnceLds<NT> &l, uint32_t counted) {
-    if (c.total == 0) return;
-    if (threadIdx.x == 0) {
-        if (counted == kNotCounted) once_count(c, counted);      // (a ticket past the last one)
-        const uint32_t group = blockIdx.x / kCloseGroup, groups = (c.total + kCloseGroup - 1u) / kCloseGroup;
-        bool last = counted + 1u == min(kCloseGroup, c.total - group * kCloseGroup);
-        if (last) last = __hip_atomic_fetch_add(reinterpret_cast<uint32_t *>(c.count), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == groups;
-        if (last) publish_outcomes(c.st, c.second, c.last, c.slot, c.tag, c.bits);
-        l.idx = last ? 1u : 0u;
-    }
-    __syncthreads();
-    if (l.idx == 0u) return;
-    // (ordinary stores: nothing reads the state any more before the launch has ended)
-    for (uint32_t i = threadIdx.x; i < c.n / 2u; i += NT) reinterpret_cast<uint4 *>(c.words)[i] = make_uint4(0u, 0u, 0u, 0u);
-    if (threadIdx.x == 0 && (c.n & 1u)) c.words[c.n - 1u] = 0;
-}
-
-// The workgroup's place in the stream, by its first wavefront; then block_info.  False where the stream does not fit.  (Every
-// wavefront gets here through a barrier, its accesses to the state complete.)
-template <int NT>
-__device__ __forceinline__ bool once_place(OnceLds<NT> &l, const OnceSide &a, const EncodeClose &c, uint32_t &counted, uint32_t idx, uint32_t first, int nblk) {
+__device__ __forceinline__ bool once_place(OnceLds<NT> &l, const OnceSide &a, uint32_t idx, uint32_t first, int nblk) {
     const uint32_t bytes = (uint32_t)__builtin_amdgcn_readfirstlane((int)l.blk_off[nblk]);
     if (threadIdx.x < 64) {
         const uint64_t off = a.base + lookback_offset<kOnceSleep>(a.st, idx, bytes, true);
@@ -167,7 +129,6 @@ __device__ __forceinline__ bool once_place(OnceLds<NT> &l, const OnceSide &a, co
         }
     }
     __syncthreads();
-    if (threadIdx.x < 64) once_count(c, counted);
     if (l.off + bytes > a.capacity) return false;
     const uint32_t tid = threadIdx.x;
     if (tid < (uint32_t)nblk) {
@@ -183,13 +144,12 @@ __device__ __forceinline__ void once_max_code(ScanState *st, uint32_t cmax, int 
         for (int d = 32; d >= 1; d >>= 1) cmax = max(cmax, __shfl_xor(cmax, d, 64));
         if ((threadIdx.x & 63) == 0) atomicMax(&st->max_code, cmax);
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // (before the barrier in front of once_place; nothing else is under way here)
 }
 
 // K: thread = (round, head of the run, lane of the unit).  The codes of a cell to the `nblk` blocks from `first` on.
 template <int NT, bool WIDE>
 __device__ __forceinline__ void k_write_once(const OnceSide &a, OnceLds<NT> &l, uint8_t *gbuf, uint32_t idx, int nblk, uint32_t first,
-                                             const uint32_t c01[16], const uint32_t c23[16], bool checked, const EncodeClose &c, uint32_t &counted) {
+                                             const uint32_t c01[16], const uint32_t c23[16], bool checked) {
     constexpr int R = OnceRun<NT>::K;
     const int tid = threadIdx.x, j = (tid >> 5) % R, r = tid / (32 * R), t = tid & 31;
     const UnitGeom g = unit_geom(a.W);
@@ -212,13 +172,13 @@ __device__ __forceinline__ void k_write_once(const OnceSide &a, OnceLds<NT> &l, 
     if (checked) once_max_code(a.st, j < nblk ? cmax : 0u, a.W);
     packs_put();
     __syncthreads();
-    if (!once_place(l, a, c, counted, idx, first, nblk)) return;
+    if (!once_place(l, a, idx, first, nblk)) return;
     const int q = tid >> 7;                                // 128 threads copy a block
     if (q < nblk) copy_out<128>(a.stream + l.off + l.blk_off[q], gbuf + (size_t)q * a.slot, l.blk_off[q + 1] - l.blk_off[q], tid & 127);
 }
 
 template <int NT, int DT, bool WIDE, bool PERM>
-__device__ __forceinline__ void k_encode_once(const OnceSide &a, OnceLds<NT> &l, uint8_t *gbuf, const EncodeClose &c, uint32_t &counted) {
+__device__ __forceinline__ void k_encode_once(const OnceSide &a, OnceLds<NT> &l, uint8_t *gbuf) {
     constexpr int R = OnceRun<NT>::K, WPR = R / 2;         // wavefronts of a round
     const uint32_t idx = once_ticket(l, a.st);
     if (idx >= a.nwg) return;
@@ -286,7 +246,7 @@ __device__ __forceinline__ void k_encode_once(const OnceSide &a, OnceLds<NT> &l,
     wave_lds_order();
     uint32_t c01[16], c23[16];
     cell_quant<DT>(xr, par, c01, c23);
-    k_write_once<NT, WIDE>(a, l, gbuf, idx, H, grp * (uint32_t)a.H + (uint32_t)hbase, c01, c23, true, c, counted);      // block index = group * heads + head
+    k_write_once<NT, WIDE>(a, l, gbuf, idx, H, grp * (uint32_t)a.H + (uint32_t)hbase, c01, c23, true);      // block index = group * heads + head
 }
 
 // V: a wavefront is 32 tokens of one head, the two rounds in its halves.  Its codes to the 2 H blocks from `first` on.
@@ -299,7 +259,7 @@ __device__ __forceinline__ void v_clear_once(const OnceSide &a, uint8_t *gbuf) {
 }
 template <int NT, bool WIDE>
 __device__ __forceinline__ void v_write_once(const OnceSide &a, OnceLds<NT> &l, uint8_t *gbuf, uint32_t idx, int H, uint32_t first,
-                                             const uint32_t c01[16], const uint32_t c23[16], bool checked, const EncodeClose &c, uint32_t &counted) {
+                                             const uint32_t c01[16], const uint32_t c23[16], bool checked) {
     constexpr int R = OnceRun<NT>::V;
     const int tid = threadIdx.x, wave = tid >> 6, it = wave / R, j = wave % R, lane = tid & 63, rp = lane >> 5, t = lane & 31;
     const int seg = it >> 1, slot = 2 * (it & 1) + rp, blkid = 2 * j + (t >> 4), w = (t >> 3) & 1, m = t & 7, nblk = 2 * H;
@@ -336,7 +296,7 @@ __device__ __forceinline__ void v_write_once(const OnceSide &a, OnceLds<NT> &l, 
     if (checked) once_max_code(a.st, j < H ? cmax : 0u, a.W);
     packs_put();
     __syncthreads();
-    if (!once_place(l, a, c, counted, idx, first, nblk)) return;
+    if (!once_place(l, a, idx, first, nblk)) return;
     // a half-wavefront copies a unit, the first of a block its header of cumulative unit sizes
     for (int i = tid >> 5; i < 4 * nblk; i += NT / 32) {
         const int q = i >> 2, un = i & 3;
@@ -351,7 +311,7 @@ __device__ __forceinline__ void v_write_once(const OnceSide &a, OnceLds<NT> &l, 
 }
 
 template <int NT, int DT, bool WIDE, bool PERM>
-__device__ __forceinline__ void v_encode_once(const OnceSide &a, OnceLds<NT> &l, uint8_t *gbuf, const EncodeClose &c, uint32_t &counted) {
+__device__ __forceinline__ void v_encode_once(const OnceSide &a, OnceLds<NT> &l, uint8_t *gbuf) {
     constexpr int R = OnceRun<NT>::V;
     v_clear_once<NT>(a, gbuf);
     const uint32_t idx = once_ticket(l, a.st);
@@ -420,17 +380,16 @@ __device__ __forceinline__ void v_encode_once(const OnceSide &a, OnceLds<NT> &l,
     wave_lds_order();
     uint32_t c01[16], c23[16];
     cell_quant<DT, false>(xr, par + 16 * rp, c01, c23);    // (the halves of the wavefront hold different tokens)
-    v_write_once<NT, WIDE>(a, l, gbuf, idx, H, grp * (uint32_t)(2 * a.H) + (uint32_t)(2 * hbase), c01, c23, true, c, counted);      // block index = group * 2 heads + 2 head + half
+    v_write_once<NT, WIDE>(a, l, gbuf, idx, H, grp * (uint32_t)(2 * a.H) + (uint32_t)(2 * hbase), c01, c23, true);      // block index = group * 2 heads + 2 head + half
 }
 
 template <int NT, int DT, bool WIDE, bool PERM>
 __global__ void __launch_bounds__(NT) quant_encode_once_kernel(const OnceSide k, const OnceSide v, const EncodeClose c) {
     extern __shared__ __align__(16) uint8_t gbuf[];
     __shared__ OnceLds<NT> l;
-    uint32_t counted = kNotCounted;
-    if (blockIdx.x < k.nwg) k_encode_once<NT, DT, WIDE, PERM>(k, l, gbuf, c, counted);
-    else v_encode_once<NT, DT, WIDE, PERM>(v, l, gbuf, c, counted);
-    once_close<NT>(c, l, counted);
+    if (blockIdx.x < k.nwg) k_encode_once<NT, DT, WIDE, PERM>(k, l, gbuf);
+    else v_encode_once<NT, DT, WIDE, PERM>(v, l, gbuf);
+    encode_close(c, l.idx);
 }
 
 // The block codec from a code matrix: the "heads" are 128-channel slices of it, nothing to quantise and nothing to exchange.
@@ -441,9 +400,8 @@ __global__ void __launch_bounds__(NT) code_encode_once_kernel(const OnceSide a, 
     constexpr int R = IS_K ? OnceRun<NT>::K : OnceRun<NT>::V;
     if (!IS_K) v_clear_once<NT>(a, gbuf);
     const uint32_t idx = once_ticket(l, a.st);
-    uint32_t counted = kNotCounted;
     if (idx >= a.nwg) {
-        once_close<NT>(c, l, counted);
+        encode_close(c, l.idx);
         return;
     }
     const uint32_t cb = idx / (uint32_t)a.nruns, hg = idx % (uint32_t)a.nruns;
@@ -454,20 +412,20 @@ __global__ void __launch_bounds__(NT) code_encode_once_kernel(const OnceSide a, 
         const int r = __builtin_amdgcn_readfirstlane(tid / (32 * R));
         code_cell_load(rows + (size_t)(16 * r) * (size_t)a.hidden, (size_t)a.hidden, (uint32_t)((tid >> 5) % R * 128 + 4 * t), w);
         code_cell_pairs(w, c01, c23);
-        k_write_once<NT, WIDE>(a, l, gbuf, idx, R, idx * (uint32_t)R, c01, c23, false, c, counted);
+        k_write_once<NT, WIDE>(a, l, gbuf, idx, R, idx * (uint32_t)R, c01, c23, false);
     } else {
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
         code_cell_load(rows + (size_t)(32 * (wave / R)) * (size_t)a.hidden, (size_t)a.hidden,
                        (uint32_t)(16 * ((tid >> 5) & 1)) * (uint32_t)a.hidden + (uint32_t)(wave % R * 128 + 4 * t), w);
         code_cell_pairs(w, c01, c23);
-        v_write_once<NT, WIDE>(a, l, gbuf, idx, R, idx * (uint32_t)(2 * R), c01, c23, false, c, counted);
+        v_write_once<NT, WIDE>(a, l, gbuf, idx, R, idx * (uint32_t)(2 * R), c01, c23, false);
     }
-    once_close<NT>(c, l, counted);
+    encode_close(c, l.idx);
 }
 
 // ---- which launches, and their shapes ----------------------------------------------------------------------------
 
-// Kernel times without the closing (once_close) by the number of workgroups (trace; fp16, 4-bit codes, 8 heads; cells kernel | 1024 threads | 256 threads):
+// Kernel times without the closing (encode_close) by the number of workgroups (trace; fp16, 4-bit codes, 8 heads; cells kernel | 1024 threads | 256 threads):
 //   tokens         512                 4096                 8192             16384            32768
 //   K           17.9 | 12.7 |  8.8   18.3 | 13.0 | 12.0   19.1 | 14.2 | 18   22.3 | 17.6 | 31   30.6 | 37 | 54 us
 //   V           23.9 | 14.9 | 10.5   25.0 | 15.8 | 13.7   25.5 | 16.8 | 19   27.0 | 20.0 | 32   31.3 | 38 | 55

@@ -274,43 +274,24 @@ OutcomeSlot::~OutcomeSlot() {
     g_free_slots.push_back(words);
 }
 
-int ClosedEncode::begin(ScanHandle &h, uint32_t total, int sizes, int bits, hipStream_t stream) {
+int ClosedEncode::begin(ScanHandle &h, uint32_t total, hipStream_t stream) {
     std::lock_guard<std::mutex> lock(g_ws_mu);
     Workspace *w = nullptr;
     int rc = workspace_for(stream, &w);
     if (rc) return rc;
     uint32_t tag = 0;
-    if ((rc = slot_take(sizes ? &close.slot : nullptr, &tag))) return rc;
+    if ((rc = slot_take(nullptr, &tag))) return rc;
     s = stream;
-    close.words = (uint64_t *)h.st;
+    close.st = h.st;
     close.n = (uint32_t)h.words64;
     close.total = total;
-    close.count = close.words + (h.words64 - close_words(total));
-    close.st = h.st;
-    close.second = h.second;
+    close.count = (uint64_t *)h.st + (h.words64 - close_words(total));
     close.last = w->last;
     close.tag = tag;
-    close.bits = bits;
     return PKV_OK;
 }
 
 int ClosedEncode::launched(ScanHandle &h) { return scan_state_cleared(h, s); }
-
-int ClosedEncode::wait(uint64_t *size_out, int bits, uint64_t *size2_out, int bits2) {
-    if (!close.slot) return PKV_OK;
-    int rc = wait_words(close.slot, close.second ? 2 * kOutcomeWords : kOutcomeWords, (uint32_t)close.tag, s);
-    waited = true;
-    if (!rc && size_out) rc = outcome(close.slot, size_out, bits);
-    if (!rc && close.second && size2_out) rc = outcome(close.slot + kOutcomeWords, size2_out, bits2);
-    return rc;
-}
-
-ClosedEncode::~ClosedEncode() {
-    if (!close.slot) return;
-    if (!waited) (void)hipStreamSynchronize(s);
-    std::lock_guard<std::mutex> lock(g_ws_mu);
-    g_free_slots.push_back(close.slot);
-}
 
 int scan_state_cleared(ScanHandle &h, hipStream_t s) {
     {

@@ -58,7 +58,7 @@ int stagger_for(const void *kernel, int threads, uint32_t lds, uint32_t nwg, Sta
 // Look-back state of the single-pass encoders, from a buffer of its own per (device, stream) that is all zero between
 // encodes: a launch finds it cleared, and the kernel finish_encode launches behind the encoder takes its outcome out
 // and clears it again.  One kernel per encode next to the encoder itself, and no copy: the outcome goes straight to
-// pinned host memory, where a waiting host thread polls for it.  (Encoders of few workgroups do the same without that kernel: ClosedEncode.)
+// pinned host memory, where a waiting host thread polls for it.  (Where no size is asked for, encoders of few workgroups do without that kernel: ClosedEncode.)
 // Fused K encode of 512 tokens x 8 heads with its size:
 // 35.8 us a call, against 49.7 with a clearing kernel in front and a copy and a stream synchronisation behind (V 42.4
 // against 55.9); without the size both ways take 19 us.
@@ -78,30 +78,24 @@ int prepare_scan_state(uint32_t nblocks, ScanHandle *out, hipStream_t s, bool wa
 // (`size2_out`: of the second state).  `bits` > 0 additionally rejects a launch whose largest code does not fit.
 // NULL: returns at once, pkv_encode_status reads the outcome later.
 int finish_encode(ScanHandle &h, uint64_t *size_out, int bits, hipStream_t s, uint64_t *size2_out = nullptr, int bits2 = 0);
-// An encoder whose last workgroup publishes the outcome and clears the state by itself (pkv_quant_once.hpp): what it needs for
-// that, in place of finish_encode's kernel.
+// An encoder whose last workgroup leaves the outcome and clears the state by itself (encode_close), in place of finish_encode's
+// kernel: for calls that hand nothing back.  A size promises that the stream, block_info and the parameters are there as
+// well, for any stream of the device, and inside the launch that takes a write-back of its XCD's L2 by every workgroup: K with its size,
+// 8 heads, behind a kernel of its own | so released, us: 4096 tokens 40.4 | 42.5, 4 x 8192 58 | 68, 16 x 8192 116 | 176.
 struct EncodeClose {
-    uint64_t *words = nullptr;     // the whole state, `n` words
+    ScanState *st = nullptr;       // the whole state, `n` words
     uint32_t n = 0, total = 0;     // total: workgroups of the launch; 0: finish_encode follows
     uint64_t *count = nullptr;     // (in the state) workgroups that are done, by groups of kCloseGroup and all together
-    ScanState *st = nullptr, *second = nullptr;
-    uint64_t *last = nullptr, *slot = nullptr;
-    uint64_t tag = 0;
-    int bits = 0;
+    uint64_t *last = nullptr, tag = 0;
 };
 constexpr uint32_t kCloseGroup = 16, kCloseStride = 16;        // words from counter to counter: a cache line of its own each
 constexpr uint32_t close_words(uint32_t total) { return kCloseStride * (1u + (total + kCloseGroup - 1u) / kCloseGroup); }
-// ... for a launch of `total` workgroups whose state was prepared with close_words(total) more words behind the last status
-// word; `sizes`: how many outcomes will be waited for (0: none).
+// ... for a launch of `total` workgroups whose state was prepared with close_words(total) more words behind the last status word.
 struct ClosedEncode {
     EncodeClose close;
     hipStream_t s = nullptr;
-    int begin(ScanHandle &h, uint32_t total, int sizes, int bits, hipStream_t stream);
+    int begin(ScanHandle &h, uint32_t total, hipStream_t stream);
     int launched(ScanHandle &h);   // the launch has been made: the state will be clear behind it
-    int wait(uint64_t *size_out, int bits, uint64_t *size2_out = nullptr, int bits2 = 0);      // finish_encode's results; at once without a size
-    ~ClosedEncode();               // gives the slot back, when nothing can write to it any more
-  private:
-    bool waited = false;
 };
 // For a kernel whose last workgroup publishes the outcome and clears the state by itself: a pinned slot of kSlotWords words
 // that are valid one by one through their tag (value, 34 bits | tag << 34), and the two ends of its life.  Refused while

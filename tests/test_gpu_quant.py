@@ -472,9 +472,9 @@ def test_padding_of_one_sequence_leaves_the_others_alone(cuda, dtype, H, T):
 
 @pytest.mark.parametrize("H,T", [(2, 128), (2, 1920), (2, 2048), (2, 2176), (8, 2048), (16, 1024), (8, 16384), (40, 640)])
 def test_encoders_that_close_by_themselves(cuda, H, T):
-    """Launches of up to 256 workgroups hand their outcome over and clear the look-back state without a kernel behind them,
-    counted in sixteens: one workgroup, counts around a multiple of sixteen, the most there are.  Each encode finds the state
-    clear, whatever the one before was -- fused K and V, K and V in one launch, codes, with and without a size, a stream that does
+    """Launches of up to 256 workgroups that hand no size back leave their outcome and clear the look-back state without a kernel
+    behind them, counted in sixteens: one workgroup, counts around a multiple of sixteen, the most there are.  Each encode finds the
+    state clear, whatever the one before was -- fused K and V, K and V in one launch, codes, with and without a size, a stream that does
     not fit -- and gives what encodes of 64 and 128 tokens appended one by one give."""
     k, v = synth.make_kv(1, H, T, seed=H + T, device=cuda)
 
@@ -506,10 +506,16 @@ def test_encoders_that_close_by_themselves(cuda, H, T):
             codes = ops.quantize(x, e["scale"], e["zero"])[0]
             s = side(x, is_k)
             check(is_k, code_enc(codes, s[2], s[4]), s[2], s[4], "codes")
+            s[2].zero_()
+            code_enc(codes, s[2], s[4], want_size=False)
+            check(is_k, ops.encode_status(cuda, bits=4), s[2], s[4], "codes, no size")
             with pytest.raises(ops.PackKVError, match="fit"):
                 code_enc(codes, s[2][:e["size"] - 2], s[4])
             with pytest.raises(ops.PackKVError, match="fit"):
                 enc(x, 0.1, stream=s[2][:e["size"] - 2], info=s[4])
+            enc(x, 0.1, stream=s[2][:e["size"] - 2], info=s[4], want_size=False)
+            with pytest.raises(ops.PackKVError, match="fit"):
+                ops.encode_status(cuda, bits=4)
 
 
 # V of 5 and 6 bits beyond the encodes at once: two segments of a block side by side; idle head slots, runs of eight heads.
@@ -597,8 +603,12 @@ def test_encoders_that_walk_and_close_by_themselves(cuda, H, T):
         first = enc(x, 0.1)
         with pytest.raises(RuntimeError, match="does not fit bits_len 3"):
             enc(x, 0.1, 3)
-        for rep in range(2):                           # (after an error, and after a launch of its own: the state is clear)
-            r = enc(x, 0.1)
+        enc(x, 0.1, 3, want_size=False)
+        with pytest.raises(RuntimeError, match="does not fit bits_len 3"):
+            ops.encode_status(cuda, bits=3)
+        for rep in range(4):                           # (after an error, and after a launch of its own kind: the state is clear)
+            r = enc(x, 0.1, want_size=rep < 2)
+            r["size"] = r["size"] or ops.encode_status(cuda, bits=4)
             assert r["size"] == first["size"] and torch.equal(r["stream"][:r["size"]], first["stream"][:r["size"]])
             assert all(torch.equal(r[f].view(torch.int16), first[f].view(torch.int16)) for f in ("info", "scale", "zero"))
         codes = torch.empty(T, H * 128, dtype=torch.uint8, device=cuda)
@@ -622,5 +632,49 @@ def test_code_encoders_that_walk_and_close_by_themselves(cuda, T, bits):
         want, table = stream[:size].clone(), info.clone()
         with pytest.raises(RuntimeError):              # (a stream that does not fit; the state is clear behind it)
             ops.encode_p(is_k, codes, stream[:size - 2], info, 16, bits)
-        assert ops.encode_p(is_k, codes, stream, info, 16, bits) == size
-        assert torch.equal(stream[:size], want) and torch.equal(info.view(torch.int32), table.view(torch.int32))
+        ops.encode_p(is_k, codes, stream[:size - 2], info, 16, bits, want_size=False)
+        with pytest.raises(RuntimeError, match="fit"):
+            ops.encode_status(cuda)
+        for want_size in (True, False, False):
+            stream.zero_()
+            got = ops.encode_p(is_k, codes, stream, info, 16, bits, want_size=want_size)
+            assert (got if want_size else ops.encode_status(cuda)) == size
+            assert torch.equal(stream[:size], want) and torch.equal(info.view(torch.int32), table.view(torch.int32))
+
+
+@pytest.fixture(scope="module")
+def other():
+    return torch.cuda.Stream()           # (one for all cases: torch hands out 32 in turn, and some tests want one without a past)
+
+
+@pytest.mark.parametrize("B,T", [(1, 512), (2, 4096), (16, 8192)])
+@pytest.mark.parametrize("kind", ["k", "v", "append", "repack", "k codes", "v codes"])
+def test_a_size_says_that_the_output_is_there_for_any_stream(cuda, other, kind, B, T):
+    """A call that hands its size back is synchronous: the stream's bytes, block_info and the parameters can be read through
+    another stream at once, without an event.  (In launches of a few, of some hundred and of 2048 workgroups; every pass has
+    other inputs, in zeroed buffers.)"""
+    H = 8
+    for seed in range(3):
+        k, v = synth.make_kv(B, H, T, seed=650 + seed, device=cuda)
+        sides = []
+        for blocks, bound in ((T // 64 * B * H, ops.block_bound(True, 64, 128, 4)), (T // 128 * 2 * B * H, ops.block_bound(False, 128, 64, 4))):
+            sides.append([torch.zeros(blocks * bound + 16, dtype=torch.uint8, device=cuda), torch.zeros(blocks, 2, dtype=torch.uint32, device=cuda),
+                          torch.zeros(B, T, dtype=k.dtype, device=cuda), torch.zeros(B, T, dtype=k.dtype, device=cuda)])
+        codes = [ops.quantize(x, *ops.quant_params(x, 0.1))[0] for x in (k, v)]
+        torch.cuda.synchronize()
+        if kind in ("k", "v"):
+            r = (ops.k_quant_encode if kind == "k" else ops.v_quant_encode)(k if kind == "k" else v, 0.1, stream=sides[kind == "v"][0], info=sides[kind == "v"][1])
+            out = [r["stream"][:r["size"]], r["info"], r["scale"], r["zero"]]
+        elif kind == "append":
+            sizes = ops.kv_quant_encode_append(k, v, T, *((0.1, 4, st, 0, *rest) for st, *rest in sides), 0)
+            out = [t for side, size in zip(sides, sizes) for t in (side[0][:size], *side[1:])]
+        elif kind == "repack":
+            out = [t for r in ops.repack_quant_encode(k, v, 0.1, 0.1)[:2] for t in (r["stream"][:r["size"]], r["info"], r["scale"], r["zero"])]
+        else:
+            i = int(kind == "v codes")
+            size = ops.encode_p(i == 0, codes[i], *sides[i][:2], 16, 4)
+            out = [sides[i][0][:size], sides[i][1]]
+        with torch.cuda.stream(other):
+            seen = [t.view(torch.uint8).clone() for t in out]
+        torch.cuda.synchronize()
+        assert all(t.numel() for t in out) and all(torch.equal(a, b.view(torch.uint8)) for a, b in zip(seen, out)), seed
