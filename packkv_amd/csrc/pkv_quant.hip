@@ -420,15 +420,17 @@ int launch_quant_dequant(const void *k, const void *v, void *k_out, void *v_out,
     return PKV_OK;
 }
 
-// bit_length of both 16-bit halves, clamped to MOST (larger values mean the codes overflow the format; the launch reports that
-// through max_code): the exponent of (2 r + 1) 2^-10 as a half, r read as a subnormal half (r 2^-24 times 2^15, exact).  Four
-// instructions; sums of min(r >> k, 1) came out of the compiler as compares and selects of single halves, 24.
+// bit_length of both 16-bit halves, at most MOST (larger values mean the codes overflow the format; the launch reports that through
+// max_code): the exponent of (2 r + 1) 2^-10 as a half, r read as a subnormal half (r 2^-24 times 2^15, exact).  Four instructions;
+// sums of min(r >> k, 1) came out of the compiler as compares and selects of single halves, 24.  (The limit comes first: 0x8000,
+// the range of a pack of NaNs of both signs, reads as -0.)
 template <int MOST>
 __device__ __forceinline__ uint32_t pk_bitlen(uint32_t r) {
-    const f16x2 f = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, r), (f16x2){(_Float16)32768.f, (_Float16)32768.f},
+    constexpr uint16_t kTop = (1u << MOST) - 1u;
+    const u16x2 v = __builtin_elementwise_min(as_u16x2(r), (u16x2){kTop, kTop});
+    const f16x2 f = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, v), (f16x2){(_Float16)32768.f, (_Float16)32768.f},
                                               (f16x2){(_Float16)0.0009765625f, (_Float16)0.0009765625f});
-    const u16x2 e = (__builtin_bit_cast(u16x2, f) >> 10) - (u16x2){5, 5};
-    return pk_u16(__builtin_elementwise_min(e, (u16x2){MOST, MOST}));
+    return pk_u16((u16x2)((__builtin_bit_cast(u16x2, f) >> 10) - (u16x2){5, 5}));
 }
 // Minimum or maximum of 16 words of two codes each, as unsigned integers: what NaN makes of a code may have its top bit set, and
 // the packs of such tokens are to be the same in every kernel (v_pk_minimum3_f16 would take three at a time, but by their sign).

@@ -678,3 +678,22 @@ def test_a_size_says_that_the_output_is_there_for_any_stream(cuda, other, kind, 
             seen = [t.view(torch.uint8).clone() for t in out]
         torch.cuda.synchronize()
         assert all(t.numel() for t in out) and all(torch.equal(a, b.view(torch.uint8)) for a, b in zip(seen, out)), seed
+
+
+@pytest.mark.parametrize("B,H,T", [(1, 8, 128), (1, 2, 256), (33, 8, 1024)])
+@pytest.mark.parametrize("rel", [0.1, 0.03])
+def test_a_pack_of_nans_of_both_signs_has_the_full_width(cuda, B, H, T, rel):
+    """The codes of such a pack lie 0x8000 apart: it is stored at the width of one whose codes span the whole range (the call
+    reports the overflow when it is asked), 4 and 6 bits, in the encoders at once and in those that walk."""
+    base = torch.linspace(-1, 1, 128, device=cuda).half().expand(B, H, T, 128)
+    for enc in (ops.k_quant_encode, ops.v_quant_encode):
+        sizes = []
+        for even, odd in ((0x7E00, -0x200), (-0x4400, 0x3C00)):           # NaN and -NaN; -1 and 1, the limits of every token
+            x = base.clone()
+            x.view(torch.int16)[:, H - 1, 0::2, 5], x.view(torch.int16)[:, H - 1, 1::2, 5] = even, odd
+            sizes.append(enc(x, rel, want_size=False)["info"].view(torch.int32)[:, 1].clone())
+        assert torch.equal(*sizes)
+        with pytest.raises(ops.PackKVError):
+            x = base.clone()
+            x.view(torch.int16)[:, H - 1, 0::2, 5], x.view(torch.int16)[:, H - 1, 1::2, 5] = 0x7E00, -0x200
+            enc(x, rel)
