@@ -6,11 +6,11 @@ something else.
 """
 import ctypes
 import os
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # PACKKV_HIP_LIB names another build of the same library (kernel development: A/B runs of two builds)
 LIB_PATH = os.environ.get("PACKKV_HIP_LIB") or os.path.join(_HERE, "libpackkv_hip.so")
-HOST_PATH = os.path.join(_HERE, "_host.so")
 HOST_SYMBOLS = ("pkv_attn_decode", "pkv_window_append", "pkv_dense_view", "pkv_kq_mat_vec_mul", "pkv_wv_mat_vec_mul", "pkv_fused_kq",
                 "pkv_fused_wv")
 
@@ -101,7 +101,7 @@ SIGNATURES = {
 }
 
 _lib = None
-host = None        # the native host side of the repeated calls (csrc/pkv_host.cpp), bound to the library once that is loaded
+host = None        # the native host side of the repeated calls (csrc/pkv_host.cpp), or NO_HOST, once the library is loaded
 
 
 class PackKVError(RuntimeError):
@@ -112,18 +112,43 @@ class PackKVError(RuntimeError):
         self.code = code
 
 
+class _NoHost:
+    """Serves no call: the general code of ops.py does them all."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+NO_HOST = _NoHost()
+
+
+def _load_host(lib):
+    """The native host side; NO_HOST, with a warning, where it is missing or was built for another torch (the library itself
+    knows nothing of torch, and the general code needs nothing but it)."""
+    import torch
+    try:
+        from . import _host
+        made_for = getattr(_host, "torch", "unknown")
+        why = None if made_for == torch.__version__ else "built for torch %s, this is %s" % (made_for, torch.__version__)
+    except ImportError as e:
+        why = str(e)
+    if why:
+        warnings.warn("packkv_amd._host is not used (%s): the calls that a decode loop repeats take 3 to 8 us more of host time each. "
+                      "`python -m packkv_amd.build` makes it." % why, RuntimeWarning, stacklevel=3)
+        return NO_HOST
+    _host.bind(*(ctypes.cast(getattr(lib, name), _vp).value for name in HOST_SYMBOLS))
+    return _host
+
+
 def load():
     """Load the library once and attach prototypes.  Raises ImportError when it is missing."""
     global _lib, host
     if _lib is not None:
         return _lib
-    for path in (LIB_PATH, HOST_PATH):
-        if not os.path.exists(path):
-            raise ImportError(
-                "%s is not built (%s). Build it with `python -m packkv_amd.build` "
-                "(needs hipcc, targets gfx950); there is no CPU fallback." % (os.path.basename(path), path))
-    import torch  # noqa: F401  (the libraries that _host.so needs)
-    from . import _host
+    if not os.path.exists(LIB_PATH):
+        raise ImportError(
+            "libpackkv_hip.so is not built (%s). Build it with `python -m packkv_amd.build` "
+            "(needs hipcc, targets gfx950); there is no CPU fallback." % LIB_PATH)
     try:
         lib = ctypes.CDLL(LIB_PATH)
     except OSError as e:  # pragma: no cover - depends on the machine
@@ -132,8 +157,7 @@ def load():
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
-    _host.bind(*(ctypes.cast(getattr(lib, name), _vp).value for name in HOST_SYMBOLS))
-    host, _lib = _host, lib
+    host, _lib = _load_host(lib), lib
     return lib
 
 

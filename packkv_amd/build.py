@@ -65,9 +65,11 @@ def _build_host(only_stale=False):
     if only_stale and os.path.exists(HOST) and not _stale("pkv_host.cpp", HOST):
         return HOST
     import sysconfig
+    import torch
     from torch.utils import cpp_extension
     torch_lib = os.path.join(os.path.dirname(os.path.dirname(cpp_extension.include_paths()[0])), "torch", "lib")
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           '-DPKV_TORCH_VERSION="%s"' % torch.__version__]
     cmd += ["-I" + d for d in [sysconfig.get_paths()["include"]] + cpp_extension.include_paths()] + ["-I/opt/rocm/include"]
     cmd += [os.path.join(CSRC, "pkv_host.cpp"), "-o", HOST, "-L" + torch_lib, "-ltorch_python", "-ltorch_cpu", "-lc10_hip", "-lc10"]
     r = subprocess.run(cmd, capture_output=True, text=True)
@@ -86,12 +88,12 @@ def build(verbose=True, only_stale=False, defines=(), out=None):
     with ThreadPoolExecutor(max_workers=8) as ex:
         host = ex.submit(_build_host, only_stale) if out is None else None
         objs = list(ex.map(lambda src: _compile(src, only_stale, defines, obj_dir), SOURCES))
-        if host is not None:
-            host.result()
     cmd = [_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", lib] + objs
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("link failed:\n" + r.stderr)
+    if host is not None:
+        host.result()                  # (raises what went wrong there; the library stands on its own)
     if verbose:
         print("built", lib)
     return lib

@@ -40,7 +40,15 @@ def _ptr(t):
 def _host():
     """The native side of the calls a decode loop repeats (csrc/pkv_host.cpp): its functions return None for a call that they do
     not serve, which then takes the general code below them."""
-    return _lib.host or (_lib.load() and _lib.host)
+    return _lib.host or _first_host()
+
+
+def _first_host():
+    try:
+        _lib.load()
+    except ImportError:          # (the general code says so where it needs the library, and refuses what it refuses without it)
+        return _lib.NO_HOST
+    return _lib.host
 
 
 # Every op makes `dev` current and passes on its current stream.  A stream object and a device context that is entered

@@ -58,3 +58,45 @@ assert ops._stream(torch.device("cuda")) == 103 and ops._stream(torch.device("cu
 assert ops._on(torch.device("cuda", 3)) is ops._here
 """
     subprocess.run([sys.executable, "-c", code], check=True, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))), timeout=300)
+
+
+@pytest.mark.parametrize("module", ["None", "types.SimpleNamespace(torch='0.0')"])
+def test_without_the_native_host_side_the_library_loads_and_the_general_code_serves(module):
+    """_host.so missing, not loadable, or built for another torch: a warning, and calls come as far as they do in ops.py."""
+    code = """
+import sys, types, warnings
+import packkv_amd
+sys.modules["packkv_amd._host"] = %s
+if sys.modules["packkv_amd._host"]:
+    packkv_amd._host = sys.modules["packkv_amd._host"]
+import torch
+from packkv_amd import _lib, ops
+with warnings.catch_warnings(record=True) as seen:
+    warnings.simplefilter("always")
+    assert _lib.load().pkv_abi_version() == 3
+assert any("_host" in str(w.message) for w in seen), seen
+assert _lib.host is _lib.NO_HOST and _lib.host.attn_decode(1, 2) is None
+try:
+    ops.attn_decode(torch.zeros(1, 8, 128, dtype=torch.float16), None, None)
+except RuntimeError as e:
+    assert "q must be a contiguous device tensor" in str(e), e
+else:
+    raise SystemExit("accepted")
+""" % module
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))), timeout=300)
+
+
+def test_the_native_host_side_is_the_one_of_this_torch():
+    _lib.load()
+    assert _lib.host is not _lib.NO_HOST and _lib.host.torch == torch.__version__
+
+
+def test_what_is_refused_needs_no_library(monkeypatch):
+    """Without libpackkv_hip.so a call that is refused says why, and any other one that the library is missing."""
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "host", None)
+    monkeypatch.setattr(_lib, "LIB_PATH", os.path.join(os.path.dirname(_lib.LIB_PATH), "nowhere.so"))
+    with pytest.raises(RuntimeError, match="q must be a 2D tensor"):
+        ops.fused_kq(*(torch.zeros(2, dtype=torch.float16) for _ in range(5)))
+    with pytest.raises(ImportError, match="not built"):
+        ops.block_bound(True, 64, 128, 4)
