@@ -41,7 +41,13 @@ bool half(const at::Tensor &t) { return t.scalar_type() == at::kHalf || t.scalar
 int code(const at::Tensor &t) { return t.scalar_type() == at::kHalf ? PKV_F16 : PKV_BF16; }
 template <typename T> T *at_ptr(const at::Tensor &t) { return reinterpret_cast<T *>(t.data_ptr()); }
 
-int here() { return c10::hip::current_device(); }
+// The current device where `t` lies on it, else -1, which is no tensor's.  (HIP is not asked about a tensor on the host: there may
+// be no GPU, and the general code has the words for that.)
+int here(const at::Tensor *t) {
+    if (!t || !t->is_cuda()) return -1;
+    const int dev = c10::hip::current_device();
+    return t->get_device() == dev ? dev : -1;
+}
 pkv_stream_t stream(int dev) { return (pkv_stream_t)c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream(); }
 
 // An int argument (a plain Python int within 32 bits).
@@ -131,8 +137,8 @@ PyObject *status(int rc) { return PyLong_FromLong(rc); }
 PyObject *attn_decode(PyObject *, PyObject *const *o, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     const at::Tensor *q = n == 7 && !modes() ? tensor(o[0]) : nullptr;
-    const int dev = here();
-    if (!q || !dense(*q, dev) || !half(*q) || q->dim() != 3 || q->size(2) != 128) Py_RETURN_NONE;
+    const int dev = here(q);
+    if (dev < 0 || !dense(*q, dev) || !half(*q) || q->dim() != 3 || q->size(2) != 128) Py_RETURN_NONE;
     pkv_attn_args a{};
     Cache c;
     c.batch = (int)q->size(0);
@@ -172,8 +178,8 @@ PyObject *plan_step(PyObject *, PyObject *const *o, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     const at::Tensor *q = n == 4 && !modes() ? tensor(o[3]) : nullptr;
     int plan_dev = -1, rows = 0;
-    const int dev = here();
-    if (!q || !PyLong_CheckExact(o[0]) || !integer(o[1], &plan_dev) || !integer(o[2], &rows) || plan_dev != dev || !dense(*q, dev)) Py_RETURN_NONE;
+    const int dev = here(q);
+    if (dev < 0 || !PyLong_CheckExact(o[0]) || !integer(o[1], &plan_dev) || !integer(o[2], &rows) || plan_dev != dev || !dense(*q, dev)) Py_RETURN_NONE;
     // (a copy: the plan's own q, out and rows stay what its owner has set, and keeps alive)
     pkv_attn_args a = *(const pkv_attn_args *)PyLong_AsVoidPtr(o[0]);
     const int64_t d = q->dim();
@@ -194,9 +200,9 @@ PyObject *window_append(PyObject *, PyObject *const *o, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     if (n != 7 || modes()) Py_RETURN_NONE;
     const at::Tensor *k = tensor(o[0]), *v = tensor(o[1]), *kw = tensor(o[4]), *vw = tensor(o[5]);
-    const int dev = here();
+    const int dev = here(k);
     int pos = 0;
-    if (!k || !v || !kw || !vw || !there(*k, dev) || !there(*v, dev) || !dense(*kw, dev) || !dense(*vw, dev) || !integer(o[6], &pos)) Py_RETURN_NONE;
+    if (dev < 0 || !v || !kw || !vw || !there(*k, dev) || !there(*v, dev) || !dense(*kw, dev) || !dense(*vw, dev) || !integer(o[6], &pos)) Py_RETURN_NONE;
     const auto type = k->scalar_type();
     if (k->dim() != 4 || k->size(3) != 128 || v->sizes() != k->sizes() || !half(*k) || v->scalar_type() != type || k->strides() != v->strides() ||
         k->stride(3) != 1 || kw->dim() != 4 || vw->sizes() != kw->sizes() || kw->size(0) != k->size(0) || kw->size(1) != k->size(1) ||
@@ -226,11 +232,11 @@ PyObject *window_append(PyObject *, PyObject *const *o, Py_ssize_t n) {
 // dense_view(k, v, k_win, v_win, win_len) -> (K, V), a status that is not zero, or None
 PyObject *dense_view(PyObject *, PyObject *const *o, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    if (n != 5 || modes() || o[0] == Py_None) Py_RETURN_NONE;
-    const int dev = here();
+    if (n != 5 || modes() || !PyDict_CheckExact(o[0])) Py_RETURN_NONE;
+    const int dev = here(tensor(PyDict_GetItemString(o[0], "scale")));
     pkv_attn_args a{};
     Cache c;
-    if (!cache_args(o[0], o[1], dev, 0, a, c) || !half(*c.like)) Py_RETURN_NONE;
+    if (dev < 0 || !cache_args(o[0], o[1], dev, 0, a, c) || !half(*c.like)) Py_RETURN_NONE;
     if (o[2] != Py_None && !window_args(tensor(o[2]), tensor(o[3]), o[4], dev, c, c.like->scalar_type(), a)) Py_RETURN_NONE;
     a.B = c.batch; a.Hkv = c.heads; a.T_c = c.tokens;
     a.dtype = code(*c.like);
@@ -259,11 +265,11 @@ PyObject *mat_vec(PyObject *, PyObject *const *o, Py_ssize_t n) {
     if (n != 11 || modes()) Py_RETURN_NONE;
     const bool is_k = o[0] == Py_True;
     const at::Tensor *stm = tensor(o[1]), *info = tensor(o[2]), *x = tensor(o[3]), *out = tensor(o[4]);
-    const int dev = here();
+    const int dev = here(x);
     int i[5];
     for (int j = 0; j < 5; j++)
         if (!integer(o[5 + j], &i[j])) Py_RETURN_NONE;
-    if (!stm || !info || !x || !out || !there(*stm, dev) || !there(*info, dev) || !there(*x, dev) || !there(*out, dev) || !half(*x) ||
+    if (dev < 0 || !stm || !info || !out || !there(*stm, dev) || !there(*info, dev) || !there(*x, dev) || !there(*out, dev) || !half(*x) ||
         (!is_k && out->scalar_type() != at::kFloat) || (o[10] != Py_True && o[10] != Py_False)) Py_RETURN_NONE;
     const uint64_t bytes = (uint64_t)stm->numel() * (uint64_t)stm->element_size();
     const pkv_stream_t s = stream(dev);
@@ -284,8 +290,8 @@ PyObject *fused(PyObject *, PyObject *const *o, Py_ssize_t n) {
     if (n != 6 || modes()) Py_RETURN_NONE;
     const bool is_k = o[0] == Py_True;
     const at::Tensor *out = tensor(o[1]), *x = tensor(o[2]), *zero = tensor(o[3]), *scale = tensor(o[4]), *t = tensor(o[5]);
-    const int dev = here();
-    if (!out || !x || !zero || !scale || !t || !dense(*out, dev) || !dense(*x, dev) || !dense(*zero, dev) || !dense(*scale, dev) || !dense(*t, dev) ||
+    const int dev = here(x);
+    if (dev < 0 || !out || !zero || !scale || !t || !dense(*out, dev) || !dense(*x, dev) || !dense(*zero, dev) || !dense(*scale, dev) || !dense(*t, dev) ||
         !half(*x)) Py_RETURN_NONE;
     if (out->dim() != 2 || x->dim() != 2 || t->dim() != 2 || zero->dim() != 1 || scale->dim() != 1) Py_RETURN_NONE;
     const int64_t M = x->size(0), K = x->size(1), T = t->size(1), columns = is_k ? T : K;

@@ -100,3 +100,21 @@ def test_what_is_refused_needs_no_library(monkeypatch):
         ops.fused_kq(*(torch.zeros(2, dtype=torch.float16) for _ in range(5)))
     with pytest.raises(ImportError, match="not built"):
         ops.block_bound(True, 64, 128, 4)
+
+
+def test_host_tensors_are_refused_by_name():
+    """The tensor is looked at before the runtime is asked for its device: there may be no GPU."""
+    half = lambda *s: torch.zeros(*s, dtype=torch.float16)
+    side = {"stream": torch.zeros(64, dtype=torch.uint8), "info": torch.zeros(2, 2, dtype=torch.uint32), "scale": half(1, 128), "zero": half(1, 128), "bits": 4}
+    stream, info = side["stream"], side["info"]
+    for call, message in ((lambda: ops.attn_decode(half(1, 8, 128), side, side), "q must be a contiguous device tensor"),
+                          (lambda: ops.window_append(half(1, 2, 1, 128), half(1, 2, 1, 128), None, None, half(1, 2, 8, 128), half(1, 2, 8, 128), 0),
+                           "K and V must be device tensors"),
+                          (lambda: ops.dense_view(side, side), "a compressed cache is on a GPU"),
+                          (lambda: ops.kq_mat_vec_mul(stream, info, half(1, 128), half(1, 64), 64, 128, 64, 128, 4), "tensor must be a CUDA tensor"),
+                          (lambda: ops.wv_mat_vec_mul(stream, info, half(1, 128), torch.zeros(1, 128), 128, 128, 128, 64, 4), "tensor must be a CUDA tensor"),
+                          (lambda: ops.fused_kq(half(1, 64), half(1, 128), half(64), half(64), half(1, 64)), "q must be a CUDA tensor"),
+                          (lambda: ops.fused_wv(half(1, 128), half(1, 64), half(64), half(64), half(1, 128)), "w must be a CUDA tensor")):
+        with pytest.raises(RuntimeError, match=message):
+            call()
+    assert _lib.host.plan_step(4096, 0, 1, half(1, 8, 128)) is None
