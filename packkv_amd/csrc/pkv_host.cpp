@@ -60,7 +60,9 @@ bool integer(PyObject *o, int *out) {
     return true;
 }
 
-template <typename F> int call(F &&f) {      // the library may wait or allocate: other threads go on
+// The library may wait or allocate: other threads go on meanwhile.  `f` calls it and nothing else: no address is taken in there (a lazily
+// cloned tensor gets its memory then, and may throw), no Python object touched.
+template <typename F> int call(F &&f) {
     int rc;
     Py_BEGIN_ALLOW_THREADS
     rc = f();
@@ -221,11 +223,12 @@ PyObject *window_append(PyObject *, PyObject *const *o, Py_ssize_t n) {
         sin_p = at_ptr<void>(*sin);
         rot = B > 1 ? cos->stride(0) : 0;
     }
+    const void *const k_p = at_ptr<void>(*k), *const v_p = at_ptr<void>(*v);
+    void *const kw_p = at_ptr<void>(*kw), *const vw_p = at_ptr<void>(*vw);
+    const int64_t sb = k->stride(0), sh = k->stride(1), st = k->stride(2);
+    const int dtype = code(*k);
     const pkv_stream_t s = stream(dev);
-    return status(call([&] {
-        return lib.window_append(at_ptr<void>(*k), at_ptr<void>(*v), cos_p, sin_p, code(*k), (int)B, (int)H, (int)rows, k->stride(0), k->stride(1), k->stride(2),
-                                 rot, at_ptr<void>(*kw), at_ptr<void>(*vw), pos, (int)cap, s);
-    }));
+    return status(call([&] { return lib.window_append(k_p, v_p, cos_p, sin_p, dtype, (int)B, (int)H, (int)rows, sb, sh, st, rot, kw_p, vw_p, pos, (int)cap, s); }));
     END_HANDLE_TH_ERRORS
 }
 
@@ -241,8 +244,9 @@ PyObject *dense_view(PyObject *, PyObject *const *o, Py_ssize_t n) {
     a.B = c.batch; a.Hkv = c.heads; a.T_c = c.tokens;
     a.dtype = code(*c.like);
     at::Tensor k = at::empty({c.batch, c.heads, (int64_t)c.tokens + a.T_w, 128}, c.like->options()), v = at::empty_like(k);
+    void *const k_p = at_ptr<void>(k), *const v_p = at_ptr<void>(v);
     const pkv_stream_t s = stream(dev);
-    const int rc = call([&] { return lib.dense_view(&a, at_ptr<void>(k), at_ptr<void>(v), s); });
+    const int rc = call([&] { return lib.dense_view(&a, k_p, v_p, s); });
     if (rc) return status(rc);
     PyObject *both = PyTuple_New(2);
     if (!both) return nullptr;
@@ -272,15 +276,14 @@ PyObject *mat_vec(PyObject *, PyObject *const *o, Py_ssize_t n) {
     if (dev < 0 || !stm || !info || !out || !there(*stm, dev) || !there(*info, dev) || !there(*x, dev) || !there(*out, dev) || !half(*x) ||
         (!is_k && out->scalar_type() != at::kFloat) || (o[10] != Py_True && o[10] != Py_False)) Py_RETURN_NONE;
     const uint64_t bytes = (uint64_t)stm->numel() * (uint64_t)stm->element_size();
+    const uint8_t *const stm_p = at_ptr<uint8_t>(*stm);
+    const uint32_t *const info_p = at_ptr<uint32_t>(*info);
+    const void *const x_p = at_ptr<void>(*x);
+    void *const out_p = at_ptr<void>(*out);
+    const int dtype = code(*x), interleaved = o[10] == Py_True;
     const pkv_stream_t s = stream(dev);
-    if (is_k)
-        return timed([&](float *ms) {
-            return lib.kq(at_ptr<uint8_t>(*stm), bytes, at_ptr<uint32_t>(*info), at_ptr<void>(*x), at_ptr<void>(*out), i[0], i[1], i[2], i[3], i[4], code(*x),
-                          o[10] == Py_True, ms, s);
-        });
-    return timed([&](float *ms) {
-        return lib.wv(at_ptr<uint8_t>(*stm), bytes, at_ptr<uint32_t>(*info), at_ptr<void>(*x), at_ptr<float>(*out), i[0], i[1], i[2], i[3], i[4], code(*x), ms, s);
-    });
+    if (is_k) return timed([&](float *ms) { return lib.kq(stm_p, bytes, info_p, x_p, out_p, i[0], i[1], i[2], i[3], i[4], dtype, interleaved, ms, s); });
+    return timed([&](float *ms) { return lib.wv(stm_p, bytes, info_p, x_p, (float *)out_p, i[0], i[1], i[2], i[3], i[4], dtype, ms, s); });
     END_HANDLE_TH_ERRORS
 }
 
@@ -297,11 +300,11 @@ PyObject *fused(PyObject *, PyObject *const *o, Py_ssize_t n) {
     const int64_t M = x->size(0), K = x->size(1), T = t->size(1), columns = is_k ? T : K;
     if (t->size(0) != M || zero->size(0) != columns || scale->size(0) != columns || out->size(0) != M || out->size(1) != T ||
         (!is_k && t->scalar_type() != x->scalar_type()) || M > INT_MAX || K > INT_MAX || T > INT_MAX) Py_RETURN_NONE;
+    void *const out_p = at_ptr<void>(*out);
+    const void *const x_p = at_ptr<void>(*x), *const zero_p = at_ptr<void>(*zero), *const scale_p = at_ptr<void>(*scale), *const t_p = at_ptr<void>(*t);
+    const int dtype = code(*x);
     const pkv_stream_t s = stream(dev);
-    return timed([&](float *ms) {
-        return (is_k ? lib.fused_kq : lib.fused_wv)(at_ptr<void>(*out), at_ptr<void>(*x), at_ptr<void>(*zero), at_ptr<void>(*scale), at_ptr<void>(*t), (int)M, (int)K,
-                                                    (int)T, code(*x), ms, s);
-    });
+    return timed([&](float *ms) { return (is_k ? lib.fused_kq : lib.fused_wv)(out_p, x_p, zero_p, scale_p, t_p, (int)M, (int)K, (int)T, dtype, ms, s); });
     END_HANDLE_TH_ERRORS
 }
 

@@ -229,3 +229,29 @@ def test_matrix_vector_ops(cuda, dtype, capsys):
                 ops.fused_kq(new(H, T + 1), q, ke["zero"].reshape(-1), ke["scale"].reshape(-1), new(H, T))
             with pytest.raises(RuntimeError):
                 ops.wv_mat_vec_mul(ve["stream"], ve["info"], w, new(H, 128), T, H * 128, 128, 64, 4)
+
+
+def test_a_tensor_that_does_not_give_its_address(cuda):
+    """data_ptr() may throw: the error is the general code's, whichever tensor it is, and the interpreter goes on."""
+    ke, ve, kw, vw, q = _cache(cuda, torch.float16, 1, 2, 256)
+    new = lambda *s: torch.zeros(*s, dtype=torch.float16, device=cuda)
+    win = [new(1, 2, 9, 128) for _ in range(2)]
+    rows, par = [new(1, 2, 1, 128) for _ in range(2)], [d[f].reshape(-1) for d in (ke, ve) for f in ("zero", "scale")]
+    table = [new(1, 1, 128) for _ in range(2)]
+    calls = {"append": (lambda a: ops.window_append(*a, 3), [*rows, *table, *win]),
+             "kq": (lambda a: ops.kq_mat_vec_mul(*a, 256, 256, 64, 128, 4), [ke["stream"], ke["info"], new(2, 128), new(2, 256)]),
+             "wv": (lambda a: ops.wv_mat_vec_mul(*a, 256, 256, 128, 64, 4), [ve["stream"], ve["info"], new(2, 256), torch.zeros(2, 128, device=cuda)]),
+             "fused_kq": (lambda a: ops.fused_kq(*a), [new(2, 256), new(2, 128), *par[:2], new(2, 256)]),
+             "fused_wv": (lambda a: ops.fused_wv(*a), [new(2, 128), new(2, 256), *par[2:], new(2, 128)]),
+             "attn": (lambda a: ops.attn_decode(a[0], ke, ve, *a[1:]), [q, kw, vw]),
+             "dense": (lambda a: ops.dense_view(ke, ve, *a), [kw, vw])}
+    for name, (call, tensors) in calls.items():
+        for i in range(len(tensors)):
+            closed = tensors[i].clone()
+            torch._C._set_throw_on_mutable_data_ptr(closed)
+            args = tensors[:i] + [closed] + tensors[i + 1:]
+            for serve in (True, False):
+                with _through(serve), pytest.raises(RuntimeError, match="data pointer"):
+                    call(args)
+        call(tensors)
+    torch.cuda.synchronize()
