@@ -254,8 +254,11 @@ __device__ __forceinline__ void wide_windows(const UnitWide &u, uint32_t e01[8],
 // reads of LDS a pack instead of four dwords: 199 us a step of 16 x 8 x 32768 tokens, now 148; 32 x 8 x 8192 with a window 110,
 // now 83.)
 #define PKV_DMA_WAVES(KW, G) ((KW) > 4 ? 2 : ((G) <= 4 ? 4 : 3))
-// Workgroups per CU that the cache is cut for (three of width 5 take 53 KB of its LDS each, width 6 takes 61; groups of 8 of
-// both keep the cut, and with it the size of their partials, that they had while one of them filled a CU's registers).
+// Workgroups per CU that the cache is cut for (three of width 5 take 53 KB of its LDS each, width 6 takes 61).  Groups of 8 of both
+// widths are cut for one, although two are resident, for the size of their partials alone: cut for two, a step of 489 to 511 (sequence, KV
+// head) pairs that share a window out would have more of them than pkv_attn_decode_noalloc's array holds, and that call takes such
+// steps.  Two are faster everywhere: 5 bits, one -> two, 3 x 4 KV heads x 11008 tokens with a window 23.5 -> 20.9 us, 1 x 8 x 65536 52 -> 37.5, 16 x
+// 8 x 8192 with a window 105 -> 71, 16 x 8 x 32768 334 -> 208, 40 x 8 x 8192 199 -> 162; 6 bits within 4 % of these.
 #define PKV_DMA_RESIDENT(KW, G) ((KW) > 4 ? ((G) > 4 ? 1 : (KW) == 5 ? 3 : 2) : ((G) <= 4 ? 4 : 3))
 template <bool WIDE> struct UnitOf { typedef UnitPairs type; };
 template <> struct UnitOf<true> { typedef UnitWide type; };
