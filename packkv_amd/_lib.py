@@ -133,7 +133,7 @@ def _load_host(lib):
     except ImportError as e:
         why = str(e)
     if why:
-        warnings.warn("packkv_amd._host is not used (%s): the calls that a decode loop repeats take 3 to 8 us more of host time each. "
+        warnings.warn("packkv_amd._host is not used (%s): the calls that a decode loop repeats take 4 to 8 us more of host time each. "
                       "`python -m packkv_amd.build` makes it." % why, RuntimeWarning, stacklevel=3)
         return NO_HOST
     _host.bind(*(ctypes.cast(getattr(lib, name), _vp).value for name in HOST_SYMBOLS))
