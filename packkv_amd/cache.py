@@ -193,8 +193,9 @@ class PackKVCompressedCache:
         kernels of ops.attn_decode (not cached as a plan)."""
         L = self.layers[layer_idx] or self._layer(layer_idx)
         q = query_states
-        if L.plan is not None and L.plan.sm_scale_arg == sm_scale and L.win_len and out is None and not (variant or ref_rounding or out_f32):
-            res = L.plan.step(q, L.win_len)
+        plan, rows = L.plan, L.win_len
+        if plan is not None and plan.sm_scale_arg == sm_scale and rows and out is None and not (variant or ref_rounding or out_f32):
+            res = plan.step(q, rows)
             if res is not None:
                 return res
         squeeze = q.dim() == 4
@@ -209,7 +210,6 @@ class PackKVCompressedCache:
             return res.unsqueeze(2) if squeeze else res
         if out is None:
             out = torch.empty_like(q)
-        plan = L.plan
         if plan is None or plan.sm_scale_arg != sm_scale or not L.win_len or plan._shape != q.shape or plan._dtype != q.dtype:
             k = L.k.as_dict() if L.k.tokens else None
             v = L.v.as_dict() if L.v.tokens else None

@@ -118,3 +118,25 @@ def test_host_tensors_are_refused_by_name():
         with pytest.raises(RuntimeError, match=message):
             call()
     assert _lib.host.plan_step(4096, 0, 1, half(1, 8, 128)) is None
+
+
+def test_a_plan_that_another_thread_drops_meanwhile_serves_the_step_that_has_it():
+    """attend looks at the layer's plan once: an update that cuts drops it at any time."""
+    from packkv_amd import cache as pc
+
+    class Plan:
+        sm_scale_arg = None
+
+        def step(self, q, rows):
+            return q, rows
+
+    class Layer:
+        win_len, plans = 3, [Plan()]
+
+        @property
+        def plan(self):
+            return self.plans.pop() if self.plans else None
+    cache = pc.PackKVCompressedCache(1, 2, 128, 1, device="cpu")
+    cache.layers[0] = Layer()
+    q = torch.zeros(1, 2, 128)
+    assert cache.attend(q, 0) == (q, 3)
